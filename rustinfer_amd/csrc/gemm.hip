@@ -2,10 +2,11 @@
 // checkpoint; reference contract: op_ports.rs:54-62).
 //
 //  * gemm_tiled: any M, N, K; float or bfloat16 inputs; FMA accumulation in a fixed order over K,
-//    so a row's result does not depend on the other rows of the batch.  This is the product of
-//    the exact 32-bit path (no reduced-precision matrix mode): for float inputs the sum is kept
-//    in 64-bit, as the reference's float path does on the CPU
-//    (crates/infer-backend-cpu/src/lib.rs:403-418), so that a long K adds no rounding of its own.
+//    so a row's result does not depend on the other rows of the batch.  It takes the products of
+//    the exact 32-bit path (no reduced-precision matrix mode) whose rows gemm_f32.hip cannot read
+//    16 bytes at a time: for float inputs the sum is kept in 64-bit, as the reference's float path
+//    does on the CPU (crates/infer-backend-cpu/src/lib.rs:403-418), so that a long K adds no
+//    rounding of its own.
 //  * gemm_skinny_bf16: M <= 64 rows against bfloat16 weights on the matrix cores, the weight
 //    matrix streamed once with 16-byte loads (reference: hgemv_bf16_v3 for one row,
 //    matmul.cu:870-929, cuBLASLt otherwise).
@@ -84,12 +85,14 @@ extern "C" int ri_gemm_tiled(const void* A, int lda, const void* W, int ldw, voi
 }
 
 // ---------------------------------------------------------------------------
-// gemm_rows_f32: the exact path's product for few rows (decoding; 16 a pass), where the tiled kernel
-// above would leave most of its 64 x 64 tile and of the chip idle.  The weights are streamed
-// once, 16 bytes a lane and row; a block brings 512 values of every activation row into LDS and
-// its four waves multiply them with four weight rows each.  Sums are kept in 64-bit as in the tiled
-// kernel; a lane adds its share of K in a fixed order and the lanes are added in a fixed tree, so
-// a row's result depends neither on the other rows nor on their number.  K % 4 == 0.
+// gemm_rows_f32: the exact path's product of up to 4 rows, where the 16 rows of a matrix instruction
+// (gemm_f32.hip) would do at least four times the work.  The weights are streamed once, 16 bytes a lane
+// and row; a block brings 512 values of every activation row into LDS and its four waves multiply
+// them with two or four weight rows each.  Sums are kept in 64-bit; a lane adds its share of K in
+// a fixed order and the lanes are added in a fixed tree, so a row's result depends neither on the
+// other rows nor on their number.  K % 4 == 0.  Measured, us, 4 rows, this kernel / gemm_f32:
+// 2048 x 8192 24 / 34; 4096 x 14336 53 / 59; 128256 x 2048 187 / 221; 16384 x 2048 37 / 32; at 6 rows
+// 32 / 34, 64 / 60, 288 / 236, 45 / 33.
 // ---------------------------------------------------------------------------
 template <int MR, int NB>
 __global__ __launch_bounds__(256) void gemm_rows_f32_kernel(
@@ -165,27 +168,14 @@ __global__ __launch_bounds__(256) void gemm_rows_f32_kernel(
 
 extern "C" int ri_gemm_rows_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
                                 int M, int N, int K, hipStream_t stream) {
-    RI_REQUIRE(M >= 1 && M <= 64 && N > 0 && K > 0 && K % 4 == 0, "ri_gemm_rows_f32: needs 1..64 rows and K %% 4 == 0 (M=%d N=%d K=%d)", M, N, K);
+    RI_REQUIRE(M >= 1 && M <= 4 && N > 0 && K > 0 && K % 4 == 0, "ri_gemm_rows_f32: needs 1..4 rows and K %% 4 == 0 (M=%d N=%d K=%d)", M, N, K);
     RI_REQUIRE(lda >= K && ldw >= K && ldc >= N && lda % 4 == 0 && ldw % 4 == 0, "ri_gemm_rows_f32: leading dimensions must be >= K and multiples of 4");
     RI_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0, "ri_gemm_rows_f32: null or unaligned pointer");
-    // 16 rows a pass: more rows stream the weights once more for every 16 (still ahead of the tiled kernel).
     // A wave owns four columns, or two where four would leave compute units without a block's worth
     // of loads in flight (a row's sums do not depend on that choice: a lane adds its share of K in
     // the same order either way).
-    const bool narrow = (N + 15) / 16 < 1024;
-    const int blocks = narrow ? (N + 7) / 8 : (N + 15) / 16;
-    for (int m0 = 0; m0 < M; m0 += 16) {
-        const int m = min(16, M - m0);
-        const float* a = A + (size_t)m0 * lda;
-        float* c = C + (size_t)m0 * ldc;
-#define RI_ROWS_F32(MR_) do { \
-        if (narrow) gemm_rows_f32_kernel<MR_, 2><<<blocks, 256, 0, stream>>>(a, lda, W, ldw, c, ldc, m, N, K); \
-        else gemm_rows_f32_kernel<MR_, 4><<<blocks, 256, 0, stream>>>(a, lda, W, ldw, c, ldc, m, N, K); } while (0)
-        if (m <= 4) RI_ROWS_F32(4);
-        else if (m <= 8) RI_ROWS_F32(8);
-        else RI_ROWS_F32(16);
-#undef RI_ROWS_F32
-    }
+    if ((N + 15) / 16 < 1024) gemm_rows_f32_kernel<4, 2><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    else gemm_rows_f32_kernel<4, 4><<<(N + 15) / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
     RI_LAUNCHED("ri_gemm_rows_f32");
     return 0;
 }

@@ -393,6 +393,20 @@ def test_linear_rows_do_not_depend_on_the_batch(ops):
             assert torch.equal(out[20], all16[3])
 
 
+@pytest.mark.parametrize("M,N,K", [(5, 16, 4), (16, 17, 60), (17, 33, 132), (31, 2064, 36), (33, 4100, 64), (49, 300, 260),
+                                   (65, 47, 1352), (160, 2050, 72), (300, 515, 516), (1030, 100, 20)])
+def test_linear_f32_on_the_matrix_instruction(ops, M, N, K):
+    # edges of every tile, a last chunk of K that is not whole, fewer chunks than waves, rows inside a wider buffer
+    xb, wb = rnd(M, K + 8, seed=M), rnd(N, K + 4, seed=N)
+    x, w = xb[:, 4:K + 4], wb[:, :K]
+    out = torch.full((M, N + 3), float("nan"), device=DEV)
+    ops.linear(x, w, out[:, :N])
+    ref = x.double() @ w.double().t()
+    # a 64-bit sum rounded once: half a unit of the last place of each result
+    assert torch.all((out[:, :N].double() - ref).abs() <= ref.abs() * 2.0 ** -24 + 1e-12 * ref.abs().max())
+    assert torch.all(torch.isnan(out[:, N:]))
+
+
 def _paged_setup(dtype, B, H, Hkv, hd, page, q_lens, starts, seed=0, num_pages=128, shuffle=True):
     """A cache with random pages for each request, the step's q/k/v, and contiguous copies."""
     g = torch.Generator().manual_seed(seed)
