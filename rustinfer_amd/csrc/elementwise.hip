@@ -407,6 +407,112 @@ __global__ __launch_bounds__(256) void rope_kv_write_bf16x8_kernel(
     }
 }
 
+// The same from the 32-bit sums of a q/k/v product whose weight has its rows in rotary order
+// (ri_qkv_rope_row_order in gemm.hip: every 16 columns are 8 features of the first half of a head and their 8
+// partners), divided over `parts` slices of K: the slices are added in order and rounded to bfloat16, as the rows
+// of an undivided projection are, then q and k are rotated.  A thread owns 16 columns: 64 contiguous bytes of each slice.  q goes to q_out, k and v to the pages.
+__global__ __launch_bounds__(256) void rope_kv_write_parts_kernel(
+        const float* __restrict__ sums, int parts, size_t part_stride, int ld, bf16_t* __restrict__ q_out, int q_stride,
+        int T, int H, int Hkv, int hd, const float* __restrict__ cos_t, const float* __restrict__ sin_t,
+        const int* __restrict__ positions, const int* __restrict__ row_of_token,
+        bf16_t* __restrict__ kc, bf16_t* __restrict__ vc, const int* __restrict__ table, int max_blocks, int page) {
+    const int half = hd >> 1, tph = hd >> 4;                     // tiles of 16 columns a head
+    auto tile_sums = [&](const float* src, float (&v)[16]) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) VecLoad<4>::ld(src + 4 * q, v + 4 * q);
+        for (int p = 1; p < parts; ++p) {
+            float o[16];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) VecLoad<4>::ld(src + p * part_stride + 4 * q, o + 4 * q);
+#pragma unroll
+            for (int e = 0; e < 16; ++e) v[e] += o[e];
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) v[e] = bf16_to_f32(f32_to_bf16(v[e]));
+    };
+    if ((int)blockIdx.x < T) {
+        const int t = blockIdx.x;
+        const int b = row_of_token[t];
+        if (b < 0) return;                       // padding token
+        const int pos = positions[t], slot = pos % page;
+        const int blk = table[(size_t)b * max_blocks + pos / page];
+        const bool own_values = blk >= 0 && !rope_value_run(t & ~15, T, row_of_token, positions, page);
+        const int heads = own_values ? H + 2 * Hkv : H + Hkv;
+        for (int idx = threadIdx.x; idx < heads * tph; idx += 256) {
+            const int h = idx / tph, i0 = (idx - h * tph) * 8;
+            if (h >= H && blk < 0) continue;
+            float v[16];
+            tile_sums(sums + (size_t)t * ld + (size_t)idx * 16, v);
+            if (h >= H + Hkv) {                  // a token whose values no group of 16 writes
+                bf16_t* dst = vc + ((size_t)blk * Hkv + (h - H - Hkv)) * page * hd + slot;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    dst[(size_t)(i0 + e) * page] = f32_to_bf16(v[e]);
+                    dst[(size_t)(half + i0 + e) * page] = f32_to_bf16(v[8 + e]);
+                }
+                continue;
+            }
+            float c[8], s[8], lo[8], hi[8];
+            VecLoad<4>::ld(cos_t + (size_t)pos * half + i0, c); VecLoad<4>::ld(cos_t + (size_t)pos * half + i0 + 4, c + 4);
+            VecLoad<4>::ld(sin_t + (size_t)pos * half + i0, s); VecLoad<4>::ld(sin_t + (size_t)pos * half + i0 + 4, s + 4);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) { lo[e] = v[e] * c[e] - v[8 + e] * s[e]; hi[e] = v[e] * s[e] + v[8 + e] * c[e]; }
+            bf16_t* dst = h < H ? q_out + (size_t)t * q_stride + (size_t)h * hd
+                                : kc + ((size_t)blk * Hkv + (h - H)) * page * hd + (size_t)slot * hd;
+            VecLoad<4>::st(dst + i0, lo); VecLoad<4>::st(dst + i0 + 4, lo + 4);
+            VecLoad<4>::st(dst + half + i0, hi); VecLoad<4>::st(dst + half + i0 + 4, hi + 4);
+        }
+        return;
+    }
+    // the values of 16 consecutive positions of one page: 32 contiguous bytes a feature
+    const int t0 = ((int)blockIdx.x - T) * 16;
+    if (!rope_value_run(t0, T, row_of_token, positions, page)) return;
+    const int b0 = row_of_token[t0], p0 = positions[t0];
+    const int blk = table[(size_t)b0 * max_blocks + p0 / page];
+    if (blk < 0) return;
+    const float* v0 = sums + (size_t)t0 * ld + (size_t)(H + Hkv) * hd;
+    for (int idx = threadIdx.x; idx < Hkv * hd; idx += 256) {    // column idx of the values
+        const int g = idx / hd, within = idx - g * hd, j = within >> 4, rr = within & 15;
+        const int feature = rr < 8 ? 8 * j + rr : half + 8 * j + rr - 8;
+        float v[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) v[i] = v0[(size_t)i * ld + idx];
+        for (int p = 1; p < parts; ++p) {
+            const float* vp = v0 + p * part_stride;
+            float o[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) o[i] = vp[(size_t)i * ld + idx];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) v[i] += o[i];
+        }
+        uint32_t w[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] = (uint32_t)f32_to_bf16(v[2 * i]) | ((uint32_t)f32_to_bf16(v[2 * i + 1]) << 16);
+        uint4* dst = reinterpret_cast<uint4*>(vc + ((size_t)blk * Hkv + g) * page * hd + (size_t)feature * page + p0 % page);
+        dst[0] = make_uint4(w[0], w[1], w[2], w[3]);
+        dst[1] = make_uint4(w[4], w[5], w[6], w[7]);
+    }
+}
+
+// sums: float32 [parts][T][ld] (part_stride elements apart), columns in rotary order; q_out [T][q_stride] bfloat16
+extern "C" int ri_rope_kv_write_parts(const float* sums, int parts, long long part_stride, int ld, void* q_out, int q_stride,
+                                      int T, int H, int Hkv, int hd, const float* cos_t, const float* sin_t, int table_rows,
+                                      const int* positions, const int* row_of_token, void* kc, void* vc, int num_pages,
+                                      const int* table, int max_blocks, int page, hipStream_t stream) {
+    RI_REQUIRE(T >= 0 && H > 0 && Hkv > 0 && hd > 0 && hd % 16 == 0 && page > 0 && parts >= 1, "ri_rope_kv_write_parts: bad sizes");
+    RI_REQUIRE(ld >= (H + 2 * Hkv) * hd && ld % 4 == 0 && q_stride >= H * hd && q_stride % 8 == 0
+               && (parts == 1 || (part_stride >= (long long)T * ld && part_stride % 4 == 0)), "ri_rope_kv_write_parts: bad strides");
+    if (T == 0) return 0;
+    RI_REQUIRE(sums && q_out && cos_t && sin_t && table_rows > 0 && positions && row_of_token && kc && vc && num_pages > 0
+               && table && max_blocks > 0, "ri_rope_kv_write_parts: null pointer or bad cache sizes");
+    RI_REQUIRE((uintptr_t)sums % 16 == 0 && (uintptr_t)q_out % 16 == 0 && (uintptr_t)cos_t % 16 == 0 && (uintptr_t)sin_t % 16 == 0
+               && (uintptr_t)kc % 16 == 0 && (uintptr_t)vc % 16 == 0 && page % 16 == 0, "ri_rope_kv_write_parts: operands must be 16-byte aligned and pages multiples of 16 tokens");
+    rope_kv_write_parts_kernel<<<T + (T + 15) / 16, 256, 0, stream>>>(sums, parts, (size_t)part_stride, ld, (bf16_t*)q_out, q_stride, T, H, Hkv, hd,
+        cos_t, sin_t, positions, row_of_token, (bf16_t*)kc, (bf16_t*)vc, table, max_blocks, page);
+    RI_LAUNCHED("ri_rope_kv_write_parts");
+    return 0;
+}
+
 extern "C" int ri_rope_kv_write(void* qkv, int act_dtype, int T, int row_stride, int H, int Hkv, int hd,
                                 int rot, const float* cos_t, const float* sin_t, int table_rows,
                                 const int* positions, const int* row_of_token,

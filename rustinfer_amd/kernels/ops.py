@@ -320,7 +320,7 @@ def _scale_args(scale, M: int, who: str):
 def qkv_rope_fused(x: torch.Tensor, w_fused: torch.Tensor, qkv: torch.Tensor, H: int, Hkv: int, hd: int,
                    rotary, positions: torch.Tensor, row_of_token: torch.Tensor, k_cache: torch.Tensor,
                    v_cache: torch.Tensor, block_table: torch.Tensor, page: int, scale=None) -> bool:
-    """For at most 64 single tokens: q/k/v projection, rotation by position and the write of k and v
+    """For steps of at most 64 tokens: q/k/v projection, rotation by position and the write of k and v
     into the cache in one kernel; rotated q lands in the first H*hd columns of ``qkv``.  Returns False
     (and does nothing) where the fused form does not apply; the caller then runs the separate kernels.
     ``scale``: see ``linear``."""
@@ -354,6 +354,54 @@ def qkv_rope_fused(x: torch.Tensor, w_fused: torch.Tensor, qkv: torch.Tensor, H:
         _ptr(x), x.stride(0), _ptr(w_fused), _ptr(qkv), qkv.stride(0), M, K, H, Hkv, hd, _ptr(cos), _ptr(sin),
         cos.shape[0], _ptr(positions), _ptr(row_of_token), _ptr(k_cache), _ptr(v_cache), k_cache.shape[0],
         _ptr(block_table), block_table.shape[1], page, sq, sp, se, _stream()))
+    return True
+
+
+def _mid_plan(M: int, N: int, K: int, swiglu: bool, any_parts: bool = False):
+    """(slices of K, whether blocks own 8 weight tiles) of ``ri_gemm_mid`` for this product; 0 slices: not its kind."""
+    parts, wide = ctypes.c_int(0), ctypes.c_int(0)
+    _check(_lib().ri_gemm_mid_plan(M, N, K, int(swiglu), int(any_parts), ctypes.byref(parts), ctypes.byref(wide)))
+    return parts.value, wide.value
+
+
+def _mid_ok(x: torch.Tensor, w, w_tiled) -> bool:
+    return (not FORCE_LIBRARY_GEMM and w_tiled is not None and x.dtype == torch.bfloat16 and x.shape[0] > SKINNY_MAX_ROWS
+            and x.stride(0) % 8 == 0 and x.stride(1) == 1 and x.data_ptr() % 16 == 0 and _tiled_ok(w, w_tiled))
+
+
+def qkv_rope_split(x: torch.Tensor, w_fused: torch.Tensor, qkv: torch.Tensor, H: int, Hkv: int, hd: int,
+                   rotary, positions: torch.Tensor, row_of_token: torch.Tensor, k_cache: torch.Tensor,
+                   v_cache: torch.Tensor, block_table: torch.Tensor, page: int, workspace) -> bool:
+    """``qkv_rope_fused`` for more tokens: the product over slices of K into 32-bit partial sums, and a kernel
+    that adds them, rotates q and k and writes k and v into the cache.  Returns False (and does nothing)
+    where that form does not apply."""
+    M, K = x.shape
+    if rotary is None or w_fused is None or page % 16 or not _mid_ok(x, w_fused, w_fused):
+        return False
+    cos, sin, rot = rotary
+    N = (H + 2 * Hkv) * hd
+    if rot != hd or qkv.dtype != torch.bfloat16 or qkv.stride(0) % 8 or qkv.data_ptr() % 16 or qkv.stride(1) != 1:
+        return False
+    parts, wide = _mid_plan(M, N, K, False, True)
+    if not parts:
+        return False
+    _dev(x, w_fused, qkv, cos, sin, positions, row_of_token, k_cache, v_cache, block_table)
+    if tuple(w_fused.shape) != (N, K) or qkv.shape[0] != M or qkv.shape[1] < H * hd:
+        raise KernelError("qkv_rope_split: shapes do not fit")
+    _check_cache(k_cache, v_cache, Hkv, hd, page, x.dtype, "qkv_rope_split")
+    _i32(positions, "positions", M)
+    _i32(row_of_token, "row_of_token", M)
+    _i32(block_table, "block_table")
+    if cos.dtype != torch.float32 or cos.shape != sin.shape or cos.shape[1] * 2 != hd or not cos.is_contiguous() or not sin.is_contiguous():
+        raise KernelError("qkv_rope_split: cos/sin must be contiguous float32 [positions, head_dim/2]")
+    lib = _lib()
+    sums = workspace.get("attn.qkv_sums", parts * M, N, torch.float32)
+    _check(lib.ri_gemm_mid(_ptr(x), x.stride(0), _ptr(w_fused), _ptr(sums), N, M, N, K, 0, parts, wide,
+                           ctypes.c_longlong(M * N), _stream()))
+    _check(lib.ri_rope_kv_write_parts(
+        _ptr(sums), parts, ctypes.c_longlong(M * N), N, _ptr(qkv), qkv.stride(0), M, H, Hkv, hd, _ptr(cos), _ptr(sin),
+        cos.shape[0], _ptr(positions), _ptr(row_of_token), _ptr(k_cache), _ptr(v_cache), k_cache.shape[0],
+        _ptr(block_table), block_table.shape[1], page, _stream()))
     return True
 
 
@@ -773,6 +821,14 @@ def linear_delta(x: torch.Tensor, w: torch.Tensor, workspace, name: str,
                                            _ptr(stack), N, M, N, K, F32, 0, parts, ctypes.c_longlong(M * N),
                                            int(tiled), ctypes.c_void_p(0), 0, ctypes.c_float(0.0), _stream()))
             return stack
+    if _mid_ok(x, w, w_tiled):
+        # more rows than that, but too few tiles for the chip: slices of K again
+        parts, wide = _mid_plan(M, N, K, False)
+        if parts > 1:
+            stack = workspace.get(name + ".parts", parts * M, N, torch.float32).view(parts, M, N)
+            _check(lib.ri_gemm_mid(_ptr(x), x.stride(0), _ptr(w_tiled), _ptr(stack), N, M, N, K, 0, parts, wide,
+                                   ctypes.c_longlong(M * N), _stream()))
+            return stack
     out = workspace.get(name, M, N, out_dtype or x.dtype)     # out_dtype: 32-bit sums of a bfloat16 product left unrounded
     linear(x, w, out, w_tiled)
     return out
@@ -809,6 +865,12 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor,
                                           w_gate_up.stride(0), _ptr(out), out.stride(0), M, I, K, BF16, 1, 1,
                                           ctypes.c_longlong(0), int(tiled), sq, sp, se, _stream()))
         return
+    if scale is None and I % 16 == 0 and out.stride(0) % 4 == 0 and out.data_ptr() % 16 == 0 and _mid_ok(x, w_gate_up, w_tiled):
+        parts, wide = _mid_plan(M, I, K, True)
+        if parts:
+            _check(_lib().ri_gemm_mid(_ptr(x), x.stride(0), _ptr(w_tiled), _ptr(out), out.stride(0), M, I, K, 1, 1, wide,
+                                      ctypes.c_longlong(0), _stream()))
+            return
     if scale is not None:
         raise KernelError("linear_swiglu: row factors of a deferred norm go with the few-row bfloat16 kernel only")
     if scratch is None or tuple(scratch.shape) != (M, 2 * I):

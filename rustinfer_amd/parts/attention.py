@@ -72,7 +72,7 @@ class PagedAttention(Mixer):
         self.rt = rt
         names = ["q_proj.weight"] + (["k_proj.weight", "v_proj.weight"] if self.own_kv else [])
         parts = [tensors[n].to(device=rt.device, dtype=rt.dtype) for n in names]
-        # for steps of few single tokens: projection, rotation and cache write in one kernel, which
+        # for steps of few tokens: projection, rotation and cache write in one kernel (or two), which
         # reads its own copy of the weight (rows ordered so that rotary partners meet in a tile);
         # the plain tile-ordered copy would never be read beside it
         make = getattr(rt.ops, "qkv_rope_weight", None)
@@ -103,10 +103,12 @@ class PagedAttention(Mixer):
         rotary = self.pos_enc.rotary() if self.pos_enc is not None else None
         table = ctx.block_tables[cache.group]
         kw = {} if scale is None else {"scale": scale}
-        fused = (self.qkv_fused is not None and cache.write and ctx.max_q_len == 1
-                 and ops.qkv_rope_fused(rows, self.qkv_fused, qkv, self.num_heads, self.num_kv_heads,
-                                        self.head_dim, rotary, ctx.positions, ctx.row_of_token,
-                                        cache.k, cache.v, table, cache.page_size, **kw))
+        fused = False
+        if self.qkv_fused is not None and cache.write:
+            args = (rows, self.qkv_fused, qkv, self.num_heads, self.num_kv_heads, self.head_dim, rotary,
+                    ctx.positions, ctx.row_of_token, cache.k, cache.v, table, cache.page_size)
+            split = getattr(ops, "qkv_rope_split", None)
+            fused = ops.qkv_rope_fused(*args, **kw) or (scale is None and split is not None and split(*args, ws))
         if not fused:
             self.qkv.forward(rows, qkv, scale)
             if self.qk_transform is not None:

@@ -640,6 +640,56 @@ def test_fused_projection_through_lds_from_17_tokens_and_in_wider_blocks(ops, mo
     assert taken
 
 
+@pytest.mark.parametrize("q_lens,starts,H,Hkv,hd,page,K,parts", [
+    ([65], [0], 4, 2, 16, 16, 64, 1), ([40, 1, 60, 33], [5, 30, 16, 0], 8, 2, 64, 16, 1024, 4), ([129], [15], 6, 6, 48, 32, 576, 2),
+    ([1] * 70, [3] * 70, 4, 4, 32, 16, 4096, 8), ([64, 200], [0, 48], 12, 4, 128, 16, 1344, 4)])
+def test_projection_in_slices_rotation_and_cache_write(ops, q_lens, starts, H, Hkv, hd, page, K, parts):
+    """More than 64 tokens: the product over slices of K and the kernel that adds, rotates and writes, against
+    projection and rope_kv_write; whole groups of 16 values and single ones, a padding token."""
+    B, T = len(q_lens), sum(q_lens)
+    qkv, kc, vc, table, ctx, _, _ = _paged_setup(torch.bfloat16, B, H, Hkv, hd, page, q_lens, starts, seed=K, num_pages=640)
+    ctx.row_of_token[T // 2] = -1
+    x, w = rnd(T, K, dtype=torch.bfloat16, seed=50), rnd((H + 2 * Hkv) * hd, K, dtype=torch.bfloat16, seed=51, scale=0.05)
+    ang = np.arange(512)[:, None] * plain_llama.rope_frequencies(hd, 10000.0, None)[None, :]
+    rotary = tuple(torch.tensor(f(ang), dtype=torch.float32, device=DEV) for f in (np.cos, np.sin)) + (hd,)
+    wf = ops.qkv_rope_weight(w, hd)
+    assert ops._mid_plan(T, (H + 2 * Hkv) * hd, K, False, True)[0] == parts
+    kc1, vc1, kc2, vc2 = kc.clone(), vc.clone(), kc.clone(), vc.clone()
+    ref, got = torch.zeros_like(qkv), torch.zeros_like(qkv)
+    ops.linear(x, w, ref)
+    ops.rope_kv_write(ref, H, Hkv, hd, rotary, ctx.positions, ctx.row_of_token, kc1, vc1, table, page)
+    assert ops.qkv_rope_split(x, wf, got, H, Hkv, hd, rotary, ctx.positions, ctx.row_of_token, kc2, vc2, table, page, Workspace(torch.device(DEV)))
+    live = (ctx.row_of_token >= 0).cpu()
+    big = max(1.0, ref[live].float().abs().max().item() / 2)       # two roundings of the largest sum against one
+    assert torch.allclose(got[live, :H * hd].float(), ref[live, :H * hd].float(), atol=2e-2 * big, rtol=2e-2)
+    assert torch.equal(torch.isnan(kc2), torch.isnan(kc1)) and torch.equal(torch.isnan(vc2), torch.isnan(vc1))
+    for a, b in ((kc2, kc1), (vc2, vc1)):
+        assert torch.allclose(torch.nan_to_num(a.float()), torch.nan_to_num(b.float()), atol=2e-2 * big, rtol=2e-2)
+    assert torch.all(got[~live] == 0)                              # the padding token
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 16, 64), (127, 112, 320), (128, 4096, 64), (129, 2064, 1088), (300, 528, 4096), (513, 240, 704)])
+def test_products_of_some_hundred_rows(ops, M, N, K):
+    """Slices of K and the gate/up product with its activation, at the edges of blocks, tiles and slices."""
+    xb = rnd(M, K + 16, dtype=torch.bfloat16, seed=M)
+    x, w = xb[:, 8:K + 8], rnd(N, K, dtype=torch.bfloat16, seed=N)
+    ref = x.double() @ w.double().t()
+    got = ops.linear_delta(x, w, Workspace(torch.device(DEV)), "t", ops.tile_weight(w))
+    parts = ops._mid_plan(M, N, K, False)[0]
+    assert parts >= 1 and (got.dim() == 3) == (parts > 1)
+    if parts > 1:                                                  # 32-bit sums of K products of numbers around one
+        assert got.shape == (parts, M, N)
+        assert torch.allclose(got.double().sum(0), ref, rtol=0, atol=2e-6 * K ** 0.5 * 4)
+    I = N // 32 * 16
+    if I:
+        w, ref = w[:2 * I], ref[:, :2 * I]
+        out = torch.full((M, I), float("nan"), dtype=torch.bfloat16, device=DEV)
+        assert ops._mid_plan(M, I, K, True)[0] == 1
+        ops.linear_swiglu(x, w, out, None, ops.tile_weight(w))
+        want = torch.nn.functional.silu(ref[:, :I]) * ref[:, I:]
+        assert torch.allclose(out.double(), want, rtol=2.0 ** -8, atol=2.0 ** -8 + 1e-5 * K ** 0.5)
+
+
 def _check_fused_projection(ops, B, H, Hkv, hd, page, K):
     q_lens, starts = [1] * B, [(7 * i + 3) % 60 for i in range(B)]
     qkv, kc, vc, table, ctx, _, _ = _paged_setup(torch.bfloat16, B, H, Hkv, hd, page, q_lens, starts, seed=K, num_pages=640)
