@@ -1162,6 +1162,23 @@ def window_attention(q: torch.Tensor, out: torch.Tensor, H: int, Hkv: int, dk: i
 # ---------------------------------------------------------------------------
 # mixers with a matrix of state for each head
 # ---------------------------------------------------------------------------
+SCAN_CHUNK_TOKENS = 32          # rows of so many tokens and more go through chunks, in a step that uses them
+
+
+def _scan_in_chunks(delta: bool, d: int, rows: int, longest: int) -> bool:
+    """Whether a step with ``rows`` prompt portions of up to ``longest`` tokens runs the state walk in chunks of
+    tokens.  The walk's time is its longest row's, whatever else is in the step, until the rows fill the chip;
+    the chunks' grows with all tokens.  Measured, us, walk / chunks, 32 heads of 64, delta form: 1 x 48 29 / 30,
+    1 x 64 37 / 31, 1 x 2048 1205 / 232, 2 x 64 38 / 34, 4 x 64 39 / 42, 4 x 128 70 / 53, 4 x 512 305 / 173,
+    8 x 512 319 / 336; decay form: 1 x 48 20 / 21, 1 x 64 24 / 21, 1 x 2048 768 / 100, 4 x 64 25 / 22, 8 x 64
+    27 / 32, 8 x 128 50 / 37, 24 x 256 205 / 228.  24 heads of 128, delta form: 1 x 64 47 / 67, 1 x 96 70 / 72,
+    1 x 2048 1741 / 559, 2 x 128 125 / 90, 4 x 512 512 / 525; decay form: 1 x 64 30 / 28, 2 x 64 32 / 36, 2 x 128
+    71 / 44, 8 x 128 143 / 90."""
+    if delta:
+        return rows * d <= 256 and longest >= max(64, 32 * rows) * d // 64
+    return rows <= 16 and longest >= (64 if rows <= 4 and d <= 64 else 128)
+
+
 def linear_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, out: torch.Tensor, ctx,
                 H: int, dk: int, dv: int, decay: Optional[torch.Tensor] = None, silu_in: bool = False,
                 wl: Optional[torch.Tensor] = None, al: Optional[torch.Tensor] = None,
@@ -1201,13 +1218,29 @@ def linear_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
     if rotary is not None:
         rot = int(rotary[2])
         rcos, rsin, rrows = _rot_tables(rotary, rot, "linear_scan")
-    _check(_lib().ri_linear_scan(
-        _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0),
-        _ptr(wl), wl.stride(0) if wl is not None else 0, _ptr(al), al.stride(0) if al is not None else 0, _dt(r),
-        _ptr(w0), _ptr(ab), _ptr(decay), int(delta), int(bool(silu_in)), ctypes.c_float(unit_eps),
-        ctypes.c_float(decay_c), _ptr(state), state.shape[0], _ptr(out), out.stride(0),
-        _ptr(ctx.cu_q), _ptr(ctx.q_start), _ptr(ctx.state_slots), ctx.num_rows, T, H, dk, dv,
-        rcos, rsin, rot, rrows, max(int(ctx.max_kv_len) - 1, 0), ctypes.c_float(k_scale), _stream()))
+    lib = _lib()
+    inputs = (_ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0),
+              _ptr(wl), wl.stride(0) if wl is not None else 0, _ptr(al), al.stride(0) if al is not None else 0)
+    form = (_ptr(w0), _ptr(ab), _ptr(decay), int(delta), int(bool(silu_in)), ctypes.c_float(unit_eps),
+            ctypes.c_float(decay_c), _ptr(state), state.shape[0], _ptr(out), out.stride(0),
+            _ptr(ctx.cu_q), _ptr(ctx.q_start), _ptr(ctx.state_slots), ctx.num_rows, T, H, dk, dv,
+            rcos, rsin, rot, rrows, max(int(ctx.max_kv_len) - 1, 0), ctypes.c_float(k_scale))
+    most = 0
+    longest, workspace = int(ctx.max_q_len), getattr(ctx, "workspace", None)
+    portions = int(getattr(ctx, "num_portion", 0) or ctx.num_rows)
+    if workspace is not None and r.dtype == torch.bfloat16 and _scan_in_chunks(delta, dk, portions, longest) \
+            and lib.ri_linear_scan_chunks_supported(int(delta), dk, dv, ctypes.c_float(decay_c)):
+        # prompts: chunks of tokens on the matrix instructions; the walk takes the rows of fewer tokens, if there are any.
+        # (32-bit projections stay with the walk, whose bits do not depend on how a request was cut into steps)
+        lib.ri_linear_scan_chunks_workspace.restype = ctypes.c_size_t
+        need = lib.ri_linear_scan_chunks_workspace(int(delta), ctx.num_rows, longest, H, dk, dv)
+        ws = workspace.get("scan.chunks", need, 1, torch.float32)
+        _check(lib.ri_linear_scan_chunks(*inputs, *form, SCAN_CHUNK_TOKENS, longest, _ptr(ws), ctypes.c_size_t(ws.numel()), _stream()))
+        most = SCAN_CHUNK_TOKENS - 1
+        host_q = getattr(ctx, "host_q_lens", None)
+        if host_q is not None and min(host_q) > most:
+            return
+    _check(lib.ri_linear_scan(*inputs, _dt(r), *form, most, _stream()))
 
 
 def gated_group_norm(o: torch.Tensor, weight: Optional[torch.Tensor], gate: Optional[torch.Tensor], out: torch.Tensor,
