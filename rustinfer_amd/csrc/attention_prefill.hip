@@ -5,10 +5,16 @@
 // A wave owns 16 consecutive queries of one request and NQ query heads of one kv head; the
 // four waves of a block own a tile of 64 consecutive queries, so they read the same keys and
 // values at about the same time.  Under the causal mask a late tile sees many keys and an
-// early one few, so every block does two tiles one after the other, the i-th from the end and
-// the i-th from the start: all waves of a launch then have the same amount of work, whatever
-// order blocks are started in.  Blocks of one kv head are Hkv apart in the grid, which with 8
-// kv heads puts each head's keys and values into one XCD's L2.  Per step of 32 keys:
+// early one few.  Where a launch has waves to spare, every block does two tiles one after the
+// other, the i-th from the end and the i-th from the start (paired): all waves then have the same
+// amount of work, whatever order blocks are started in.  Elsewhere a block does one tile, a
+// row's tiles from the end, the rows side by side; where all blocks fit on the chip at once (folded),
+// the earlier half of the tiles follows from the start, so that a compute unit that is given two
+// blocks in turn comes out even.  That is twice the
+// blocks, or the same number with two heads a wave, which halves the reads of LDS a product (the
+// bound with one head: eight fragments of 1 KB a step for eight products).  Blocks of one kv head
+// are Hkv apart in the grid, which with 8 kv heads puts each head's keys and values into one XCD's
+// L2.  Per step of 32 keys:
 //   S^T[key, q] = K_tile[16 keys, hd] . Q^T[hd, 16 q]      (two tiles)   v_mfma_f32_16x16x32_bf16
 //   online softmax per query in 32-bit (running maximum and sum, exp2)
 //   O[q, d]    += P[16 q, 32 keys] . V[32 keys, 16 d]                    v_mfma_f32_16x16x32_bf16
@@ -56,7 +62,7 @@ struct PrefillFrags {
 // walk the keys in step, up to the last key any of them sees; a quarter of the traffic between
 // L2 and the CUs, which is what bounds the kernel once a prompt portion has waves enough.
 // SPLIT (with SHARE): the keys are also divided between blocks, split_keys of them (a multiple of
-// 128) to each value of the grid's third index; a block leaves what its range of keys gives a
+// 128) to each range, nsplit ranges next to each other in the grid's third index; a block leaves what its range of keys gives a
 // query (the sums, their softmax reference and the probabilities' total, in 32-bit) in part_o /
 // part_ml, and attn_prefill_combine_kernel puts a query's ranges together.  For short portions
 // behind a long cached prefix, whose few tiles would otherwise each walk all the keys one step
@@ -67,14 +73,17 @@ __global__ __launch_bounds__(256, WPE) void attn_prefill_kernel(
         const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
         const int* __restrict__ table, int max_blocks,
         const int* __restrict__ cu_q, const int* __restrict__ q_start, const int* __restrict__ kv_lens,
-        int H, int Hkv, int page_arg, float scale_log2e, int window_arg, int head_groups, int min_q_len,
+        int H, int Hkv, int page_arg, float scale_log2e, int window_arg, int min_q_len,
         int split_keys, int nsplit, float* __restrict__ part_o, float* __restrict__ part_ml, int part_tokens,
-        const int* __restrict__ row_list) {
+        const int* __restrict__ row_list, int order) {
     typedef PrefillFrags<HD> Frags;
     static_assert(!SHARE || FAST, "fragments are shared only with pages of 16 and no window");
     static_assert(!SPLIT || SHARE, "the keys are divided between blocks only in the shared form");
     // this block's range of keys [kb, ke)
-    const int split = SPLIT ? (int)__builtin_amdgcn_workgroup_id_z() : 0;
+    // the grid's second and third index: row and place among the row's blocks; in pairs, place and row
+    const bool paired = order == 1;
+    const int by = __builtin_amdgcn_workgroup_id_y(), bz = __builtin_amdgcn_workgroup_id_z();
+    const int split = SPLIT ? bz % nsplit : 0, at = SPLIT ? bz / nsplit : paired ? by : bz;
     const int kb = SPLIT ? split * split_keys : 0;
     const int ke = SPLIT && split + 1 < nsplit ? kb + split_keys : 0x7fffffff;     // the last range takes what is left
     constexpr int NF = HD / 8;                                   // fragments of a step: 2 * HD/32 of keys, HD/16 of values
@@ -84,19 +93,19 @@ __global__ __launch_bounds__(256, WPE) void attn_prefill_kernel(
     // Block and thread ids are taken from the builtins: this file's floating-point flags keep
     // the device library's id functions from being inlined, and a call would hide from the
     // compiler that block ids are the same for all lanes.
-    // row_list (may be null): the rows this kernel is for, then -1; the grid's second index then runs over those
+    // row_list (may be null): the rows this kernel is for, then -1; the grid then runs over those
     const int bx = __builtin_amdgcn_workgroup_id_x();
-    const int b = row_list ? row_list[__builtin_amdgcn_workgroup_id_y()] : (int)__builtin_amdgcn_workgroup_id_y();
+    const int at_row = paired && !SPLIT ? bz : by;
+    const int b = row_list ? row_list[at_row] : at_row;
     if (b < 0) return;
     const int tx = __builtin_amdgcn_workitem_id_x();
     const int t_lo = cu_q[b], q_len = cu_q[b + 1] - t_lo;
     // the wave index is the same for all lanes; telling the compiler lets it keep the key loop
     // and the block-table reads on the scalar unit
     const int wave = __builtin_amdgcn_readfirstlane(tx >> 6), lane = tx & 63;
-    const int g = bx % Hkv, rest = bx / Hkv;
-    const int hsub = rest % head_groups, pair = rest / head_groups;
-    const int ntiles = (q_len + 63) / 64;                        // tiles of 64 queries of this row
-    if (q_len < min_q_len || pair >= (ntiles + 1) / 2) return;
+    const int g = bx % Hkv, hsub = bx / Hkv;
+    const int ntiles = (q_len + 63) / 64, late = (ntiles + 1) / 2;    // tiles of 64 queries of this row, and how many are the later half
+    if (q_len < min_q_len || at >= (paired ? late : ntiles)) return;
     const int G = H / Hkv;
     const int col = lane & 15, grp = lane >> 4;
     const int start = q_start[b];
@@ -113,8 +122,9 @@ __global__ __launch_bounds__(256, WPE) void attn_prefill_kernel(
 
 #pragma unroll 1
     for (int half = 0; half < 2; ++half) {
-        const int tile = half == 0 ? ntiles - 1 - pair : pair;   // the late tile first
-        if (half == 1 && tile == ntiles - 1 - pair) break;       // the middle tile of an odd number is done once
+        // paired: the late tile first; else the one tile of this block
+        const int tile = half == 0 && (at < late || order == 0) ? ntiles - 1 - at : paired ? at : at - late;
+        if (half == 1 && (!paired || tile == ntiles - 1 - at)) break;     // the middle tile of an odd number is done once
         if constexpr (SPLIT) {
             // no query of the tile sees a key of this block's range (the same for all waves)
             if (min(kv_len, start + min(q_len, tile * 64 + 64)) <= kb) continue;
@@ -576,37 +586,84 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(
     dst[3] = f32_to_bf16(acc.w * inv);
 }
 
-// How a step's prompt portions are divided over ranges of keys: 1 (not at all) where the tiles of
-// queries alone give the chip its waves or few keys lie before the portion, else as many ranges
-// (multiples of 128 keys) as bring the waves to about two a SIMD, at most one for every 256 keys
-// that were cached before the step.  Measured on 32 heads over 8 kv heads of 128, us, undivided ->
-// divided: 16 tokens behind 2,048: 40 -> 20; 256 behind 2,048: 78 -> 40; 256 behind 8,192: 271 ->
-// 73; 512 behind 1,536: 66 -> 43; 512 behind 7,680: 259 -> 110; 1,024 behind 3,072: 126 -> 99.  A
-// portion that starts a prompt has its work balanced by the pairing of late and early tiles and
-// only loses (1,024 tokens: 28 -> 40 in two ranges).
-static void prefill_split_plan(int H, int Hkv, int hd, int page, int window, int total_q, int max_prefix,
-                               int max_kv_len, int forced, int* nsplit, int* split_keys) {
-    *nsplit = 1;
-    *split_keys = 0;
-    if (!(page == 16 && window == 0 && (hd == 64 || hd == 128)) || max_kv_len <= 0 || forced == 1) return;
-    const long long tile_pairs = ((total_q + 63) / 64 + 1) / 2;
-    const long long waves = tile_pairs * 4 * H;                  // of one head each
-    int n = forced > 1 ? forced : (int)std::min<long long>(2048 / std::max<long long>(waves, 1), std::max(max_prefix, 0) / 256);
-    n = std::min(n, 32);
-    if (n < 2) return;
-    const int keys = (((max_kv_len + n - 1) / n + 127) / 128) * 128;
-    n = (max_kv_len + keys - 1) / keys;
-    if (n < 2) return;
-    *nsplit = n;
-    *split_keys = keys;
+// How a step's prompt portions are divided: the heads a wave takes, whether a block does two tiles of queries
+// (paired), and over how many ranges of keys (multiples of 128).  The chip wants about two waves a SIMD, 2,048;
+// w1 is what one head a wave and one tile a block would give.
+//
+// Ranges of keys: for portions that have fewer waves than that behind many cached keys.  A portion that
+// starts a prompt only loses.  One head a wave and at least 512 keys a range (256 up to half the waves); from
+// 1,024 keys a range and a prefix of four times the step's tokens on two heads a wave and twice the ranges, which
+// read LDS half as often.  Measured on 32 heads over 8 kv heads, us, undivided with one tile a block -> divided:
+// head 128: 16 tokens behind 2,048: 40 -> 20; 256 behind 8,192: 142 -> 63; 512 behind 7,680: 139 -> 88 (one head
+// a wave: 104); 512 behind 1,536 stays undivided (40; 44).  head 64: 128 behind 2,048: 27 -> 19; 512 behind 8,192:
+// 94 -> 61.
+//
+// Undivided, pages of 16 without a window (blocks that share keys and values through LDS).  us, one head a wave in
+// pairs of tiles (what ran before where nothing else is said) -> now:
+//   head 64: one head a wave and one tile a block up to 4,608 waves (2,048 tokens 37 -> 31, 1,100 23.6 -> 20.5); from
+//     5,120 on, and from 3,072 where a third or more of the keys lie before the step, two heads (3,000 tokens 63 -> 55;
+//     2,048 behind 2,048 92 -> 68, behind 14,336 404 -> 295), in pairs again from 8,192 on without such a prefix
+//     (6,000 tokens 215 -> 179; single tiles 188); with one, four heads (4,096 behind 8,192 449 -> 349; two 379); from
+//     16,384 waves on four heads in pairs (8,192 tokens 300; four heads single 329).
+//   head 128: two heads a wave from 4,096 waves on, from 3,072 behind such a prefix (2,048 tokens 58 -> 56, 3,000
+//     124 -> 94, 2,048 behind 8,192 432 -> 296, 1,500 behind 1,500 103 -> 87), in pairs from 8,192 on (4,096 tokens 147;
+//     single tiles 161); below that one head (1,024 tokens 28.2 -> 24.7, 1,763 in five rows of 24 heads 50 -> 46); rows none
+//     of which is half the step stay with one head in pairs up to 8,192 (four rows of 512 27; two heads 28, single 30).
+//   An odd number of heads a kv head would leave a wave's second head idle: one head (head 128: two in pairs from 2,048
+//   such waves on, 4,096 tokens of 24 heads 163 -> 147).  One head of 64 a wave goes in pairs from 4,608 waves on without
+//   such a prefix (4,096 tokens of 24 heads: 83; single 90).
+//   Folded or not, head 128: 1,500 tokens 43 / 37, 3,000 101 / 94, but 2,048 behind 1,024, whose blocks all fit, 81 / 85;
+//   head 64 (blocks of 32 KB): 3,000 behind 3,000 of 24 heads 138 / 147, 4,096 behind 2,048 155 / 174, never slower by more than noise.
+struct PrefillPlan { int heads, nsplit, split_keys, order; };      // order: 0 single tiles from the end, 1 pairs, 2 folded
+
+static PrefillPlan prefill_plan(int H, int Hkv, int hd, int page, int window, int total_q, int longest_q,
+                                int max_prefix, int max_kv_len, int forced) {
+    PrefillPlan p{1, 1, 0, 1};
+    const int G = H / Hkv;
+    const bool even = G % 2 == 0;
+    if (page != 16 || window != 0) {
+        // query heads per wave: more of them share each key and value load, fewer of them give more
+        // waves.  Four (head size 64) or two as long as that leaves two waves for every SIMD of the chip.
+        p.heads = G < 2 ? G : 2;
+        for (int n = hd == 64 ? 4 : 2; n > 2; --n) {
+            const long long waves = (long long)((total_q + 15) / 16) * Hkv * (G / n);
+            if (G % n == 0 && waves >= 2048) { p.heads = n; break; }
+        }
+        return p;
+    }
+    const long long tiles = std::max((total_q + 63) / 64, 1);
+    const long long w1 = tiles * 4 * H;
+    const int prefix = std::max(max_prefix, 0);
+    if (max_kv_len > 0 && forced != 1) {
+        const long long two = even && prefix >= 4LL * total_q ? std::min<long long>(4096 / w1, 32) : 0;
+        long long n = std::max(std::min<long long>(2048 / w1, prefix / 512), std::min<long long>(1024 / w1, prefix / 256));
+        if (two >= 2 && prefix >= 1024 * two) { n = two; p.heads = 2; }
+        if (forced > 1) n = forced;
+        n = std::min<long long>(n, 32);
+        if (n >= 2) {
+            p.split_keys = (int)((((long long)max_kv_len + n - 1) / n + 127) / 128) * 128;
+            p.nsplit = (max_kv_len + p.split_keys - 1) / p.split_keys;
+            if (p.nsplit >= 2) { p.order = 2; return p; }
+        }
+        p = PrefillPlan{1, 1, 0, 1};
+    }
+    const bool behind = prefix >= (total_q + 1) / 2;
+    bool paired;
+    if (hd == 64 && G % 4 == 0 && (w1 >= 16384 || (w1 >= 8192 && behind))) { p.heads = 4; paired = w1 >= 16384; }
+    else if (even && (w1 >= (hd == 64 ? 5120 : 4096) || (w1 >= 3072 && behind))) { p.heads = 2; paired = w1 >= 8192; }
+    else if (hd == 128 && G >= 3 && (tiles + 1) / 2 * 4 * Hkv * ((G + 1) / 2) >= 2048) { p.heads = 2; paired = true; }
+    else { p.heads = 1; paired = w1 >= 4608 && !behind && !(hd == 128 && G > 1); }
+    if (hd == 128 && even && w1 >= 4096 && w1 < 8192 && !behind && 2 * longest_q < total_q) { p.heads = 1; paired = true; }
+    // a block of head 128 holds 64 KB of LDS: two on a compute unit
+    p.order = paired ? 1 : hd == 64 || tiles * Hkv * ((G + p.heads - 1) / p.heads) <= 512 ? 2 : 0;
+    return p;
 }
 
 // bytes of workspace ri_attention_prefill may use for a step of total_q tokens whose rows hold at
 // most max_kv_len keys (0: it will not divide the keys)
 extern "C" size_t ri_attention_prefill_workspace(int H, int Hkv, int hd, int page, int window, int total_q,
                                                  int max_prefix, int max_kv_len, int splits) {
-    int n, keys;
-    prefill_split_plan(H, Hkv, hd, page, window, total_q, max_prefix, max_kv_len, splits, &n, &keys);
+    const int n = prefill_plan(H, Hkv, hd, page, window, total_q, total_q, max_prefix, max_kv_len, splits).nsplit;
     return n < 2 ? 0 : (size_t)n * total_q * H * (hd + 2) * sizeof(float);
 }
 
@@ -641,87 +698,55 @@ extern "C" int ri_attention_prefill(
     RI_REQUIRE((uintptr_t)q % 16 == 0 && (uintptr_t)kc % 16 == 0 && (uintptr_t)vc % 16 == 0, "ri_attention_prefill: operands must be 16-byte aligned");
     const int G = H / Hkv;
     const bool fast = page == 16 && window == 0;
-    // Query heads per wave: more of them share each key and value load, fewer of them give more
-    // waves.  Four (head size 64) or two as long as that leaves two waves for every SIMD of the chip.
-    int NQ = G < 2 ? G : 2;
-    for (int n = hd == 64 ? 4 : 2; n > 2; --n) {
-        const long long waves = (long long)((total_q + 15) / 16) * Hkv * (G / n);
-        if (G % n == 0 && waves >= 2048) { NQ = n; break; }
-    }
-    // Pages of 16, no window: the waves of a block may hand each other the keys and values
-    // through LDS (SHARE).  Measured on 32 heads over 8 kv heads, times of the plain form = 1:
-    //   head 128: one head per wave (twice the waves, and sharing takes away what that would
-    //     cost in traffic) 0.77 at 2,048 tokens, 0.59 for 512 tokens behind 1,536; from 2,048
-    //     waves of two heads on, two heads per wave with registers capped at 256 so that two
-    //     waves share a SIMD: 0.68 at 4,096 tokens, 0.61 at 8,192, 0.56 behind 16,384.
-    //   head 64: one head per wave up to 8,192 waves of one head (against the plain form with
-    //     four heads per wave: 0.85 at 2,048 tokens, 0.86 at 4,096); beyond that four heads per
-    //     wave, two waves per SIMD (0.84 at 8,192 tokens, 0.78 behind 16,384; one head per wave
-    //     there: 1.0 and 1.05).
     const float sl2 = scale * 1.4426950408889634f;
-    const long long pairs = ((max_q_len + 63) / 64 + 1) / 2;
+    const PrefillPlan plan = prefill_plan(H, Hkv, hd, page, window, total_q, max_q_len, max_prefix, max_kv_len, workspace ? splits : 1);
+    const int NQ = plan.heads, nsplit = plan.nsplit, split_keys = plan.split_keys;
+    const bool paired = plan.order == 1;
+    const long long row_tiles = (max_q_len + 63) / 64, places = (paired ? (row_tiles + 1) / 2 : row_tiles) * nsplit;
+    const int head_groups = (G + NQ - 1) / NQ;
     RI_REQUIRE(B <= 65535, "ri_attention_prefill: too many rows");
-    int nsplit = 1, split_keys = 0;
-    prefill_split_plan(H, Hkv, hd, page, window, total_q, max_prefix, max_kv_len, workspace ? splits : 1, &nsplit, &split_keys);
+    RI_REQUIRE((long long)Hkv * head_groups <= 0x7fffffffLL && places <= 65535, "ri_attention_prefill: grid too large");
+    float *part_o = nullptr, *part_ml = nullptr;
     if (nsplit > 1) {
         const size_t need = (size_t)nsplit * total_q * H * (hd + 2) * sizeof(float);
         RI_REQUIRE(workspace_bytes >= need && (uintptr_t)workspace % 16 == 0, "ri_attention_prefill: workspace of %zu bytes, %zu needed", workspace_bytes, need);
-        RI_REQUIRE(pairs * Hkv * G <= 0x7fffffffLL && nsplit <= 65535, "ri_attention_prefill: grid too large");
-        float* part_o = (float*)workspace;
-        float* part_ml = part_o + (size_t)nsplit * total_q * H * hd;
-        dim3 grid((unsigned)(pairs * Hkv * G), BY, nsplit);
-#define RI_PREFILL_SPLIT_ARGS (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)kc, (const bf16_t*)vc, table, max_blocks, cu_q, q_start, kv_lens, H, Hkv, page, sl2, window, G, min_q_len, split_keys, nsplit, part_o, part_ml, total_q, row_list
+        part_o = (float*)workspace;
+        part_ml = part_o + (size_t)nsplit * total_q * H * hd;
+    }
+    dim3 grid(Hkv * head_groups, paired ? (unsigned)places : BY, paired ? BY : (unsigned)places);
+#define RI_PREFILL_LAUNCH(...) attn_prefill_kernel<__VA_ARGS__><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)kc, (const bf16_t*)vc, table, max_blocks, cu_q, q_start, kv_lens, H, Hkv, page, sl2, window, min_q_len, split_keys, nsplit, part_o, part_ml, total_q, row_list, plan.order)
+    if (nsplit > 1) {
+        if (hd == 64 && NQ == 2) RI_PREFILL_LAUNCH(64, 2, true, true, 3, true);
+        else if (hd == 64) RI_PREFILL_LAUNCH(64, 1, true, true, 1, true);
+        else if (NQ == 2) RI_PREFILL_LAUNCH(128, 2, true, true, 2, true);
+        else RI_PREFILL_LAUNCH(128, 1, true, true, 1, true);
+        RI_LAUNCHED("ri_attention_prefill(ranges)");
         const long long per_row = (long long)max_q_len * H * (hd / 4);
         dim3 cgrid((unsigned)((per_row + 255) / 256), BY);
-        if (hd == 64) {
-            attn_prefill_kernel<64, 1, true, true, 1, true><<<grid, 256, 0, stream>>>(RI_PREFILL_SPLIT_ARGS);
-            RI_LAUNCHED("ri_attention_prefill(ranges)");
-            attn_prefill_combine_kernel<64><<<cgrid, 256, 0, stream>>>(part_o, part_ml, total_q, nsplit, split_keys, (bf16_t*)out, out_stride, cu_q, q_start, kv_lens, H, min_q_len, row_list);
-        } else {
-            attn_prefill_kernel<128, 1, true, true, 1, true><<<grid, 256, 0, stream>>>(RI_PREFILL_SPLIT_ARGS);
-            RI_LAUNCHED("ri_attention_prefill(ranges)");
-            attn_prefill_combine_kernel<128><<<cgrid, 256, 0, stream>>>(part_o, part_ml, total_q, nsplit, split_keys, (bf16_t*)out, out_stride, cu_q, q_start, kv_lens, H, min_q_len, row_list);
-        }
-#undef RI_PREFILL_SPLIT_ARGS
+        if (hd == 64) attn_prefill_combine_kernel<64><<<cgrid, 256, 0, stream>>>(part_o, part_ml, total_q, nsplit, split_keys, (bf16_t*)out, out_stride, cu_q, q_start, kv_lens, H, min_q_len, row_list);
+        else attn_prefill_combine_kernel<128><<<cgrid, 256, 0, stream>>>(part_o, part_ml, total_q, nsplit, split_keys, (bf16_t*)out, out_stride, cu_q, q_start, kv_lens, H, min_q_len, row_list);
         RI_LAUNCHED("ri_attention_prefill(combine)");
         return 0;
     }
-    bool share = false, two_per_simd = false;
-    const long long tile_pairs = ((total_q + 63) / 64 + 1) / 2;
-    if (hd == 128 && fast) {
-        const long long waves_two_heads = tile_pairs * 4 * Hkv * ((G + 1) / 2);
-        share = true;
-        two_per_simd = G >= 2 && waves_two_heads >= 2048;
-        NQ = two_per_simd ? 2 : 1;
-    } else if (hd == 64 && fast) {
-        const long long waves_one_head = tile_pairs * 4 * Hkv * G;
-        share = true;
-        if (waves_one_head >= 8192 && G % 4 == 0) { two_per_simd = true; NQ = 4; }
-        else NQ = 1;
-    }
-    const int head_groups = (G + NQ - 1) / NQ;
-    RI_REQUIRE(pairs * Hkv * head_groups <= 0x7fffffffLL, "ri_attention_prefill: grid too large");
-    dim3 grid((unsigned)(pairs * Hkv * head_groups), BY);
-#define RI_PREFILL_ARGS (const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)kc, (const bf16_t*)vc, table, max_blocks, cu_q, q_start, kv_lens, H, Hkv, page, sl2, window, head_groups, min_q_len, 0, 1, nullptr, nullptr, 0, row_list
-    // pages of 16 without a window always take a shared form; the plain form serves the rest
-#define RI_PREFILL_LAUNCH(HD_, NQ_) attn_prefill_kernel<HD_, NQ_, false><<<grid, 256, 0, stream>>>(RI_PREFILL_ARGS)
-    if (hd == 64 && share) {
-        if (two_per_simd) attn_prefill_kernel<64, 4, true, true, 2><<<grid, 256, 0, stream>>>(RI_PREFILL_ARGS);
-        else attn_prefill_kernel<64, 1, true, true><<<grid, 256, 0, stream>>>(RI_PREFILL_ARGS);
+    // pages of 16 without a window always take a shared form (registers capped so that two waves, or three, share a
+    // SIMD); the plain form serves the rest
+    if (hd == 64 && fast) {
+        if (NQ == 4) RI_PREFILL_LAUNCH(64, 4, true, true, 2);
+        else if (NQ == 2) RI_PREFILL_LAUNCH(64, 2, true, true, 3);
+        else RI_PREFILL_LAUNCH(64, 1, true, true);
     } else if (hd == 64) {
-        if (NQ == 1) RI_PREFILL_LAUNCH(64, 1);
-        else if (NQ == 2) RI_PREFILL_LAUNCH(64, 2);
-        else if (NQ == 3) RI_PREFILL_LAUNCH(64, 3);
-        else RI_PREFILL_LAUNCH(64, 4);
-    } else if (share) {
-        if (two_per_simd) attn_prefill_kernel<128, 2, true, true, 2><<<grid, 256, 0, stream>>>(RI_PREFILL_ARGS);
-        else attn_prefill_kernel<128, 1, true, true><<<grid, 256, 0, stream>>>(RI_PREFILL_ARGS);
+        if (NQ == 1) RI_PREFILL_LAUNCH(64, 1, false);
+        else if (NQ == 2) RI_PREFILL_LAUNCH(64, 2, false);
+        else if (NQ == 3) RI_PREFILL_LAUNCH(64, 3, false);
+        else RI_PREFILL_LAUNCH(64, 4, false);
+    } else if (fast) {
+        if (NQ == 2) RI_PREFILL_LAUNCH(128, 2, true, true, 2);
+        else RI_PREFILL_LAUNCH(128, 1, true, true);
     } else {
-        if (NQ == 1) RI_PREFILL_LAUNCH(128, 1);
-        else RI_PREFILL_LAUNCH(128, 2);
+        if (NQ == 1) RI_PREFILL_LAUNCH(128, 1, false);
+        else RI_PREFILL_LAUNCH(128, 2, false);
     }
 #undef RI_PREFILL_LAUNCH
-#undef RI_PREFILL_ARGS
     RI_LAUNCHED("ri_attention_prefill");
     return 0;
 }

@@ -511,6 +511,23 @@ def test_attention_of_a_long_portion_at_head_size_64(ops):
     _check_rope_write_and_attention(ops, torch.bfloat16, (1, 128, 32, 64, 16, [2100], [0]), 0, kv_heads=(0, 13, 31))
 
 
+@pytest.mark.parametrize("H,hd,q_lens,starts", [
+    # 32 kv heads, pages of 16: what a wave and a block take, by waves and by the keys before the step
+    (128, 64, [70, 1, 33], [30, 40, 0]),                         # one head, one tile a block; odd numbers of tiles
+    (128, 64, [570], [0]), (128, 64, [400, 65, 129], [300, 0, 7]),    # two heads, one tile a block
+    (128, 64, [1040, 3], [0, 50]),                               # two heads, pairs of tiles
+    (128, 64, [1030], [600]),                                    # four heads, one tile a block
+    (96, 64, [800, 2], [0, 9]),                                  # three heads a kv head: one head, pairs of tiles
+    (128, 64, [200], [2100]), (128, 128, [200], [2100]),         # two ranges of keys, two heads a wave
+    (128, 128, [520, 70], [0, 129]), (128, 128, [1100], [0]),    # two heads, single tiles and pairs
+    (96, 128, [500], [0]), (96, 128, [1000], [64]),              # three heads a kv head: one head, and two with one idle
+])
+def test_attention_of_portions_however_they_are_divided(ops, H, hd, q_lens, starts):
+    """Tiles of queries, heads and ranges of keys dealt to waves and blocks in each way the sizes can ask for; three kv
+    heads' groups are compared with the plain computation."""
+    _check_rope_write_and_attention(ops, torch.bfloat16, (len(q_lens), H, 32, hd, 16, q_lens, starts), 0, kv_heads=(0, 13, 31))
+
+
 RANGE_CASES = [
     # B, H, Hkv, hd, page, q_lens, starts; ranges of keys asked for (0: the kernel's own choice)
     ((1, 8, 2, 128, 16, [16], [2040]), 0),                       # a short portion behind many keys: six ranges of 384
