@@ -7,8 +7,11 @@
 // bfloat16 instructions do sixteen times the work of the 32-bit ones, so three of them are a fifth of one.
 //
 // Keys in sight, heads of two maps and their difference: attention_masks.h, attention_window.hip (which
-// takes what these kernels do not: 32-bit storage, turned values, kept first positions, sigmoid
-// weights, other page sizes).  A sink joins the denominator at the end.  Scores may be soft-capped, c tanh(s / c), and
+// takes what these kernels do not: 32-bit storage, kept first positions, sigmoid
+// weights, other page sizes).  A sink joins the denominator at the end.  Values may be cached turned by
+// their positions; a query's sums are then turned back by its own, in 32-bit (Turn).  That is a few operations an
+// output; on the 32-bit instructions, where such values went before, 2,048 tokens with a window of 1,024 took 294 us
+// a layer of 32 heads over 8 of 64 and now take 66, and 8 single tokens behind some forty keys 18.2 and 10.3.  Scores may be soft-capped, c tanh(s / c), and
 // a head's output may be multiplied by a sigmoid (HeadGate).
 // Cache layout: keys [pages][Hkv][page][maps dk], values [pages][Hkv][dv][page]; pages of a multiple of 16.
 //
@@ -65,6 +68,23 @@ struct ScoreHow {
     }
 };
 
+// c, s [positions][dv / 2]: the cosines and sines values are turned by (null: not); the pairs are features (m, m + dv / 2), or
+// (2 m, 2 m + 1)
+struct Turn {
+    const float *c, *s;
+    int interleaved;
+    // writes the sums o (32-bit, dv of them) of a query at position p, turned back
+    __device__ __forceinline__ void write(bf16_t* out, const float* o, int p, int dv, int lane) const {
+        const int vh = dv >> 1;
+        for (int m = lane; m < vh; m += 64) {
+            const int i0 = interleaved ? 2 * m : m, i1 = interleaved ? 2 * m + 1 : m + vh;
+            const float a = o[i0], b = o[i1], cc = c[(size_t)p * vh + m], ss = s[(size_t)p * vh + m];
+            st_f32(out + i0, a * cc + b * ss);
+            st_f32(out + i1, b * cc - a * ss);
+        }
+    }
+};
+
 // 1 / denominator of a map from its reference m (log2 domain) and sum l, a sink (natural domain) joining
 __device__ __forceinline__ float ap_final(float m, float l, const float* __restrict__ sink, int vh) {
     if (!(l > 0.f)) return 0.f;
@@ -86,7 +106,7 @@ __global__ __launch_bounds__(256, FT <= 4 && DU <= 8 ? 2 : 1) void attn_parts_pr
         const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc, const int* __restrict__ table, int max_blocks,
         const int* __restrict__ cu_q, const int* __restrict__ q_start, const int* __restrict__ kv_lens,
         int num_rows, int H, int Hkv, int dk, int dv, int page, ScoreHow how, int window, int chunk, int maps, DiffHow diff,
-        const float* __restrict__ sink, HeadGate<bf16_t> hgate, int tiles) {
+        const float* __restrict__ sink, HeadGate<bf16_t> hgate, Turn turn, int tiles) {
     const float scale_log2e = how.scale_log2e;
     extern __shared__ __align__(16) float lds[];       // [4 waves][32][dv + 4]: the outputs, after the last keys
     const int G = H / Hkv, HB = G < 4 ? G : 4, SB = 4 / HB, TQB = 32 * SB;
@@ -271,6 +291,10 @@ __global__ __launch_bounds__(256, FT <= 4 && DU <= 8 ? 2 : 1) void attn_parts_pr
         }
         return;
     }
+    if (turn.c) {
+        for (int r = 0; r < ntw; ++r) turn.write(out + (size_t)(t0w + r) * out_stride + vh * dv, ow + r * os, p0w + r, dv, lane);
+        return;
+    }
     for (int r = 0; r < ntw; ++r)
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
@@ -425,7 +449,7 @@ __global__ __launch_bounds__(256) void attn_parts_combine_kernel(
         const float* __restrict__ part_ml, const float* __restrict__ part_o, bf16_t* __restrict__ out, int out_stride,
         const int* __restrict__ cu_q, const int* __restrict__ q_start, const int* __restrict__ kv_lens,
         int H, int dv, int window, int chunk, int slots, DiffHow diff, const float* __restrict__ sink,
-        HeadGate<bf16_t> hgate) {
+        HeadGate<bf16_t> hgate, Turn turn) {
     __shared__ float wts[MAPS][AP_SLOTS];
     __shared__ float acc_s[4][MAPS][64 * NC];
     const int b = blockIdx.y, ho = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -473,6 +497,11 @@ __global__ __launch_bounds__(256) void attn_parts_combine_kernel(
     bf16_t* o = out + (size_t)t * out_stride + ho * dv;
     if constexpr (MAPS == 2) {
         aw_write_difference<bf16_t, NC>(o, acc[0], acc[1], dv, lane, diff);
+    } else if (turn.c) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) acc_s[0][0][lane + 64 * c] = acc[0][c];
+        __builtin_amdgcn_wave_barrier();                   // (one wave is left; its stores and loads of LDS keep their order)
+        turn.write(o, acc_s[0][0], p, dv, lane);
     } else {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
@@ -504,17 +533,20 @@ extern "C" size_t ri_attention_parts_workspace(int T, int H, int dv, int maps, i
 // single_tokens != 0: every row has at most one token, row b's is token cu_q[b] (workspace needed).
 // softcap > 0: a score s becomes softcap tanh(s / softcap).  gate [T][>= H] (null: none) with a row stride: a head's
 // output is multiplied by the sigmoid of its number there (maps = 1).
+// vcos / vsin [v_table_rows][dv / 2] (null: none): the sums are turned back by the query's position (maps = 1, no gate).
 extern "C" int ri_attention_parts(
         const void* q, int q_stride, void* out, int out_stride, const void* kc, const void* vc, int num_pages, int page,
         int H, int Hkv, int dk, int dv, const int* table, int max_blocks, const int* cu_q, const int* q_start, const int* kv_lens,
         int num_rows, int T, float scale, int window, int chunk, int maps, float diff_lam, float diff_gain, float diff_eps,
-        const float* sink, float softcap, const void* gate, int gate_stride, int single_tokens, int max_kv_len, float* workspace,
+        const float* sink, const float* vcos, const float* vsin, int v_table_rows, int v_interleaved,
+        float softcap, const void* gate, int gate_stride, int single_tokens, int max_kv_len, float* workspace,
         size_t workspace_floats, hipStream_t stream) {
     RI_REQUIRE(ri_attention_parts_supported(H, Hkv, dk, dv, maps, page), "ri_attention_parts: sizes not taken (H=%d Hkv=%d dk=%d dv=%d maps=%d page=%d)", H, Hkv, dk, dv, maps, page);
     RI_REQUIRE(T >= 0 && num_rows >= 0 && max_blocks > 0 && num_pages > 0 && window >= 0 && chunk >= 0, "ri_attention_parts: bad sizes");
     RI_REQUIRE(maps == 1 || diff_eps > 0.f, "ri_attention_parts: the difference of two maps takes an eps > 0");
     RI_REQUIRE(q_stride >= H * maps * dk && out_stride >= H * dv && q_stride % 8 == 0, "ri_attention_parts: row strides too small, or a query stride that is no multiple of 8");
     RI_REQUIRE(softcap >= 0.f && (!gate || (maps == 1 && gate_stride >= H)), "ri_attention_parts: softcap must be >= 0; a gate goes with one map a head and a row stride of at least the heads");
+    RI_REQUIRE(!vcos || (vsin && v_table_rows > 0 && maps == 1 && !gate), "ri_attention_parts: turned values need both tables, one map a head and no gate");
     if (T == 0 || num_rows == 0) return 0;
     RI_REQUIRE(q && out && kc && vc && table && cu_q && q_start && kv_lens, "ri_attention_parts: null pointer");
     RI_REQUIRE((uintptr_t)q % 16 == 0 && (uintptr_t)kc % 16 == 0 && (uintptr_t)vc % 16 == 0, "ri_attention_parts: operands must be aligned to 16 bytes");
@@ -526,6 +558,7 @@ extern "C" int ri_attention_parts(
     bf16_t* ob = (bf16_t*)out;
     const ScoreHow how{softcap > 0.f ? 1.f : scale * LOG2E, softcap * LOG2E, softcap > 0.f ? 2.f * scale * LOG2E / softcap : 0.f};
     const HeadGate<bf16_t> hgate{(const bf16_t*)gate, gate_stride};
+    const Turn turn{vcos, vsin, v_interleaved};
     if (single_tokens) {
         const int slots = ap_slots(window, chunk, max_kv_len), CG = (G + 15) / 16;
         RI_REQUIRE(workspace && max_kv_len > 0 && workspace_floats >= (size_t)T * Hm * slots * (dv + 2), "ri_attention_parts: workspace of %zu floats for %d slots", workspace_floats, slots);
@@ -543,7 +576,7 @@ extern "C" int ri_attention_parts(
                          : NC == 3 ? attn_parts_combine_kernel<3, MM> : attn_parts_combine_kernel<4, MM>)
         auto combine = maps == 2 ? RI_AP_COMBINE(2) : RI_AP_COMBINE(1);
 #undef RI_AP_COMBINE
-        combine<<<dim3(H, num_rows), 256, 0, stream>>>(part_ml, part_o, ob, out_stride, cu_q, q_start, kv_lens, Hm, dv, window, chunk, slots, diff, sink, hgate);
+        combine<<<dim3(H, num_rows), 256, 0, stream>>>(part_ml, part_o, ob, out_stride, cu_q, q_start, kv_lens, Hm, dv, window, chunk, slots, diff, sink, hgate, turn);
         RI_LAUNCHED("ri_attention_parts");
         return 0;
     }
@@ -561,7 +594,7 @@ extern "C" int ri_attention_parts(
             } \
         } \
         kernel<<<dim3(tiles * Hkv, (G + 3) / 4), 256, lds, stream>>>(qb, q_stride, ob, out_stride, kb, vb, table, max_blocks, cu_q, q_start, kv_lens, num_rows, \
-            Hm, Hkv, dk, dv, page, how, window, chunk, maps, diff, sink, hgate, tiles); } while (0)
+            Hm, Hkv, dk, dv, page, how, window, chunk, maps, diff, sink, hgate, turn, tiles); } while (0)
 #define RI_AP_F(D) do { if (FT <= 2) RI_AP(D, 2); else if (FT <= 4) RI_AP(D, 4); else RI_AP(D, 8); } while (0)
     if (DU <= 4) RI_AP_F(4);
     else if (DU <= 8) RI_AP_F(8);

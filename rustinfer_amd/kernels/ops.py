@@ -1121,7 +1121,7 @@ def window_attention(q: torch.Tensor, out: torch.Tensor, H: int, Hkv: int, dk: i
     vcos, vsin, vrows = _rot_tables(value_rotary, dv, "window_attention (values)")
     lib = _lib()
     single = int(ctx.max_q_len == 1 and T <= ctx.num_rows)
-    if WINDOW_ATTENTION_PARTS and q.dtype == torch.bfloat16 and value_rotary is None and keep_first == 0 and sigmoid_bias is None \
+    if WINDOW_ATTENTION_PARTS and q.dtype == torch.bfloat16 and keep_first == 0 and sigmoid_bias is None \
             and scale > 0 and q.stride(0) % 8 == 0 and q.data_ptr() % 16 == 0 \
             and lib.ri_attention_parts_supported(H, Hkv, dk, dv, maps, page):
         # both products on the bfloat16 matrix instructions, the weights as three bfloat16 parts
@@ -1133,8 +1133,8 @@ def window_attention(q: torch.Tensor, out: torch.Tensor, H: int, Hkv: int, dk: i
         _check(lib.ri_attention_parts(
             _ptr(q), q.stride(0), _ptr(out), out.stride(0), _ptr(k_cache), _ptr(v_cache), k_cache.shape[0], page,
             H, Hkv, dk, dv, _ptr(block_table), block_table.shape[1], _ptr(ctx.cu_q), _ptr(ctx.q_start), _ptr(ctx.kv_lens),
-            ctx.num_rows, T, ctypes.c_float(scale), int(window), int(chunk), maps, lam, gain, diff_eps, _ptr(sink), *extras,
-            single, int(ctx.max_kv_len), _ptr(ws), ctypes.c_size_t(need), _stream()))
+            ctx.num_rows, T, ctypes.c_float(scale), int(window), int(chunk), maps, lam, gain, diff_eps, _ptr(sink), vcos, vsin, vrows,
+            int(bool(interleaved_values)), *extras, single, int(ctx.max_kv_len), _ptr(ws), ctypes.c_size_t(need), _stream()))
         return
     if ctx.max_q_len > 1 and WINDOW_ATTENTION_MFMA and lib.ri_attention_window_mfma_supported(H, Hkv, dk, dv, maps):
         # steps with prompt portions: both products on the 32-bit matrix instructions

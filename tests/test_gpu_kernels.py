@@ -528,6 +528,36 @@ def test_attention_of_portions_however_they_are_divided(ops, H, hd, q_lens, star
     _check_rope_write_and_attention(ops, torch.bfloat16, (len(q_lens), H, 32, hd, 16, q_lens, starts), 0, kv_heads=(0, 13, 31))
 
 
+@pytest.mark.parametrize("interleaved", [False, True])
+@pytest.mark.parametrize("H,Hkv,hd,q_lens,starts,window", [
+    (8, 2, 64, [70, 1, 33], [30, 200, 0], 50), (3, 3, 24, [40, 7], [0, 90], 0), (6, 2, 128, [33], [64], 33), (2, 1, 256, [9, 1], [20, 40], 17),
+    (8, 2, 64, [1] * 4, [0, 31, 64, 300], 100), (12, 2, 40, [1, 1], [5, 130], 0), (2, 2, 128, [1], [4500], 0), (2, 1, 256, [1, 1], [63, 65], 1)])
+def test_turned_values_with_weights_in_three_parts(ops, monkeypatch, H, Hkv, hd, q_lens, starts, window, interleaved):
+    """Values cached turned by their positions: the bfloat16 matrix instructions with the weights in three parts give what
+    the 32-bit kernel gives, to the outputs' rounding (two roundings of one number: a unit in the last place, 2^-7 at
+    most), in portions, mixed steps and single tokens, over the edges of tiles and partial results."""
+    B = len(q_lens)
+    need = sum((s + q + 15) // 16 for s, q in zip(starts, q_lens))
+    qkv, kc, vc, table, ctx, hist_k, hist_v = _paged_setup(torch.bfloat16, B, H, Hkv, hd, 16, q_lens, starts, seed=hd + H,
+                                                           num_pages=max(128, need + 16))
+    for b in range(B):
+        for j in range(starts[b], starts[b] + q_lens[b]):
+            kc[int(table[b, j // 16]), :, j % 16] = hist_k[b][j].to(DEV)
+            vc[int(table[b, j // 16]), :, :, j % 16] = hist_v[b][j].to(DEV)
+    ang = torch.arange(5000, dtype=torch.float64)[:, None] * 300.0 ** (-torch.arange(hd // 2, dtype=torch.float64) / (hd // 2))
+    tables = (ang.cos().float().to(DEV), ang.sin().float().to(DEV))
+    q, got = qkv[:, :H * hd].contiguous(), []
+    for parts in (True, False):
+        monkeypatch.setattr(ops, "WINDOW_ATTENTION_PARTS", parts)
+        monkeypatch.setattr(ops, "WINDOW_ATTENTION_MFMA", False)
+        out = torch.empty_like(q)
+        ops.window_attention(q, out, H, Hkv, hd, hd, kc, vc, table, 16, ctx, hd ** -0.5, window, value_rotary=tables,
+                             interleaved_values=interleaved)
+        got.append(out.float())
+    assert got[1].isfinite().all() and got[1].abs().max() > 0.02      # (a mean of n unit normals is about n^-0.5: 0.015 for the longest row)
+    assert ((got[0] - got[1]).abs() <= 2.0 ** -7 * got[1].abs() + 2e-5).all()
+
+
 RANGE_CASES = [
     # B, H, Hkv, hd, page, q_lens, starts; ranges of keys asked for (0: the kernel's own choice)
     ((1, 8, 2, 128, 16, [16], [2040]), 0),                       # a short portion behind many keys: six ranges of 384
