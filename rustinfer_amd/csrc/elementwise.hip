@@ -599,18 +599,35 @@ extern "C" int ri_swiglu(const void* gate_up, void* out, int act_dtype, int T, i
 // ---------------------------------------------------------------------------
 // out[t, i] = f(in[t, i]) over n columns of rows with strides of their own (columns of a wider
 // buffer; in place where out == in).  f: 0 = relu(z)^2, 1 = tanh(z); 32-bit arithmetic.
+// unary_bf16x8: 16 bytes a thread, where rows begin at multiples of that and hold whole ones and there are a block's worth for
+// every compute unit; bound by memory then, where two bytes a thread are bound by the number of waves (2,048 rows of
+// 8,192: 31.3 us -> 13.2; 8 rows take 4.7 either way, and stay with the waves of the plain form).
 // ---------------------------------------------------------------------------
+__device__ __forceinline__ float unary_of(float z, int op) {
+    if (op != 0) return tanhf(z);
+    const float r = fmaxf(z, 0.f);
+    return r * r;
+}
+
+__global__ __launch_bounds__(256) void unary_bf16x8_kernel(const bf16_t* __restrict__ in, int in_stride, bf16_t* __restrict__ out,
+                                                           int out_stride, int n, int op) {
+    const int i = (blockIdx.x * 256 + threadIdx.x) * 8;
+    if (i >= n) return;
+    const size_t t = blockIdx.y;
+    union { uint4 v; bf16_t u[8]; } x;
+    x.v = *reinterpret_cast<const uint4*>(in + t * in_stride + i);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) st_f32(x.u + k, unary_of(ld_f32(x.u + k), op));
+    *reinterpret_cast<uint4*>(out + t * out_stride + i) = x.v;
+}
+
 template <typename T>
 __global__ __launch_bounds__(256) void unary_kernel(const T* __restrict__ in, int in_stride, T* __restrict__ out,
                                                     int out_stride, int n, int op) {
     const int t = blockIdx.y;
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= n) return;
-    const float z = ld_f32(in + (size_t)t * in_stride + i);
-    float y;
-    if (op == 0) { const float r = fmaxf(z, 0.f); y = r * r; }
-    else y = tanhf(z);
-    st_f32(out + (size_t)t * out_stride + i, y);
+    st_f32(out + (size_t)t * out_stride + i, unary_of(ld_f32(in + (size_t)t * in_stride + i), op));
 }
 
 extern "C" int ri_unary(const void* in, int in_stride, void* out, int out_stride, int dtype, int T, int n, int op,
@@ -621,7 +638,9 @@ extern "C" int ri_unary(const void* in, int in_stride, void* out, int out_stride
     RI_REQUIRE(in && out, "ri_unary: null pointer");
     RI_REQUIRE(T <= 65535, "ri_unary: too many rows for the grid");
     dim3 grid((n + 255) / 256, T);
-    if (dtype == RI_F32) unary_kernel<float><<<grid, 256, 0, stream>>>((const float*)in, in_stride, (float*)out, out_stride, n, op);
+    const bool vec = dtype == RI_BF16 && (long long)T * n >= 256 * 256 * 8 && n % 8 == 0 && in_stride % 8 == 0 && out_stride % 8 == 0 && ((uintptr_t)in | (uintptr_t)out) % 16 == 0;
+    if (vec) unary_bf16x8_kernel<<<dim3((n / 8 + 255) / 256, T), 256, 0, stream>>>((const bf16_t*)in, in_stride, (bf16_t*)out, out_stride, n, op);
+    else if (dtype == RI_F32) unary_kernel<float><<<grid, 256, 0, stream>>>((const float*)in, in_stride, (float*)out, out_stride, n, op);
     else if (dtype == RI_BF16) unary_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)in, in_stride, (bf16_t*)out, out_stride, n, op);
     else return ri_fail("ri_unary: unknown dtype %d", dtype);
     RI_LAUNCHED("ri_unary");

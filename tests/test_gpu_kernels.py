@@ -1193,3 +1193,25 @@ def test_state_walk_in_chunks(ops, monkeypatch, form, d, keys):
         errors[chunks] = worst
     # (measured: 1.0 to 1.25 of the walk's error, 0.45 in the decay form)
     assert errors[True] <= 1.5 * errors[False], errors
+
+
+@pytest.mark.parametrize("T,n,pad,shift", [(300, 2056, 8, 0), (257, 2048, 0, 8), (600, 1000, 4, 0), (256, 2048, 8, 3), (65, 8200, 8, 16), (4, 7, 1, 0), (3, 64, 0, 0)])
+@pytest.mark.parametrize("name", ["relu2", "tanh"])
+def test_unary_in_wide_and_single_elements(ops, name, T, n, pad, shift):
+    """Rows that allow 16 bytes a thread and rows that do not (odd widths, strides and offsets): the same bits as the
+    function in 32-bit, rounded once (the square of relu), and as a contiguous copy of the rows gives (both); in place
+    too, infinities and what is no number included."""
+    fn = [k for k in ops.UNARY if ("tanh" in k) == (name == "tanh")][0]
+    wide = torch.randn(T, n + pad + shift, generator=torch.Generator().manual_seed(n)).to(torch.bfloat16).to(DEV)
+    wide[0, shift:shift + 3] = torch.tensor([float("inf"), float("-inf"), float("nan")], device=DEV)
+    x = wide[:, shift:shift + n]
+    out = torch.empty_like(wide)[:, shift:shift + n]
+    ops.unary(fn, x, out)
+    single = torch.empty(T, n + 1, dtype=torch.bfloat16, device=DEV)[:, 1:]      # never 16-byte rows
+    ops.unary(fn, x, single)
+    assert torch.equal(out.contiguous().view(torch.int16), single.contiguous().view(torch.int16))
+    if name != "tanh":
+        z = x.float()
+        assert torch.equal(out[:, 3:], (z.clamp(min=0) ** 2).to(torch.bfloat16)[:, 3:])
+    ops.unary(fn, x, x)
+    assert torch.equal(x.contiguous().view(torch.int16), single.contiguous().view(torch.int16))
