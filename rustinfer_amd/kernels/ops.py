@@ -1061,7 +1061,7 @@ def rotate_kv_write(q: torch.Tensor, k: Optional[torch.Tensor], v: Optional[torc
         int(bool(write_kv)), ctypes.c_float(unit_eps), _stream()))
 
 
-# bfloat16 attention without turned values, kept first positions and sigmoid weights, on pages of a multiple of 16, takes the
+# bfloat16 attention without kept first positions and sigmoid weights, on pages of a multiple of 16, takes the
 # kernels of attention_parts.hip (False: the ones below, for comparison)
 WINDOW_ATTENTION_PARTS = True
 WINDOW_ATTENTION_MFMA = True     # steps with prompt portions take the matrix-instruction kernel (False: the FMA one, for comparison)
