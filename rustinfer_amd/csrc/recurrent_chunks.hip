@@ -134,7 +134,7 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
                 const int idx = e * 64 + lane;
                 if (idx >= DK) continue;
                 const int ch = h * DK + idx;
-                const float u = k[e] * inv;
+                const float u = on ? k[e] * inv : 0.f;       // (with a unit_eps of 0 a token past the end would make it 0 * inf)
                 Um[tt * KP + idx] = u;
                 Bm[tt * KP + idx] = on ? sigmoid_(bf16_to_f32(a.al[t * a.al_stride + ch]) + a.ab[ch]) * u : 0.f;
                 Xm[tt * XP + idx] = on ? __expf(-a.decay_c * sigmoid_(bf16_to_f32(a.wl[t * a.wl_stride + ch]) + a.w0[ch])) : 1.f;

@@ -1195,6 +1195,40 @@ def test_state_walk_in_chunks(ops, monkeypatch, form, d, keys):
     assert errors[True] <= 1.5 * errors[False], errors
 
 
+def _scan_step(form, d, H, q_lens, starts, seed=20, unit_eps=1e-6):
+    """(r, k, v, state, ctx, keywords) of ``linear_scan`` for a step of these rows."""
+    T, B = sum(q_lens), len(q_lens)
+    bf = lambda i: rnd(T, H * d, dtype=torch.bfloat16, seed=seed + i)  # noqa: E731
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    several = [b for b, n in enumerate(q_lens) if n > 1]
+    ctx = SimpleNamespace(cu_q=i32([0] + list(np.cumsum(q_lens))), q_start=i32(starts), state_slots=i32(list(range(B))), num_rows=B,
+                          max_q_len=max(q_lens), max_kv_len=max(s + n for s, n in zip(starts, q_lens)), host_q_lens=list(q_lens),
+                          portion_rows=i32(several + [-1] * (B - len(several))), num_portion=len(several), workspace=Workspace(torch.device(DEV)))
+    kw = dict(wl=bf(4), al=bf(5), w0=rnd(H * d, seed=seed + 6), ab=rnd(H * d, seed=seed + 7), unit_eps=unit_eps, decay_c=math.exp(-0.5)) \
+        if form == "delta" else dict(decay=torch.linspace(0.9, 0.999, H, device=DEV), silu_in=True)
+    return bf(1), bf(2), bf(3), rnd(B, H, d, d, seed=seed + 8), ctx, kw
+
+
+def _scan_both_ways(ops, monkeypatch, H, d, r, k, v, state0, ctx, kw):
+    """[(outputs, states)] of the walk and of the chunks."""
+    got = []
+    for chunks in (False, True):
+        monkeypatch.setattr(ops, "_scan_in_chunks", lambda *a: chunks)
+        state, out = state0.clone(), torch.full((r.shape[0], H * d), 7.0, device=DEV)
+        ops.linear_scan(r, k, v, state, out, ctx, H, d, d, **kw)
+        got.append((out, state))
+    return got
+
+
+@pytest.mark.parametrize("d", [64, 128])
+def test_state_walk_in_chunks_of_keys_without_an_epsilon(ops, monkeypatch, d):
+    """unit_eps = 0: the places past the end of a last chunk hold no key that could be divided by its length of zero."""
+    r, k, v, state, ctx, kw = _scan_step("delta", d, 2, [33, 64, 95], [0, 5, 70], unit_eps=0.0)
+    (out0, state0), (out1, state1) = _scan_both_ways(ops, monkeypatch, 2, d, r, k, v, state, ctx, kw)
+    for a, b in ((out1, out0), (state1, state0)):
+        assert a.isfinite().all() and (a - b).norm() <= 5e-7 * b.norm()
+
+
 @pytest.mark.parametrize("T,n,pad,shift", [(300, 2056, 8, 0), (257, 2048, 0, 8), (600, 1000, 4, 0), (256, 2048, 8, 3), (65, 8200, 8, 16), (4, 7, 1, 0), (3, 64, 0, 0)])
 @pytest.mark.parametrize("name", ["relu2", "tanh"])
 def test_unary_in_wide_and_single_elements(ops, name, T, n, pad, shift):
