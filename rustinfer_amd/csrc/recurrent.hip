@@ -64,7 +64,10 @@ struct ScanArgs {
     // the channel forms: al holds the decays' inputs ([T][>= H dk], or [T][>= H] for a decay a head) in the gates'
     // dtype; ab their bias; w0 = A [H] where the form has one; decay_c = 1 / tau; skip [H] or null
     const float* skip;
-    int most = 0;        // rows of more tokens than this are left alone (0: none are)
+    // rows of more tokens than `most` (0: none) have had their first from[(row H + head) from_cols] done by another kernel
+    int most = 0;
+    const int* from = nullptr;
+    int from_cols = 0;
 };
 
 __device__ __forceinline__ float ld_gate(const void* p, size_t at, int is_bf16) {
@@ -131,14 +134,20 @@ __global__ __launch_bounds__(NW * 64) void linear_scan_kernel(const ScanArgs a) 
     const int CW = 64 / P, CPB = NW * CW;
     const int BUF = NA * SC_CH * DKP + SC_CH * CPB;    // floats of one of the two stretch buffers
     const int b = blockIdx.z, h = blockIdx.y;
-    const int t_lo = a.cu_q[b], n = a.cu_q[b + 1] - t_lo;
-    if (n <= 0 || (a.most > 0 && n > a.most)) return;  // a row without tokens (padding of a captured shape), or another kernel's
+    const int row_lo = a.cu_q[b], row_n = a.cu_q[b + 1] - row_lo;
+    if (row_n <= 0) return;                            // a row without tokens (padding of a captured shape)
+    int done = 0;                                      // tokens that another kernel has walked
+    if (a.most > 0 && row_n > a.most) {
+        done = min(max(a.from[((size_t)b * H + h) * a.from_cols], 0), row_n);
+        if (done == row_n) return;
+    }
+    const int t_lo = row_lo + done, n = row_n - done;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int pl = lane % P, cl = lane / P;            // the P lanes of a column are neighbours
     const int jc = wave * CW + cl, j = blockIdx.x * CPB + jc;
     const bool col_ok = j < dv;
     float* Sg = a.state + ((size_t)a.slots[b] * H + h) * (size_t)dk * dv;
-    const bool fresh = a.q_start[b] == 0;              // a request's first tokens start from nothing
+    const bool fresh = a.q_start[b] + done == 0;       // a request's first tokens start from nothing
     float S[R];
 #pragma unroll
     for (int ii = 0; ii < R; ++ii) {
@@ -158,7 +167,7 @@ __global__ __launch_bounds__(NW * 64) void linear_scan_kernel(const ScanArgs a) 
     // ROT: the rotation partners of r and k (feature idx +- rot/2), asked for with them
     float part_r[ROT ? TPW : 1][SC_EPL], part_k[ROT ? TPW : 1][SC_EPL];
     const int rot_half = ROT ? a.rot >> 1 : 0;
-    const int pos0 = ROT ? a.q_start[b] : 0;
+    const int pos0 = ROT ? a.q_start[b] + done : 0;
     auto ask = [&](int c0) {
         const int nc = min(SC_CH, n - c0);
 #pragma unroll
@@ -448,8 +457,8 @@ int launch_scan(const ScanArgs& a, int num_rows, hipStream_t stream) {
 // The walk for the tokens of a step.  r, k [T, >= H dk], v [T, >= H dv] are columns of the
 // projections (any row stride), in `dtype`; wl, al, w0, ab go with the delta form (delta != 0),
 // decay [H] with the decay form.  state [slots][H][dk][dv] and out [T][out_stride >= H dv] are
-// 32-bit.  A row whose q_start is 0 starts from a state of zeros (its slot is overwritten).  most > 0: rows of more
-// tokens than that are left alone (ri_linear_scan_chunks takes them).
+// 32-bit.  A row whose q_start is 0 starts from a state of zeros (its slot is overwritten).  most > 0: of rows of more
+// tokens than that the first from[(row H + head) from_cols] tokens are done (ri_linear_scan_chunks).
 extern "C" int ri_linear_scan(
         const void* r, int r_stride, const void* k, int k_stride, const void* v, int v_stride,
         const void* wl, int wl_stride, const void* al, int al_stride, int dtype,
@@ -457,7 +466,8 @@ extern "C" int ri_linear_scan(
         float unit_eps, float decay_c, float* state, int num_slots, float* out, int out_stride,
         const int* cu_q, const int* q_start, const int* slots, int num_rows, int T,
         int H, int dk, int dv, const float* rot_cos, const float* rot_sin, int rot, int rot_rows, int max_position,
-        float k_scale, int most, hipStream_t stream) {
+        float k_scale, int most, const int* from, int from_cols, hipStream_t stream) {
+    RI_REQUIRE(most <= 0 || (from && from_cols > 0), "ri_linear_scan: rows of more than %d tokens need their first tokens", most);
     RI_REQUIRE(H > 0 && dk > 0 && dv > 0 && dk <= 256, "ri_linear_scan: bad sizes H=%d dk=%d dv=%d (dk <= 256)", H, dk, dv);
     RI_REQUIRE(num_rows >= 0 && T >= 0 && num_slots > 0, "ri_linear_scan: bad counts");
     RI_REQUIRE(r_stride >= H * dk && k_stride >= H * dk && v_stride >= H * dv && out_stride >= H * dv,
@@ -481,7 +491,8 @@ extern "C" int ri_linear_scan(
     a.cu_q = cu_q; a.q_start = q_start; a.slots = slots;
     a.H = H; a.dk = dk; a.dv = dv; a.P = P; a.silu_in = silu_in; a.unit_eps = unit_eps; a.decay_c = decay_c;
     a.rot_cos = rot_cos; a.rot_sin = rot_sin; a.rot = rot_cos ? rot : 0; a.k_scale = k_scale;
-    a.gate_bf16 = 0; a.kv_group = 1; a.q_scale = 1.f; a.skip = nullptr; a.decay_bf16 = 0; a.most = most;
+    a.gate_bf16 = 0; a.kv_group = 1; a.q_scale = 1.f; a.skip = nullptr; a.decay_bf16 = 0;
+    a.most = most; a.from = from; a.from_cols = from_cols;
     int rc;
 #define RI_SCAN(TT, DD) (R == 8 ? launch_scan<TT, DD, 8>(a, num_rows, stream) : launch_scan<TT, DD, 16>(a, num_rows, stream))
     if (dtype == RI_F32) rc = delta ? RI_SCAN(float, true) : RI_SCAN(float, false);

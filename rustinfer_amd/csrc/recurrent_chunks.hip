@@ -17,9 +17,13 @@
 // W only ever divides what is multiplied by a later W: a ratio W_t / W_s is as exact as the product of the decays
 // between, however small both are.  That needs W_C > 0: the caller takes this form where the design bounds the
 // decays (w >= exp(-decay_c)).  A substitution and not a product of powers of L: where keys repeat, those grow
-// beyond what cancels.  A token whose vectors are not finite spoils its chunk from the first token on.  Sums are in chains of 8 or 16 products, and the
+// beyond what cancels.  Sums are in chains of 8 or 16 products, and the
 // delta form's W and its four C x C matrices in 64 bits: with single chains the outputs are two to three times
 // further from 64-bit arithmetic than the walk's, so they are as close (1.0e-7; the decay form 1.2e-7 against 2.6e-7).
+//
+// What holds the tokens of a chunk apart is zeros, which a value that is not finite passes.  A chunk and head whose operators
+// are not finite (a token's vectors were not, or k / W_t left the range of 32 bits) is therefore only marked; the states
+// stop in front of it, and the walk does that head of that row from there on, so that every token gets what the walk gives.
 //
 // 2,048 tokens of 32 heads of 64, us a layer: delta form 1205 -> 232 (137 the operators, 95 the states), decay form
 // 768 -> 100; 24 heads of 128: 1741 -> 559, 1011 -> 174.  The operators are bound by the steps of a block following
@@ -49,7 +53,8 @@ struct ChunkArgs {
     const float *rot_cos, *rot_sin;
     int rot;
     float k_scale;
-    float* ws;                          // [row][chunk of the segment][head][UNIT]
+    float* ws;                          // [row][chunk of the segment][head][Unit::SIZE]
+    int* from;                          // [row][head][dv / 16]: the token that the walk goes on from
     int c0, seg;                        // the segment's first chunk of every row, its chunks
 };
 
@@ -57,11 +62,13 @@ __device__ __forceinline__ float sigmoid_(float z) { return __fdividef(1.f, 1.f 
 __device__ __forceinline__ float silu_(float z) { return __fdividef(z, 1.f + __expf(-z)); }
 
 // Floats of a chunk and head in the workspace: R' [2 tiles of 16 tokens][dk / 16][64][4], S_add [dv / 16][dk / 16][64][4]
-// and, in the delta form, M [dk / 16][dk / 16][64][4]: each in the order the lanes of chunk_states_kernel read it.
+// and, in the delta form, M [dk / 16][dk / 16][64][4]: each in the order the lanes of chunk_states_kernel read it; BAD: not
+// zero where something in it is not finite.
 template <int DK, int DV, bool DELTA>
 struct Unit {
-    static constexpr int R = 0, S = C * DK, M = S + DK * DV, SIZE = M + (DELTA ? DK * DK : 0);
+    static constexpr int R = 0, S = C * DK, M = S + DK * DV, BAD = M + (DELTA ? DK * DK : 0), SIZE = BAD + 4;
 };
+__device__ __forceinline__ bool endless(float x) { return !(fabsf(x) < __builtin_inff()); }
 
 // d to the power n (0 <= n <= C), rounded once
 __device__ __forceinline__ float power(float d, int n) {
@@ -301,6 +308,11 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
         for (int e = 0; e < 16; ++e) x[e] = -x[e];
         return x;
     };
+    bool bad = false;
+    const auto check = [&](const f32x16_t& x) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) bad |= endless(x[e]);
+    };
     // R' transposed (rows: channels, columns: tokens), so that a lane's four consecutive rows are one store
     for (int it = wave; it < TK; it += 4) {
         f32x16_t acc;
@@ -310,6 +322,7 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
             acc[e] = Rm[l32 * KP + ch] * (DELTA ? 1.f : Wc[l32 + 1]);
         }
         if (DELTA) acc = minus(product(minus(acc), across(Xm, XP, it * 32), lower(Ab)));
+        check(acc);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int kt = it * 2 + (q >> 1), g = (q & 1) * 2 + hi;
@@ -322,6 +335,7 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
         f32x16_t acc = {};
         if (DELTA) acc = minus(product(acc, lower(Ab), across(Xm, XP, DK + ct * 32)));
         acc = product(acc, lower(Ak), across(Vm, VP, ct * 32));
+        check(acc);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int t = 8 * (e >> 2) + 4 * hi + (e & 3);
@@ -342,6 +356,7 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
                 return Km[t * KP + it * 32 + l32] * Wc[max(nc - 1 - t, 0)];      // (k is zero past the end)
             }, across(Vm, VP, ct * 32));
         }
+        check(acc);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const int kt = it * 2 + (q >> 1), g = (q & 1) * 2 + hi, cb = ct * 2 + (l32 >> 4);
@@ -359,6 +374,7 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
 #pragma unroll
             for (int e = 0; e < 16; ++e)
                 if (jt == it && 8 * (e >> 2) + 4 * hi + (e & 3) == l32) acc[e] += wc;
+            check(acc);
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
                 const int kt = jt * 2 + (q >> 1), g = (q & 1) * 2 + hi, rt = it * 2 + (l32 >> 4);
@@ -367,6 +383,8 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
             }
         }
     }
+    const int any = __syncthreads_or(bad);
+    if (tid == 0) reinterpret_cast<int*>(unit)[U::BAD] = any;
 }
 
 // The state through the segment's chunks, 16 of its columns a block.  A wave owns 32 rows (two tiles of 16); with
@@ -380,8 +398,14 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
     const int b = blockIdx.z, h = blockIdx.y, cb = blockIdx.x;
     const int t_lo = a.cu_q[b], n = a.cu_q[b + 1] - t_lo;
     if (n < a.min_tokens || a.c0 * C >= n) return;
-    const int chunks = min(a.seg, (n + C - 1) / C - a.c0);
+    int* const from = a.from + ((size_t)b * a.H + h) * (DV / 16) + cb;       // (this block's own, the same in all of a head's)
+    if (a.c0 > 0 && *from < a.c0 * C) return;          // the walk takes the row over before this segment
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
+    const int all = min(a.seg, (n + C - 1) / C - a.c0);          // at most 64
+    const float* units = a.ws + ((size_t)b * a.seg * a.H + h) * U::SIZE;
+    const unsigned long long bads = __ballot(lane < all && reinterpret_cast<const int*>(units + (size_t)lane * a.H * U::SIZE)[U::BAD] != 0);
+    const int chunks = bads ? __ffsll(bads) - 1 : all;
+    if (threadIdx.x == 0) *from = (a.c0 + chunks) * C;
     __shared__ __align__(16) f32x4_t St[2][NA][64];
     float* Sg = a.state + ((size_t)a.slots[b] * a.H + h) * (size_t)DK * DV + cb * 16 + col;
     const bool fresh = a.c0 == 0 && a.q_start[b] == 0;
@@ -395,7 +419,7 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
     const float d = DELTA ? 0.f : a.decay[h];
     const float d_chunk = DELTA ? 0.f : power(d, C);
     auto ask = [&](int c, Ops& x) {
-        const f32x4_t* unit = reinterpret_cast<const f32x4_t*>(a.ws + (((size_t)b * a.seg + c) * a.H + h) * U::SIZE);
+        const f32x4_t* unit = reinterpret_cast<const f32x4_t*>(units + (size_t)c * a.H * U::SIZE);
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             x.add[q] = unit[U::S / 4 + (cb * NA + wave * 2 + q) * 64 + lane];
@@ -453,7 +477,7 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
     };
     static_assert(NW >= 2, "two waves make the outputs");
     Ops x0, x1;
-    ask(0, x0);
+    if (chunks > 0) ask(0, x0);
     for (int c = 0; c < chunks; c += 2) {
         if (c + 1 < chunks) ask(c + 1, x1);
         step(c, x0);
@@ -510,13 +534,26 @@ extern "C" int ri_linear_scan_chunks_supported(int delta, int dk, int dv, float 
     return (dk == 64 || dk == 128) && dv == dk;
 }
 
-// Floats of workspace for steps of up to num_rows rows of at most max_tokens tokens.
-extern "C" size_t ri_linear_scan_chunks_workspace(int delta, int num_rows, int max_tokens, int H, int dk, int dv) {
-    return (size_t)num_rows * segment(num_rows, max_tokens) * H * ((size_t)C * dk + (size_t)dk * dv + (delta ? (size_t)dk * dk : 0));
+static size_t unit_floats(int delta, int num_rows, int max_tokens, int H, int dk, int dv) {
+    return (size_t)num_rows * segment(num_rows, max_tokens) * H * ((size_t)C * dk + (size_t)dk * dv + (delta ? (size_t)dk * dk : 0) + 4);
 }
 
-// ri_linear_scan for the rows of at least min_tokens tokens (max_tokens at most, or an upper bound); the others are
-// left alone.  bfloat16 projections.
+// Floats of workspace for steps of up to num_rows rows of at most max_tokens tokens.
+extern "C" size_t ri_linear_scan_chunks_workspace(int delta, int num_rows, int max_tokens, int H, int dk, int dv) {
+    return unit_floats(delta, num_rows, max_tokens, H, dk, dv) + (size_t)num_rows * H * (dv / 16);
+}
+
+extern "C" int ri_linear_scan(
+        const void* r, int r_stride, const void* k, int k_stride, const void* v, int v_stride,
+        const void* wl, int wl_stride, const void* al, int al_stride, int dtype,
+        const float* w0, const float* ab, const float* decay, int delta, int silu_in,
+        float unit_eps, float decay_c, float* state, int num_slots, float* out, int out_stride,
+        const int* cu_q, const int* q_start, const int* slots, int num_rows, int T,
+        int H, int dk, int dv, const float* rot_cos, const float* rot_sin, int rot, int rot_rows, int max_position,
+        float k_scale, int most, const int* from, int from_cols, hipStream_t stream);
+
+// ri_linear_scan with the rows of at least min_tokens tokens (max_tokens at most, or an upper bound) in chunks; the walk
+// does the others, and what the chunks leave to it.  bfloat16 projections.
 extern "C" int ri_linear_scan_chunks(
         const void* r, int r_stride, const void* k, int k_stride, const void* v, int v_stride,
         const void* wl, int wl_stride, const void* al, int al_stride,
@@ -526,7 +563,7 @@ extern "C" int ri_linear_scan_chunks(
         int H, int dk, int dv, const float* rot_cos, const float* rot_sin, int rot, int rot_rows, int max_position,
         float k_scale, int min_tokens, int max_tokens, float* ws, size_t ws_floats, hipStream_t stream) {
     RI_REQUIRE(H > 0 && ri_linear_scan_chunks_supported(delta, dk, dv, decay_c), "ri_linear_scan_chunks: does not take H=%d dk=%d dv=%d decay_c=%g", H, dk, dv, (double)decay_c);
-    RI_REQUIRE(num_rows >= 0 && T >= 0 && num_slots > 0 && min_tokens > 0, "ri_linear_scan_chunks: bad counts");
+    RI_REQUIRE(num_rows >= 0 && T >= 0 && num_slots > 0 && min_tokens > 1, "ri_linear_scan_chunks: bad counts");
     RI_REQUIRE(r_stride >= H * dk && k_stride >= H * dk && v_stride >= H * dv && out_stride >= H * dv, "ri_linear_scan_chunks: row strides too small");
     if (num_rows == 0 || T == 0 || max_tokens <= 0) return 0;
     RI_REQUIRE(r && k && v && state && out && cu_q && q_start && slots && ws, "ri_linear_scan_chunks: null pointer");
@@ -543,10 +580,13 @@ extern "C" int ri_linear_scan_chunks(
     a.cu_q = cu_q; a.q_start = q_start; a.slots = slots; a.H = H; a.silu_in = silu_in; a.min_tokens = min_tokens;
     a.unit_eps = unit_eps; a.decay_c = decay_c; a.rot_cos = rot_cos; a.rot_sin = rot_sin; a.rot = rot_cos ? rot : 0; a.k_scale = k_scale;
     a.ws = ws; a.c0 = 0; a.seg = segment(num_rows, max_tokens);
+    a.from = reinterpret_cast<int*>(ws + unit_floats(delta, num_rows, max_tokens, H, dk, dv));
     int rc;
     if (dk == 64) rc = delta ? launch_chunks<64, 64, true>(a, num_rows, max_tokens, stream) : launch_chunks<64, 64, false>(a, num_rows, max_tokens, stream);
     else rc = delta ? launch_chunks<128, 128, true>(a, num_rows, max_tokens, stream) : launch_chunks<128, 128, false>(a, num_rows, max_tokens, stream);
     if (rc) return rc;
     RI_LAUNCHED("ri_linear_scan_chunks");
-    return 0;
+    return ri_linear_scan(r, r_stride, k, k_stride, v, v_stride, wl, wl_stride, al, al_stride, RI_BF16, w0, ab, decay, delta, silu_in,
+                          unit_eps, decay_c, state, num_slots, out, out_stride, cu_q, q_start, slots, num_rows, T, H, dk, dv,
+                          rot_cos, rot_sin, rot, rot_rows, max_position, k_scale, min_tokens - 1, a.from, dv / 16, stream);
 }

@@ -1225,22 +1225,18 @@ def linear_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
             ctypes.c_float(decay_c), _ptr(state), state.shape[0], _ptr(out), out.stride(0),
             _ptr(ctx.cu_q), _ptr(ctx.q_start), _ptr(ctx.state_slots), ctx.num_rows, T, H, dk, dv,
             rcos, rsin, rot, rrows, max(int(ctx.max_kv_len) - 1, 0), ctypes.c_float(k_scale))
-    most = 0
     longest, workspace = int(ctx.max_q_len), getattr(ctx, "workspace", None)
     portions = int(getattr(ctx, "num_portion", 0) or ctx.num_rows)
     if workspace is not None and r.dtype == torch.bfloat16 and _scan_in_chunks(delta, dk, portions, longest) \
             and lib.ri_linear_scan_chunks_supported(int(delta), dk, dv, ctypes.c_float(decay_c)):
-        # prompts: chunks of tokens on the matrix instructions; the walk takes the rows of fewer tokens, if there are any.
-        # (32-bit projections stay with the walk, whose bits do not depend on how a request was cut into steps)
+        # prompts: chunks of tokens on the matrix instructions; the walk takes the rows of fewer tokens, and heads with
+        # something not finite.  (32-bit projections stay with the walk, whose bits do not depend on how a request was cut into steps)
         lib.ri_linear_scan_chunks_workspace.restype = ctypes.c_size_t
         need = lib.ri_linear_scan_chunks_workspace(int(delta), ctx.num_rows, longest, H, dk, dv)
         ws = workspace.get("scan.chunks", need, 1, torch.float32)
         _check(lib.ri_linear_scan_chunks(*inputs, *form, SCAN_CHUNK_TOKENS, longest, _ptr(ws), ctypes.c_size_t(ws.numel()), _stream()))
-        most = SCAN_CHUNK_TOKENS - 1
-        host_q = getattr(ctx, "host_q_lens", None)
-        if host_q is not None and min(host_q) > most:
-            return
-    _check(lib.ri_linear_scan(*inputs, _dt(r), *form, most, _stream()))
+        return
+    _check(lib.ri_linear_scan(*inputs, _dt(r), *form, 0, None, 0, _stream()))
 
 
 def gated_group_norm(o: torch.Tensor, weight: Optional[torch.Tensor], gate: Optional[torch.Tensor], out: torch.Tensor,

@@ -1229,6 +1229,31 @@ def test_state_walk_in_chunks_of_keys_without_an_epsilon(ops, monkeypatch, d):
         assert a.isfinite().all() and (a - b).norm() <= 5e-7 * b.norm()
 
 
+@pytest.mark.parametrize("form,d,what,value,at", [
+    ("delta", 64, "v", "inf", 705), ("delta", 64, "k", "nan", 40), ("delta", 128, "k", 1e37, 40), ("delta", 64, "r", "-inf", 50), ("delta", 64, "wl", "nan", 45),
+    ("delta", 128, "al", "nan", 690), ("delta", 64, "v", "nan", 0), ("decay", 64, "v", "-inf", 44), ("decay", 64, "k", "inf", 700), ("decay", 128, "r", "nan", 63)])
+def test_state_walk_in_chunks_of_tokens_that_are_not_finite(ops, monkeypatch, form, d, what, value, at):
+    """One number of one token of the first of three rows (of 22 chunks a pass its first or second): the tokens before it, the
+    other head and the other rows stay what they are, the rest is what the walk makes of it; a key so large that its
+    quotient by a chunk's decays has no 32-bit value stays one that the walk can take."""
+    H, q_lens = 2, [720, 33, 64]
+    r, k, v, state, ctx, kw = _scan_step(form, d, H, q_lens, [0, 5, 70], seed=40)
+    if value == 1e37:
+        v = v * 1e-3
+        kw["w0"] = torch.full_like(kw["w0"], 12.0)                 # decays at their bound: 1e37 / w^32 is beyond 32 bits
+    {"r": r, "k": k, "v": v, "wl": kw.get("wl"), "al": kw.get("al")}[what][at, d + 3] = float(value)     # head 1
+    (out0, state0), (out1, state1) = _scan_both_ways(ops, monkeypatch, H, d, r, k, v, state, ctx, kw)
+    assert torch.equal(out0.isfinite(), out1.isfinite()) and torch.equal(state0.isfinite(), state1.isfinite())
+    assert out0[:at].isfinite().all() and (value == 1e37 or not out0[at, d:].isfinite().all())
+    lo = 0
+    for b, n in enumerate(q_lens):
+        for h in range(H):
+            for x, y in ((out1[lo:lo + n, h * d:(h + 1) * d], out0[lo:lo + n, h * d:(h + 1) * d]), (state1[b, h], state0[b, h])):
+                x, y = (torch.where(y.isfinite(), t, 0.0).double() for t in (x, y))
+                assert (x - y).norm() <= 5e-7 * y.norm(), (b, h)
+        lo += n
+
+
 @pytest.mark.parametrize("T,n,pad,shift", [(300, 2056, 8, 0), (257, 2048, 0, 8), (600, 1000, 4, 0), (256, 2048, 8, 3), (65, 8200, 8, 16), (4, 7, 1, 0), (3, 64, 0, 0)])
 @pytest.mark.parametrize("name", ["relu2", "tanh"])
 def test_unary_in_wide_and_single_elements(ops, name, T, n, pad, shift):
