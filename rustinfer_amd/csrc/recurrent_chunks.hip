@@ -1,15 +1,15 @@
-// The state walk of recurrent.hip for prompts, 32 tokens at a time on the 32-bit matrix instructions:
+// The state walk of recurrent.hip for prompts, 32 tokens at a time on the matrix instructions:
 //
 //   delta form:  S_t = diag(w_t) S_(t-1) - b_t (u_t^T S_(t-1)) + k_t v_t^T,   o_t = S_t^T r_t
 //   decay form:  S_t = d S_(t-1) + k_t v_t^T,                                 o_t = S_t^T r_t
 //
 // per head, S of [dk][dv], b = a * u.  Token by token that is a chain of thousands of short steps on a quarter of
 // the chip's SIMDs.  Within a chunk of C tokens, with W_t = w_1 * .. * w_t (per key channel) and
-//   U_t = u_t W_(t-1),   R_t = r_t W_t,   K_t = k_t / W_t,   B_t = b_t / W_t,
-// the tokens' d_t = u_t^T S_(t-1) solve (I + L) D = U S_0 + N V with L, N the strictly lower parts of U B^T and U K^T,
-// so D = X S_0 + Y V' with X, Y from one substitution on [U | N V], and
-//   o   = (R - A_b X) S_0 + (A_k V - A_b Y),      A_k, A_b the lower parts of R K^T, R B^T
-//   S_C = (diag(W_C) - B~^T X) S_0 + (K~^T V - B~^T Y),      K~ = K W_C, B~ = B W_C.
+//   U_t = u_t W_(t-1),   R_t = r_t W_t,   K_t = k_t / W_t,   B_t = b_t / W_t,   K~ = K W_C,   B~ = B W_C,
+// the tokens' d_t = u_t^T S_(t-1) solve (I + L) D = U S_0 + N V with L, N the strictly lower parts of U B^T and U K^T.
+// With T = (I + L)^-1, the lower parts A_k, A_b of R K^T, R B^T, and P = A_b T, G = B~^T T (dk x C),
+//   o   = (R - P U) S_0 + (A_k - P N) V,
+//   S_C = (diag(W_C) - G U) S_0 + (K~^T - G N) V.
 // Everything but S_0 is the chunk's own: `chunk_operators_kernel` makes it for all chunks at once (a block a
 // chunk and head), and `chunk_states_kernel` passes the state through the chunks: one product of dk x dk and one of
 // C x dk against 16 of its columns a block.  The decay form has powers of d in place of the operators.
@@ -17,28 +17,33 @@
 // W only ever divides what is multiplied by a later W: a ratio W_t / W_s is as exact as the product of the decays
 // between, however small both are.  That needs W_C > 0: the caller takes this form where the design bounds the
 // decays (w >= exp(-decay_c)).  A substitution and not a product of powers of L: where keys repeat, those grow
-// beyond what cancels.  Sums are in chains of 8 or 16 products, and the
-// delta form's W and its four C x C matrices in 64 bits: with single chains the outputs are two to three times
-// further from 64-bit arithmetic than the walk's, so they are as close (1.0e-7; the decay form 1.2e-7 against 2.6e-7).
+// beyond what cancels.
+//
+// The walk rounds a state once a token, in every element; a chunk has several products between two roundings of the
+// state, and where keys share a direction those cancel.  With sums in 32 bits its states were up to 2.4 times further
+// from 64-bit arithmetic than the walk's.  So all that a chunk computes from its scaled vectors (32 bits each) is 64-bit,
+// on v_mfma_f64_16x16x4_f64, rounded where it is stored for the states; M is stored without W_C, so that what is rounded
+// is only what the chunk changes; and the new state is rounded once.  Errors against 64 bits, of the walk's, outputs / states,
+// rows of 32 to 300 tokens: random keys 0.65 / 0.90, keys around one direction 0.83 / 0.87, one repeated key 0.98 / 0.99, decay
+// form 0.69 to 0.76 / 0.34 to 0.39.  (A decay as fast as 0.5 a token behind a chunk that is not whole: states up to 1.2 of
+// half a unit in the last place, outputs 0.4.)
 //
 // What holds the tokens of a chunk apart is zeros, which a value that is not finite passes.  A chunk and head whose operators
 // are not finite (a token's vectors were not, or k / W_t left the range of 32 bits) is therefore only marked; the states
 // stop in front of it, and the walk does that head of that row from there on, so that every token gets what the walk gives.
 //
-// 2,048 tokens of 32 heads of 64, us a layer: delta form 1205 -> 232 (137 the operators, 95 the states), decay form
-// 768 -> 100; 24 heads of 128: 1741 -> 559, 1011 -> 174.  The operators are bound by the steps of a block following
-// each other (matrix instructions a quarter of the time, two blocks a compute unit), the states by the chain of chunks.
+// 2,048 tokens of 32 heads of 64, us a layer: delta form 1174 -> 260, decay form 789 -> 109; 24 heads of 128: 1692 -> 617, 977 ->
+// 188 (with 32-bit sums 223, 96, 551 and 173).  The operators are bound by the steps of a block following each other (two
+// blocks a compute unit), the states by the chain of chunks.
 #include "common.h"
 #include <mutex>
 
 namespace {
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef float f32x16_t __attribute__((ext_vector_type(16)));
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
 constexpr int C = 32;                   // tokens a chunk
-constexpr int CP = C + 4;               // floats a row of a C x C matrix takes in LDS
 
 struct ChunkArgs {
     const bf16_t *r, *k, *v, *wl, *al;
@@ -62,58 +67,76 @@ __device__ __forceinline__ float sigmoid_(float z) { return __fdividef(1.f, 1.f 
 __device__ __forceinline__ float silu_(float z) { return __fdividef(z, 1.f + __expf(-z)); }
 
 // Floats of a chunk and head in the workspace: R' [2 tiles of 16 tokens][dk / 16][64][4], S_add [dv / 16][dk / 16][64][4]
-// and, in the delta form, M [dk / 16][dk / 16][64][4]: each in the order the lanes of chunk_states_kernel read it; BAD: not
-// zero where something in it is not finite.
+// and, in the delta form, M [dk / 16][dk / 16][64][4] without its diagonal part, W_C [dk]: each in the order the lanes of
+// chunk_states_kernel read it; BAD: not zero where something in it is not finite.
 template <int DK, int DV, bool DELTA>
 struct Unit {
-    static constexpr int R = 0, S = C * DK, M = S + DK * DV, BAD = M + (DELTA ? DK * DK : 0), SIZE = BAD + 4;
+    static constexpr int R = 0, S = C * DK, M = S + DK * DV, W = M + (DELTA ? DK * DK : 0), BAD = W + (DELTA ? DK : 0), SIZE = BAD + 4;
 };
 __device__ __forceinline__ bool endless(float x) { return !(fabsf(x) < __builtin_inff()); }
 
-// d to the power n (0 <= n <= C), rounded once
-__device__ __forceinline__ float power(float d, int n) {
+// d to the power n (0 <= n <= C)
+__device__ __forceinline__ double power(float d, int n) {
     double p = 1.0, q = (double)d;
     for (int m = n; m > 0; m >>= 1) {
         if (m & 1) p *= q;
         q *= q;
     }
-    return (float)p;
+    return p;
 }
 
-// acc += A B over the C tokens of a chunk, two a matrix instruction: a lane's operands are rows / columns l % 32,
-// token 2 s + l / 32.  Four chains of sums: the instruction adds in order, and one chain of 32 or 64 products is
-// two to three times further from the exact sum than the walk's eight-row sums are.
-template <typename FA, typename FB>
-__device__ __forceinline__ f32x16_t product(f32x16_t acc, FA a, FB b) {
-    f32x16_t p[4] = {};
+// acc += A B over the tokens 4 S0 .. 4 S1 of a chunk, in 64 bits (v_mfma_f64_16x16x4_f64): lane 16 g + i brings row or column i
+// and token 4 s + g, and has results (4 e + g, i) in element e.  Fed with row turned(i) in the place of i, it has rows
+// 4 g + e: four consecutive ones.
+template <int S0, int S1, typename FA, typename FB>
+__device__ __forceinline__ f64x4_t product(f64x4_t acc, int g, FA a, FB b) {
 #pragma unroll
-    for (int s = 0; s < C / 2; ++s) p[s & 3] = __builtin_amdgcn_mfma_f32_32x32x2f32(a(s), b(s), p[s & 3], 0, 0, 0);
-    return acc + ((p[0] + p[1]) + (p[2] + p[3]));
+    for (int s = S0; s < S1; ++s) acc = __builtin_amdgcn_mfma_f64_16x16x4f64(a(4 * s + g), b(4 * s + g), acc, 0, 0, 0);
+    return acc;
 }
-// rows of a 32 x 32 result in element e of a lane: 8 (e / 4) + 4 (l / 32) + e % 4; column l % 32
+__device__ __forceinline__ int turned(int i) { return 4 * (i & 3) + (i >> 2); }
+
+// Two lower triangles of C x C share one array of C x (C + 1): (t, s) of the first is at t (C + 1) + s, of the second at
+// s (C + 1) + t + 1.
+constexpr int TP = C + 1;
+__device__ __forceinline__ double first_of(const double* m, int t, int s) { const double x = m[t * TP + s]; return s <= t ? x : 0.0; }
+__device__ __forceinline__ double second_of(const double* m, int t, int s) { const double x = m[s * TP + t + 1]; return s <= t ? x : 0.0; }
+__device__ __forceinline__ double second_strictly(const double* m, int t, int s) { const double x = m[s * TP + t + 1]; return s < t ? x : 0.0; }
+
+// LDS of a block, in floats
+template <int DK, int DV, bool DELTA>
+struct Lds {
+    static constexpr int KP = DK + 4, VP = DV + 4, HP = DK + 2;
+    static constexpr int R = 0, U = R + C * KP, V = U + (DELTA ? C * KP : 0), K = V + C * VP, B = K + C * KP,
+                         G = B + (DELTA ? C * KP : 0), A = G + (DELTA ? 2 * C * HP : 0), T = A + 2 * C * TP,
+                         W = T + (DELTA ? 2 * C * TP : 0), SIZE = W + 2 * (DELTA ? DK : C + 1);
+    static_assert(G % 2 == 0 && A % 2 == 0 && T % 2 == 0 && W % 2 == 0, "64-bit numbers lie at even places");
+};
 
 template <int DK, int DV, bool DELTA>
 __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a) {
-    constexpr int KP = DK + 4, VP = DV + 4, NX = DELTA ? DK + DV : 0, XP = NX + 4;
+    using At = Lds<DK, DV, DELTA>;
+    constexpr int KP = At::KP, VP = At::VP, HP = At::HP;
     constexpr int EK = DK / 64 > 0 ? DK / 64 : 1, TK = DK / 32, TV = DV / 32;
     using U = Unit<DK, DV, DELTA>;
     const int b = blockIdx.z, h = blockIdx.y, cs = blockIdx.x, c = a.c0 + cs;
     const int t_lo = a.cu_q[b], n = a.cu_q[b + 1] - t_lo;
     if (n < a.min_tokens || c * C >= n) return;
     const int nc = min(C, n - c * C), t0 = t_lo + c * C;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hi = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), i16 = lane & 15, g = lane >> 4;
     extern __shared__ __align__(16) float lds[];
-    float* Rm = lds;                          // [C][KP]: r, then R
-    float* Km = Rm + C * KP;                  // k, then K
-    float* Vm = Km + C * KP;                  // [C][VP]
-    float* Ak = Vm + C * VP;                  // [C][CP]
-    float* Wc = Ak + C * CP;                  // [DK]: W_C; the decay form: powers of d, 0 .. C
-    float* Um = Wc + (DK > C + 4 ? DK : C + 4);       // delta: u, then U
-    float* Bm = Um + C * KP;                  // b, then B
-    float* Lm = Bm + C * KP;                  // [C][CP]
-    float* Nm = Lm + C * CP;
-    float* Ab = Nm + C * CP;
-    float* Xm = Ab + C * CP;                  // [C][XP]: w first, then [U | N V], then [X | Y]
+    float* Rm = lds + At::R;                  // [C][KP]: r, then R
+    float* Um = lds + At::U;                  // delta: u, then U
+    float* Vm = lds + At::V;                  // [C][VP]
+    float* Km = lds + At::K;                  // k, then K
+    float* Bm = lds + At::B;                  // delta: b, then B
+    float* Ws = lds + At::G;                  // delta: [C][DK] of w, until W is made
+    double* Gs = reinterpret_cast<double*>(lds + At::G);       // delta: [C][HP] of G
+    double* Hs = reinterpret_cast<double*>(lds + At::K);       // delta: [C][HP] of H, in the place of K and B
+    double* A2 = reinterpret_cast<double*>(lds + At::A);       // A_k, then E; delta: and A_b, then P
+    double* T2 = reinterpret_cast<double*>(lds + At::T);       // delta: L, then T; and N
+    double* Wc = reinterpret_cast<double*>(lds + At::W);       // delta: [DK] of W_C; else powers of d, 0 .. C
+    static_assert(2 * HP <= 2 * KP, "H fits where K and B were");
     float* unit = a.ws + (((size_t)b * a.seg + cs) * a.H + h) * U::SIZE;
     const float d = DELTA ? 0.f : a.decay[h];
 
@@ -144,7 +167,7 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
                 const float u = on ? k[e] * inv : 0.f;       // (with a unit_eps of 0 a token past the end would make it 0 * inf)
                 Um[tt * KP + idx] = u;
                 Bm[tt * KP + idx] = on ? sigmoid_(bf16_to_f32(a.al[t * a.al_stride + ch]) + a.ab[ch]) * u : 0.f;
-                Xm[tt * XP + idx] = on ? __expf(-a.decay_c * sigmoid_(bf16_to_f32(a.wl[t * a.wl_stride + ch]) + a.w0[ch])) : 1.f;
+                Ws[tt * DK + idx] = on ? __expf(-a.decay_c * sigmoid_(bf16_to_f32(a.wl[t * a.wl_stride + ch]) + a.w0[ch])) : 1.f;
             }
         } else {
             if (a.silu_in) {
@@ -182,205 +205,240 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
     if (!DELTA && tid <= C) Wc[tid] = power(d, tid);
     __syncthreads();
     if (DELTA) {
-        // W up to each token: a wave has 8 tokens and multiplies those before them again; the products first, in
-        // registers, because the rows of w are where [U | N V] goes
+        // W up to each token: a wave has 8 tokens and multiplies those before them again
         constexpr int PER = C / 4;
-        double wt[EK][PER + 1];                // W before the wave's first token, then after each (64-bit: each factor is rounded once)
-#pragma unroll
-        for (int e = 0; e < EK; ++e) {
-            const int idx = min(e * 64 + lane, DK - 1);
-            double p = 1.0;
-            for (int tt = 0; tt < wave * PER; ++tt) p *= (double)Xm[tt * XP + idx];
-            wt[e][0] = p;
-#pragma unroll
-            for (int i = 0; i < PER; ++i) { p *= (double)Xm[(wave * PER + i) * XP + idx]; wt[e][i + 1] = p; }
-            if (wave == 3 && e * 64 + lane < DK) Wc[idx] = (float)p;
-        }
-        __syncthreads();
 #pragma unroll
         for (int e = 0; e < EK; ++e) {
             const int idx = e * 64 + lane;
             if (idx >= DK) continue;
+            double p = 1.0;
+            for (int tt = 0; tt < wave * PER; ++tt) p *= (double)Ws[tt * DK + idx];
 #pragma unroll
             for (int i = 0; i < PER; ++i) {
-                const int at = (wave * PER + i) * KP + idx;
-                const double inv = 1.0 / wt[e][i + 1];
-                const float U_ = (float)((double)Um[at] * wt[e][i]);
-                Um[at] = U_;
-                Xm[(wave * PER + i) * XP + idx] = U_;
-                Rm[at] = (float)((double)Rm[at] * wt[e][i + 1]);
+                const int tt = wave * PER + i, at = tt * KP + idx;
+                Um[at] = (float)((double)Um[at] * p);
+                p *= (double)Ws[tt * DK + idx];
+                const double inv = 1.0 / p;
+                Rm[at] = (float)((double)Rm[at] * p);
                 Km[at] = (float)((double)Km[at] * inv);
                 Bm[at] = (float)((double)Bm[at] * inv);
             }
+            if (wave == 3) Wc[idx] = p;
         }
         __syncthreads();
     }
-    // the four matrices of C x C: a wave each (the decay form: the first wave)
-    if (DELTA || wave == 0) {
+    // the matrices of C x C, without the tile above the diagonal.  16 bytes of a row a lane make four steps of the
+    // instruction.  Delta: a wave a matrix; else a wave a tile.
+    {
         const float* X = !DELTA || (wave & 1) ? Rm : Um;
         const float* Y = !DELTA || wave < 2 ? Km : Bm;
-        float* D = !DELTA ? Ak : (wave == 0 ? Nm : wave == 1 ? Ak : wave == 2 ? Lm : Ab);
-        const bool strict = DELTA && !(wave & 1);
-        if (DELTA) {
-            // in 64 bits (v_mfma_f64_16x16x4_f64: lane 16 g + i has row or column i and one of four k; 16 bytes of K a lane
-            // make four steps): what the substitution starts from decides how exact the chunk is
-            const int i16 = lane & 15, g = lane >> 4;
-            f64x4_t acc[2][2] = {};
+        double* D = !DELTA || (wave & 1) ? A2 : T2;
+        f64x4_t acc[3] = {};                                   // tiles (0, 0), (1, 0), (1, 1)
+        const int p0 = !DELTA && wave > 0, q0 = !DELTA && wave > 1;    // the decay form's tile
+        if (DELTA || wave < 3) {
 #pragma unroll 2
             for (int j = 0; j < DK / 16; ++j) {
                 float4 x[2], y[2];
 #pragma unroll
-                for (int q = 0; q < 2; ++q) {
-                    x[q] = *reinterpret_cast<const float4*>(X + (16 * q + i16) * KP + 16 * j + 4 * g);
-                    y[q] = *reinterpret_cast<const float4*>(Y + (16 * q + i16) * KP + 16 * j + 4 * g);
+                for (int q = 0; q < (DELTA ? 2 : 1); ++q) {
+                    x[q] = *reinterpret_cast<const float4*>(X + (16 * (q + p0) + i16) * KP + 16 * j + 4 * g);
+                    y[q] = *reinterpret_cast<const float4*>(Y + (16 * (q + q0) + i16) * KP + 16 * j + 4 * g);
                 }
 #pragma unroll
-                for (int s = 0; s < 4; ++s)
-#pragma unroll
-                    for (int p = 0; p < 2; ++p)
-#pragma unroll
-                        for (int q = 0; q < 2; ++q)
-                            acc[p][q] = __builtin_amdgcn_mfma_f64_16x16x4f64((double)(s == 0 ? x[p].x : s == 1 ? x[p].y : s == 2 ? x[p].z : x[p].w),
-                                                                             (double)(s == 0 ? y[q].x : s == 1 ? y[q].y : s == 2 ? y[q].z : y[q].w), acc[p][q], 0, 0, 0);
-            }
-#pragma unroll
-            for (int p = 0; p < 2; ++p)
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const int t = 16 * p + 4 * e + g, s = 16 * q + i16;
-                        D[t * CP + s] = (strict ? s < t : s <= t) ? (float)acc[p][q][e] : 0.f;
+                for (int s = 0; s < 4; ++s) {
+                    const auto of = [&](const float4& v) { return (double)(s == 0 ? v.x : s == 1 ? v.y : s == 2 ? v.z : v.w); };
+                    acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(of(x[0]), of(y[0]), acc[0], 0, 0, 0);
+                    if (DELTA) {
+                        acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(of(x[1]), of(y[0]), acc[1], 0, 0, 0);
+                        acc[2] = __builtin_amdgcn_mfma_f64_16x16x4f64(of(x[1]), of(y[1]), acc[2], 0, 0, 0);
                     }
-        } else {
-            f32x16_t p[4] = {};
-#pragma unroll
-            for (int j = 0; j < DK / 8; ++j) {
-                const float4 x = *reinterpret_cast<const float4*>(X + l32 * KP + 8 * j + 4 * hi);
-                const float4 y = *reinterpret_cast<const float4*>(Y + l32 * KP + 8 * j + 4 * hi);
-                p[0] = __builtin_amdgcn_mfma_f32_32x32x2f32(x.x, y.x, p[0], 0, 0, 0);
-                p[1] = __builtin_amdgcn_mfma_f32_32x32x2f32(x.y, y.y, p[1], 0, 0, 0);
-                p[2] = __builtin_amdgcn_mfma_f32_32x32x2f32(x.z, y.z, p[2], 0, 0, 0);
-                p[3] = __builtin_amdgcn_mfma_f32_32x32x2f32(x.w, y.w, p[3], 0, 0, 0);
+                }
             }
-            const f32x16_t acc = (p[0] + p[1]) + (p[2] + p[3]);
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int t = 8 * (e >> 2) + 4 * hi + (e & 3);
-                D[t * CP + l32] = l32 <= t ? acc[e] * Wc[t - l32] : 0.f;
-            }
+            for (int i = 0; i < (DELTA ? 3 : 1); ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = 16 * (DELTA ? i > 0 : p0) + 4 * e + g, s = 16 * (DELTA ? i > 1 : q0) + i16;
+                    if (!DELTA) { if (s <= t) D[t * TP + s] = acc[i][e] * Wc[t - s]; }
+                    else if (wave == 1) { if (s <= t) D[t * TP + s] = acc[i][e]; }               // A_k
+                    else if (wave == 2) { if (s < t) D[t * TP + s] = acc[i][e]; }                // L
+                    else if (s < t || (wave == 3 && s == t)) D[s * TP + t + 1] = acc[i][e];      // N, A_b
+                }
         }
     }
     __syncthreads();
-    const auto lower = [&](const float* D) { return [=](int s) { return D[l32 * CP + 2 * s + hi]; }; };          // row l32
-    const auto across = [&](const float* D, int stride, int at) { return [=](int s) { return D[(2 * s + hi) * stride + at + l32]; }; };
     if (DELTA) {
-        // N V, where the substitution expects it
-        for (int ct = wave; ct < TV; ct += 4) {
-            const f32x16_t acc = product(f32x16_t{}, lower(Nm), across(Vm, VP, ct * 32));
-#pragma unroll
-            for (int e = 0; e < 16; ++e) Xm[(8 * (e >> 2) + 4 * hi + (e & 3)) * XP + DK + ct * 32 + l32] = acc[e];
-        }
-        __syncthreads();
-        // (I + L) [X | Y] = [U | N V], a column a thread
-        if (tid < NX) {
-            float x[C];
+        // T = (I + L)^-1, a column a lane
+        if (wave == 0) {
+            const int j = lane & 31;
+            double x[C], row[2][C];
 #pragma unroll
             for (int t = 0; t < C; ++t) {
-                float s = Xm[t * XP + tid];
+                if (t + 1 < C) {
 #pragma unroll
-                for (int q = 0; q < t; q += 4) {
-                    const float4 l4 = *reinterpret_cast<const float4*>(Lm + t * CP + q);      // zeros from the diagonal on
-                    s = fmaf(-l4.x, x[q], s);
-                    if (q + 1 < t) s = fmaf(-l4.y, x[q + 1], s);
-                    if (q + 2 < t) s = fmaf(-l4.z, x[q + 2], s);
-                    if (q + 3 < t) s = fmaf(-l4.w, x[q + 3], s);
+                    for (int q = 0; q <= t; ++q) row[(t + 1) & 1][q] = T2[(t + 1) * TP + q];
                 }
-                x[t] = s;
+                double s[4] = {t == j ? 1.0 : 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+                for (int q = 0; q < t; ++q) s[q & 3] = fma(-row[t & 1][q], x[q], s[q & 3]);
+                x[t] = (s[0] + s[1]) + (s[2] + s[3]);
+                asm volatile("" : "+v"(x[t]) :: "memory");       // one row of L ahead of its use, not all of them (registers)
             }
 #pragma unroll
-            for (int t = 0; t < C; ++t) Xm[t * XP + tid] = x[t];
+            for (int t = 0; t < C; ++t)
+                if (t >= j) T2[t * TP + j] = x[t];
+        }
+        __syncthreads();
+        // P = A_b T in the place of A_b: the first wave, which reads all of it before it writes.  The others G = T^T B~ ..
+        constexpr int UNITS = 2 * (DK / 16), MINE = (UNITS + 2) / 3;       // tiles of [C][DK], of one of three waves
+        if (wave == 0) {
+            f64x4_t x[3] = {};
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const int t = 16 * (i > 0) + i16, col = 16 * (i > 1) + i16;
+                const auto ab = [&](int s) { return second_of(A2, t, s); };
+                const auto ts = [&](int s) { return first_of(T2, s, col); };
+                x[i] = i == 0 ? product<0, 4>(x[i], g, ab, ts) : i == 1 ? product<0, 8>(x[i], g, ab, ts) : product<4, 8>(x[i], g, ab, ts);
+            }
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = 16 * (i > 0) + 4 * e + g, s = 16 * (i > 1) + i16;
+                    if (s <= t) A2[s * TP + t + 1] = x[i][e];
+                }
+        } else {
+            for (int u = wave - 1; u < UNITS; u += 3) {
+                const int half = u & 1, ch = (u >> 1) * 16 + i16;
+                const double wc = Wc[ch];
+                const auto ts = [&](int s) { return first_of(T2, s, 16 * half + i16); };
+                const auto bs = [&](int s) { return (double)Bm[s * KP + ch] * wc; };
+                f64x4_t x = {};
+                x = half ? product<4, 8>(x, g, ts, bs) : product<0, 8>(x, g, ts, bs);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) Gs[(16 * half + 4 * e + g) * HP + ch] = x[e];
+            }
+        }
+        __syncthreads();
+        // .. then E = A_k - P N in the place of A_k, and H = K~ - N^T G
+        f64x4_t hs[MINE];
+        if (wave == 0) {
+            f64x4_t x[3];
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const int t = 16 * (i > 0) + i16, col = 16 * (i > 1) + i16;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) x[i][e] = first_of(A2, 16 * (i > 0) + 4 * e + g, col);
+                const auto ps = [&](int s) { return -second_of(A2, t, s); };
+                const auto ns = [&](int s) { return second_strictly(T2, s, col); };
+                x[i] = i == 0 ? product<0, 4>(x[i], g, ps, ns) : i == 1 ? product<0, 8>(x[i], g, ps, ns) : product<4, 8>(x[i], g, ps, ns);
+            }
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = 16 * (i > 0) + 4 * e + g, s = 16 * (i > 1) + i16;
+                    if (s <= t) A2[t * TP + s] = x[i][e];
+                }
+        } else {
+#pragma unroll
+            for (int m = 0; m < MINE; ++m) {
+                const int u = min(wave - 1 + 3 * m, UNITS - 1), half = u & 1, ch = (u >> 1) * 16 + i16;
+                const double wc = Wc[ch];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) hs[m][e] = (double)Km[(16 * half + 4 * e + g) * KP + ch] * wc;
+                const auto ns = [&](int s) { return -second_strictly(T2, s, 16 * half + i16); };
+                const auto gs = [&](int s) { return Gs[s * HP + ch]; };
+                hs[m] = half ? product<4, 8>(hs[m], g, ns, gs) : product<0, 8>(hs[m], g, ns, gs);
+            }
+        }
+        __syncthreads();
+        if (wave > 0) {
+#pragma unroll
+            for (int m = 0; m < MINE; ++m) {
+                const int u = wave - 1 + 3 * m, half = u & 1, ch = (u >> 1) * 16 + i16;
+                if (u >= UNITS) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) Hs[(16 * half + 4 * e + g) * HP + ch] = hs[m][e];
+            }
         }
         __syncthreads();
     }
-    const auto minus = [](f32x16_t x) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) x[e] = -x[e];
-        return x;
-    };
     bool bad = false;
-    const auto check = [&](const f32x16_t& x) {
-#pragma unroll
-        for (int e = 0; e < 16; ++e) bad |= endless(x[e]);
+    const auto rounded = [&](const f64x4_t& x) {
+        const float4 y = make_float4((float)x[0], (float)x[1], (float)x[2], (float)x[3]);
+        bad |= endless(y.x) || endless(y.y) || endless(y.z) || endless(y.w);
+        return y;
     };
-    // R' transposed (rows: channels, columns: tokens), so that a lane's four consecutive rows are one store
-    for (int it = wave; it < TK; it += 4) {
-        f32x16_t acc;
+    const auto place = [&](int from, int tile) { return reinterpret_cast<float4*>(unit + from) + tile * 64 + lane; };
+    // R' transposed (rows: channels, columns: tokens)
+    for (int kt = wave; kt < DK / 16; kt += 4) {
+        const auto us = [&](int s) { return -(double)Um[s * KP + kt * 16 + turned(i16)]; };
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int ch = it * 32 + 8 * (e >> 2) + 4 * hi + (e & 3);
-            acc[e] = Rm[l32 * KP + ch] * (DELTA ? 1.f : Wc[l32 + 1]);
-        }
-        if (DELTA) acc = minus(product(minus(acc), across(Xm, XP, it * 32), lower(Ab)));
-        check(acc);
+        for (int half = 0; half < 2; ++half) {
+            const int t = 16 * half + i16;
+            const float4 r4 = *reinterpret_cast<const float4*>(Rm + t * KP + kt * 16 + 4 * g);
+            f64x4_t x = {(double)r4.x, (double)r4.y, (double)r4.z, (double)r4.w};
+            if (DELTA) {
+                const auto ps = [&](int s) { return second_of(A2, t, s); };
+                x = half ? product<0, 8>(x, g, us, ps) : product<0, 4>(x, g, us, ps);
+            } else {
+                const double w = Wc[t + 1];
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int kt = it * 2 + (q >> 1), g = (q & 1) * 2 + hi;
-            *reinterpret_cast<float4*>(unit + U::R + ((((l32 >> 4) * (DK / 16) + kt) * 64 + g * 16 + (l32 & 15)) * 4)) =
-                make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
+                for (int e = 0; e < 4; ++e) x[e] *= w;
+            }
+            *place(U::R, half * (DK / 16) + kt) = rounded(x);
         }
     }
     // the chunk's own part of the outputs
-    for (int ct = (wave + 2) & 3; ct < TV; ct += 4) {
-        f32x16_t acc = {};
-        if (DELTA) acc = minus(product(acc, lower(Ab), across(Xm, XP, DK + ct * 32)));
-        acc = product(acc, lower(Ak), across(Vm, VP, ct * 32));
-        check(acc);
+    for (int ct = (wave + 2) & 3; ct < DV / 16; ct += 4) {
+        const auto vs = [&](int s) { return (double)Vm[s * VP + ct * 16 + i16]; };
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int t = 8 * (e >> 2) + 4 * hi + (e & 3);
-            if (t < nc) a.out[(size_t)(t0 + t) * a.out_stride + h * DV + ct * 32 + l32] = acc[e];
+        for (int half = 0; half < 2; ++half) {
+            const auto es = [&](int s) { return first_of(A2, 16 * half + i16, s); };
+            f64x4_t x = {};
+            x = half ? product<0, 8>(x, g, es, vs) : product<0, 4>(x, g, es, vs);
+            const float4 y = rounded(x);
+            const float ye[4] = {y.x, y.y, y.z, y.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int t = 16 * half + 4 * e + g;
+                if (t < nc) a.out[(size_t)(t0 + t) * a.out_stride + h * DV + ct * 16 + i16] = ye[e];
+            }
         }
     }
+    // 32 x 32 results: rows of A's channels, columns of B's
+    const auto square = [&](int from, int rows, int cols, int rt, int ct, auto fa, auto fb) {
+        f64x4_t x[2][2] = {};
+#pragma unroll
+        for (int s = 0; s < C / 4; ++s) {
+            double p[2], q[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) { p[i] = fa(4 * s + g, (2 * rt + i) * 16 + turned(i16)); q[i] = fb(4 * s + g, (2 * ct + i) * 16 + i16); }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) x[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(p[i], q[j], x[i][j], 0, 0, 0);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) *place(from, (2 * ct + j) * (rows / 16) + 2 * rt + i) = rounded(x[i][j]);
+    };
     // what the chunk adds to the state
     for (int m = wave; m < TK * TV; m += 4) {
-        const int it = m / TV, ct = m % TV;
-        const float wc = DELTA ? Wc[it * 32 + l32] : 0.f;
-        f32x16_t acc = {};
-        if (DELTA) {
-            acc = minus(product(acc, [&](int s) { return Bm[(2 * s + hi) * KP + it * 32 + l32] * wc; }, across(Xm, XP, DK + ct * 32)));
-            acc = product(acc, [&](int s) { return Km[(2 * s + hi) * KP + it * 32 + l32] * wc; }, across(Vm, VP, ct * 32));
-        } else {
-            acc = product(acc, [&](int s) {
-                const int t = 2 * s + hi;
-                return Km[t * KP + it * 32 + l32] * Wc[max(nc - 1 - t, 0)];      // (k is zero past the end)
-            }, across(Vm, VP, ct * 32));
-        }
-        check(acc);
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const int kt = it * 2 + (q >> 1), g = (q & 1) * 2 + hi, cb = ct * 2 + (l32 >> 4);
-            *reinterpret_cast<float4*>(unit + U::S + ((cb * (DK / 16) + kt) * 64 + g * 16 + (l32 & 15)) * 4) =
-                make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-        }
+        const auto vs = [&](int t, int col) { return (double)Vm[t * VP + col]; };
+        if (DELTA) square(U::S, DK, DV, m / TV, m % TV, [&](int t, int ch) { return Hs[t * HP + ch]; }, vs);
+        else square(U::S, DK, DV, m / TV, m % TV, [&](int t, int ch) { return (double)Km[t * KP + ch] * Wc[max(nc - 1 - t, 0)]; }, vs);   // (k is zero past the end)
     }
     if (DELTA) {
-        // M transposed (rows: the channel it is summed over, columns: the channel it goes to)
-        for (int m = wave; m < TK * TK; m += 4) {
-            const int jt = m / TK, it = m % TK;
-            const float wc = Wc[it * 32 + l32];
-            f32x16_t acc = minus(product(f32x16_t{}, across(Xm, XP, jt * 32),
-                                         [&](int s) { return Bm[(2 * s + hi) * KP + it * 32 + l32] * wc; }));
-#pragma unroll
-            for (int e = 0; e < 16; ++e)
-                if (jt == it && 8 * (e >> 2) + 4 * hi + (e & 3) == l32) acc[e] += wc;
-            check(acc);
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int kt = jt * 2 + (q >> 1), g = (q & 1) * 2 + hi, rt = it * 2 + (l32 >> 4);
-                *reinterpret_cast<float4*>(unit + U::M + ((rt * (DK / 16) + kt) * 64 + g * 16 + (l32 & 15)) * 4) =
-                    make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3]);
-            }
+        // M transposed (rows: the channel it is summed over, columns: the channel it goes to), without W_C on its diagonal
+        for (int m = wave; m < TK * TK; m += 4)
+            square(U::M, DK, DK, m / TK, m % TK, [&](int t, int ch) { return -(double)Um[t * KP + ch]; }, [&](int t, int ch) { return Gs[t * HP + ch]; });
+        if (tid < DK) {
+            const float w = (float)Wc[tid];
+            unit[U::W + tid] = w;
+            bad |= endless(w);
         }
     }
     const int any = __syncthreads_or(bad);
@@ -414,10 +472,10 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
     for (int q = 0; q < 2; ++q)
 #pragma unroll
         for (int i = 0; i < 4; ++i) S[q][i] = fresh ? 0.f : Sg[(size_t)((wave * 2 + q) * 16 + 4 * g + i) * DV];
-    struct Ops { f32x4_t m[DELTA ? 2 : 1][DELTA ? NA : 1], r[NA], add[2], o; };
+    struct Ops { f32x4_t m[DELTA ? 2 : 1][DELTA ? NA : 1], w[DELTA ? 2 : 1], r[NA], add[2], o; };
     const bool outputs = wave < 2;               // two tiles of 16 tokens
     const float d = DELTA ? 0.f : a.decay[h];
-    const float d_chunk = DELTA ? 0.f : power(d, C);
+    const double d_chunk = DELTA ? 0.0 : power(d, C);
     auto ask = [&](int c, Ops& x) {
         const f32x4_t* unit = reinterpret_cast<const f32x4_t*>(units + (size_t)c * a.H * U::SIZE);
 #pragma unroll
@@ -426,6 +484,7 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
             if (DELTA) {
 #pragma unroll
                 for (int k = 0; k < NA; ++k) x.m[q][k] = unit[U::M / 4 + ((wave * 2 + q) * NA + k) * 64 + lane];
+                x.w[q] = unit[U::W / 4 + (wave * 2 + q) * 4 + g];
             }
         }
         if (outputs) {
@@ -442,37 +501,38 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
 #pragma unroll
         for (int q = 0; q < 2; ++q) St[c & 1][wave * 2 + q][lane] = S[q];
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // LDS only: the next chunk's loads stay under way
-        const float dc = DELTA ? 0.f : ((a.c0 + c + 1) * C <= n ? d_chunk : power(d, n - (a.c0 + c) * C));
-        constexpr int CH = 4;                                                // chains of sums, as in product
-        f32x4_t next[2][CH] = {}, o[CH] = {};
+        const double dc = DELTA ? 0.0 : ((a.c0 + c + 1) * C <= n ? d_chunk : power(d, n - (a.c0 + c) * C));
+        // the instruction adds in order: short chains, for the outputs of 8 or 16 products
+        constexpr int CH = 4, CO = 8;
+        f32x4_t next[2][CH] = {}, o[CO] = {};
 #pragma unroll
         for (int k = 0; k < NA; ++k) {
             const f32x4_t s = St[c & 1][k][lane];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (DELTA) {
-                    next[0][i % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[0][k][i], s[i], next[0][i % CH], 0, 0, 0);
-                    next[1][i % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[1][k][i], s[i], next[1][i % CH], 0, 0, 0);
+                    next[0][(4 * k + i) % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[0][k][i], s[i], next[0][(4 * k + i) % CH], 0, 0, 0);
+                    next[1][(4 * k + i) % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[1][k][i], s[i], next[1][(4 * k + i) % CH], 0, 0, 0);
                 }
-                if (outputs) o[i % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.r[k][i], s[i], o[i % CH], 0, 0, 0);
+                if (outputs) o[(4 * k + i) % CO] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.r[k][i], s[i], o[(4 * k + i) % CO], 0, 0, 0);
             }
         }
-        const auto whole = [](const f32x4_t (&p)[CH]) { return (p[0] + p[1]) + (p[2] + p[3]); };
         if (outputs) {
+            const f32x4_t whole = ((o[0] + o[1]) + (o[2] + o[3])) + ((o[4] + o[5]) + (o[6] + o[7]));
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int t = (a.c0 + c) * C + wave * 16 + 4 * g + i;
-                if (t < n) a.out[(size_t)(t_lo + t) * a.out_stride + h * DV + cb * 16 + col] = x.o[i] + whole(o)[i];
+                if (t < n) a.out[(size_t)(t_lo + t) * a.out_stride + h * DV + cb * 16 + col] = x.o[i] + whole[i];
             }
         }
+        // the new state, rounded once
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
-            if (DELTA) {
-                S[q] = x.add[q] + whole(next[q]);
-            } else {
+            const f32x4_t whole = (next[q][0] + next[q][1]) + (next[q][2] + next[q][3]);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) S[q][i] = fmaf(dc, S[q][i], x.add[q][i]);
-            }
+            for (int i = 0; i < 4; ++i)
+                S[q][i] = DELTA ? (float)(fma((double)x.w[q][i], (double)S[q][i], (double)x.add[q][i]) + (double)whole[i])
+                                : (float)fma(dc, (double)S[q][i], (double)x.add[q][i]);
         }
     };
     static_assert(NW >= 2, "two waves make the outputs");
@@ -494,10 +554,8 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
 
 template <int DK, int DV, bool DELTA>
 int launch_chunks(ChunkArgs a, int num_rows, int max_tokens, hipStream_t stream) {
-    constexpr int KP = DK + 4, VP = DV + 4;
-    constexpr size_t lds = sizeof(float) * (C * (2 * KP + VP + CP) + (DK > C + 4 ? DK : C + 4)
-                                            + (DELTA ? C * (2 * KP + 3 * CP + DK + DV + 4) : 0));
-    static_assert(lds <= 160 * 1024, "more LDS than a compute unit has");
+    constexpr size_t lds = sizeof(float) * Lds<DK, DV, DELTA>::SIZE;
+    static_assert(lds <= 160 * 1024 && (DK > 64 || lds <= 80 * 1024), "more LDS than a compute unit has, or than half of it");
     auto operators = chunk_operators_kernel<DK, DV, DELTA>;
     if (lds > 64 * 1024) {          // beyond what a kernel may take unasked: ask once a device
         static std::mutex mu;
@@ -535,7 +593,7 @@ extern "C" int ri_linear_scan_chunks_supported(int delta, int dk, int dv, float 
 }
 
 static size_t unit_floats(int delta, int num_rows, int max_tokens, int H, int dk, int dv) {
-    return (size_t)num_rows * segment(num_rows, max_tokens) * H * ((size_t)C * dk + (size_t)dk * dv + (delta ? (size_t)dk * dk : 0) + 4);
+    return (size_t)num_rows * segment(num_rows, max_tokens) * H * ((size_t)C * dk + (size_t)dk * dv + (delta ? (size_t)dk * dk + dk : 0) + 4);
 }
 
 // Floats of workspace for steps of up to num_rows rows of at most max_tokens tokens.

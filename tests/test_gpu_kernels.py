@@ -1136,11 +1136,13 @@ def _walk64(r, k, v, S, w, b, u):
     return torch.stack(out), S
 
 
-@pytest.mark.parametrize("form,d,keys", [("delta", 64, "random"), ("delta", 128, "random"), ("delta", 64, "repeated"), ("delta", 64, "fast decay"),
-                                         ("decay", 64, "random"), ("decay", 128, "random"), ("rotated", 64, "random"), ("rotated", 128, "random")])
+@pytest.mark.parametrize("form,d,keys", [("delta", 64, "random"), ("delta", 128, "random"), ("delta", 64, "repeated"), ("delta", 128, "repeated"), ("delta", 64, "fast decay"),
+                                         ("delta", 64, "shared"), ("delta", 128, "shared"), ("decay", 64, "random"), ("decay", 128, "random"),
+                                         ("decay", 64, "shared"), ("decay", 128, "shared"), ("rotated", 64, "random"), ("rotated", 128, "random")])
 def test_state_walk_in_chunks(ops, monkeypatch, form, d, keys):
     """Rows of many tokens go through chunks of 32, the others through the walk; new and continued states, last chunks
-    that are not whole, more chunks than a pass takes.  Both against 64 bits: the chunks are as exact as the walk."""
+    that are not whole, more chunks than a pass takes.  Both against 64 bits: neither the outputs nor the states of the chunks
+    are further from it than the walk's, whatever the keys have in common."""
     H, q_lens, starts = 3, [32, 5, 33, 1, 300, 64], [0, 3, 40, 7, 31, 0]
     T, B = sum(q_lens), len(q_lens)
     bf = lambda *shape, seed, scale=1.0: rnd(*shape, dtype=torch.bfloat16, seed=seed, scale=scale)  # noqa: E731
@@ -1148,6 +1150,8 @@ def test_state_walk_in_chunks(ops, monkeypatch, form, d, keys):
     wl, al, w0, ab = bf(T, H * d, seed=4), bf(T, H * d, seed=5), rnd(H * d, seed=6), rnd(H * d, seed=7)
     if keys == "repeated":                        # one key all along, given up and written whole, hardly any decay: L is all ones
         k, w0, ab = k[:1].repeat(T, 1), torch.full_like(w0, -12.0), torch.full_like(ab, 12.0)
+    elif keys == "shared":                        # keys around one direction, as a trained model's are, given up slowly
+        r, k, w0, ab = r + k[:1] if form == "decay" else r, k[:1] + 0.3 * k, w0 - 3.0, ab + 2.0
     elif keys == "fast decay":                    # decays at their bound and next to one side by side
         w0 = torch.where(torch.arange(H * d, device=DEV) % 2 == 0, 12.0, -12.0)
     decay = torch.tensor([0.999, 0.7, 0.02], device=DEV)
@@ -1181,18 +1185,19 @@ def test_state_walk_in_chunks(ops, monkeypatch, form, d, keys):
         monkeypatch.setattr(ops, "_scan_in_chunks", lambda *a: chunks)
         state, out = state0.clone(), torch.full((T, H * d), float("nan"), device=DEV)
         ops.linear_scan(r, k, v, state, out, ctx, H, d, d, **kw)
-        worst, lo = 0.0, 0
+        worst, lo = [0.0, 0.0], 0                                  # outputs and states, added over the rows of many tokens
         for b, n in enumerate(q_lens):
             S = state0[slots[b]].double() if starts[b] else torch.zeros(H, d, d, dtype=torch.float64, device=DEV)
             part = slice(lo, lo + n)
             o64, S64 = _walk64(r64[part], k64[part], v64[part], S, w64[part], b64[part], u64[part])
-            for got, want in ((out[part].double().view(n, H, d), o64), (state[slots[b]].double(), S64)):
-                worst = max(worst, ((got - want).norm() / want.norm()).item())
+            for i, (got, want) in enumerate(((out[part].double().view(n, H, d), o64), (state[slots[b]].double(), S64))):
+                error = ((got - want).norm() / want.norm()).item()
+                assert error < 2e-6, (b, i, error)
+                worst[i] += error if n >= 32 else 0.0
             lo += n
         assert torch.equal(state[4], state0[4])                    # no request's slot
         errors[chunks] = worst
-    # (measured: 1.0 to 1.25 of the walk's error, 0.45 in the decay form)
-    assert errors[True] <= 1.5 * errors[False], errors
+    assert all(c <= 1.02 * w for c, w in zip(errors[True], errors[False])), errors       # (0.02: what rounds otherwise by chance)
 
 
 def _scan_step(form, d, H, q_lens, starts, seed=20, unit_eps=1e-6):
