@@ -58,7 +58,8 @@ struct ChunkArgs {
     const float *rot_cos, *rot_sin;
     int rot;
     float k_scale;
-    float* ws;                          // [row][chunk of the segment][head][Unit::SIZE]
+    const int* rows;                    // the grid's rows, then -1 (null: all, in order)
+    float* ws;                          // [row of the grid][chunk of the segment][head][Unit::SIZE]
     int* from;                          // [row][head][dv / 16]: the token that the walk goes on from
     int c0, seg;                        // the segment's first chunk of every row, its chunks
 };
@@ -119,7 +120,8 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
     constexpr int KP = At::KP, VP = At::VP, HP = At::HP;
     constexpr int EK = DK / 64 > 0 ? DK / 64 : 1, TK = DK / 32, TV = DV / 32;
     using U = Unit<DK, DV, DELTA>;
-    const int b = blockIdx.z, h = blockIdx.y, cs = blockIdx.x, c = a.c0 + cs;
+    const int b = a.rows ? a.rows[blockIdx.z] : (int)blockIdx.z, h = blockIdx.y, cs = blockIdx.x, c = a.c0 + cs;
+    if (b < 0) return;
     const int t_lo = a.cu_q[b], n = a.cu_q[b + 1] - t_lo;
     if (n < a.min_tokens || c * C >= n) return;
     const int nc = min(C, n - c * C), t0 = t_lo + c * C;
@@ -137,7 +139,7 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
     double* T2 = reinterpret_cast<double*>(lds + At::T);       // delta: L, then T; and N
     double* Wc = reinterpret_cast<double*>(lds + At::W);       // delta: [DK] of W_C; else powers of d, 0 .. C
     static_assert(2 * HP <= 2 * KP, "H fits where K and B were");
-    float* unit = a.ws + (((size_t)b * a.seg + cs) * a.H + h) * U::SIZE;
+    float* unit = a.ws + (((size_t)blockIdx.z * a.seg + cs) * a.H + h) * U::SIZE;
     const float d = DELTA ? 0.f : a.decay[h];
 
     // the tokens' vectors, activated; tokens past the end leave the state alone (w = 1, the others 0)
@@ -453,14 +455,15 @@ template <int DK, int DV, bool DELTA>
 __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a) {
     constexpr int NW = DK / 32, NA = DK / 16;
     using U = Unit<DK, DV, DELTA>;
-    const int b = blockIdx.z, h = blockIdx.y, cb = blockIdx.x;
+    const int b = a.rows ? a.rows[blockIdx.z] : (int)blockIdx.z, h = blockIdx.y, cb = blockIdx.x;
+    if (b < 0) return;
     const int t_lo = a.cu_q[b], n = a.cu_q[b + 1] - t_lo;
     if (n < a.min_tokens || a.c0 * C >= n) return;
     int* const from = a.from + ((size_t)b * a.H + h) * (DV / 16) + cb;       // (this block's own, the same in all of a head's)
     if (a.c0 > 0 && *from < a.c0 * C) return;          // the walk takes the row over before this segment
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
     const int all = min(a.seg, (n + C - 1) / C - a.c0);          // at most 64
-    const float* units = a.ws + ((size_t)b * a.seg * a.H + h) * U::SIZE;
+    const float* units = a.ws + ((size_t)blockIdx.z * a.seg * a.H + h) * U::SIZE;
     const unsigned long long bads = __ballot(lane < all && reinterpret_cast<const int*>(units + (size_t)lane * a.H * U::SIZE)[U::BAD] != 0);
     const int chunks = bads ? __ffsll(bads) - 1 : all;
     if (threadIdx.x == 0) *from = (a.c0 + chunks) * C;
@@ -553,7 +556,7 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
 }
 
 template <int DK, int DV, bool DELTA>
-int launch_chunks(ChunkArgs a, int num_rows, int max_tokens, hipStream_t stream) {
+int launch_chunks(ChunkArgs a, int rows, int max_tokens, hipStream_t stream) {
     constexpr size_t lds = sizeof(float) * Lds<DK, DV, DELTA>::SIZE;
     static_assert(lds <= 160 * 1024 && (DK > 64 || lds <= 80 * 1024), "more LDS than a compute unit has, or than half of it");
     auto operators = chunk_operators_kernel<DK, DV, DELTA>;
@@ -572,15 +575,15 @@ int launch_chunks(ChunkArgs a, int num_rows, int max_tokens, hipStream_t stream)
     }
     const int chunks = (max_tokens + C - 1) / C;
     for (a.c0 = 0; a.c0 < chunks; a.c0 += a.seg) {
-        operators<<<dim3(min(a.seg, chunks - a.c0), a.H, num_rows), 256, lds, stream>>>(a);
-        chunk_states_kernel<DK, DV, DELTA><<<dim3(DV / 16, a.H, num_rows), DK * 2, 0, stream>>>(a);
+        operators<<<dim3(min(a.seg, chunks - a.c0), a.H, rows), 256, lds, stream>>>(a);
+        chunk_states_kernel<DK, DV, DELTA><<<dim3(DV / 16, a.H, rows), DK * 2, 0, stream>>>(a);
     }
     return 0;
 }
 
-// chunks of every row that one pass takes: the workspace holds some 64 chunks of all heads
-int segment(int num_rows, int max_tokens) {
-    const int chunks = (max_tokens + C - 1) / C, most = num_rows < 64 ? 64 / num_rows : 1;
+// chunks of each of so many rows that one pass takes: the workspace holds some 64 chunks of all heads
+int segment(int rows, int max_tokens) {
+    const int chunks = (max_tokens + C - 1) / C, most = rows < 64 ? 64 / rows : 1;
     return chunks < most ? chunks : most;
 }
 
@@ -592,13 +595,13 @@ extern "C" int ri_linear_scan_chunks_supported(int delta, int dk, int dv, float 
     return (dk == 64 || dk == 128) && dv == dk;
 }
 
-static size_t unit_floats(int delta, int num_rows, int max_tokens, int H, int dk, int dv) {
-    return (size_t)num_rows * segment(num_rows, max_tokens) * H * ((size_t)C * dk + (size_t)dk * dv + (delta ? (size_t)dk * dk + dk : 0) + 4);
+static size_t unit_floats(int delta, int rows, int max_tokens, int H, int dk, int dv) {
+    return (size_t)rows * segment(rows, max_tokens) * H * ((size_t)C * dk + (size_t)dk * dv + (delta ? (size_t)dk * dk + dk : 0) + 4);
 }
 
-// Floats of workspace for steps of up to num_rows rows of at most max_tokens tokens.
-extern "C" size_t ri_linear_scan_chunks_workspace(int delta, int num_rows, int max_tokens, int H, int dk, int dv) {
-    return unit_floats(delta, num_rows, max_tokens, H, dk, dv) + (size_t)num_rows * H * (dv / 16);
+// Floats of workspace for a step of num_rows rows, `listed` of which the chunks may take, of at most max_tokens tokens.
+extern "C" size_t ri_linear_scan_chunks_workspace(int delta, int num_rows, int listed, int max_tokens, int H, int dk, int dv) {
+    return unit_floats(delta, listed, max_tokens, H, dk, dv) + (size_t)num_rows * H * (dv / 16);
 }
 
 extern "C" int ri_linear_scan(
@@ -611,7 +614,9 @@ extern "C" int ri_linear_scan(
         float k_scale, int most, const int* from, int from_cols, hipStream_t stream);
 
 // ri_linear_scan with the rows of at least min_tokens tokens (max_tokens at most, or an upper bound) in chunks; the walk
-// does the others, and what the chunks leave to it.  bfloat16 projections.
+// does the others, and what the chunks leave to it.  row_list [listed]: the rows of several tokens, then -1, which must
+// hold all rows of min_tokens and more; a pass, its grid and the workspace are theirs, however many rows of
+// single tokens the step has (null: all rows, listed = num_rows).  bfloat16 projections.
 extern "C" int ri_linear_scan_chunks(
         const void* r, int r_stride, const void* k, int k_stride, const void* v, int v_stride,
         const void* wl, int wl_stride, const void* al, int al_stride,
@@ -619,14 +624,15 @@ extern "C" int ri_linear_scan_chunks(
         float unit_eps, float decay_c, float* state, int num_slots, float* out, int out_stride,
         const int* cu_q, const int* q_start, const int* slots, int num_rows, int T,
         int H, int dk, int dv, const float* rot_cos, const float* rot_sin, int rot, int rot_rows, int max_position,
-        float k_scale, int min_tokens, int max_tokens, float* ws, size_t ws_floats, hipStream_t stream) {
+        float k_scale, int min_tokens, int max_tokens, const int* row_list, int listed, float* ws, size_t ws_floats, hipStream_t stream) {
     RI_REQUIRE(H > 0 && ri_linear_scan_chunks_supported(delta, dk, dv, decay_c), "ri_linear_scan_chunks: does not take H=%d dk=%d dv=%d decay_c=%g", H, dk, dv, (double)decay_c);
-    RI_REQUIRE(num_rows >= 0 && T >= 0 && num_slots > 0 && min_tokens > 1, "ri_linear_scan_chunks: bad counts");
+    RI_REQUIRE(num_rows >= 0 && T >= 0 && num_slots > 0 && min_tokens > 1 && (row_list ? listed >= 0 && listed <= num_rows : listed == num_rows), "ri_linear_scan_chunks: bad counts");
     RI_REQUIRE(r_stride >= H * dk && k_stride >= H * dk && v_stride >= H * dv && out_stride >= H * dv, "ri_linear_scan_chunks: row strides too small");
-    if (num_rows == 0 || T == 0 || max_tokens <= 0) return 0;
+    if (num_rows == 0 || T == 0) return 0;
+    RI_REQUIRE(listed > 0 && max_tokens > 0, "ri_linear_scan_chunks: no row of several tokens");
     RI_REQUIRE(r && k && v && state && out && cu_q && q_start && slots && ws, "ri_linear_scan_chunks: null pointer");
     RI_REQUIRE(H <= 65535 && num_rows <= 65535, "ri_linear_scan_chunks: too many heads or rows for the grid");
-    RI_REQUIRE((uintptr_t)ws % 16 == 0 && ws_floats >= ri_linear_scan_chunks_workspace(delta, num_rows, max_tokens, H, dk, dv), "ri_linear_scan_chunks: the workspace is too small");
+    RI_REQUIRE((uintptr_t)ws % 16 == 0 && ws_floats >= ri_linear_scan_chunks_workspace(delta, num_rows, listed, max_tokens, H, dk, dv), "ri_linear_scan_chunks: the workspace is too small");
     if (delta) RI_REQUIRE(wl && al && w0 && ab && wl_stride >= H * dk && al_stride >= H * dk && !rot_cos && k_scale == 1.f, "ri_linear_scan_chunks: the delta form needs wl, al, w0, ab and no rotation or key factor");
     else RI_REQUIRE(decay, "ri_linear_scan_chunks: the decay form needs a decay for each head");
     if (rot_cos) RI_REQUIRE(!silu_in && rot_sin && rot > 0 && rot % 2 == 0 && rot <= dk && rot_rows > 0 && max_position < rot_rows,
@@ -637,11 +643,11 @@ extern "C" int ri_linear_scan_chunks(
     a.w0 = w0; a.ab = ab; a.decay = decay; a.state = state; a.out = out; a.out_stride = out_stride;
     a.cu_q = cu_q; a.q_start = q_start; a.slots = slots; a.H = H; a.silu_in = silu_in; a.min_tokens = min_tokens;
     a.unit_eps = unit_eps; a.decay_c = decay_c; a.rot_cos = rot_cos; a.rot_sin = rot_sin; a.rot = rot_cos ? rot : 0; a.k_scale = k_scale;
-    a.ws = ws; a.c0 = 0; a.seg = segment(num_rows, max_tokens);
-    a.from = reinterpret_cast<int*>(ws + unit_floats(delta, num_rows, max_tokens, H, dk, dv));
+    a.rows = row_list; a.ws = ws; a.c0 = 0; a.seg = segment(listed, max_tokens);
+    a.from = reinterpret_cast<int*>(ws + unit_floats(delta, listed, max_tokens, H, dk, dv));
     int rc;
-    if (dk == 64) rc = delta ? launch_chunks<64, 64, true>(a, num_rows, max_tokens, stream) : launch_chunks<64, 64, false>(a, num_rows, max_tokens, stream);
-    else rc = delta ? launch_chunks<128, 128, true>(a, num_rows, max_tokens, stream) : launch_chunks<128, 128, false>(a, num_rows, max_tokens, stream);
+    if (dk == 64) rc = delta ? launch_chunks<64, 64, true>(a, listed, max_tokens, stream) : launch_chunks<64, 64, false>(a, listed, max_tokens, stream);
+    else rc = delta ? launch_chunks<128, 128, true>(a, listed, max_tokens, stream) : launch_chunks<128, 128, false>(a, listed, max_tokens, stream);
     if (rc) return rc;
     RI_LAUNCHED("ri_linear_scan_chunks");
     return ri_linear_scan(r, r_stride, k, k_stride, v, v_stride, wl, wl_stride, al, al_stride, RI_BF16, w0, ab, decay, delta, silu_in,

@@ -1226,15 +1226,19 @@ def linear_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
             _ptr(ctx.cu_q), _ptr(ctx.q_start), _ptr(ctx.state_slots), ctx.num_rows, T, H, dk, dv,
             rcos, rsin, rot, rrows, max(int(ctx.max_kv_len) - 1, 0), ctypes.c_float(k_scale))
     longest, workspace = int(ctx.max_q_len), getattr(ctx, "workspace", None)
-    portions = int(getattr(ctx, "num_portion", 0) or ctx.num_rows)
-    if workspace is not None and r.dtype == torch.bfloat16 and _scan_in_chunks(delta, dk, portions, longest) \
+    listed, row_list = int(getattr(ctx, "num_portion", 0)), getattr(ctx, "portion_rows", None)
+    if listed <= 0 or row_list is None:
+        listed, row_list = ctx.num_rows, None
+    else:
+        _i32(row_list, "portion_rows", listed)
+    if workspace is not None and r.dtype == torch.bfloat16 and _scan_in_chunks(delta, dk, listed, longest) \
             and lib.ri_linear_scan_chunks_supported(int(delta), dk, dv, ctypes.c_float(decay_c)):
         # prompts: chunks of tokens on the matrix instructions; the walk takes the rows of fewer tokens, and heads with
         # something not finite.  (32-bit projections stay with the walk, whose bits do not depend on how a request was cut into steps)
         lib.ri_linear_scan_chunks_workspace.restype = ctypes.c_size_t
-        need = lib.ri_linear_scan_chunks_workspace(int(delta), ctx.num_rows, longest, H, dk, dv)
+        need = lib.ri_linear_scan_chunks_workspace(int(delta), ctx.num_rows, listed, longest, H, dk, dv)
         ws = workspace.get("scan.chunks", need, 1, torch.float32)
-        _check(lib.ri_linear_scan_chunks(*inputs, *form, SCAN_CHUNK_TOKENS, longest, _ptr(ws), ctypes.c_size_t(ws.numel()), _stream()))
+        _check(lib.ri_linear_scan_chunks(*inputs, *form, SCAN_CHUNK_TOKENS, longest, _ptr(row_list), listed, _ptr(ws), ctypes.c_size_t(ws.numel()), _stream()))
         return
     _check(lib.ri_linear_scan(*inputs, _dt(r), *form, 0, None, 0, _stream()))
 

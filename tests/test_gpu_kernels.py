@@ -1259,6 +1259,23 @@ def test_state_walk_in_chunks_of_tokens_that_are_not_finite(ops, monkeypatch, fo
         lo += n
 
 
+@pytest.mark.parametrize("form,d", [("delta", 64), ("decay", 64), ("delta", 128), ("decay", 128)])
+def test_state_walk_in_chunks_beside_decoding_rows(ops, monkeypatch, form, d):
+    """Two portions among more rows of single tokens than a pass has chunks: what the chunks need is the portions', not the
+    rows', and the other rows' tokens and states are the walk's to the bit."""
+    H, q_lens = 2, [1] * 33 + [130] + [1] * 20 + [2, 75] + [1] * 17
+    starts = [(7 * i) % 50 for i in range(len(q_lens))]
+    r, k, v, state, ctx, kw = _scan_step(form, d, H, q_lens, starts, seed=60)
+    (out0, state0), (out1, state1) = _scan_both_ways(ops, monkeypatch, H, d, r, k, v, state, ctx, kw)
+    unit = 32 * d + d * d + (d * d + d if form == "delta" else 0) + 4
+    assert 0 < ctx.workspace.nbytes() <= 4 * (64 * H * unit + len(q_lens) * H * d // 16)
+    lo = 0
+    for b, n in enumerate(q_lens):
+        for x, y in ((out1[lo:lo + n], out0[lo:lo + n]), (state1[b], state0[b])):
+            assert torch.equal(x, y) if n < 32 else (x - y).norm() <= 5e-7 * y.norm(), b
+        lo += n
+
+
 @pytest.mark.parametrize("T,n,pad,shift", [(300, 2056, 8, 0), (257, 2048, 0, 8), (600, 1000, 4, 0), (256, 2048, 8, 3), (65, 8200, 8, 16), (4, 7, 1, 0), (3, 64, 0, 0)])
 @pytest.mark.parametrize("name", ["relu2", "tanh"])
 def test_unary_in_wide_and_single_elements(ops, name, T, n, pad, shift):
