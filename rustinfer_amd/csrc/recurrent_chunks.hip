@@ -599,9 +599,10 @@ static size_t unit_floats(int delta, int rows, int max_tokens, int H, int dk, in
     return (size_t)rows * segment(rows, max_tokens) * H * ((size_t)C * dk + (size_t)dk * dv + (delta ? (size_t)dk * dk + dk : 0) + 4);
 }
 
-// Floats of workspace for a step of num_rows rows, `listed` of which the chunks may take, of at most max_tokens tokens.
-extern "C" size_t ri_linear_scan_chunks_workspace(int delta, int num_rows, int listed, int max_tokens, int H, int dk, int dv) {
-    return unit_floats(delta, listed, max_tokens, H, dk, dv) + (size_t)num_rows * H * (dv / 16);
+// Floats of workspace that are enough for any step of at most num_rows rows: 64 chunks of all heads, whatever the number
+// and length of its portions up to 64 of them.
+extern "C" size_t ri_linear_scan_chunks_workspace(int delta, int num_rows, int H, int dk, int dv) {
+    return unit_floats(delta, 1, 64 * C, H, dk, dv) + (size_t)num_rows * H * (dv / 16);
 }
 
 extern "C" int ri_linear_scan(
@@ -632,7 +633,7 @@ extern "C" int ri_linear_scan_chunks(
     RI_REQUIRE(listed > 0 && max_tokens > 0, "ri_linear_scan_chunks: no row of several tokens");
     RI_REQUIRE(r && k && v && state && out && cu_q && q_start && slots && ws, "ri_linear_scan_chunks: null pointer");
     RI_REQUIRE(H <= 65535 && num_rows <= 65535, "ri_linear_scan_chunks: too many heads or rows for the grid");
-    RI_REQUIRE((uintptr_t)ws % 16 == 0 && ws_floats >= ri_linear_scan_chunks_workspace(delta, num_rows, listed, max_tokens, H, dk, dv), "ri_linear_scan_chunks: the workspace is too small");
+    RI_REQUIRE((uintptr_t)ws % 16 == 0 && ws_floats >= unit_floats(delta, listed, max_tokens, H, dk, dv) + (size_t)num_rows * H * (dv / 16), "ri_linear_scan_chunks: the workspace is too small");
     if (delta) RI_REQUIRE(wl && al && w0 && ab && wl_stride >= H * dk && al_stride >= H * dk && !rot_cos && k_scale == 1.f, "ri_linear_scan_chunks: the delta form needs wl, al, w0, ab and no rotation or key factor");
     else RI_REQUIRE(decay, "ri_linear_scan_chunks: the decay form needs a decay for each head");
     if (rot_cos) RI_REQUIRE(!silu_in && rot_sin && rot > 0 && rot % 2 == 0 && rot <= dk && rot_rows > 0 && max_position < rot_rows,

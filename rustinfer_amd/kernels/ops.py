@@ -1231,15 +1231,18 @@ def linear_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.
         listed, row_list = ctx.num_rows, None
     else:
         _i32(row_list, "portion_rows", listed)
-    if workspace is not None and r.dtype == torch.bfloat16 and _scan_in_chunks(delta, dk, listed, longest) \
+    if workspace is not None and r.dtype == torch.bfloat16 and longest >= SCAN_CHUNK_TOKENS \
             and lib.ri_linear_scan_chunks_supported(int(delta), dk, dv, ctypes.c_float(decay_c)):
         # prompts: chunks of tokens on the matrix instructions; the walk takes the rows of fewer tokens, and heads with
-        # something not finite.  (32-bit projections stay with the walk, whose bits do not depend on how a request was cut into steps)
+        # something not finite.  (32-bit projections stay with the walk, whose bits do not depend on how a request was cut into steps.)
+        # The workspace is that of the largest step and taken by every step with portions: the first one, or the one that
+        # the cache pool's size is measured with, takes it once and for all.
         lib.ri_linear_scan_chunks_workspace.restype = ctypes.c_size_t
-        need = lib.ri_linear_scan_chunks_workspace(int(delta), ctx.num_rows, listed, longest, H, dk, dv)
-        ws = workspace.get("scan.chunks", need, 1, torch.float32)
-        _check(lib.ri_linear_scan_chunks(*inputs, *form, SCAN_CHUNK_TOKENS, longest, _ptr(row_list), listed, _ptr(ws), ctypes.c_size_t(ws.numel()), _stream()))
-        return
+        ws = workspace.get("scan.chunks", lib.ri_linear_scan_chunks_workspace(int(delta), state.shape[0], H, dk, dv), 1, torch.float32)
+        if _scan_in_chunks(delta, dk, listed, longest):
+            _check(lib.ri_linear_scan_chunks(*inputs, *form, SCAN_CHUNK_TOKENS, longest, _ptr(row_list), listed, _ptr(ws),
+                                             ctypes.c_size_t(ws.numel()), _stream()))
+            return
     _check(lib.ri_linear_scan(*inputs, _dt(r), *form, 0, None, 0, _stream()))
 
 

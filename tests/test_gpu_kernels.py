@@ -1276,6 +1276,21 @@ def test_state_walk_in_chunks_beside_decoding_rows(ops, monkeypatch, form, d):
         lo += n
 
 
+@pytest.mark.parametrize("form", ["delta", "decay"])
+def test_state_walk_takes_its_workspace_with_the_first_portion(ops, form):
+    """A step whose portions the walk takes (so may the one that the cache pool's size is measured with) leaves nothing for later
+    steps to allocate, whatever they hold."""
+    H, d, ws = 2, 64, Workspace(torch.device(DEV))
+    sizes = []
+    for q_lens in ([40] * 24, [100], [3000], [400, 300], [1] * 24, [200] * 4 + [1] * 20):
+        r, k, v, _, ctx, kw = _scan_step(form, d, H, q_lens, [0] * len(q_lens))
+        ctx.workspace = ws
+        ops.linear_scan(r, k, v, torch.zeros(25, H, d, d, device=DEV), torch.empty(r.shape[0], H * d, device=DEV), ctx, H, d, d, **kw)
+        sizes.append(ws.nbytes())
+    assert not ops._scan_in_chunks(form == "delta", d, 24, 40) and ops._scan_in_chunks(form == "delta", d, 1, 3000)
+    assert sizes[0] > 0 and len(set(sizes)) == 1, sizes
+
+
 @pytest.mark.parametrize("T,n,pad,shift", [(300, 2056, 8, 0), (257, 2048, 0, 8), (600, 1000, 4, 0), (256, 2048, 8, 3), (65, 8200, 8, 16), (4, 7, 1, 0), (3, 64, 0, 0)])
 @pytest.mark.parametrize("name", ["relu2", "tanh"])
 def test_unary_in_wide_and_single_elements(ops, name, T, n, pad, shift):
