@@ -1168,15 +1168,17 @@ SCAN_CHUNK_TOKENS = 32          # rows of so many tokens and more go through chu
 def _scan_in_chunks(delta: bool, d: int, rows: int, longest: int) -> bool:
     """Whether a step with ``rows`` prompt portions of up to ``longest`` tokens runs the state walk in chunks of
     tokens.  The walk's time is its longest row's, whatever else is in the step, until the rows fill the chip;
-    the chunks' grows with all tokens.  Measured, us, walk / chunks, 32 heads of 64, delta form: 1 x 48 29 / 30,
-    1 x 64 37 / 31, 1 x 2048 1205 / 232, 2 x 64 38 / 34, 4 x 64 39 / 42, 4 x 128 70 / 53, 4 x 512 305 / 173,
-    8 x 512 319 / 336; decay form: 1 x 48 20 / 21, 1 x 64 24 / 21, 1 x 2048 768 / 100, 4 x 64 25 / 22, 8 x 64
-    27 / 32, 8 x 128 50 / 37, 24 x 256 205 / 228.  24 heads of 128, delta form: 1 x 64 47 / 67, 1 x 96 70 / 72,
-    1 x 2048 1741 / 559, 2 x 128 125 / 90, 4 x 512 512 / 525; decay form: 1 x 64 30 / 28, 2 x 64 32 / 36, 2 x 128
-    71 / 44, 8 x 128 143 / 90."""
+    the chunks' grows with all tokens, and rows of single tokens beside them are a walk after it.  Measured, us, walk / chunks, alone |
+    beside 8 | 64 decoding rows.  32 heads of 64, delta form: 1 x 64 35 / 36 | 37 / 40 | 70 / 71, 1 x 96 50 / 38 | 53 / 43 | 89 / 72, 1 x 2048
+    1174 / 259 | 1176 / 266 | 1227 / 290, 2 x 64 36 / 39 | 38 / 44 | 71 / 72, 4 x 64 36 / 50 | 38 / 54 | 70 / 76, 4 x 128
+    67 / 61 | 70 / 64 | 108 / 88, 8 x 256 160 / 193 | 177 / 198 | 197 / 223; decay form: 1 x 64 25 / 17 | 27 / 22 | 51 / 45, 1 x 2048 790 / 109 |
+    790 / 114 | 811 / 132, 4 x 64 25 / 25 | 27 / 30 | 52 / 49, 8 x 128 52 / 42 | 57 / 47 | 78 / 65, 16 x 256 119 / 143 | 122 / 147 | 140 / 166.
+    24 heads of 128, delta form: 1 x 96 65 / 80 | 116 / 100 | 224 / 216, 1 x 128 96 / 84 | 145 / 104 | 254 / 220, 2 x 128 122 / 101 | 149 / 122 |
+    255 / 235, 4 x 256 256 / 269 | 274 / 293 | 385 / 414; decay form: 1 x 64 29 / 31 | 50 / 58 | 131 / 138, 1 x 128 52 / 38 | 80 / 62 | 163 / 140,
+    2 x 64 32 / 42 | 53 / 63 | 133 / 141, 16 x 128 228 / 175 | 244 / 194 | 321 / 311."""
     if delta:
-        return rows * d <= 256 and longest >= max(64, 32 * rows) * d // 64
-    return rows <= 16 and longest >= (64 if rows <= 4 and d <= 64 else 128)
+        return rows * d <= 256 and longest >= max(96 if d <= 64 else 128, 32 * rows)
+    return rows <= (8 if d <= 64 else 16) and longest >= (64 if rows <= 2 and d <= 64 else 128)
 
 
 def linear_scan(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor, out: torch.Tensor, ctx,

@@ -101,3 +101,13 @@ def test_bare_tensor_names_reach_their_parts():
     assert lazy.narrow("embed")[""] == 5 and lazy.narrow("l0").narrow("mix")["a.b"] == 3
     assert sorted(lazy.narrow("l0").keys()) == ["mix.a", "mix.a.b", "norm1"]
     assert join_name("l0", "") == "l0" and join_name("", "x") == "x" and join_name("l0", "mix.q") == "l0.mix.q"
+
+
+@pytest.mark.parametrize("delta,d,rows,longest,chunks", [
+    (True, 64, 1, 64, False), (True, 64, 1, 96, True), (True, 64, 2, 64, False), (True, 64, 4, 128, True), (True, 64, 8, 256, False),
+    (True, 128, 1, 96, False), (True, 128, 2, 128, True), (True, 128, 4, 256, False), (False, 64, 1, 64, True), (False, 64, 4, 64, False),
+    (False, 64, 8, 128, True), (False, 64, 16, 256, False), (False, 128, 1, 64, False), (False, 128, 16, 128, True)])
+def test_where_the_state_walk_goes_in_chunks(delta, d, rows, longest, chunks):
+    """Portions on both sides of each line, as they were measured alone and beside up to 128 decoding rows."""
+    from rustinfer_amd.kernels import ops
+    assert ops._scan_in_chunks(delta, d, rows, longest) is chunks
