@@ -7,8 +7,9 @@
 // 4,096 cycles.  So nothing passes through LDS on the way in: every lane reads 16 bytes of K of its row
 // of A and of W straight into registers, a chunk ahead of the one that is multiplied, and the four
 // steps of such 16 bytes take the K values {4g + s} of the four lane groups g, for A and W alike.  The
-// waves of a block share one tile of results and take chunks of K in turn; their 64-bit sums meet in LDS
-// once, in the order of the waves, so a row's result does not depend on the other rows or on the tile.
+// waves of a block share one tile of results and take 32 values of K in turn, whatever the tile; their 64-bit sums meet in
+// LDS once, in the order of the waves, so a row's result does not depend on the other rows or on the tile.  (Products
+// of up to four rows, gemm_rows_f32, add in another order: the same to the rounding of a 64-bit sum.)
 // Blocks of one column tile run on one XCD (consecutive block ids go around the eight of them), so a
 // tile's weights pass through one L2.  K % 4 == 0, rows 16-byte aligned.
 //
@@ -19,13 +20,15 @@
 
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
-// MT x NT tiles of 16 x 16 results a block, WAVES waves that share K, chunks of 16 U values of K.
+// MT x NT tiles of 16 x 16 results a block, WAVES waves that share K, chunks of 16 U values of K (U = 1: two of them, one
+// after the other, are a wave's turn of 32).
 // STREAM: W is read once (a single row of tiles), past the caches.
 template <int MT, int NT, int WAVES, int U, bool STREAM>
 __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(
         const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
         float* __restrict__ C, int ldc, int M, int N, int K, int mtiles, int ntiles) {
-    constexpr int KC = 16 * U;
+    constexpr int KC = 16 * U, TURN = WAVES * 32, K1 = U == 1 ? KC : TURN, K2 = U == 1 ? TURN : 2 * TURN;
+    static_assert(U == 1 || U == 2, "a wave's turn of K is 32 values");
     __shared__ double sums[WAVES][16][NT * 16];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int xcd = (int)blockIdx.x & 7, turn = (int)blockIdx.x >> 3;
@@ -74,10 +77,10 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(
             }
     };
     float4 a0[U][MT], w0[U][NT], a1[U][MT], w1[U][NT];
-    int k = wave * KC;
+    int k = wave * 32;
     if (k < K) ask(k, a0, w0);
-    for (; k < K; k += 2 * WAVES * KC) {
-        const int k1 = k + WAVES * KC, k2 = k1 + WAVES * KC;
+    for (; k < K; k += K2) {
+        const int k1 = k + K1, k2 = k + K2;
         if (k1 < K) ask(k1, a1, w1);
         add(a0, w0);
         if (k1 < K) {
@@ -133,6 +136,13 @@ static void launch_f32(const float* A, int lda, const float* W, int ldw, float* 
     const int blocks = (ntiles + 7) / 8 * 8 * mtiles;
     if (mtiles == 1) gemm_f32_kernel<MT, NT, 8, U, true><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles);
     else gemm_f32_kernel<MT, NT, 8, U, false><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles);
+}
+
+// The rows and columns of the tile that ri_gemm_f32 takes for M rows and N columns.
+extern "C" void ri_gemm_f32_tile(int M, int N, int* rows, int* columns) {
+    const F32Tile& t = F32_TILES[f32_tile(M, N)];
+    *rows = 16 * t.mt;
+    *columns = 16 * t.nt;
 }
 
 // The 32-bit product of any number of rows (K % 4 == 0, operands and rows 16-byte aligned).

@@ -1,6 +1,7 @@
 """Each kernel alone against a plain PyTorch 32-bit/64-bit reference of the same op, at sizes
 other than the engine tests use (widths and vocabularies that are no power of two, head sizes
 in steps of 16, odd head counts and groups)."""
+import ctypes
 import math
 from types import SimpleNamespace
 
@@ -405,6 +406,31 @@ def test_linear_f32_on_the_matrix_instruction(ops, M, N, K):
     # a 64-bit sum rounded once: half a unit of the last place of each result
     assert torch.all((out[:, :N].double() - ref).abs() <= ref.abs() * 2.0 ** -24 + 1e-12 * ref.abs().max())
     assert torch.all(torch.isnan(out[:, N:]))
+
+
+def test_linear_f32_gives_a_row_the_same_bits_on_every_tile(ops):
+    """Rows of terms that cancel to some 2^-23 of the largest, so that the order of the 64-bit sums shows in the 32-bit
+    results: the first rows alone and among more rows, on each of the tiles, edges and a last part of K that is no
+    whole turn of a wave included."""
+    M, N, K = 600, 3075, 532
+    g = torch.Generator().manual_seed(3)
+    x = torch.randn(M, K, generator=g) * 2.0 ** torch.randint(-20, 21, (M, K), generator=g)
+    x[:, K // 2:] = -x[:, :K // 2]
+    w = torch.randn(N, K, generator=g)
+    w[:, K // 2:] = w[:, :K // 2] * (1 + torch.randint(0, 2, (N, K // 2), generator=g) * 2.0 ** -23)
+    x, w = x.to(DEV), w.to(DEV)
+    tiles, first = set(), None
+    for rows in (5, 17, 65, 300, 600):
+        a, b = ctypes.c_int(0), ctypes.c_int(0)
+        ops._lib().ri_gemm_f32_tile(rows, N, ctypes.byref(a), ctypes.byref(b))
+        tiles.add((a.value, b.value))
+        out = torch.full((rows, N), float("nan"), device=DEV)
+        ops.linear(x[:rows], w, out)
+        first = out[:5].clone() if first is None else first
+        assert torch.equal(out[:5], first), rows
+        ref = x[:rows].double() @ w.double().t()                   # K products in 64 bits, added in another order
+        assert torch.all((out.double() - ref).abs() <= ref.abs() * 2.0 ** -24 + K * 2.0 ** -52 * (x[:rows].double().abs() @ w.double().abs().t()))
+    assert tiles == {(16, 16), (32, 16), (16, 32), (32, 32), (48, 32)}
 
 
 def _paged_setup(dtype, B, H, Hkv, hd, page, q_lens, starts, seed=0, num_pages=128, shuffle=True):
