@@ -130,12 +130,18 @@ static int f32_tile(int M, int N) {
     return best;
 }
 
+// A launch holds fewer than 2^32 threads, 8 M blocks of 512: larger products take several, of whole rows of tiles each.
 template <int MT, int NT, int U>
 static void launch_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K, hipStream_t stream) {
-    const int mtiles = (M + 16 * MT - 1) / (16 * MT), ntiles = (N + 16 * NT - 1) / (16 * NT);
-    const int blocks = (ntiles + 7) / 8 * 8 * mtiles;
-    if (mtiles == 1) gemm_f32_kernel<MT, NT, 8, U, true><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles);
-    else gemm_f32_kernel<MT, NT, 8, U, false><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles);
+    const int ntiles = (N + 16 * NT - 1) / (16 * NT), across = (ntiles + 7) / 8 * 8;
+    const int most = ((1 << 23) - 1) / across * 16 * MT;
+    for (int m0 = 0; m0 < M; m0 += most) {
+        const int m = min(M - m0, most), mtiles = (m + 16 * MT - 1) / (16 * MT);
+        const float* a = A + (size_t)m0 * lda;
+        float* c = C + (size_t)m0 * ldc;
+        if (mtiles == 1) gemm_f32_kernel<MT, NT, 8, U, true><<<across, 512, 0, stream>>>(a, lda, W, ldw, c, ldc, m, N, K, mtiles, ntiles);
+        else gemm_f32_kernel<MT, NT, 8, U, false><<<across * mtiles, 512, 0, stream>>>(a, lda, W, ldw, c, ldc, m, N, K, mtiles, ntiles);
+    }
 }
 
 // The rows and columns of the tile that ri_gemm_f32 takes for M rows and N columns.
@@ -151,7 +157,7 @@ extern "C" int ri_gemm_f32(const float* A, int lda, const float* W, int ldw, flo
     RI_REQUIRE(M >= 1 && N > 0 && K > 0 && K % 4 == 0, "ri_gemm_f32: needs rows and K %% 4 == 0 (M=%d N=%d K=%d)", M, N, K);
     RI_REQUIRE(lda >= K && ldw >= K && ldc >= N && lda % 4 == 0 && ldw % 4 == 0, "ri_gemm_f32: leading dimensions must be >= K and multiples of 4");
     RI_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0, "ri_gemm_f32: null or unaligned pointer");
-    RI_REQUIRE((long long)((M + 15) / 16) * ((N + 15) / 16 + 7) < (1ll << 31), "ri_gemm_f32: M=%d N=%d exceed the grid limit", M, N);
+    RI_REQUIRE(N <= (1 << 26), "ri_gemm_f32: N=%d exceeds the grid limit", N);
     switch (f32_tile(M, N)) {
         case 0: launch_f32<2, 2, 2>(A, lda, W, ldw, C, ldc, M, N, K, stream); break;
         case 1: launch_f32<3, 2, 1>(A, lda, W, ldw, C, ldc, M, N, K, stream); break;

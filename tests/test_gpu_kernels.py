@@ -433,6 +433,25 @@ def test_linear_f32_gives_a_row_the_same_bits_on_every_tile(ops):
     assert tiles == {(16, 16), (32, 16), (16, 32), (32, 32), (48, 32)}
 
 
+def test_linear_f32_of_more_tiles_than_a_launch_holds(ops):
+    """66,016 rows of 131,072 columns, as the logits of a whole large batch are: 34.6 GB in two launches; rows around the
+    seam, the first and the last."""
+    M, N, K = 66016, 131072, 4
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    out = torch.full((M, N), float("nan"), device=DEV)
+    a, b = ctypes.c_int(0), ctypes.c_int(0)
+    ops._lib().ri_gemm_f32_tile(M, N, ctypes.byref(a), ctypes.byref(b))
+    seam = ((1 << 23) - 1) // (N // b.value) * a.value
+    assert 0 < seam < M - 64
+    ops.linear(x, w, out)
+    assert not out.sum().isnan()
+    for r in (0, 31, 32, seam - 1, seam, seam + 40, M - 1):
+        ref = x[r].double() @ w.double().t()
+        assert torch.all((out[r].double() - ref).abs() <= ref.abs() * 2.0 ** -24 + 1e-15), r
+    del out
+    torch.cuda.empty_cache()
+
+
 def _paged_setup(dtype, B, H, Hkv, hd, page, q_lens, starts, seed=0, num_pages=128, shuffle=True):
     """A cache with random pages for each request, the step's q/k/v, and contiguous copies."""
     g = torch.Generator().manual_seed(seed)
