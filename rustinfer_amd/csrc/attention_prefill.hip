@@ -75,15 +75,15 @@ __global__ __launch_bounds__(256, WPE) void attn_prefill_kernel(
         const int* __restrict__ cu_q, const int* __restrict__ q_start, const int* __restrict__ kv_lens,
         int H, int Hkv, int page_arg, float scale_log2e, int window_arg, int min_q_len,
         int split_keys, int nsplit, float* __restrict__ part_o, float* __restrict__ part_ml, int part_tokens,
-        const int* __restrict__ row_list, int order) {
+        const int* __restrict__ row_list, int order, int first_place) {
     typedef PrefillFrags<HD> Frags;
     static_assert(!SHARE || FAST, "fragments are shared only with pages of 16 and no window");
     static_assert(!SPLIT || SHARE, "the keys are divided between blocks only in the shared form");
     // this block's range of keys [kb, ke)
-    // the grid's second and third index: row and place among the row's blocks; in pairs, place and row
+    // the grid's second and third index: row and place among the row's blocks from first_place on; in pairs, place and row
     const bool paired = order == 1;
     const int by = __builtin_amdgcn_workgroup_id_y(), bz = __builtin_amdgcn_workgroup_id_z();
-    const int split = SPLIT ? bz % nsplit : 0, at = SPLIT ? bz / nsplit : paired ? by : bz;
+    const int split = SPLIT ? bz % nsplit : 0, at = SPLIT ? bz / nsplit : first_place + (paired ? by : bz);
     const int kb = SPLIT ? split * split_keys : 0;
     const int ke = SPLIT && split + 1 < nsplit ? kb + split_keys : 0x7fffffff;     // the last range takes what is left
     constexpr int NF = HD / 8;                                   // fragments of a step: 2 * HD/32 of keys, HD/16 of values
@@ -705,7 +705,7 @@ extern "C" int ri_attention_prefill(
     const long long row_tiles = (max_q_len + 63) / 64, places = (paired ? (row_tiles + 1) / 2 : row_tiles) * nsplit;
     const int head_groups = (G + NQ - 1) / NQ;
     RI_REQUIRE(B <= 65535, "ri_attention_prefill: too many rows");
-    RI_REQUIRE((long long)Hkv * head_groups <= 0x7fffffffLL && places <= 65535, "ri_attention_prefill: grid too large");
+    RI_REQUIRE((long long)Hkv * head_groups <= 0x7fffffffLL && (nsplit < 2 || places <= 65535), "ri_attention_prefill: grid too large");
     float *part_o = nullptr, *part_ml = nullptr;
     if (nsplit > 1) {
         const size_t need = (size_t)nsplit * total_q * H * (hd + 2) * sizeof(float);
@@ -713,13 +713,15 @@ extern "C" int ri_attention_prefill(
         part_o = (float*)workspace;
         part_ml = part_o + (size_t)nsplit * total_q * H * hd;
     }
-    dim3 grid(Hkv * head_groups, paired ? (unsigned)places : BY, paired ? BY : (unsigned)places);
-#define RI_PREFILL_LAUNCH(...) attn_prefill_kernel<__VA_ARGS__><<<grid, 256, 0, stream>>>((const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)kc, (const bf16_t*)vc, table, max_blocks, cu_q, q_start, kv_lens, H, Hkv, page, sl2, window, min_q_len, split_keys, nsplit, part_o, part_ml, total_q, row_list, plan.order)
+    // a grid's second and third index end at 65535: a row of more places (4 M tokens, 8 M in pairs) takes several launches
+#define RI_PREFILL_LAUNCH(...) for (long long first = 0; first < places; first += 65535) { \
+        const unsigned here = (unsigned)std::min<long long>(places - first, 65535); \
+        attn_prefill_kernel<__VA_ARGS__><<<dim3(Hkv * head_groups, paired ? here : BY, paired ? BY : here), 256, 0, stream>>>((const bf16_t*)q, q_stride, (bf16_t*)out, out_stride, (const bf16_t*)kc, (const bf16_t*)vc, table, max_blocks, cu_q, q_start, kv_lens, H, Hkv, page, sl2, window, min_q_len, split_keys, nsplit, part_o, part_ml, total_q, row_list, plan.order, (int)first); }
     if (nsplit > 1) {
-        if (hd == 64 && NQ == 2) RI_PREFILL_LAUNCH(64, 2, true, true, 3, true);
-        else if (hd == 64) RI_PREFILL_LAUNCH(64, 1, true, true, 1, true);
-        else if (NQ == 2) RI_PREFILL_LAUNCH(128, 2, true, true, 2, true);
-        else RI_PREFILL_LAUNCH(128, 1, true, true, 1, true);
+        if (hd == 64 && NQ == 2) RI_PREFILL_LAUNCH(64, 2, true, true, 3, true)
+        else if (hd == 64) RI_PREFILL_LAUNCH(64, 1, true, true, 1, true)
+        else if (NQ == 2) RI_PREFILL_LAUNCH(128, 2, true, true, 2, true)
+        else RI_PREFILL_LAUNCH(128, 1, true, true, 1, true)
         RI_LAUNCHED("ri_attention_prefill(ranges)");
         const long long per_row = (long long)max_q_len * H * (hd / 4);
         dim3 cgrid((unsigned)((per_row + 255) / 256), BY);
@@ -731,20 +733,20 @@ extern "C" int ri_attention_prefill(
     // pages of 16 without a window always take a shared form (registers capped so that two waves, or three, share a
     // SIMD); the plain form serves the rest
     if (hd == 64 && fast) {
-        if (NQ == 4) RI_PREFILL_LAUNCH(64, 4, true, true, 2);
-        else if (NQ == 2) RI_PREFILL_LAUNCH(64, 2, true, true, 3);
-        else RI_PREFILL_LAUNCH(64, 1, true, true);
+        if (NQ == 4) RI_PREFILL_LAUNCH(64, 4, true, true, 2)
+        else if (NQ == 2) RI_PREFILL_LAUNCH(64, 2, true, true, 3)
+        else RI_PREFILL_LAUNCH(64, 1, true, true)
     } else if (hd == 64) {
-        if (NQ == 1) RI_PREFILL_LAUNCH(64, 1, false);
-        else if (NQ == 2) RI_PREFILL_LAUNCH(64, 2, false);
-        else if (NQ == 3) RI_PREFILL_LAUNCH(64, 3, false);
-        else RI_PREFILL_LAUNCH(64, 4, false);
+        if (NQ == 1) RI_PREFILL_LAUNCH(64, 1, false)
+        else if (NQ == 2) RI_PREFILL_LAUNCH(64, 2, false)
+        else if (NQ == 3) RI_PREFILL_LAUNCH(64, 3, false)
+        else RI_PREFILL_LAUNCH(64, 4, false)
     } else if (fast) {
-        if (NQ == 2) RI_PREFILL_LAUNCH(128, 2, true, true, 2);
-        else RI_PREFILL_LAUNCH(128, 1, true, true);
+        if (NQ == 2) RI_PREFILL_LAUNCH(128, 2, true, true, 2)
+        else RI_PREFILL_LAUNCH(128, 1, true, true)
     } else {
-        if (NQ == 1) RI_PREFILL_LAUNCH(128, 1, false);
-        else RI_PREFILL_LAUNCH(128, 2, false);
+        if (NQ == 1) RI_PREFILL_LAUNCH(128, 1, false)
+        else RI_PREFILL_LAUNCH(128, 2, false)
     }
 #undef RI_PREFILL_LAUNCH
     RI_LAUNCHED("ri_attention_prefill");

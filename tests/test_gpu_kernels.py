@@ -603,6 +603,25 @@ def test_turned_values_with_weights_in_three_parts(ops, monkeypatch, H, Hkv, hd,
     assert ((got[0] - got[1]).abs() <= 2.0 ** -7 * got[1].abs() + 2e-5).all()
 
 
+def test_attention_of_more_tiles_than_a_grid_has_places_for(ops):
+    """One row of 8.4 M tokens with a window: some pairs of tiles beyond 65,535, the middle of the row."""
+    hd, window, T = 64, 32, 2 * 65535 * 64 + 1000
+    pages = -(-T // 16)
+    q, k, v = (torch.randn(pages * 16, hd, device=DEV, dtype=torch.bfloat16, generator=torch.Generator(DEV).manual_seed(i)) for i in range(3))
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    pos = torch.arange(T, dtype=torch.int32, device=DEV)
+    ctx = SimpleNamespace(num_tokens=T, num_rows=1, cu_q=i32([0, T]), q_start=i32([0]), kv_lens=i32([T]), positions=pos,
+                          row_of_token=torch.zeros_like(pos), max_q_len=T, max_kv_len=T, host_q_lens=[T], workspace=Workspace(torch.device(DEV)))
+    out = torch.full((T, hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.paged_attention(q[:T], out, 1, 1, hd, k.view(pages, 1, 16, hd), v.view(pages, 16, hd).transpose(1, 2).contiguous().view(pages, 1, hd, 16),
+                        torch.arange(pages, dtype=torch.int32, device=DEV).view(1, pages), 16, ctx, hd ** -0.5, window)
+    assert out.isfinite().all()
+    for p in (0, 40, 65535 * 64 - 1, 65535 * 64, 65535 * 64 + 500, 65535 * 64 + 999, 65535 * 64 + 1000, T - 1):
+        lo = max(0, p + 1 - window)
+        w = torch.softmax((k[lo:p + 1].double() @ q[p].double()) * hd ** -0.5, 0)
+        assert ((w @ v[lo:p + 1].double()) - out[p].double()).abs().max() < 2e-2, p
+
+
 RANGE_CASES = [
     # B, H, Hkv, hd, page, q_lens, starts; ranges of keys asked for (0: the kernel's own choice)
     ((1, 8, 2, 128, 16, [16], [2040]), 0),                       # a short portion behind many keys: six ranges of 384
