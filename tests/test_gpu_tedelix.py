@@ -474,3 +474,54 @@ def test_trace_replay_of_a_tedelix_model(tdirs, plain_logits, tmp_path):
         if n:
             results[st["step"]] = np.fromfile(os.path.join(str(tmp_path), f"{st['step']}.f32"), dtype="<f4").reshape(n, -1)
     check_rows(steps, results, logits, "float32", "trace replay")
+
+
+CHUNKED = dict(architecture="Tedelix", vocab=190, width=128, norm=dict(eps=1e-5), logit_scale=1.0, logit_softcap=30.0, layers=[
+    dict(type="general_delta", mixer=dict(heads=2, dim=64), mlp=dict(kind="dense", ff=192)),
+    dict(type="lightning", mixer=dict(heads=3, dim=64, vdim=64, decay=[0.97, 0.999, 0.5]), mlp=dict(kind="dense", ff=64)),
+    dict(type="attention", mixer=dict(heads=4, kv_heads=2, dim=32, vdim=32, mask=dict(size=150), scale=0.18, rot=dict(base=10000.0, dims=32)), mlp=None),
+    dict(type="general_delta", mixer=dict(heads=1, dim=128), mlp=dict(kind="dense", ff=128)),
+    dict(type="lightning", mixer=dict(heads=1, dim=128, vdim=128, decay=[0.99]), mlp=None),
+])
+
+
+@pytest.mark.parametrize("graphs,rows,portions", [(False, 0, [[700], [33]]), (False, 70, [[200], [200], [130, 96], [31], [240, 64]]),
+                                                  (True, 38, [[200], [200], [200], [201], [130, 96], [138, 96]]), (True, 0, [[300], [299], [298]])])
+def test_prompts_whose_states_go_through_chunks(tmp_path, monkeypatch, graphs, rows, portions):
+    """Heads of 64 and 128 in bfloat16, the state walk's route as the engine's own steps choose it: prompts alone and
+    beside more decoding rows than a pass has chunks, portions of one request after the other and of two at once,
+    eagerly and in graphs that are captured once and replayed for other portions of the shape."""
+    from rustinfer_amd.engine import StepEntry, build_engine
+    from rustinfer_amd.kernels import ops
+    from rustinfer_amd.weights import write_safetensors
+    with open(tmp_path / "config.json", "w") as f:
+        json.dump(CHUNKED, f)
+    write_safetensors(str(tmp_path / "model.safetensors"), draw_weights(CHUNKED, 6, 77))
+    cfg, w = P.read_model(str(tmp_path))
+    longs = max(len(p) for p in portions)
+    totals = [sum(p[i] for p in portions if i < len(p)) for i in range(longs)]
+    reqs = random_requests(cfg["vocab"], totals + [3 + len(portions)] * rows, 91)
+    logits = {rid: P.forward(cfg, w, toks) for rid, toks in reqs.items()}
+    steps, pos = [], {rid: 0 for rid in reqs}
+
+    def entry(rid, n):
+        pos[rid] += n
+        return dict(id=rid, tokens=reqs[rid][pos[rid] - n:pos[rid]], want=[n - 1])
+    if rows:
+        steps.append([entry(f"r{i}", 3) for i in range(longs, longs + rows)])
+    for p in portions:
+        steps.append([entry(f"r{i}", n) for i, n in enumerate(p)] + [entry(f"r{i}", 1) for i in range(longs, longs + rows)])
+    eng = build_engine(str(tmp_path), dtype="bfloat16", device=DEV, page_size=16, num_pages=400, max_requests=rows + 3, max_model_len=2048,
+                       max_batch_tokens=2048)
+    if graphs:
+        eng.enable_graphs(True, capture_sizes=(1, 2, 37, 38, 40), mixed_tokens=1024)   # (so that the bound of the portions is two)
+    taken, rule = [], ops._scan_in_chunks
+    monkeypatch.setattr(ops, "_scan_in_chunks", lambda *a: taken.append(rule(*a)) or taken[-1])
+    results = {}
+    for i, entries in enumerate(steps):
+        results[i] = eng.step([StepEntry(e["id"], e["tokens"], e["want"]) for e in entries]).cpu().numpy()
+    steps = [dict(step=i, entries=entries, end=[]) for i, entries in enumerate(steps)]
+    check_rows(steps, results, logits, "bfloat16", f"chunks, graphs {graphs}, {rows} rows")
+    assert any(taken) and (not graphs or eng.mixed_graph_replays == len(steps))
+    if graphs:
+        assert len(eng._graphs) < len(steps)             # (some were replayed for portions they were not captured with)
