@@ -12,9 +12,9 @@
 // it is LDS (a wave of 32 x 64 results reads 6 KiB for 8 matrix instructions of 16 cycles); measured for
 // 28672 x 4096 and 128 rows: 50 us, 45 with all weights from one tile, 38 without the matrix instructions.  A
 // deeper ring for the weights alone, another first stretch for each block and loads past the caches gave nothing.
-// Measured (us, the GEMM library's kernel / this): 4096 x 14336, 96, 128, 256, 512 rows 63 75 61 92 / 28 28 39 64;
-// 4096 x 4096 20 22 22 29 / 12 13 16 24; 6144 x 4096 22 25 40 37 / 16 18 25 38; 2048 x 8192 19 20 27 34 /
-// 12 13 17 25; gate/up with SwiGLU 16384 x 2048 24 23 33 42 / 20 20 25 38, 28672 x 4096 54 58 77 108 / 48 50 74 115.
+// Measured (us, the GEMM library's kernel / this, alone, without what adds the slices up): 4096 x 14336, 96, 128, 256, 512
+// rows 63 75 61 92 / 28 28 39 64; 4096 x 4096 20 22 22 29 / 12 13 16 24; 6144 x 4096 22 25 40 37 / 16 18 25 38; 2048 x 8192
+// 19 20 27 34 / 12 13 17 25.  With what follows, and gate/up with SwiGLU: ri_gemm_mid_plan, ops._slices_pay, ops.qkv_split_pays.
 #include "common.h"
 #include <mutex>
 
@@ -98,8 +98,10 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_mid_kernel(
 #pragma unroll
             for (int j = 0; j < NTW; ++j) acc[j][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j], x[i], acc[j][i], 0, 0, 0);
     };
-    // A stage is read in two halves, each a half ahead of its matrix instructions; between them all waves meet: the
-    // stage has been read by all (its place is free for the stage ST further on), and the next one has arrived.
+    // A stage is read in two halves, each asked for ahead of the other half's matrix instructions; between them all waves
+    // meet: the stage has been read by all (its place is free for the stage ST further on), and the next one has arrived.
+    // (Only the second half's reads have instructions beside them: behind the branch for a last stage the compiled loop waits
+    // for all of LDS, so the next stage's first half is in before the second half is multiplied.)
     mbf16x8_t x0[MW], w0[NTW], x1[MW], w1[NTW];
 #pragma unroll
     for (int p = 0; p < ST; ++p)
@@ -188,37 +190,57 @@ int dispatch_mid(const bf16_t* A, int lda, const bf16_t* W, TO* C, int ldc, int 
 
 }  // namespace
 
+// What a product in `parts` slices and the kernel after it take, in us, fitted to 860 measured triples of sizes, slices and
+// widths (16 and 9 weights from 768 x 768 to 12288 x 4096, 65 to 2,048 rows, replayed in a graph; 5 % off for the norm, 11 % for
+// the rotation): a stretch of 64 values of K takes a wide block 0.48, a narrow one 0.39, or two narrow ones on a unit 0.60; the
+// chip does 256 wide blocks at once, or 512 narrow ones, as long as no XCD gets more than its share, which `across` counts (the
+// blocks of one block of columns run on one XCD: 20 of those leave four XCDs with three, so 384 rows of 2560 x 2560 in
+// four slices took two rounds, 29 us, 21 in the library); then the sums: c0 a result and c1 a result and slice,
+// and what the rotation's kernel takes to read a token's row, slice after slice.
+static float mid_time(int M, int N, int K, int parts, int wide, int rotated) {
+    const int bt = wide ? 8 : 4;
+    const long long across = ((N / 16 + bt - 1) / bt + 7) / 8 * 8, blocks = across * ((M + 127) / 128) * parts;
+    const int stretches = (K / 64 + parts - 1) / parts;
+    // (slices that make a second round never paid: 4096 x 14336 with 300 rows, 2 slices 66 us, 4 76, 8 74)
+    if (parts > 1 && blocks > (wide ? 256 : 512)) return 1e30f;
+    const float stretch = wide ? 0.48f * ((blocks + 255) / 256) : blocks <= 256 ? 0.39f : 0.60f * ((blocks + 511) / 512);
+    const float results = 1e-6f * M * N;
+    return stretch * stretches + (rotated ? results * (3.07f + 1.02f * parts) + 0.38e-3f * N * parts : results * (1.55f + 1.57f * parts));
+}
+
 // Whether and how gemm_mid takes a product of M rows, N columns (SwiGLU: of each half) and K inner values: the
 // slices of K (0: it does not) and whether a block owns 8 weight tiles or 4.  It takes what leaves the GEMM
-// library's tiles of 128 x 128 on at most half of the 256 compute units (figures at the top: with 192 such tiles
-// the library is as fast, and faster beyond), and divides K so that the blocks fill them once; a SwiGLU product,
-// whose sums cannot be divided, where its blocks fit the units once (beyond that the library is faster by more
-// than its activation kernel takes).  `any_parts`: any number of slices up to 8, else a power of two.
-extern "C" int ri_gemm_mid_plan(int M, int N, int K, int swiglu, int any_parts, int* parts_out, int* wide_out) {
+// library's tiles of 128 x 128 on at most half of the 256 compute units (with 192 such tiles the library is as fast, and
+// faster beyond), in the slices, of at least 256 values of K, that take the least time.  `rotated`: the kernel that
+// rotates adds the sums, any number of slices up to 8; else the norm does, a power of two.
+//
+// A SwiGLU product, whose sums cannot be divided, is taken where its blocks fit the units once, narrow ones if those do.
+// us, weights from memory, library with its activation kernel / narrow / wide: 2 x 8192 x 2048, 128 rows (128 wide blocks) 30 / 21 / 25;
+// 2 x 8704 x 4096, 128 rows (136) 46 / 54 / 43; 2 x 11008 x 4096, 128 rows (172) 49 / 57 / 46; 2 x 5632 x 4096, 256 rows (176) 52 / 51 / 41;
+// 2 x 14336 x 4096, 128 rows (224) 58 / 60 / 51; 2 x 9472 x 2560, 256 rows (296) 51 / 54 / 54; 2 x 8192 x 2048, 320 rows (384)
+// 34 / 41 / 41, 512 rows (512) 42 / 54 / 44.
+extern "C" int ri_gemm_mid_plan(int M, int N, int K, int swiglu, int rotated, int* parts_out, int* wide_out) {
     RI_REQUIRE(parts_out && wide_out && M > 0 && N > 0 && K > 0, "ri_gemm_mid_plan: bad arguments");
     *parts_out = 0;
     *wide_out = 1;
     if (M <= 64 || N % 16 || K % 64) return 0;
     const long long mblocks = (M + 127) / 128;
-    const long long b8 = mblocks * ((N / 16 + (swiglu ? 3 : 7)) / (swiglu ? 4 : 8));
-    const long long b4 = mblocks * ((N / 16 + (swiglu ? 1 : 3)) / (swiglu ? 2 : 4));
     if (swiglu) {
-        if (b8 > 256) return 0;
-        *wide_out = b8 >= 192;
+        auto blocks = [&](int tiles) { return ((N / 16 + tiles - 1) / tiles + 7) / 8 * 8 * mblocks; };
+        if (blocks(4) > 256) return 0;
+        *wide_out = blocks(2) > 256;
         *parts_out = 1;
         return 0;
     }
-    if (b8 > 128) return 0;
-    const int stretches = K / 64;
-    auto slices = [&](long long blocks) {
-        int p = 1;
-        for (int c = 2; c <= 8; c = any_parts ? c + 1 : 2 * c)
-            if (blocks * c <= 256 && stretches / c >= 4) p = c;
-        return p;
-    };
-    const int p8 = slices(b8), p4 = slices(b4);
-    *wide_out = !(b8 * p8 < 192 && b4 * p4 > b8 * p8);
-    *parts_out = *wide_out ? p8 : p4;
+    if (mblocks * ((N / 16 + 7) / 8) > 128) return 0;
+    float least = 0.f;
+    for (int p = 1; p <= 8; p = rotated ? p + 1 : 2 * p) {
+        if (p > 1 && K / 64 / p < 4) break;
+        for (int wide = 0; wide < 2; ++wide) {
+            const float t = mid_time(M, N, K, p, wide, rotated);
+            if (*parts_out == 0 || t < least) { least = t; *parts_out = p; *wide_out = wide; }
+        }
+    }
     return 0;
 }
 

@@ -357,10 +357,10 @@ def qkv_rope_fused(x: torch.Tensor, w_fused: torch.Tensor, qkv: torch.Tensor, H:
     return True
 
 
-def _mid_plan(M: int, N: int, K: int, swiglu: bool, any_parts: bool = False):
+def _mid_plan(M: int, N: int, K: int, swiglu: bool, rotated: bool = False):
     """(slices of K, whether blocks own 8 weight tiles) of ``ri_gemm_mid`` for this product; 0 slices: not its kind."""
     parts, wide = ctypes.c_int(0), ctypes.c_int(0)
-    _check(_lib().ri_gemm_mid_plan(M, N, K, int(swiglu), int(any_parts), ctypes.byref(parts), ctypes.byref(wide)))
+    _check(_lib().ri_gemm_mid_plan(M, N, K, int(swiglu), int(rotated), ctypes.byref(parts), ctypes.byref(wide)))
     return parts.value, wide.value
 
 

@@ -369,10 +369,10 @@ def test_linear_rows_do_not_depend_on_the_batch(ops):
     one = torch.empty(1, 257, device=DEV)
     for r in (0, 33, 69):
         ops.linear(x[r:r + 1], w, one)
-        # one row goes to the few-row kernel, 70 to the tiled one: both keep 64-bit sums, so the 32-bit
+        # one row goes to the few-row kernel, 70 to the matrix instruction: both keep 64-bit sums, so the 32-bit
         # results agree to the last bit but for a sum that lies on a rounding boundary to 1e-16
         assert torch.equal(one[0], full[r])
-    # the few-row kernel alone: 1, 5, 8, 13 and 16 rows
+    # 1, 5, 8, 13 and 16 rows: the few-row kernel and one row of tiles of 16 x 16
     x2, w2 = rnd(16, 1352, seed=13), rnd(1001, 1352, seed=14)
     all16 = torch.empty(16, 1001, device=DEV)
     ops.linear(x2, w2, all16)
@@ -382,7 +382,7 @@ def test_linear_rows_do_not_depend_on_the_batch(ops):
         sub = torch.empty(len(rows), 1001, device=DEV)
         ops.linear(x2[rows].contiguous(), w2, sub)
         assert torch.equal(sub, all16[rows])
-    # 17..64 rows: the same kernel, 16 rows a pass
+    # 17..64 rows: more rows of such tiles
     x3 = rnd(64, 1352, seed=15)
     x3[20] = x2[3]
     for M in (17, 37, 64):
@@ -397,7 +397,7 @@ def test_linear_rows_do_not_depend_on_the_batch(ops):
 @pytest.mark.parametrize("M,N,K", [(5, 16, 4), (16, 17, 60), (17, 33, 132), (31, 2064, 36), (33, 4100, 64), (49, 300, 260),
                                    (65, 47, 1352), (160, 2050, 72), (300, 515, 516), (1030, 100, 20)])
 def test_linear_f32_on_the_matrix_instruction(ops, M, N, K):
-    # edges of every tile, a last chunk of K that is not whole, fewer chunks than waves, rows inside a wider buffer
+    # edges of the tiles of 16 x 16, 32 x 16 and 16 x 32 (the larger ones: the test below), a last chunk of K that is not whole, fewer chunks than waves, rows inside a wider buffer
     xb, wb = rnd(M, K + 8, seed=M), rnd(N, K + 4, seed=N)
     x, w = xb[:, 4:K + 4], wb[:, :K]
     out = torch.full((M, N + 3), float("nan"), device=DEV)
@@ -753,7 +753,7 @@ def test_fused_projection_through_lds_from_17_tokens_and_in_wider_blocks(ops, mo
 
 @pytest.mark.parametrize("q_lens,starts,H,Hkv,hd,page,K,parts", [
     ([65], [0], 4, 2, 16, 16, 64, 1), ([40, 1, 60, 33], [5, 30, 16, 0], 8, 2, 64, 16, 1024, 4), ([129], [15], 6, 6, 48, 32, 576, 2),
-    ([1] * 70, [3] * 70, 4, 4, 32, 16, 4096, 8), ([64, 200], [0, 48], 12, 4, 128, 16, 1344, 4)])
+    ([1] * 70, [3] * 70, 4, 4, 32, 16, 4096, 8), ([64, 200], [0, 48], 12, 4, 128, 16, 1344, 2)])
 def test_projection_in_slices_rotation_and_cache_write(ops, q_lens, starts, H, Hkv, hd, page, K, parts):
     """More than 64 tokens: the product over slices of K and the kernel that adds, rotates and writes, against
     projection and rope_kv_write; whole groups of 16 values and single ones, a padding token."""
@@ -799,6 +799,33 @@ def test_products_of_some_hundred_rows(ops, M, N, K):
         ops.linear_swiglu(x, w, out, None, ops.tile_weight(w))
         want = torch.nn.functional.silu(ref[:, :I]) * ref[:, I:]
         assert torch.allclose(out.double(), want, rtol=2.0 ** -8, atol=2.0 ** -8 + 1e-5 * K ** 0.5)
+
+
+@pytest.mark.parametrize("parts,wide", [(p, w) for p in (2, 3, 5, 8) for w in (0, 1)])
+def test_slices_of_any_number_in_blocks_of_either_width(ops, monkeypatch, parts, wide):
+    """What the plan may choose for products of some hundred rows: blocks that are no whole number of rounds, a last
+    block of columns that is not whole, slices of unequal length and one without any."""
+    monkeypatch.setattr(ops, "_mid_plan", lambda *a: (parts, wide))
+    for M, N, K in ((129, 2064, 1088), (300, 720, 832), (200, 272, 576)):
+        x, w = rnd(M, K, dtype=torch.bfloat16, seed=M), rnd(N, K, dtype=torch.bfloat16, seed=N)
+        got = ops.linear_delta(x, w, Workspace(torch.device(DEV)), "t", ops.tile_weight(w))
+        assert got.shape == (parts, M, N)                          # 32-bit sums of K products of numbers around one
+        assert torch.allclose(got.double().sum(0), x.double() @ w.double().t(), rtol=0, atol=2e-6 * K ** 0.5 * 4)
+
+
+@pytest.mark.parametrize("M,N,K,rotated,plan", [
+    (256, 4096, 14336, False, (4, 1)), (384, 2560, 2560, False, (2, 0)), (100, 2048, 2048, False, (8, 0)), (256, 2048, 2048, False, (4, 0)),
+    (224, 6144, 4096, True, (2, 1)), (65, 5120, 3072, True, (3, 0)), (65, 128, 64, True, (1, 0)), (2048, 4096, 4096, False, (0, 1))])
+def test_plan_of_products_of_some_hundred_rows(ops, M, N, K, rotated, plan):
+    """The slices and widths that were fastest, or next to it, of all that were measured."""
+    assert ops._mid_plan(M, N, K, False, rotated) == plan
+
+
+@pytest.mark.parametrize("M,I,K,plan", [(128, 8192, 2048, (1, 0)), (128, 8704, 4096, (1, 1)), (128, 11008, 4096, (1, 1)), (256, 5632, 4096, (1, 1)),
+                                        (384, 5376, 2048, (0, 1)), (320, 8192, 2048, (0, 1))])
+def test_plan_of_gate_up_products(ops, M, I, K, plan):
+    """Narrow blocks where they fit the units once, wide ones where those do, each XCD taking whole columns of blocks."""
+    assert ops._mid_plan(M, I, K, True) == plan
 
 
 def _check_fused_projection(ops, B, H, Hkv, hd, page, K):
