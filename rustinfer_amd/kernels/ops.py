@@ -369,6 +369,29 @@ def _mid_ok(x: torch.Tensor, w, w_tiled) -> bool:
             and x.stride(0) % 8 == 0 and x.stride(1) == 1 and x.data_ptr() % 16 == 0 and _tiled_ok(w, w_tiled))
 
 
+def _slices_pay(M: int, N: int, K: int) -> bool:
+    """Whether ``M`` rows through slices of K and the norm that adds them up beat the GEMM library's product and the norm:
+    what the library leaves idle on few tiles lasts as long as K, what slices cost is the results' number.  us, library /
+    slices, each product of a chain of them: 1024 x 1024 512 rows 13.3 / 12.9, 768 14.2 / 14.8; 768 x 768 640 12.0 / 11.8, 1024 13.0 /
+    14.1; 4608 x 640 100 11.9 / 11.1, 160 13.1 / 13.9; 1536 x 1536 200 13.0 / 12.8, 512 15.7 / 17.2; 2048 x 2048 256 15.8 / 15.3, 512
+    18.9 / 19.7; 1024 x 4096 768 25.3 / 22.3, 1536 30.6 / 29.7; 2560 x 2560 512 26.2 / 25.1; 4096 x 14336 512 96.7 / 79.8.  In a whole
+    prompt at the 1B sizes slices gain more: with 2048 x 2048 in slices too 300 rows take 1,813 us, 700 2,629; in the library 1,858
+    and 2,658."""
+    return 4096 * M <= K * K or (K <= 1152 and M * N <= 1 << 19)
+
+
+def qkv_split_pays(M: int, N: int, K: int) -> bool:
+    """``_slices_pay`` where the kernel that rotates adds the slices up (``qkv_rope_split`` against the library's product and
+    ``rope_kv_write``), which reads them a token a block.  us: 6144 x 4096 66 rows 28.8 / 27.4, 256 46.5 / 35.0; 5120 x 3072 128
+    25.5 / 23.3, 200 25.0 / 26.4, 256 37.5 / 28.4, 384 29.5 / 30.4; 3840 x 2560 128 23.6 / 20.7, 256 23.1 / 24.1; 3072 x 2048 128
+    19.3 / 16.8, 256 18.4 / 20.5 (whole prompts at the 1B sizes: 200 rows 1,484 / 1,460, 256 1,509 / 1,515, 512 2,088 / 2,103); 2048 x 2304
+    100 13.8 / 15.3; 2048 x 1536 100 11.8 / 12.2; 1536 x 1024 200 13.0 / 12.3, 384 14.2 / 14.4; many columns for their K: 6144 x 2048
+    128 22.4 / 25.7, 7680 x 2560 128 27.9 / 31.2, 12288 x 4096 128 43.5 / 52.9."""
+    if 4 * N > 7 * K:
+        return False
+    return 10 * M <= K if K >= 3072 else M * N <= 300_000 if K <= 1024 else M <= 256 and N >= 2560
+
+
 def qkv_rope_split(x: torch.Tensor, w_fused: torch.Tensor, qkv: torch.Tensor, H: int, Hkv: int, hd: int,
                    rotary, positions: torch.Tensor, row_of_token: torch.Tensor, k_cache: torch.Tensor,
                    v_cache: torch.Tensor, block_table: torch.Tensor, page: int, workspace) -> bool:
@@ -821,7 +844,7 @@ def linear_delta(x: torch.Tensor, w: torch.Tensor, workspace, name: str,
                                            _ptr(stack), N, M, N, K, F32, 0, parts, ctypes.c_longlong(M * N),
                                            int(tiled), ctypes.c_void_p(0), 0, ctypes.c_float(0.0), _stream()))
             return stack
-    if _mid_ok(x, w, w_tiled):
+    if _mid_ok(x, w, w_tiled) and _slices_pay(M, N, K):
         # more rows than that, but too few tiles for the chip: slices of K again
         parts, wide = _mid_plan(M, N, K, False)
         if parts > 1:

@@ -108,7 +108,9 @@ class PagedAttention(Mixer):
             args = (rows, self.qkv_fused, qkv, self.num_heads, self.num_kv_heads, self.head_dim, rotary,
                     ctx.positions, ctx.row_of_token, cache.k, cache.v, table, cache.page_size)
             split = getattr(ops, "qkv_rope_split", None)
-            fused = ops.qkv_rope_fused(*args, **kw) or (scale is None and split is not None and split(*args, ws))
+            fused = ops.qkv_rope_fused(*args, **kw) or (
+                scale is None and split is not None
+                and ops.qkv_split_pays(rows.shape[0], self.qkv_fused.shape[0], self.qkv_fused.shape[1]) and split(*args, ws))
         if not fused:
             self.qkv.forward(rows, qkv, scale)
             if self.qk_transform is not None:

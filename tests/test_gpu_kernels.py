@@ -806,6 +806,7 @@ def test_slices_of_any_number_in_blocks_of_either_width(ops, monkeypatch, parts,
     """What the plan may choose for products of some hundred rows: blocks that are no whole number of rounds, a last
     block of columns that is not whole, slices of unequal length and one without any."""
     monkeypatch.setattr(ops, "_mid_plan", lambda *a: (parts, wide))
+    monkeypatch.setattr(ops, "_slices_pay", lambda *a: True)
     for M, N, K in ((129, 2064, 1088), (300, 720, 832), (200, 272, 576)):
         x, w = rnd(M, K, dtype=torch.bfloat16, seed=M), rnd(N, K, dtype=torch.bfloat16, seed=N)
         got = ops.linear_delta(x, w, Workspace(torch.device(DEV)), "t", ops.tile_weight(w))
@@ -819,6 +820,14 @@ def test_slices_of_any_number_in_blocks_of_either_width(ops, monkeypatch, parts,
 def test_plan_of_products_of_some_hundred_rows(ops, M, N, K, rotated, plan):
     """The slices and widths that were fastest, or next to it, of all that were measured."""
     assert ops._mid_plan(M, N, K, False, rotated) == plan
+
+
+def test_where_slices_pay(ops):
+    """Sizes on both sides of each line."""
+    assert all(ops._slices_pay(*a) for a in ((512, 1024, 1024), (113, 4608, 640), (700, 2048, 2048), (2048, 896, 4864)))
+    assert not any(ops._slices_pay(*a) for a in ((768, 1024, 1024), (160, 4608, 640), (640, 1536, 1536), (1025, 2048, 2048)))
+    assert all(ops.qkv_split_pays(*a) for a in ((256, 6144, 4096), (307, 5120, 3072), (256, 3072, 2048), (195, 1536, 1024)))
+    assert not any(ops.qkv_split_pays(*a) for a in ((384, 5120, 3072), (257, 3072, 2048), (100, 2048, 2304), (300, 1536, 1024), (128, 6144, 2048), (100, 12288, 4096)))
 
 
 @pytest.mark.parametrize("M,I,K,plan", [(128, 8192, 2048, (1, 0)), (128, 8704, 4096, (1, 1)), (128, 11008, 4096, (1, 1)), (256, 5632, 4096, (1, 1)),
