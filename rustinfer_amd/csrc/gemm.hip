@@ -212,7 +212,7 @@ struct VecLoad4 {       // four consecutive outputs of a lane in one store
 // memory system serves about a third faster than 64-byte pieces of 16 rows.  The copy is made
 // once when the weights are loaded (N % 16 == 0 and K % 32 == 0).
 //
-// ROPE: the product is the fused q/k/v projection of single tokens and the kernel finishes what
+// ROPE: the product is the fused q/k/v projection of a step's tokens and the kernel finishes what
 // would otherwise be a kernel of its own: it rotates q and k by the token's position and writes
 // k and v into the token's cache page; only q goes to C.  For that the rows of W are permuted
 // within each head (qkv_rope_row_order below) so that a tile holds 8 features of the first half
@@ -698,7 +698,7 @@ static int row_scale(const float* ssq, int ssq_parts, float eps, int K, RowScale
     return 0;
 }
 
-// q/k/v projection of M <= 64 single tokens with rotation and cache write fused (see RopeEpilogue).
+// q/k/v projection of M <= 64 tokens, of any rows of the step, with rotation and cache write fused (see RopeEpilogue).
 // W: the row-permuted weight in tile order.  C [M, ldc]: receives rotated q in its first H*hd columns.
 extern "C" int ri_gemm_qkv_rope(const void* A, int lda, const void* W, void* C, int ldc, int M, int K,
                                 int H, int Hkv, int hd, const float* cos_t, const float* sin_t, int table_rows,

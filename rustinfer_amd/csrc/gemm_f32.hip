@@ -5,8 +5,10 @@
 //
 // The instruction is slow next to what feeds it: a wave that owns 64 x 64 results asks for 8 KiB in
 // 4,096 cycles.  So nothing passes through LDS on the way in: every lane reads 16 bytes of K of its row
-// of A and of W straight into registers, a chunk ahead of the one that is multiplied, and the four
-// steps of such 16 bytes take the K values {4g + s} of the four lane groups g, for A and W alike.  The
+// of A and of W straight into registers, and the four
+// steps of such 16 bytes take the K values {4g + s} of the four lane groups g, for A and W alike.  (A chunk is asked for
+// before the one ahead of it is multiplied, but under conditions of the lanes, for which the compiled loop waits for
+// every load before it multiplies: what covers a trip to memory is the unit's other waves.)  The
 // waves of a block share one tile of results and take 32 values of K in turn, whatever the tile; their 64-bit sums meet in
 // LDS once, in the order of the waves, so a row's result does not depend on the other rows or on the tile.  (Products
 // of up to four rows, gemm_rows_f32, add in another order: the same to the rounding of a 64-bit sum.)

@@ -48,7 +48,7 @@ __device__ __forceinline__ int lds_unit(int ks, int mt, int g, int c) {
     return ((ks * MT + mt) * 4 + g) * 16 + (c ^ ((4 * ks + g) & 15));
 }
 
-// ROPE: the product is the fused q/k/v projection of single tokens, with the weight's rows permuted
+// ROPE: the product is the fused q/k/v projection of a step's tokens, with the weight's rows permuted
 // within each head as for the few-row kernel (gemm.hip, ri_qkv_rope_row_order): a tile holds 8
 // features of the first half of a head and their 8 partners, the partner of a lane's value sits in
 // lane ^ 32.  The epilogue rotates q and k by the token's position (32-bit, one rounding), writes
@@ -427,7 +427,7 @@ extern "C" int ri_gemm_rows_bf16(const void* A, int lda, const void* W, void* C,
     return 0;
 }
 
-// The q/k/v projection of 17..64 single tokens with rotation and cache write in the epilogue, as
+// The q/k/v projection of 17..64 tokens with rotation and cache write in the epilogue, as
 // ri_gemm_qkv_rope (gemm.hip) does it for fewer rows: W is the same row-permuted weight in tile
 // order, C [M, ldc] receives rotated q in its first H * hd columns.  Measured at 64 rows against
 // the few-row kernel (product alone, us): 6144 x 4096 25.9 -> 21.5, 5120 x 3072 21.1 -> 16.5,
