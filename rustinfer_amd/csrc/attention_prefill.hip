@@ -597,6 +597,9 @@ __global__ __launch_bounds__(256) void attn_prefill_combine_kernel(
 // head 128: 16 tokens behind 2,048: 40 -> 20; 256 behind 8,192: 142 -> 63; 512 behind 7,680: 139 -> 88 (one head
 // a wave: 104); 512 behind 1,536 stays undivided (40; 44).  head 64: 128 behind 2,048: 27 -> 19; 512 behind 8,192:
 // 94 -> 61.
+// Of several rows only some may have the long prefix, and their waves are what walks it: as many ranges as the longest row's
+// waves allow, up to 4,096 / w1.  us, ranges by w1 alone -> now: 24 heads of 128, five rows of 100, two behind 8,722 and 2,424, 99 -> 59;
+// 14 heads of 64, rows of 769 and 893, the second behind 11,976, 164 -> 138; 32 heads of 64, five rows of 361, one behind 4,150, 88 -> 83.
 //
 // Undivided, pages of 16 without a window (blocks that share keys and values through LDS).  us, one head a wave in
 // pairs of tiles (what ran before where nothing else is said) -> now:
@@ -638,6 +641,8 @@ static PrefillPlan prefill_plan(int H, int Hkv, int hd, int page, int window, in
         const long long two = even && prefix >= 4LL * total_q ? std::min<long long>(4096 / w1, 32) : 0;
         long long n = std::max(std::min<long long>(2048 / w1, prefix / 512), std::min<long long>(1024 / w1, prefix / 256));
         if (two >= 2 && prefix >= 1024 * two) { n = two; p.heads = 2; }
+        // of several rows some may start their prompts: the long prefix is then walked by the waves of its row only
+        else if (longest_q < total_q) n = std::max(n, std::min({2048 / (((longest_q + 63) / 64) * 4LL * H), 4096 / w1, prefix / 512LL}));
         if (forced > 1) n = forced;
         n = std::min<long long>(n, 32);
         if (n >= 2) {
@@ -660,10 +665,10 @@ static PrefillPlan prefill_plan(int H, int Hkv, int hd, int page, int window, in
 }
 
 // bytes of workspace ri_attention_prefill may use for a step of total_q tokens whose rows hold at
-// most max_kv_len keys (0: it will not divide the keys)
+// most max_kv_len keys, however long each row is (the shorter the longest, the more ranges); 0: it will not divide the keys
 extern "C" size_t ri_attention_prefill_workspace(int H, int Hkv, int hd, int page, int window, int total_q,
                                                  int max_prefix, int max_kv_len, int splits) {
-    const int n = prefill_plan(H, Hkv, hd, page, window, total_q, total_q, max_prefix, max_kv_len, splits).nsplit;
+    const int n = prefill_plan(H, Hkv, hd, page, window, total_q, std::min(total_q, 1), max_prefix, max_kv_len, splits).nsplit;
     return n < 2 ? 0 : (size_t)n * total_q * H * (hd + 2) * sizeof(float);
 }
 

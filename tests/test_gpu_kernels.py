@@ -631,6 +631,7 @@ RANGE_CASES = [
     ((2, 4, 1, 128, 16, [130, 64], [1000, 129]), 5),             # a tile of queries that begins in one range and ends in the next
     ((2, 4, 1, 128, 16, [130, 64], [1000, 129]), 2),
     ((1, 8, 8, 64, 16, [1000], [0]), 4),                         # from the first token: ranges that the early tiles never reach
+    ((3, 24, 8, 128, 16, [300, 300, 200], [2100, 0, 17]), 0),    # waves enough but for the one row behind many keys: three ranges
     ((2, 6, 2, 128, 16, [3, 259], [381, 250]), 2),               # a range's edge (256) inside a portion, odd lengths
 ]
 
