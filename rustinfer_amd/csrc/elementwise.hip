@@ -600,8 +600,9 @@ extern "C" int ri_swiglu(const void* gate_up, void* out, int act_dtype, int T, i
 // out[t, i] = f(in[t, i]) over n columns of rows with strides of their own (columns of a wider
 // buffer; in place where out == in).  f: 0 = relu(z)^2, 1 = tanh(z); 32-bit arithmetic.
 // unary_bf16x8: 16 bytes a thread, where rows begin at multiples of that and hold whole ones and there are a block's worth for
-// every compute unit; bound by memory then, where two bytes a thread are bound by the number of waves (2,048 rows of
-// 8,192: 31.3 us -> 13.2; 8 rows take 4.7 either way, and stay with the waves of the plain form).
+// every compute unit (tanh, whose eight a thread are a chain of their own: four); bound by memory then, where two bytes a thread are bound by the number of waves (2,048 rows of
+// 8,192: 31.3 us -> 13.2; 8 rows take 4.7 either way, and stay with the waves of the plain form; tanh of 2,103 rows of 2,048
+// 10.4 -> 7.2, of 57 rows of 11,264 3.1 -> 3.8).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float unary_of(float z, int op) {
     if (op != 0) return tanhf(z);
@@ -638,7 +639,7 @@ extern "C" int ri_unary(const void* in, int in_stride, void* out, int out_stride
     RI_REQUIRE(in && out, "ri_unary: null pointer");
     RI_REQUIRE(T <= 65535, "ri_unary: too many rows for the grid");
     dim3 grid((n + 255) / 256, T);
-    const bool vec = dtype == RI_BF16 && (long long)T * n >= 256 * 256 * 8 && n % 8 == 0 && in_stride % 8 == 0 && out_stride % 8 == 0 && ((uintptr_t)in | (uintptr_t)out) % 16 == 0;
+    const bool vec = dtype == RI_BF16 && (long long)T * n >= (op == 0 ? 1 : 4) * 256 * 256 * 8 && n % 8 == 0 && in_stride % 8 == 0 && out_stride % 8 == 0 && ((uintptr_t)in | (uintptr_t)out) % 16 == 0;
     if (vec) unary_bf16x8_kernel<<<dim3((n / 8 + 255) / 256, T), 256, 0, stream>>>((const bf16_t*)in, in_stride, (bf16_t*)out, out_stride, n, op);
     else if (dtype == RI_F32) unary_kernel<float><<<grid, 256, 0, stream>>>((const float*)in, in_stride, (float*)out, out_stride, n, op);
     else if (dtype == RI_BF16) unary_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)in, in_stride, (bf16_t*)out, out_stride, n, op);
