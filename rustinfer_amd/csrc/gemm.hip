@@ -92,8 +92,8 @@ extern "C" int ri_gemm_tiled(const void* A, int lda, const void* W, int ldw, voi
 // a fixed order and the lanes are added in a fixed tree, so a row's result depends neither on the
 // other rows nor on their number.  K % 4 == 0.  Measured, us, 4 rows, this kernel / gemm_f32:
 // 2048 x 8192 24 / 34; 4096 x 14336 53 / 59; 128256 x 2048 187 / 221; 16384 x 2048 37 / 32; at 6 rows
-// 32 / 34, 64 / 60, 288 / 236, 45 / 33, and 6144 x 4096 29 / 36 (of 22 such sizes of 5 to 16 rows the one where it is slower by more
-// than a tenth; the others take 0.32 to 0.96 of the time).
+// 32 / 34, 64 / 60, 288 / 236, 45 / 33, and 6144 x 4096 29 / 36 (of 45 products of 5 to 16 rows drawn at random, the two of that
+// size are slower; the others take 0.31 to 1.01 of the time that this kernel took with more rows).
 // ---------------------------------------------------------------------------
 template <int MR, int NB>
 __global__ __launch_bounds__(256) void gemm_rows_f32_kernel(
