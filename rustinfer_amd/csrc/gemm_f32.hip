@@ -6,19 +6,23 @@
 // The instruction is slow next to what feeds it: a wave that owns 64 x 64 results asks for 8 KiB in
 // 4,096 cycles.  So nothing passes through LDS on the way in: every lane reads 16 bytes of K of its row
 // of A and of W straight into registers, and the four
-// steps of such 16 bytes take the K values {4g + s} of the four lane groups g, for A and W alike.  (A chunk is asked for
-// before the one ahead of it is multiplied, but under conditions of the lanes, for which the compiled loop waits for
-// every load before it multiplies: what covers a trip to memory is the unit's other waves.)  The
+// steps of such 16 bytes take the K values {4g + s} of the four lane groups g, for A and W alike.  A chunk is asked for
+// two ahead of the one that is multiplied; nothing on that way depends on the lane, so the compiled loop waits for a
+// chunk's own loads only.  The
 // waves of a block share one tile of results and take 32 values of K in turn, whatever the tile; their 64-bit sums meet in
-// LDS once, in the order of the waves, so a row's result does not depend on the other rows or on the tile.  (Products
-// of up to four rows, gemm_rows_f32, add in another order: the same to the rounding of a 64-bit sum.)
+// LDS once, in the order of the waves, so a row's result does not depend on the other rows or on the tile.
 // Blocks of one column tile run on one XCD (consecutive block ids go around the eight of them), so a
 // tile's weights pass through one L2.  K % 4 == 0, rows 16-byte aligned.
 //
-// Against the FMA kernels with 64-bit sums that were here before, us: 600 rows of 2048 x 8192 1451 -> 366
-// (55 TFLOP/s), 256 rows of 16384 x 2048 596 -> 308, 100 rows of 2048 x 2048 296 -> 27, 64 rows of
-// 28672 x 4096 801 -> 275, 16 rows of 16384 x 2048 76 -> 41, 8 rows 47 -> 35 (134 MB: 20 at 6.9 TB/s).
+// What is left to bound the large products: other instructions hold the 64-bit matrix instruction up (a loop of it alone reaches 72
+// TFLOP/s on random operands, one with the widening of one operand value an instruction, as in tiles of 32 x 32, 61),
+// and that is what they take.  Loads waited for under conditions of the lanes before, now, us: 600 rows of 16384 x 2048 707, 662
+// (61 TFLOP/s), of 2048 x 8192 364, 333, of 2048 x 2048 100, 93; 230 rows 268, 250 / 154, 137 / 44, 39; 37 rows of
+// 16384 x 2048 67, 60; 13 rows 43, 37.  (As FMA kernels with 64-bit sums: 600 rows of 2048 x 8192 1451.)
 #include "common.h"
+
+extern "C" int ri_gemm_tiled(const void* A, int lda, const void* W, int ldw, void* C, int ldc,
+                             int M, int N, int K, int in_dtype, int out_dtype, hipStream_t stream);      // gemm.hip
 
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
@@ -26,40 +30,52 @@ typedef double f64x4_t __attribute__((ext_vector_type(4)));
 // after the other, are a wave's turn of 32).
 // STREAM: W is read once (a single row of tiles), past the caches.
 template <int MT, int NT, int WAVES, int U, bool STREAM>
-__global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(
+__global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
         const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
         float* __restrict__ C, int ldc, int M, int N, int K, int mtiles, int ntiles) {
-    constexpr int KC = 16 * U, TURN = WAVES * 32, K1 = U == 1 ? KC : TURN, K2 = U == 1 ? TURN : 2 * TURN;
+    constexpr int KC = 16 * U, TURN = WAVES * 32;
     static_assert(U == 1 || U == 2, "a wave's turn of K is 32 values");
     __shared__ double sums[WAVES][16][NT * 16];
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
     const int xcd = (int)blockIdx.x & 7, turn = (int)blockIdx.x >> 3;
     const int nt = (turn / mtiles) * 8 + xcd, mt = turn % mtiles;
     if (nt >= ntiles) return;
     const int m0 = mt * MT * 16, n0 = nt * NT * 16;
-    const float* arow[MT];
-    const float* wrow[NT];
+    // the block's first rows, the same in all lanes, and each lane's rows as 32-bit distances in bytes from there
+    const char* abase = reinterpret_cast<const char*>(A + (size_t)m0 * lda);
+    const char* wbase = reinterpret_cast<const char*>(W + (size_t)n0 * ldw);
+    uint32_t arow[MT], wrow[NT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) arow[i] = A + (size_t)min(m0 + i * 16 + r, M - 1) * lda + 4 * g;
+    for (int i = 0; i < MT; ++i) arow[i] = ((uint32_t)min(i * 16 + r, M - 1 - m0) * (uint32_t)lda + 4 * g) * 4;
 #pragma unroll
-    for (int j = 0; j < NT; ++j) wrow[j] = W + (size_t)min(n0 + j * 16 + r, N - 1) * ldw + 4 * g;
+    for (int j = 0; j < NT; ++j) wrow[j] = ((uint32_t)min(j * 16 + r, N - 1 - n0) * (uint32_t)ldw + 4 * g) * 4;
+    auto of_a = [&](int i, int k) { return *reinterpret_cast<const float4*>(abase + (size_t)k * 4 + arow[i]); };
+    auto of_w = [&](int j, int k) {
+        const char* p = wbase + (size_t)k * 4 + wrow[j];
+        return STREAM ? ld_stream16<float4>(p) : *reinterpret_cast<const float4*>(p);
+    };
     f64x4_t acc[MT][NT] = {};
-    auto ask = [&](int k0, float4 (&a)[U][MT], float4 (&w)[U][NT]) {
-        const bool whole = k0 + KC <= K;
+    auto at = [&](int step) { return wave * 32 + (U == 2 ? step * TURN : (step >> 1) * TURN + (step & 1) * KC); };
+    // a whole chunk: no condition of the lanes, so that the loads stay in flight while the chunk ahead is multiplied
+    auto ask = [&](int step, float4 (&a)[U][MT], float4 (&w)[U][NT]) {
+        const int k0 = at(step);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = k0 + 16 * u;
-            const bool in = whole || k + 4 * g < K;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) {
-                w[u][j] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (in) w[u][j] = STREAM ? ld_stream16<float4>(wrow[j] + k) : *reinterpret_cast<const float4*>(wrow[j] + k);
-            }
+            for (int j = 0; j < NT; ++j) w[u][j] = of_w(j, k0 + 16 * u);
 #pragma unroll
-            for (int i = 0; i < MT; ++i) {
-                a[u][i] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (in) a[u][i] = *reinterpret_cast<const float4*>(arow[i] + k);
-            }
+            for (int i = 0; i < MT; ++i) a[u][i] = of_a(i, k0 + 16 * u);
+        }
+    };
+    auto ask_part = [&](int step, float4 (&a)[U][MT], float4 (&w)[U][NT]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = at(step) + 16 * u;
+            const bool in = k + 4 * g < K;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) w[u][j] = in ? of_w(j, k) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+            for (int i = 0; i < MT; ++i) a[u][i] = in ? of_a(i, k) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     };
     auto add = [&](const float4 (&a)[U][MT], const float4 (&w)[U][NT]) {
@@ -78,17 +94,40 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(
                     for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i], y[j], acc[i][j], 0, 0, 0);
             }
     };
+    // whole chunks of this wave: step s is whole if at(s) + KC <= K
+    int whole = 0;
+    const int left = K - wave * 32;
+    if (U == 2) whole = left >= 32 ? (left - 32) / TURN + 1 : 0;
+    else whole = left < 16 ? 0 : left / TURN * 2 + (left % TURN >= 32 ? 2 : left % TURN >= 16 ? 1 : 0);
     float4 a0[U][MT], w0[U][NT], a1[U][MT], w1[U][NT];
-    int k = wave * 32;
-    if (k < K) ask(k, a0, w0);
-    for (; k < K; k += K2) {
-        const int k1 = k + K1, k2 = k + K2;
-        if (k1 < K) ask(k1, a1, w1);
-        add(a0, w0);
-        if (k1 < K) {
-            if (k2 < K) ask(k2, a0, w0);
+    // One way into the loop, both chunks asked for: at a place that can be reached with fewer loads under way, the compiled
+    // code would wait for more of them.  The scheduler's barriers keep the second chunk's conversions, and so the wait for it,
+    // behind the first's products.
+    if (whole >= 2) {
+        int step = 0;
+        ask(0, a0, w0);
+        ask(1, a1, w1);
+        for (; step + 4 <= whole; step += 2) {
+            add(a0, w0);
+            ask(step + 2, a0, w0);
+            __builtin_amdgcn_sched_barrier(0);
             add(a1, w1);
+            ask(step + 3, a1, w1);
+            __builtin_amdgcn_sched_barrier(0);
         }
+        add(a0, w0);                             // two or three are left
+        if (step + 2 < whole) ask(step + 2, a0, w0);
+        __builtin_amdgcn_sched_barrier(0);
+        add(a1, w1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (step + 2 < whole) add(a0, w0);
+    } else if (whole == 1) {
+        ask(0, a0, w0);
+        add(a0, w0);
+    }
+    if (at(whole) < K) {                         // and perhaps a part of one
+        ask_part(whole, a0, w0);
+        add(a0, w0);
     }
     // result (row 4 i + g, column r) of a tile lies in element i of lane 16 g + r
 #pragma unroll
@@ -107,6 +146,114 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_f32_kernel(
             const int m = m0 + i * 16 + row, n = n0 + col;
             if (m < M && n < N) C[(size_t)m * ldc + n] = (float)v;
         }
+    }
+}
+
+// Up to eight rows: a tile of the instruction holds eight rows and eight columns of W twice, once for each of two turns of K.
+// Lanes r < 8 of A and W hold the values of K of wave w, lanes r >= 8 those of wave w + 4, so the tile's upper left
+// quarter is the one wave's sum and the lower right the other's (the other two are not read): four waves do what the eight of
+// the kernel above do, in the same order, and a block takes 8 NT columns, so that a product of 2,048 columns gives every
+// compute unit a block and no lane loads what another has.  D turns of each wave are under way at a time.  What bounds it is the
+// one pass over W.  Measured, us, 6 rows, tiles of 16 rows (half of them no row of the product) with loads that the compiled loop waited for / this
+// kernel: 2048 x 2048 10.3 / 6.7, 3072 x 2048 10.8 / 10.2, 16384 x 2048 41 / 31 (134 MB: 4.3 TB/s),
+// 2048 x 8192 33 / 17.6, 128256 x 2048 264 / 193 (5.4 TB/s).  Four rows, against FMAs with the lanes' sums added up in a tree: 3072 x 2048
+// 11.5 / 9.9, 16384 x 2048 36 / 30, 2048 x 8192 23.5 / 17.1, 28672 x 4096 100 / 87, 4096 x 14336 53 / 55, 128256 x 2048 182 / 188.
+template <int NT, int D>
+__global__ __launch_bounds__(256) void gemm_f32_few_kernel(
+        const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
+        float* __restrict__ C, int ldc, int M, int N, int K) {
+    constexpr int TURN = 256;
+    __shared__ double sums[8][8][NT * 8];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    const int r = lane & 7, second = (lane >> 3) & 1, g = lane >> 4;
+    const int n0 = (int)blockIdx.x * NT * 8;
+    const char* abase = reinterpret_cast<const char*>(A + wave * 32);
+    const char* wbase = reinterpret_cast<const char*>(W + (size_t)n0 * ldw + wave * 32);
+    const int kl = second * 128 + 4 * g;
+    const uint32_t arow = ((uint32_t)min(r, M - 1) * (uint32_t)lda + kl) * 4;
+    uint32_t wrow[NT];
+#pragma unroll
+    for (int j = 0; j < NT; ++j) wrow[j] = ((uint32_t)min(j * 8 + r, N - 1 - n0) * (uint32_t)ldw + kl) * 4;
+    f64x4_t acc[NT] = {};
+    auto ask = [&](int turn, float4 (&a)[2], float4 (&w)[2][NT]) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const size_t at = ((size_t)turn * TURN + 16 * u) * 4;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) w[u][j] = ld_stream16<float4>(wbase + at + wrow[j]);
+            a[u] = *reinterpret_cast<const float4*>(abase + at + arow);
+        }
+    };
+    auto add = [&](const float4 (&a)[2], const float4 (&w)[2][NT]) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int s = 0; s < 4; ++s) {
+                const double x = (double)(s == 0 ? a[u].x : s == 1 ? a[u].y : s == 2 ? a[u].z : a[u].w);
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    const double y = (double)(s == 0 ? w[u][j].x : s == 1 ? w[u][j].y : s == 2 ? w[u][j].z : w[u][j].w);
+                    acc[j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x, y, acc[j], 0, 0, 0);
+                }
+            }
+    };
+    // turns that are whole for both halves of the lanes
+    const int left = K - wave * 32 - 160;
+    const int whole = left >= 0 ? left / TURN + 1 : 0;
+    float4 a[D][2], w[D][2][NT];
+    if (whole >= D) {
+        int turn = 0;
+#pragma unroll
+        for (int d = 0; d < D; ++d) ask(d, a[d], w[d]);
+        for (; turn + 2 * D <= whole; turn += D) {
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                add(a[d], w[d]);
+                ask(turn + d + D, a[d], w[d]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+        }
+        const int more = whole - turn - D;       // of the next D turns, so many are there
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            add(a[d], w[d]);
+            if (d < more) ask(turn + d + D, a[d], w[d]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (d < more) add(a[d], w[d]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else {
+        for (int turn = 0; turn < whole; ++turn) {
+            ask(turn, a[0], w[0]);
+            add(a[0], w[0]);
+        }
+    }
+    if (wave * 32 + whole * TURN < K) {          // a turn that ends within the lanes' chunks, or before the second half's
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const bool in = wave * 32 + whole * TURN + 16 * u + kl < K;
+            const size_t at = ((size_t)whole * TURN + 16 * u) * 4;
+#pragma unroll
+            for (int j = 0; j < NT; ++j)
+                w[0][u][j] = in ? *reinterpret_cast<const float4*>(wbase + at + wrow[j]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            a[0][u] = in ? *reinterpret_cast<const float4*>(abase + at + arow) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        add(a[0], w[0]);
+    }
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int e = 0; e < 2; ++e) sums[wave + 4 * second][4 * e + g][j * 8 + r] = second ? acc[j][2 + e] : acc[j][e];
+    __syncthreads();
+    for (int e = threadIdx.x; e < 8 * NT * 8; e += 256) {
+        const int row = e / (NT * 8), col = e % (NT * 8);
+        double v = sums[0][row][col];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) v += sums[i][row][col];
+        if (row < M && n0 + col < N) C[(size_t)row * ldc + n0 + col] = (float)v;
     }
 }
 
@@ -146,7 +293,8 @@ static void launch_f32(const float* A, int lda, const float* W, int ldw, float* 
     }
 }
 
-// The rows and columns of the tile that ri_gemm_f32 takes for M rows and N columns.
+// The rows and columns of the tile that ri_gemm_f32 takes for M rows and N columns (of gemm_f32_kernel: up to eight rows, the tiles
+// of gemm_f32_few_kernel hold eight).
 extern "C" void ri_gemm_f32_tile(int M, int N, int* rows, int* columns) {
     const F32Tile& t = F32_TILES[f32_tile(M, N)];
     *rows = 16 * t.mt;
@@ -160,6 +308,18 @@ extern "C" int ri_gemm_f32(const float* A, int lda, const float* W, int ldw, flo
     RI_REQUIRE(lda >= K && ldw >= K && ldc >= N && lda % 4 == 0 && ldw % 4 == 0, "ri_gemm_f32: leading dimensions must be >= K and multiples of 4");
     RI_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0, "ri_gemm_f32: null or unaligned pointer");
     RI_REQUIRE(N <= (1 << 26), "ri_gemm_f32: N=%d exceeds the grid limit", N);
+    // lanes find their rows by 32-bit distances in bytes from the first of up to 48
+    if (lda > (1 << 24) || ldw > (1 << 24)) return ri_gemm_tiled(A, lda, W, ldw, C, ldc, M, N, K, RI_F32, RI_F32, stream);
+    if (M <= 8) {
+        // Columns a block, turns under way a wave.  Measured, us, 6 rows, 8 columns and 4 turns / 16 and 4 / 24 and 1:
+        // 2048 x 2048 6.7 / 10.1 / -, 3072 x 2048 10.2 / 10.4 / 12.2, 2048 x 8192 17.6 / 27 / -, 16384 x 2048 33 / 31 / 32, 128256 x 2048
+        // 241 / 205 / 193; 4 rows: 4096 x 14336 55 / 52 / 70, 28672 x 4096 91 / 101 / 87; 1 row: 4096 x 4096 14.5 / 18.9 / 19.9.
+        if (N <= 4096) gemm_f32_few_kernel<1, 4><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+        else if (N < 24576) gemm_f32_few_kernel<2, 4><<<(N + 15) / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+        else gemm_f32_few_kernel<3, 1><<<(N + 23) / 24, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+        RI_LAUNCHED("ri_gemm_f32");
+        return 0;
+    }
     switch (f32_tile(M, N)) {
         case 0: launch_f32<2, 2, 2>(A, lda, W, ldw, C, ldc, M, N, K, stream); break;
         case 1: launch_f32<3, 2, 1>(A, lda, W, ldw, C, ldc, M, N, K, stream); break;

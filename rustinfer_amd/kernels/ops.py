@@ -658,7 +658,6 @@ QKV_ROPE_LDS_MIN_COLUMNS = 4096 # ... and columns (128 blocks of 32; in a step o
 QKV_ROPE_LDS_LARGE = 40 << 20   # ... and from 17 tokens on where the weight has this many elements (product alone at 24
                                 # rows, us: 12288 x 4096 27.3 -> 23.5, 15360 x 5120 35.9 -> 28.8, 10240 x 8192 49.0 -> 42.4;
                                 # 6144 x 4096 15.4 -> 16.3, 5120 x 3072 12.5 -> 12.5)
-F32_ROWS_MAX = 4                # the exact path's kernel without matrix instructions; from 5 rows on their 16 rows pay
 ROWS_LDS_MIN_ROWS = 17          # from here to 64 rows, products whose partial sums a norm adds up take the LDS kernel
 ROWS_LDS_WIDE_COLUMNS = 16384   # whole products (no slices of K) take it from this many columns on: the output head, 250 -> 205 us at 64 rows
 ROWS_LDS_SWIGLU_MIN_ROWS = 33   # the fused gate/up product only with more rows, and with columns enough for its blocks
@@ -804,9 +803,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: Optiona
                     return
     if x.dtype == torch.float32 and out.dtype == torch.float32 and K % 4 == 0 and x.stride(0) % 4 == 0 \
             and w.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
-        # the exact path: 64-bit sums, weights streamed once for few rows, the 64-bit matrix instruction for more
-        kernel = lib.ri_gemm_rows_f32 if M <= F32_ROWS_MAX else lib.ri_gemm_f32
-        _check(kernel(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), M, N, K, _stream()))
+        # the exact path: 64-bit sums on the 64-bit matrix instruction
+        _check(lib.ri_gemm_f32(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), M, N, K, _stream()))
         return
     _check(lib.ri_gemm_tiled(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0),
                              M, N, K, _dt(x), _dt(out), _stream()))

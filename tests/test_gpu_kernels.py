@@ -369,8 +369,7 @@ def test_linear_rows_do_not_depend_on_the_batch(ops):
     one = torch.empty(1, 257, device=DEV)
     for r in (0, 33, 69):
         ops.linear(x[r:r + 1], w, one)
-        # one row goes to the few-row kernel, 70 to the matrix instruction: both keep 64-bit sums, so the 32-bit
-        # results agree to the last bit but for a sum that lies on a rounding boundary to 1e-16
+        # one row and 70 take tiles of other sizes: the sums are made in one order
         assert torch.equal(one[0], full[r])
     # 1, 5, 8, 13 and 16 rows: the few-row kernel and one row of tiles of 16 x 16
     x2, w2 = rnd(16, 1352, seed=13), rnd(1001, 1352, seed=14)
@@ -431,6 +430,44 @@ def test_linear_f32_gives_a_row_the_same_bits_on_every_tile(ops):
         ref = x[:rows].double() @ w.double().t()                   # K products in 64 bits, added in another order
         assert torch.all((out.double() - ref).abs() <= ref.abs() * 2.0 ** -24 + K * 2.0 ** -52 * (x[:rows].double().abs() @ w.double().abs().t()))
     assert tiles == {(16, 16), (32, 16), (16, 32), (32, 32), (48, 32)}
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 1, 4), (8, 7, 28), (3, 9, 32), (7, 17, 124), (5, 8, 128), (2, 33, 132), (8, 4097, 160), (6, 4096, 164), (4, 24577, 256),
+                                   (7, 24599, 292), (8, 40, 1020), (1, 25, 1024), (6, 4111, 1056), (5, 4100, 1284), (8, 24600, 548), (3, 300, 2316)])
+def test_linear_f32_of_up_to_eight_rows(ops, M, N, K):
+    # 8, 16 and 24 columns a block and their edges; K below, at and past a half's and a turn's chunks, with fewer turns than
+    # are under way, as many, and more; the last row of x not finite, which only its own results may show
+    xb, wb = rnd(M + 1, K + 8, seed=M), rnd(N, K + 4, seed=N)
+    x, w = xb[:M, 4:K + 4], wb[:, :K]
+    out = torch.full((M, N + 3), float("nan"), device=DEV)
+    ops.linear(x, w, out[:, :N])
+    ref = x.double() @ w.double().t()
+    # a 64-bit sum rounded once: half a unit of the last place of each result
+    assert torch.all((out[:, :N].double() - ref).abs() <= ref.abs() * 2.0 ** -24 + 1e-12 * ref.abs().max())
+    assert torch.all(torch.isnan(out[:, N:]))
+    more = torch.empty(9, N, device=DEV)               # nine rows: tiles of sixteen, the same sums in the same order
+    ops.linear(torch.cat([x, rnd(9 - M, K, seed=5)]), w, more)
+    assert torch.equal(more[:M], out[:, :N])
+    if M > 1:
+        y = x.clone()
+        y[M - 1, K // 2] = float("inf")
+        y[M - 1, K - 1] = float("nan")
+        bad = torch.empty(M, N, device=DEV)
+        ops.linear(y, w, bad)
+        assert torch.equal(bad[:M - 1], out[:M - 1, :N]) and torch.all(torch.isnan(bad[M - 1]))
+
+
+@pytest.mark.parametrize("M", [3, 20])
+def test_linear_f32_of_rows_further_apart_than_32_bit_distances_reach(ops, M):
+    far, K = (1 << 24) + 4, 12                          # 48 rows of such a distance: over 3 GiB
+    buf = torch.empty(M * far, device=DEV)
+    x = buf.as_strided((M, K), (far, 1))
+    x.copy_(rnd(M, K, seed=1))
+    w = rnd(19, K, seed=2)
+    out = torch.empty(M, 19, device=DEV)
+    ops.linear(x, w, out)
+    ref = x.double() @ w.double().t()
+    assert torch.all((out.double() - ref).abs() <= ref.abs() * 2.0 ** -24 + 1e-12 * ref.abs().max())
 
 
 def test_linear_f32_of_more_tiles_than_a_launch_holds(ops):
