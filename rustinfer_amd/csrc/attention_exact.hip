@@ -2,23 +2,21 @@
 // as attention_generic.hip (reference: fused_ops.rs:430-535), tiled so that the keys and values a
 // block needs are read once for a tile of query tokens and all query heads of a key/value head.
 //
-// A block of four waves owns up to 32 query rows: TQ = 32 / G consecutive tokens of one request
-// (G = H / Hkv query heads each) on one key/value head.  Keys go by in blocks of 64 that are
+// A block of four waves owns 16 query rows (32 where a token's heads are more): consecutive tokens of one request, all query
+// heads of one key/value head.  Keys go by in blocks of 64 that are
 // aligned to absolute key positions (block c holds keys 64 c .. 64 c + 63), so that what a query
 // row adds up, and in which order, depends on its position alone and not on how the prompt was
-// cut.  A block of keys and values is brought into LDS by all threads; a wave then works on
-// four of its rows at a time with one key a lane: dot products of head-size terms in ascending
-// order, the row's maximum and sum over the 64 lanes in a fixed tree, the probabilities to LDS,
-// and then, one value feature a lane (two above 64), the weighted sum over the 64 keys in
-// ascending order.  All arithmetic is 32-bit FMA; nothing is rounded below that.
+// cut: dot products of head-size terms in ascending order, the row's maximum and sum over the block in a
+// fixed tree, and the weighted sum over the 64 keys in ascending order.  All arithmetic is 32-bit: fused multiply-adds, on
+// the 32-bit matrix instruction; nothing is rounded below that.
 // Cache layout: keys [pages][Hkv][page][hd], values [pages][Hkv][hd][page].  hd % 4 == 0, hd <= 128.
 //
-// What a query row adds up, and in which order, is the same in both kernels of this file (the
-// tiled one for prompt portions and the split-key one for single tokens), so that a token's
+// What a query row adds up, and in which order, is the same in all forms of the kernel (for
+// prompt portions, for a token's keys in turn and for one block of them), so that a token's
 // output has the same bits whether its step held prompt portions or not:
 //   - a block of 64 keys gives the row a partial result of its own: the largest score m_b, the
 //     probabilities exp(s - m_b), their sum l_b and the weighted values acc_b, each summed in
-//     ascending order from zero (block_scores / the P.V loops);
+//     ascending order from zero;
 //   - the partial results are merged in ascending order of the blocks (merge_block).
 // Products and sums that must round the same way everywhere are written with fmaf, __fmul_rn and
 // __fsub_rn, and contraction is switched off for the file.
@@ -29,20 +27,8 @@
 
 namespace {
 
-constexpr int EX_ROWS = 32;      // query rows a block
+constexpr int EX_ROWS = 32;      // query rows a block, at most
 constexpr int EX_KEYS = 64;      // keys a step: one a lane
-
-// One row's scores against the 64 keys of a block, one key a lane: s = q.k * scale (or -inf where
-// the key is not the row's), the block's maximum, exp(s - maximum) and its sum over the lanes.
-// Returns this lane's probability; m_b = -inf (and l_b = 0) if the row sees no key of the block.
-__device__ __forceinline__ float block_scores(float dot, bool mine, float scale, float& m_b, float& l_b) {
-    const float sc = mine ? __fmul_rn(dot, scale) : -INFINITY;
-    m_b = wave_max(sc);
-    float pj = 0.f;
-    if (m_b > -INFINITY) pj = mine ? expf(__fsub_rn(sc, m_b)) : 0.f;
-    l_b = wave_sum(pj);
-    return pj;
-}
 
 // Merge a block's partial result (m_b, l_b, acc_b) into the running one (m, l, acc).
 template <int NC>
@@ -57,315 +43,331 @@ __device__ __forceinline__ void merge_block(float& m, float& l, float (&acc)[NC]
     m = M;
 }
 
-template <int NC>                // 64-wide slices of the head size a lane holds: 1 or 2
-__global__ __launch_bounds__(256) void attn_exact_f32_kernel(
+typedef float exf32x4_t __attribute__((ext_vector_type(4)));
+
+// Four registers of the four lane groups (lane / 16), transposed: register s of group g becomes register g of group s.
+__device__ __forceinline__ void transpose_groups(float4& v) {
+    uint32_t x0 = __float_as_uint(v.x), x1 = __float_as_uint(v.y), x2 = __float_as_uint(v.z), x3 = __float_as_uint(v.w);
+    auto a = __builtin_amdgcn_permlane32_swap(x0, x2, false, false);
+    auto b = __builtin_amdgcn_permlane32_swap(x1, x3, false, false);
+    auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);
+    auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    v = make_float4(__uint_as_float(c[0]), __uint_as_float(c[1]), __uint_as_float(d[0]), __uint_as_float(d[1]));
+}
+__device__ __forceinline__ float elem(const float4& v, int i) { return i == 0 ? v.x : i == 1 ? v.y : i == 2 ? v.z : v.w; }
+
+// v_mfma_f32_16x16x4_f32 gives D = A.B + C with the four products added to C one after the other, each a fused multiply-add
+// rounded to 32 bits (denormals kept): the sums of an FMA loop over the same index, bit for bit, at twice its rate and with
+// no operand read from LDS.
+//
+// A block owns RT tiles of 16 query rows on one key/value head; its four waves take a block of 64 keys together:
+//   - scores: wave w multiplies keys 16 w .. 16 w + 15 with all rows.  Row m of the instruction's A holds key 4 (m % 4) + m / 4, so
+//     that element i of lane group g of the result is key 4 i + g, which is where the second product wants it.  A lane reads four
+//     consecutive features of its key; transpose_groups makes them the four steps' operands.
+//   - the waves' maxima meet in LDS, then their probabilities (two barriers a block of keys, two buffers of each); every wave
+//     reads all 64 of its lanes' rows and makes their sum itself, whose tree is that of wave_sum over a lane a key.
+//   - weighted values: wave w makes the features 16 w .. 16 w + 15 (and those 64 on), keys in ascending order.
+// Keys, values and page ids are asked for a block of keys ahead.  SINGLE: a block's rows are one token's heads.
+// What bounds it: the chain of a block of keys (16 dependent matrix instructions, two barriers, exponentials, 16 more), about 1.7 us
+// where a unit holds one block, and the instructions beside the matrix instructions where it holds four.  Measured, us, with FMAs on
+// operands from LDS (and a key a lane for single tokens) before / now, 32 heads, 8 of keys: 600 tokens at head 64 151 / 45, 100 tokens 31 / 7.5,
+// 2,048 tokens 1024 / 327 (52 TFLOP/s), 64 tokens behind 2,000 544 / 66, 7 single tokens behind 1,500 beside 64 more 416 / 52; head 128:
+// 600 tokens 471 / 84; 2,048 tokens of 24 heads 2748 / 504.
+enum { EX_PORTIONS = 0, EX_SINGLE = 1, EX_BLOCKS = 2 };
+template <int NJ, int RT, int MODE, bool ANY>          // NJ: groups of 16 features, 4 or 8; ANY: pages of any size, else of 2^page_shift >= 4
+__global__ __launch_bounds__(256, NJ * RT > 4 ? 2 : 4) void attn_exact_f32_kernel(
         const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
         const float* __restrict__ kc, const float* __restrict__ vc,
         const int* __restrict__ table, int max_blocks,
-        const int* __restrict__ cu_q, const int* __restrict__ q_start, const int* __restrict__ kv_lens,
-        int num_rows, int H, int Hkv, int hd, int page, float scale, int window, int TQ) {
-    extern __shared__ __align__(16) float lds[];
-    const int ks_stride = hd + 4, vs_stride = hd + 1;
-    float* Qs = lds;                                   // [EX_ROWS][hd]
-    float* Ks = Qs + EX_ROWS * hd;                     // [EX_KEYS][hd + 4]
-    float* Vs = Ks + EX_KEYS * ks_stride;              // [EX_KEYS][hd + 1]
-    float* Ps = Vs + EX_KEYS * vs_stride;              // [EX_ROWS][EX_KEYS]
-    int* koff = reinterpret_cast<int*>(Ps + EX_ROWS * EX_KEYS);   // [EX_KEYS] key slot in the cache, -1: none
-
-    // which request and which of its tokens: tiles are numbered request by request
-    const int tile = blockIdx.x, g = blockIdx.y, G = H / Hkv;
-    int b = -1, t0 = 0, nt = 0, before = 0;
-    for (int r = 0; r < num_rows; ++r) {
-        const int lo = cu_q[r], ql = cu_q[r + 1] - lo, tiles = (ql + TQ - 1) / TQ;
-        if (tile < before + tiles) {
-            b = r;
-            t0 = lo + (tile - before) * TQ;
-            nt = min(TQ, lo + ql - t0);
-            break;
+        const int* __restrict__ cu_q, const int* __restrict__ q_start, const int* __restrict__ row_of_token,
+        const int* __restrict__ positions, const int* __restrict__ kv_lens,
+        int num_rows, int H, int Hkv, int hd, int page, int page_shift, float scale, int window, int TQ,
+        int slots, float* __restrict__ part_ml, float* __restrict__ part_o) {
+    constexpr int NF = NJ / 4;                         // feature tiles a wave
+    __shared__ float4 probs[2][RT][4][64];             // [buffer][row tile][key tile][lane]
+    __shared__ float tops[2][RT][4][16];               // [buffer][row tile][key tile][row]
+    const int g_kv = blockIdx.y, G = H / Hkv;
+    int b = -1, t0 = 0, nt = 0, p0 = 0;
+    if (MODE != EX_PORTIONS) {
+        t0 = MODE == EX_SINGLE ? blockIdx.x : blockIdx.z;
+        nt = 1;
+        b = row_of_token[t0];
+        p0 = positions[t0];
+    } else {
+        // which request and which of its tokens: tiles are numbered request by request; late tiles, which see the most keys, run first
+        const int tile = (int)gridDim.x - 1 - (int)blockIdx.x;
+        int before = 0;
+        for (int r = 0; r < num_rows; ++r) {
+            const int lo = cu_q[r], ql = cu_q[r + 1] - lo, tiles = (ql + TQ - 1) / TQ;
+            if (tile < before + tiles) {
+                b = r;
+                t0 = lo + (tile - before) * TQ;
+                nt = min(TQ, lo + ql - t0);
+                break;
+            }
+            before += tiles;
         }
-        before += tiles;
+        if (b < 0) return;
+        p0 = q_start[b] + (t0 - cu_q[b]);              // position of the tile's first token
     }
-    if (b < 0) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int R = nt * G;                              // rows in use: row r = token r / G, head g G + r % G
-    const int p0 = q_start[b] + (t0 - cu_q[b]);        // position of the tile's first token
-    const int kv_len = kv_lens[b];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
+    const int R = nt * G;                              // rows in use: row i = token i / G, head i % G of the group
+    const int kv_len = b >= 0 ? kv_lens[b] : 0;        // a padding token sees nothing
     const int last_visible = min(kv_len, p0 + nt);     // of the tile's last token
     const int first_key = window > 0 ? max(0, p0 + 1 - window) : 0;   // of its first
+    const int* pages = table + (size_t)max(b, 0) * max_blocks;
+    auto page_of = [&](int key) { return (uint32_t)(ANY ? key / page : key >> page_shift); };
+    auto slot_of = [&](int key) { return ANY ? key % page : key & (page - 1); };
+    const uint32_t page_size = (uint32_t)Hkv * page * hd;                     // values of a page
+    const float* kg = kc + (size_t)g_kv * page * hd;
+    const float* vg = vc + (size_t)g_kv * page * hd;
 
-    for (int e = tid; e < EX_ROWS * hd; e += 256) {
-        const int r = e / hd, dd = e % hd;
-        Qs[e] = r < R ? q[(size_t)(t0 + r / G) * q_stride + (g * G + r % G) * hd + dd] : 0.f;
-    }
-
-    // this wave's rows: wave, wave + 4, ...; four of them a batch
-    const int batches = (R + 15) / 16;                 // the same for all waves: they share the barriers
-    float m[8], l[8], acc[8][NC];
-    int row_lo[8], row_hi[8];                          // keys [row_lo, row_hi) are the row's
+    float4 qt[RT][NJ];                                 // .x .. .w: features 16 j + 4 s + g of the lane's row
+    int row_lo[RT], row_hi[RT];                        // keys [row_lo, row_hi) are the row's
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        m[i] = -INFINITY;
-        l[i] = 0.f;
+    for (int rt = 0; rt < RT; ++rt) {
+        const int i = rt * 16 + r, p = p0 + i / G;
+        row_hi[rt] = i < R ? min(kv_len, p + 1) : 0;
+        row_lo[rt] = window > 0 ? max(0, p + 1 - window) : 0;
+        const float* qr = q + (size_t)(t0 + (i < R ? i / G : 0)) * q_stride + (size_t)(g_kv * G + (i < R ? i % G : 0)) * hd;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) acc[i][c] = 0.f;
-        const int r = wave + 4 * i, p = p0 + r / G;
-        row_hi[i] = r < R ? min(kv_len, p + 1) : 0;
-        row_lo[i] = window > 0 ? max(0, p + 1 - window) : 0;
-    }
-
-    for (int kb = first_key / EX_KEYS; kb * EX_KEYS < last_visible; ++kb) {
-        const int j_base = kb * EX_KEYS;
-        __syncthreads();                               // the last block of keys has been used (first pass: Qs is written)
-        if (tid < EX_KEYS) {
-            const int j = j_base + tid;
-            int off = -1;
-            if (j < last_visible) {
-                const int pid = table[(size_t)b * max_blocks + j / page];
-                if (pid >= 0) off = (pid * Hkv + g) * page + j % page;      // -1: a page the window has passed and given back
-            }
-            koff[tid] = off;
-        }
-        __syncthreads();
-        // keys: 16-byte pieces, hd / 4 a key
-        const int pieces = hd / 4;
-        for (int e = tid; e < EX_KEYS * pieces; e += 256) {
-            const int jj = e / pieces, pc = e % pieces, off = koff[jj];
+        for (int j = 0; j < NJ; ++j) {
             float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (off >= 0) v = *reinterpret_cast<const float4*>(kc + (size_t)off * hd + pc * 4);
-            *reinterpret_cast<float4*>(Ks + jj * ks_stride + pc * 4) = v;
+            const int d = 16 * j + 4 * g;
+            if (i < R && d < hd) v = make_float4(qr[d], qr[d + 1], qr[d + 2], qr[d + 3]);
+            transpose_groups(v);
+            qt[rt][j] = v;
         }
-        // values: thread -> key tid % 64, features tid / 64, + 4, ...; zero where there is no key (0 * garbage)
-        {
-            const int jj = tid & 63, off = koff[jj];
-            const size_t vbase = off >= 0 ? (size_t)(off / page) * page * hd + off % page : 0;
-            for (int d = tid >> 6; d < hd; d += 4)
-                Vs[jj * vs_stride + d] = off >= 0 ? vc[vbase + (size_t)d * page] : 0.f;
+    }
+    float m[RT], l[RT];
+    exf32x4_t acc[RT][NF];
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+        m[rt] = -INFINITY;
+        l[rt] = 0.f;
+#pragma unroll
+        for (int f = 0; f < NF; ++f) acc[rt][f] = exf32x4_t{0.f, 0.f, 0.f, 0.f};
+    }
+
+    // The lane's key of a block's tile w, and its four keys of each tile of values.  Every load is made, from the last visible
+    // key or from page 0 where there is none to make, and what it brings is put to zero where it is used: loads under a
+    // condition would be waited for all at once.
+    const int kj = 16 * wave + 4 * (r & 3) + (r >> 2);
+    int kb0 = first_key / EX_KEYS, kb1 = last_visible > first_key ? (last_visible + EX_KEYS - 1) / EX_KEYS : kb0;
+    if (MODE == EX_BLOCKS) {                           // one block of keys
+        kb0 += blockIdx.x;
+        if (kb0 >= kb1) return;
+        kb1 = kb0 + 1;
+    }
+    int pk = -1, pv[4] = {-1, -1, -1, -1};             // pages of the block that is asked for next
+    bool v_there[4] = {};                              // of the block that is used next
+    auto ask_pages = [&](int kb) {
+        pk = pages[page_of(min(kb * EX_KEYS + kj, last_visible - 1))];
+        if (!ANY)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) pv[t] = pages[page_of(min(kb * EX_KEYS + 16 * t + 4 * g, last_visible - 1))];
+    };
+    float4 kt[NJ], vt[NF][4];
+    auto ask_keys = [&](int kb) {                      // where there is no key: its score is not looked at
+        const float* kr = kg + (size_t)(uint32_t)max(pk, 0) * page_size + (uint32_t)slot_of(kb * EX_KEYS + kj) * (uint32_t)hd;
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) {
+            const int d = 16 * jj + 4 * g;
+            kt[jj] = *reinterpret_cast<const float4*>(kr + (d < hd ? d : 0));
+        }
+    };
+    auto ask_values = [&](int kb) {
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int key = kb * EX_KEYS + 16 * t + 4 * g;
+            if (!ANY) {
+                v_there[t] = pv[t] >= 0;
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    const int d = min(16 * (wave + 4 * f) + r, hd - 1);
+                    vt[f][t] = *reinterpret_cast<const float4*>(vg + (size_t)(uint32_t)max(pv[t], 0) * page_size + (uint32_t)(d * page + slot_of(key)));
+                }
+            } else {
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    const int d = min(16 * (wave + 4 * f) + r, hd - 1);
+                    float x[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const int pid = key + u < last_visible ? pages[page_of(key + u)] : -1;
+                        x[u] = pid >= 0 ? vg[(size_t)(uint32_t)pid * page_size + (uint32_t)(d * page + slot_of(key + u))] : 0.f;
+                    }
+                    vt[f][t] = make_float4(x[0], x[1], x[2], x[3]);
+                }
+            }
+        }
+    };
+    if (kb0 < kb1) {
+        ask_pages(kb0);
+        ask_keys(kb0);
+        ask_values(kb0);
+        if (MODE != EX_BLOCKS) ask_pages(min(kb0 + 1, kb1 - 1));
+    }
+    for (int kb = kb0; kb < kb1; ++kb) {
+        const int j_base = kb * EX_KEYS, buf = kb & 1;
+        const int next = min(kb + 1, kb1 - 1);
+        exf32x4_t s[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) s[rt] = exf32x4_t{0.f, 0.f, 0.f, 0.f};
+        float4 k4[NJ];
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj) {
+            const uint32_t feature = 16 * jj + 4 * g < hd ? 0xffffffffu : 0u;          // (as a mask: no branch around the wait)
+            k4[jj] = make_float4(__uint_as_float(__float_as_uint(kt[jj].x) & feature), __uint_as_float(__float_as_uint(kt[jj].y) & feature),
+                                 __uint_as_float(__float_as_uint(kt[jj].z) & feature), __uint_as_float(__float_as_uint(kt[jj].w) & feature));
+            transpose_groups(k4[jj]);
+        }
+        if (MODE != EX_BLOCKS) ask_keys(next);
+#pragma unroll
+        for (int jj = 0; jj < NJ; ++jj)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+#pragma unroll
+                for (int rt = 0; rt < RT; ++rt)
+                    s[rt] = __builtin_amdgcn_mfma_f32_16x16x4f32(elem(k4[jj], u), elem(qt[rt][jj], u), s[rt], 0, 0, 0);
+        // element i: key 16 w + 4 i + g of the block
+        float sc[RT][4];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int j = j_base + 16 * wave + 4 * i + g;
+                sc[rt][i] = j >= row_lo[rt] && j < row_hi[rt] ? __fmul_rn(s[rt][i], scale) : -INFINITY;
+            }
+            float top = fmaxf(fmaxf(sc[rt][0], sc[rt][1]), fmaxf(sc[rt][2], sc[rt][3]));
+            top = fmaxf(top, __shfl_xor(top, 16, 64));
+            top = fmaxf(top, __shfl_xor(top, 32, 64));
+            if (g == 0) tops[buf][rt][wave][r] = top;
         }
         __syncthreads();
-        // scores and probabilities of the block, each row's relative to the block's own maximum
-        float m_b[8], l_b[8], acc_b[8][NC];
+        float m_b[RT], l_b[RT];
+        float4 p[RT][4];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            m_b[i] = -INFINITY;
-            l_b[i] = 0.f;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) acc_b[i][c] = 0.f;
+        for (int rt = 0; rt < RT; ++rt) {
+            // a key that is not the row's has the score -inf and the probability zero, also where the row has no key here
+            m_b[rt] = fmaxf(fmaxf(fmaxf(tops[buf][rt][0][r], tops[buf][rt][1][r]), fmaxf(tops[buf][rt][2][r], tops[buf][rt][3][r])), -INFINITY);
+            const float top = m_b[rt] > -INFINITY ? m_b[rt] : 0.f;
+            probs[buf][rt][wave][lane] = make_float4(expf(__fsub_rn(sc[rt][0], top)), expf(__fsub_rn(sc[rt][1], top)),
+                                                     expf(__fsub_rn(sc[rt][2], top)), expf(__fsub_rn(sc[rt][3], top)));
         }
+        __syncthreads();
 #pragma unroll
-        for (int bi = 0; bi < 2; ++bi) {               // unrolled: the rows' registers are indexed by constants
-            if (bi >= batches) break;
-            float s[4] = {0.f, 0.f, 0.f, 0.f};
-            const float* kr = Ks + lane * ks_stride;
-#pragma unroll 2
-            for (int dd = 0; dd < hd; dd += 4) {
-                const float4 k4 = *reinterpret_cast<const float4*>(kr + dd);
+        for (int rt = 0; rt < RT; ++rt) {
 #pragma unroll
-                for (int rb = 0; rb < 4; ++rb) {
-                    const float4 q4 = *reinterpret_cast<const float4*>(Qs + (wave + 4 * (4 * bi + rb)) * hd + dd);
-                    s[rb] = fmaf(q4.x, k4.x, s[rb]);
-                    s[rb] = fmaf(q4.y, k4.y, s[rb]);
-                    s[rb] = fmaf(q4.z, k4.z, s[rb]);
-                    s[rb] = fmaf(q4.w, k4.w, s[rb]);
-                }
-            }
-            const int j = j_base + lane;
+            for (int t = 0; t < 4; ++t) p[rt][t] = probs[buf][rt][t][lane];
+            // wave_sum's tree with key = 16 t + 4 i + g for the lane: t ^ 2, t ^ 1, i ^ 2, i ^ 1, g ^ 2, g ^ 1
+            float e[4];
 #pragma unroll
-            for (int rb = 0; rb < 4; ++rb) {
-                const int i = 4 * bi + rb;
-                const bool mine = j >= row_lo[i] && j < row_hi[i];
-                Ps[(wave + 4 * i) * EX_KEYS + lane] = block_scores(s[rb], mine, scale, m_b[i], l_b[i]);
-            }
+            for (int i = 0; i < 4; ++i)
+                e[i] = (elem(p[rt][0], i) + elem(p[rt][2], i)) + (elem(p[rt][1], i) + elem(p[rt][3], i));
+            float sum = (e[0] + e[2]) + (e[1] + e[3]);
+            sum += __shfl_xor(sum, 32, 64);
+            sum += __shfl_xor(sum, 16, 64);
+            l_b[rt] = sum;
         }
-        __syncthreads();                               // probabilities written (each wave reads its own rows)
+        exf32x4_t acc_b[RT][NF];
 #pragma unroll
-        for (int bi = 0; bi < 2; ++bi) {
-            if (bi >= batches) break;
-#pragma unroll 1
-            for (int jj = 0; jj < EX_KEYS; jj += 4) {
-                float4 p4[4];
+        for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-                for (int rb = 0; rb < 4; ++rb)
-                    p4[rb] = *reinterpret_cast<const float4*>(Ps + (wave + 4 * (4 * bi + rb)) * EX_KEYS + jj);
+            for (int f = 0; f < NF; ++f) acc_b[rt][f] = exf32x4_t{0.f, 0.f, 0.f, 0.f};
+        float4 v4[NF][4];
+        // the rest of a last page, and a page that the window has passed and given back, may hold anything
+        const bool cut = !ANY && (j_base + EX_KEYS > last_visible || __any(!(v_there[0] && v_there[1] && v_there[2] && v_there[3])));
 #pragma unroll
-                for (int u = 0; u < 4; ++u) {
+        for (int f = 0; f < NF; ++f)
 #pragma unroll
-                    for (int c = 0; c < NC; ++c) {
-                        const int d = lane + 64 * c;
-                        const float v = d < hd ? Vs[(jj + u) * vs_stride + d] : 0.f;
+            for (int t = 0; t < 4; ++t) v4[f][t] = vt[f][t];
+        if (cut) {
 #pragma unroll
-                        for (int rb = 0; rb < 4; ++rb) {
-                            const float pv = u == 0 ? p4[rb].x : u == 1 ? p4[rb].y : u == 2 ? p4[rb].z : p4[rb].w;
-                            acc_b[4 * bi + rb][c] = fmaf(pv, v, acc_b[4 * bi + rb][c]);
-                        }
-                    }
+            for (int t = 0; t < 4; ++t) {
+                const int key = j_base + 16 * t + 4 * g, there = v_there[t] ? last_visible : 0;
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    v4[f][t].x = key < there ? v4[f][t].x : 0.f;
+                    v4[f][t].y = key + 1 < there ? v4[f][t].y : 0.f;
+                    v4[f][t].z = key + 2 < there ? v4[f][t].z : 0.f;
+                    v4[f][t].w = key + 3 < there ? v4[f][t].w : 0.f;
                 }
             }
         }
 #pragma unroll
-        for (int i = 0; i < 8; ++i) merge_block<NC>(m[i], l[i], acc[i], m_b[i], l_b[i], acc_b[i]);
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int t = 0; t < 4; ++t) transpose_groups(v4[f][t]);
+        if (MODE != EX_BLOCKS) {
+            ask_values(next);
+            ask_pages(min(kb + 2, kb1 - 1));
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int f = 0; f < NF; ++f)
+#pragma unroll
+                    for (int rt = 0; rt < RT; ++rt)
+                        acc_b[rt][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(elem(v4[f][t], i), elem(p[rt][t], i), acc_b[rt][f], 0, 0, 0);
+        if (MODE == EX_BLOCKS) {                       // the block's partial results
+#pragma unroll
+            for (int rt = 0; rt < RT; ++rt) {
+                const int i = rt * 16 + r;
+                if (i >= R) continue;
+                const size_t at = ((size_t)t0 * H + (size_t)g_kv * G + i) * slots + blockIdx.x;
+                if (wave == 0 && g == 0) {
+                    part_ml[at * 2] = m_b[rt];
+                    part_ml[at * 2 + 1] = l_b[rt];
+                }
+#pragma unroll
+                for (int f = 0; f < NF; ++f) {
+                    const int d = 16 * (wave + 4 * f) + 4 * g;         // hd % 4 == 0
+                    if (d < hd) *reinterpret_cast<float4*>(part_o + at * hd + d) =
+                        make_float4(acc_b[rt][f][0], acc_b[rt][f][1], acc_b[rt][f][2], acc_b[rt][f][3]);
+                }
+            }
+            return;
+        }
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+            float add[NF * 4], sum[NF * 4];
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) { add[f * 4 + e] = acc_b[rt][f][e]; sum[f * 4 + e] = acc[rt][f][e]; }
+            merge_block<NF * 4>(m[rt], l[rt], sum, m_b[rt], l_b[rt], add);
+#pragma unroll
+            for (int f = 0; f < NF; ++f)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[rt][f][e] = sum[f * 4 + e];
+        }
     }
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int r = wave + 4 * i;
-        if (r >= R) continue;
-        float* o = out + (size_t)(t0 + r / G) * out_stride + (g * G + r % G) * hd;
+    for (int rt = 0; rt < RT; ++rt) {
+        const int i = rt * 16 + r;
+        if (i >= R) continue;
+        float* o = out + (size_t)(t0 + i / G) * out_stride + (size_t)(g_kv * G + i % G) * hd;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            const int d = lane + 64 * c;
-            if (d < hd) o[d] = l[i] > 0.f ? acc[i][c] / l[i] : 0.f;
-        }
+        for (int f = 0; f < NF; ++f)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int d = 16 * (wave + 4 * f) + 4 * g + e;
+                if (d < hd) o[d] = l[rt] > 0.f ? acc[rt][f][e] / l[rt] : 0.f;
+            }
     }
 }
 
 // ---------------------------------------------------------------------------
-// Single tokens: the key range is split over waves, one block of 64 keys each ("flash decoding";
-// reference: crates/infer-backend-cuda/src/kernels/flash_attn_gqa/flash_attn_paged_decode.cu:75-337),
-// so that a step of few tokens still fills the chip: the tiled kernel above would give a token
-// one block of threads for all its keys.  A wave computes the partial result of its key block for
-// all G query heads of one key/value head, with one key a lane for the scores (the key's row is
-// read straight from the cache, 16 bytes at a time; the query rows are the same for all lanes) and
-// one value feature a lane (two above 64) for the weighted values, the probabilities passing
-// through LDS.  The arithmetic of a row is that of the tiled kernel, term for term.  A second
-// kernel merges a row's partial results in ascending order of the blocks.
+// Single tokens.  Where they are few, a block takes one block of 64 keys of a token ("flash decoding"; reference:
+// crates/infer-backend-cuda/src/kernels/flash_attn_gqa/flash_attn_paged_decode.cu:75-337) and leaves its partial result, and a
+// second kernel merges a row's partial results in ascending order of the blocks; where (token, key/value head) pairs fill the
+// chip, a block takes all of its token's keys in turn and there is no second kernel.
 // Partial results: part_ml [T][H][slots][2] = (m_b, l_b), part_o [T][H][slots][hd]; slot s of a
 // token is key block first_block + s, first_block = (first visible key) / 64.
 // ---------------------------------------------------------------------------
-template <int NC>
-__global__ __launch_bounds__(256) void attn_exact_decode_kernel(
-        const float* __restrict__ q, int q_stride, const float* __restrict__ kc, const float* __restrict__ vc,
-        const int* __restrict__ table, int max_blocks, const int* __restrict__ row_of_token,
-        const int* __restrict__ positions, const int* __restrict__ kv_lens,
-        int H, int Hkv, int hd, int page, float scale, int window, int slots,
-        float* __restrict__ part_ml, float* __restrict__ part_o) {
-    extern __shared__ __align__(16) float lds[];       // [4 waves][G][64] probabilities
-    const int t = blockIdx.z, g = blockIdx.y, G = H / Hkv;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int b = row_of_token[t];
-    if (b < 0) return;                                  // a padding token
-    const int p = positions[t];
-    const int visible = min(kv_lens[b], p + 1);
-    const int j0 = window > 0 ? max(0, p + 1 - window) : 0;
-    if (visible <= j0) return;
-    const int first_block = j0 / EX_KEYS;
-    const int slot = (int)blockIdx.x * 4 + wave;
-    const int kb = first_block + slot;
-    if (kb * EX_KEYS >= visible) return;
-    float* Ps = lds + (size_t)wave * G * EX_KEYS;
-
-    // this lane's key
-    const int j = kb * EX_KEYS + lane;
-    long long off = -1;                                 // key slot in the cache; -1: none
-    if (j < visible) {
-        const int pid = table[(size_t)b * max_blocks + j / page];
-        if (pid >= 0) off = ((long long)pid * Hkv + g) * page + j % page;
-    }
-    const bool mine = j >= j0 && j < visible;
-    const float* kr = off >= 0 ? kc + (size_t)off * hd : nullptr;
-    const float* qrow = q + (size_t)t * q_stride + (size_t)g * G * hd;
-    float* ml = part_ml + (((size_t)t * H + (size_t)g * G) * slots + slot) * 2;
-    // scores: four heads a pass over the key's row (which the next pass finds in the cache)
-    for (int h0 = 0; h0 < G; h0 += 4) {
-        float s[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-        for (int dd = 0; dd < hd; dd += 4) {
-            float4 k4 = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (kr) k4 = *reinterpret_cast<const float4*>(kr + dd);
-#pragma unroll
-            for (int rb = 0; rb < 4; ++rb) {
-                const float4 q4 = *reinterpret_cast<const float4*>(qrow + (size_t)min(h0 + rb, G - 1) * hd + dd);
-                s[rb] = fmaf(q4.x, k4.x, s[rb]);
-                s[rb] = fmaf(q4.y, k4.y, s[rb]);
-                s[rb] = fmaf(q4.z, k4.z, s[rb]);
-                s[rb] = fmaf(q4.w, k4.w, s[rb]);
-            }
-        }
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-            if (h0 + rb >= G) break;
-            float m_b, l_b;
-            Ps[(h0 + rb) * EX_KEYS + lane] = block_scores(s[rb], mine, scale, m_b, l_b);
-            if (lane == 0) {
-                float* dst = ml + (size_t)(h0 + rb) * slots * 2;
-                dst[0] = m_b;
-                dst[1] = l_b;
-            }
-        }
-    }
-    // weighted values: lane = feature; four keys a load where pages allow (the value cache keeps
-    // the positions of a feature contiguous)
-    const bool vec = (page & 3) == 0;
-    for (int h0 = 0; h0 < G; h0 += 4) {
-        float acc_b[4][NC];
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb)
-#pragma unroll
-            for (int c = 0; c < NC; ++c) acc_b[rb][c] = 0.f;
-#pragma unroll 4
-        for (int jj = 0; jj < EX_KEYS; jj += 4) {
-            const int key = kb * EX_KEYS + jj;         // four keys of one page if page % 4 == 0
-            float v[4][NC];
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int c = 0; c < NC; ++c) v[u][c] = 0.f;
-            if (key < visible) {
-                if (vec) {
-                    const int pid = table[(size_t)b * max_blocks + key / page];
-                    if (pid >= 0) {
-#pragma unroll
-                        for (int c = 0; c < NC; ++c) {
-                            const int d = lane + 64 * c;
-                            if (d < hd) {
-                                const float4 v4 = *reinterpret_cast<const float4*>(
-                                    vc + (((size_t)pid * Hkv + g) * hd + d) * page + key % page);
-                                v[0][c] = v4.x;
-                                v[1][c] = key + 1 < visible ? v4.y : 0.f;      // slots never written may hold anything
-                                v[2][c] = key + 2 < visible ? v4.z : 0.f;
-                                v[3][c] = key + 3 < visible ? v4.w : 0.f;
-                            }
-                        }
-                    }
-                } else {
-#pragma unroll
-                    for (int u = 0; u < 4; ++u) {
-                        if (key + u >= visible) continue;
-                        const int pid = table[(size_t)b * max_blocks + (key + u) / page];
-                        if (pid < 0) continue;
-#pragma unroll
-                        for (int c = 0; c < NC; ++c) {
-                            const int d = lane + 64 * c;
-                            if (d < hd) v[u][c] = vc[(((size_t)pid * Hkv + g) * hd + d) * page + (key + u) % page];
-                        }
-                    }
-                }
-            }
-            float4 p4[4];
-#pragma unroll
-            for (int rb = 0; rb < 4; ++rb)
-                p4[rb] = *reinterpret_cast<const float4*>(Ps + min(h0 + rb, G - 1) * EX_KEYS + jj);
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-#pragma unroll
-                for (int c = 0; c < NC; ++c)
-#pragma unroll
-                    for (int rb = 0; rb < 4; ++rb) {
-                        const float pv = u == 0 ? p4[rb].x : u == 1 ? p4[rb].y : u == 2 ? p4[rb].z : p4[rb].w;
-                        acc_b[rb][c] = fmaf(pv, v[u][c], acc_b[rb][c]);
-                    }
-        }
-#pragma unroll
-        for (int rb = 0; rb < 4; ++rb) {
-            if (h0 + rb >= G) break;
-            float* dst = part_o + (((size_t)t * H + (size_t)g * G + h0 + rb) * slots + slot) * hd;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                const int d = lane + 64 * c;
-                if (d < hd) dst[d] = acc_b[rb][c];
-            }
-        }
-    }
-}
-
 // One wave per (token, head): the partial results of its key blocks, merged in ascending order.
 template <int NC>
 __global__ __launch_bounds__(64) void attn_exact_combine_kernel(
@@ -412,9 +414,29 @@ __global__ __launch_bounds__(64) void attn_exact_combine_kernel(
     }
 }
 
-size_t exact_lds_bytes(int hd) {
-    return sizeof(float) * ((size_t)EX_ROWS * hd + (size_t)EX_KEYS * (hd + 4) + (size_t)EX_KEYS * (hd + 1) + (size_t)EX_ROWS * EX_KEYS)
-           + sizeof(int) * EX_KEYS;
+// Single tokens: from so many (token, key/value head) pairs on, or up to so many keys, a block takes all of a token's keys.
+// Measured, us, a key a lane and a wave a block of keys (before) / all keys a block / a block of keys a block and the merge, 8 key/value heads of
+// 64: 1 token of 100 keys 16.7 / 7.1 / 8.6, of 500 18.2 / 17.4 / 8.4, of 2,000 22 / 57 / 13; 6 tokens of 100 17 / 7.3 / 8.6, of 1,000 21 / 32 / 14, of
+// 4,000 42 / 120 / 34; 32 tokens of 500 28 / 20 / 20, of 2,000 79 / 65 / 55; 64 tokens of 100 20 / 10 / 12, of 2,000 169 / 101 / 120.
+constexpr int EX_SINGLE_PAIRS = 512, EX_SINGLE_KEYS = 128;
+
+// Two tiles of rows a block where a token's heads fill more than one, or the pages are of no power of two of four keys and more.
+// (For long prompts too: 2,048 tokens of 32 heads of 64 453 -> 485 us.)
+int exact_page_shift(int page) { return page >= 4 && (page & (page - 1)) == 0 ? __builtin_ctz((unsigned)page) : -1; }
+bool exact_two_tiles(int G, int page) { return G > 16 || exact_page_shift(page) < 0; }
+
+template <int MODE>
+void launch_exact(dim3 grid, int hd, int TQ, const float* q, int q_stride, float* out, int out_stride, const float* kc, const float* vc,
+                  const int* table, int max_blocks, const int* cu_q, const int* q_start, const int* row_of_token, const int* positions,
+                  const int* kv_lens, int num_rows, int H, int Hkv, int page, float scale, int window, int slots, float* part_ml, float* part_o,
+                  hipStream_t stream) {
+    const int shift = exact_page_shift(page);
+    const bool two = exact_two_tiles(H / Hkv, page);
+#define RI_EXACT(NJ_, RT_, ANY_) attn_exact_f32_kernel<NJ_, RT_, MODE, ANY_><<<grid, 256, 0, stream>>>(q, q_stride, out, out_stride, kc, vc, table, max_blocks, \
+        cu_q, q_start, row_of_token, positions, kv_lens, num_rows, H, Hkv, hd, page, shift, scale, window, TQ, slots, part_ml, part_o)
+    if (hd <= 64) { if (shift < 0) RI_EXACT(4, 2, true); else if (two) RI_EXACT(4, 2, false); else RI_EXACT(4, 1, false); }
+    else { if (shift < 0) RI_EXACT(8, 2, true); else if (two) RI_EXACT(8, 2, false); else RI_EXACT(8, 1, false); }
+#undef RI_EXACT
 }
 
 }  // namespace
@@ -425,7 +447,7 @@ extern "C" int ri_attention_exact_supported(int H, int Hkv, int hd, int page) {
 }
 
 // Every token of the step belongs to a request row (cu_q covers all T tokens); rows of one token
-// are taken as well, but a step of single tokens only is better served by the generic kernel,
+// are taken as well, but a step of single tokens only is better served by the entry point below,
 // which spreads it over more blocks.
 extern "C" int ri_attention_exact_f32(
         const float* q, int q_stride, float* out, int out_stride, const float* kc, const float* vc,
@@ -439,25 +461,11 @@ extern "C" int ri_attention_exact_f32(
     RI_REQUIRE(q && out && kc && vc && table && cu_q && q_start && kv_lens, "ri_attention_exact_f32: null pointer");
     RI_REQUIRE((uintptr_t)kc % 16 == 0, "ri_attention_exact_f32: unaligned key cache");
     RI_REQUIRE(Hkv <= 65535, "ri_attention_exact_f32: too many key/value heads for the grid");
-    const int G = H / Hkv, TQ = EX_ROWS / G;
+    const int G = H / Hkv;
+    const int TQ = (exact_two_tiles(G, page) ? 32 : 16) / G;
     const int tiles = (T + TQ - 1) / TQ + num_rows;    // at most: every request may end in a short tile
-    const size_t lds = exact_lds_bytes(hd);
-    auto kernel = hd <= 64 ? attn_exact_f32_kernel<1> : attn_exact_f32_kernel<2>;
-    if (lds > 64 * 1024) {
-        // more LDS than a kernel gets unasked: requested once a device
-        static bool asked[64] = {};
-        int dev = 0;
-        RI_REQUIRE(hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < 64, "ri_attention_exact_f32: no current device");
-        if (!asked[dev]) {
-            const size_t most = exact_lds_bytes(128);           // the largest head this kernel takes
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(attn_exact_f32_kernel<2>),
-                                               hipFuncAttributeMaxDynamicSharedMemorySize, (int)most);
-            RI_REQUIRE(e == hipSuccess, "ri_attention_exact_f32: %zu bytes of LDS refused: %s", most, hipGetErrorString(e));
-            asked[dev] = true;
-        }
-    }
-    kernel<<<dim3(tiles, Hkv), 256, lds, stream>>>(q, q_stride, out, out_stride, kc, vc, table, max_blocks, cu_q, q_start,
-                                                   kv_lens, num_rows, H, Hkv, hd, page, scale, window, TQ);
+    launch_exact<EX_PORTIONS>(dim3(tiles, Hkv), hd, TQ, q, q_stride, out, out_stride, kc, vc, table, max_blocks, cu_q, q_start, nullptr, nullptr, kv_lens,
+                              num_rows, H, Hkv, page, scale, window, 0, nullptr, nullptr, stream);
     RI_LAUNCHED("ri_attention_exact_f32");
     return 0;
 }
@@ -487,25 +495,20 @@ extern "C" int ri_attention_exact_decode_f32(
     RI_REQUIRE(workspace_floats >= ri_attention_exact_decode_workspace(T, H, hd, max_kv_len),
                "ri_attention_exact_decode_f32: workspace of %zu floats, %zu needed", workspace_floats,
                ri_attention_exact_decode_workspace(T, H, hd, max_kv_len));
-    const int G = H / Hkv;
-    const int slots = (max_kv_len + EX_KEYS - 1) / EX_KEYS + 1;       // a window may begin inside a block: one more
-    float* part_ml = workspace;
-    float* part_o = workspace + (size_t)T * H * slots * 2;
-    const size_t lds = sizeof(float) * 4 * G * EX_KEYS;
-    dim3 grid((slots + 3) / 4, Hkv, T);
-    if (hd <= 64) {
-        attn_exact_decode_kernel<1><<<grid, 256, lds, stream>>>(q, q_stride, kc, vc, table, max_blocks, row_of_token, positions,
-                                                               kv_lens, H, Hkv, hd, page, scale, window, slots, part_ml, part_o);
+    if ((long long)T * Hkv >= EX_SINGLE_PAIRS || max_kv_len <= EX_SINGLE_KEYS) {
+        launch_exact<EX_SINGLE>(dim3(T, Hkv), hd, 1, q, q_stride, out, out_stride, kc, vc, table, max_blocks, nullptr, nullptr, row_of_token, positions,
+                                kv_lens, T, H, Hkv, page, scale, window, 0, nullptr, nullptr, stream);
         RI_LAUNCHED("ri_attention_exact_decode_f32");
-        attn_exact_combine_kernel<1><<<dim3(H, T), 64, 0, stream>>>(part_ml, part_o, row_of_token, positions, kv_lens, H, hd, window,
-                                                                     slots, out, out_stride);
-    } else {
-        attn_exact_decode_kernel<2><<<grid, 256, lds, stream>>>(q, q_stride, kc, vc, table, max_blocks, row_of_token, positions,
-                                                               kv_lens, H, Hkv, hd, page, scale, window, slots, part_ml, part_o);
-        RI_LAUNCHED("ri_attention_exact_decode_f32");
-        attn_exact_combine_kernel<2><<<dim3(H, T), 64, 0, stream>>>(part_ml, part_o, row_of_token, positions, kv_lens, H, hd, window,
-                                                                     slots, out, out_stride);
+        return 0;
     }
+    const int slots = (max_kv_len + EX_KEYS - 1) / EX_KEYS + 1;       // a window may begin inside a block: one more
+    float* part_ml = workspace + (size_t)T * H * slots * hd;
+    float* part_o = workspace;
+    launch_exact<EX_BLOCKS>(dim3(slots, Hkv, T), hd, 1, q, q_stride, out, out_stride, kc, vc, table, max_blocks, nullptr, nullptr, row_of_token, positions,
+                            kv_lens, T, H, Hkv, page, scale, window, slots, part_ml, part_o, stream);
+    RI_LAUNCHED("ri_attention_exact_decode_f32");
+    auto combine = hd <= 64 ? attn_exact_combine_kernel<1> : attn_exact_combine_kernel<2>;
+    combine<<<dim3(H, T), 64, 0, stream>>>(part_ml, part_o, row_of_token, positions, kv_lens, H, hd, window, slots, out, out_stride);
     RI_LAUNCHED("ri_attention_exact_decode_f32(combine)");
     return 0;
 }

@@ -1099,6 +1099,51 @@ def test_exact_attention_of_a_portion_does_not_depend_on_the_cut(ops, H, Hkv, hd
         kc[blk, :, far % page] = saved
 
 
+@pytest.mark.parametrize("H,Hkv,hd,page,window", [(8, 2, 64, 16, 0), (40, 2, 80, 16, 0), (40, 2, 64, 4, 90), (3, 3, 4, 1, 0), (6, 2, 100, 5, 33), (32, 1, 128, 64, 0),
+                                                  (12, 4, 128, 2, 0), (7, 1, 20, 128, 130), (34, 2, 128, 6, 0)])
+def test_exact_attention_of_single_tokens_on_every_route(ops, H, Hkv, hd, page, window):
+    """Tokens as part of portions, a block of keys a block, and all keys a block (many tokens, or few keys): the same bits, and
+    64-bit arithmetic to 32-bit rounding.  Keys end in a block of 64, at its edge, and one past it; slots never written are NaN."""
+    from types import SimpleNamespace
+    ends = [1, 2, 63, 64, 65, 127, 128, 129, 192, 200, 260]
+    starts = [max(0, e - 20) for e in ends]
+    q_lens = [e - s for e, s in zip(ends, starts)]
+    qkv, kc, vc, table, ctx, hk, hv = _paged_setup(torch.float32, len(ends), H, Hkv, hd, page, q_lens, starts, seed=hd, num_pages=max(64, 1400 // page + 16))
+    ops.rope_kv_write(qkv, H, Hkv, hd, None, ctx.positions, ctx.row_of_token, kc, vc, table, page)
+    scale = 1.0 / math.sqrt(hd)
+    whole = torch.full((sum(q_lens), H * hd), float("nan"), device=DEV)
+    ops.paged_attention(qkv, whole, H, Hkv, hd, kc, vc, table, page, ctx, scale, window)
+    assert torch.isfinite(whole).all()
+    # 64-bit arithmetic over what the cache holds
+    at = torch.tensor([sum(q_lens[:b + 1]) - 1 for b in range(len(ends))], device=DEV)      # the last token of each request
+    G = H // Hkv
+    ref = torch.empty(len(ends), H, hd, dtype=torch.float64, device=DEV)
+    for b, n in enumerate(ends):
+        pages = table[b, :(n + page - 1) // page].long()
+        k = kc[pages].permute(1, 0, 2, 3).reshape(Hkv, -1, hd)[:, :n].double()
+        v = vc[pages].permute(1, 0, 3, 2).reshape(Hkv, -1, hd)[:, :n].double()
+        lo = max(0, n - window) if window else 0
+        q = qkv[at[b], :H * hd].view(Hkv, G, 1, hd).double()
+        p = torch.softmax((q * k[:, None, lo:]).sum(-1) * scale, -1)
+        ref[b] = (p[..., None] * v[:, None, lo:]).sum(2).reshape(H, hd)
+    # scores of a few units: a 32-bit sum of hd terms, exp, and a sum of up to 260 weights
+    assert torch.allclose(whole[at].double(), ref.view(len(ends), -1), rtol=0, atol=4e-6)
+
+    def single(rows, longest):
+        toks = at[rows]
+        c = SimpleNamespace(num_tokens=len(rows), num_rows=len(rows), positions=ctx.positions[toks].contiguous(),
+                            row_of_token=torch.arange(len(rows), dtype=torch.int32, device=DEV), kv_lens=ctx.kv_lens[rows].contiguous(),
+                            max_q_len=1, max_kv_len=longest, decode_only=True, workspace=ctx.workspace)
+        o = torch.full((len(rows), H * hd), float("nan"), device=DEV)
+        ops.paged_attention(qkv[toks].contiguous(), o, H, Hkv, hd, kc, vc, table[rows].contiguous(), page, c, scale, window)
+        assert torch.equal(o, whole[toks])
+
+    single(list(range(len(ends))), 260)                       # a block of keys a block (or all keys, from 512 pairs on)
+    single(list(range(len(ends))) * 3, 1024)                  # as a captured step passes it: a longest length that none has
+    single([0, 3, 6], 128)                                    # few keys
+    single((list(range(len(ends))) * 50)[:512 // Hkv + 1], 260)
+
+
 def test_attention_padding_rows_touch_nothing(ops):
     qkv, kc, vc, table, ctx, _, _ = _paged_setup(torch.float32, 2, 4, 2, 16, 16, [1, 1], [5, 9])
     kc0, vc0 = kc.clone(), vc.clone()
