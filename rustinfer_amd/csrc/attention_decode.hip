@@ -291,6 +291,240 @@ __global__ __launch_bounds__(BW * 64) void attn_decode_split_kernel(
     }
 }
 
+constexpr int LIST_SPAN = 32, LIST_ROWS = 64, LIST_WAVES = 512;
+
+// The rows' keys as one list.  Rows differ in length, and 2,049 keys are one span more than 32 waves of 64 keys take at once, so
+// a number of blocks a row leaves units idle or a few waves with twice the others' work.  Here the spans of 32
+// keys of all rows (up to 64, a lane each) are numbered one after the other, and wave w of a key/value head takes the stretch
+// [w total / W, (w + 1) total / W) of them, with a running maximum and sum; where a row ends it leaves that row's partial result
+// in slot w - (the first wave that has a span of the row).  count[b]: the row's slots.  A span's keys and values are asked for
+// while the one before it is worked on, its pages' ids a span earlier, under no lane's condition (what lies beyond the row is
+// put to zero, or its score to -inf, where it is used).  Two waves a unit in all: more leave more partial results for the same bytes.
+// The sums are O^T[d, q] = V^T . P^T, so that a query's factors lie in the lanes that hold its sums; the weights go
+// to the matrix instruction as the sum of two bfloat16, which costs a bound-by-memory kernel nothing (error of the
+// output against 64 bits 2.1e-3 -> 1.7e-3, that of its own rounding).
+// What bounds it: the bytes, and 8 us of launches, chains of small loads and the merge.  Head 128, page 16, with the merge, us, before (blocks a
+// row) / now, and the bytes at 6.87 TB/s: 43 rows of 210..3,000 keys 54.7 / 37.2 (29.2), 30 of them 54.9 / 29.2 (19.8), 20 rows of 97..1,333
+// 20.2 / 14.7 (6.1), 24 rows of 1,500 41 / 29 (21.5), 8 rows of 700 13.2 / 11.2, 40 rows of 60 17 / 9.2, 64 rows of 2,050 95 / 92 (78); equal: 8 rows of 2,050 17.8 /
+// 17.5; slower: 32 rows of 2,050 48.7 / 49.9 and 30 of 700 18.4 / 20.7, where one block a row fills the chip and needs no merge.
+__global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
+        const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
+        const int* __restrict__ table, int max_blocks, const int* __restrict__ row_of_token, const int* __restrict__ positions,
+        const int* __restrict__ kv_lens, int H, int Hkv, int page, int page_shift, float scale, int window, int splits,
+        float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ count, int tokens, int rows) {
+    constexpr int HD = 128, KT = 2, SPAN = LIST_SPAN;       // 16 KiB of keys and values
+    const int lane = threadIdx.x, col = lane & 15, grp = lane >> 4, g = blockIdx.y, G = H / Hkv;
+    // lane i: token i, its row, keys [first, end), and the spans up to and with it
+    int row = -1, first = 0, end = 0, ends = 0;
+    if (lane < tokens) {
+        const int guess = min(lane, rows - 1);              // rows usually come in the order of their tokens
+        int len = kv_lens[guess];
+        const int p = positions[lane];
+        row = row_of_token[lane];
+        if (row >= 0 && row != guess) len = kv_lens[row];
+        if (row >= 0) {                                     // else a padding token
+            end = min(len, p + 1);
+            first = window > 0 ? max(0, p + 1 - window) : 0;
+        }
+    }
+    ends = end > first ? (end + SPAN - 1) / SPAN - first / SPAN : 0;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int up = __shfl_up(ends, o, 64);
+        if (lane >= o) ends += up;
+    }
+    const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(ends, 63);
+    if (total == 0) return;
+    const uint32_t W = min((uint32_t)gridDim.x, max(total / 2, 1u)), w = blockIdx.x;       // a stretch is two spans or more, or all
+    if (w >= W) return;
+    const int f0 = (int)(w * total / W), f1 = (int)((w + 1) * total / W);       // (W total < 2^32: the host's rule)
+    struct Row { int tok, row, first, end, f0, n; };        // spans [f0, f0 + n) of the list
+    auto row_of = [&](int f) {                              // the row of span f < total
+        const int who = __popcll(__ballot(ends <= f));      // rows that end at or before it
+        Row x;
+        x.tok = who;
+        x.row = __builtin_amdgcn_readlane(row, who);
+        x.first = __builtin_amdgcn_readlane(first, who);
+        x.end = __builtin_amdgcn_readlane(end, who);
+        x.n = (x.end + SPAN - 1) / SPAN - x.first / SPAN;
+        x.f0 = __builtin_amdgcn_readlane(ends, who) - x.n;
+        return x;
+    };
+
+    struct Span { bf16x8_t k[KT][HD / 32], v[KT / 2][HD / 16]; };
+    struct Pages { int id[KT]; };                           // of the span's stretches of 16 keys
+    bf16x8_t qf[HD / 32], q_next[HD / 32];
+    auto ask_query = [&](int t, bf16x8_t (&to)[HD / 32]) {      // columns beyond the group repeat its last head; nothing is kept of them
+        const bf16_t* src = q + (size_t)t * q_stride + (size_t)(g * G + min(col, G - 1)) * HD + grp * 8;
+#pragma unroll
+        for (int kk = 0; kk < HD / 32; ++kk) to[kk] = *reinterpret_cast<const bf16x8_t*>(src + kk * 32);
+    };
+    const size_t page_size = (size_t)Hkv * page * HD;
+    auto pages_of = [&](const Row& r, int key0, Pages& p) {
+        const int* ids = table + (size_t)r.row * max_blocks;
+#pragma unroll
+        for (int x = 0; x < KT; ++x) {
+            const int k = min(key0 + 16 * x, r.end - 1);
+            p.id[x] = ids[k >> page_shift];
+        }
+    };
+    auto slot_of = [&](int key) { return key & (page - 1); };
+    auto ask = [&](Span& s, int key0, const Pages& p) {
+#pragma unroll
+        for (int h = 0; h < KT / 2; ++h) {
+            // keys: row r of tile e is key 8 (r / 4) + 4 e + r % 4 of the half; values: the lane's 8 keys are 8 grp .. + 7
+            const int k0 = key0 + 32 * h;
+            const bf16_t* k = kc + (size_t)max(col < 8 ? p.id[2 * h] : p.id[2 * h + 1], 0) * page_size + (size_t)g * page * HD
+                              + slot_of(k0 + (col >> 2) * 8 + (col & 3)) * HD + grp * 8;
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int kk = 0; kk < HD / 32; ++kk) s.k[2 * h + e][kk] = ld_stream16<bf16x8_t>(k + 4 * e * HD + kk * 32);
+            const bf16_t* v = vc + (size_t)max(grp < 2 ? p.id[2 * h] : p.id[2 * h + 1], 0) * page_size + (size_t)g * page * HD
+                              + col * page + slot_of(k0 + grp * 8);
+#pragma unroll
+            for (int db = 0; db < HD / 16; ++db) s.v[h][db] = ld_stream16<bf16x8_t>(v + (size_t)db * 16 * page);
+        }
+    };
+    f32x4_t o[HD / 16];
+    float m_run = -INFINITY, l_run = 0.f;                   // l_run: this lane's keys alone, until the row's end
+    auto clear = [&]() {
+#pragma unroll
+        for (int db = 0; db < HD / 16; ++db) o[db] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        m_run = -INFINITY;
+        l_run = 0.f;
+    };
+    // keys [lo, hi) of a row are its own; p are the span's pages
+    auto work = [&](Span& s, int key0, int lo, int hi, const Pages& p) {
+        f32x4_t st[KT];
+#pragma unroll
+        for (int t = 0; t < KT; ++t) {
+            st[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int kk = 0; kk < HD / 32; ++kk) st[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.k[t][kk], qf[kk], st[t], 0, 0, 0);
+        }
+        const bool cut = key0 < lo || key0 + SPAN > hi;
+        float m = m_run;
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int key = key0 + (t >> 1) * 32 + grp * 8 + (t & 1) * 4 + i;        // of query col
+                float sc = st[t][i] * scale;
+                if (cut) sc = key >= lo && key < hi ? sc : -INFINITY;
+                st[t][i] = sc;
+                m = fmaxf(m, sc);
+            }
+        m = fmaxf(m, __shfl_xor(m, 16, 64));
+        m = fmaxf(m, __shfl_xor(m, 32, 64));
+        const float alpha = __expf(m_run - m);              // 0 if nothing was seen so far
+        float sum = 0.f;
+        bf16x8_t pf[KT / 2], rest[KT / 2];
+#pragma unroll
+        for (int t = 0; t < KT; ++t)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const float x = __expf(st[t][i] - m);       // exp(-inf) = 0 for masked keys
+                sum += x;
+                const __bf16 y = (__bf16)x;
+                pf[t >> 1][4 * (t & 1) + i] = y;
+                rest[t >> 1][4 * (t & 1) + i] = (__bf16)(x - (float)y);
+            }
+        l_run = l_run * alpha + sum;
+        m_run = m;
+#pragma unroll
+        for (int db = 0; db < HD / 16; ++db)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[db][i] *= alpha;
+        bool gone = false;
+#pragma unroll
+        for (int x = 0; x < KT; ++x) gone |= p.id[x] < 0;
+        if (cut || gone) {                                  // slots never written and pages given back may hold anything, NaN included
+#pragma unroll
+            for (int h = 0; h < KT / 2; ++h) {
+                const int there = (grp < 2 ? p.id[2 * h] : p.id[2 * h + 1]) >= 0 ? hi - (key0 + 32 * h + grp * 8) : 0;
+#pragma unroll
+                for (int db = 0; db < HD / 16; ++db)
+#pragma unroll
+                    for (int x = 0; x < 8; ++x)
+                        if (x >= there) s.v[h][db][x] = (__bf16)0.f;
+            }
+        }
+#pragma unroll
+        for (int h = 0; h < KT / 2; ++h)
+#pragma unroll
+            for (int db = 0; db < HD / 16; ++db) {
+                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.v[h][db], pf[h], o[db], 0, 0, 0);
+                o[db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s.v[h][db], rest[h], o[db], 0, 0, 0);
+            }
+    };
+    auto leave = [&](int b, int f, int n) {                 // row b: spans [f, f + n) of the list
+        const uint32_t w0 = (((uint32_t)f + 1) * W - 1) / total;
+        float l = l_run;
+        l += __shfl_xor(l, 16, 64);
+        l += __shfl_xor(l, 32, 64);
+        if (col < G) {
+            const size_t slot = ((size_t)b * H + g * G + col) * splits + (w - w0);
+#pragma unroll
+            for (int db = 0; db < HD / 16; ++db)
+                *reinterpret_cast<float4*>(part_o + slot * HD + db * 16 + grp * 4) = make_float4(o[db][0], o[db][1], o[db][2], o[db][3]);
+            if (grp == 0) *reinterpret_cast<float2*>(part_ml + slot * 2) = make_float2(m_run, l);
+        }
+        if (w == w0 && g == 0 && lane == 0) count[b] = (int)((((uint32_t)(f + n)) * W - 1) / total - w0 + 1);
+    };
+    clear();
+    Span sa, sb;
+    // the span that is worked on, and the one after it, whose pages' ids are asked for before its turn comes
+    Row now = row_of(f0), next = now;
+    Pages p, np;
+    int key = (now.first / SPAN + f0 - now.f0) * SPAN, next_key = key;
+    auto after = [&](int f, const Row& r, int at) {         // span f follows the one at key `at` of row r
+        next = r;
+        next_key = at + SPAN;
+        if (f == r.f0 + r.n && f < f1) {
+            next = row_of(f);
+            next_key = next.first / SPAN * SPAN;
+        }
+        pages_of(next, next_key, np);
+    };
+    ask_query(now.tok, qf);
+    pages_of(now, key, p);
+    ask(sa, key, p);
+    after(f0 + 1, now, key);
+    // one span: the one after it is asked for first, perhaps of another row
+    auto step = [&](Span& here, Span& there, int f) {
+        const Row r = now;
+        const Pages pages = p;
+        const int at = key;
+        const bool last = f + 1 == r.f0 + r.n;              // of its row
+        if (last) ask_query(next.tok, q_next);
+        ask(there, next_key, np);
+        now = next;
+        key = next_key;
+        p = np;
+        after(f + 2, now, key);
+        work(here, at, r.first, r.end, pages);
+        if (last) {
+            leave(r.row, r.f0, r.n);
+            clear();
+#pragma unroll
+            for (int kk = 0; kk < HD / 32; ++kk) qf[kk] = q_next[kk];
+        }
+    };
+    int f = f0;
+    for (; f + 2 < f1; f += 2) {
+        step(sa, sb, f);
+        step(sb, sa, f + 1);
+    }
+    if (f + 1 < f1) {
+        step(sa, sb, f);
+        work(sb, key, now.first, now.end, p);
+    } else {
+        work(sa, key, now.first, now.end, p);
+    }
+    leave(now.row, now.f0, now.n);
+}
+
 // One block of CW waves per (token, head).  The partial results of the chunks are rows of HD
 // floats; a wave reads them 16 bytes a lane, 64 / (HD / 4) rows per load instruction, several
 // instructions in flight, and each wave takes its share of the rows, so that long contexts
@@ -300,7 +534,7 @@ __global__ __launch_bounds__(CW * 64) void attn_decode_combine_kernel(
         const float* __restrict__ part_o, const float* __restrict__ part_ml, int splits, int chunk,
         const int* __restrict__ row_of_token, const int* __restrict__ positions,
         const int* __restrict__ kv_lens, const int* __restrict__ cu_q, int H, int window,
-        bf16_t* __restrict__ out, int out_stride, int rows, const int* __restrict__ single_tokens) {
+        bf16_t* __restrict__ out, int out_stride, int rows, const int* __restrict__ single_tokens, const int* __restrict__ count) {
     constexpr int LPP = HD / 4;               // lanes per row of partial results (a float4 each)
     constexpr int PPW = 64 / LPP;             // rows per load instruction of a wave
     constexpr int UNR = 4;                    // load instructions in flight
@@ -333,7 +567,7 @@ __global__ __launch_bounds__(CW * 64) void attn_decode_combine_kernel(
         return;
     }
     // the waves of the first kernel left one slot each; those beyond the row's last chunk none
-    const int n = min(splits, (visible - 1) / chunk + 1);
+    const int n = count ? count[b] : min(splits, (visible - 1) / chunk + 1);
     const float2* ml = reinterpret_cast<const float2*>(part_ml) + ((size_t)b * H + h) * splits;
     const float4* po = reinterpret_cast<const float4*>(part_o + ((size_t)b * H + h) * splits * HD);
     float m = tid < n ? m_first : -INFINITY;             // slots beyond n hold nothing of this step
@@ -394,9 +628,12 @@ static int decode_chunk(int T, int Hkv, int hd, int max_kv_len) {
     return waves128 >= 4096 ? 128 : 64;
 }
 
+// slots a row of the list's form: its waves' stretches are two spans or more
+static int list_slots(int max_kv_len) { return (max_kv_len + LIST_SPAN - 1) / LIST_SPAN / 2 + 1; }
+
 extern "C" size_t ri_attention_decode_workspace(int rows, int H, int hd, int max_kv_len) {
-    const size_t splits = (size_t)(max_kv_len + 63) / 64;        // the smaller chunk bounds both
-    return (size_t)rows * H * splits * (hd + 2) * sizeof(float);
+    const size_t splits = (size_t)list_slots(max_kv_len);       // no other form leaves more
+    return ((size_t)rows * H * splits * (hd + 2) + rows) * sizeof(float);
 }
 
 extern "C" int ri_attention_decode_supported(int H, int Hkv, int hd, int page) {
@@ -456,6 +693,28 @@ extern "C" int ri_attention_decode(
     // 50.6, 4 rows 20.3 -> 18.0 (8); head 64: 16 rows of 2,048 keys 23.8 -> 18.1, 8 rows of 4,096
     // 20.7 -> 18.1.  pair_blocks: 0 lets the entry point choose, 1 forbids several blocks a pair,
     // more asks for that many.
+    // A step of single tokens alone, three to as many as a wave has lanes: one list of spans (see the kernel; two rows of 2,050 keys take 11.3 us either
+    // way, one of 91 7.3 without and 9.0 with it; head 64: 43 rows of 210..3,000 37 / 25 us, but 16 rows of 2,050 18.4 / 19.8 and 32
+    // 27 / 31, so it keeps its blocks a row).  w total stays below 2^32.
+    const long long spans = (long long)T * ((max_kv_len + LIST_SPAN - 1) / LIST_SPAN + 1);
+    if (hd == 128 && pair_blocks == 0 && !cu_q && T >= 3 && T <= LIST_ROWS && (page & (page - 1)) == 0 && spans < (1ll << 32) / LIST_WAVES) {
+        const int W = (int)std::max(1ll, std::min<long long>(LIST_WAVES / Hkv, spans / 2));
+        const int slots = list_slots(max_kv_len);
+        float* sums = (float*)workspace;
+        float* ml = sums + (size_t)rows * H * slots * hd;
+        int* count = (int*)(ml + (size_t)rows * H * slots * 2);
+        attn_decode_list_kernel<<<dim3(W, Hkv), 64, 0, stream>>>(
+            (const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, table, max_blocks, row_of_token, positions, kv_lens, H, Hkv,
+            page, __builtin_ctz((unsigned)page), scale, window, slots, sums, ml, count, T, rows);
+        RI_LAUNCHED("ri_attention_decode(list)");
+        // a row has as many slots as waves, at most
+        const bool one = std::min(slots, W) <= 64;
+        auto combine = one ? attn_decode_combine_kernel<128, 1> : attn_decode_combine_kernel<128, 4>;
+        combine<<<dim3(T, H), one ? 64 : 256, 0, stream>>>(sums, ml, slots, 0, row_of_token, positions, kv_lens, nullptr, H, window, (bf16_t*)out,
+                                                           out_stride, rows, nullptr, count);
+        RI_LAUNCHED("ri_attention_decode(combine)");
+        return 0;
+    }
     const int bw_ = hd == 64 ? 16 : 8;
     const int chunks64_ = (max_kv_len + 63) / 64;
     const bool lds_ok = (size_t)bw_ * ((size_t)(H / Hkv) * hd + 32) * sizeof(float) <= 64 * 1024;
@@ -499,8 +758,8 @@ extern "C" int ri_attention_decode(
         if (nblk == 1) return 0;                          // the block has written the output itself
         dim3 grid2(TZ, H);
         const int block_keys = 64 * bw_;                  // a block's first chunk begins a multiple of this many keys in
-        if (hd == 64) attn_decode_combine_kernel<64, 1><<<grid2, 64, 0, stream>>>(part_o, part_ml, splits, block_keys, row_of_token, positions, kv_lens, cu_q, H, window, (bf16_t*)out, out_stride, rows, sel);
-        else attn_decode_combine_kernel<128, 1><<<grid2, 64, 0, stream>>>(part_o, part_ml, splits, block_keys, row_of_token, positions, kv_lens, cu_q, H, window, (bf16_t*)out, out_stride, rows, sel);
+        if (hd == 64) attn_decode_combine_kernel<64, 1><<<grid2, 64, 0, stream>>>(part_o, part_ml, splits, block_keys, row_of_token, positions, kv_lens, cu_q, H, window, (bf16_t*)out, out_stride, rows, sel, nullptr);
+        else attn_decode_combine_kernel<128, 1><<<grid2, 64, 0, stream>>>(part_o, part_ml, splits, block_keys, row_of_token, positions, kv_lens, cu_q, H, window, (bf16_t*)out, out_stride, rows, sel, nullptr);
         RI_LAUNCHED("ri_attention_decode(combine)");
         return 0;
     }
@@ -517,7 +776,7 @@ extern "C" int ri_attention_decode(
 #undef RI_DECODE_ARGS
     RI_LAUNCHED("ri_attention_decode");
     // more waves per (token, head) where there are many chunks to combine
-#define RI_COMBINE_ARGS part_o, part_ml, splits, chunk, row_of_token, positions, kv_lens, cu_q, H, window, (bf16_t*)out, out_stride, rows, sel
+#define RI_COMBINE_ARGS part_o, part_ml, splits, chunk, row_of_token, positions, kv_lens, cu_q, H, window, (bf16_t*)out, out_stride, rows, sel, nullptr
     if (hd == 64 && splits <= 64) attn_decode_combine_kernel<64, 1><<<grid2, 64, 0, stream>>>(RI_COMBINE_ARGS);
     else if (hd == 64) attn_decode_combine_kernel<64, 4><<<grid2, 256, 0, stream>>>(RI_COMBINE_ARGS);
     else if (splits <= 32) attn_decode_combine_kernel<128, 1><<<grid2, 64, 0, stream>>>(RI_COMBINE_ARGS);

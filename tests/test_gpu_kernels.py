@@ -706,6 +706,40 @@ def test_single_token_attention_with_several_blocks_a_pair(ops, monkeypatch, cas
     _check_rope_write_and_attention(ops, torch.bfloat16, case, window)
 
 
+@pytest.mark.parametrize("case,window", [
+    ((3, 8, 4, 128, 16, [1] * 3, [0, 0, 0]), 0),                                             # one span a row, fewer than waves
+    ((5, 12, 4, 128, 16, [1] * 5, [30, 31, 32, 63, 64]), 0),                                 # ends around a span's
+    ((9, 16, 1, 128, 64, [1] * 9, [2500, 0, 700, 15, 16, 17, 1300, 95, 3]), 0),              # 512 waves a head; rows of one span among long ones
+    ((7, 8, 8, 128, 32, [1] * 7, [4200, 63, 4159, 10, 1024, 4223, 17]), 700),
+    ((4, 6, 2, 128, 16, [1] * 4, [999, 1000, 1001, 1040]), 33),                              # a window that begins inside a span
+    ((64, 8, 2, 128, 16, [1] * 64, [(i * 37) % 211 for i in range(64)]), 0),                 # a row a lane
+    ((65, 8, 2, 128, 16, [1] * 65, [(i * 37) % 211 for i in range(65)]), 0),                 # one more: not as a list
+])
+def test_single_token_attention_of_rows_of_any_lengths(ops, case, window):
+    """Rows' keys as one list whose stretches end anywhere in a row; slots never written and pages given back are NaN."""
+    _check_rope_write_and_attention(ops, torch.bfloat16, case, window)
+
+
+def test_single_token_attention_as_a_list_with_padding_and_rows_out_of_order(ops):
+    B, H, Hkv, hd, page = 6, 8, 2, 128, 16
+    lens = [300, 7, 1200, 64, 65, 500]
+    qkv, kc, vc, table, ctx, _, _ = _paged_setup(torch.bfloat16, B, H, Hkv, hd, page, [1] * B, [n - 1 for n in lens], seed=3, num_pages=160)
+    ops.rope_kv_write(qkv, H, Hkv, hd, None, ctx.positions, ctx.row_of_token, kc, vc, table, page)
+    want = torch.empty(B, H * hd, dtype=torch.bfloat16, device=DEV)
+    ops.paged_attention(qkv, want, H, Hkv, hd, kc, vc, table, page, ctx, 0.1, 0)
+    order = [4, -1, 2, 0, -1, 5, 3, 1]                                     # token -> row
+    at = torch.tensor([max(b, 0) for b in order], device=DEV)
+    ctx.num_tokens, ctx.num_rows = len(order), B
+    ctx.row_of_token, ctx.positions = torch.tensor(order, dtype=torch.int32, device=DEV), ctx.positions[at].contiguous()
+    got = torch.full((len(order), H * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.paged_attention(qkv[at].contiguous(), got, H, Hkv, hd, kc, vc, table, page, ctx, 0.1, 0)
+    for t, b in enumerate(order):
+        if b < 0:
+            assert torch.all(got[t] == 0)
+        else:                                                              # stretches of the list end elsewhere: rounding of the output
+            assert torch.allclose(got[t].float(), want[b].float(), rtol=2.0 ** -7, atol=1e-3), t
+
+
 def _check_rope_write_and_attention(ops, dtype, case, window, kv_heads=None):
     B, H, Hkv, hd, page, q_lens, starts = case
     need = sum((s + q + page - 1) // page for s, q in zip(starts, q_lens))
