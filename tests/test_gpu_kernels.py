@@ -489,6 +489,29 @@ def test_linear_f32_of_more_tiles_than_a_launch_holds(ops):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("T,n,group,pad", [(1, 8, 8, 0), (3, 2048, 2048, 0), (5, 2304, 256, 8), (2, 3072, 1024, 16), (7, 1024, 512, 0), (4, 4096, 2048, 8), (3, 192, 64, 4),
+                                           (2, 72, 24, 0), (2, 4096, 4096, 0), (300, 128, 16, 8)])
+@pytest.mark.parametrize("dtype,w_dtype", [(torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
+def test_gated_group_norm_of_eight_values_a_thread(ops, T, n, group, pad, dtype, w_dtype):
+    # groups in a few lanes, a wave, two and four waves; rows that end inside a block; and what the other kernel keeps (strides, sizes)
+    o = (rnd(T, n + pad, seed=n) * 3)[:, :n]
+    gate = rnd(T, n + pad, seed=1).to(dtype)[:, :n]
+    w = (rnd(n, seed=2) + 1).to(w_dtype)
+    for kw in (dict(), dict(gate_activation="silu"), dict(gate_activation="silu", gate_first=True)):
+        for weight, z in ((w, gate), (None, gate), (w, None)):
+            out = torch.full((T, n + 8), float("nan"), dtype=dtype, device=DEV)
+            ops.gated_group_norm(o, weight, z, out[:, :n], group, 1e-5, **kw)
+            a = o.double()
+            g = torch.ones_like(a) if z is None else torch.sigmoid(z.double()) if not kw else torch.nn.functional.silu(z.double())
+            if kw.get("gate_first"):
+                a, g = a * g, torch.ones_like(g)
+            y = a.view(T, -1, group)
+            y = (y / torch.sqrt(y.square().mean(-1, keepdim=True) + 1e-5)).reshape(T, n) * g * (1.0 if weight is None else weight.double())
+            tol = 2e-6 if dtype == torch.float32 else 2.0 ** -8 + 2e-6          # rounding, and 32-bit arithmetic
+            assert torch.all((out[:, :n].double() - y).abs() <= tol * y.abs() + 1e-6)
+            assert torch.isnan(out[:, n:]).all()
+
+
 def _paged_setup(dtype, B, H, Hkv, hd, page, q_lens, starts, seed=0, num_pages=128, shuffle=True):
     """A cache with random pages for each request, the step's q/k/v, and contiguous copies."""
     g = torch.Generator().manual_seed(seed)
