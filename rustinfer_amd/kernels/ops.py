@@ -810,6 +810,35 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: Optiona
                              M, N, K, _dt(x), _dt(out), _stream()))
 
 
+def linear_activated(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: Optional[torch.Tensor], acts) -> None:
+    """``linear``, and for each ``(c0, n, name, dst)`` of ``acts``: ``dst [M, n] = f(out[:, c0:c0 + n])`` for ``f`` in
+    ``UNARY``; ``dst`` may be those columns of ``out`` (columns whose ``dst`` is another buffer need not be
+    left in ``out``).  Few bfloat16 rows: in the product's own epilogue, on sums that have not been rounded."""
+    M, K = x.shape
+    N = w.shape[0]
+    lds = N >= ROWS_LDS_WIDE_COLUMNS and out.stride(0) % 4 == 0 and _rows_ok(x, w, w_tiled, M, N, K)      # as `linear` routes it
+    if 0 < len(acts) <= 2 and not lds and _skinny_ok(x, w, M, K) and _tiled_ok(w, w_tiled) and N % 16 == 0 and K % 32 == 0 \
+            and out.dtype == torch.bfloat16 and all(c0 % 16 == 0 and n % 16 == 0 and dst.dtype == torch.bfloat16 for c0, n, _, dst in acts):
+        _dev(x, w, out, *(dst for _, _, _, dst in acts))
+        _rows2d(x, "x")
+        _rows2d(out, "out")
+        if w.shape[1] != K or tuple(out.shape) != (M, N):
+            raise KernelError(f"linear_activated: shapes {tuple(x.shape)} x {tuple(w.shape)}^T -> {tuple(out.shape)} do not fit")
+        for c0, n, name, dst in acts:
+            _rows2d(dst, "dst")
+            if name not in UNARY or tuple(dst.shape) != (M, n) or c0 + n > N:
+                raise KernelError(f"linear_activated: unknown function {name!r}, or columns {c0} to {c0 + n} do not fit")
+        ints = lambda v: (ctypes.c_int * len(acts))(*v)
+        _check(_lib().ri_gemm_skinny_activated(
+            _ptr(x), x.stride(0), _ptr(w_tiled), _ptr(out), out.stride(0), M, N, K, len(acts), ints([a[0] for a in acts]),
+            ints([a[0] + a[1] for a in acts]), ints([UNARY[a[2]] for a in acts]), (ctypes.c_void_p * len(acts))(*[a[3].data_ptr() for a in acts]),
+            ints([a[3].stride(0) for a in acts]), _stream()))
+        return
+    linear(x, w, out, w_tiled)
+    for c0, n, name, dst in acts:
+        unary(name, out[:, c0:c0 + n], dst)
+
+
 def linear_delta(x: torch.Tensor, w: torch.Tensor, workspace, name: str,
                  w_tiled: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """``x @ w^T`` as a residual delta for ``add_rmsnorm``: ``[M, N]`` in the dtype of ``x``, or,

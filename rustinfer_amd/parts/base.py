@@ -364,6 +364,12 @@ class ProjectedPart(Part):
         pairs of neighbouring features may ask for the pairs' halves apart, say); as stored by default."""
         return w
 
+    def in_activations(self):
+        """``{in-projection: (function, into_act)}``: elementwise functions (of the kernels' list) that are to be applied to
+        projected rows before ``core`` sees them, in their place or (``into_act``) into the part's columns of the
+        activations: the product can do that on its way."""
+        return {}
+
     def core(self, ctx, proj, act, cache) -> None:
         raise NotImplementedError
 
@@ -466,12 +472,21 @@ class ProjectionSet:
         self.w_in.set_weight(w_in, rt)
         self.w_out.set_weight(w_out, rt)
 
-    def project(self, ctx, normed):
-        """(projected rows [T, n_in], the buffer [T, n_act] the parts' ``core`` fill)."""
+    def project(self, ctx, normed, members=None):
+        """(projected rows [T, n_in], the buffer [T, n_act] the parts' ``core`` fill), the parts' ``in_activations`` applied
+        (``members``: of the first so many parts alone, where the others' ``core`` does not run)."""
         T = normed.shape[0]
         proj = ctx.workspace.get("projset.in", T, self.n_in, self.rt.dtype)
-        self.w_in.forward(normed, proj)
         act = ctx.workspace.get("projset.act", T, self.n_act, self.rt.dtype)
+        acts = []
+        for i, (_, part) in enumerate(self.members[:members]):
+            for name, (f, into_act) in part.in_activations().items():
+                c0, rows = self.in_slices[i][name]
+                acts.append((c0, rows, f, self.act_view(i, act) if into_act else proj[:, c0:c0 + rows]))
+        if acts:
+            self.rt.ops.linear_activated(normed, self.w_in.weight, proj, self.w_in.weight_tiled, acts)
+        else:
+            self.w_in.forward(normed, proj)
         for a, b in self._gaps:                          # scratch may hold anything, and 0 * NaN is NaN
             act[:, a:b].zero_()
         return proj, act

@@ -257,7 +257,7 @@ class ParallelBlock(Part):
     def _run(self, ctx, hidden: Hidden, cache, mixer_only: bool):
         normed = ctx.workspace.get("block.normed", hidden.x.shape[0], self.hidden_size, self.rt.dtype)
         inp = hidden.input_behind(ctx, self.norm, normed)
-        proj, act = self.set.project(ctx, inp)
+        proj, act = self.set.project(ctx, inp, members=int(self.mixer is not None) if mixer_only else None)
         i = 0
         if self.mixer is not None:
             self.mixer.core(ctx, self.set.views(0, proj), self.set.act_view(0, act), cache)

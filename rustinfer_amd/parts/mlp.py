@@ -94,8 +94,11 @@ class DenseMLP(ProjectedPart, FeedForward):
     def out_projection(self):
         return (self.down_name, self.intermediate_size)
 
+    def in_activations(self):
+        return {self.up_name: (self.activation, True)}
+
     def core(self, ctx, proj, act, cache=None) -> None:
-        self.rt.ops.unary(self.activation, proj[self.up_name], act)
+        return None                                  # the activation is all there is between the products
 
     def forward(self, ctx, normed):
         return ProjectedPart.forward(self, ctx, normed, None)

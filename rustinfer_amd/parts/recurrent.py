@@ -114,11 +114,13 @@ class GeneralDeltaRule(ProjectedPart, Mixer):
         self.w0, self.a_bias, self.norm_weight = f32(n["w0"]), f32(n["a_bias"]), f32(n["norm"])
         self.w2.set_weight(tensors[n["w2"]], rt)
 
+    def in_activations(self):
+        return {self.names["w1"]: ("tanh", False)}
+
     def core(self, ctx, proj, act, cache) -> None:
         ops, n = self.rt.ops, self.names
         T, hd = act.shape[0], self.num_heads * self.head_dim
         w1 = proj[n["w1"]]
-        ops.unary("tanh", w1, w1)
         wl = ctx.workspace.get("gdr.wl", T, hd, self.rt.dtype)
         self.w2.forward(w1, wl)
         o = ctx.workspace.get("scan.o", T, hd, torch.float32)

@@ -489,6 +489,33 @@ def test_linear_f32_of_more_tiles_than_a_launch_holds(ops):
     torch.cuda.empty_cache()
 
 
+@pytest.mark.parametrize("M,N,K,acts", [(1, 64, 32, [(0, 64, "relu2")]), (8, 2064, 64, [(16, 2048, "relu2")]), (5, 96, 96, [(16, 16, "tanh"), (48, 32, "relu2")]),
+                                        (16, 32800, 64, [(32784, 16, "tanh"), (0, 32768, "relu2")]), (17, 4112, 128, [(2048, 2064, "relu2")]), (40, 160, 2048, [(0, 32, "tanh"), (144, 16, "relu2")]),
+                                        (64, 16400, 32, [(0, 16400, "relu2")]), (9, 80, 32, [(8, 24, "tanh")]), (70, 64, 64, [(16, 32, "relu2")])])
+def test_linear_with_activated_columns(ops, M, N, K, acts):
+    """In the product's epilogue (edges of tiles and of the stretches, one and several tiles a wave) and behind it (more rows, columns that
+    begin inside a tile): against 64-bit arithmetic on the unrounded sums, and nothing else is touched."""
+    x = rnd(M, K, seed=M).to(torch.bfloat16)
+    w = (rnd(N, K, seed=N) * 0.2).to(torch.bfloat16)
+    out = torch.full((M, N + 8), float("nan"), dtype=torch.bfloat16, device=DEV)
+    bufs = [torch.full((M, n + 24), float("nan"), dtype=torch.bfloat16, device=DEV) for _, n, _ in acts]
+    given = [(c0, n, f, out[:, c0:c0 + n] if f == "tanh" else b[:, 8:8 + n]) for (c0, n, f), b in zip(acts, bufs)]
+    ops.linear_activated(x, w, out[:, :N], ops.tile_weight(w) if N % 16 == 0 and K % 32 == 0 else None, given)
+    ref = x.double() @ w.double().t()
+    plain = torch.ones(N, dtype=torch.bool)
+    for (c0, n, f), b in zip(acts, bufs):
+        z = ref[:, c0:c0 + n]
+        want = torch.relu(z).square() if f == "relu2" else torch.tanh(z)
+        got = out[:, c0:c0 + n] if f == "tanh" else b[:, 8:8 + n]
+        # bfloat16 rounds to 2^-8: the result, and behind the product the sum too, which the square doubles; 2^-6 covers the three
+        assert torch.all((got.double() - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -8 * z.abs().clamp(max=1.0) * (f == "tanh") + 1e-4)
+        if f == "relu2":
+            assert torch.isnan(b[:, :8]).all() and torch.isnan(b[:, 8 + n:]).all()
+        plain[c0:c0 + n] = False
+    assert torch.all((out[:, :N][:, plain].double() - ref[:, plain]).abs() <= 2.0 ** -8 * ref[:, plain].abs() + 1e-4)
+    assert torch.isnan(out[:, N:]).all()
+
+
 @pytest.mark.parametrize("T,n,group,pad", [(1, 8, 8, 0), (3, 2048, 2048, 0), (5, 2304, 256, 8), (2, 3072, 1024, 16), (7, 1024, 512, 0), (4, 4096, 2048, 8), (3, 192, 64, 4),
                                            (2, 72, 24, 0), (2, 4096, 4096, 0), (300, 128, 16, 8)])
 @pytest.mark.parametrize("dtype,w_dtype", [(torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
