@@ -32,9 +32,10 @@
 // are not finite (a token's vectors were not, or k / W_t left the range of 32 bits) is therefore only marked; the states
 // stop in front of it, and the walk does that head of that row from there on, so that every token gets what the walk gives.
 //
-// 2,048 tokens of 32 heads of 64, us a layer: delta form 1174 -> 260, decay form 789 -> 109; 24 heads of 128: 1692 -> 617, 977 ->
-// 188 (with 32-bit sums 223, 96, 551 and 173).  The operators are bound by the steps of a block following each other (two
-// blocks a compute unit), the states by the chain of chunks.
+// 2,048 tokens of 32 heads of 64, us a layer, the walk / this: delta form 1174 / 223, decay form 789 / 96; 24 heads of 128: 1692 / 583, 977 /
+// 192.  The operators (163 and 50 of the first two) are bound by the steps of a block following each other (two
+// blocks a compute unit), the states (86, 55) by the chain of chunks: 64 chunks of about 1.3 us, 0.5 of which are its matrix instructions
+// (101, 69 with two waves, and with loads under a lane's condition, which the compiled loop waited for, 123 and 69).
 #include "common.h"
 #include <mutex>
 
@@ -451,17 +452,21 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
 // v_mfma_f32_16x16x4_f32 a result (row 4 g + i, column l % 16 in element i of lane 16 g + l % 16) is the operand of
 // the next product as it lies, for the four k values {16 a + 4 g + i}: the operators are stored for that order.  The
 // waves hand their rows to each other through LDS.
+// Tiles of 16 key rows of the state a wave: one where a chunk's operators fit two waves more beside each other, us a layer of 2,048
+// tokens, 32 heads of 64, two tiles / one: delta form 101 / 86; the decay form, whose waves then no longer all have outputs, 55 / 69.
+constexpr int state_tiles(int dk, bool delta) { return delta && dk <= 64 ? 1 : 2; }
+
 template <int DK, int DV, bool DELTA>
-__global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a) {
-    constexpr int NW = DK / 32, NA = DK / 16;
+__global__ __launch_bounds__(DK * 4 / state_tiles(DK, DELTA)) void chunk_states_kernel(const ChunkArgs a) {
+    constexpr int Q = state_tiles(DK, DELTA), NA = DK / 16, NW = NA / Q;
     using U = Unit<DK, DV, DELTA>;
-    const int b = a.rows ? a.rows[blockIdx.z] : (int)blockIdx.z, h = blockIdx.y, cb = blockIdx.x;
+    const int b = a.rows ? a.rows[blockIdx.z] : (int)blockIdx.z, h = blockIdx.x, cb = blockIdx.y;
     if (b < 0) return;
     const int t_lo = a.cu_q[b], n = a.cu_q[b + 1] - t_lo;
     if (n < a.min_tokens || a.c0 * C >= n) return;
     int* const from = a.from + ((size_t)b * a.H + h) * (DV / 16) + cb;       // (this block's own, the same in all of a head's)
     if (a.c0 > 0 && *from < a.c0 * C) return;          // the walk takes the row over before this segment
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, col = lane & 15, g = lane >> 4;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, g = lane >> 4;
     const int all = min(a.seg, (n + C - 1) / C - a.c0);          // at most 64
     const float* units = a.ws + ((size_t)blockIdx.z * a.seg * a.H + h) * U::SIZE;
     const unsigned long long bads = __ballot(lane < all && reinterpret_cast<const int*>(units + (size_t)lane * a.H * U::SIZE)[U::BAD] != 0);
@@ -470,24 +475,24 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
     __shared__ __align__(16) f32x4_t St[2][NA][64];
     float* Sg = a.state + ((size_t)a.slots[b] * a.H + h) * (size_t)DK * DV + cb * 16 + col;
     const bool fresh = a.c0 == 0 && a.q_start[b] == 0;
-    f32x4_t S[2];
+    f32x4_t S[Q];
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int q = 0; q < Q; ++q)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) S[q][i] = fresh ? 0.f : Sg[(size_t)((wave * 2 + q) * 16 + 4 * g + i) * DV];
-    struct Ops { f32x4_t m[DELTA ? 2 : 1][DELTA ? NA : 1], w[DELTA ? 2 : 1], r[NA], add[2], o; };
-    const bool outputs = wave < 2;               // two tiles of 16 tokens
+        for (int i = 0; i < 4; ++i) S[q][i] = fresh ? 0.f : Sg[(size_t)((wave * Q + q) * 16 + 4 * g + i) * DV];
+    struct Ops { f32x4_t m[DELTA ? Q : 1][DELTA ? NA : 1], w[DELTA ? Q : 1], r[NA], add[Q], o; };
+    const bool outputs = NW == 2 || wave < 2;    // two tiles of 16 tokens
     const float d = DELTA ? 0.f : a.decay[h];
     const double d_chunk = DELTA ? 0.0 : power(d, C);
     auto ask = [&](int c, Ops& x) {
         const f32x4_t* unit = reinterpret_cast<const f32x4_t*>(units + (size_t)c * a.H * U::SIZE);
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
-            x.add[q] = unit[U::S / 4 + (cb * NA + wave * 2 + q) * 64 + lane];
+        for (int q = 0; q < Q; ++q) {
+            x.add[q] = unit[U::S / 4 + (cb * NA + wave * Q + q) * 64 + lane];
             if (DELTA) {
 #pragma unroll
-                for (int k = 0; k < NA; ++k) x.m[q][k] = unit[U::M / 4 + ((wave * 2 + q) * NA + k) * 64 + lane];
-                x.w[q] = unit[U::W / 4 + (wave * 2 + q) * 4 + g];
+                for (int k = 0; k < NA; ++k) x.m[q][k] = unit[U::M / 4 + ((wave * Q + q) * NA + k) * 64 + lane];
+                x.w[q] = unit[U::W / 4 + (wave * Q + q) * 4 + g];
             }
         }
         if (outputs) {
@@ -495,27 +500,28 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
             for (int k = 0; k < NA; ++k) x.r[k] = unit[U::R / 4 + (wave * NA + k) * 64 + lane];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int t = (a.c0 + c) * C + wave * 16 + 4 * g + i;
-                x.o[i] = t < n ? a.out[(size_t)(t_lo + t) * a.out_stride + h * DV + cb * 16 + col] : 0.f;
+                const int t = min((a.c0 + c) * C + wave * 16 + 4 * g + i, n - 1);          // what lies behind the last token is not stored
+                x.o[i] = a.out[(size_t)(t_lo + t) * a.out_stride + h * DV + cb * 16 + col];
             }
         }
     };
     auto step = [&](int c, Ops& x) {
 #pragma unroll
-        for (int q = 0; q < 2; ++q) St[c & 1][wave * 2 + q][lane] = S[q];
+        for (int q = 0; q < Q; ++q) St[c & 1][wave * Q + q][lane] = S[q];
         asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");      // LDS only: the next chunk's loads stay under way
         const double dc = DELTA ? 0.0 : ((a.c0 + c + 1) * C <= n ? d_chunk : power(d, n - (a.c0 + c) * C));
         // the instruction adds in order: short chains, for the outputs of 8 or 16 products
         constexpr int CH = 4, CO = 8;
-        f32x4_t next[2][CH] = {}, o[CO] = {};
+        f32x4_t next[Q][CH] = {}, o[CO] = {};
 #pragma unroll
         for (int k = 0; k < NA; ++k) {
             const f32x4_t s = St[c & 1][k][lane];
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 if (DELTA) {
-                    next[0][(4 * k + i) % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[0][k][i], s[i], next[0][(4 * k + i) % CH], 0, 0, 0);
-                    next[1][(4 * k + i) % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[1][k][i], s[i], next[1][(4 * k + i) % CH], 0, 0, 0);
+#pragma unroll
+                    for (int q = 0; q < Q; ++q)
+                        next[q][(4 * k + i) % CH] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.m[q][k][i], s[i], next[q][(4 * k + i) % CH], 0, 0, 0);
                 }
                 if (outputs) o[(4 * k + i) % CO] = __builtin_amdgcn_mfma_f32_16x16x4f32(x.r[k][i], s[i], o[(4 * k + i) % CO], 0, 0, 0);
             }
@@ -530,7 +536,7 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
         }
         // the new state, rounded once
 #pragma unroll
-        for (int q = 0; q < 2; ++q) {
+        for (int q = 0; q < Q; ++q) {
             const f32x4_t whole = (next[q][0] + next[q][1]) + (next[q][2] + next[q][3]);
 #pragma unroll
             for (int i = 0; i < 4; ++i)
@@ -539,20 +545,30 @@ __global__ __launch_bounds__(DK * 2) void chunk_states_kernel(const ChunkArgs a)
         }
     };
     static_assert(NW >= 2, "two waves make the outputs");
-    Ops x0, x1;
-    if (chunks > 0) ask(0, x0);
-    for (int c = 0; c < chunks; c += 2) {
-        if (c + 1 < chunks) ask(c + 1, x1);
-        step(c, x0);
-        if (c + 1 < chunks) {
-            if (c + 2 < chunks) ask(c + 2, x0);
-            step(c + 1, x1);
-        }
+    // D chunks' operands under way, asked for under no condition (the last one's again behind the end): at a place that can be
+    // reached with fewer loads under way the compiled code would wait for more of them.
+    // (Heads of 128: with three, 2,048 tokens of 24 heads 192 -> 179 us in the decay form, but three rows of 200 67 -> 75.)
+    constexpr int D = DK > 64 ? 2 : 4;
+    Ops x[D];
+    if (chunks > 0) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) ask(min(d, chunks - 1), x[d]);
+        int c = 0;
+        for (; c + D <= chunks; c += D)
+#pragma unroll
+            for (int d = 0; d < D; ++d) {
+                step(c + d, x[d]);
+                ask(min(c + d + D, chunks - 1), x[d]);
+                __builtin_amdgcn_sched_barrier(0);
+            }
+#pragma unroll
+        for (int d = 0; d < D - 1; ++d)
+            if (c + d < chunks) step(c + d, x[d]);
     }
 #pragma unroll
-    for (int q = 0; q < 2; ++q)
+    for (int q = 0; q < Q; ++q)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) Sg[(size_t)((wave * 2 + q) * 16 + 4 * g + i) * DV] = S[q][i];
+        for (int i = 0; i < 4; ++i) Sg[(size_t)((wave * Q + q) * 16 + 4 * g + i) * DV] = S[q][i];
 }
 
 template <int DK, int DV, bool DELTA>
@@ -576,7 +592,7 @@ int launch_chunks(ChunkArgs a, int rows, int max_tokens, hipStream_t stream) {
     const int chunks = (max_tokens + C - 1) / C;
     for (a.c0 = 0; a.c0 < chunks; a.c0 += a.seg) {
         operators<<<dim3(min(a.seg, chunks - a.c0), a.H, rows), 256, lds, stream>>>(a);
-        chunk_states_kernel<DK, DV, DELTA><<<dim3(DV / 16, a.H, rows), DK * 2, 0, stream>>>(a);
+        chunk_states_kernel<DK, DV, DELTA><<<dim3(a.H, DV / 16, rows), DK * 4 / state_tiles(DK, DELTA), 0, stream>>>(a);     // a head on one XCD: its blocks read the same operators
     }
     return 0;
 }
