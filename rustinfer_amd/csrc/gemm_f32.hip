@@ -158,7 +158,9 @@ __global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
 // kernel: 2048 x 2048 10.3 / 6.7, 3072 x 2048 10.8 / 10.2, 16384 x 2048 41 / 31 (134 MB: 4.3 TB/s),
 // 2048 x 8192 33 / 17.6, 128256 x 2048 264 / 193 (5.4 TB/s).  Four rows, against FMAs with the lanes' sums added up in a tree: 3072 x 2048
 // 11.5 / 9.9, 16384 x 2048 36 / 30, 2048 x 8192 23.5 / 17.1, 28672 x 4096 100 / 87, 4096 x 14336 53 / 55, 128256 x 2048 182 / 188.
-template <int NT, int D>
+// SWIGLU: W is [2N, K] (gate rows, then up rows), a block's two tiles are the gate's and the up rows of the same eight columns, and
+// C = silu(gate) * up of the rounded sums: the activation's kernel (4.3 us for 6 rows of 8,192) and what it reads and writes.
+template <int NT, int D, bool SWIGLU = false>
 __global__ __launch_bounds__(256) void gemm_f32_few_kernel(
         const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
         float* __restrict__ C, int ldc, int M, int N, int K) {
@@ -166,21 +168,24 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(
     __shared__ double sums[8][8][NT * 8];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 7, second = (lane >> 3) & 1, g = lane >> 4;
-    const int n0 = (int)blockIdx.x * NT * 8;
+    static_assert(!SWIGLU || NT == 2, "a tile of gate rows and one of up rows");
+    constexpr int COLS = SWIGLU ? 8 : NT * 8;
+    const int n0 = (int)blockIdx.x * COLS;
     const char* abase = reinterpret_cast<const char*>(A + wave * 32);
     const char* wbase = reinterpret_cast<const char*>(W + (size_t)n0 * ldw + wave * 32);
+    const char* ubase = SWIGLU ? reinterpret_cast<const char*>(W + ((size_t)N + n0) * ldw + wave * 32) : wbase;     // of the last tile
     const int kl = second * 128 + 4 * g;
     const uint32_t arow = ((uint32_t)min(r, M - 1) * (uint32_t)lda + kl) * 4;
     uint32_t wrow[NT];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) wrow[j] = ((uint32_t)min(j * 8 + r, N - 1 - n0) * (uint32_t)ldw + kl) * 4;
+    for (int j = 0; j < NT; ++j) wrow[j] = ((uint32_t)min((SWIGLU ? 0 : j * 8) + r, N - 1 - n0) * (uint32_t)ldw + kl) * 4;
     f64x4_t acc[NT] = {};
     auto ask = [&](int turn, float4 (&a)[2], float4 (&w)[2][NT]) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
             const size_t at = ((size_t)turn * TURN + 16 * u) * 4;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) w[u][j] = ld_stream16<float4>(wbase + at + wrow[j]);
+            for (int j = 0; j < NT; ++j) w[u][j] = ld_stream16<float4>((j == NT - 1 ? ubase : wbase) + at + wrow[j]);
             a[u] = *reinterpret_cast<const float4*>(abase + at + arow);
         }
     };
@@ -238,7 +243,7 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(
             const size_t at = ((size_t)whole * TURN + 16 * u) * 4;
 #pragma unroll
             for (int j = 0; j < NT; ++j)
-                w[0][u][j] = in ? *reinterpret_cast<const float4*>(wbase + at + wrow[j]) : make_float4(0.f, 0.f, 0.f, 0.f);
+                w[0][u][j] = in ? *reinterpret_cast<const float4*>((j == NT - 1 ? ubase : wbase) + at + wrow[j]) : make_float4(0.f, 0.f, 0.f, 0.f);
             a[0][u] = in ? *reinterpret_cast<const float4*>(abase + at + arow) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         add(a[0], w[0]);
@@ -248,12 +253,17 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(
 #pragma unroll
         for (int e = 0; e < 2; ++e) sums[wave + 4 * second][4 * e + g][j * 8 + r] = second ? acc[j][2 + e] : acc[j][e];
     __syncthreads();
-    for (int e = threadIdx.x; e < 8 * NT * 8; e += 256) {
-        const int row = e / (NT * 8), col = e % (NT * 8);
+    auto sum = [&](int row, int col) {
         double v = sums[0][row][col];
 #pragma unroll
         for (int i = 1; i < 8; ++i) v += sums[i][row][col];
-        if (row < M && n0 + col < N) C[(size_t)row * ldc + n0 + col] = (float)v;
+        return (float)v;
+    };
+    for (int e = threadIdx.x; e < 8 * COLS; e += 256) {
+        const int row = e / COLS, col = e % COLS;
+        float v = sum(row, col);
+        if (SWIGLU) v = v / (1.f + expf(-v)) * sum(row, 8 + col);
+        if (row < M && n0 + col < N) C[(size_t)row * ldc + n0 + col] = v;
     }
 }
 
@@ -299,6 +309,19 @@ extern "C" void ri_gemm_f32_tile(int M, int N, int* rows, int* columns) {
     const F32Tile& t = F32_TILES[f32_tile(M, N)];
     *rows = 16 * t.mt;
     *columns = 16 * t.nt;
+}
+
+// C[M, N] = silu(A . gate^T) * (A . up^T) of up to eight rows, W = [gate; up] of 2N rows: what ri_gemm_f32 and the activation's kernel
+// give, bit for bit.
+extern "C" int ri_gemm_f32_swiglu(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
+                                  int M, int N, int K, hipStream_t stream) {
+    RI_REQUIRE(M >= 1 && M <= 8 && N > 0 && K > 0 && K % 4 == 0, "ri_gemm_f32_swiglu: needs 1 to 8 rows and K %% 4 == 0 (M=%d N=%d K=%d)", M, N, K);
+    RI_REQUIRE(lda >= K && ldw >= K && ldc >= N && lda % 4 == 0 && ldw % 4 == 0 && lda <= (1 << 24) && ldw <= (1 << 24),
+               "ri_gemm_f32_swiglu: leading dimensions must be >= K, multiples of 4 and at most 2^24");
+    RI_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && N <= (1 << 26), "ri_gemm_f32_swiglu: null or unaligned pointer, or N=%d", N);
+    gemm_f32_few_kernel<2, 4, true><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    RI_LAUNCHED("ri_gemm_f32_swiglu");
+    return 0;
 }
 
 // The 32-bit product of any number of rows (K % 4 == 0, operands and rows 16-byte aligned).

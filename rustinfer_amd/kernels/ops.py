@@ -925,6 +925,10 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor,
         raise KernelError("linear_swiglu: row factors of a deferred norm go with the few-row bfloat16 kernel only")
     if scratch is None or tuple(scratch.shape) != (M, 2 * I):
         raise KernelError("linear_swiglu: needs scratch [M, 2I] for this size")
+    if x.dtype == torch.float32 and M <= 8 and K % 4 == 0 and all(t.stride(0) % 4 == 0 and t.stride(0) <= 1 << 24 and t.data_ptr() % 16 == 0 for t in (x, w_gate_up)):
+        # the exact path's few rows: the activation in the product's epilogue, the same bits
+        _check(_lib().ri_gemm_f32_swiglu(_ptr(x), x.stride(0), _ptr(w_gate_up), w_gate_up.stride(0), _ptr(out), out.stride(0), M, I, K, _stream()))
+        return
     linear(x, w_gate_up, scratch)
     swiglu(scratch, out)
 

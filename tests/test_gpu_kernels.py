@@ -457,6 +457,17 @@ def test_linear_f32_of_up_to_eight_rows(ops, M, N, K):
         assert torch.equal(bad[:M - 1], out[:M - 1, :N]) and torch.all(torch.isnan(bad[M - 1]))
 
 
+@pytest.mark.parametrize("M,I,K", [(1, 1, 4), (8, 7, 132), (3, 8, 288), (6, 4099, 1028), (5, 24, 2304), (2, 9001, 160)])
+def test_swiglu_f32_of_up_to_eight_rows_is_the_product_and_the_activation(ops, M, I, K):
+    x, w = rnd(M, K + 4, seed=M)[:, :K], rnd(2 * I, K, seed=I) * 0.3
+    scratch, want = torch.empty(M, 2 * I, device=DEV), torch.empty(M, I, device=DEV)
+    ops.linear(x, w, scratch)
+    ops.swiglu(scratch, want)
+    out = torch.full((M, I + 5), float("nan"), device=DEV)
+    ops.linear_swiglu(x, w, out[:, :I], torch.empty(M, 2 * I, device=DEV))
+    assert torch.equal(out[:, :I], want) and torch.isnan(out[:, I:]).all()
+
+
 @pytest.mark.parametrize("M", [3, 20])
 def test_linear_f32_of_rows_further_apart_than_32_bit_distances_reach(ops, M):
     far, K = (1 << 24) + 4, 12                          # 48 rows of such a distance: over 3 GiB
