@@ -159,7 +159,8 @@ __global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
 // 2048 x 8192 33 / 17.6, 128256 x 2048 264 / 193 (5.4 TB/s).  Four rows, against FMAs with the lanes' sums added up in a tree: 3072 x 2048
 // 11.5 / 9.9, 16384 x 2048 36 / 30, 2048 x 8192 23.5 / 17.1, 28672 x 4096 100 / 87, 4096 x 14336 53 / 55, 128256 x 2048 182 / 188.
 // SWIGLU: W is [2N, K] (gate rows, then up rows), a block's two tiles are the gate's and the up rows of the same eight columns, and
-// C = silu(gate) * up of the rounded sums: the activation's kernel (4.3 us for 6 rows of 8,192) and what it reads and writes.
+// C = silu(gate) * up of the rounded sums, in place of the activation's kernel (six requests generating 12 tokens at the 1B sizes 32.81 -> 32.64 ms:
+// two streams of eight rows take most of what the launch of 4.3 us gives back).
 template <int NT, int D, bool SWIGLU = false>
 __global__ __launch_bounds__(256) void gemm_f32_few_kernel(
         const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
