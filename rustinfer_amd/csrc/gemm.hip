@@ -85,6 +85,99 @@ extern "C" int ri_gemm_tiled(const void* A, int lda, const void* W, int ldw, voi
 }
 
 // ---------------------------------------------------------------------------
+// gemm_rows_f32: the exact path's product of up to 4 rows where gemm_f32_rows_pay (gemm_f32.hip) says so.  The weights are
+// streamed once, a kilobyte of a row a load instruction; a block brings 512 values of every activation row into LDS and its
+// four waves multiply them with two or four weight rows each.  Sums are kept in 64-bit; a lane adds its share of K in
+// a fixed order and the lanes are added in a fixed tree, so a row's result depends neither on the
+// other rows nor on their number (against the matrix instruction's order: to the rounding of a 64-bit sum).  K % 4 == 0.
+// ---------------------------------------------------------------------------
+template <int MR, int NB>
+__global__ __launch_bounds__(256) void gemm_rows_f32_kernel(
+        const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
+        float* __restrict__ C, int ldc, int M, int N, int K) {
+    constexpr int KC = 512;
+    __shared__ __align__(16) float xs[MR][KC];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int n0 = ((int)blockIdx.x * 4 + wave) * NB;
+    const float* wrow[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) wrow[j] = W + (size_t)min(n0 + j, N - 1) * ldw;
+    double acc[MR][NB];
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) acc[m][j] = 0.0;
+    // The weights are read once (the streaming form of the load) and a stretch ahead: while the
+    // sums of one stretch are made, the loads of the next are under way.
+    auto ask = [&](int k0, float4 (&w)[KC / 256][NB]) {
+#pragma unroll
+        for (int i = 0; i < KC / 256; ++i) {
+            const int k = k0 + i * 256 + lane * 4;
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+                w[i][j] = k < K ? ld_stream16<float4>(wrow[j] + k) : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    auto stretch = [&](int k0, const float4 (&w)[KC / 256][NB], float4 (&w_next)[KC / 256][NB]) {
+        __syncthreads();                                        // the last stretch has been read
+        for (int e = threadIdx.x * 4; e < MR * KC; e += 256 * 4) {
+            const int m = e / KC, k = k0 + e % KC;
+            float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (m < M && k < K) v = *reinterpret_cast<const float4*>(A + (size_t)m * lda + k);
+            *reinterpret_cast<float4*>(&xs[m][e % KC]) = v;
+        }
+        ask(k0 + KC, w_next);
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < KC / 256; ++i) {
+            const int kk = i * 256 + lane * 4;
+#pragma unroll
+            for (int m = 0; m < MR; ++m) {
+                const float4 x = *reinterpret_cast<const float4*>(&xs[m][kk]);
+#pragma unroll
+                for (int j = 0; j < NB; ++j) {
+                    double a = acc[m][j];
+                    a = fma((double)x.x, (double)w[i][j].x, a);
+                    a = fma((double)x.y, (double)w[i][j].y, a);
+                    a = fma((double)x.z, (double)w[i][j].z, a);
+                    a = fma((double)x.w, (double)w[i][j].w, a);
+                    acc[m][j] = a;
+                }
+            }
+        }
+    };
+    float4 wa[KC / 256][NB], wb[KC / 256][NB];
+    ask(0, wa);
+    for (int k0 = 0; k0 < K; k0 += 2 * KC) {
+        stretch(k0, wa, wb);
+        if (k0 + KC < K) stretch(k0 + KC, wb, wa);
+    }
+#pragma unroll
+    for (int m = 0; m < MR; ++m)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            double a = acc[m][j];
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o, 64);
+            if (lane == 0 && m < M && n0 + j < N) C[(size_t)m * ldc + n0 + j] = (float)a;
+        }
+}
+
+extern "C" int ri_gemm_rows_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
+                                int M, int N, int K, hipStream_t stream) {
+    RI_REQUIRE(M >= 1 && M <= 4 && N > 0 && K > 0 && K % 4 == 0, "ri_gemm_rows_f32: needs 1..4 rows and K %% 4 == 0 (M=%d N=%d K=%d)", M, N, K);
+    RI_REQUIRE(lda >= K && ldw >= K && ldc >= N && lda % 4 == 0 && ldw % 4 == 0, "ri_gemm_rows_f32: leading dimensions must be >= K and multiples of 4");
+    RI_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0, "ri_gemm_rows_f32: null or unaligned pointer");
+    // A wave owns four columns, or two where four would leave compute units without a block's worth
+    // of loads in flight (a row's sums do not depend on that choice: a lane adds its share of K in
+    // the same order either way).
+    if ((N + 15) / 16 < 1024) gemm_rows_f32_kernel<4, 2><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    else gemm_rows_f32_kernel<4, 4><<<(N + 15) / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    RI_LAUNCHED("ri_gemm_rows_f32");
+    return 0;
+}
+
+// ---------------------------------------------------------------------------
 // gemm_skinny_bf16: C[M, N] = A[M, K] . W[N, K]^T for M <= 64 on the matrix cores.
 // The product is bound by the one pass over W, so the kernel is built around that stream:
 // a block owns 16 rows of W (one MFMA tile); its waves take the 32-wide k-steps in turn

@@ -10,7 +10,8 @@
 // two ahead of the one that is multiplied; nothing on that way depends on the lane, so the compiled loop waits for a
 // chunk's own loads only.  The
 // waves of a block share one tile of results and take 32 values of K in turn, whatever the tile; their 64-bit sums meet in
-// LDS once, in the order of the waves, so a row's result does not depend on the other rows or on the tile.
+// LDS once, in the order of the waves, so a row's result does not depend on the other rows or on the tile.  (Up to four rows of
+// products that gemm_f32_rows_pay names go to gemm_rows_f32, gemm.hip, which adds in another order: the same to the rounding of a 64-bit sum.)
 // Blocks of one column tile run on one XCD (consecutive block ids go around the eight of them), so a
 // tile's weights pass through one L2.  K % 4 == 0, rows 16-byte aligned.
 //
@@ -23,6 +24,8 @@
 
 extern "C" int ri_gemm_tiled(const void* A, int lda, const void* W, int ldw, void* C, int ldc,
                              int M, int N, int K, int in_dtype, int out_dtype, hipStream_t stream);      // gemm.hip
+extern "C" int ri_gemm_rows_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
+                                int M, int N, int K, hipStream_t stream);                               // gemm.hip
 
 typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
@@ -156,8 +159,7 @@ __global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
 // compute unit a block and no lane loads what another has.  D turns of each wave are under way at a time.  What bounds it is the
 // one pass over W.  Measured, us, 6 rows, tiles of 16 rows (half of them no row of the product) with loads that the compiled loop waited for / this
 // kernel: 2048 x 2048 10.3 / 6.7, 3072 x 2048 10.8 / 10.2, 16384 x 2048 41 / 31 (134 MB: 4.3 TB/s),
-// 2048 x 8192 33 / 17.6, 128256 x 2048 264 / 193 (5.4 TB/s).  Four rows, against FMAs with the lanes' sums added up in a tree: 3072 x 2048
-// 11.5 / 9.9, 16384 x 2048 36 / 30, 2048 x 8192 23.5 / 17.1, 28672 x 4096 100 / 87, 4096 x 14336 53 / 55, 128256 x 2048 182 / 188.
+// 2048 x 8192 33 / 17.6, 128256 x 2048 264 / 193 (5.4 TB/s).
 // SWIGLU: W is [2N, K] (gate rows, then up rows), a block's two tiles are the gate's and the up rows of the same eight columns, and
 // C = silu(gate) * up of the rounded sums, in place of the activation's kernel (six requests generating 12 tokens at the 1B sizes 32.81 -> 32.64 ms:
 // two streams of eight rows take most of what the launch of 4.3 us gives back).
@@ -305,22 +307,73 @@ static void launch_f32(const float* A, int lda, const float* W, int ldw, float* 
 }
 
 // The rows and columns of the tile that ri_gemm_f32 takes for M rows and N columns (of gemm_f32_kernel: up to eight rows, the tiles
-// of gemm_f32_few_kernel hold eight).
+// of gemm_f32_few_kernel hold eight, and gemm_rows_f32 has none; see ri_gemm_f32_form).
 extern "C" void ri_gemm_f32_tile(int M, int N, int* rows, int* columns) {
     const F32Tile& t = F32_TILES[f32_tile(M, N)];
     *rows = 16 * t.mt;
     *columns = 16 * t.nt;
 }
 
-// C[M, N] = silu(A . gate^T) * (A . up^T) of up to eight rows, W = [gate; up] of 2N rows: what ri_gemm_f32 and the activation's kernel
-// give, bit for bit.
+// The form of gemm_f32_few_kernel: 0: 8 columns a block and 4 turns under way, 1: 16 and 2, 2: 16 and 1, 3: 24 and 1.  Above 4,096 columns
+// the one whose rounds of 256 blocks take the least (*cost: in rounds of 8 columns a block); with fewer columns a block the rows of A
+// are read more often.  Measured, us, forms 0 / 2 / 3 at 1 and 8 rows: 6144 x 4096 20.7 26.4 / 26.7 29.7 / 21.9 22.9, 16384 x 2048
+// 27.7 35.4 / 27.9 30.7 / 30.6 33.4, 12288 x 4096 37 48 / 40 43 / 37 41, 28672 x 4096 81 108 / 84 93 / 85 92, 128256 x 1024 95 134 / 97
+// 113 / 92 107; 0 / 1: 2048 x 8192 16 19 / 24 28, 4096 x 4096 14.8 18.6 / 16.1 17.1, 4096 x 14336 49 64 / 49 56.  (Two forms by
+// columns alone, before: 6144 x 4096 29, 16384 x 2048 29 32, 4096 x 14336 49 64.)
+static int few_form(int M, int N, int K, float* cost) {
+    auto rounds = [&](int columns) { return (float)(((N + columns - 1) / columns + 255) / 256); };
+    const float one = rounds(8) * (0.96f + 0.0225f * (float)M + (K < 1024 ? 0.1f : 0.f));
+    const float two = rounds(16) * 2.f, three = rounds(24) * 2.8f;
+    *cost = fminf(one, fminf(two, three));
+    if (N <= 4096) return M > 4 && N > 2048 && K >= 1536 && !(K >= 8192 && (K & (K - 1)) == 0) ? 1 : 0;
+    return one == *cost ? 0 : two < three ? 2 : 3;
+}
+
+// Whether up to four rows go to the kernel of FMAs, gemm_rows_f32: it reads a kilobyte of a row of W at a time, the tiles 64 bytes
+// of each of 16 places, which costs more the longer the rows are.  But where rows begin a power of two apart its long reads meet on the same
+// channels of memory, and there it pays only against rounds of blocks that are far from full.  Measured, us, 1 and 4 rows, gemm_rows_f32 / the best form of
+// the tiles: 5120 x 3072 16.6 18.6 / 17.4 19.3, 5120 x 5120 23.7 27.1 / 28.5 30.5, 27648 x 5120 97 107 / 120 130, 12288 x 6912 60 68 / 68 71,
+// 128256 x 1536 129 141 / 146 155, 2560 x 11008 35 40 / 37 40, 7000 x 4096 25.1 26.6 / 25.9 27.4; not taken: 12288 x 1536 18.4 21.8 / 17.7
+// 18.9, 28672 x 4096 95 98 / 81 87, 16384 x 2048 34 37 / 28 29, 4096 x 3072 14.9 16.3 / 12.8 14.4, 2048 x 8192 21 24 / 16 17.
+static bool gemm_f32_rows_pay(int M, int N, int K, int ldw) {
+    if (M > 4) return false;
+    if ((ldw & (ldw - 1)) == 0) {
+        float cost = 0.f;
+        few_form(M, N, K, &cost);
+        return N > 4096 && ((K == 2048 && N > 65536) || (K >= 4096 && cost > 1.1f * (float)N / 2048.f));
+    }
+    if (N > 4096) return K > 2048 || (K > 1024 && N > 32768) || (K >= 768 && K % 128 != 0);
+    return N > 2048 && K >= (N > 3072 ? 7168 : 5120);
+}
+
+// The kernel that ri_gemm_f32 takes: -1 gemm_rows_f32, 0 to 3 the form of gemm_f32_few_kernel, 4 the tiles of 16 rows and more.
+extern "C" int ri_gemm_f32_form(int M, int N, int K, int ldw) {
+    if (gemm_f32_rows_pay(M, N, K, ldw)) return -1;
+    // (of 5 to 8 rows with a K that ends inside a turn, wide products stay with the tiles of 16 rows: 12288 x 900 16.9 -> 15.5)
+    if (M > 8 || (M > 4 && N > 4096 && K >= 768 && K % 128 != 0)) return 4;
+    float cost = 0.f;
+    return few_form(M, N, K, &cost);
+}
+
+// Whether up to eight rows' gate and up product takes ri_gemm_f32_swiglu rather than ri_gemm_f32 and the activation's kernel: not where gemm_rows_f32
+// has that product to itself, but for rows of up to 3,072 values whose rounds of blocks are full.  Measured, us, 1 and 4 rows, two kernels / this:
+// 8192 x 3072 46.7 50.3 / 43.8 45.9, 9728 x 2560 40.4 44.2 / 42.4 45.4, 6912 x 2560 29.6 34.6 / 36.1 38.4, 13824 x 5120 98 109 / 128 137, 18944 x 3584
+// 92 98 / 107 115, 14336 x 4096 83 90 / 82 85, 8192 x 2048 29.7 30.9 / 29.0 29.8.
+extern "C" int ri_gemm_f32_swiglu_pays(int M, int I, int K, int ldw) {
+    if (M > 8) return 0;
+    const bool full = (float)((I + 2047) / 2048) * 2048.f <= 1.03f * (float)I;
+    return !(K > 2048 && gemm_f32_rows_pay(M, 2 * I, K, ldw) && (K > 3072 || !full));
+}
+
+// C[M, N] = silu(A . gate^T) * (A . up^T) of up to eight rows, W = [gate; up] of 2N rows: what the tiles of ri_gemm_f32 and the activation's
+// kernel give, bit for bit.
 extern "C" int ri_gemm_f32_swiglu(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
                                   int M, int N, int K, hipStream_t stream) {
     RI_REQUIRE(M >= 1 && M <= 8 && N > 0 && K > 0 && K % 4 == 0, "ri_gemm_f32_swiglu: needs 1 to 8 rows and K %% 4 == 0 (M=%d N=%d K=%d)", M, N, K);
     RI_REQUIRE(lda >= K && ldw >= K && ldc >= N && lda % 4 == 0 && ldw % 4 == 0 && lda <= (1 << 24) && ldw <= (1 << 24),
                "ri_gemm_f32_swiglu: leading dimensions must be >= K, multiples of 4 and at most 2^24");
     RI_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && N <= (1 << 26), "ri_gemm_f32_swiglu: null or unaligned pointer, or N=%d", N);
-    gemm_f32_few_kernel<2, 4, true><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    gemm_f32_few_kernel<2, 1, true><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
     RI_LAUNCHED("ri_gemm_f32_swiglu");
     return 0;
 }
@@ -333,14 +386,16 @@ extern "C" int ri_gemm_f32(const float* A, int lda, const float* W, int ldw, flo
     RI_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0, "ri_gemm_f32: null or unaligned pointer");
     RI_REQUIRE(N <= (1 << 26), "ri_gemm_f32: N=%d exceeds the grid limit", N);
     // lanes find their rows by 32-bit distances in bytes from the first of up to 48
+    if (M <= 4 && (lda > (1 << 24) || ldw > (1 << 24))) return ri_gemm_rows_f32(A, lda, W, ldw, C, ldc, M, N, K, stream);
     if (lda > (1 << 24) || ldw > (1 << 24)) return ri_gemm_tiled(A, lda, W, ldw, C, ldc, M, N, K, RI_F32, RI_F32, stream);
-    if (M <= 8) {
-        // Columns a block, turns under way a wave.  Measured, us, 6 rows, 8 columns and 4 turns / 16 and 4 / 24 and 1:
-        // 2048 x 2048 6.7 / 10.1 / -, 3072 x 2048 10.2 / 10.4 / 12.2, 2048 x 8192 17.6 / 27 / -, 16384 x 2048 33 / 31 / 32, 128256 x 2048
-        // 241 / 205 / 193; 4 rows: 4096 x 14336 55 / 52 / 70, 28672 x 4096 91 / 101 / 87; 1 row: 4096 x 4096 14.5 / 18.9 / 19.9.
-        if (N <= 4096) gemm_f32_few_kernel<1, 4><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
-        else if (N < 24576) gemm_f32_few_kernel<2, 4><<<(N + 15) / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
-        else gemm_f32_few_kernel<3, 1><<<(N + 23) / 24, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+    if (const int form = ri_gemm_f32_form(M, N, K, ldw); form < 4) {
+        switch (form) {
+            case -1: return ri_gemm_rows_f32(A, lda, W, ldw, C, ldc, M, N, K, stream);
+            case 0: gemm_f32_few_kernel<1, 4><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K); break;
+            case 1: gemm_f32_few_kernel<2, 2><<<(N + 15) / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K); break;
+            case 2: gemm_f32_few_kernel<2, 1><<<(N + 15) / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K); break;
+            default: gemm_f32_few_kernel<3, 1><<<(N + 23) / 24, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K); break;
+        }
         RI_LAUNCHED("ri_gemm_f32");
         return 0;
     }

@@ -803,7 +803,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: Optiona
                     return
     if x.dtype == torch.float32 and out.dtype == torch.float32 and K % 4 == 0 and x.stride(0) % 4 == 0 \
             and w.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
-        # the exact path: 64-bit sums on the 64-bit matrix instruction
+        # the exact path: 64-bit sums, on the 64-bit matrix instruction or, for up to four rows of long ones, in FMAs
         _check(lib.ri_gemm_f32(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), M, N, K, _stream()))
         return
     _check(lib.ri_gemm_tiled(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0),
@@ -925,8 +925,9 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor,
         raise KernelError("linear_swiglu: row factors of a deferred norm go with the few-row bfloat16 kernel only")
     if scratch is None or tuple(scratch.shape) != (M, 2 * I):
         raise KernelError("linear_swiglu: needs scratch [M, 2I] for this size")
-    if x.dtype == torch.float32 and M <= 8 and K % 4 == 0 and all(t.stride(0) % 4 == 0 and t.stride(0) <= 1 << 24 and t.data_ptr() % 16 == 0 for t in (x, w_gate_up)):
-        # the exact path's few rows: the activation in the product's epilogue, the same bits
+    if x.dtype == torch.float32 and M <= 8 and K % 4 == 0 and all(t.stride(0) % 4 == 0 and t.stride(0) <= 1 << 24 and t.data_ptr() % 16 == 0 for t in (x, w_gate_up)) \
+            and (_lib().ri_gemm_f32_swiglu_pays(M, I, K, w_gate_up.stride(0)) or not (out.is_contiguous() and scratch.is_contiguous())):
+        # the exact path's few rows: the activation in the product's epilogue, on the rounded sums (the activation's kernel takes whole buffers only)
         _check(_lib().ri_gemm_f32_swiglu(_ptr(x), x.stride(0), _ptr(w_gate_up), w_gate_up.stride(0), _ptr(out), out.stride(0), M, I, K, _stream()))
         return
     linear(x, w_gate_up, scratch)

@@ -457,6 +457,42 @@ def test_linear_f32_of_up_to_eight_rows(ops, M, N, K):
         assert torch.equal(bad[:M - 1], out[:M - 1, :N]) and torch.all(torch.isnan(bad[M - 1]))
 
 
+@pytest.mark.parametrize("M,N,K,form", [(1, 4097, 2052, -1), (4, 5001, 2304, -1), (3, 2049, 5124, -1), (2, 3077, 7172, -1), (4, 32771, 1028, -1), (3, 4111, 772, -1),
+                                        (2, 5120, 4096, -1), (8, 3000, 1540, 1), (5, 4096, 4096, 1), (6, 8190, 1024, 2), (2, 16384, 2048, 2), (8, 6144, 896, 3),
+                                        (7, 12287, 1536, 3), (1, 8192, 1664, 0), (8, 4100, 900, 4), (8, 2056, 8192, 0)])
+def test_linear_f32_of_up_to_eight_rows_on_every_form(ops, M, N, K, form):
+    """The kernel of FMAs (long rows, but for rows a power of two apart whose tiles fill their rounds) and the forms of the tiles: 64-bit sums
+    rounded once, and a row that is not finite alone with its results."""
+    assert ops._lib().ri_gemm_f32_form(M, N, K, K) == form
+    x, w = rnd(M, K + 4, seed=M)[:, :K], rnd(N, K, seed=N)
+    out = torch.full((M, N + 3), float("nan"), device=DEV)
+    ops.linear(x, w, out[:, :N])
+    ref = x.double() @ w.double().t()
+    # a 64-bit sum rounded once: half a unit of the last place of each result
+    assert torch.all((out[:, :N].double() - ref).abs() <= ref.abs() * 2.0 ** -24 + 1e-12 * ref.abs().max())
+    assert torch.all(torch.isnan(out[:, N:]))
+    if M > 1:
+        y = x.clone()
+        y[M - 1, K // 2] = float("inf")
+        y[M - 1, K - 1] = float("nan")
+        bad = torch.empty(M, N, device=DEV)
+        ops.linear(y, w, bad)
+        assert torch.equal(bad[:M - 1], out[:M - 1, :N]) and torch.all(torch.isnan(bad[M - 1]))
+
+
+@pytest.mark.parametrize("M,I,K,fused", [(1, 6912, 2560, 0), (4, 2560, 3588, 0), (2, 8192, 2560, 1), (4, 4096, 4096, 1), (8, 6912, 2560, 1)])
+def test_swiglu_f32_of_up_to_eight_rows_by_the_length_of_rows(ops, M, I, K, fused):
+    assert ops._lib().ri_gemm_f32_swiglu_pays(M, I, K, K) == fused
+    x, w = rnd(M, K, seed=M), rnd(2 * I, K, seed=I) * (8.0 / K) ** 0.5
+    ref = x.double() @ w.double().t()
+    ref = torch.nn.functional.silu(ref[:, :I]) * ref[:, I:]
+    for out in (torch.empty(M, I, device=DEV), torch.full((M, I + 5), float("nan"), device=DEV)[:, :I]):       # whole, and columns of a wider buffer
+        ops.linear_swiglu(x, w, out, torch.empty(M, 2 * I, device=DEV))
+        # a rounding of the gate's sum x moves silu by up to 1 + |x| times as much, |x| < 16; the up sum, exp to 2 units of the last
+        # place and three 32-bit operations: 32 half units in all
+        assert torch.all((out.double() - ref).abs() <= 2.0 ** -19 * ref.abs() + 1e-7)
+
+
 @pytest.mark.parametrize("M,I,K", [(1, 1, 4), (8, 7, 132), (3, 8, 288), (6, 4099, 1028), (5, 24, 2304), (2, 9001, 160)])
 def test_swiglu_f32_of_up_to_eight_rows_is_the_product_and_the_activation(ops, M, I, K):
     x, w = rnd(M, K + 4, seed=M)[:, :K], rnd(2 * I, K, seed=I) * 0.3
