@@ -293,13 +293,30 @@ __global__ __launch_bounds__(BW * 64) void attn_decode_split_kernel(
 
 constexpr int LIST_SPAN = 32, LIST_ROWS = 64, LIST_WAVES = 512;
 
+// How the list below is divided: spans of keys [first, end), the waves of a list of `total` spans (a stretch is two spans or more, or
+// all), the first span of wave w, the wave of span f, and the slots a row of at most max_kv_len keys needs: the waves between its
+// first and its last have two of its spans or more.
+__host__ __device__ inline int list_spans(int first, int end) { return end > first ? (end + LIST_SPAN - 1) / LIST_SPAN - first / LIST_SPAN : 0; }
+__host__ __device__ inline uint32_t list_waves(uint32_t total, uint32_t most) { const uint32_t two = total / 2 > 1 ? total / 2 : 1; return most < two ? most : two; }
+__host__ __device__ inline uint32_t list_from(uint32_t w, uint32_t total, uint32_t waves) { return w * total / waves; }       // (waves total < 2^32: the host's rule)
+__host__ __device__ inline uint32_t list_wave_of(uint32_t f, uint32_t total, uint32_t waves) { return ((f + 1) * waves - 1) / total; }
+__host__ __device__ inline int list_slots(int max_kv_len) { return (max_kv_len + LIST_SPAN - 1) / LIST_SPAN / 2 + 1; }
+
+// The same for a test that divides a list without a GPU.
+extern "C" int ri_attention_list_spans(int first, int end) { return list_spans(first, end); }
+extern "C" unsigned ri_attention_list_waves(unsigned total, unsigned most) { return list_waves(total, most); }
+extern "C" unsigned ri_attention_list_from(unsigned w, unsigned total, unsigned waves) { return list_from(w, total, waves); }
+extern "C" unsigned ri_attention_list_wave_of(unsigned f, unsigned total, unsigned waves) { return list_wave_of(f, total, waves); }
+extern "C" int ri_attention_list_slots(int max_kv_len) { return list_slots(max_kv_len); }
+
 // The rows' keys as one list.  Rows differ in length, and 2,049 keys are one span more than 32 waves of 64 keys take at once, so
 // a number of blocks a row leaves units idle or a few waves with twice the others' work.  Here the spans of 32
 // keys of all rows (up to 64, a lane each) are numbered one after the other, and wave w of a key/value head takes the stretch
 // [w total / W, (w + 1) total / W) of them, with a running maximum and sum; where a row ends it leaves that row's partial result
 // in slot w - (the first wave that has a span of the row).  count[b]: the row's slots.  A span's keys and values are asked for
 // while the one before it is worked on, its pages' ids a span earlier, under no lane's condition (what lies beyond the row is
-// put to zero, or its score to -inf, where it is used).  Two waves a unit in all: more leave more partial results for the same bytes.
+// put to zero, or its score to -inf, where it is used).  Keys from max_kv_len on are not looked at, whatever kv_lens says: slots,
+// page ids and the list's numbers are bounded by it.  Two waves a unit in all: more leave more partial results for the same bytes.
 // The sums are O^T[d, q] = V^T . P^T, so that a query's factors lie in the lanes that hold its sums; the weights go
 // to the matrix instruction as the sum of two bfloat16, which costs a bound-by-memory kernel nothing (error of the
 // output against 64 bits 2.1e-3 -> 1.7e-3, that of its own rounding).
@@ -310,7 +327,7 @@ constexpr int LIST_SPAN = 32, LIST_ROWS = 64, LIST_WAVES = 512;
 __global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
         const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
         const int* __restrict__ table, int max_blocks, const int* __restrict__ row_of_token, const int* __restrict__ positions,
-        const int* __restrict__ kv_lens, int H, int Hkv, int page, int page_shift, float scale, int window, int splits,
+        const int* __restrict__ kv_lens, int H, int Hkv, int page, int page_shift, float scale, int window, int max_kv_len, int splits,
         float* __restrict__ part_o, float* __restrict__ part_ml, int* __restrict__ count, int tokens, int rows) {
     constexpr int HD = 128, KT = 2, SPAN = LIST_SPAN;       // 16 KiB of keys and values
     const int lane = threadIdx.x, col = lane & 15, grp = lane >> 4, g = blockIdx.y, G = H / Hkv;
@@ -323,11 +340,11 @@ __global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
         row = row_of_token[lane];
         if (row >= 0 && row != guess) len = kv_lens[row];
         if (row >= 0) {                                     // else a padding token
-            end = min(len, p + 1);
+            end = min(min(len, p + 1), max_kv_len);
             first = window > 0 ? max(0, p + 1 - window) : 0;
         }
     }
-    ends = end > first ? (end + SPAN - 1) / SPAN - first / SPAN : 0;
+    ends = list_spans(first, end);
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
         const int up = __shfl_up(ends, o, 64);
@@ -335,9 +352,9 @@ __global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
     }
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(ends, 63);
     if (total == 0) return;
-    const uint32_t W = min((uint32_t)gridDim.x, max(total / 2, 1u)), w = blockIdx.x;       // a stretch is two spans or more, or all
+    const uint32_t W = list_waves(total, gridDim.x), w = blockIdx.x;
     if (w >= W) return;
-    const int f0 = (int)(w * total / W), f1 = (int)((w + 1) * total / W);       // (W total < 2^32: the host's rule)
+    const int f0 = (int)list_from(w, total, W), f1 = (int)list_from(w + 1, total, W);
     struct Row { int tok, row, first, end, f0, n; };        // spans [f0, f0 + n) of the list
     auto row_of = [&](int f) {                              // the row of span f < total
         const int who = __popcll(__ballot(ends <= f));      // rows that end at or before it
@@ -346,7 +363,7 @@ __global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
         x.row = __builtin_amdgcn_readlane(row, who);
         x.first = __builtin_amdgcn_readlane(first, who);
         x.end = __builtin_amdgcn_readlane(end, who);
-        x.n = (x.end + SPAN - 1) / SPAN - x.first / SPAN;
+        x.n = list_spans(x.first, x.end);
         x.f0 = __builtin_amdgcn_readlane(ends, who) - x.n;
         return x;
     };
@@ -459,7 +476,7 @@ __global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
             }
     };
     auto leave = [&](int b, int f, int n) {                 // row b: spans [f, f + n) of the list
-        const uint32_t w0 = (((uint32_t)f + 1) * W - 1) / total;
+        const uint32_t w0 = list_wave_of(f, total, W);
         float l = l_run;
         l += __shfl_xor(l, 16, 64);
         l += __shfl_xor(l, 32, 64);
@@ -470,7 +487,7 @@ __global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
                 *reinterpret_cast<float4*>(part_o + slot * HD + db * 16 + grp * 4) = make_float4(o[db][0], o[db][1], o[db][2], o[db][3]);
             if (grp == 0) *reinterpret_cast<float2*>(part_ml + slot * 2) = make_float2(m_run, l);
         }
-        if (w == w0 && g == 0 && lane == 0) count[b] = (int)((((uint32_t)(f + n)) * W - 1) / total - w0 + 1);
+        if (w == w0 && g == 0 && lane == 0) count[b] = (int)(list_wave_of(f + n - 1, total, W) - w0 + 1);
     };
     clear();
     Span sa, sb;
@@ -560,6 +577,7 @@ __global__ __launch_bounds__(CW * 64) void attn_decode_combine_kernel(
     int visible = 0, j0 = 0;
     if (b >= 0) {
         visible = min(kv_len, p + 1);
+        if (count) visible = min(visible, chunk);        // (of the list's form: the longest length, which its spans end at)
         j0 = window > 0 ? max(0, p + 1 - window) : 0;
     }
     if (visible <= j0) {                      // a padding token, or nothing to see: zeros
@@ -627,9 +645,6 @@ static int decode_chunk(int T, int Hkv, int hd, int max_kv_len) {
     const long long waves128 = (long long)T * Hkv * ((max_kv_len + 127) / 128);
     return waves128 >= 4096 ? 128 : 64;
 }
-
-// slots a row of the list's form: its waves' stretches are two spans or more
-static int list_slots(int max_kv_len) { return (max_kv_len + LIST_SPAN - 1) / LIST_SPAN / 2 + 1; }
 
 extern "C" size_t ri_attention_decode_workspace(int rows, int H, int hd, int max_kv_len) {
     const size_t splits = (size_t)list_slots(max_kv_len);       // no other form leaves more
@@ -705,12 +720,12 @@ extern "C" int ri_attention_decode(
         int* count = (int*)(ml + (size_t)rows * H * slots * 2);
         attn_decode_list_kernel<<<dim3(W, Hkv), 64, 0, stream>>>(
             (const bf16_t*)q, q_stride, (const bf16_t*)kc, (const bf16_t*)vc, table, max_blocks, row_of_token, positions, kv_lens, H, Hkv,
-            page, __builtin_ctz((unsigned)page), scale, window, slots, sums, ml, count, T, rows);
+            page, __builtin_ctz((unsigned)page), scale, window, max_kv_len, slots, sums, ml, count, T, rows);
         RI_LAUNCHED("ri_attention_decode(list)");
         // a row has as many slots as waves, at most
         const bool one = std::min(slots, W) <= 64;
         auto combine = one ? attn_decode_combine_kernel<128, 1> : attn_decode_combine_kernel<128, 4>;
-        combine<<<dim3(T, H), one ? 64 : 256, 0, stream>>>(sums, ml, slots, 0, row_of_token, positions, kv_lens, nullptr, H, window, (bf16_t*)out,
+        combine<<<dim3(T, H), one ? 64 : 256, 0, stream>>>(sums, ml, slots, max_kv_len, row_of_token, positions, kv_lens, nullptr, H, window, (bf16_t*)out,
                                                            out_stride, rows, nullptr, count);
         RI_LAUNCHED("ri_attention_decode(combine)");
         return 0;

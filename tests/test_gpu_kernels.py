@@ -837,6 +837,24 @@ def test_single_token_attention_as_a_list_with_padding_and_rows_out_of_order(ops
             assert torch.allclose(got[t].float(), want[b].float(), rtol=2.0 ** -7, atol=1e-3), t
 
 
+@pytest.mark.parametrize("window", [0, 500])
+def test_single_token_attention_as_a_list_ends_at_the_steps_longest_length(ops, window):
+    """A row that kv_lens says is longer than the step was planned for: its keys beyond that are not looked at, and the others' results
+    are theirs."""
+    B, H, Hkv, hd, page, longest = 12, 8, 8, 128, 16, 320
+    lens = [300, 7, 900, 64, 320, 321, 5, 17, 310, 32, 33, 1]
+    qkv, kc, vc, table, ctx, _, _ = _paged_setup(torch.bfloat16, B, H, Hkv, hd, page, [1] * B, [n - 1 for n in lens], seed=4, num_pages=200)
+    ops.rope_kv_write(qkv, H, Hkv, hd, None, ctx.positions, ctx.row_of_token, kc, vc, table, page)
+    ctx.max_kv_len = longest
+    got, want = (torch.full((B, H * hd), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.paged_attention(qkv, got, H, Hkv, hd, kc, vc, table, page, ctx, 0.1, window)
+    ctx.kv_lens = ctx.kv_lens.clamp(max=longest)
+    ops.paged_attention(qkv, want, H, Hkv, hd, kc, vc, table, page, ctx, 0.1, window)
+    assert torch.equal(got, want) and torch.isfinite(got).all()
+    if window:                                         # the row of 900: its window of keys 400 .. 899 begins behind the last key
+        assert torch.all(got[2] == 0)
+
+
 def _check_rope_write_and_attention(ops, dtype, case, window, kv_heads=None):
     B, H, Hkv, hd, page, q_lens, starts = case
     need = sum((s + q + page - 1) // page for s, q in zip(starts, q_lens))

@@ -1,0 +1,60 @@
+"""What the kernels' entry points decide and check on the host, without a GPU: how the list of single-token attention is
+divided, and operands that are refused before anything is launched."""
+import random
+
+import pytest
+
+
+@pytest.fixture(scope="module")
+def lib():
+    from rustinfer_amd.kernels import build
+    return build.load()
+
+
+def _divide(lib, rows, max_kv_len, heads):
+    """The list of ``rows`` = [(first, end)] as the kernel walks it: {row: {slot: [spans]}} and {row: slots counted}.  ``end`` is cut
+    at max_kv_len, as the kernel cuts it."""
+    rows = [(a, min(b, max_kv_len)) for a, b in rows]
+    n = [lib.ri_attention_list_spans(a, b) for a, b in rows]
+    total = sum(n)
+    if not total:
+        return {}, {}
+    planned = len(rows) * ((max_kv_len + 31) // 32 + 1)                       # the entry point's bound of the list
+    assert planned >= total and planned * 512 < 1 << 32
+    waves = lib.ri_attention_list_waves(total, max(1, min(512 // heads, planned // 2)))
+    begins = [sum(n[:i]) for i in range(len(n))]
+    slots, counts = {}, {}
+    assert lib.ri_attention_list_from(0, total, waves) == 0 and lib.ri_attention_list_from(waves, total, waves) == total
+    for w in range(waves):
+        f0, f1 = lib.ri_attention_list_from(w, total, waves), lib.ri_attention_list_from(w + 1, total, waves)
+        assert f1 > f0
+        for i, (b, m) in enumerate(zip(begins, n)):
+            mine = range(max(f0, b), min(f1, b + m))
+            if len(mine):
+                w0 = lib.ri_attention_list_wave_of(b, total, waves)
+                slots.setdefault(i, {}).setdefault(w - w0, []).extend(rows[i][0] // 32 + f - b for f in mine)
+                if w == w0:
+                    counts[i] = lib.ri_attention_list_wave_of(b + m - 1, total, waves) - w0 + 1
+    return slots, counts
+
+
+@pytest.mark.parametrize("seed", range(40))
+def test_list_of_spans_holds_every_span_once_in_slots_that_are_there(lib, seed):
+    rng = random.Random(seed)
+    for _ in range(10):
+        T, heads, window = rng.randint(1, 64), rng.choice([1, 2, 3, 8, 32, 512]), rng.choice([0, 0, 1, 33, 700])
+        longest = rng.choice([1, 31, 32, 33, 64, 700, 3000])
+        ends = [rng.choice([0, 1, longest, rng.randint(0, longest)]) for _ in range(T)]
+        # kv_lens may say more than the step was planned for
+        max_kv_len = rng.choice([longest, -(-longest // 1024) * 1024, max(1, longest // 2)])
+        rows = [(max(0, e - window) if window else 0, e) for e in ends]
+        slots, counts = _divide(lib, rows, max_kv_len, heads)
+        assert counts.keys() == slots.keys()
+        for i, (a, b) in enumerate(rows):
+            b = min(b, max_kv_len)
+            if b <= a:
+                assert i not in slots
+                continue
+            got = slots[i]
+            assert sorted(s for spans in got.values() for s in spans) == list(range(a // 32, (b + 31) // 32))
+            assert sorted(got) == list(range(counts[i])) and counts[i] <= lib.ri_attention_list_slots(max_kv_len)
