@@ -420,18 +420,18 @@ __global__ __launch_bounds__(64) void attn_exact_combine_kernel(
 // 4,000 42 / 120 / 34; 32 tokens of 500 28 / 20 / 20, of 2,000 79 / 65 / 55; 64 tokens of 100 20 / 10 / 12, of 2,000 169 / 101 / 120.
 constexpr int EX_SINGLE_PAIRS = 512, EX_SINGLE_KEYS = 128;
 
-// Two tiles of rows a block where a token's heads fill more than one, or the pages are of no power of two of four keys and more.
-// (For long prompts too: 2,048 tokens of 32 heads of 64 453 -> 485 us.)
-int exact_page_shift(int page) { return page >= 4 && (page & (page - 1)) == 0 ? __builtin_ctz((unsigned)page) : -1; }
-bool exact_two_tiles(int G, int page) { return G > 16 || exact_page_shift(page) < 0; }
+// Two tiles of rows a block where a token's heads fill more than one, or values are read one at a time: pages of no power of two of four keys and
+// more, or a value cache that does not begin at a multiple of 16 bytes (shift -1).
+int exact_page_shift(int page, const float* vc) { return page >= 4 && (page & (page - 1)) == 0 && (uintptr_t)vc % 16 == 0 ? __builtin_ctz((unsigned)page) : -1; }
+bool exact_two_tiles(int G, int shift) { return G > 16 || shift < 0; }
 
 template <int MODE>
 void launch_exact(dim3 grid, int hd, int TQ, const float* q, int q_stride, float* out, int out_stride, const float* kc, const float* vc,
                   const int* table, int max_blocks, const int* cu_q, const int* q_start, const int* row_of_token, const int* positions,
                   const int* kv_lens, int num_rows, int H, int Hkv, int page, float scale, int window, int slots, float* part_ml, float* part_o,
                   hipStream_t stream) {
-    const int shift = exact_page_shift(page);
-    const bool two = exact_two_tiles(H / Hkv, page);
+    const int shift = exact_page_shift(page, vc);
+    const bool two = exact_two_tiles(H / Hkv, shift);
 #define RI_EXACT(NJ_, RT_, ANY_) attn_exact_f32_kernel<NJ_, RT_, MODE, ANY_><<<grid, 256, 0, stream>>>(q, q_stride, out, out_stride, kc, vc, table, max_blocks, \
         cu_q, q_start, row_of_token, positions, kv_lens, num_rows, H, Hkv, hd, page, shift, scale, window, TQ, slots, part_ml, part_o)
     if (hd <= 64) { if (shift < 0) RI_EXACT(4, 2, true); else if (two) RI_EXACT(4, 2, false); else RI_EXACT(4, 1, false); }
@@ -462,7 +462,7 @@ extern "C" int ri_attention_exact_f32(
     RI_REQUIRE((uintptr_t)kc % 16 == 0, "ri_attention_exact_f32: unaligned key cache");
     RI_REQUIRE(Hkv <= 65535, "ri_attention_exact_f32: too many key/value heads for the grid");
     const int G = H / Hkv;
-    const int TQ = (exact_two_tiles(G, page) ? 32 : 16) / G;
+    const int TQ = (exact_two_tiles(G, exact_page_shift(page, vc)) ? 32 : 16) / G;
     const int tiles = (T + TQ - 1) / TQ + num_rows;    // at most: every request may end in a short tile
     launch_exact<EX_PORTIONS>(dim3(tiles, Hkv), hd, TQ, q, q_stride, out, out_stride, kc, vc, table, max_blocks, cu_q, q_start, nullptr, nullptr, kv_lens,
                               num_rows, H, Hkv, page, scale, window, 0, nullptr, nullptr, stream);
@@ -490,7 +490,8 @@ extern "C" int ri_attention_exact_decode_f32(
     RI_REQUIRE(q_stride >= H * hd && out_stride >= H * hd && q_stride % 4 == 0, "ri_attention_exact_decode_f32: bad row strides");
     if (T == 0) return 0;
     RI_REQUIRE(q && out && kc && vc && table && row_of_token && positions && kv_lens && workspace, "ri_attention_exact_decode_f32: null pointer");
-    RI_REQUIRE((uintptr_t)kc % 16 == 0 && (uintptr_t)vc % 16 == 0 && (uintptr_t)q % 16 == 0, "ri_attention_exact_decode_f32: unaligned operands");
+    RI_REQUIRE((uintptr_t)kc % 16 == 0 && (uintptr_t)vc % 16 == 0 && (uintptr_t)q % 16 == 0 && (uintptr_t)workspace % 16 == 0,
+               "ri_attention_exact_decode_f32: unaligned operands");
     RI_REQUIRE(Hkv <= 65535 && T <= 65535 && H <= 65535, "ri_attention_exact_decode_f32: too many heads or tokens for the grid");
     RI_REQUIRE(workspace_floats >= ri_attention_exact_decode_workspace(T, H, hd, max_kv_len),
                "ri_attention_exact_decode_f32: workspace of %zu floats, %zu needed", workspace_floats,

@@ -1248,6 +1248,19 @@ def test_exact_attention_of_a_portion_does_not_depend_on_the_cut(ops, H, Hkv, hd
         kc[blk, :, far % page] = saved
 
 
+@pytest.mark.parametrize("H,Hkv,hd,page,window", [(8, 2, 64, 16, 0), (4, 4, 128, 4, 40)])
+def test_exact_attention_of_portions_takes_values_from_any_address(ops, H, Hkv, hd, page, window):
+    qkv, kc, vc, table, ctx, _, _ = _paged_setup(torch.float32, 2, H, Hkv, hd, page, [40, 70], [90, 0], seed=hd)
+    ops.rope_kv_write(qkv, H, Hkv, hd, None, ctx.positions, ctx.row_of_token, kc, vc, table, page)
+    want, got = (torch.full((110, H * hd), float("nan"), device=DEV) for _ in range(2))
+    ops.paged_attention(qkv, want, H, Hkv, hd, kc, vc, table, page, ctx, 0.1, window)
+    off = torch.empty(vc.numel() + 1, device=DEV)[1:].view(vc.shape)
+    off.copy_(vc)
+    assert off.data_ptr() % 16 == 4
+    ops.paged_attention(qkv, got, H, Hkv, hd, kc, off, table, page, ctx, 0.1, window)
+    assert torch.equal(got, want) and torch.isfinite(got).all()
+
+
 @pytest.mark.parametrize("H,Hkv,hd,page,window", [(8, 2, 64, 16, 0), (40, 2, 80, 16, 0), (40, 2, 64, 4, 90), (3, 3, 4, 1, 0), (6, 2, 100, 5, 33), (32, 1, 128, 64, 0),
                                                   (12, 4, 128, 2, 0), (7, 1, 20, 128, 130), (34, 2, 128, 6, 0)])
 def test_exact_attention_of_single_tokens_on_every_route(ops, H, Hkv, hd, page, window):

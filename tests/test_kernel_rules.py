@@ -1,5 +1,6 @@
 """What the kernels' entry points decide and check on the host, without a GPU: how the list of single-token attention is
 divided, and operands that are refused before anything is launched."""
+import ctypes
 import random
 
 import pytest
@@ -58,3 +59,21 @@ def test_list_of_spans_holds_every_span_once_in_slots_that_are_there(lib, seed):
             got = slots[i]
             assert sorted(s for spans in got.values() for s in spans) == list(range(a // 32, (b + 31) // 32))
             assert sorted(got) == list(range(counts[i])) and counts[i] <= lib.ri_attention_list_slots(max_kv_len)
+
+
+@pytest.mark.parametrize("shifted", ["k", "v", "q", "workspace"])
+def test_exact_attention_refuses_operands_that_its_loads_cannot_take(lib, shifted):
+    """Single tokens: values and partial results go 16 bytes at a time; portions take values from any address.  (Addresses that are never used: the check
+    comes before the launch.)"""
+    at = {name: ctypes.c_void_p((1 << 20) + 4 * (name == shifted)) for name in ("q", "out", "k", "v", "table", "i32", "workspace")}
+    i = at["i32"]
+    f, zero = ctypes.c_float(0.125), ctypes.c_void_p(0)
+    H, Hkv, hd, page, T, longest = 4, 2, 64, 16, 3, 300
+    lib.ri_attention_exact_decode_workspace.restype = ctypes.c_size_t
+    need = lib.ri_attention_exact_decode_workspace(T, H, hd, longest)
+    rc = lib.ri_attention_exact_decode_f32(at["q"], H * hd, at["out"], H * hd, at["k"], at["v"], 64, page, H, Hkv, hd, at["table"], 32, i, i, i, T, longest, f, 0,
+                                           at["workspace"], ctypes.c_size_t(need), zero)
+    assert rc != 0 and b"unaligned" in lib.ri_last_error()
+    if shifted == "k":
+        rc = lib.ri_attention_exact_f32(at["q"], H * hd, at["out"], H * hd, at["k"], at["v"], 64, page, H, Hkv, hd, at["table"], 32, i, i, i, 1, T, f, 0, zero)
+        assert rc != 0 and b"unaligned" in lib.ri_last_error()
