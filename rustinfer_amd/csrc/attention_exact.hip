@@ -21,6 +21,7 @@
 // Products and sums that must round the same way everywhere are written with fmaf, __fmul_rn and
 // __fsub_rn, and contraction is switched off for the file.
 #include "common.h"
+#include <algorithm>
 #include <math.h>
 
 #pragma clang fp contract(off)
@@ -73,7 +74,8 @@ __device__ __forceinline__ float elem(const float4& v, int i) { return i == 0 ? 
 // operands from LDS (and a key a lane for single tokens) before / now, 32 heads, 8 of keys: 600 tokens at head 64 151 / 45, 100 tokens 31 / 7.5,
 // 2,048 tokens 1024 / 327 (52 TFLOP/s), 64 tokens behind 2,000 544 / 66, 7 single tokens behind 1,500 beside 64 more 416 / 52; head 128:
 // 600 tokens 471 / 84; 2,048 tokens of 24 heads 2748 / 504.
-enum { EX_PORTIONS = 0, EX_SINGLE = 1, EX_BLOCKS = 2 };
+constexpr uint32_t EX_FEW_BLOCKS = 2048;               // up to so many, the chip holds half of them at once
+enum { EX_PORTIONS = 0, EX_SINGLE = 1, EX_BLOCKS = 2, EX_RANGES = 3 };
 template <int NJ, int RT, int MODE, bool ANY>          // NJ: groups of 16 features, 4 or 8; ANY: pages of any size, else of 2^page_shift >= 4
 __global__ __launch_bounds__(256, NJ * RT > 4 ? 2 : 4) void attn_exact_f32_kernel(
         const float* __restrict__ q, int q_stride, float* __restrict__ out, int out_stride,
@@ -82,8 +84,9 @@ __global__ __launch_bounds__(256, NJ * RT > 4 ? 2 : 4) void attn_exact_f32_kerne
         const int* __restrict__ cu_q, const int* __restrict__ q_start, const int* __restrict__ row_of_token,
         const int* __restrict__ positions, const int* __restrict__ kv_lens,
         int num_rows, int H, int Hkv, int hd, int page, int page_shift, float scale, int window, int TQ,
-        int slots, float* __restrict__ part_ml, float* __restrict__ part_o) {
+        int slots, int range, float* __restrict__ part_ml, float* __restrict__ part_o) {
     constexpr int NF = NJ / 4;                         // feature tiles a wave
+    constexpr bool PARTIAL = MODE == EX_BLOCKS || MODE == EX_RANGES;       // every block of keys leaves a partial result
     __shared__ float4 probs[2][RT][4][64];             // [buffer][row tile][key tile][lane]
     __shared__ float tops[2][RT][4][16];               // [buffer][row tile][key tile][row]
     const int g_kv = blockIdx.y, G = H / Hkv;
@@ -93,6 +96,8 @@ __global__ __launch_bounds__(256, NJ * RT > 4 ? 2 : 4) void attn_exact_f32_kerne
         nt = 1;
         b = row_of_token[t0];
         p0 = positions[t0];
+        // a padding token, or behind the token, as most blocks of a large step are: gone after one trip to memory (which costs the others 0.5 us)
+        if (PARTIAL && gridDim.x * gridDim.y * gridDim.z > EX_FEW_BLOCKS && (b < 0 || ((window > 0 ? max(0, p0 + 1 - window) : 0) / EX_KEYS + (int)blockIdx.x * (MODE == EX_BLOCKS ? 1 : range)) * EX_KEYS > p0)) return;
     } else {
         // which request and which of its tokens: tiles are numbered request by request; late tiles, which see the most keys, run first
         const int tile = (int)gridDim.x - 1 - (int)blockIdx.x;
@@ -154,10 +159,12 @@ __global__ __launch_bounds__(256, NJ * RT > 4 ? 2 : 4) void attn_exact_f32_kerne
     // condition would be waited for all at once.
     const int kj = 16 * wave + 4 * (r & 3) + (r >> 2);
     int kb0 = first_key / EX_KEYS, kb1 = last_visible > first_key ? (last_visible + EX_KEYS - 1) / EX_KEYS : kb0;
-    if (MODE == EX_BLOCKS) {                           // one block of keys
-        kb0 += blockIdx.x;
+    const int kb_first = kb0;                          // of the token: slot 0 of its partial results
+    if (PARTIAL) {                                     // one block of keys, or `range` of them in turn
+        kb0 += (int)blockIdx.x * (MODE == EX_BLOCKS ? 1 : range);
+        kb1 = min(kb1, kb_first + slots);              // whatever kv_lens says
         if (kb0 >= kb1) return;
-        kb1 = kb0 + 1;
+        kb1 = MODE == EX_BLOCKS ? kb0 + 1 : min(kb1, kb0 + range);
     }
     int pk = -1, pv[4] = {-1, -1, -1, -1};             // pages of the block that is asked for next
     bool v_there[4] = {};                              // of the block that is used next
@@ -312,12 +319,12 @@ __global__ __launch_bounds__(256, NJ * RT > 4 ? 2 : 4) void attn_exact_f32_kerne
 #pragma unroll
                     for (int rt = 0; rt < RT; ++rt)
                         acc_b[rt][f] = __builtin_amdgcn_mfma_f32_16x16x4f32(elem(v4[f][t], i), elem(p[rt][t], i), acc_b[rt][f], 0, 0, 0);
-        if (MODE == EX_BLOCKS) {                       // the block's partial results
+        if (PARTIAL) {                                 // the block's partial results
 #pragma unroll
             for (int rt = 0; rt < RT; ++rt) {
                 const int i = rt * 16 + r;
                 if (i >= R) continue;
-                const size_t at = ((size_t)t0 * H + (size_t)g_kv * G + i) * slots + blockIdx.x;
+                const size_t at = ((size_t)t0 * H + (size_t)g_kv * G + i) * slots + (kb - kb_first);
                 if (wave == 0 && g == 0) {
                     part_ml[at * 2] = m_b[rt];
                     part_ml[at * 2 + 1] = l_b[rt];
@@ -329,7 +336,7 @@ __global__ __launch_bounds__(256, NJ * RT > 4 ? 2 : 4) void attn_exact_f32_kerne
                         make_float4(acc_b[rt][f][0], acc_b[rt][f][1], acc_b[rt][f][2], acc_b[rt][f][3]);
                 }
             }
-            return;
+            continue;
         }
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt) {
@@ -345,6 +352,7 @@ __global__ __launch_bounds__(256, NJ * RT > 4 ? 2 : 4) void attn_exact_f32_kerne
                 for (int e = 0; e < 4; ++e) acc[rt][f][e] = sum[f * 4 + e];
         }
     }
+    if (PARTIAL) return;
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt) {
         const int i = rt * 16 + r;
@@ -361,10 +369,10 @@ __global__ __launch_bounds__(256, NJ * RT > 4 ? 2 : 4) void attn_exact_f32_kerne
 }
 
 // ---------------------------------------------------------------------------
-// Single tokens.  Where they are few, a block takes one block of 64 keys of a token ("flash decoding"; reference:
-// crates/infer-backend-cuda/src/kernels/flash_attn_gqa/flash_attn_paged_decode.cu:75-337) and leaves its partial result, and a
-// second kernel merges a row's partial results in ascending order of the blocks; where (token, key/value head) pairs fill the
-// chip, a block takes all of its token's keys in turn and there is no second kernel.
+// Single tokens.  A block takes one block of 64 keys of a token ("flash decoding"; reference:
+// crates/infer-backend-cuda/src/kernels/flash_attn_gqa/flash_attn_paged_decode.cu:75-337), or several in turn, and leaves their partial
+// results, and a second kernel merges a row's partial results in ascending order of the blocks; of few keys a block takes
+// all of its token's, and there is no second kernel (exact_split).
 // Partial results: part_ml [T][H][slots][2] = (m_b, l_b), part_o [T][H][slots][hd]; slot s of a
 // token is key block first_block + s, first_block = (first visible key) / 64.
 // ---------------------------------------------------------------------------
@@ -381,7 +389,7 @@ __global__ __launch_bounds__(64) void attn_exact_combine_kernel(
         const int p = positions[t];
         const int visible = min(kv_lens[b], p + 1);
         const int j0 = window > 0 ? max(0, p + 1 - window) : 0;
-        if (visible > j0) n = (visible - 1) / EX_KEYS - j0 / EX_KEYS + 1;
+        if (visible > j0) n = min((visible - 1) / EX_KEYS - j0 / EX_KEYS + 1, slots);
     }
     const float* ml = part_ml + ((size_t)t * H + h) * slots * 2;
     const float* po = part_o + ((size_t)t * H + h) * slots * hd;
@@ -414,11 +422,25 @@ __global__ __launch_bounds__(64) void attn_exact_combine_kernel(
     }
 }
 
-// Single tokens: from so many (token, key/value head) pairs on, or up to so many keys, a block takes all of a token's keys.
-// Measured, us, a key a lane and a wave a block of keys (before) / all keys a block / a block of keys a block and the merge, 8 key/value heads of
-// 64: 1 token of 100 keys 16.7 / 7.1 / 8.6, of 500 18.2 / 17.4 / 8.4, of 2,000 22 / 57 / 13; 6 tokens of 100 17 / 7.3 / 8.6, of 1,000 21 / 32 / 14, of
-// 4,000 42 / 120 / 34; 32 tokens of 500 28 / 20 / 20, of 2,000 79 / 65 / 55; 64 tokens of 100 20 / 10 / 12, of 2,000 169 / 101 / 120.
-constexpr int EX_SINGLE_PAIRS = 512, EX_SINGLE_KEYS = 128;
+// How a single token's keys are divided between blocks: `range` blocks of 64 keys a block, in turn, and `blocks` blocks a (token, key/value
+// head) pair; range 0: all of them in one block that writes the output itself, with no merge.  The step is planned for a longest length that
+// its rows need not have (a captured step for its bucket's), and rows differ: blocks beyond a row's end are as common as others, so they leave after
+// one trip to memory, and a long row is not left to one block.  One block of keys a block while there are up to 30,000 blocks; above, ranges of 4 to 64.
+// An odd number of blocks a pair: consecutive ones go around the eight XCDs, and the empty ones would all be some XCDs'.
+// Measured, us, a key a lane and a wave a block of keys (first) / a block of keys a block, all of a token's from 512 pairs on (then) / now, 8 key/value heads
+// of 64: 64 tokens, one of 16,000 keys and the others of 200 97 / 703 / 86, one of 3,000 and the others of 100 42 / 137 / 30; 64 ragged up to 1,000
+// keys 51 / 52 / 30, up to 4,000 155 / 186 / 120, equal 1,000 95 / 54 / 64, 4,000 313 / 195 / 230; 16, one of 16,000 84 / 94 / 73; 128 tokens of 32
+// heads of 128 with keys of their own, ragged up to 1,000 424 / 461 / 356, but up to 60 67 / 80 / 91.  (Equal rows lose what ragged ones need: no length but
+// the longest is known here.)
+constexpr int EX_SINGLE_KEYS = 128;
+struct ExactSplit { int blocks, range; };
+ExactSplit exact_split(long long pairs, int max_kv_len) {
+    if (max_kv_len <= EX_SINGLE_KEYS) return {1, 0};
+    const int slots = (max_kv_len + EX_KEYS - 1) / EX_KEYS + 1;           // a window may begin inside a block: one more
+    const long long most = std::max(30000 / pairs, 1ll);
+    const int range = most >= slots ? 1 : (int)std::min(std::max((slots + most - 1) / most, 4ll), 64ll);
+    return {((slots + range - 1) / range) | 1, range};
+}
 
 // Two tiles of rows a block where a token's heads fill more than one, or values are read one at a time: pages of no power of two of four keys and
 // more, or a value cache that does not begin at a multiple of 16 bytes (shift -1).
@@ -428,18 +450,25 @@ bool exact_two_tiles(int G, int shift) { return G > 16 || shift < 0; }
 template <int MODE>
 void launch_exact(dim3 grid, int hd, int TQ, const float* q, int q_stride, float* out, int out_stride, const float* kc, const float* vc,
                   const int* table, int max_blocks, const int* cu_q, const int* q_start, const int* row_of_token, const int* positions,
-                  const int* kv_lens, int num_rows, int H, int Hkv, int page, float scale, int window, int slots, float* part_ml, float* part_o,
+                  const int* kv_lens, int num_rows, int H, int Hkv, int page, float scale, int window, int slots, int range, float* part_ml, float* part_o,
                   hipStream_t stream) {
     const int shift = exact_page_shift(page, vc);
     const bool two = exact_two_tiles(H / Hkv, shift);
 #define RI_EXACT(NJ_, RT_, ANY_) attn_exact_f32_kernel<NJ_, RT_, MODE, ANY_><<<grid, 256, 0, stream>>>(q, q_stride, out, out_stride, kc, vc, table, max_blocks, \
-        cu_q, q_start, row_of_token, positions, kv_lens, num_rows, H, Hkv, hd, page, shift, scale, window, TQ, slots, part_ml, part_o)
+        cu_q, q_start, row_of_token, positions, kv_lens, num_rows, H, Hkv, hd, page, shift, scale, window, TQ, slots, range, part_ml, part_o)
     if (hd <= 64) { if (shift < 0) RI_EXACT(4, 2, true); else if (two) RI_EXACT(4, 2, false); else RI_EXACT(4, 1, false); }
     else { if (shift < 0) RI_EXACT(8, 2, true); else if (two) RI_EXACT(8, 2, false); else RI_EXACT(8, 1, false); }
 #undef RI_EXACT
 }
 
 }  // namespace
+
+// exact_split, for a test without a GPU.
+extern "C" void ri_attention_exact_split(int T, int Hkv, int max_kv_len, int* blocks, int* range) {
+    const ExactSplit split = exact_split((long long)T * Hkv, max_kv_len);
+    *blocks = split.blocks;
+    *range = split.range;
+}
 
 // Whether ri_attention_exact_f32 takes these sizes (else: the generic kernel).
 extern "C" int ri_attention_exact_supported(int H, int Hkv, int hd, int page) {
@@ -465,7 +494,7 @@ extern "C" int ri_attention_exact_f32(
     const int TQ = (exact_two_tiles(G, exact_page_shift(page, vc)) ? 32 : 16) / G;
     const int tiles = (T + TQ - 1) / TQ + num_rows;    // at most: every request may end in a short tile
     launch_exact<EX_PORTIONS>(dim3(tiles, Hkv), hd, TQ, q, q_stride, out, out_stride, kc, vc, table, max_blocks, cu_q, q_start, nullptr, nullptr, kv_lens,
-                              num_rows, H, Hkv, page, scale, window, 0, nullptr, nullptr, stream);
+                              num_rows, H, Hkv, page, scale, window, 0, 0, nullptr, nullptr, stream);
     RI_LAUNCHED("ri_attention_exact_f32");
     return 0;
 }
@@ -496,17 +525,23 @@ extern "C" int ri_attention_exact_decode_f32(
     RI_REQUIRE(workspace_floats >= ri_attention_exact_decode_workspace(T, H, hd, max_kv_len),
                "ri_attention_exact_decode_f32: workspace of %zu floats, %zu needed", workspace_floats,
                ri_attention_exact_decode_workspace(T, H, hd, max_kv_len));
-    if ((long long)T * Hkv >= EX_SINGLE_PAIRS || max_kv_len <= EX_SINGLE_KEYS) {
+    const ExactSplit split = exact_split((long long)T * Hkv, max_kv_len);
+    if (split.range == 0) {
         launch_exact<EX_SINGLE>(dim3(T, Hkv), hd, 1, q, q_stride, out, out_stride, kc, vc, table, max_blocks, nullptr, nullptr, row_of_token, positions,
-                                kv_lens, T, H, Hkv, page, scale, window, 0, nullptr, nullptr, stream);
+                                kv_lens, T, H, Hkv, page, scale, window, 0, 0, nullptr, nullptr, stream);
         RI_LAUNCHED("ri_attention_exact_decode_f32");
         return 0;
     }
-    const int slots = (max_kv_len + EX_KEYS - 1) / EX_KEYS + 1;       // a window may begin inside a block: one more
+    const int slots = (max_kv_len + EX_KEYS - 1) / EX_KEYS + 1;
     float* part_ml = workspace + (size_t)T * H * slots * hd;
     float* part_o = workspace;
-    launch_exact<EX_BLOCKS>(dim3(slots, Hkv, T), hd, 1, q, q_stride, out, out_stride, kc, vc, table, max_blocks, nullptr, nullptr, row_of_token, positions,
-                            kv_lens, T, H, Hkv, page, scale, window, slots, part_ml, part_o, stream);
+    const dim3 grid(split.blocks, Hkv, T);
+    if (split.range == 1)
+        launch_exact<EX_BLOCKS>(grid, hd, 1, q, q_stride, out, out_stride, kc, vc, table, max_blocks, nullptr, nullptr, row_of_token, positions,
+                                kv_lens, T, H, Hkv, page, scale, window, slots, 1, part_ml, part_o, stream);
+    else
+        launch_exact<EX_RANGES>(grid, hd, 1, q, q_stride, out, out_stride, kc, vc, table, max_blocks, nullptr, nullptr, row_of_token, positions,
+                                kv_lens, T, H, Hkv, page, scale, window, slots, split.range, part_ml, part_o, stream);
     RI_LAUNCHED("ri_attention_exact_decode_f32");
     auto combine = hd <= 64 ? attn_exact_combine_kernel<1> : attn_exact_combine_kernel<2>;
     combine<<<dim3(H, T), 64, 0, stream>>>(part_ml, part_o, row_of_token, positions, kv_lens, H, hd, window, slots, out, out_stride);

@@ -1304,6 +1304,8 @@ def test_exact_attention_of_single_tokens_on_every_route(ops, H, Hkv, hd, page, 
     single(list(range(len(ends))) * 3, 1024)                  # as a captured step passes it: a longest length that none has
     single([0, 3, 6], 128)                                    # few keys
     single((list(range(len(ends))) * 50)[:512 // Hkv + 1], 260)
+    single((list(range(len(ends))) * 50)[:512 // Hkv + 1], 2000)        # ranges of four blocks of keys, two to a row
+    single(list(range(len(ends))), 60000 * 8 // Hkv)          # ranges of several blocks of keys, most of them behind the rows' ends
 
 
 def test_attention_padding_rows_touch_nothing(ops):

@@ -77,3 +77,20 @@ def test_exact_attention_refuses_operands_that_its_loads_cannot_take(lib, shifte
     if shifted == "k":
         rc = lib.ri_attention_exact_f32(at["q"], H * hd, at["out"], H * hd, at["k"], at["v"], 64, page, H, Hkv, hd, at["table"], 32, i, i, i, 1, T, f, 0, zero)
         assert rc != 0 and b"unaligned" in lib.ri_last_error()
+
+
+def test_exact_attention_of_single_tokens_divides_long_rows(lib):
+    """A row of any length is taken by blocks of at most 64 blocks of keys in turn (a chain of some 110 us), whatever the number of rows; every slot
+    has a block, and no half of the chip is left the empty ones."""
+    blocks, rng = ctypes.c_int(), ctypes.c_int()
+    for T in (1, 3, 16, 63, 64, 100, 128, 1000, 60000):
+        for heads in (1, 2, 8, 32):
+            for longest in (1, 128, 129, 500, 1024, 1025, 2048, 4096, 16000, 131072):
+                lib.ri_attention_exact_split(T, heads, longest, ctypes.byref(blocks), ctypes.byref(rng))
+                slots = (longest + 63) // 64 + 1
+                if longest <= 128:
+                    assert (blocks.value, rng.value) == (1, 0)
+                    continue
+                assert 1 <= rng.value <= 64 and blocks.value * rng.value >= slots and blocks.value % 2 == 1
+                assert (blocks.value - 2) * rng.value < slots
+                assert rng.value == 1 or T * heads * slots > 30000
