@@ -293,18 +293,24 @@ __global__ __launch_bounds__(BW * 64) void attn_decode_split_kernel(
 
 constexpr int LIST_SPAN = 32, LIST_ROWS = 64, LIST_WAVES = 512;
 
-// How the list below is divided: spans of keys [first, end), the waves of a list of `total` spans (a stretch is two spans or more, or
-// all), the first span of wave w, the wave of span f, and the slots a row of at most max_kv_len keys needs: the waves between its
-// first and its last have two of its spans or more.
+// How the list below is divided: spans of keys [first, end), the waves of a list of `total` spans, the first span of wave w, the wave of
+// span f, and the slots a row of at most max_kv_len keys has: one a span up to 64, else as many as it meets waves whose stretches are two spans or
+// more (those between its first and its last have two of its spans or more).  Stretches of one span are for short lists: 5 rows of 20 keys 10.9 -> 7.9 us.
 __host__ __device__ inline int list_spans(int first, int end) { return end > first ? (end + LIST_SPAN - 1) / LIST_SPAN - first / LIST_SPAN : 0; }
-__host__ __device__ inline uint32_t list_waves(uint32_t total, uint32_t most) { const uint32_t two = total / 2 > 1 ? total / 2 : 1; return most < two ? most : two; }
+__host__ __device__ inline int list_slots(int max_kv_len) {
+    const int spans = (max_kv_len + LIST_SPAN - 1) / LIST_SPAN, two = spans / 2 + 1;
+    return spans <= 64 ? spans : two > 64 ? two : 64;
+}
+__host__ __device__ inline uint32_t list_waves(uint32_t total, uint32_t most, int max_kv_len) {
+    const uint32_t useful = max_kv_len <= 64 * LIST_SPAN || total <= 64 ? total : total / 2;
+    return most < useful ? most : useful;
+}
 __host__ __device__ inline uint32_t list_from(uint32_t w, uint32_t total, uint32_t waves) { return w * total / waves; }       // (waves total < 2^32: the host's rule)
 __host__ __device__ inline uint32_t list_wave_of(uint32_t f, uint32_t total, uint32_t waves) { return ((f + 1) * waves - 1) / total; }
-__host__ __device__ inline int list_slots(int max_kv_len) { return (max_kv_len + LIST_SPAN - 1) / LIST_SPAN / 2 + 1; }
 
 // The same for a test that divides a list without a GPU.
 extern "C" int ri_attention_list_spans(int first, int end) { return list_spans(first, end); }
-extern "C" unsigned ri_attention_list_waves(unsigned total, unsigned most) { return list_waves(total, most); }
+extern "C" unsigned ri_attention_list_waves(unsigned total, unsigned most, int max_kv_len) { return list_waves(total, most, max_kv_len); }
 extern "C" unsigned ri_attention_list_from(unsigned w, unsigned total, unsigned waves) { return list_from(w, total, waves); }
 extern "C" unsigned ri_attention_list_wave_of(unsigned f, unsigned total, unsigned waves) { return list_wave_of(f, total, waves); }
 extern "C" int ri_attention_list_slots(int max_kv_len) { return list_slots(max_kv_len); }
@@ -321,9 +327,8 @@ extern "C" int ri_attention_list_slots(int max_kv_len) { return list_slots(max_k
 // to the matrix instruction as the sum of two bfloat16, which costs a bound-by-memory kernel nothing (error of the
 // output against 64 bits 2.1e-3 -> 1.7e-3, that of its own rounding).
 // What bounds it: the bytes, and 8 us of launches, chains of small loads and the merge.  Head 128, page 16, with the merge, us, before (blocks a
-// row) / now, and the bytes at 6.87 TB/s: 43 rows of 210..3,000 keys 54.7 / 37.2 (29.2), 30 of them 54.9 / 29.2 (19.8), 20 rows of 97..1,333
-// 20.2 / 14.7 (6.1), 24 rows of 1,500 41 / 29 (21.5), 8 rows of 700 13.2 / 11.2, 40 rows of 60 17 / 9.2, 64 rows of 2,050 95 / 92 (78); equal: 8 rows of 2,050 17.8 /
-// 17.5; slower: 32 rows of 2,050 48.7 / 49.9 and 30 of 700 18.4 / 20.7, where one block a row fills the chip and needs no merge.
+// row) / now, and the bytes at 6.87 TB/s: 43 rows of 210..3,000 keys 54.7 / 37.2 (29.2), 20 rows of 97..1,333
+// 20.2 / 14.7 (6.1), 24 rows of 1,500 41 / 29 (21.5), 8 rows of 700 13.2 / 11.2, 64 rows of 2,050 95 / 92 (78).  list_pays says where it is taken.
 __global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
         const bf16_t* __restrict__ q, int q_stride, const bf16_t* __restrict__ kc, const bf16_t* __restrict__ vc,
         const int* __restrict__ table, int max_blocks, const int* __restrict__ row_of_token, const int* __restrict__ positions,
@@ -352,7 +357,7 @@ __global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
     }
     const uint32_t total = (uint32_t)__builtin_amdgcn_readlane(ends, 63);
     if (total == 0) return;
-    const uint32_t W = list_waves(total, gridDim.x), w = blockIdx.x;
+    const uint32_t W = list_waves(total, gridDim.x, max_kv_len), w = blockIdx.x;
     if (w >= W) return;
     const int f0 = (int)list_from(w, total, W), f1 = (int)list_from(w + 1, total, W);
     struct Row { int tok, row, first, end, f0, n; };        // spans [f0, f0 + n) of the list
@@ -647,12 +652,30 @@ static int decode_chunk(int T, int Hkv, int hd, int max_kv_len) {
 }
 
 extern "C" size_t ri_attention_decode_workspace(int rows, int H, int hd, int max_kv_len) {
-    const size_t splits = (size_t)list_slots(max_kv_len);       // no other form leaves more
+    const size_t splits = (size_t)std::max(list_slots(max_kv_len), (max_kv_len + 63) / 64);       // of the list's form, and of the others
     return ((size_t)rows * H * splits * (hd + 2) + rows) * sizeof(float);
 }
 
 extern "C" int ri_attention_decode_supported(int H, int Hkv, int hd, int page) {
     return (hd == 64 || hd == 128) && page % 16 == 0 && Hkv > 0 && H % Hkv == 0 && H / Hkv <= 16;
+}
+
+// Whether a step of T single tokens alone takes the list of spans.  It divides rows of any lengths evenly, and pays a merge for it.  Blocks a row are better
+// where one block a (key/value head, token) pair nearly fills the chip and writes its output itself, for rows that are short or alike.  Which rows are is not
+// known here, only the longest length the step was planned for, so 129 to 256 pairs keep their blocks up to 1,024 keys.
+// Measured, us, head 128, blocks a row / list, 8 heads: 24 equal rows of 20 keys 5.5 / 8.2, of 100 6.5 / 9.2, of 700 16.6 / 18.5, of 1,500 32.6 / 27.6, ragged ones
+// up to 1,000 20.3 / 13.7 (given up for the equal ones), up to 3,000 42 / 24; 32 rows, equal 700 18.5 / 21.1, 1,500 35.5 / 36.4, 2,050 46.6 / 48.3, 4,000 86 / 84,
+// ragged up to 3,000 54 / 28 (kept).  Elsewhere: 8 rows of 20 9.0 / 7.8, of 2,050 18.4 / 17.9, 12 of 100 9.4 / 8.6, 40 of 100 18 / 10, 64 of 100 11.8 / 12.0, of 700
+// 35 / 34, ragged up to 1,000 34 / 21; the worst, 56 of 65 10.2 / 11.3.  Fewer than 12 pairs: 3 ragged rows of 2 heads up to 3,000 10.5 / 11.2.  Head 64:
+// 43 rows of 210..3,000 37 / 25, but 16 rows of 2,050 18.4 / 19.8 and 32 27 / 31: never.
+static bool list_pays(long long pairs, int hd, int max_kv_len) {
+    return hd == 128 && pairs >= 12 && !(pairs > 128 && pairs <= 256 && max_kv_len <= 1024);
+}
+
+// Whether a step of T single tokens alone goes as a list: what it takes (rows for the lanes of a wave, w total below 2^32), and where it pays.
+extern "C" int ri_attention_decode_as_list(int T, int Hkv, int hd, int page, int max_kv_len) {
+    const long long spans = (long long)T * ((max_kv_len + LIST_SPAN - 1) / LIST_SPAN + 1);
+    return T >= 3 && T <= LIST_ROWS && (page & (page - 1)) == 0 && spans < (1ll << 32) / LIST_WAVES && list_pays((long long)T * Hkv, hd, max_kv_len);
 }
 
 extern "C" int ri_attention_decode(
@@ -708,12 +731,9 @@ extern "C" int ri_attention_decode(
     // 50.6, 4 rows 20.3 -> 18.0 (8); head 64: 16 rows of 2,048 keys 23.8 -> 18.1, 8 rows of 4,096
     // 20.7 -> 18.1.  pair_blocks: 0 lets the entry point choose, 1 forbids several blocks a pair,
     // more asks for that many.
-    // A step of single tokens alone, three to as many as a wave has lanes: one list of spans (see the kernel; two rows of 2,050 keys take 11.3 us either
-    // way, one of 91 7.3 without and 9.0 with it; head 64: 43 rows of 210..3,000 37 / 25 us, but 16 rows of 2,050 18.4 / 19.8 and 32
-    // 27 / 31, so it keeps its blocks a row).  w total stays below 2^32.
-    const long long spans = (long long)T * ((max_kv_len + LIST_SPAN - 1) / LIST_SPAN + 1);
-    if (hd == 128 && pair_blocks == 0 && !cu_q && T >= 3 && T <= LIST_ROWS && (page & (page - 1)) == 0 && spans < (1ll << 32) / LIST_WAVES) {
-        const int W = (int)std::max(1ll, std::min<long long>(LIST_WAVES / Hkv, spans / 2));
+    if (pair_blocks == 0 && !cu_q && ri_attention_decode_as_list(T, Hkv, hd, page, max_kv_len)) {
+        const long long spans = (long long)T * ((max_kv_len + LIST_SPAN - 1) / LIST_SPAN + 1);
+        const int W = (int)std::max(1ll, std::min<long long>(LIST_WAVES / Hkv, spans));
         const int slots = list_slots(max_kv_len);
         float* sums = (float*)workspace;
         float* ml = sums + (size_t)rows * H * slots * hd;

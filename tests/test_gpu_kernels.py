@@ -817,8 +817,29 @@ def test_single_token_attention_of_rows_of_any_lengths(ops, case, window):
     _check_rope_write_and_attention(ops, torch.bfloat16, case, window)
 
 
-def test_single_token_attention_as_a_list_with_padding_and_rows_out_of_order(ops):
-    B, H, Hkv, hd, page = 6, 8, 2, 128, 16
+@pytest.mark.parametrize("case,window,as_list", [
+    ((5, 16, 8, 128, 16, [1] * 5, [30, 31, 32, 63, 64]), 0, 1),                                  # ends around a span's
+    ((3, 3, 3, 128, 16, [1] * 3, [0, 63, 300]), 0, 0),                                           # fewer than 12 pairs
+    ((3, 8, 4, 128, 16, [1] * 3, [0, 64, 1]), 0, 1),
+    ((64, 4, 1, 128, 16, [1] * 64, [2047, 0] * 32), 0, 1),                                       # 64 spans: a slot a span
+    ((64, 4, 1, 128, 16, [1] * 64, [2048, 0] * 32), 0, 1),                                       # one more: stretches of two
+    ((32, 4, 1, 128, 64, [1] * 32, [2500, 0, 700, 15, 16, 17, 1300, 95] * 4), 0, 1),             # 512 waves a head; rows of one span among long ones
+    ((16, 6, 2, 128, 16, [1] * 16, [999, 1000, 1001, 1040] * 4), 33, 1),                         # a window that begins inside a span
+    ((17, 8, 8, 128, 16, [1] * 17, [1023] * 9 + [5] * 8), 0, 0),                                 # one block a pair nearly fills the chip ...
+    ((17, 8, 8, 128, 16, [1] * 17, [1024] * 9 + [5] * 8), 0, 1),                                 # ... from so many keys on not
+    ((32, 8, 8, 128, 64, [1] * 32, [700] + [40] * 31), 0, 0),
+    ((16, 8, 8, 128, 64, [1] * 16, [700] + [40] * 15), 0, 1),
+    ((33, 8, 8, 128, 32, [1] * 33, [(i * 29) % 300 for i in range(33)]), 0, 1),                  # 264 pairs
+])
+def test_single_token_attention_as_a_list_where_it_pays(ops, case, window, as_list):
+    B, H, Hkv, hd, page, q_lens, starts = case
+    assert ops._lib().ri_attention_decode_as_list(B, Hkv, hd, page, max(starts) + 1) == as_list
+    _check_rope_write_and_attention(ops, torch.bfloat16, case, window)
+
+
+@pytest.mark.parametrize("heads", [2, 8])
+def test_single_token_attention_as_a_list_with_padding_and_rows_out_of_order(ops, heads):
+    B, H, Hkv, hd, page = 6, 8, heads, 128, 16
     lens = [300, 7, 1200, 64, 65, 500]
     qkv, kc, vc, table, ctx, _, _ = _paged_setup(torch.bfloat16, B, H, Hkv, hd, page, [1] * B, [n - 1 for n in lens], seed=3, num_pages=160)
     ops.rope_kv_write(qkv, H, Hkv, hd, None, ctx.positions, ctx.row_of_token, kc, vc, table, page)

@@ -22,7 +22,7 @@ def _divide(lib, rows, max_kv_len, heads):
         return {}, {}
     planned = len(rows) * ((max_kv_len + 31) // 32 + 1)                       # the entry point's bound of the list
     assert planned >= total and planned * 512 < 1 << 32
-    waves = lib.ri_attention_list_waves(total, max(1, min(512 // heads, planned // 2)))
+    waves = lib.ri_attention_list_waves(total, max(1, min(512 // heads, planned)), max_kv_len)
     begins = [sum(n[:i]) for i in range(len(n))]
     slots, counts = {}, {}
     assert lib.ri_attention_list_from(0, total, waves) == 0 and lib.ri_attention_list_from(waves, total, waves) == total
@@ -44,7 +44,7 @@ def test_list_of_spans_holds_every_span_once_in_slots_that_are_there(lib, seed):
     rng = random.Random(seed)
     for _ in range(10):
         T, heads, window = rng.randint(1, 64), rng.choice([1, 2, 3, 8, 32, 512]), rng.choice([0, 0, 1, 33, 700])
-        longest = rng.choice([1, 31, 32, 33, 64, 700, 3000])
+        longest = rng.choice([1, 31, 32, 33, 64, 700, 2048, 2049, 3000, 9000])
         ends = [rng.choice([0, 1, longest, rng.randint(0, longest)]) for _ in range(T)]
         # kv_lens may say more than the step was planned for
         max_kv_len = rng.choice([longest, -(-longest // 1024) * 1024, max(1, longest // 2)])
