@@ -439,14 +439,15 @@ __global__ __launch_bounds__(64, 2) void attn_decode_list_kernel(
             }
         m = fmaxf(m, __shfl_xor(m, 16, 64));
         m = fmaxf(m, __shfl_xor(m, 32, 64));
-        const float alpha = __expf(m_run - m);              // 0 if nothing was seen so far
+        const float top = m > -INFINITY ? m : 0.f;          // (a span whose every score is -inf has no weight, and takes none from the others)
+        const float alpha = __expf(m_run - top);            // 0 if nothing was seen so far
         float sum = 0.f;
         bf16x8_t pf[KT / 2], rest[KT / 2];
 #pragma unroll
         for (int t = 0; t < KT; ++t)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float x = __expf(st[t][i] - m);       // exp(-inf) = 0 for masked keys
+                const float x = __expf(st[t][i] - top);     // exp(-inf) = 0 for masked keys
                 sum += x;
                 const __bf16 y = (__bf16)x;
                 pf[t >> 1][4 * (t & 1) + i] = y;

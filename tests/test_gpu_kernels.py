@@ -858,6 +858,30 @@ def test_single_token_attention_as_a_list_with_padding_and_rows_out_of_order(ops
             assert torch.allclose(got[t].float(), want[b].float(), rtol=2.0 ** -7, atol=1e-3), t
 
 
+def test_single_token_attention_as_a_list_with_scores_of_minus_infinity(ops):
+    """Keys whose scores are -inf have no weight, also where a whole span of 32 has no other (its first, in the middle, its last) or a wave's whole stretch."""
+    B, H, Hkv, hd, page = 12, 8, 8, 128, 16
+    lens = [300, 64, 90, 33, 300, 200, 40, 70, 100, 300, 65, 96]
+    qkv, kc, vc, table, ctx, _, _ = _paged_setup(torch.bfloat16, B, H, Hkv, hd, page, [1] * B, [n - 1 for n in lens], seed=6, num_pages=200)
+    qkv[:, :H * hd] = qkv[:, :H * hd].abs()             # so that a key of -inf scores -inf
+    ops.rope_kv_write(qkv, H, Hkv, hd, None, ctx.positions, ctx.row_of_token, kc, vc, table, page)
+    dead = [range(0, 32), range(32, 63), range(0, 64), range(0, 32), range(0, 288), range(64, 192), range(0, 39), range(10, 69), range(0, 96), range(5, 299), (), range(32, 64)]
+    for b, keys in enumerate(dead):
+        for j in keys:
+            kc[int(table[b, j // page]), :, j % page] = float("-inf")
+    assert ops._lib().ri_attention_decode_as_list(B, Hkv, hd, page, max(lens)) == 1
+    got = torch.full((B, H * hd), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.paged_attention(qkv, got, H, Hkv, hd, kc, vc, table, page, ctx, 0.01, 0)
+    for b, n in enumerate(lens):
+        pages = table[b, :(n + page - 1) // page].long()
+        k = kc[pages].permute(1, 0, 2, 3).reshape(Hkv, -1, hd)[:, :n].double()
+        v = vc[pages].permute(1, 0, 3, 2).reshape(Hkv, -1, hd)[:, :n].double()
+        p = torch.softmax((qkv[b, :H * hd].view(H, 1, hd).double() * k).sum(-1) * 0.01, -1)
+        ref = (p[..., None] * v).sum(1).reshape(-1)
+        # one bfloat16 rounding of the output, on weights of two bfloat16 (2^-16)
+        assert torch.all((got[b].double() - ref).abs() <= 2.0 ** -8 * ref.abs() + 1e-4), b
+
+
 @pytest.mark.parametrize("window", [0, 500])
 def test_single_token_attention_as_a_list_ends_at_the_steps_longest_length(ops, window):
     """A row that kv_lens says is longer than the step was planned for: its keys beyond that are not looked at, and the others' results
