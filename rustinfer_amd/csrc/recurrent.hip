@@ -663,7 +663,7 @@ __global__ __launch_bounds__(256) void gated_group_norm_kernel(
 }
 
 // Eight values a thread, read once: groups of 8 to 2,048 values, a power of two, rows and pointers at multiples of 16 bytes.  A group
-// lies in group / 8 neighbouring lanes, or in whole waves of the block whose sums meet in LDS.  What bounds it: the bytes, or for a
+// lies in group / 8 neighbouring lanes, or in whole waves of the block (of 64 to 256 threads) whose sums meet in LDS.  What bounds it: the bytes, or for a
 // few rows the launch and one round trip; the kernel above waits for each value it squares and reads every row again.  Measured, us, above / this,
 // with a gate: 2,048 rows of 32 groups of 64 24.3 / 9.6 and of one group of 2,048 21.0 / 9.6 (33 MB: 4.9 at 6.9 TB/s), 8 rows 4.7 / 4.7 and 10.6 / 4.7.
 template <typename T, typename TW>
@@ -671,7 +671,7 @@ __global__ __launch_bounds__(256) void gated_group_norm_x8_kernel(
         const float* __restrict__ o, int o_stride, int n, int group, const TW* __restrict__ w,
         const T* __restrict__ gate, int gate_stride, T* __restrict__ out, int out_stride, float eps, int gate_silu, int gate_first) {
     __shared__ float red[4];
-    const int t = blockIdx.x, wave = threadIdx.x >> 6, c = ((int)blockIdx.y * 256 + (int)threadIdx.x) * 8;
+    const int t = blockIdx.x, wave = threadIdx.x >> 6, c = ((int)blockIdx.y * (int)blockDim.x + (int)threadIdx.x) * 8;
     const bool live = c < n;
     float x[8], z[8], wt[8];
 #pragma unroll
@@ -716,6 +716,18 @@ __global__ __launch_bounds__(256) void gated_group_norm_x8_kernel(
 }
 }  // namespace
 
+// Where the kernel of eight values a thread is the better one: not for narrow rows, and for groups that are a wave's one value a lane or fewer only from so many
+// values on.  Measured, us, one value a lane / eight: groups of 64, 8 rows of 2,048 2.66 / 2.96, 43 2.81 / 3.00, 100 3.05 / 3.09, 300 4.3 / 3.6, 8,192 rows of 64 4.6 /
+// 6.7, 300 of 768 3.15 / 3.41; groups of 16, 8 rows of 2,048 2.67 / 2.86, 43 of 1,024 2.9 / 2.75, 1,000 of 64 3.2 / 3.5; of 128, 8 rows of 4,096 3.1 / 3.1, 8,192 of 128 5.5 / 6.6; of
+// 512, 8 rows 5.9 / 3.0.  In 32-bit the choice does not look at the number of rows: a row has the same bits beside any others.
+static bool group_norm_x8_pays(int T, int n, int group, int dtype) {
+    if (dtype == RI_F32) return n >= 256;
+    const long long values = (long long)T * n;
+    if (group >= 256 || group == 8) return true;
+    if (group == 16) return values >= 1 << 16;
+    return n >= 256 && (group == 128 || values >= 1 << 18);
+}
+
 extern "C" int ri_gated_group_norm(const float* o, int o_stride, int T, int n, int group, const void* w, int w_dtype,
                                    const void* gate, int gate_stride, void* out, int out_stride, int dtype,
                                    float eps, int gate_silu, int gate_first, hipStream_t stream) {
@@ -731,11 +743,12 @@ extern "C" int ri_gated_group_norm(const float* o, int o_stride, int T, int n, i
     const dim3 grid(T, big ? groups : (groups + block / 64 - 1) / (block / 64));
     // eight values a thread, from 16 bytes to 16 bytes (four 32-bit values, eight of bfloat16)
     const int per = dtype == RI_F32 ? 4 : 8;
-    const bool x8 = group >= 8 && group <= 2048 && (group & (group - 1)) == 0 && o_stride % 4 == 0 && out_stride % per == 0
+    const bool x8 = group_norm_x8_pays(T, n, group, dtype) && group >= 8 && group <= 2048 && (group & (group - 1)) == 0 && o_stride % 4 == 0 && out_stride % per == 0
                     && (!gate || gate_stride % per == 0) && (((uintptr_t)o | (uintptr_t)out | (uintptr_t)gate | (uintptr_t)w) & 15) == 0;
-    const dim3 grid8(T, (n + 2047) / 2048);
+    const int threads8 = min((n / 8 + 63) / 64 * 64, 256);
+    const dim3 grid8(T, (n / 8 + threads8 - 1) / threads8);
 #define RI_GGN(TT, TW) do { \
-        if (x8) gated_group_norm_x8_kernel<TT, TW><<<grid8, 256, 0, stream>>>(o, o_stride, n, group, (const TW*)w, (const TT*)gate, gate_stride, (TT*)out, out_stride, eps, gate_silu, gate_first); \
+        if (x8) gated_group_norm_x8_kernel<TT, TW><<<grid8, threads8, 0, stream>>>(o, o_stride, n, group, (const TW*)w, (const TT*)gate, gate_stride, (TT*)out, out_stride, eps, gate_silu, gate_first); \
         else if (big) gated_group_norm_kernel<TT, TW, true><<<grid, block, 0, stream>>>(o, o_stride, n, group, (const TW*)w, (const TT*)gate, gate_stride, (TT*)out, out_stride, eps, gate_silu, gate_first); \
         else gated_group_norm_kernel<TT, TW, false><<<grid, block, 0, stream>>>(o, o_stride, n, group, (const TW*)w, (const TT*)gate, gate_stride, (TT*)out, out_stride, eps, gate_silu, gate_first); } while (0)
     if (dtype == RI_F32 && w_dtype == RI_F32) RI_GGN(float, float);
