@@ -33,7 +33,7 @@
 // stop in front of it, and the walk does that head of that row from there on, so that every token gets what the walk gives.
 //
 // 2,048 tokens of 32 heads of 64, us a layer, the walk / this: delta form 1174 / 223, decay form 789 / 96; 24 heads of 128: 1692 / 583, 977 /
-// 192.  The operators (163 and 50 of the first two) are bound by the steps of a block following each other (two
+// 182.  The operators (163 and 50 of the first two) are bound by the steps of a block following each other (two
 // blocks a compute unit), the states (86, 55) by the chain of chunks: 64 chunks of about 1.3 us, 0.5 of which are its matrix instructions
 // (101, 69 with two waves, and with loads under a lane's condition, which the compiled loop waited for, 123 and 69).
 #include "common.h"
@@ -456,7 +456,8 @@ __global__ __launch_bounds__(256) void chunk_operators_kernel(const ChunkArgs a)
 // tokens, 32 heads of 64, two tiles / one: delta form 101 / 86; the decay form, whose waves then no longer all have outputs, 55 / 69.
 constexpr int state_tiles(int dk, bool delta) { return delta && dk <= 64 ? 1 : 2; }
 
-template <int DK, int DV, bool DELTA>
+// D: chunks whose operands are under way.
+template <int DK, int DV, bool DELTA, int D>
 __global__ __launch_bounds__(DK * 4 / state_tiles(DK, DELTA)) void chunk_states_kernel(const ChunkArgs a) {
     constexpr int Q = state_tiles(DK, DELTA), NA = DK / 16, NW = NA / Q;
     using U = Unit<DK, DV, DELTA>;
@@ -547,8 +548,6 @@ __global__ __launch_bounds__(DK * 4 / state_tiles(DK, DELTA)) void chunk_states_
     static_assert(NW >= 2, "two waves make the outputs");
     // D chunks' operands under way, asked for under no condition (the last one's again behind the end): at a place that can be
     // reached with fewer loads under way the compiled code would wait for more of them.
-    // (Heads of 128: with three, 2,048 tokens of 24 heads 192 -> 179 us in the decay form, but three rows of 200 67 -> 75.)
-    constexpr int D = DK > 64 ? 2 : 4;
     Ops x[D];
     if (chunks > 0) {
 #pragma unroll
@@ -592,7 +591,11 @@ int launch_chunks(ChunkArgs a, int rows, int max_tokens, hipStream_t stream) {
     const int chunks = (max_tokens + C - 1) / C;
     for (a.c0 = 0; a.c0 < chunks; a.c0 += a.seg) {
         operators<<<dim3(min(a.seg, chunks - a.c0), a.H, rows), 256, lds, stream>>>(a);
-        chunk_states_kernel<DK, DV, DELTA><<<dim3(a.H, DV / 16, rows), DK * 4 / state_tiles(DK, DELTA), 0, stream>>>(a);     // a head on one XCD: its blocks read the same operators
+        // a head on one XCD: its blocks read the same operators.  Four chunks under way, of heads of 128 two, and three of a single row in the decay form,
+        // us, two / three: 24 heads, 2,048 tokens 195 / 182 (190 with loads that the compiled loop waited for), 300 51.6 / 50.2; rows of 200, two 59.7 / 65.2, three 70 / 77
+        auto states = chunk_states_kernel<DK, DV, DELTA, DK <= 64 ? 4 : 2>;
+        if constexpr (DK > 64 && !DELTA) if (rows == 1) states = chunk_states_kernel<DK, DV, DELTA, 3>;
+        states<<<dim3(a.H, DV / 16, rows), DK * 4 / state_tiles(DK, DELTA), 0, stream>>>(a);
     }
     return 0;
 }

@@ -1628,6 +1628,21 @@ def test_state_walk_in_chunks_of_keys_without_an_epsilon(ops, monkeypatch, d):
         assert a.isfinite().all() and (a - b).norm() <= 5e-7 * b.norm()
 
 
+@pytest.mark.parametrize("n", [32, 64, 65, 96, 128, 150, 192, 1000])
+def test_state_walk_in_chunks_of_a_single_row(ops, monkeypatch, n):
+    """Heads of 128 with fixed decays: three chunks are under way for a single row, two beside another: the same bits, and the walk's to 32-bit rounding."""
+    H, d = 2, 128
+    r, k, v, state, ctx, kw = _scan_step("decay", d, H, [n], [40])
+    (out0, state0), (out1, state1) = _scan_both_ways(ops, monkeypatch, H, d, r, k, v, state, ctx, kw)
+    for a, b in ((out1, out0), (state1, state0)):
+        assert a.isfinite().all() and (a - b).norm() <= 5e-7 * b.norm()
+    _, _, _, _, ctx2, _ = _scan_step("decay", d, H, [n, 33], [40, 0])
+    more = [torch.cat([t, t[:33] if n >= 33 else t.repeat(2, 1)[:33]]) for t in (r, k, v)]
+    both, out2 = torch.cat([state, state]), torch.empty(n + 33, H * d, device=DEV)
+    ops.linear_scan(*more, both, out2, ctx2, H, d, d, **kw)
+    assert torch.equal(out2[:n], out1) and torch.equal(both[:1], state1)
+
+
 @pytest.mark.parametrize("form,d,what,value,at", [
     ("delta", 64, "v", "inf", 705), ("delta", 64, "k", "nan", 40), ("delta", 128, "k", 1e37, 40), ("delta", 64, "r", "-inf", 50), ("delta", 64, "wl", "nan", 45),
     ("delta", 128, "al", "nan", 690), ("delta", 64, "v", "nan", 0), ("decay", 64, "v", "-inf", 44), ("decay", 64, "k", "inf", 700), ("decay", 128, "r", "nan", 63)])
