@@ -563,6 +563,27 @@ def test_linear_with_activated_columns(ops, M, N, K, acts):
     assert torch.isnan(out[:, N:]).all()
 
 
+@pytest.mark.parametrize("M,N,K,acts", [(1, 64, 32, [(0, 64, "relu2")]), (8, 2064, 64, [(16, 2048, "relu2"), (0, 16, "tanh")]), (16, 32800, 64, [(0, 32768, "relu2")]),
+                                        (33, 4112, 2048, [(2048, 2064, "relu2")]), (64, 160, 2048, [(0, 32, "tanh"), (144, 16, "relu2")])])
+def test_activated_columns_are_made_of_unrounded_sums(ops, monkeypatch, M, N, K, acts):
+    """In the product's epilogue, no kernel behind it: one bfloat16 rounding (2^-8 of the value) and 32-bit sums, where rounded sums would be squared with twice
+    that of their own."""
+    def refuse(*a):
+        raise AssertionError("the activation's kernel ran")
+    monkeypatch.setattr(ops, "unary", refuse)
+    x = rnd(M, K, seed=M).to(torch.bfloat16)
+    w = (rnd(N, K, seed=N) * 0.2).to(torch.bfloat16)
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    bufs = [torch.empty(M, n, dtype=torch.bfloat16, device=DEV) for _, n, _ in acts]
+    ops.linear_activated(x, w, out, ops.tile_weight(w), [(c0, n, f, b) for (c0, n, f), b in zip(acts, bufs)])
+    ref = x.double() @ w.double().t()
+    size = x.double().abs() @ w.double().abs().t()                 # of the sums' terms: 32-bit rounding of a sum is under 2^-18 of it
+    for (c0, n, f), b in zip(acts, bufs):
+        z, e = ref[:, c0:c0 + n], size[:, c0:c0 + n] * 2.0 ** -18
+        want, slope = (torch.relu(z).square(), 2 * torch.relu(z) + e) if f == "relu2" else (torch.tanh(z), torch.ones_like(z))
+        assert torch.all((b.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1.01 * slope * e + 1e-30)
+
+
 @pytest.mark.parametrize("T,n,group,pad", [(1, 8, 8, 0), (3, 2048, 2048, 0), (5, 2304, 256, 8), (2, 3072, 1024, 16), (7, 1024, 512, 0), (4, 4096, 2048, 8), (3, 192, 64, 4),
                                            (2, 72, 24, 0), (2, 4096, 4096, 0), (300, 128, 16, 8),
                                            (2, 1024, 1024, 0), (3, 1536, 512, 8), (2, 512, 512, 0), (5, 1536, 256, 0), (128, 2048, 64, 0), (127, 2048, 64, 8),
@@ -1293,6 +1314,51 @@ def test_exact_attention_of_a_portion_does_not_depend_on_the_cut(ops, H, Hkv, hd
         for g in range(Hkv):
             assert torch.allclose(o[n - 1, g * G * hd:(g * G + 1) * hd], vc[blk, g, :, far % page], atol=1e-4), far
         kc[blk, :, far % page] = saved
+
+
+@pytest.mark.parametrize("hd", [20, 64, 128])
+@pytest.mark.parametrize("size,scale", [(1.0, 2.0 ** 40), (2.0 ** -67, 2.0 ** 126)])
+@pytest.mark.parametrize("single", [True, False])
+def test_exact_attention_sums_are_a_chain_of_fused_multiply_adds(ops, hd, size, scale, single):
+    """Bit for bit, products and sums below the smallest normal number kept.  Scores: of two keys one is random and the other scores what libm's fmaf gives
+    for the first; at this scale half a unit between them moves the weights from one half each.  Weighted values: 50 keys of one score, whose weights are
+    one, so the sum is the values' in ascending order, rounded at each."""
+    fmaf = ctypes.CDLL("libm.so.6").fmaf
+    fmaf.restype, fmaf.argtypes = ctypes.c_float, [ctypes.c_float] * 3
+    H, page, n = 6, 16, 50
+    g = torch.Generator().manual_seed(hd)
+    q, k, v = torch.randn(H, hd, generator=g) * size, torch.randn(H, hd, generator=g) * size, torch.randn(H, n, hd, generator=g) * (1.0 if size == 1.0 else 2.0 ** -130)
+    q[:, 0] = size
+    want = torch.zeros(H)
+    for h in range(H):
+        s = 0.0
+        for a, b in zip(q[h].tolist(), k[h].tolist()):
+            s = fmaf(a, b, s)
+        want[h] = s
+    assert size == 1.0 or (want.abs() < 2.0 ** -126).any()
+    total = torch.zeros(H, hd)
+    for j in range(n):
+        total = total + v[:, j]                      # 32-bit additions on the host
+    kc, vc = torch.full((8, H, page, hd), float("nan"), device=DEV), torch.full((8, H, hd, page), float("nan"), device=DEV)
+    kc[0, :, 0], kc[0, :, 1] = k.to(DEV), torch.cat([(want / size)[:, None], torch.zeros(H, hd - 1)], 1).to(DEV)     # (size is a power of two: exact)
+    vc[0, :, :, 0], vc[0, :, :, 1] = 1.0, 0.0
+    pages = torch.tensor([1, 2, 3, 4])
+    for j in range(n):
+        kc[int(pages[j // page]), :, j % page] = 0.0
+        vc[int(pages[j // page]), :, :, j % page] = v[:, j].to(DEV)
+    i32 = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    # two rows: the two keys, and the 50; as single tokens, or each behind a token of a portion whose output nobody looks at
+    rows, positions, first = ([0, 1], [1, n - 1], [1, n - 1]) if single else ([0, 0, 1, 1], [0, 1, n - 2, n - 1], [0, n - 2])
+    ctx = SimpleNamespace(num_tokens=len(rows), num_rows=2, positions=i32(positions), row_of_token=i32(rows), kv_lens=i32([2, n]), q_start=i32(first),
+                          cu_q=i32([0, 1, 2] if single else [0, 2, 4]), max_q_len=1 if single else 2, max_kv_len=n, decode_only=single, workspace=Workspace(DEV))
+    table = i32([[0] * 4, [1, 2, 3, 4]])
+    qkv = torch.zeros(len(rows), H * hd, device=DEV)
+    at = [0, 1] if single else [1, 3]
+    qkv[at[0]] = q.view(-1).to(DEV)
+    out = torch.empty(len(rows), H * hd, device=DEV)
+    ops.paged_attention(qkv, out, H, H, hd, kc, vc, table, page, ctx, scale, 0)
+    assert torch.all(out[at[0]] == 0.5)
+    assert torch.equal(out[at[1]].cpu().view(H, hd), total / n)
 
 
 @pytest.mark.parametrize("H,Hkv,hd,page,window", [(8, 2, 64, 16, 0), (4, 4, 128, 4, 40)])
