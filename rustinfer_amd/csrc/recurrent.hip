@@ -745,7 +745,7 @@ extern "C" int ri_gated_group_norm(const float* o, int o_stride, int T, int n, i
     const int per = dtype == RI_F32 ? 4 : 8;
     const bool x8 = group_norm_x8_pays(T, n, group, dtype) && group >= 8 && group <= 2048 && (group & (group - 1)) == 0 && o_stride % 4 == 0 && out_stride % per == 0
                     && (!gate || gate_stride % per == 0) && (((uintptr_t)o | (uintptr_t)out | (uintptr_t)gate | (uintptr_t)w) & 15) == 0;
-    const int threads8 = min((n / 8 + 63) / 64 * 64, 256);
+    const int threads8 = max(64, min((n / 8 + 63) / 64 * 64, 256));
     const dim3 grid8(T, (n / 8 + threads8 - 1) / threads8);
 #define RI_GGN(TT, TW) do { \
         if (x8) gated_group_norm_x8_kernel<TT, TW><<<grid8, threads8, 0, stream>>>(o, o_stride, n, group, (const TW*)w, (const TT*)gate, gate_stride, (TT*)out, out_stride, eps, gate_silu, gate_first); \

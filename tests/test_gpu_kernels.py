@@ -587,7 +587,7 @@ def test_activated_columns_are_made_of_unrounded_sums(ops, monkeypatch, M, N, K,
 @pytest.mark.parametrize("T,n,group,pad", [(1, 8, 8, 0), (3, 2048, 2048, 0), (5, 2304, 256, 8), (2, 3072, 1024, 16), (7, 1024, 512, 0), (4, 4096, 2048, 8), (3, 192, 64, 4),
                                            (2, 72, 24, 0), (2, 4096, 4096, 0), (300, 128, 16, 8),
                                            (2, 1024, 1024, 0), (3, 1536, 512, 8), (2, 512, 512, 0), (5, 1536, 256, 0), (128, 2048, 64, 0), (127, 2048, 64, 8),
-                                           (1030, 256, 32, 0), (9, 256, 128, 0), (9, 128, 128, 0), (1100, 64, 16, 0)])
+                                           (1030, 256, 32, 0), (9, 256, 128, 0), (9, 128, 128, 0), (1100, 64, 16, 0), (2, 4, 4, 0), (3, 6, 2, 2)])
 @pytest.mark.parametrize("dtype,w_dtype", [(torch.bfloat16, torch.float32), (torch.bfloat16, torch.bfloat16), (torch.float32, torch.float32)])
 def test_gated_group_norm_of_eight_values_a_thread(ops, T, n, group, pad, dtype, w_dtype):
     # groups in a few lanes, a wave, two and four waves; rows that end inside a block; and what the other kernel keeps (strides, sizes)
