@@ -653,7 +653,8 @@ static int decode_chunk(int T, int Hkv, int hd, int max_kv_len) {
 }
 
 extern "C" size_t ri_attention_decode_workspace(int rows, int H, int hd, int max_kv_len) {
-    const size_t splits = (size_t)std::max(list_slots(max_kv_len), (max_kv_len + 63) / 64);       // of the list's form, and of the others
+    const int blocks = (max_kv_len + 63) / 64;                  // no form of blocks a row leaves more; the list is head 128's
+    const size_t splits = (size_t)(hd == 128 ? std::max(list_slots(max_kv_len), blocks) : blocks);
     return ((size_t)rows * H * splits * (hd + 2) + rows) * sizeof(float);
 }
 
