@@ -621,11 +621,45 @@ def swiglu(gate_up: torch.Tensor, out: torch.Tensor) -> None:
     _check(_lib().ri_swiglu(_ptr(gate_up), _ptr(out), _dt(out), T, I, _stream()))
 
 
-def tile_weight(w: torch.Tensor) -> Optional[torch.Tensor]:
-    """A copy of ``w[N, K]`` in the order the weight-streaming kernel reads it:
-    ``[N/16][K/32][64 lanes][8]`` with lane ``g * 16 + r`` holding ``w[16 nt + r, 32 ks + 8 g : +8]``.
-    None if the shape has no such form (N % 16 or K % 32) or the dtype is not bfloat16."""
+class DigitWeight:
+    """A 32-bit weight as whole numbers of five 8-bit digits and an exponent a row (csrc/gemm_digits.hip)."""
+
+    def __init__(self, w: torch.Tensor):
+        N, K = w.shape
+        lib = _lib()
+        lib.ri_digits_bytes.restype = ctypes.c_longlong
+        self.shape, self.device = (N, K), w.device
+        self.planes = torch.empty(int(lib.ri_digits_bytes(N, K)), dtype=torch.uint8, device=w.device)
+        self.exps = torch.empty(N, dtype=torch.int32, device=w.device)
+        _check(lib.ri_digits_split(_ptr(w), w.stride(0), N, K, 0, _ptr(self.planes), _ptr(self.exps), _stream()))
+        self.whole = not bool((self.exps == NO_DIGITS).any())       # every row has digits
+
+
+NO_DIGITS = -(1 << 31)              # in the place of a row's exponent: not finite, or values that spread too far
+DIGITS_MIN_WEIGHTS = 1 << 19        # smaller weights never pay for digits (ri_gemm_digits_plan)
+
+
+def _digits_shape(w: torch.Tensor) -> bool:
     N, K = w.shape
+    return (w.dtype == torch.float32 and w.is_cuda and N % 32 == 0 and K % 32 == 0 and 256 <= K <= _lib().ri_digits_max_k()
+            and N * K >= DIGITS_MIN_WEIGHTS and N <= 1 << 22 and w.stride(1) == 1 and w.stride(0) % 4 == 0 and w.data_ptr() % 16 == 0)
+
+
+def tiled_bytes(w: torch.Tensor) -> int:
+    """Bytes that ``tile_weight(w)`` takes, if there is such a copy."""
+    N, K = w.shape
+    return N * K * 5 + 4 * N if w.dtype == torch.float32 else w.numel() * w.element_size()
+
+
+def tile_weight(w: torch.Tensor):
+    """A copy of ``w[N, K]`` in the order the weight-streaming kernel reads it:
+    ``[N/16][K/32][64 lanes][8]`` with lane ``g * 16 + r`` holding ``w[16 nt + r, 32 ks + 8 g : +8]``;
+    of a float32 weight its digits, a ``DigitWeight``.  None if the shape has no such form (bfloat16: N % 16 or
+    K % 32; float32: N % 32, K % 32, too small, or a row that has no digits)."""
+    N, K = w.shape
+    if w.dtype == torch.float32 and _digits_shape(w):
+        d = DigitWeight(w)
+        return d if d.whole else None
     if w.dtype != torch.bfloat16 or N % 16 or K % 32:
         return None
     return w.view(N // 16, 16, K // 32, 4, 8).permute(0, 2, 3, 1, 4).contiguous().view(N, K)
@@ -744,10 +778,34 @@ def gemm_tuned_shapes() -> int:
     return int(_lib().ri_gemm_library_tuned_shapes())
 
 
-def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: Optional[torch.Tensor] = None,
-           scale=None) -> None:
+def _digits_parts(x: torch.Tensor, w: torch.Tensor, w_tiled, M: int, N: int, K: int) -> int:
+    """Slices of K in which the product goes through digits, 0 if it does not."""
+    if not isinstance(w_tiled, DigitWeight) or x.dtype != torch.float32 or x.stride(0) % 4 or x.data_ptr() % 16:
+        return 0
+    if w_tiled.shape != (N, K) or w.dtype != torch.float32 or w_tiled.device != w.device:
+        raise KernelError("the weight's digits do not belong to the weight")
+    return int(_lib().ri_gemm_digits_plan(M, N, K))
+
+
+def _linear_digits(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: DigitWeight, workspace, parts: int, gate: int = 0) -> None:
+    """``out[M, N]`` from the digits of ``x[:, :K]``, with ``gate`` of ``silu(x[:, :K]) * x[:, gate : gate + K]``."""
+    lib = _lib()
+    M, (N, K) = x.shape[0], w_tiled.shape
+    rows = (M + 31) // 32 * 32
+    planes = workspace.get("digits.planes", rows, 5 * K, torch.uint8)
+    exps = workspace.get("digits.exps", rows, 1, torch.int32)
+    sums = workspace.get("digits.sums", parts * M, N, torch.int64) if parts > 1 else None
+    _check(lib.ri_digits_split(_ptr(x), x.stride(0), M, K, gate, _ptr(planes), _ptr(exps), _stream()))
+    _check(lib.ri_gemm_digits(_ptr(planes), _ptr(exps), _ptr(x), x.stride(0), gate, _ptr(w_tiled.planes), _ptr(w_tiled.exps),
+                              _ptr(w), w.stride(0), _ptr(out), out.stride(0), _ptr(sums) if parts > 1 else ctypes.c_void_p(0), parts,
+                              M, N, K, _stream()))
+
+
+def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled=None,
+           scale=None, workspace=None) -> None:
     """``out[M, N] = x[M, K] @ w[N, K]^T``; ``out`` may be float32 for bfloat16 operands.
-    ``w_tiled`` (from ``tile_weight``) is read instead of ``w`` where the kernel has a use for it.
+    ``w_tiled`` (from ``tile_weight``) is read instead of ``w`` where the kernel has a use for it (the digits of a float32
+    weight: with a ``workspace`` to hold those of ``x``).
     ``scale = (ssq [M, P], eps)``: the rows of ``x`` are ``(r * w_norm)`` of a norm this product
     finishes: row m of the result is multiplied by ``rsqrt(sum(ssq[m]) / K + eps)`` (few bfloat16
     rows only)."""
@@ -801,6 +859,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: Optiona
                                                    M, N, K, _dt(out), 0, 1, ctypes.c_longlong(0), 0,
                                                    ctypes.c_void_p(0), 0, ctypes.c_float(0.0), _stream()))
                     return
+    if workspace is not None and out.dtype == torch.float32:
+        parts = _digits_parts(x, w, w_tiled, M, N, K)
+        if parts:
+            _linear_digits(x, w, out, w_tiled, workspace, parts)
+            return
     if x.dtype == torch.float32 and out.dtype == torch.float32 and K % 4 == 0 and x.stride(0) % 4 == 0 \
             and w.stride(0) % 4 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0:
         # the exact path: 64-bit sums, on the 64-bit matrix instruction or, for up to four rows of long ones, in FMAs
@@ -810,7 +873,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: Optiona
                              M, N, K, _dt(x), _dt(out), _stream()))
 
 
-def linear_activated(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: Optional[torch.Tensor], acts) -> None:
+def linear_activated(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled, acts, workspace=None) -> None:
     """``linear``, and for each ``(c0, n, name, dst)`` of ``acts``: ``dst [M, n] = f(out[:, c0:c0 + n])`` for ``f`` in
     ``UNARY``; ``dst`` may be those columns of ``out`` (columns whose ``dst`` is another buffer need not be
     left in ``out``).  Few bfloat16 rows: in the product's own epilogue, on sums that have not been rounded."""
@@ -834,13 +897,13 @@ def linear_activated(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tile
             ints([a[0] + a[1] for a in acts]), ints([UNARY[a[2]] for a in acts]), (ctypes.c_void_p * len(acts))(*[a[3].data_ptr() for a in acts]),
             ints([a[3].stride(0) for a in acts]), _stream()))
         return
-    linear(x, w, out, w_tiled)
+    linear(x, w, out, w_tiled, workspace=workspace)
     for c0, n, name, dst in acts:
         unary(name, out[:, c0:c0 + n], dst)
 
 
 def linear_delta(x: torch.Tensor, w: torch.Tensor, workspace, name: str,
-                 w_tiled: Optional[torch.Tensor] = None, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
+                 w_tiled=None, out_dtype: Optional[torch.dtype] = None) -> torch.Tensor:
     """``x @ w^T`` as a residual delta for ``add_rmsnorm``: ``[M, N]`` in the dtype of ``x``, or,
     for few bfloat16 rows and few output columns, a float32 stack ``[P, M, N]`` of partial sums
     over slices of K (so that the product still fills the chip) which the norm adds up."""
@@ -880,13 +943,13 @@ def linear_delta(x: torch.Tensor, w: torch.Tensor, workspace, name: str,
                                    ctypes.c_longlong(M * N), _stream()))
             return stack
     out = workspace.get(name, M, N, out_dtype or x.dtype)     # out_dtype: 32-bit sums of a bfloat16 product left unrounded
-    linear(x, w, out, w_tiled)
+    linear(x, w, out, w_tiled, workspace=workspace)
     return out
 
 
 def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor,
-                  scratch: Optional[torch.Tensor] = None, w_tiled: Optional[torch.Tensor] = None,
-                  scale=None) -> None:
+                  scratch: Optional[torch.Tensor] = None, w_tiled=None,
+                  scale=None, workspace=None) -> None:
     """``out[M, I] = silu(x @ gate^T) * (x @ up^T)`` with ``w_gate_up = [gate; up]`` stacked
     ``[2I, K]``.  Few bfloat16 rows: one fused kernel; otherwise the product into ``scratch``
     ``[M, 2I]`` and the activation kernel.  ``scale``: see ``linear``."""
@@ -930,8 +993,26 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor,
         # the exact path's few rows: the activation in the product's epilogue, on the rounded sums (the activation's kernel takes whole buffers only)
         _check(_lib().ri_gemm_f32_swiglu(_ptr(x), x.stride(0), _ptr(w_gate_up), w_gate_up.stride(0), _ptr(out), out.stride(0), M, I, K, _stream()))
         return
-    linear(x, w_gate_up, scratch)
+    linear(x, w_gate_up, scratch, w_tiled if isinstance(w_tiled, DigitWeight) else None, workspace=workspace)
     swiglu(scratch, out)
+
+
+def linear_swiglu_delta(x: torch.Tensor, w_gate_up: torch.Tensor, gate_up_tiled, w_down: torch.Tensor, down_tiled, scratch: torch.Tensor,
+                        workspace, name: str) -> Optional[torch.Tensor]:
+    """``(silu(x @ gate^T) * (x @ up^T)) @ down^T`` of a float32 portion whose products go through digits: the activation is
+    computed where the second product's digits are made.  ``scratch [M, 2I]``.  None, and nothing done, where they do not."""
+    M, K = x.shape
+    D, I = w_down.shape
+    if x.dtype != torch.float32 or w_gate_up.shape != (2 * I, K) or tuple(scratch.shape) != (M, 2 * I) or not scratch.is_contiguous():
+        return None
+    parts = _digits_parts(scratch, w_down, down_tiled, M, D, I)
+    if not parts:
+        return None
+    _dev(x, w_gate_up, w_down, scratch)
+    linear(x, w_gate_up, scratch, gate_up_tiled, workspace=workspace)
+    out = workspace.get(name, M, D, torch.float32)
+    _linear_digits(scratch, w_down, out, down_tiled, workspace, parts, gate=I)
+    return out
 
 
 def argmax(logits: torch.Tensor, out: torch.Tensor) -> None:

@@ -112,7 +112,7 @@ class PagedAttention(Mixer):
                 scale is None and split is not None
                 and ops.qkv_split_pays(rows.shape[0], self.qkv_fused.shape[0], self.qkv_fused.shape[1]) and split(*args, ws))
         if not fused:
-            self.qkv.forward(rows, qkv, scale)
+            self.qkv.forward(rows, qkv, scale, workspace=ws)
             if self.qk_transform is not None:
                 self.qk_transform(ctx, qkv, self)
             ops.rope_kv_write(qkv, self.num_heads, self.num_kv_heads, self.head_dim, rotary,

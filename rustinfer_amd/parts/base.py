@@ -226,7 +226,8 @@ class Runtime:
     dtype: torch.dtype            # torch.bfloat16 (serving) or torch.float32 (exact path)
     ops: Any                      # the kernel module (rustinfer_amd.kernels.ops)
     # A second copy of every projection weight in the order the few-row kernels stream it (and a
-    # third, row-permuted one of the q/k/v weight for the fused projection).  False: one copy, as
+    # third, row-permuted one of the q/k/v weight for the fused projection; of a 32-bit weight its
+    # digits, five bytes a value, for the products of prompts).  False: one copy, as
     # the checkpoint has it; single-token steps then read row-major weights, more slowly, and the
     # weights take half the memory.
     tiled_weight_copy: bool = True
@@ -259,11 +260,13 @@ class Runtime:
         make = getattr(self.ops, "tile_weight", None)
         if make is None or not self.tiled_weight_copy:
             return None
-        if not self.take_tile_budget(w.numel() * w.element_size()):
+        size = getattr(self.ops, "tiled_bytes", None)
+        nbytes = size(w) if size is not None else w.numel() * w.element_size()
+        if not self.take_tile_budget(nbytes):
             return None
         t = make(w)
         if t is None:
-            self.give_tile_budget_back(w.numel() * w.element_size())
+            self.give_tile_budget_back(nbytes)
         return t
 
 
@@ -484,9 +487,9 @@ class ProjectionSet:
                 c0, rows = self.in_slices[i][name]
                 acts.append((c0, rows, f, self.act_view(i, act) if into_act else proj[:, c0:c0 + rows]))
         if acts:
-            self.rt.ops.linear_activated(normed, self.w_in.weight, proj, self.w_in.weight_tiled, acts)
+            self.rt.ops.linear_activated(normed, self.w_in.weight, proj, self.w_in.weight_tiled, acts, workspace=ctx.workspace)
         else:
-            self.w_in.forward(normed, proj)
+            self.w_in.forward(normed, proj, workspace=ctx.workspace)
         for a, b in self._gaps:                          # scratch may hold anything, and 0 * NaN is NaN
             act[:, a:b].zero_()
         return proj, act

@@ -78,7 +78,7 @@ class LMHead(Part):
     def forward(self, ctx, normed, logits: torch.Tensor) -> torch.Tensor:
         rows, scale = split_normed(normed)
         if scale is None:
-            self.rt.ops.linear(rows, self.weight, logits, self.weight_tiled)
+            self.rt.ops.linear(rows, self.weight, logits, self.weight_tiled, workspace=getattr(ctx, "workspace", None))
         else:
             self.rt.ops.linear(rows, self.weight, logits, self.weight_tiled, scale=scale)
         if self.logit_scale != 1.0 or self.softcap > 0.0:

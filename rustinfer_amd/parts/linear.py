@@ -24,10 +24,11 @@ class Linear:
         # a second copy in the order the few-row kernel streams it (memory is plentiful, bandwidth is not)
         self.weight_tiled = rt.tile(self.weight) if tile else None
 
-    def forward(self, x: torch.Tensor, out: torch.Tensor, scale=None) -> torch.Tensor:
-        """``scale``: the row factors of a norm this product finishes (``DeferredNorm.scale``)."""
+    def forward(self, x: torch.Tensor, out: torch.Tensor, scale=None, workspace=None) -> torch.Tensor:
+        """``scale``: the row factors of a norm this product finishes (``DeferredNorm.scale``).  ``workspace``: scratch for
+        the forms that need some."""
         if scale is None:
-            self.rt.ops.linear(x, self.weight, out, self.weight_tiled)
+            self.rt.ops.linear(x, self.weight, out, self.weight_tiled, workspace=workspace)
         else:
             self.rt.ops.linear(x, self.weight, out, self.weight_tiled, scale=scale)
         return out

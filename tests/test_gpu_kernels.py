@@ -504,6 +504,118 @@ def test_swiglu_f32_of_up_to_eight_rows_is_the_product_and_the_activation(ops, M
     assert torch.equal(out[:, :I], want) and torch.isnan(out[:, I:]).all()
 
 
+# Digits (gemm_digits): each value of a row is within 2^-40 of the row's largest a (half a unit of 40 bits, of which one may
+# be lost to the first digit's range), so K (2^-40 a |w| + 2^-40 w |a|); the products left out, four of digits 0 to 3 with i + j = 3 and what is
+# below them, are at most 4.02 x 2^14 x 256^3 units of 2^-78 (a w times at most 4.1): under 2^-36 K a w.  Signs of both are random: a 64th of the sum of bounds.
+def _digits_bound(x, w):
+    a, b = x.double().abs(), w.double().abs()
+    K = x.shape[1]
+    am, bm = a.amax(1, keepdim=True), b.amax(1)[None]
+    return 2.0 ** -40 * (am * b.sum(1)[None] + bm * a.sum(1, keepdim=True)) + 2.0 ** -36 * K * am * bm
+
+
+@pytest.mark.parametrize("M,N,K", [(24, 1024, 1024), (33, 3072, 2048), (64, 2080, 4096), (65, 4128, 1056), (129, 544, 9120), (100, 992, 14336), (300, 2048, 25984), (193, 8192, 288)])
+def test_linear_f32_from_digits(ops, M, N, K):
+    """Edges of tiles and of the slices of K, a last block of fewer than four tiles of columns, rows inside a wider buffer; exponents from the
+    least to the largest, rows of zeros; a row's bits are the same alone with others, whatever the slices."""
+    from rustinfer_amd.engine.context import Workspace
+    xb = rnd(M, K + 8, seed=M)
+    x, w = xb[:, 4:K + 4], rnd(N, K, seed=N) * 0.02
+    x[3] = 0
+    x[5] *= 1e-38                                        # some of them below the normal numbers
+    x[7] *= 1e34
+    w[9] *= 2.0 ** -100
+    x[11] = x[11].abs().clamp(min=0.5)                   # first digits near their ends
+    x[11, 1] = -(2.0 - 2.0 ** -23)
+    wt = ops.tile_weight(w)
+    assert wt is not None and wt.whole
+    ws = Workspace(torch.device(DEV))
+    parts = ops._digits_parts(x, w, wt, M, N, K) or 1
+    ref = x.double() @ w.double().t()
+    outs = []
+    for p in {1, 2, parts}:
+        out = torch.full((M, N + 3), float("nan"), device=DEV)
+        ops._linear_digits(x, w, out[:, :N], wt, ws, p)
+        assert torch.isnan(out[:, N:]).all()
+        outs.append(out[:, :N])
+        assert torch.equal(outs[-1], outs[0])
+    few = torch.empty(M - 20, N, device=DEV)
+    ops._linear_digits(x[20:].contiguous(), w, few, wt, ws, 1)
+    assert torch.equal(few, outs[0][20:])
+    # rounded once: half a unit of the last place, of the least of them for results below the normal numbers
+    err = (outs[0].double() - ref).abs()
+    assert torch.all(err <= ref.abs() * 2.0 ** -24 + 2.0 ** -150 + _digits_bound(x, w))
+    rows = [i for i in range(M) if i not in (3, 5)]
+    plain = torch.empty(M, N, device=DEV)
+    ops.linear(x, w, plain)
+    e = lambda y: ((y[rows].double() - ref[rows]) / ref[rows].norm(dim=1, keepdim=True)).norm().item()
+    assert e(outs[0]) <= 1.0005 * e(plain)               # no further from 64 bits than 64-bit sums are
+
+
+def test_linear_f32_rows_without_digits(ops):
+    """Rows that hold an infinity or a NaN, and rows whose values spread over more than the digits hold, go by 64-bit sums, in whole products
+    and in slices; the other rows keep their bits."""
+    from rustinfer_amd.engine.context import Workspace
+    M, N, K = 100, 2080, 2048
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
+    wt, ws = ops.tile_weight(w), Workspace(torch.device(DEV))
+    clean = torch.empty(M, N, device=DEV)
+    ops._linear_digits(x, w, clean, wt, ws, 1)
+    y = x.clone()
+    y[2, 7], y[40, 0], y[40, 1], y[99, K - 1] = float("inf"), float("nan"), 1.0, -float("inf")
+    spread = [0, 33, 64]
+    g = torch.Generator().manual_seed(3)
+    y[spread] = (torch.randn(3, K, generator=g) * 2.0 ** torch.randint(-60, 61, (3, K), generator=g)).to(DEV)
+    ref = y.double() @ w.double().t()
+    for parts in (1, 4):
+        out = torch.full((M, N), float("nan"), device=DEV)
+        ops._linear_digits(y, w, out, wt, ws, parts)
+        special = [2, 40, 99] + spread
+        rest = [i for i in range(M) if i not in special]
+        assert torch.equal(out[rest], clean[rest])
+        assert torch.isnan(out[40]).all() and torch.equal(out[[2, 99]], ref[[2, 99]].float())
+        mag = y[spread].double().abs() @ w.double().abs().t()
+        assert torch.all((out[spread].double() - ref[spread]).abs() <= ref[spread].abs() * 2.0 ** -24 + K * 2.0 ** -52 * mag)
+    w2 = w.clone()
+    w2[70, 3] = float("inf")
+    assert ops.tile_weight(w2) is None and ops.tile_weight(w[:, :2046]) is None and ops.tile_weight(w[:2047]) is None
+
+
+@pytest.mark.parametrize("M,I,K", [(40, 1024, 2048), (130, 8192, 1024), (64, 2720, 1056), (33, 14336, 512)])
+def test_swiglu_mlp_f32_from_digits(ops, M, I, K):
+    """The activation where the second product's digits are made: no further from 64 bits than the activation's own kernel, in whole products
+    and slices the same bits; a row that is not finite, one whose activation passes the 32-bit range, and one by 64-bit sums."""
+    from rustinfer_amd.engine.context import Workspace
+    D = 1024
+    x, wgu, wd = rnd(M, K, seed=1), rnd(2 * I, K, seed=2) * 0.05, rnd(D, I, seed=3) * 0.02
+    tgu, td, ws = ops.tile_weight(wgu), ops.tile_weight(wd), Workspace(torch.device(DEV))
+    scratch, act, old = torch.empty(M, 2 * I, device=DEV), torch.empty(M, I, device=DEV), torch.empty(M, D, device=DEV)
+    ops.linear(x, wgu, scratch, tgu, workspace=ws)
+    scratch[1, 5] = float("nan")
+    scratch[2, 7], scratch[2, I + 7] = 1e20, 1e20
+    g = torch.Generator().manual_seed(3)
+    scratch[3, I:] = (torch.randn(I, generator=g) * 2.0 ** torch.randint(-60, 61, (I,), generator=g)).to(DEV)
+    ops.swiglu(scratch, act)
+    ops._linear_digits(act, wd, old, td, ws, 1)
+    z = scratch.double()
+    ref = (torch.nn.functional.silu(z[:, :I]) * z[:, I:]) @ wd.double().t()
+    outs = []
+    for parts in (1, 3):
+        outs.append(torch.full((M, D), float("nan"), device=DEV))
+        ops._linear_digits(scratch, wd, outs[-1], td, ws, parts, gate=I)
+    got = outs[0]
+    assert torch.equal(torch.nan_to_num(got, nan=7.0), torch.nan_to_num(outs[1], nan=7.0))
+    assert torch.isnan(got[1]).all() and torch.isinf(got[2]).all() and torch.equal(got[2], old[2])
+    rows = [i for i in range(M) if i not in (1, 2)]
+    e = lambda y: (y[rows].double() - ref[rows]).norm(dim=1) / ref[rows].norm(dim=1)
+    assert torch.all(e(got) <= e(old) * 1.05) and torch.all(e(got) <= 2.0 ** -23)
+    scratch[:] = float("nan")
+    both = ops.linear_swiglu_delta(x, wgu, tgu, wd, td, scratch, ws, "d")
+    assert (both is None) == (ops._digits_parts(scratch, wd, td, M, D, I) == 0)
+    if both is not None:
+        assert torch.equal(both[4:], got[4:])
+
+
 @pytest.mark.parametrize("M", [3, 20])
 def test_linear_f32_of_rows_further_apart_than_32_bit_distances_reach(ops, M):
     far, K = (1 << 24) + 4, 12                          # 48 rows of such a distance: over 3 GiB
