@@ -558,6 +558,85 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_bf16_kernel(
     }
 }
 
+// The product before a norm (RESID above) of up to eight rows: a tile of the instruction holds eight columns of W and the rows twice, for two steps of K:
+// lanes of columns 0 to 7 read step s of a block's eight columns, lanes of columns 8 to 15 step s + 1 (of the rows alike), so the tile's upper left quarter
+// is the sum of the even steps and its lower right that of the odd ones.  A product of 2,048 columns so has a block for every compute unit with whole
+// loads, where half a tile a block (`halves`) leaves half of each load's lanes idle.  Loads by offsets from descriptors that end with the block's weights and with
+// the last row: what lies beyond is zero and is not fetched, so that no load stands under a lane's condition; the first batch goes out before anything is
+// waited for.  What bounds it is the one pass over W, whose loads in flight come from sixteen waves a block: measured, us, 16 columns a block (8 with
+// idle lanes up to 2,048) / this, and a kernel that only reads as much, 1 and 8 rows: 2048 x 2048 4.8 5.4 / 4.0 4.5 (2.8), 2048 x 8192 10.5 11.3 / 8.1 9.3
+// (6.5), 1536 x 8960 10.8 12.0 / 7.8 9.7 (5.6), 5120 x 8192 21.3 24.4 / 16.6 21.0 (13.8); 1 and 4 rows: 4096 x 4096 8.9 9.0 / 7.7 8.1 (6.5), 4096 x 14336 22.8
+// 23.1 / 20.9 22.5 (18.6), 3072 x 8192 12.7 12.9 / 11.2 12.5 (8.9).  Eight waves: 8.3 and 10.0 for 2048 x 8192.
+template <int U, int WAVES>
+__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_pairs_kernel(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
+                                                                       int M, int N, int K, ResidualEpilogue re) {
+    __shared__ float red[WAVES][64];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 7, second = (lane >> 3) & 1, g = lane >> 4;
+    const int steps = K / 32;
+    const __amdgpu_buffer_rsrc_t wd = __builtin_amdgcn_make_buffer_rsrc((void*)(W + (size_t)(blockIdx.x >> 1) * steps * 512), 0, steps * 1024, 0x00020000);
+    const __amdgpu_buffer_rsrc_t xd = __builtin_amdgcn_make_buffer_rsrc((void*)A, 0, (int)(((size_t)(M - 1) * lda + K) * 2), 0x00020000);
+    constexpr uint32_t OUT = 0x7ffffff0u;                    // beyond any descriptor
+    const uint32_t wat = (uint32_t)(g * 256 + ((int)blockIdx.x & 1) * 128 + r * 16 + second * 1024);
+    const uint32_t xat = r < M ? (uint32_t)(r * lda + g * 8 + second * 32) * 2 : OUT;
+    gbf16x8_t wf[U], xf[U];
+    auto ask = [&](int s0) {
+        if (s0 + (U - 1) * WAVES * 2 + 2 <= steps) {         // a whole batch: nothing to compute in the lanes
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                wf[u] = __builtin_bit_cast(gbf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(wd, wat, (s0 + u * WAVES * 2) * 1024, 2));
+#pragma unroll
+            for (int u = 0; u < U; ++u)
+                xf[u] = __builtin_bit_cast(gbf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(xd, xat, (s0 + u * WAVES * 2) * 64, 0));
+            return;
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t s = (uint32_t)(s0 + u * WAVES * 2);
+            const bool in = (int)s + second < steps;
+            wf[u] = __builtin_bit_cast(gbf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(wd, in ? wat + s * 1024 : OUT, 0, 2));
+            xf[u] = __builtin_bit_cast(gbf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(xd, in ? xat + s * 64 : OUT, 0, 0));
+        }
+    };
+    int s0 = wave * 2;
+    if (s0 < steps) ask(s0);
+    __builtin_amdgcn_sched_barrier(0);
+    // the end: a lane a result, row lane / 8 of column lane % 8
+    const int m = lane >> 3, n = (int)blockIdx.x * 8 + (lane & 7);
+    float x = 0.f, w = 0.f;
+    if (wave == 0 && m < M) {
+        x = re.x[(size_t)m * N + n];
+        w = re.w16 ? bf16_to_f32(re.w16[n]) : re.w32[n];
+    }
+    gf32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+    while (s0 < steps) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u], xf[u], acc, 0, 0, 0);
+        s0 += WAVES * 2 * U;
+        if (s0 < steps) ask(s0);
+    }
+    // element i of lane 16 g + c: column 4 g + i of the tile, row c
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float both = acc[i] + __shfl(acc[i], (lane + 40) & 63, 64);
+        if (g < 2 && !second) red[wave][r * 8 + g * 4 + i] = both;
+    }
+    __syncthreads();
+    if (wave != 0) return;
+    float v = red[0][lane];
+#pragma unroll
+    for (int i = 1; i < WAVES; ++i) v += red[i][lane];
+    v += x;
+    float sq = m < M ? v * v : 0.f;
+    if (m < M) {
+        re.x[(size_t)m * N + n] = v;
+        re.a_out[(size_t)m * N + n] = f32_to_bf16(v * w);
+    }
+#pragma unroll
+    for (int o = 1; o < 8; o <<= 1) sq += __shfl_xor(sq, o, 64);
+    if (m < M && (lane & 7) == 0) re.ssq[(size_t)m * gridDim.x + blockIdx.x] = sq;
+}
+
 // Tiles of W a wave owns (NT) and slices of K given to separate blocks (parts).
 //
 // With few rows the activations cost as much as the weights once a wave asks for as many
@@ -801,7 +880,7 @@ extern "C" int ri_gemm_skinny_activated(const void* A, int lda, const void* W, v
 }
 
 // The product before a norm, for M <= 16 rows (see ResidualEpilogue):
-//   x[M, N] += A[M, K] . W[N, K]^T;  a_out[M, N] = x * w_norm (bfloat16);  ssq[M][N / 16] = partial sums of x^2
+//   x[M, N] += A[M, K] . W[N, K]^T;  a_out[M, N] = x * w_norm (bfloat16);  ssq[M][ri_gemm_skinny_residual_parts] = partial sums of x^2
 // W in tile order (N % 16 == 0, K % 32 == 0).  No split over K between blocks: the eight waves of a
 // block share K.  One weight tile a block: with two the activations are asked for half as often, but
 // products of 4,096 columns then leave half the chip idle (measured, 8 rows, us: 4096 x 14336: 25.2
@@ -812,15 +891,25 @@ extern "C" int ri_gemm_skinny_residual_max_rows() { return 16; }
 // at batch 8 of the 1B shape 2 % faster; 3,072 columns: 9 % slower).
 // (with up to four rows half tiles at 4,096 columns too: 7 % of a decode step slower)
 static int residual_halves(int N) { return N / 16 <= 128 ? 1 : 0; }
-// slots of partial sums a row: one for every 16 columns, or for every 8 where blocks own half tiles
-extern "C" int ri_gemm_skinny_residual_parts(int N) { return residual_halves(N) ? N / 8 : N / 16; }
+// Whether a product takes gemm_skinny_pairs: up to eight rows where its blocks of eight columns take fewer rounds of 256 units than blocks of 16 (and
+// always up to 2,048 columns), up to four rows where they take as many and fill three quarters of them or more: the rows are asked for twice as often.
+// Measured, us, 16 columns a block / pairs at 1, 4, 8 rows: 3072 x 3072 6.6 6.8 7.2 / 6.1 6.6 7.5; 3072 x 8192 12.7 12.9 14.0 / 11.2 12.5 14.8; 4096 x 14336
+// 22.8 23.1 24.7 / 20.9 22.5 25.8; 8192 x 8192 25.9 26.7 28.6 / 23.3 24.7 28.8; 2560 x 9728 (320 blocks of pairs) 13.2 13.7 15.5 / 13.3 15.0 18.0.
+static bool residual_pairs(int M, int N) {
+    if (M > 8) return false;
+    const int eights = N / 8, rounds = (eights + 255) / 256, before = (N / 16 + 255) / 256;
+    if (N <= 2048 || rounds < 2 * before) return true;
+    return M <= 4 && eights * 4 >= rounds * 256 * 3;
+}
+// slots of partial sums a row: one for every 16 columns, or for every 8 where blocks own as many
+extern "C" int ri_gemm_skinny_residual_parts(int M, int N) { return residual_halves(N) || residual_pairs(M, N) ? N / 8 : N / 16; }
 
 extern "C" int ri_gemm_skinny_residual(const void* A, int lda, const void* W, int M, int N, int K,
                                        float* x, const void* w_norm, int w_dtype, void* a_out, float* ssq,
                                        hipStream_t stream) {
     RI_REQUIRE(M >= 1 && M <= 16, "ri_gemm_skinny_residual: M=%d not in [1, 16]", M);
     RI_REQUIRE(N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0, "ri_gemm_skinny_residual: needs N %% 16 == 0 and K %% 32 == 0 (N=%d K=%d)", N, K);
-    RI_REQUIRE(lda >= K && lda % 8 == 0, "ri_gemm_skinny_residual: bad leading dimension");
+    RI_REQUIRE(lda >= K && lda % 8 == 0 && lda <= (1 << 27), "ri_gemm_skinny_residual: bad leading dimension");
     RI_REQUIRE(A && W && x && w_norm && a_out && ssq, "ri_gemm_skinny_residual: null pointer");
     RI_REQUIRE(w_dtype == RI_F32 || w_dtype == RI_BF16, "ri_gemm_skinny_residual: the norm's weight must be float32 or bfloat16");
     RI_REQUIRE((uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w_norm % 16 == 0
@@ -831,7 +920,9 @@ extern "C" int ri_gemm_skinny_residual(const void* A, int lda, const void* W, in
     const bf16_t* a = (const bf16_t*)A;
     const bf16_t* w = (const bf16_t*)W;
     const int nks = K / 32, blocks = (N / 16) * (halves ? 2 : 1);
-    if (nks >= 16)
+    if (residual_pairs(M, N) && K <= 2048) gemm_skinny_pairs_kernel<2, 16><<<N / 8, 1024, 0, stream>>>(a, lda, w, M, N, K, re);
+    else if (residual_pairs(M, N)) gemm_skinny_pairs_kernel<4, 16><<<N / 8, 1024, 0, stream>>>(a, lda, w, M, N, K, re);
+    else if (nks >= 16)
         gemm_skinny_bf16_kernel<1, 1, 8, float, false, true><<<dim3(blocks, 1), 512, 0, stream>>>(
             a, lda, w, K, (float*)nullptr, N, M, N, K, nks, 0, RopeEpilogue{}, RowScale{}, re);
     else

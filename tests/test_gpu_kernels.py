@@ -1246,6 +1246,35 @@ def _check_fused_projection(ops, B, H, Hkv, hd, page, K):
         assert np.all(np.abs(got[b, :H * hd].double().cpu().numpy() - want) <= 2.0 ** -8 * np.maximum(1.0, np.abs(want)))
 
 
+@pytest.mark.parametrize("M,N,K", [(1, 16, 32), (8, 48, 96), (3, 2048, 2048), (8, 2048, 2080), (7, 1024, 4128), (4, 3072, 3104), (2, 4096, 1056),
+                                   (8, 5120, 2048), (1, 6144, 8192), (8, 2048, 8224)])
+def test_the_product_before_a_norm_in_pairs_of_steps(ops, M, N, K):
+    """Eight columns a block, two steps of K a load: an odd number of steps, fewer than the waves, whole batches and parts of one; what lies beside the
+    rows in a wider buffer, and a row that is not finite, touch nothing else."""
+    lib = ops._lib()
+    assert lib.ri_gemm_skinny_residual_parts(M, N) == N // 8
+    buf = torch.full((M + 1, K + 64), float("nan"), dtype=torch.bfloat16, device=DEV)
+    act = buf[:M, 32:K + 32]
+    act.copy_(rnd(M, K, dtype=torch.bfloat16, seed=1))
+    w = rnd(N, K, dtype=torch.bfloat16, seed=2, scale=0.05)
+    wt, wn, x0, ws = ops.tile_weight(w), 1.0 + rnd(N, seed=3, scale=0.1), rnd(M, N, seed=4), Workspace(DEV)
+    x = x0.clone()
+    a, ssq = ops.linear_residual(act, w, wt, x, wn, ws, "t")
+    a, ssq = a.clone(), ssq.clone()
+    prod = act.double() @ w.double().t()
+    # sums of K products in 32 bits, of random signs: 8 half units of the root of the sum of squares, and the addition's own
+    mag = ((act.double() ** 2) @ (w.double() ** 2).t()).sqrt()
+    assert torch.all((x.double() - x0.double() - prod).abs() <= 2.0 ** -21 * mag * max(1.0, K / 512) ** 0.5 + 2.0 ** -23 * x.double().abs())
+    assert torch.equal(a, (x * wn).to(torch.bfloat16)) and tuple(ssq.shape) == (M, N // 8)
+    assert torch.allclose(ssq.double(), (x.double() ** 2).view(M, N // 8, 8).sum(2), rtol=1e-6)
+    if M > 1:
+        act[1, K - 1] = float("inf")
+        y = x0.clone()
+        ops.linear_residual(act, w, wt, y, wn, ws, "u")
+        rest = [i for i in range(M) if i != 1]
+        assert torch.equal(y[rest], x[rest]) and not torch.isfinite(y[1]).any()
+
+
 @pytest.mark.parametrize("wdtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K,I,eps", [(1, 64, 64, 176, 1e-5), (5, 384, 1056, 416, 1e-6), (8, 2048, 8192, 1024, 1e-5),
                                          (16, 4096, 14336, 512, 1e-5), (13, 160, 416, 48, 1e-5), (2, 2304, 2304, 1184, 1e-6)])
