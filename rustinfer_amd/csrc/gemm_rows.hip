@@ -3,20 +3,23 @@
 //
 // With that many rows a wave of the few-row kernel (gemm.hip) asks for as many bytes of
 // activations as of weights, and the product takes as long as if both came from memory.  Here
-// the four waves of a block work on the same 256 values of K at a time: the block brings that
-// stretch of all (up to 64) rows into LDS once, in the order the matrix instructions read them,
-// and every wave multiplies it with weight tiles of its own, which it streams from memory
-// straight into registers, a whole stretch (8 k-steps) ahead.  What is asked of memory is then
-// the weights, once, and one copy of the activations a block.
+// the waves of a group work on the same 64 values of K at a time: the group brings that stretch of all (up to 64) rows into LDS once,
+// and each of its waves the stretch of weight tiles of its own beside it, with loads that write LDS directly, into a ring of
+// two to four stages, in the order in which the matrix instructions read them.  What is asked of memory is then the weights, once, and
+// one copy of the activations a block, and nothing but a wave's own counter of loads and one barrier a stage stands between
+// them and the products.  (Through registers a stretch ahead, the compiled loop waited for every load before it asked for the next stretch;
+// with those waits gone, copies of the loads' registers still waited for most of them.)
 //
-// A block owns 4 * NT tiles of 16 columns (SWIGLU: as many of the gate half and of the up half of
+// A block owns 2 or 4 waves' NT tiles of 16 columns (SWIGLU: as many of the gate half and of the up half of
 // a stacked [2N, K] matrix, and writes silu(gate) * up).  Products with few columns are also
 // split over K between blocks (blockIdx.y), each leaving 32-bit partial sums in its own slice of
-// C, which the norm that follows adds up.  N % 16 == 0, K % 32 == 0.
+// C, which the norm that follows adds up, and a block holds two or four groups of waves, which split its share of K between them
+// through rings of their own.  N % 16 == 0, K % 32 == 0.
 //
-// At 64 rows the two stretch buffers of a block take 64 KB, two blocks of four waves a compute
-// unit; where the columns give too few blocks for that, a block holds two or four groups of waves
-// instead, which split its share of K between them through buffers of their own (128 KB).
+// What bounds it: bytes in flight, and the launch.  Measured, us, 20 / 40 / 64 rows, through registers / now, and a kernel that only reads as much: gate/up
+// 2 x 8192 x 2048 16.4 17.1 18.1 / 14.3 15.0 16.8 (11.3), 2 x 8192 x 3072 22.6 24.2 25.5 / 19.7 21.1 22.9 (16.2), 2 x 14336 x 4096 48 49 52 / 45 47 49 (35.6); q/k/v with
+// rotation 5120 x 3072 13.3 15.8 19.1 / 11.3 13.8 16.4 (6.2); in slices 2048 x 8192 11.0 11.0 12.1 / 8.5 9.0 9.9 (6.5), 3072 x 3072 7.7 8.3 9.4 / 6.1 7.1 8.2 (4.3); whole
+// 128256 x 3072 137 144 154 / 134 141 149 (116).
 #include "common.h"
 #include <mutex>
 
@@ -25,7 +28,10 @@ typedef float rf32x4_t __attribute__((ext_vector_type(4)));
 
 namespace {
 
-constexpr int KS_LONG = 8;                // k-steps of 32 in a stretch; 4 where four groups share a block
+constexpr int KS = 2;                     // k-steps of 32 in a stretch: 128 bytes of a row
+
+// s_waitcnt: at most n loads under way, whatever is asked of LDS
+constexpr int loads_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
 struct Store4 {
     static __device__ __forceinline__ void st(float* p, const float* v) {
@@ -38,15 +44,6 @@ struct Store4 {
         *reinterpret_cast<uint2*>(p) = t;
     }
 };
-
-// LDS holds a stretch as [k-step][m-tile][k-group][row of the tile] in units of 8 values (16
-// bytes), the order in which a wave's lanes read an operand; the row index is xor-ed with
-// (4 * k-step + k-group) % 16 so that the threads that bring a row in (32 of them write the
-// 32 units of one row) spread over the banks, while a read still takes 64 different units.
-template <int MT>
-__device__ __forceinline__ int lds_unit(int ks, int mt, int g, int c) {
-    return ((ks * MT + mt) * 4 + g) * 16 + (c ^ ((4 * ks + g) & 15));
-}
 
 // ROPE: the product is the fused q/k/v projection of a step's tokens, with the weight's rows permuted
 // within each head as for the few-row kernel (gemm.hip, ri_qkv_rope_row_order): a tile holds 8
@@ -61,25 +58,24 @@ struct RowsRope {
     int H, Hkv, hd, page;
 };
 
-// KG groups of WAVES waves share a block: each group takes its own half of the block's stretches,
-// through LDS buffers of its own, and the groups' sums meet in LDS at the end.  That doubles the
-// waves and the bytes under way on a compute unit where the columns make too few blocks for two a unit.
-template <int MT, int NT, bool SWIGLU, typename TO, int WAVES, int KG, int KS, bool ROPE = false>
+// KG groups of WAVES waves share a block: each group takes its own share of the block's stretches, through a ring of its own of ST stages, and the
+// groups' sums meet in LDS at the end.
+template <int MT, int NT, bool SWIGLU, typename TO, int WAVES, int KG, int ST, bool ROPE = false>
 __global__ __launch_bounds__(WAVES * KG * 64) void gemm_rows_lds_kernel(
         const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W,
         TO* __restrict__ C, int ldc, int M, int N, int K, int stretches_per_block, size_t part_stride,
         RowsRope rp) {
     static_assert(!ROPE || (NT == 1 && !SWIGLU && sizeof(TO) == 2), "the rotation goes with one bfloat16 tile a wave");
     constexpr int NW = SWIGLU ? 2 * NT : NT;
-    constexpr int THREADS = WAVES * 64;                     // of a group
-    constexpr int XP = MT * KS / WAVES;                     // 16-byte pieces of a stretch a thread brings in
-    constexpr int RU = KS * 4;                              // such pieces in a row of a stretch
-    static_assert(MT * 16 * RU == XP * THREADS, "a stretch must divide evenly over the threads of a group");
-    constexpr int STRETCH = KS * MT * 64;                   // units of a stretch in LDS
-    extern __shared__ __align__(16) rbf16x8_t xs_all[];     // [KG][2][STRETCH]
-    const int kg = threadIdx.x / THREADS, tid = threadIdx.x % THREADS;
-    rbf16x8_t* xs = xs_all + kg * 2 * STRETCH;
-    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, grp = lane >> 4;   // the same in all lanes of a wave
+    constexpr int XPIECES = MT * 2, FX = (XPIECES + WAVES - 1) / WAVES;        // kilobytes of the rows in a stage: eight rows each; a wave's
+    constexpr int XA = XPIECES * 64, STAGE = XA + WAVES * NW * KS * 64;        // in units of 16 bytes
+    constexpr int PER = FX + NW * KS;                                          // loads of a wave a stage
+    static_assert((ST - 1) * PER < 64, "more loads under way than the counter counts");
+    extern __shared__ __align__(16) rbf16x8_t xs_all[];     // [KG][ST][STAGE]
+    // a wave's group and its number in it, the same in all its lanes
+    const int all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), kg = all / WAVES, wave = all % WAVES;
+    rbf16x8_t* xs = xs_all + kg * ST * STAGE;
+    const int lane = threadIdx.x & 63, col = lane & 15, grp = lane >> 4;
     const int ntiles = N / 16, nks_all = K / 32;
     const int s_all = (nks_all + KS - 1) / KS;
     const int b_begin = blockIdx.y * stretches_per_block;
@@ -89,65 +85,73 @@ __global__ __launch_bounds__(WAVES * KG * 64) void gemm_rows_lds_kernel(
     const int s_end = min(b_end, s_begin + span);
     C += (size_t)blockIdx.y * part_stride;
 
+    // What this wave brings in.  Rows: eight a load, 128 bytes each, eight lanes a row; a row's eight units of 16 bytes are xor-ed
+    // with the row's number and the parity of its eight, so that the 16 rows of a read lie in different banks.  Weights: its own
+    // tiles, as they lie.  Rows and tiles beyond the end are read (clamped) and never stored; of an odd last step, the step before it is
+    // read again and not multiplied.
+    size_t fx[FX];
+#pragma unroll
+    for (int i = 0; i < FX; ++i) {
+        const int p = min(wave * FX + i, XPIECES - 1);
+        fx[i] = (size_t)min(p * 8 + (lane >> 3), M - 1) * lda + ((lane & 7) ^ (lane >> 3) ^ (p & 1)) * 8;
+    }
     const bf16_t* wp[NW];
 #pragma unroll
     for (int a = 0; a < NW; ++a) {
-        // tiles beyond N are read (clamped) but never stored
         const int tile = min(((int)blockIdx.x * WAVES + wave) * NT + (a % NT), ntiles - 1) + (a >= NT ? ntiles : 0);
         wp[a] = W + ((size_t)tile * nks_all * 64 + lane) * 8;
     }
+    auto fetch = [&](int s, int at) {
+#pragma unroll
+        for (int u = 0; u < KS; ++u)
+#pragma unroll
+            for (int a = 0; a < NW; ++a)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(wp[a] + (size_t)min(s * KS + u, nks_all - 1) * 512),
+                    (__attribute__((address_space(3))) void*)(xs + at + XA + ((wave * NW + a) * KS + u) * 64), 16, 0, 2);
+        const bool odd = (s + 1) * KS > nks_all;
+#pragma unroll
+        for (int i = 0; i < FX; ++i) {
+            const int p = min(wave * FX + i, XPIECES - 1);
+            const size_t from = fx[i] - (odd && (((lane & 7) ^ (lane >> 3) ^ (p & 1)) & 4) ? 32 : 0);
+            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(A + (size_t)s * (KS * 32) + from),
+                (__attribute__((address_space(3))) void*)(xs + at + p * 64), 16, 0, 0);
+        }
+    };
     rf32x4_t acc[NW][MT];
 #pragma unroll
     for (int a = 0; a < NW; ++a)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[a][mt] = rf32x4_t{0.f, 0.f, 0.f, 0.f};
-    const rbf16x8_t zero = {};
-
-    // piece j of this thread: row m = p / RU, values k = 8 * (p % RU) .. + 7 of the stretch, p = tid + THREADS j
-    auto load_x = [&](int s, rbf16x8_t (&xr)[XP]) {
+    const int xat = (col >> 3) * 64 + (col & 7) * 8, xsw = grp ^ (col & 7) ^ (col >> 3);
+    const int wat = XA + wave * NW * KS * 64 + lane;
+    auto multiply = [&](int at, int u) {
+        rbf16x8_t xf[MT], wf[NW];
 #pragma unroll
-        for (int j = 0; j < XP; ++j) {
-            const int p = tid + THREADS * j;
-            const int m = p / RU, k = s * (KS * 32) + (p % RU) * 8;
-            xr[j] = (m < M && k < K) ? *reinterpret_cast<const rbf16x8_t*>(A + (size_t)m * lda + k) : zero;
-        }
+        for (int a = 0; a < NW; ++a) wf[a] = xs[at + wat + (a * KS + u) * 64];
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) xf[mt] = xs[at + xat + mt * 128 + (xsw ^ (u * 4))];
+#pragma unroll
+        for (int a = 0; a < NW; ++a)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+                acc[a][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a], xf[mt], acc[a][mt], 0, 0, 0);
     };
-    auto store_x = [&](int buf, const rbf16x8_t (&xr)[XP]) {
-#pragma unroll
-        for (int j = 0; j < XP; ++j) {
-            const int p = tid + THREADS * j;
-            const int m = p / RU, kp = p % RU;
-            xs[buf * STRETCH + lds_unit<MT>(kp >> 2, m >> 4, kp & 3, m & 15)] = xr[j];
-        }
-    };
-    auto load_w = [&](int s, rbf16x8_t (&wf)[NW][KS]) {
-#pragma unroll
-        for (int u = 0; u < KS; ++u) {
-            const int ks = s * KS + u;
-#pragma unroll
-            for (int a = 0; a < NW; ++a)
-                wf[a][u] = ks < nks_all ? ld_stream16<rbf16x8_t>(wp[a] + (size_t)ks * 512) : zero;
-        }
-    };
-    auto multiply = [&](int buf, const rbf16x8_t (&wf)[NW][KS]) {
-#pragma unroll
-        for (int u = 0; u < KS; ++u) {
-            rbf16x8_t xf[MT];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) xf[mt] = xs[buf * STRETCH + lds_unit<MT>(u, mt, grp, col)];
-#pragma unroll
-            for (int a = 0; a < NW; ++a)
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    acc[a][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[a][u], xf[mt], acc[a][mt], 0, 0, 0);
-        }
-    };
-
-    // what the rotation needs of each token is asked for now: a chain of small loads at the end of
-    // a short kernel would cost microseconds
+    // What the rotation needs of each token is asked for at the start, its row and position ahead of the first stages, its page, cosines and sines behind
+    // them: a chain of small loads at the end of a short kernel would cost microseconds.
     int rp_section = 0, rp_head = 0, rp_j = 0;
     int rp_b[ROPE ? MT : 1], rp_blk[ROPE ? MT : 1], rp_slot[ROPE ? MT : 1];
     float4 rp_c[ROPE ? MT : 1], rp_s[ROPE ? MT : 1];
+    if constexpr (ROPE) {
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            const int m = mt * 16 + col;
+            rp_b[mt] = -1; rp_slot[mt] = 0;
+            if (kg == 0 && m < M) { rp_b[mt] = rp.row_of_token[m]; rp_slot[mt] = rp.positions[m]; }
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < ST - 1; ++p)
+        if (s_begin + p < s_end) fetch(s_begin + p, p * STAGE);
     if constexpr (ROPE) {
         const int hd = rp.hd, half = hd >> 1, q_dim = rp.H * hd, kv_dim = rp.Hkv * hd;
         const int n0 = min(((int)blockIdx.x * WAVES + wave), ntiles - 1) * 16;
@@ -157,49 +161,40 @@ __global__ __launch_bounds__(WAVES * KG * 64) void gemm_rows_lds_kernel(
         rp_j = (within % hd) >> 4;                                                       // the tile is tile j of its head
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
-            const int m = mt * 16 + col;
-            rp_b[mt] = -1; rp_blk[mt] = -1; rp_slot[mt] = 0;
+            const int b = rp_b[mt], pos = rp_slot[mt];
+            rp_blk[mt] = -1;
+            rp_slot[mt] = pos % rp.page;
             rp_c[mt] = make_float4(1.f, 1.f, 1.f, 1.f);
             rp_s[mt] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (kg == 0 && m < M) {
-                const int b = rp.row_of_token[m], pos = rp.positions[m];
-                rp_b[mt] = b;
-                rp_slot[mt] = pos % rp.page;
-                if (b >= 0) {
-                    if (rp_section != 0) rp_blk[mt] = rp.table[(size_t)b * rp.max_blocks + pos / rp.page];
-                    if (rp_section != 2) {
-                        // this lane's four values are features 8 j + (grp & 1) 4 + i of a half
-                        const size_t at = (size_t)pos * half + 8 * rp_j + (grp & 1) * 4;
-                        rp_c[mt] = *reinterpret_cast<const float4*>(rp.cos_t + at);
-                        rp_s[mt] = *reinterpret_cast<const float4*>(rp.sin_t + at);
-                    }
+            if (b >= 0) {
+                if (rp_section != 0) rp_blk[mt] = rp.table[(size_t)b * rp.max_blocks + pos / rp.page];
+                if (rp_section != 2) {
+                    // this lane's four values are features 8 j + (grp & 1) 4 + i of a half
+                    const size_t at = (size_t)pos * half + 8 * rp_j + (grp & 1) * 4;
+                    rp_c[mt] = *reinterpret_cast<const float4*>(rp.cos_t + at);
+                    rp_s[mt] = *reinterpret_cast<const float4*>(rp.sin_t + at);
                 }
             }
         }
     }
 
-    // two stretches an iteration, so that the weights' registers swap roles without being copied;
-    // every wave of the block passes the same barriers, with or without a stretch of its own left
-    rbf16x8_t w0[NW][KS], w1[NW][KS], xr[XP];
-    if (s_begin < s_end) {
-        load_x(s_begin, xr);
-        load_w(s_begin, w0);
-        store_x(0, xr);
+    // A stage: this wave's loads of it have arrived, then, behind the barrier, everyone's, and all have read the stage before it, into whose
+    // place the next loads go.  Every wave passes the same barriers, with or without a stretch of its own left.
+    int at = 0;
+    for (int s = s_begin; s < s_begin + span; ++s) {
+        // (what the rotation asked for behind the first stages counts as under way: fewer may, for one stage)
+        if (s + ST - 2 < s_end) __builtin_amdgcn_s_waitcnt(loads_imm((ST - 2) * PER));
+        else __builtin_amdgcn_s_waitcnt(loads_imm(0));
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (s + ST - 1 < s_end) fetch(s + ST - 1, at == 0 ? (ST - 1) * STAGE : at - STAGE);
+        if (s < s_end) {
+            multiply(at, 0);
+            if (s * KS + 1 < nks_all) multiply(at, 1);
+        }
+        at = at + STAGE == ST * STAGE ? 0 : at + STAGE;
     }
-    __syncthreads();
-    for (int i = 0; i < span; i += 2) {
-        const int s = s_begin + i;
-        const bool have0 = s < s_end, more1 = s + 1 < s_end, more2 = s + 2 < s_end;
-        if (more1) { load_x(s + 1, xr); load_w(s + 1, w1); }
-        if (have0) multiply(0, w0);
-        if (more1) store_x(1, xr);
-        __syncthreads();
-        if (i + 1 >= span) break;
-        if (more2) { load_x(s + 2, xr); load_w(s + 2, w0); }
-        if (more1) multiply(1, w1);
-        if (more2) store_x(0, xr);
-        __syncthreads();
-    }
+    if (KG > 1) __syncthreads();
     if (KG > 1) {
         // the other groups' sums, through the LDS the stretches have left: [group - 1][wave][a][mt][lane]
         rf32x4_t* red = reinterpret_cast<rf32x4_t*>(xs_all);
@@ -279,15 +274,22 @@ __global__ __launch_bounds__(WAVES * KG * 64) void gemm_rows_lds_kernel(
     }
 }
 
+// Stages of a ring: what fits half a compute unit's LDS with one group, a whole one's with more, two to four.
+constexpr int ring(int stage_units, int kg, int most) {
+    const int fit = (kg == 1 ? 80 : 152) * 64 / (stage_units * kg);
+    return fit < 2 ? 2 : fit > most ? most : fit;
+}
+
 template <int MT, int NT, bool SWIGLU, typename TO, int KG>
 int launch_rows_groups(const bf16_t* A, int lda, const bf16_t* W, TO* C, int ldc, int M, int N, int K,
                        int parts, size_t part_stride, hipStream_t stream) {
-    // four waves a group (eight: twice the columns, half the blocks, slower throughout); four groups:
-    // of two waves and half as long stretches, so that twice the blocks take the same LDS
-    constexpr int waves = KG == 4 ? 2 : 4;
-    constexpr int KS = KG == 4 ? KS_LONG / 2 : KS_LONG;
-    constexpr size_t lds = (size_t)KG * 2 * KS * MT * 64 * sizeof(rbf16x8_t);
-    auto kernel = gemm_rows_lds_kernel<MT, NT, SWIGLU, TO, waves, KG, KS>;
+    // Four waves a group; `four groups`: of two waves, so that a block owns half the columns.  With two weight tiles a wave (SwiGLU) four groups leave
+    // room for two stages, which is not enough under way: two groups of four stages (8192 x 3072, 40 rows, four groups of two 24.7 us, two of four 21.1).
+    constexpr int waves = KG == 4 ? 2 : 4, groups = KG == 4 && SWIGLU ? 2 : KG;
+    constexpr int stage = MT * 128 + waves * (SWIGLU ? 2 * NT : NT) * KS * 64, ST = ring(stage, groups, KG == 4 && SWIGLU ? 4 : 3);
+    constexpr size_t lds = (size_t)groups * ST * stage * sizeof(rbf16x8_t);
+    static_assert(lds <= 160 * 1024, "a compute unit's LDS");
+    auto kernel = gemm_rows_lds_kernel<MT, NT, SWIGLU, TO, waves, groups, ST>;
     if (lds > 64 * 1024) {          // beyond what a kernel may take unasked: ask once a device
         static std::mutex mu;
         static bool asked[64] = {};
@@ -304,7 +306,7 @@ int launch_rows_groups(const bf16_t* A, int lda, const bf16_t* W, TO* C, int ldc
     const int s_all = (K / 32 + KS - 1) / KS;
     const int per = (s_all + parts - 1) / parts;
     const int blocks = (N / 16 + waves * NT - 1) / (waves * NT);
-    kernel<<<dim3(blocks, parts), waves * KG * 64, lds, stream>>>(A, lda, W, C, ldc, M, N, K, per, part_stride, RowsRope{});
+    kernel<<<dim3(blocks, parts), waves * groups * 64, lds, stream>>>(A, lda, W, C, ldc, M, N, K, per, part_stride, RowsRope{});
     return 0;
 }
 
@@ -330,9 +332,10 @@ template <int MT, int KG>
 int launch_rows_rope(const bf16_t* A, int lda, const bf16_t* W, bf16_t* C, int ldc, int M, int N, int K,
                      const RowsRope& rp, hipStream_t stream) {
     static_assert(KG == 2 || KG == 4, "two or four groups");
-    constexpr int waves = KG == 4 ? 2 : 4, KS = KG == 4 ? KS_LONG / 2 : KS_LONG;
-    constexpr size_t lds = (size_t)KG * 2 * KS * MT * 64 * sizeof(rbf16x8_t);
-    auto kernel = gemm_rows_lds_kernel<MT, 1, false, bf16_t, waves, KG, KS, true>;
+    constexpr int waves = KG == 4 ? 2 : 4, stage = MT * 128 + waves * KS * 64, ST = ring(stage, KG, 3);
+    constexpr size_t lds = (size_t)KG * ST * stage * sizeof(rbf16x8_t);
+    static_assert(lds <= 160 * 1024, "a compute unit's LDS");
+    auto kernel = gemm_rows_lds_kernel<MT, 1, false, bf16_t, waves, KG, ST, true>;
     if (lds > 64 * 1024) {
         static std::mutex mu;
         static bool asked[64] = {};
@@ -361,28 +364,32 @@ int launch_rows_rope_groups(const bf16_t* A, int lda, const bf16_t* W, bf16_t* C
 
 }  // namespace
 
-// Slices of K, and wave groups a block, for a product of M rows, N columns and K inner values whose
-// partial sums a norm adds up.  Blocks enough to fill the chip twice, at most 8 slices (measured
-// at 64 rows, us: 4096 x 4096 with 2, 4, 8, 16 slices 16.5, 12.2, 11.3, 15.0; 4096 x 14336: 53,
-// 35, 29, 32; 2048 x 8192: 26, 16, 11.8, 11.2, but the norm that adds 16 slices up loses more than
-// that gains: 64 rows decode at 29,200 tokens a second with 8 slices at most and at 26,600 with
-// 16).  With more than 32 rows a block of two groups takes 128 KB of LDS, one block a compute
-// unit: then two groups pay where a block's share of K is short (half the slices do as well:
-// 4096 x 4096, 8 slices of one group 12.1, 4 of two 12.1; 3072 x 3072: 9.7, 8.9) or where all
-// blocks still fit the chip at once (2048 x 8192: 8 slices, 12.9 with one group, 11.6 with two);
-// not for a long K over many columns (4096 x 14336: 8 of one 28.5, 4 of two 32.2, 8 of two 35.2).
+// Slices of K, and wave groups a block, for a product of M rows, N columns and K inner values whose partial sums a norm adds up: blocks enough to
+// fill the chip twice, at most 8 slices (16 of 2048 x 8192 take less here and cost the norm more), then groups where that fills the units better with as many
+// slices or fewer.  A block of two groups has a unit to itself (two share it up to 32 rows), three of one group share one
+// (four up to 32 rows), and one of four groups, of half the columns, has one to itself.  Measured, us (slices/groups), at 20, 32, 48, 64 rows: 2048 x 2048
+// 4/4 4.5 4.7 5.2 5.6, 8/1 4.9 5.2 5.7 6.0; 1024 x 3072 8/4 4.1 4.3 4.8 5.3, 8/1 4.7 5.0 5.5 5.9; 2048 x 8192 8/2 8.5 8.7 9.2 9.9, 4/4 9.9 10.4 11.2 11.7, 8/1 9.0 9.1
+// 9.8 10.6; 3072 x 8192 4/2 11.6 12.0 13.2 14.3, 8/1 11.1 11.7 13.7 15.4; 4096 x 4096 8/2 9.0 9.5 - -, 4/2 9.9 10.2 10.8 11.5, 8/1 9.6 10.1 10.8 11.8; 4096 x 14336 8/2
+// 22.0 22.9 27.3 29.7, 4/2 21.2 21.9 23.9 25.4, 8/1 21.5 21.7 24.4 26.5; 5120 x 13824 8/1 28.1 29.5 33.1 35.8, 4/1 29.4 31.6 36.7 40.5; 5120 x 5120 4/1 12.7 13.9 16.8
+// 18.1, 8/1 12.5 13.7 15.8 17.3 (and the norm's slices); 8192 x 8192 4/2 28.1 26.7 30.1 31.7, 4/1 29.0 27.8 26.3 28.3.  (Through registers, with the plan of then: 2048 x 2048
+// 5.0 5.3 6.4 6.9, 2048 x 8192 11.1 11.3 11.2 12.1, 3072 x 8192 12.5 13.0 14.0 15.6, 4096 x 4096 10.1 10.5 12.2 13.0, 4096 x 14336 22.8 23.2 24.6 26.4.)
 extern "C" int ri_gemm_rows_plan(int M, int N, int K, int nt, int* parts_out, int* groups_out) {
     RI_REQUIRE(parts_out && groups_out && N > 0 && K > 0 && (nt == 1 || nt == 2), "ri_gemm_rows_plan: bad arguments");
-    const int blocks = (N / 16 + 4 * nt - 1) / (4 * nt), stretches = (K / 32 + KS_LONG - 1) / KS_LONG;
+    const int blocks = (N / 16 + 4 * nt - 1) / (4 * nt), stretches = (K + 63) / 64;
     int parts = 1, groups = 1;
-    while (parts < 8 && blocks * parts < 512 && stretches / (parts * 2) >= 1) parts *= 2;
-    // with more than 32 rows two blocks fit a compute unit: no more blocks than the chip holds at once
-    // (5120 x 5120 at 64 rows, 80 blocks of columns: 8 slices 19.9 us, 4 slices 18.2)
-    if (M > 32 && parts > 1 && blocks * parts > 512) parts /= 2;
-    if (M > 32 && parts == 8) {
-        if (blocks * parts <= 256 && stretches / parts >= 4) groups = 2;
-        else if (stretches / parts <= 2 && blocks * 4 <= 256) { parts = 4; groups = 2; }
+    while (parts < 8 && blocks * parts < 512 && stretches / (parts * 8) >= 1) parts *= 2;
+    // with more than 32 rows no more blocks than the chip holds at once (a long K: three a unit; the norm adds the slices of a short one)
+    if (M > 32 && parts > 1 && blocks * parts > (K >= 8192 ? 768 : 512)) parts /= 2;
+    if (blocks <= 32 && K <= 4096) {
+        parts = blocks <= 16 ? 8 : 4;
+        groups = 4;
+    } else if (M <= 32) {
+        if (blocks * parts <= 256 || (blocks * parts > 460 && blocks * parts <= 512 && K <= 8192)) groups = 2;
+    } else if (parts == 8) {
+        if (blocks * 8 <= 256) groups = 2;
+        else if (blocks * 4 < 256 || (blocks * 4 == 256 && K <= 4096)) { parts = 4; groups = 2; }
     }
+    while (parts * groups > 1 && stretches < parts * groups) (groups > 1 ? groups : parts) /= 2;
     *parts_out = parts;
     *groups_out = groups;
     return 0;
@@ -435,11 +442,8 @@ extern "C" int ri_gemm_rows_bf16(const void* A, int lda, const void* W, void* C,
 // few-row kernel is as fast or faster at these sizes and slower at larger ones (24 rows: 12288 x
 // 4096 27.3 -> 23.5, 15360 x 5120 35.9 -> 28.8, 10240 x 8192 49.0 -> 42.4): the caller chooses.
 //
-// Blocks of 32 columns (four pairs of waves) where all of them run at once: a block takes the LDS
-// of a whole compute unit with more than 32 rows and half of it with fewer; else blocks of 64
-// columns (two groups of four waves), half as many.  64 rows, 32 / 64 columns a block, us: 6144
-// columns of K = 4096 22.7 / 28.1, 12288: 43.2 / 32.1; 15360 x 5120: 55.2 / 40.5; 10240 x 8192:
-// 79.1 / 56.7; with 32 rows 12288 x 4096 24.6 / 27.1, 15360 x 5120 31.5 / 33.7.
+// Blocks of 32 columns (four pairs of waves) where all of them run at once, one a compute unit; else blocks of 64
+// columns (two groups of four waves), half as many: 288 blocks of 32 columns (9216 x 4096) took 27.1 us with 32 rows, 144 of 64 23.0 with 33.
 extern "C" int ri_gemm_rows_qkv_rope(const void* A, int lda, const void* W, void* C, int ldc, int M, int K,
                                      int H, int Hkv, int hd, const float* cos_t, const float* sin_t, int table_rows,
                                      const int* positions, const int* row_of_token, void* kc, void* vc,
@@ -455,8 +459,7 @@ extern "C" int ri_gemm_rows_qkv_rope(const void* A, int lda, const void* W, void
     const RowsRope rp{cos_t, sin_t, positions, row_of_token, table, max_blocks, (bf16_t*)kc, (bf16_t*)vc, H, Hkv, hd, page};
     const bf16_t* a = (const bf16_t*)A;
     const bf16_t* w = (const bf16_t*)W;
-    const int at_once = M <= 32 ? 512 : 256;
-    const int groups = (N / 16 + 1) / 2 <= at_once ? 4 : 2;
+    const int groups = (N / 16 + 1) / 2 <= 256 ? 4 : 2;
     int rc;
     if (M <= 32) rc = launch_rows_rope_groups<2>(a, lda, w, (bf16_t*)C, ldc, M, N, K, groups, rp, stream);
     else if (M <= 48) rc = launch_rows_rope_groups<3>(a, lda, w, (bf16_t*)C, ldc, M, N, K, groups, rp, stream);

@@ -343,7 +343,7 @@ def qkv_rope_fused(x: torch.Tensor, w_fused: torch.Tensor, qkv: torch.Tensor, H:
         raise KernelError("qkv_rope_fused: cos/sin must be contiguous float32 [positions, head_dim/2]")
     lds_rows = (M >= QKV_ROPE_LDS_MIN_ROWS and N >= QKV_ROPE_LDS_MIN_COLUMNS) or (M >= ROWS_LDS_MIN_ROWS and N * K >= QKV_ROPE_LDS_LARGE)
     if scale is None and lds_rows and K % 32 == 0 and hd % 16 == 0:
-        # 33..64 tokens, or 17 and more over a large weight: the kernel whose blocks share the activations through LDS
+        # the kernel whose blocks share the activations through LDS
         _check(_lib().ri_gemm_rows_qkv_rope(
             _ptr(x), x.stride(0), _ptr(w_fused), _ptr(qkv), qkv.stride(0), M, K, H, Hkv, hd, _ptr(cos), _ptr(sin),
             cos.shape[0], _ptr(positions), _ptr(row_of_token), _ptr(k_cache), _ptr(v_cache), k_cache.shape[0],
@@ -686,26 +686,21 @@ def _skinny_ok(x, w, M, K):
             and w.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
 
 
-QKV_ROPE_LDS_MIN_ROWS = 33      # the fused q/k/v projection takes the LDS kernel from this many tokens on ...
-QKV_ROPE_LDS_MIN_COLUMNS = 4096 # ... and columns (128 blocks of 32; in a step of 64 tokens, us: 6144 columns 28.0 -> 24.8,
-                                # 5120: 22.6 -> 20.3, 3072: 13.9 -> 14.9)
-QKV_ROPE_LDS_LARGE = 40 << 20   # ... and from 17 tokens on where the weight has this many elements (product alone at 24
-                                # rows, us: 12288 x 4096 27.3 -> 23.5, 15360 x 5120 35.9 -> 28.8, 10240 x 8192 49.0 -> 42.4;
-                                # 6144 x 4096 15.4 -> 16.3, 5120 x 3072 12.5 -> 12.5)
+QKV_ROPE_LDS_LARGE = 14 << 20   # the fused q/k/v projection takes the LDS kernel from 17 tokens on where the weight has this many elements (us at
+                                # 17 and 32 tokens: 6144 x 4096 15.1 17.9 -> 14.7 15.7, 5120 x 3072 12.0 14.4 -> 11.0 12.3, 3072 x 2048 7.5 8.7 -> 8.0 8.7) ...
+QKV_ROPE_LDS_MIN_ROWS = 33      # ... and from 33 with this many columns (3072 x 2048 at 33, 48, 64 tokens: 9.6 11.2 13.4 -> 9.6 10.2 11.8; 1536 x 1024
+QKV_ROPE_LDS_MIN_COLUMNS = 3072 # 7.2 7.5 9.3 -> 7.2 7.6 8.8)
 ROWS_LDS_MIN_ROWS = 17          # from here to 64 rows, products whose partial sums a norm adds up take the LDS kernel
 ROWS_LDS_WIDE_COLUMNS = 16384   # whole products (no slices of K) take it from this many columns on: the output head, 250 -> 205 us at 64 rows
-ROWS_LDS_SWIGLU_MIN_ROWS = 33   # the fused gate/up product only with more rows, and with columns enough for its blocks
 
 
 def _swiglu_groups(I: int) -> int:
-    """Wave groups a block of the LDS kernel for a fused gate/up product of ``I`` columns with more
-    than 32 rows (0: the few-row kernel does better).  A block of four groups of two waves owns 32
-    columns and one of two groups of four waves 64: either takes the LDS of a whole compute unit,
-    so its blocks should be most of 256 and no more; a block of one group of four waves owns 64
-    columns and half that LDS, which is the form for more than 256 such blocks.  Measured at 64
-    rows, us, few-row kernel / one / two / four groups: I = 8192, K = 2048: 22 / 25 / 22 / 18;
-    8192 x 3072: 32 / 36 / 32 / 25; 11008 x 4096: 62 / 52 / 44 / 54; 14336 x 4096: 57 / 56 / 50 /
-    58; 13824 x 5120: 83 / 66 / 58 / 71; 28672 x 8192: 194 / 159 / 179 / 208."""
+    """Wave groups a block of the LDS kernel for a fused gate/up product of ``I`` columns (0: the few-row kernel does
+    better).  4: blocks of 32 columns, 2: of 64; either takes the LDS of a whole compute unit, so its blocks should be most of
+    256 and no more; 1: blocks of 64 columns and half that LDS, the form for more than 256 such
+    blocks.  Measured, us, few-row kernel / this form at 17, 32, 48, 64 rows: 8192 x 2048 16.0 16.4 19.3 21.8 / 14.3 13.9 15.1 16.7; 8192 x
+    3072 20.7 22.1 26.4 30.2 / 19.7 19.6 21.1 23.1; 11008 x 4096 39 41 54 61 / 35 36 38 39; 14336 x 4096 47 47 51 56 / 46 47 48 48; 9728 x 2560
+    27 31 37 43 / 23 23 25 27; 4864 x 896 7.9 9.0 11.1 13.3 / 6.7 7.0 8.2 9.1; not 3072 x 1024 (96 blocks) 7.3 7.8 9.0 10.6 / 9.2 8.9 10.4 11.6."""
     b64, b32 = (I + 63) // 64, (I + 31) // 32
     if 128 <= b32 <= 256:
         return 4
@@ -716,10 +711,9 @@ def _swiglu_groups(I: int) -> int:
     return 0
 
 
-def _rows_ok(x, w, w_tiled, M, N, K, min_rows=None):
+def _rows_ok(x, w, w_tiled, M, N, K):
     """Whether the kernel that shares a block's activations through LDS takes this product."""
-    lo = ROWS_LDS_MIN_ROWS if min_rows is None else min_rows
-    return (not FORCE_LIBRARY_GEMM and w_tiled is not None and x.dtype == torch.bfloat16 and lo <= M <= SKINNY_MAX_ROWS and N % 16 == 0
+    return (not FORCE_LIBRARY_GEMM and w_tiled is not None and x.dtype == torch.bfloat16 and ROWS_LDS_MIN_ROWS <= M <= SKINNY_MAX_ROWS and N % 16 == 0
             and K % 32 == 0 and x.stride(0) % 8 == 0 and x.stride(1) == 1 and x.data_ptr() % 16 == 0 and _tiled_ok(w, w_tiled))
 
 
@@ -822,9 +816,13 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled=None,
     lib = _lib()
     if scale is None and N >= ROWS_LDS_WIDE_COLUMNS and out.dtype in (torch.bfloat16, torch.float32) \
             and out.stride(0) % 4 == 0 and _rows_ok(x, w, w_tiled, M, N, K):
-        # 17..64 rows against a very wide matrix (the output head): activations shared through LDS
+        # 17..64 rows against a very wide matrix (the output head): activations shared through LDS.  Two tiles a wave halve what is asked for of
+        # the activations, but rows a power of two apart then meet on the same channels of memory, which costs more where they are short or the
+        # rows few.  Us, one / two tiles at 20, 40, 64 rows: 128256 x 3072 134 149 164 / 134 141 149, x 2048 96 101 111 / 108 113 115, x 4096
+        # 190 211 224 / 194 199 205, 151936 x 1536 87 103 114 / 87 94 103, 64000 x 5120 108 124 141 / 106 110 120.
+        tiles = 2 if K & (K - 1) or (K >= 4096 and M > 32) else 1
         _check(lib.ri_gemm_rows_bf16(_ptr(x), x.stride(0), _ptr(w_tiled), _ptr(out), out.stride(0), M, N, K, _dt(out), 0, 1,
-                                     ctypes.c_longlong(0), 1, 1, _stream()))
+                                     ctypes.c_longlong(0), tiles, 1, _stream()))
         return
     to_library = scale is None and out.dtype in (torch.bfloat16, torch.float32) and _untiled_to_library(x, w, w_tiled, M) \
         and (N, K, x.stride(0), w.stride(0), out.stride(0), out.dtype) not in _LIBRARY_REFUSED
@@ -965,7 +963,7 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor,
     if M == 0:
         return
     groups = _swiglu_groups(I)
-    if scale is None and groups and _rows_ok(x, w_gate_up, w_tiled, M, I, K, ROWS_LDS_SWIGLU_MIN_ROWS):
+    if scale is None and groups and _rows_ok(x, w_gate_up, w_tiled, M, I, K):
         # many rows and blocks enough for the chip: activations shared through LDS
         _check(_lib().ri_gemm_rows_bf16(_ptr(x), x.stride(0), _ptr(w_tiled), _ptr(out), out.stride(0), M, I, K, BF16, 1, 1,
                                         ctypes.c_longlong(0), 1, groups, _stream()))
