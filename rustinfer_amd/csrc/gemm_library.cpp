@@ -263,21 +263,9 @@ int make_plan(const Key& k, Plan& p, const void* A, const void* W, void* ws, hip
     return 0;
 }
 
-}  // namespace
-
-// workspace: device memory the library may use (split products); the same size must be passed
-// for a shape each time.  Returns 0, or non-zero with a message in ri_last_error():
-// RI_NO_LIBRARY_KERNEL (2) if the library has no kernel for the problem (nothing was launched; the
-// caller may take a kernel of its own), 1 for every other failure.
-// out_f32 != 0: C is float32 (logits), else bfloat16.
-extern "C" int ri_gemm_library_bf16(const void* A, int lda, const void* W, int ldw, void* C, int ldc,
-                                    int M, int N, int K, int out_f32, void* workspace, size_t workspace_bytes,
-                                    hipStream_t stream) {
-    RI_REQUIRE(M > 0 && N > 0 && K > 0 && lda >= K && ldw >= K && ldc >= N, "ri_gemm_library: bad sizes M=%d N=%d K=%d", M, N, K);
-    RI_REQUIRE(A && W && C && (workspace || workspace_bytes == 0), "ri_gemm_library: null pointer");
-    // one caller at a time: the table of shapes may be emptied, and its descriptors with it
-    std::lock_guard<std::mutex> lock(g_mutex);
-    if (!g_handle) RI_LT(hipblasLtCreate(&g_handle), "hipblasLtCreate");
+// One product of the library (the caller holds g_mutex).
+int product(const void* A, int lda, const void* W, int ldw, void* C, int ldc, int M, int N, int K, int out_f32, void* workspace,
+            size_t workspace_bytes, hipStream_t stream) {
     const Key key{M, N, K, lda, ldw, ldc, out_f32 ? 1 : 0, workspace_bytes};
     auto it = g_plans.find(key);
     if (it == g_plans.end()) {
@@ -304,6 +292,43 @@ extern "C" int ri_gemm_library_bf16(const void* A, int lda, const void* W, int l
     return 0;
 }
 
+// Rows of a product that go in a call of their own: as many as make whole rounds of 256 tiles of 256 x 256 where there are two rounds or more and what is left
+// is at most four fifths of one; 0: all in one call.  Between whole rounds the library's choice divides tiles between units so that the product takes up
+// to twice what it should.  Measured, us, one call / two: 16384 x 3072, 2,100 rows 198 / 168, 2,385 290 / 186, 2,816 311 / 206, 3,328 272 / 247, 3,840 281 / 277; x 2048
+// 131 118, 158 127, 165 145, 175 170, 185 187; 16384 x 5120, 2,385 rows 452 / 307; 32768 x 4096, 1,280 366 / 255, 1,664 340 / 327; 8192 x 4096, 4,177 320 / 196, 5,120 361 / 232;
+// 4096 x 4096, 8,355 312 / 194.  Not with less than two rounds before (16384 x 3072, 1,064 rows 114 / 105, but 1,280 114 / 116; 8192 x 8192, 2,293 243 / 244), nor before a
+// round that is nearly whole (16384 x 3072, 2,969 rows 212 / 222).
+int rows_of_whole_rounds(int M, int N) {
+    if (N % 256 || N > 128 * 256 || 256 % (N / 256)) return 0;
+    const int round = 65536 / (N / 256), whole = M / round * round;
+    return whole >= 2 * round && M > whole && (long long)(M - whole) * 5 <= 4ll * round ? whole : 0;
+}
+
+}  // namespace
+
+// workspace: device memory the library may use (split products); the same size must be passed
+// for a shape each time.  Returns 0, or non-zero with a message in ri_last_error():
+// RI_NO_LIBRARY_KERNEL (2) if the library has no kernel for the problem (nothing was launched; the
+// caller may take a kernel of its own), 1 for every other failure.
+// out_f32 != 0: C is float32 (logits), else bfloat16.
+extern "C" int ri_gemm_library_bf16(const void* A, int lda, const void* W, int ldw, void* C, int ldc,
+                                    int M, int N, int K, int out_f32, void* workspace, size_t workspace_bytes,
+                                    hipStream_t stream) {
+    RI_REQUIRE(M > 0 && N > 0 && K > 0 && lda >= K && ldw >= K && ldc >= N, "ri_gemm_library: bad sizes M=%d N=%d K=%d", M, N, K);
+    RI_REQUIRE(A && W && C && (workspace || workspace_bytes == 0), "ri_gemm_library: null pointer");
+    // one caller at a time: the table of shapes may be emptied, and its descriptors with it
+    std::lock_guard<std::mutex> lock(g_mutex);
+    if (!g_handle) RI_LT(hipblasLtCreate(&g_handle), "hipblasLtCreate");
+    // (a tuned kernel has been chosen by time, for all rows)
+    const int first = g_tune ? 0 : rows_of_whole_rounds(M, N);
+    if (first) {
+        if (int rc = product(A, lda, W, ldw, C, ldc, first, N, K, out_f32, workspace, workspace_bytes, stream)) return rc;
+        A = (const char*)A + (size_t)first * lda * 2;
+        C = (char*)C + (size_t)first * ldc * (out_f32 ? 4 : 2);
+    }
+    return product(A, lda, W, ldw, C, ldc, M - first, N, K, out_f32, workspace, workspace_bytes, stream);
+}
+
 // on != 0: products of more than 64 rows look for the library's fastest kernel the first time a
 // (row bucket, N, K) is met (the device is synchronised and memory allocated, so the first product
 // of a shape must not fall into a graph capture; inside one the library's own choice is taken).
@@ -328,6 +353,9 @@ extern "C" int ri_gemm_library_reset() {
     g_bucket_algo.clear();
     return 0;
 }
+
+// For a test: see rows_of_whole_rounds.
+extern "C" int ri_gemm_library_first_rows(int M, int N) { return rows_of_whole_rounds(M, N); }
 
 // (shapes kept, questions put to the library's heuristic so far)
 extern "C" int ri_gemm_library_stats(int* plans, int* heuristic_calls) {

@@ -287,6 +287,25 @@ def test_slices_and_groups_of_the_rows_kernel(ops):
     assert pays(8, shape(8192, 8192)) and not pays(16, shape(8192, 8192)) and pays(16, shape(2048, 8192))
 
 
+@pytest.mark.parametrize("M,N,f32,first", [(1153, 32768, 0, 1024), (1433, 32768, 1, 1024), (1434, 32768, 0, 0), (1024, 32768, 0, 0), (767, 32768, 0, 0), (2049, 16384, 0, 2048),
+                                           (2100, 16640, 0, 0), (4500, 8192, 1, 4096)])
+def test_library_gemm_of_whole_rounds_and_the_rest(ops, M, N, f32, first):
+    """Rows that make whole rounds of tiles go in a call of their own: every row once, rows inside wider buffers, nothing beside them."""
+    K = 128
+    assert ops._lib().ri_gemm_library_first_rows(M, N) == first
+    xb = rnd(M, K + 8, dtype=torch.bfloat16, seed=1)
+    x, w = xb[:, :K], rnd(N, K, dtype=torch.bfloat16, seed=2, scale=0.1)
+    out = torch.full((M, N + 8), float("nan"), dtype=torch.float32 if f32 else torch.bfloat16, device=DEV)
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device=DEV)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    assert ops._lib().ri_gemm_library_bf16(p(x), K + 8, p(w), K, p(out), N + 8, M, N, K, f32, p(ws), ctypes.c_size_t(ws.numel()),
+                                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    ref = x.float() @ w.float().t()
+    # one rounding to bfloat16, or a sum of 128 products in 32 bits
+    assert torch.all((out[:, :N].float() - ref).abs() <= (2.0 ** -8 * ref.abs() if not f32 else 0) + 2.0 ** -16 * ref.abs().max())
+    assert torch.isnan(out[:, N:]).all()
+
+
 def test_library_gemm_with_a_tuned_kernel(ops, tmp_path):
     """With tuning on, a product of more than 64 rows times the library's kernels once for its row
     bucket, keeps the choice in a file, and gives the same result (to bfloat16 rounding) as before."""
