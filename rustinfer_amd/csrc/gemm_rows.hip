@@ -1,8 +1,9 @@
-// C[M, N] = A[M, K] . W[N, K]^T for 17..64 rows of bfloat16 against weights in tile order
+// C[M, N] = A[M, K] . W[N, K]^T for 8 to 64 rows of bfloat16 against weights in tile order
 // ([N/16][K/32][64 lanes][8], see gemm.hip), with the activations shared through LDS.
 //
-// With that many rows a wave of the few-row kernel (gemm.hip) asks for as many bytes of
-// activations as of weights, and the product takes as long as if both came from memory.  Here
+// From 17 rows on a wave of the few-row kernel (gemm.hip) asks for as many bytes of
+// activations as of weights, and the product takes as long as if both came from memory; with fewer it is the kernel's registers that limit what
+// is under way.  Here
 // the waves of a group work on the same 64 values of K at a time: the group brings that stretch of all (up to 64) rows into LDS once,
 // and each of its waves the stretch of weight tiles of its own beside it, with loads that write LDS directly, into a ring of
 // two to four stages, in the order in which the matrix instructions read them.  What is asked of memory is then the weights, once, and
@@ -19,7 +20,9 @@
 // What bounds it: bytes in flight, and the launch.  Measured, us, 20 / 40 / 64 rows, through registers / now, and a kernel that only reads as much: gate/up
 // 2 x 8192 x 2048 16.4 17.1 18.1 / 14.3 15.0 16.8 (11.3), 2 x 8192 x 3072 22.6 24.2 25.5 / 19.7 21.1 22.9 (16.2), 2 x 14336 x 4096 48 49 52 / 45 47 49 (35.6); q/k/v with
 // rotation 5120 x 3072 13.3 15.8 19.1 / 11.3 13.8 16.4 (6.2); in slices 2048 x 8192 11.0 11.0 12.1 / 8.5 9.0 9.9 (6.5), 3072 x 3072 7.7 8.3 9.4 / 6.1 7.1 8.2 (4.3); whole
-// 128256 x 3072 137 144 154 / 134 141 149 (116).
+// 128256 x 3072 137 144 154 / 134 141 149 (116).  Up to 16 rows, the few-row kernel / this one at 8, 16 rows: in slices 2048 x 8192 9.0 9.1 / 7.7 7.8 (6.5),
+// 3072 x 8192 14.1 12.6 / 11.0 11.1 (8.9), 5120 x 5120 13.7 14.0 / 11.3 12.1 (9.2); whole 16384 x 2048 14.9 18.0 / 13.7 13.8 (11.3).
+// Whole products of fewer columns at 17, 33, 64 rows: 8192 x 2048 10.1 19.1 20.6 / 8.9 9.8 11.1, 12288 x 4096 26 36 36 / 24 25 26.
 #include "common.h"
 #include <mutex>
 
@@ -321,6 +324,7 @@ int launch_rows(const bf16_t* A, int lda, const bf16_t* W, TO* C, int ldc, int M
 template <int NT, bool SWIGLU, typename TO>
 int dispatch_rows(const bf16_t* A, int lda, const bf16_t* W, TO* C, int ldc, int M, int N, int K,
                   int parts, size_t part_stride, int groups, hipStream_t stream) {
+    if (M <= 16) return launch_rows<1, NT, SWIGLU, TO>(A, lda, W, C, ldc, M, N, K, parts, part_stride, groups, stream);
     if (M <= 32) return launch_rows<2, NT, SWIGLU, TO>(A, lda, W, C, ldc, M, N, K, parts, part_stride, groups, stream);
     if (M <= 48) return launch_rows<3, NT, SWIGLU, TO>(A, lda, W, C, ldc, M, N, K, parts, part_stride, groups, stream);
     return launch_rows<4, NT, SWIGLU, TO>(A, lda, W, C, ldc, M, N, K, parts, part_stride, groups, stream);
@@ -366,7 +370,9 @@ int launch_rows_rope_groups(const bf16_t* A, int lda, const bf16_t* W, bf16_t* C
 
 // Slices of K, and wave groups a block, for a product of M rows, N columns and K inner values whose partial sums a norm adds up: blocks enough to
 // fill the chip twice, at most 8 slices (16 of 2048 x 8192 take less here and cost the norm more), then groups where that fills the units better with as many
-// slices or fewer.  A block of two groups has a unit to itself (two share it up to 32 rows), three of one group share one
+// slices or fewer.  Up to 16 rows: eight slices and four groups where their blocks are whole rounds of the 512 that the chip holds at once, two groups where
+// those of 64 columns are just that, else one group, and all blocks run at once; parts 1 where the few-row kernel is as fast.  us, few-row / this at 9 to 16 rows: 2048 x 2048 4.6
+// / 4.1, 2048 x 8192 8.8 / 7.7, 3072 x 8192 12.5 / 11.0, 4096 x 4096 8.7 / 8.5, 4096 x 14336 22.2 / 20.9, 5120 x 5120 14.0 / 12.1, 5120 x 13824 29.4 / 27.5.  With more: a block of two groups has a unit to itself (two share it up to 32 rows), three of one group share one
 // (four up to 32 rows), and one of four groups, of half the columns, has one to itself.  Measured, us (slices/groups), at 20, 32, 48, 64 rows: 2048 x 2048
 // 4/4 4.5 4.7 5.2 5.6, 8/1 4.9 5.2 5.7 6.0; 1024 x 3072 8/4 4.1 4.3 4.8 5.3, 8/1 4.7 5.0 5.5 5.9; 2048 x 8192 8/2 8.5 8.7 9.2 9.9, 4/4 9.9 10.4 11.2 11.7, 8/1 9.0 9.1
 // 9.8 10.6; 3072 x 8192 4/2 11.6 12.0 13.2 14.3, 8/1 11.1 11.7 13.7 15.4; 4096 x 4096 8/2 9.0 9.5 - -, 4/2 9.9 10.2 10.8 11.5, 8/1 9.6 10.1 10.8 11.8; 4096 x 14336 8/2
@@ -377,6 +383,17 @@ extern "C" int ri_gemm_rows_plan(int M, int N, int K, int nt, int* parts_out, in
     RI_REQUIRE(parts_out && groups_out && N > 0 && K > 0 && (nt == 1 || nt == 2), "ri_gemm_rows_plan: bad arguments");
     const int blocks = (N / 16 + 4 * nt - 1) / (4 * nt), stretches = (K + 63) / 64;
     int parts = 1, groups = 1;
+    if (M <= 16) {
+        const bool one_round = blocks >= 56 && blocks <= 64 && K < 8192;
+        *parts_out = *groups_out = 1;
+        if (blocks < 16 || blocks > 80 || stretches < 8) return 0;
+        parts = 8;
+        groups = one_round ? 2 : blocks <= 32 || (blocks % 32 == 0 && K >= 8192) ? 4 : 1;
+        while (groups > 1 && stretches < parts * groups) groups /= 2;
+        *parts_out = parts;
+        *groups_out = groups;
+        return 0;
+    }
     while (parts < 8 && blocks * parts < 512 && stretches / (parts * 8) >= 1) parts *= 2;
     // with more than 32 rows no more blocks than the chip holds at once (a long K: three a unit; the norm adds the slices of a short one)
     if (M > 32 && parts > 1 && blocks * parts > (K >= 8192 ? 768 : 512)) parts /= 2;
@@ -434,7 +451,7 @@ extern "C" int ri_gemm_rows_bf16(const void* A, int lda, const void* W, void* C,
     return 0;
 }
 
-// The q/k/v projection of 17..64 tokens with rotation and cache write in the epilogue, as
+// The q/k/v projection of 9..64 tokens with rotation and cache write in the epilogue, as
 // ri_gemm_qkv_rope (gemm.hip) does it for fewer rows: W is the same row-permuted weight in tile
 // order, C [M, ldc] receives rotated q in its first H * hd columns.  Measured at 64 rows against
 // the few-row kernel (product alone, us): 6144 x 4096 25.9 -> 21.5, 5120 x 3072 21.1 -> 16.5,
@@ -449,7 +466,7 @@ extern "C" int ri_gemm_rows_qkv_rope(const void* A, int lda, const void* W, void
                                      const int* positions, const int* row_of_token, void* kc, void* vc,
                                      int num_pages, const int* table, int max_blocks, int page, hipStream_t stream) {
     const int N = (H + 2 * Hkv) * hd;
-    RI_REQUIRE(M >= 17 && M <= 64, "ri_gemm_rows_qkv_rope: M=%d not in [17, 64]", M);
+    RI_REQUIRE(M >= 9 && M <= 64, "ri_gemm_rows_qkv_rope: M=%d not in [9, 64]", M);
     RI_REQUIRE(H > 0 && Hkv > 0 && hd > 0 && hd % 16 == 0 && K > 0 && K % 32 == 0, "ri_gemm_rows_qkv_rope: needs head size %% 16 == 0 and K %% 32 == 0 (hd=%d K=%d)", hd, K);
     RI_REQUIRE(lda >= K && lda % 8 == 0 && ldc >= H * hd, "ri_gemm_rows_qkv_rope: bad leading dimensions");
     RI_REQUIRE(page > 0 && max_blocks > 0 && num_pages > 0 && table_rows > 0, "ri_gemm_rows_qkv_rope: bad cache sizes");
@@ -461,7 +478,8 @@ extern "C" int ri_gemm_rows_qkv_rope(const void* A, int lda, const void* W, void
     const bf16_t* w = (const bf16_t*)W;
     const int groups = (N / 16 + 1) / 2 <= 256 ? 4 : 2;
     int rc;
-    if (M <= 32) rc = launch_rows_rope_groups<2>(a, lda, w, (bf16_t*)C, ldc, M, N, K, groups, rp, stream);
+    if (M <= 16) rc = launch_rows_rope_groups<1>(a, lda, w, (bf16_t*)C, ldc, M, N, K, groups, rp, stream);
+    else if (M <= 32) rc = launch_rows_rope_groups<2>(a, lda, w, (bf16_t*)C, ldc, M, N, K, groups, rp, stream);
     else if (M <= 48) rc = launch_rows_rope_groups<3>(a, lda, w, (bf16_t*)C, ldc, M, N, K, groups, rp, stream);
     else rc = launch_rows_rope_groups<4>(a, lda, w, (bf16_t*)C, ldc, M, N, K, groups, rp, stream);
     if (rc) return rc;

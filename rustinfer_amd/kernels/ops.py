@@ -342,6 +342,7 @@ def qkv_rope_fused(x: torch.Tensor, w_fused: torch.Tensor, qkv: torch.Tensor, H:
     if cos.dtype != torch.float32 or cos.shape != sin.shape or cos.shape[1] * 2 != hd or not cos.is_contiguous():
         raise KernelError("qkv_rope_fused: cos/sin must be contiguous float32 [positions, head_dim/2]")
     lds_rows = (M >= QKV_ROPE_LDS_MIN_ROWS and N >= QKV_ROPE_LDS_MIN_COLUMNS) or (M >= ROWS_LDS_MIN_ROWS and N * K >= QKV_ROPE_LDS_LARGE)
+    lds_rows = lds_rows or (QKV_ROPE_LDS_FEW_ROWS <= M <= 16 and N * K >= QKV_ROPE_LDS_LARGE and (N <= 8192 or M >= 12))
     if scale is None and lds_rows and K % 32 == 0 and hd % 16 == 0:
         # the kernel whose blocks share the activations through LDS
         _check(_lib().ri_gemm_rows_qkv_rope(
@@ -690,18 +691,24 @@ QKV_ROPE_LDS_LARGE = 14 << 20   # the fused q/k/v projection takes the LDS kerne
                                 # 17 and 32 tokens: 6144 x 4096 15.1 17.9 -> 14.7 15.7, 5120 x 3072 12.0 14.4 -> 11.0 12.3, 3072 x 2048 7.5 8.7 -> 8.0 8.7) ...
 QKV_ROPE_LDS_MIN_ROWS = 33      # ... and from 33 with this many columns (3072 x 2048 at 33, 48, 64 tokens: 9.6 11.2 13.4 -> 9.6 10.2 11.8; 1536 x 1024
 QKV_ROPE_LDS_MIN_COLUMNS = 3072 # 7.2 7.5 9.3 -> 7.2 7.6 8.8)
+QKV_ROPE_LDS_FEW_ROWS = 9       # tokens up to 16 from which it takes weights of QKV_ROPE_LDS_LARGE elements (of more than 8,192 columns: from 12): us, few-row kernel /
+                                # this at 9, 12, 16: 6144 x 4096 14.0 15.2 15.9 / 13.9 14.0 14.3, 5120 x 3072 11.0 11.8 12.4 / 10.7 10.9 11.3, 12288 x 4096 25.8 26.8 26.8 /
+                                # 25.4 25.6 25.2, 10240 x 8192 39.5 42.1 45.4 / 39.5 34.2 35.3; not 3072 x 2048 6.4 6.6 7.0 / 7.1 7.3 7.5
 ROWS_LDS_MIN_ROWS = 17          # from here to 64 rows, products whose partial sums a norm adds up take the LDS kernel
 ROWS_LDS_WIDE_COLUMNS = 16384   # whole products (no slices of K) take it from this many columns on: the output head, 250 -> 205 us at 64 rows
 
 
-def _swiglu_groups(I: int) -> int:
+def _swiglu_groups(I: int, M: int = 17) -> int:
     """Wave groups a block of the LDS kernel for a fused gate/up product of ``I`` columns (0: the few-row kernel does
     better).  4: blocks of 32 columns, 2: of 64; either takes the LDS of a whole compute unit, so its blocks should be most of
     256 and no more; 1: blocks of 64 columns and half that LDS, the form for more than 256 such
     blocks.  Measured, us, few-row kernel / this form at 17, 32, 48, 64 rows: 8192 x 2048 16.0 16.4 19.3 21.8 / 14.3 13.9 15.1 16.7; 8192 x
     3072 20.7 22.1 26.4 30.2 / 19.7 19.6 21.1 23.1; 11008 x 4096 39 41 54 61 / 35 36 38 39; 14336 x 4096 47 47 51 56 / 46 47 48 48; 9728 x 2560
-    27 31 37 43 / 23 23 25 27; 4864 x 896 7.9 9.0 11.1 13.3 / 6.7 7.0 8.2 9.1; not 3072 x 1024 (96 blocks) 7.3 7.8 9.0 10.6 / 9.2 8.9 10.4 11.6."""
+    27 31 37 43 / 23 23 25 27; 4864 x 896 7.9 9.0 11.1 13.3 / 6.7 7.0 8.2 9.1; not 3072 x 1024 (96 blocks) 7.3 7.8 9.0 10.6 / 9.2 8.9 10.4 11.6.
+    Up to 16 rows 4 for all that many blocks: 16 rows, 5632 x 2048 13.2 / 10.2, 8192 x 2048 14.6 / 13.6, 8192 x 3072 21.0 / 19.3, 14336 x 4096 43.8 / 41.6 (2 groups 46)."""
     b64, b32 = (I + 63) // 64, (I + 31) // 32
+    if M <= 16:
+        return 4 if b32 >= 128 else 0
     if 128 <= b32 <= 256:
         return 4
     if 154 <= b64 <= 256:
@@ -711,10 +718,33 @@ def _swiglu_groups(I: int) -> int:
     return 0
 
 
-def _rows_ok(x, w, w_tiled, M, N, K):
+def _rows_ok(x, w, w_tiled, M, N, K, min_rows=ROWS_LDS_MIN_ROWS):
     """Whether the kernel that shares a block's activations through LDS takes this product."""
-    return (not FORCE_LIBRARY_GEMM and w_tiled is not None and x.dtype == torch.bfloat16 and ROWS_LDS_MIN_ROWS <= M <= SKINNY_MAX_ROWS and N % 16 == 0
+    return (not FORCE_LIBRARY_GEMM and w_tiled is not None and x.dtype == torch.bfloat16 and min_rows <= M <= SKINNY_MAX_ROWS and N % 16 == 0
             and K % 32 == 0 and x.stride(0) % 8 == 0 and x.stride(1) == 1 and x.data_ptr() % 16 == 0 and _tiled_ok(w, w_tiled))
+
+
+def _rows_whole(M: int, N: int, K: int):
+    """(tiles a wave, wave groups a block) of the LDS kernel for a whole product, without slices of K; 0 tiles: the few-row kernel does as well.
+
+    Up to 16 rows: four groups of two waves, 32 columns a block, where the blocks are many, and from 8 rows on either at most one a compute unit or nearly twice that (two
+    share one).  us, few-row kernel / this at 8, 16 rows: 5120 x 2048 8.0 9.6 / 6.5 7.0; 6144 x 4096 13.8 17.0 / 12.7 12.9; 8192 x 2048 8.7 10.3 / 8.4 8.5; 16384 x 2048 14.9
+    18.0 / 13.7 13.8; 18448 x 2048 17.3 21.3 / 16.7 17.2; 14336 x 4096 25.0 31.1 / 24.4 25.0; from 12 rows 12288 x 4096 20.9 25.1 / 22.7 23.2; not 4096 x 2048 6.3 7.1 / 6.3 6.7, 1024 x
+    4096 7.5 8.9 / 8.4 8.8.  Wide ones of long rows: two tiles a wave (32000 x 4096 50 62 / 49 49, 24576 x 4096 37 47 / 35 35); the
+    output head not: 128256 x 2048 85 88 / 83 86, x 3072 119 126 / 117 123, x 4096 166 173 / 179 180.
+    From 17: blocks of 32 columns where they are at most one a unit, else of 64: 17, 33, 64 rows: 2048 x 2048 8.2 18.1 19.5 / 6.8 7.9 9.4; 8192 x 2048 10.1 19.1 20.6 / 8.9 9.8 11.1;
+    11264 x 2048 14.8 20.1 21.5 / 12.2 13.0 14.3; 14336 x 4096 27.2 36.8 37.6 / 27.3 27.0 28.5; 896 x 896 7.4 11.4 13.5 / 4.8 5.5 6.2.
+    Very wide ones (the output head): two tiles a wave halve what is asked for of the activations, but rows a power of two apart then meet on the same
+    channels of memory, which costs more where they are short or the rows few.  One / two tiles at 20, 40, 64 rows: 128256 x 3072 134 149 164 / 134 141 149, x 2048 96 101 111
+    / 108 113 115, x 4096 190 211 224 / 194 199 205, 151936 x 1536 87 103 114 / 87 94 103, 64000 x 5120 108 124 141 / 106 110 120."""
+    blocks = -(-N // 32)
+    if M <= 16:
+        if N < 5120 or M < 8 or N >= 65536 or (M < 12 and 256 < blocks < 448):
+            return 0, 0
+        return (2, 1) if N >= ROWS_LDS_WIDE_COLUMNS and K >= 4096 else (1, 4)
+    if N >= ROWS_LDS_WIDE_COLUMNS:
+        return (2 if K & (K - 1) or (K >= 4096 and M > 32) else 1), 1
+    return 1, 4 if blocks <= 256 else 2
 
 
 def _tiled_ok(w, w_tiled):
@@ -814,16 +844,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled=None,
     if M == 0:
         return
     lib = _lib()
-    if scale is None and N >= ROWS_LDS_WIDE_COLUMNS and out.dtype in (torch.bfloat16, torch.float32) \
-            and out.stride(0) % 4 == 0 and _rows_ok(x, w, w_tiled, M, N, K):
-        # 17..64 rows against a very wide matrix (the output head): activations shared through LDS.  Two tiles a wave halve what is asked for of
-        # the activations, but rows a power of two apart then meet on the same channels of memory, which costs more where they are short or the
-        # rows few.  Us, one / two tiles at 20, 40, 64 rows: 128256 x 3072 134 149 164 / 134 141 149, x 2048 96 101 111 / 108 113 115, x 4096
-        # 190 211 224 / 194 199 205, 151936 x 1536 87 103 114 / 87 94 103, 64000 x 5120 108 124 141 / 106 110 120.
-        tiles = 2 if K & (K - 1) or (K >= 4096 and M > 32) else 1
-        _check(lib.ri_gemm_rows_bf16(_ptr(x), x.stride(0), _ptr(w_tiled), _ptr(out), out.stride(0), M, N, K, _dt(out), 0, 1,
-                                     ctypes.c_longlong(0), tiles, 1, _stream()))
-        return
+    if scale is None and out.dtype in (torch.bfloat16, torch.float32) and out.stride(0) % 4 == 0 and _rows_ok(x, w, w_tiled, M, N, K, 8):
+        tiles, groups = _rows_whole(M, N, K)
+        if tiles:
+            _check(lib.ri_gemm_rows_bf16(_ptr(x), x.stride(0), _ptr(w_tiled), _ptr(out), out.stride(0), M, N, K, _dt(out), 0, 1,
+                                         ctypes.c_longlong(0), tiles, groups, _stream()))
+            return
     to_library = scale is None and out.dtype in (torch.bfloat16, torch.float32) and _untiled_to_library(x, w, w_tiled, M) \
         and (N, K, x.stride(0), w.stride(0), out.stride(0), out.dtype) not in _LIBRARY_REFUSED
     if x.dtype == torch.bfloat16 and not to_library:
@@ -877,7 +903,7 @@ def linear_activated(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tile
     left in ``out``).  Few bfloat16 rows: in the product's own epilogue, on sums that have not been rounded."""
     M, K = x.shape
     N = w.shape[0]
-    lds = N >= ROWS_LDS_WIDE_COLUMNS and out.stride(0) % 4 == 0 and _rows_ok(x, w, w_tiled, M, N, K)      # as `linear` routes it
+    lds = N >= ROWS_LDS_WIDE_COLUMNS and out.stride(0) % 4 == 0 and _rows_ok(x, w, w_tiled, M, N, K)      # wide enough that the activations' own kernels cost less
     if 0 < len(acts) <= 2 and not lds and _skinny_ok(x, w, M, K) and _tiled_ok(w, w_tiled) and N % 16 == 0 and K % 32 == 0 \
             and out.dtype == torch.bfloat16 and all(c0 % 16 == 0 and n % 16 == 0 and dst.dtype == torch.bfloat16 for c0, n, _, dst in acts):
         _dev(x, w, out, *(dst for _, _, _, dst in acts))
@@ -913,8 +939,8 @@ def linear_delta(x: torch.Tensor, w: torch.Tensor, workspace, name: str,
     if w.shape[1] != K or x.dtype != w.dtype:
         raise KernelError(f"linear_delta: shapes {tuple(x.shape)} x {tuple(w.shape)}^T or dtypes do not fit")
     lib = _lib()
-    if _rows_ok(x, w, w_tiled, M, N, K):
-        # 17..64 rows: the kernel that shares the activations of a block through LDS
+    if _rows_ok(x, w, w_tiled, M, N, K, 9):
+        # 9..64 rows (up to eight the copy in tile order gives what the weight itself does, to the bit): the kernel that shares the activations of a block through LDS
         parts, groups = ctypes.c_int(0), ctypes.c_int(0)
         _check(lib.ri_gemm_rows_plan(M, N, K, 1, ctypes.byref(parts), ctypes.byref(groups)))
         parts, groups = parts.value, groups.value
@@ -962,8 +988,8 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor,
         raise KernelError("linear_swiglu: shapes or dtypes do not fit")
     if M == 0:
         return
-    groups = _swiglu_groups(I)
-    if scale is None and groups and _rows_ok(x, w_gate_up, w_tiled, M, I, K):
+    groups = _swiglu_groups(I, M)
+    if scale is None and groups and _rows_ok(x, w_gate_up, w_tiled, M, I, K, 9):
         # many rows and blocks enough for the chip: activations shared through LDS
         _check(_lib().ri_gemm_rows_bf16(_ptr(x), x.stride(0), _ptr(w_tiled), _ptr(out), out.stride(0), M, I, K, BF16, 1, 1,
                                         ctypes.c_longlong(0), 1, groups, _stream()))

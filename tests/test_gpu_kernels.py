@@ -1265,7 +1265,7 @@ def _check_fused_projection(ops, B, H, Hkv, hd, page, K):
         assert np.all(np.abs(got[b, :H * hd].double().cpu().numpy() - want) <= 2.0 ** -8 * np.maximum(1.0, np.abs(want)))
 
 
-@pytest.mark.parametrize("M,K", [(17, 32), (32, 96), (33, 64), (48, 160), (49, 1056), (64, 2080), (20, 4128), (37, 8160)])
+@pytest.mark.parametrize("M,K", [(17, 32), (32, 96), (33, 64), (48, 160), (49, 1056), (64, 2080), (20, 4128), (37, 8160), (4, 32), (9, 96), (15, 1056), (16, 8160)])
 def test_products_of_some_rows_through_the_ring(ops, M, K):
     """Fewer stretches of 64 than groups and stages, an odd last step, 16 columns and edges of blocks; rows beside and beyond which all is NaN; every number of groups
     and slices: partial sums, gate/up, whole products of one and two tiles a wave."""
@@ -1300,6 +1300,47 @@ def test_products_of_some_rows_through_the_ring(ops, M, K):
     assert lib.ri_gemm_rows_bf16(p(x), x.stride(0), p(wt1), p(bad), N, M, N, K, ops.F32, 0, 1, ctypes.c_longlong(0), 1, 2, st) == 0
     rest = [i for i in range(M) if i != 3]
     assert torch.all((bad[rest].double() - ref[rest, :N]).abs() <= tol[rest, :N]) and not torch.isfinite(bad[3]).any()
+
+
+@pytest.mark.parametrize("M,N,K,delta,whole", [(9, 2048, 8192, (8, 4), None), (12, 1024, 544, (8, 1), None), (16, 3072, 1056, (8, 1), None), (8, 2048, 2048, None, None),
+                                               (9, 4096, 2080, (8, 2), None), (16, 5136, 2048, None, (1, 4)), (7, 5120, 512, None, None), (8, 5120, 512, None, (1, 4)),
+                                               (10, 5120, 512, (8, 1), (1, 4)), (10, 960, 1024, None, None),
+                                               (11, 8208, 256, None, None), (12, 8208, 256, None, (1, 4)), (9, 16400, 4128, None, (2, 1)), (17, 272, 96, None, (1, 4)),
+                                               (64, 8208, 160, None, (1, 2))])
+def test_where_products_take_the_ring(ops, monkeypatch, M, N, K, delta, whole):
+    """Slices for a norm, whole products and gate/up on both sides of the lines between the kernels, against 64-bit sums."""
+    lib, taken, entry = ops._lib(), [], ops._lib().ri_gemm_rows_bf16
+    monkeypatch.setattr(lib, "ri_gemm_rows_bf16", lambda *a: taken.append((a[10], a[12], a[13])) or entry(*a))
+    x = rnd(M, K, dtype=torch.bfloat16, seed=1)
+    w = rnd(N, K, dtype=torch.bfloat16, seed=2, scale=0.1)
+    wt, ws = ops.tile_weight(w), Workspace(torch.device(DEV))
+    ref = x.double() @ w.double().t()
+    tol = K * 2.0 ** -23 * ((x.double() ** 2) @ (w.double() ** 2).t()).sqrt()      # as for the ring itself
+    out = torch.full((M, N), float("nan"), device=DEV)
+    ops.linear(x, w, out, wt)
+    assert taken == ([(1,) + whole] if whole else [])
+    assert torch.all((out.double() - ref).abs() <= tol)
+    if M <= 16:
+        taken.clear()
+        got = ops.linear_delta(x, w, ws, "t", wt, torch.float32)
+        assert taken == ([(delta[0], 1, delta[1])] if delta else [(1,) + whole] if whole and got.dim() == 2 else [])
+        assert torch.all(((got.double().sum(0) if got.dim() == 3 else got.double()) - ref).abs() <= tol)
+    half = N // 2 // 16 * 16
+    gu, act = w[:2 * half].contiguous(), torch.full((M, half), float("nan"), dtype=torch.bfloat16, device=DEV)
+    taken.clear()
+    ops.linear_swiglu(x, gu, act, None, ops.tile_weight(gu))
+    assert len(taken) == (M >= 9 and half >= 4096)
+    want = torch.nn.functional.silu(ref[:, :half]) * ref[:, half:2 * half]
+    assert torch.all((act.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4 * want.abs().max())
+
+
+@pytest.mark.parametrize("B,H,Hkv,hd,K", [(9, 32, 8, 128, 2400), (16, 24, 8, 128, 3072), (12, 70, 10, 128, 1536)])
+def test_fused_projection_of_up_to_sixteen_tokens_through_the_ring(ops, monkeypatch, B, H, Hkv, hd, K):
+    lib, taken = ops._lib(), []
+    entry = lib.ri_gemm_rows_qkv_rope
+    monkeypatch.setattr(lib, "ri_gemm_rows_qkv_rope", lambda *a: taken.append(1) or entry(*a))
+    _check_fused_projection(ops, B, H, Hkv, hd, 64, K)
+    assert taken == [1]
 
 
 @pytest.mark.parametrize("M,N,K", [(1, 16, 32), (8, 48, 96), (3, 2048, 2048), (8, 2048, 2080), (7, 1024, 4128), (4, 3072, 3104), (2, 4096, 1056),
