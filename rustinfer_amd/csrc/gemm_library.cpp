@@ -304,6 +304,19 @@ int rows_of_whole_rounds(int M, int N) {
     return whole >= 2 * round && M > whole && (long long)(M - whole) * 5 <= 4ll * round ? whole : 0;
 }
 
+// The same for columns, where the tiles of the rows divide a round (and are nearly full): what is left may be two fifths of a round after one, half of
+// one after more, and more than two thirds after two, of which the library makes the least.  us, one call / two: 2,048 rows x 2048 9,216 columns 83 / 68, 11,264 84 / 80, 16,624
+// 163 / 115, 18,448 195 / 133, 20,480 158 / 131, 23,552 221 / 145, 24,816 233 / 165, 28,672 184 / 182; x 4096 9,216 138 / 120, 19,456 349 / 231, 22,016 402 / 259, 28,672
+// 341 / 335; 1,024 rows x 4096 18,448 141 / 132, 34,832 342 / 225; 512 rows 33,744 148 / 122, 77,824 350 / 263; 8,192 rows x 2048 2,304 80 / 69, 5,120 148 / 126.  Not 13,312 (87 / 93), 21,504
+// (136 / 140), 29,696 (187 / 191), nor one round in 32 bits (2,048 rows x 2048 10,240 82 / 85).
+int columns_of_whole_rounds(int M, int N, int out_f32) {
+    const int mt = (M + 255) / 256;
+    if (mt < 2 || mt > 32 || 256 % mt || M * 8 < mt * 256 * 7) return 0;
+    const int round = 65536 / mt, rounds = N / round, rest = N - rounds * round;
+    if (!rest || !rounds || (rounds == 1 && (out_f32 || rest * 5 > round * 2))) return 0;
+    return rest * 2 <= round || (rounds == 2 && rest * 16 >= round * 11) ? rounds * round : 0;
+}
+
 }  // namespace
 
 // workspace: device memory the library may use (split products); the same size must be passed
@@ -325,6 +338,11 @@ extern "C" int ri_gemm_library_bf16(const void* A, int lda, const void* W, int l
         if (int rc = product(A, lda, W, ldw, C, ldc, first, N, K, out_f32, workspace, workspace_bytes, stream)) return rc;
         A = (const char*)A + (size_t)first * lda * 2;
         C = (char*)C + (size_t)first * ldc * (out_f32 ? 4 : 2);
+    } else if (const int columns = g_tune ? 0 : columns_of_whole_rounds(M, N, out_f32)) {
+        if (int rc = product(A, lda, W, ldw, C, ldc, M, columns, K, out_f32, workspace, workspace_bytes, stream)) return rc;
+        W = (const char*)W + (size_t)columns * ldw * 2;
+        C = (char*)C + (size_t)columns * (out_f32 ? 4 : 2);
+        N -= columns;
     }
     return product(A, lda, W, ldw, C, ldc, M - first, N, K, out_f32, workspace, workspace_bytes, stream);
 }
@@ -354,7 +372,8 @@ extern "C" int ri_gemm_library_reset() {
     return 0;
 }
 
-// For a test: see rows_of_whole_rounds.
+// For a test: see rows_of_whole_rounds and columns_of_whole_rounds.
+extern "C" int ri_gemm_library_first_columns(int M, int N, int out_f32) { return columns_of_whole_rounds(M, N, out_f32); }
 extern "C" int ri_gemm_library_first_rows(int M, int N) { return rows_of_whole_rounds(M, N); }
 
 // (shapes kept, questions put to the library's heuristic so far)

@@ -306,6 +306,25 @@ def test_library_gemm_of_whole_rounds_and_the_rest(ops, M, N, f32, first):
     assert torch.isnan(out[:, N:]).all()
 
 
+@pytest.mark.parametrize("M,N,f32,first", [(2048, 8208, 0, 8192), (1793, 11456, 0, 8192), (1792, 11456, 0, 0), (2000, 18448, 1, 16384), (2048, 11600, 0, 0), (2048, 8208, 1, 0),
+                                           (512, 33000, 0, 32768), (448, 33000, 0, 32768), (447, 33000, 0, 0), (1024, 44096, 0, 32768), (1024, 42000, 0, 0), (8192, 2300, 0, 2048)])
+def test_library_gemm_of_whole_rounds_of_columns(ops, M, N, f32, first):
+    """Columns that make whole rounds of tiles likewise."""
+    K = 128
+    assert ops._lib().ri_gemm_library_first_rows(M, N) == 0 and ops._lib().ri_gemm_library_first_columns(M, N, f32) == first
+    xb = rnd(M, K + 8, dtype=torch.bfloat16, seed=1)
+    x, w = xb[:, :K], rnd(N, K, dtype=torch.bfloat16, seed=2, scale=0.1)
+    out = torch.full((M, N + 8), float("nan"), dtype=torch.float32 if f32 else torch.bfloat16, device=DEV)
+    ws = torch.empty(64 << 20, dtype=torch.uint8, device=DEV)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    assert ops._lib().ri_gemm_library_bf16(p(x), K + 8, p(w), K, p(out), N + 8, M, N, K, f32, p(ws), ctypes.c_size_t(ws.numel()),
+                                           ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+    ref = x.float() @ w.float().t()
+    # one rounding to bfloat16, or a sum of 128 products in 32 bits
+    assert torch.all((out[:, :N].float() - ref).abs() <= (2.0 ** -8 * ref.abs() if not f32 else 0) + 2.0 ** -16 * ref.abs().max())
+    assert torch.isnan(out[:, N:]).all()
+
+
 def test_library_gemm_with_a_tuned_kernel(ops, tmp_path):
     """With tuning on, a product of more than 64 rows times the library's kernels once for its row
     bucket, keeps the choice in a file, and gives the same result (to bfloat16 rounding) as before."""
