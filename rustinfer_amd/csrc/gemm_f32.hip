@@ -15,7 +15,7 @@
 // Blocks of one column tile run on one XCD (consecutive block ids go around the eight of them), so a
 // tile's weights pass through one L2.  K % 4 == 0, rows 16-byte aligned.
 //
-// What is left to bound the large products: other instructions hold the 64-bit matrix instruction up (a loop of it alone reaches 72
+// (Prompts of 24 rows or more go to gemm_digits.hip where the weight's digits are laid out.)  What is left to bound the large products: other instructions hold the 64-bit matrix instruction up (a loop of it alone reaches 72
 // TFLOP/s on random operands, one with the widening of one operand value an instruction, as in tiles of 32 x 32, 61),
 // and that is what they take.  Loads waited for under conditions of the lanes before, now, us: 600 rows of 16384 x 2048 707, 662
 // (61 TFLOP/s), of 2048 x 8192 364, 333, of 2048 x 2048 100, 93; 230 rows 268, 250 / 154, 137 / 44, 39; 37 rows of
