@@ -21,6 +21,8 @@
 // (61 TFLOP/s), of 2048 x 8192 364, 333, of 2048 x 2048 100, 93; 230 rows 268, 250 / 154, 137 / 44, 39; 37 rows of
 // 16384 x 2048 67, 60; 13 rows 43, 37.  (As FMA kernels with 64-bit sums: 600 rows of 2048 x 8192 1451.)
 #include "common.h"
+#include <algorithm>
+#include <type_traits>
 
 extern "C" int ri_gemm_tiled(const void* A, int lda, const void* W, int ldw, void* C, int ldc,
                              int M, int N, int K, int in_dtype, int out_dtype, hipStream_t stream);      // gemm.hip
@@ -32,24 +34,41 @@ typedef double f64x4_t __attribute__((ext_vector_type(4)));
 // MT x NT tiles of 16 x 16 results a block, WAVES waves that share K, chunks of 16 U values of K (U = 1: two of them, one
 // after the other, are a wave's turn of 32).
 // STREAM: W is read once (a single row of tiles), past the caches.
-template <int MT, int NT, int WAVES, int U, bool STREAM>
+// LISTED: of the rows of A and C only those whose numbers stand in list[1] and on, list[0] of them, which the launch does not know: as many blocks as the chip
+// holds take their tiles in turn (an empty list 2 us, where a block for each tile of 600 rows of 16384 columns took 6).
+template <int MT, int NT, int WAVES, int U, bool STREAM, bool LISTED = false>
 __global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
         const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
-        float* __restrict__ C, int ldc, int M, int N, int K, int mtiles, int ntiles) {
+        float* __restrict__ C, int ldc, int M, int N, int K, int mtiles, int ntiles, const int* __restrict__ list = nullptr) {
     constexpr int KC = 16 * U, TURN = WAVES * 32;
     static_assert(U == 1 || U == 2, "a wave's turn of K is 32 values");
     __shared__ double sums[WAVES][16][NT * 16];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    const int xcd = (int)blockIdx.x & 7, turn = (int)blockIdx.x >> 3;
+    if (LISTED) {
+        M = list[0];
+        mtiles = (M + MT * 16 - 1) / (MT * 16);
+    }
+    for (int id = (int)blockIdx.x;; id += (int)gridDim.x) {
+    if (LISTED && id >= (ntiles + 7) / 8 * 8 * mtiles) return;
+    const int xcd = id & 7, turn = id >> 3;
     const int nt = (turn / mtiles) * 8 + xcd, mt = turn % mtiles;
-    if (nt >= ntiles) return;
+    if (nt >= ntiles) {
+        if (LISTED) continue;
+        return;
+    }
     const int m0 = mt * MT * 16, n0 = nt * NT * 16;
-    // the block's first rows, the same in all lanes, and each lane's rows as 32-bit distances in bytes from there
-    const char* abase = reinterpret_cast<const char*>(A + (size_t)m0 * lda);
+    // the block's first rows, the same in all lanes, and each lane's rows as 32-bit distances in bytes from there (listed rows, which may lie
+    // anywhere, as 64-bit ones from the first of all)
+    const char* abase = reinterpret_cast<const char*>(LISTED ? A : A + (size_t)m0 * lda);
     const char* wbase = reinterpret_cast<const char*>(W + (size_t)n0 * ldw);
-    uint32_t arow[MT], wrow[NT];
+    typename std::conditional<LISTED, size_t, uint32_t>::type arow[MT];
+    uint32_t wrow[NT];
 #pragma unroll
-    for (int i = 0; i < MT; ++i) arow[i] = ((uint32_t)min(i * 16 + r, M - 1 - m0) * (uint32_t)lda + 4 * g) * 4;
+    for (int i = 0; i < MT; ++i) {
+        const int row = min(i * 16 + r, M - 1 - m0);
+        if constexpr (LISTED) arow[i] = ((size_t)list[1 + m0 + row] * lda + 4 * g) * 4;
+        else arow[i] = ((uint32_t)row * (uint32_t)lda + 4 * g) * 4;
+    }
 #pragma unroll
     for (int j = 0; j < NT; ++j) wrow[j] = ((uint32_t)min(j * 16 + r, N - 1 - n0) * (uint32_t)ldw + 4 * g) * 4;
     auto of_a = [&](int i, int k) { return *reinterpret_cast<const float4*>(abase + (size_t)k * 4 + arow[i]); };
@@ -147,8 +166,11 @@ __global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
 #pragma unroll
             for (int w = 1; w < WAVES; ++w) v += sums[w][row][col];
             const int m = m0 + i * 16 + row, n = n0 + col;
-            if (m < M && n < N) C[(size_t)m * ldc + n] = (float)v;
+            if (m < M && n < N) C[(size_t)(LISTED ? list[1 + m] : m) * ldc + n] = (float)v;
         }
+    }
+    if (!LISTED) return;
+    __syncthreads();
     }
 }
 
@@ -304,6 +326,27 @@ static void launch_f32(const float* A, int lda, const float* W, int ldw, float* 
         if (mtiles == 1) gemm_f32_kernel<MT, NT, 8, U, true><<<across, 512, 0, stream>>>(a, lda, W, ldw, c, ldc, m, N, K, mtiles, ntiles);
         else gemm_f32_kernel<MT, NT, 8, U, false><<<across * mtiles, 512, 0, stream>>>(a, lda, W, ldw, c, ldc, m, N, K, mtiles, ntiles);
     }
+}
+
+// The rows of A[M, K] and C[M, N] whose numbers stand in list[1] and on, list[0] of them (on the device, 0 to M): what ri_gemm_f32 gives for them, in the tiles that it
+// takes for M rows.
+extern "C" int ri_gemm_f32_listed(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K,
+                                  const int* list, hipStream_t stream) {
+    RI_REQUIRE(M >= 1 && N > 0 && K > 0 && K % 4 == 0 && lda >= K && ldw >= K && ldc >= N && lda % 4 == 0 && ldw % 4 == 0 && ldw <= (1 << 24),
+               "ri_gemm_f32_listed: needs rows, K %% 4 == 0 and leading dimensions >= K and multiples of 4 (M=%d N=%d K=%d)", M, N, K);
+    RI_REQUIRE(A && W && C && list && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0, "ri_gemm_f32_listed: null or unaligned pointer");
+    RI_REQUIRE((long long)M * ((N + 15) / 16 + 7) < (1ll << 31), "ri_gemm_f32_listed: M=%d N=%d exceed the grid limit", M, N);
+    const F32Tile& t = F32_TILES[f32_tile(M, N)];
+    const int mtiles = (M + 16 * t.mt - 1) / (16 * t.mt), ntiles = (N + 16 * t.nt - 1) / (16 * t.nt), blocks = std::min((ntiles + 7) / 8 * 8 * mtiles, 512);
+    switch (f32_tile(M, N)) {
+        case 0: gemm_f32_kernel<2, 2, 8, 2, false, true><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles, list); break;
+        case 1: gemm_f32_kernel<3, 2, 8, 1, false, true><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles, list); break;
+        case 2: gemm_f32_kernel<2, 1, 8, 2, false, true><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles, list); break;
+        case 3: gemm_f32_kernel<1, 2, 8, 2, false, true><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles, list); break;
+        default: gemm_f32_kernel<1, 1, 8, 2, false, true><<<blocks, 512, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles, list); break;
+    }
+    RI_LAUNCHED("ri_gemm_f32_listed");
+    return 0;
 }
 
 // The rows and columns of the tile that ri_gemm_f32 takes for M rows and N columns (of gemm_f32_kernel: up to eight rows, the tiles

@@ -623,20 +623,19 @@ def swiglu(gate_up: torch.Tensor, out: torch.Tensor) -> None:
 
 
 class DigitWeight:
-    """A 32-bit weight as whole numbers of five 8-bit digits and an exponent a row (csrc/gemm_digits.hip)."""
+    """A 32-bit weight as whole numbers of five 8-bit digits, and what is known of each row: exponent and norms (csrc/gemm_digits.hip)."""
 
     def __init__(self, w: torch.Tensor):
         N, K = w.shape
         lib = _lib()
         lib.ri_digits_bytes.restype = ctypes.c_longlong
         self.shape, self.device = (N, K), w.device
-        self.planes = torch.empty(int(lib.ri_digits_bytes(N, K)), dtype=torch.uint8, device=w.device)
-        self.exps = torch.empty(N, dtype=torch.int32, device=w.device)
-        _check(lib.ri_digits_split(_ptr(w), w.stride(0), N, K, 0, _ptr(self.planes), _ptr(self.exps), _stream()))
-        self.whole = not bool((self.exps == NO_DIGITS).any())       # every row has digits
+        self.planes = torch.empty(int(lib.ri_digits_bytes(N, K, 5)), dtype=torch.uint8, device=w.device)
+        self.known = torch.empty((N, 8), dtype=torch.float32, device=w.device)
+        _check(lib.ri_digits_split(_ptr(w), w.stride(0), N, K, 5, _ptr(self.planes), _ptr(self.known), ctypes.c_void_p(0), 0, _stream()))
+        self.whole = not bool(torch.isinf(self.known[:, 0]).any())       # every row has digits (none is not finite, or spreads too far)
 
 
-NO_DIGITS = -(1 << 31)              # in the place of a row's exponent: not finite, or values that spread too far
 DIGITS_MIN_WEIGHTS = 1 << 19        # smaller weights never pay for digits (ri_gemm_digits_plan)
 
 
@@ -649,7 +648,7 @@ def _digits_shape(w: torch.Tensor) -> bool:
 def tiled_bytes(w: torch.Tensor) -> int:
     """Bytes that ``tile_weight(w)`` takes, if there is such a copy."""
     N, K = w.shape
-    return N * K * 5 + 4 * N if w.dtype == torch.float32 else w.numel() * w.element_size()
+    return N * K * 5 + 32 * N if w.dtype == torch.float32 else w.numel() * w.element_size()
 
 
 def tile_weight(w: torch.Tensor):
@@ -804,24 +803,25 @@ def gemm_tuned_shapes() -> int:
 
 def _digits_parts(x: torch.Tensor, w: torch.Tensor, w_tiled, M: int, N: int, K: int) -> int:
     """Slices of K in which the product goes through digits, 0 if it does not."""
-    if not isinstance(w_tiled, DigitWeight) or x.dtype != torch.float32 or x.stride(0) % 4 or x.data_ptr() % 16:
+    if not isinstance(w_tiled, DigitWeight) or x.dtype != torch.float32 or x.stride(0) % 4 or x.data_ptr() % 16 or x.stride(0) > 1 << 24 or w.stride(0) > 1 << 24:
         return 0
     if w_tiled.shape != (N, K) or w.dtype != torch.float32 or w_tiled.device != w.device:
         raise KernelError("the weight's digits do not belong to the weight")
     return int(_lib().ri_gemm_digits_plan(M, N, K))
 
 
-def _linear_digits(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: DigitWeight, workspace, parts: int, gate: int = 0) -> None:
-    """``out[M, N]`` from the digits of ``x[:, :K]``, with ``gate`` of ``silu(x[:, :K]) * x[:, gate : gate + K]``."""
+def _linear_digits(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled: DigitWeight, workspace, parts: int) -> None:
+    """``out[M, N]`` from the digits of ``x`` and of the weight, and from 64-bit sums where they do not hold it."""
     lib = _lib()
     M, (N, K) = x.shape[0], w_tiled.shape
     rows = (M + 31) // 32 * 32
-    planes = workspace.get("digits.planes", rows, 5 * K, torch.uint8)
-    exps = workspace.get("digits.exps", rows, 1, torch.int32)
-    sums = workspace.get("digits.sums", parts * M, N, torch.int64) if parts > 1 else None
-    _check(lib.ri_digits_split(_ptr(x), x.stride(0), M, K, gate, _ptr(planes), _ptr(exps), _stream()))
-    _check(lib.ri_gemm_digits(_ptr(planes), _ptr(exps), _ptr(x), x.stride(0), gate, _ptr(w_tiled.planes), _ptr(w_tiled.exps),
-                              _ptr(w), w.stride(0), _ptr(out), out.stride(0), _ptr(sums) if parts > 1 else ctypes.c_void_p(0), parts,
+    planes = workspace.get("digits.planes", rows, 6 * K, torch.uint8)
+    known = workspace.get("digits.known", rows, 8, torch.float32)
+    again = workspace.get("digits.again", M + 1, N // 32 + 2, torch.int32)       # what is computed again: csrc/gemm_digits.hip
+    sums = workspace.get("digits.sums", parts * M, N, torch.float64) if parts > 1 else None
+    _check(lib.ri_digits_split(_ptr(x), x.stride(0), M, K, 6, _ptr(planes), _ptr(known), _ptr(again), N, _stream()))
+    _check(lib.ri_gemm_digits(_ptr(planes), _ptr(known), _ptr(x), x.stride(0), _ptr(w_tiled.planes), _ptr(w_tiled.known),
+                              _ptr(w), w.stride(0), _ptr(out), out.stride(0), _ptr(sums) if parts > 1 else ctypes.c_void_p(0), parts, _ptr(again),
                               M, N, K, _stream()))
 
 
@@ -1019,24 +1019,6 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor,
         return
     linear(x, w_gate_up, scratch, w_tiled if isinstance(w_tiled, DigitWeight) else None, workspace=workspace)
     swiglu(scratch, out)
-
-
-def linear_swiglu_delta(x: torch.Tensor, w_gate_up: torch.Tensor, gate_up_tiled, w_down: torch.Tensor, down_tiled, scratch: torch.Tensor,
-                        workspace, name: str) -> Optional[torch.Tensor]:
-    """``(silu(x @ gate^T) * (x @ up^T)) @ down^T`` of a float32 portion whose products go through digits: the activation is
-    computed where the second product's digits are made.  ``scratch [M, 2I]``.  None, and nothing done, where they do not."""
-    M, K = x.shape
-    D, I = w_down.shape
-    if x.dtype != torch.float32 or w_gate_up.shape != (2 * I, K) or tuple(scratch.shape) != (M, 2 * I) or not scratch.is_contiguous():
-        return None
-    parts = _digits_parts(scratch, w_down, down_tiled, M, D, I)
-    if not parts:
-        return None
-    _dev(x, w_gate_up, w_down, scratch)
-    linear(x, w_gate_up, scratch, gate_up_tiled, workspace=workspace)
-    out = workspace.get(name, M, D, torch.float32)
-    _linear_digits(scratch, w_down, out, down_tiled, workspace, parts, gate=I)
-    return out
 
 
 def argmax(logits: torch.Tensor, out: torch.Tensor) -> None:

@@ -57,16 +57,8 @@ class SwiGLUMLP(FeedForward):
         return act
 
     def forward(self, ctx, normed) -> torch.Tensor:
-        ops, ws = self.rt.ops, ctx.workspace
-        rows, scale = split_normed(normed)
-        both = getattr(ops, "linear_swiglu_delta", None)
-        if both is not None and scale is None and self.rt.dtype == torch.float32:
-            scratch = ws.get("ffn.gate_up", rows.shape[0], 2 * self.intermediate_size, torch.float32)
-            delta = both(rows, self.gate_up.weight, self.gate_up.weight_tiled, self.down.weight, self.down.weight_tiled, scratch, ws, "ffn.out")
-            if delta is not None:
-                return delta
         act = self._activation(ctx, normed)
-        return ops.linear_delta(act, self.down.weight, ctx.workspace, "ffn.out", self.down.weight_tiled,
+        return self.rt.ops.linear_delta(act, self.down.weight, ctx.workspace, "ffn.out", self.down.weight_tiled,
                                         out_dtype=self.delta_dtype)
 
     def forward_into(self, ctx, normed, x: torch.Tensor, next_norm):

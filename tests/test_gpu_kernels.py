@@ -542,14 +542,11 @@ def test_swiglu_f32_of_up_to_eight_rows_is_the_product_and_the_activation(ops, M
     assert torch.equal(out[:, :I], want) and torch.isnan(out[:, I:]).all()
 
 
-# Digits (gemm_digits): each value of a row is within 2^-40 of the row's largest a (half a unit of 40 bits, of which one may
-# be lost to the first digit's range), so K (2^-40 a |w| + 2^-40 w |a|); the products left out, four of digits 0 to 3 with i + j = 3 and what is
-# below them, are at most 4.02 x 2^14 x 256^3 units of 2^-78 (a w times at most 4.1): under 2^-36 K a w.  Signs of both are random: a 64th of the sum of bounds.
-def _digits_bound(x, w):
-    a, b = x.double().abs(), w.double().abs()
-    K = x.shape[1]
-    am, bm = a.amax(1, keepdim=True), b.amax(1)[None]
-    return 2.0 ** -40 * (am * b.sum(1)[None] + bm * a.sum(1, keepdim=True)) + 2.0 ** -36 * K * am * bm
+# Digits (gemm_digits): whatever the rows hold, a result is rounded once (half a unit of the last place, of the least of them for results below the
+# normal numbers) and is within 2^-27 of itself, or is a 64-bit sum, as the reference here: K 2^-52 of the sum of magnitudes for both.
+def _digits_bound(x, w, ref):
+    mag = x.double().abs() @ w.double().abs().t()
+    return ref.abs() * (2.0 ** -24 + 2.0 ** -27) + 2.0 ** -150 + x.shape[1] * 2.0 ** -52 * mag
 
 
 @pytest.mark.parametrize("M,N,K", [(24, 1024, 1024), (33, 3072, 2048), (64, 2080, 4096), (65, 4128, 1056), (129, 544, 9120), (100, 992, 14336), (300, 2048, 25984), (193, 8192, 288)])
@@ -580,9 +577,7 @@ def test_linear_f32_from_digits(ops, M, N, K):
     few = torch.empty(M - 20, N, device=DEV)
     ops._linear_digits(x[20:].contiguous(), w, few, wt, ws, 1)
     assert torch.equal(few, outs[0][20:])
-    # rounded once: half a unit of the last place, of the least of them for results below the normal numbers
-    err = (outs[0].double() - ref).abs()
-    assert torch.all(err <= ref.abs() * 2.0 ** -24 + 2.0 ** -150 + _digits_bound(x, w))
+    assert torch.all((outs[0].double() - ref).abs() <= _digits_bound(x, w, ref))
     rows = [i for i in range(M) if i not in (3, 5)]
     plain = torch.empty(M, N, device=DEV)
     ops.linear(x, w, plain)
@@ -619,39 +614,65 @@ def test_linear_f32_rows_without_digits(ops):
     assert ops.tile_weight(w2) is None and ops.tile_weight(w[:, :2046]) is None and ops.tile_weight(w[:2047]) is None
 
 
-@pytest.mark.parametrize("M,I,K", [(40, 1024, 2048), (130, 8192, 1024), (64, 2720, 1056), (33, 14336, 512)])
-def test_swiglu_mlp_f32_from_digits(ops, M, I, K):
-    """The activation where the second product's digits are made: no further from 64 bits than the activation's own kernel, in whole products
-    and slices the same bits; a row that is not finite, one whose activation passes the 32-bit range, and one by 64-bit sums."""
+@pytest.mark.parametrize("M,N,K,bad", [(600, 4128, 256, 600), (100, 8224, 288, 37), (24, 2048, 1056, 1)])
+def test_linear_f32_rows_without_digits_are_those_of_64_bit_sums(ops, M, N, K, bad):
+    """More tiles of listed rows than blocks, a last tile of them that is not full, a single one: to the bit what the kernel of 64-bit sums gives."""
     from rustinfer_amd.engine.context import Workspace
-    D = 1024
-    x, wgu, wd = rnd(M, K, seed=1), rnd(2 * I, K, seed=2) * 0.05, rnd(D, I, seed=3) * 0.02
-    tgu, td, ws = ops.tile_weight(wgu), ops.tile_weight(wd), Workspace(torch.device(DEV))
-    scratch, act, old = torch.empty(M, 2 * I, device=DEV), torch.empty(M, I, device=DEV), torch.empty(M, D, device=DEV)
-    ops.linear(x, wgu, scratch, tgu, workspace=ws)
-    scratch[1, 5] = float("nan")
-    scratch[2, 7], scratch[2, I + 7] = 1e20, 1e20
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2)
     g = torch.Generator().manual_seed(3)
-    scratch[3, I:] = (torch.randn(I, generator=g) * 2.0 ** torch.randint(-60, 61, (I,), generator=g)).to(DEV)
-    ops.swiglu(scratch, act)
-    ops._linear_digits(act, wd, old, td, ws, 1)
-    z = scratch.double()
-    ref = (torch.nn.functional.silu(z[:, :I]) * z[:, I:]) @ wd.double().t()
-    outs = []
+    rows = torch.randperm(M, generator=g)[:bad]
+    x[rows.to(DEV)] *= (2.0 ** torch.randint(-60, 61, (bad, K), generator=g).float()).to(DEV)
+    wt, ws = ops.DigitWeight(w), Workspace(torch.device(DEV))
+    want, out = torch.empty(M, N, device=DEV), torch.full((M, N + 4), float("nan"), device=DEV)
+    ops.linear(x, w, want)
     for parts in (1, 3):
-        outs.append(torch.full((M, D), float("nan"), device=DEV))
-        ops._linear_digits(scratch, wd, outs[-1], td, ws, parts, gate=I)
-    got = outs[0]
-    assert torch.equal(torch.nan_to_num(got, nan=7.0), torch.nan_to_num(outs[1], nan=7.0))
-    assert torch.isnan(got[1]).all() and torch.isinf(got[2]).all() and torch.equal(got[2], old[2])
-    rows = [i for i in range(M) if i not in (1, 2)]
-    e = lambda y: (y[rows].double() - ref[rows]).norm(dim=1) / ref[rows].norm(dim=1)
-    assert torch.all(e(got) <= e(old) * 1.05) and torch.all(e(got) <= 2.0 ** -23)
-    scratch[:] = float("nan")
-    both = ops.linear_swiglu_delta(x, wgu, tgu, wd, td, scratch, ws, "d")
-    assert (both is None) == (ops._digits_parts(scratch, wd, td, M, D, I) == 0)
-    if both is not None:
-        assert torch.equal(both[4:], got[4:])
+        ops._linear_digits(x, w, out[:, :N], wt, ws, parts)
+        again = ws.get("digits.again", M + 1, N // 32 + 2, torch.int32).flatten()
+        assert again[0] == bad and sorted(again[1:1 + bad].tolist()) == sorted(rows.tolist())
+        assert torch.equal(out[rows.to(DEV), :N], want[rows.to(DEV)]) and torch.isnan(out[:, N:]).all()
+
+
+def _digits_operands(form, M, N, K):
+    """Finite rows whose results lie far below the products of the rows' largest values, or do in some columns."""
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2) * 0.02
+    at = torch.arange(K, device=DEV)
+    if form.startswith("outliers"):                      # one large value in each row of both, in other columns, where the other's are zero in the last form
+        p = int(form.split()[1])
+        x[:, 5] *= 2.0 ** p
+        w[:, 9] *= 2.0 ** p
+        if form.endswith("apart"):
+            x[:, 9] = 0
+            w[:, 5] = 0
+    elif form.startswith("halves"):                      # a little more than half of x large, where w is zero
+        small = at % 100 >= 54
+        x[:, small] *= 2.0 ** -int(form.split()[1])
+        w[:, ~small] = 0
+    elif form == "cancelling":                           # sums of large products that cancel but for the values' last bits
+        x[:, 1::2] = x[:, ::2]
+        w[:, 1::2] = -w[:, ::2] * (1 + 2.0 ** -22)
+    elif form == "some rows":                            # rows of all kinds, in one tile and apart
+        x[::7, 11] *= 2.0 ** 20
+        x[3] = x[3] * 2.0 ** (-(at % 40).float())
+        w[::5, 13] *= 2.0 ** 14
+        w[4] = w[4] * 2.0 ** (-(at % 40).float())
+    return x.contiguous(), w.contiguous()
+
+
+@pytest.mark.parametrize("form", ["outliers 10", "outliers 12", "outliers 12 apart", "halves 20", "halves 30", "halves 42", "cancelling", "some rows"])
+@pytest.mark.parametrize("M,N,K", [(70, 544, 8192), (33, 1056, 2048)])
+def test_linear_f32_from_digits_whatever_the_rows_hold(ops, form, M, N, K):
+    """Each result to its own bound, not to that of the rows' largest values; in whole products and in slices."""
+    from rustinfer_amd.engine.context import Workspace
+    x, w = _digits_operands(form, M, N, K)
+    wt, ws = ops.DigitWeight(w), Workspace(torch.device(DEV))
+    ref = x.double() @ w.double().t()
+    plain = torch.empty(M, N, device=DEV)
+    ops.linear(x, w, plain)
+    for parts in (1, 3):
+        out = torch.full((M, N), float("nan"), device=DEV)
+        ops._linear_digits(x, w, out, wt, ws, parts)
+        assert torch.all((out.double() - ref).abs() <= _digits_bound(x, w, ref)), (form, parts)
+        assert (out.double() - ref).norm() <= 1.0005 * (plain.double() - ref).norm() + 2.0 ** -40 * ref.norm()
 
 
 @pytest.mark.parametrize("M", [3, 20])
