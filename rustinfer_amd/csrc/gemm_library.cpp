@@ -317,12 +317,25 @@ int columns_of_whole_rounds(int M, int N, int out_f32) {
     return rest * 2 <= round || (rounds == 2 && rest * 16 >= round * 11) ? rounds * round : 0;
 }
 
+// The calls of a product, part(first row, rows, first column, columns): a tuned kernel has been chosen by time, for all rows.  Where the library has nothing for
+// a part, the whole product is asked for, and writes again what the other part wrote: that is the one whose refusal the caller hears of.
+template <typename Part>
+int in_rounds(int M, int N, int out_f32, Part part) {
+    const int rows = g_tune ? 0 : rows_of_whole_rounds(M, N), columns = g_tune || rows ? 0 : columns_of_whole_rounds(M, N, out_f32);
+    if (rows || columns) {
+        int rc = rows ? part(0, rows, 0, N) : part(0, M, 0, columns);
+        if (rc == 0) rc = rows ? part(rows, M - rows, 0, N) : part(0, M, columns, N - columns);
+        if (rc != RI_NO_LIBRARY_KERNEL) return rc;
+    }
+    return part(0, M, 0, N);
+}
+
 }  // namespace
 
 // workspace: device memory the library may use (split products); the same size must be passed
 // for a shape each time.  Returns 0, or non-zero with a message in ri_last_error():
-// RI_NO_LIBRARY_KERNEL (2) if the library has no kernel for the problem (nothing was launched; the
-// caller may take a kernel of its own), 1 for every other failure.
+// RI_NO_LIBRARY_KERNEL (2) if the library has no kernel for the problem (the caller may take a kernel of its own, on
+// the same stream: of a product in two calls the first may be under way), 1 for every other failure.
 // out_f32 != 0: C is float32 (logits), else bfloat16.
 extern "C" int ri_gemm_library_bf16(const void* A, int lda, const void* W, int ldw, void* C, int ldc,
                                     int M, int N, int K, int out_f32, void* workspace, size_t workspace_bytes,
@@ -332,19 +345,10 @@ extern "C" int ri_gemm_library_bf16(const void* A, int lda, const void* W, int l
     // one caller at a time: the table of shapes may be emptied, and its descriptors with it
     std::lock_guard<std::mutex> lock(g_mutex);
     if (!g_handle) RI_LT(hipblasLtCreate(&g_handle), "hipblasLtCreate");
-    // (a tuned kernel has been chosen by time, for all rows)
-    const int first = g_tune ? 0 : rows_of_whole_rounds(M, N);
-    if (first) {
-        if (int rc = product(A, lda, W, ldw, C, ldc, first, N, K, out_f32, workspace, workspace_bytes, stream)) return rc;
-        A = (const char*)A + (size_t)first * lda * 2;
-        C = (char*)C + (size_t)first * ldc * (out_f32 ? 4 : 2);
-    } else if (const int columns = g_tune ? 0 : columns_of_whole_rounds(M, N, out_f32)) {
-        if (int rc = product(A, lda, W, ldw, C, ldc, M, columns, K, out_f32, workspace, workspace_bytes, stream)) return rc;
-        W = (const char*)W + (size_t)columns * ldw * 2;
-        C = (char*)C + (size_t)columns * (out_f32 ? 4 : 2);
-        N -= columns;
-    }
-    return product(A, lda, W, ldw, C, ldc, M - first, N, K, out_f32, workspace, workspace_bytes, stream);
+    return in_rounds(M, N, out_f32, [&](int m0, int m, int n0, int n) {
+        return product((const char*)A + (size_t)m0 * lda * 2, lda, (const char*)W + (size_t)n0 * ldw * 2, ldw,
+                       (char*)C + ((size_t)m0 * ldc + n0) * (out_f32 ? 4 : 2), ldc, m, n, K, out_f32, workspace, workspace_bytes, stream);
+    });
 }
 
 // on != 0: products of more than 64 rows look for the library's fastest kernel the first time a
@@ -370,6 +374,18 @@ extern "C" int ri_gemm_library_reset() {
     g_plans.clear();
     g_bucket_algo.clear();
     return 0;
+}
+
+// For a test: the calls of a product, four numbers each, where a part of `refused_rows` rows and `refused_columns` columns is refused; *count of them.
+extern "C" int ri_gemm_library_calls(int M, int N, int out_f32, int refused_rows, int refused_columns, int* calls, int* count) {
+    RI_REQUIRE(M > 0 && N > 0 && calls && count, "ri_gemm_library_calls: bad arguments");
+    std::lock_guard<std::mutex> lock(g_mutex);
+    *count = 0;
+    return in_rounds(M, N, out_f32, [&](int m0, int m, int n0, int n) {
+        int* c = calls + 4 * (*count)++;
+        c[0] = m0; c[1] = m; c[2] = n0; c[3] = n;
+        return m == refused_rows && n == refused_columns ? (int)RI_NO_LIBRARY_KERNEL : 0;
+    });
 }
 
 // For a test: see rows_of_whole_rounds and columns_of_whole_rounds.

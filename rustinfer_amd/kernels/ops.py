@@ -756,7 +756,7 @@ def _tiled_ok(w, w_tiled):
 
 
 _LIBRARY_WS = {}
-NO_LIBRARY_KERNEL = 2          # ri_gemm_library_bf16: the library offers no kernel, nothing was launched
+NO_LIBRARY_KERNEL = 2          # ri_gemm_library_bf16: the library offers no kernel for the product
 _LIBRARY_REFUSED = set()       # (N, K, strides, out dtype) for which it said so
 
 

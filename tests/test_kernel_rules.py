@@ -94,3 +94,23 @@ def test_exact_attention_of_single_tokens_divides_long_rows(lib):
                 assert 1 <= rng.value <= 64 and blocks.value * rng.value >= slots and blocks.value % 2 == 1
                 assert (blocks.value - 2) * rng.value < slots
                 assert rng.value == 1 or T * heads * slots > 30000
+
+
+@pytest.mark.parametrize("M,N,out_f32,parts", [
+    (2385, 16384, 0, [(0, 2048, 0, 16384), (2048, 337, 0, 16384)]),           # rows that make whole rounds, and the rest
+    (2048, 18448, 0, [(0, 2048, 0, 16384), (0, 2048, 16384, 2064)]),          # columns
+    (600, 5000, 1, [(0, 600, 0, 5000)])])
+def test_a_library_product_in_parts_is_asked_for_whole_where_a_part_is_refused(lib, M, N, out_f32, parts):
+    """Only the whole product's refusal is the caller's: it bars the weight's size from the library for every number of rows."""
+    whole = (0, M, 0, N)
+
+    def calls(refused):
+        got, count = (ctypes.c_int * 16)(), ctypes.c_int(0)
+        rc = lib.ri_gemm_library_calls(M, N, out_f32, refused[1], refused[3], got, ctypes.byref(count))
+        return rc, [tuple(got[4 * i:4 * i + 4]) for i in range(count.value)]
+
+    assert calls((0, 0, 0, 0)) == (0, parts)
+    if len(parts) == 2:
+        assert calls(parts[1]) == (0, parts + [whole])
+        assert calls(parts[0]) == (0, [parts[0], whole])
+    assert calls(whole) == ((0, parts) if len(parts) == 2 else (2, [whole]))
