@@ -909,19 +909,21 @@ extern "C" int ri_gemm_skinny_residual(const void* A, int lda, const void* W, in
                                        hipStream_t stream) {
     RI_REQUIRE(M >= 1 && M <= 16, "ri_gemm_skinny_residual: M=%d not in [1, 16]", M);
     RI_REQUIRE(N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0, "ri_gemm_skinny_residual: needs N %% 16 == 0 and K %% 32 == 0 (N=%d K=%d)", N, K);
-    RI_REQUIRE(lda >= K && lda % 8 == 0 && lda <= (1 << 27), "ri_gemm_skinny_residual: bad leading dimension");
+    RI_REQUIRE(lda >= K && lda % 8 == 0, "ri_gemm_skinny_residual: bad leading dimension");
     RI_REQUIRE(A && W && x && w_norm && a_out && ssq, "ri_gemm_skinny_residual: null pointer");
     RI_REQUIRE(w_dtype == RI_F32 || w_dtype == RI_BF16, "ri_gemm_skinny_residual: the norm's weight must be float32 or bfloat16");
     RI_REQUIRE((uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && (uintptr_t)x % 16 == 0 && (uintptr_t)w_norm % 16 == 0
                && (uintptr_t)a_out % 8 == 0, "ri_gemm_skinny_residual: operands must be 16-byte aligned");
-    const int halves = residual_halves(N);
+    // rows further apart than the pairs' 32-bit distances reach: half tiles, whose slots are as many
+    const bool pairs = residual_pairs(M, N), far = M > 1 && lda > (1 << 27);
+    const int halves = residual_halves(N) || (pairs && far);
     ResidualEpilogue re{x, w_dtype == RI_F32 ? (const float*)w_norm : nullptr, w_dtype == RI_BF16 ? (const bf16_t*)w_norm : nullptr,
                         (bf16_t*)a_out, ssq, halves};
     const bf16_t* a = (const bf16_t*)A;
     const bf16_t* w = (const bf16_t*)W;
     const int nks = K / 32, blocks = (N / 16) * (halves ? 2 : 1);
-    if (residual_pairs(M, N) && K <= 2048) gemm_skinny_pairs_kernel<2, 16><<<N / 8, 1024, 0, stream>>>(a, lda, w, M, N, K, re);
-    else if (residual_pairs(M, N)) gemm_skinny_pairs_kernel<4, 16><<<N / 8, 1024, 0, stream>>>(a, lda, w, M, N, K, re);
+    if (pairs && !far && K <= 2048) gemm_skinny_pairs_kernel<2, 16><<<N / 8, 1024, 0, stream>>>(a, lda, w, M, N, K, re);
+    else if (pairs && !far) gemm_skinny_pairs_kernel<4, 16><<<N / 8, 1024, 0, stream>>>(a, lda, w, M, N, K, re);
     else if (nks >= 16)
         gemm_skinny_bf16_kernel<1, 1, 8, float, false, true><<<dim3(blocks, 1), 512, 0, stream>>>(
             a, lda, w, K, (float*)nullptr, N, M, N, K, nks, 0, RopeEpilogue{}, RowScale{}, re);

@@ -1413,6 +1413,22 @@ def test_the_product_before_a_norm_in_pairs_of_steps(ops, M, N, K):
         assert torch.equal(y[rest], x[rest]) and not torch.isfinite(y[1]).any()
 
 
+@pytest.mark.parametrize("M,N", [(1, 3072), (3, 3072), (2, 64)])
+def test_the_product_before_a_norm_of_rows_further_apart_than_32_bit_distances_reach(ops, M, N):
+    far, K = (1 << 27) + 8, 1056
+    buf = torch.empty((M - 1) * far + K, dtype=torch.bfloat16, device=DEV)
+    act = buf.as_strided((M, K), (far, 1))
+    act.copy_(rnd(M, K, dtype=torch.bfloat16, seed=1))
+    w = rnd(N, K, dtype=torch.bfloat16, seed=2, scale=0.05)
+    wt, wn, ws = ops.tile_weight(w), 1.0 + rnd(N, seed=3, scale=0.1), Workspace(DEV)
+    x = torch.zeros(M, N, device=DEV)
+    a, ssq = ops.linear_residual(act, w, wt, x, wn, ws, "t")
+    mag = ((act.double() ** 2) @ (w.double() ** 2).t()).sqrt()                  # the bound of the test above
+    assert torch.all((x.double() - act.double() @ w.double().t()).abs() <= K * 2.0 ** -23 * mag)
+    assert torch.equal(a, (x * wn).to(torch.bfloat16))
+    assert torch.allclose(ssq.double().sum(1), (x.double() ** 2).sum(1), rtol=1e-5)
+
+
 @pytest.mark.parametrize("wdtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("M,N,K,I,eps", [(1, 64, 64, 176, 1e-5), (5, 384, 1056, 416, 1e-6), (8, 2048, 8192, 1024, 1e-5),
                                          (16, 4096, 14336, 512, 1e-5), (13, 160, 416, 48, 1e-5), (2, 2304, 2304, 1184, 1e-6)])
