@@ -47,8 +47,8 @@ struct RowOf {
     int e, unused;
 };
 
-// s_waitcnt: at most n loads under way, whatever is asked of LDS
-constexpr int loads_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+// s_waitcnt: at most n loads under way, and nothing asked of LDS: a stage is written over behind the barrier only when what was read of it has arrived
+constexpr int loads_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 
 __device__ __forceinline__ float bound(const float (&x)[6], const float (&w)[6]) {
     float b = x[0] * w[0];

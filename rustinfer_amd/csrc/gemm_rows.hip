@@ -33,8 +33,8 @@ namespace {
 
 constexpr int KS = 2;                     // k-steps of 32 in a stretch: 128 bytes of a row
 
-// s_waitcnt: at most n loads under way, whatever is asked of LDS
-constexpr int loads_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
+// s_waitcnt: at most n loads under way, and nothing asked of LDS: a stage is written over behind the barrier only when what was read of it has arrived
+constexpr int loads_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4); }
 
 struct Store4 {
     static __device__ __forceinline__ void st(float* p, const float* v) {
