@@ -18,7 +18,8 @@ staying on the device for the next step (the serving loop's way).  Prints one JS
                        beside the requests that decode: tok/s generated from the first arrival to the
                        last token, and the share of steps that replayed a graph
   peaks                what a bare read, a copy, a loop of bfloat16 matrix instructions and a loop of
-                       32-bit FMAs reach on this GPU now; ``frac_measured`` prices against these
+                       32-bit FMAs reach on this GPU now; ``frac_measured`` prices against these (32-bit prompts
+                       against the 8-bit matrix instruction, see DIGIT_PRODUCTS)
   shape_1b, shape_3b   decode at batch 8 and prefill at the Llama-3.2-1B / 3B layer sizes
   fp32                 the true 32-bit path at the headline shape: decode at batch 8 and prefill
                        (the last three only with the default shape)
@@ -58,7 +59,9 @@ SHAPES = {
                                   high_freq_factor=4.0, original_max_position_embeddings=8192)),
 }
 PEAK_HBM_GBS = 8000.0
-PEAK_FLOPS = {"bf16": 2.5e15, "fp32": 157.3e12}
+# 32-bit prompts multiply 8-bit digits, at twice the rate of bfloat16, 20 products of digits for each of two values (csrc/gemm_digits.hip)
+DIGIT_PRODUCTS = 20
+PEAK_FLOPS = {"bf16": 2.5e15, "fp32": 2 * 2.5e15 / DIGIT_PRODUCTS}
 PAGE = 16
 MIN_POINT_STEPS = 64
 
@@ -730,7 +733,7 @@ def other_shape(name, args, dtype, peaks):
     gbs = step_bytes / step_s / 1e9
     rec = {"value": round(tok_s, 1), "ms_per_step": round(step_s * 1e3, 4), "roofline_frac": round(gbs / PEAK_HBM_GBS, 4),
            "roofline_frac_measured": round(gbs / peaks["hbm_read_gbs"], 4), "prefill": s.prefill(reps=5 if dtype == "bf16" else 2)}
-    flops_peak = peaks["mfma_bf16_tflops"] if dtype == "bf16" else peaks["fma_f32_tflops"]
+    flops_peak = peaks["mfma_bf16_tflops"] * PEAK_FLOPS[dtype] / PEAK_FLOPS["bf16"]
     rec["prefill"]["frac_measured"] = round(rec["prefill"]["frac"] * PEAK_FLOPS[dtype] / (flops_peak * 1e12), 4)
     s.close()
     return rec
@@ -865,7 +868,7 @@ def main() -> int:
                      "peak_measured": peaks["hbm_read_gbs"], "frac_measured": round(achieved / peaks["hbm_read_gbs"], 4)},
         "peaks": peaks,
     }
-    flops_peak = (peaks["mfma_bf16_tflops"] if args.dtype == "bf16" else peaks["fma_f32_tflops"]) * 1e12
+    flops_peak = peaks["mfma_bf16_tflops"] * PEAK_FLOPS[args.dtype] / PEAK_FLOPS["bf16"] * 1e12
     if not args.no_points:
         out["prefill"] = b.prefill()
         out["prefill"]["frac_measured"] = round(out["prefill"]["frac"] * PEAK_FLOPS[args.dtype] / flops_peak, 4)

@@ -675,6 +675,8 @@ static bool list_pays(long long pairs, int hd, int max_kv_len) {
 }
 
 // Whether a step of T single tokens alone goes as a list: what it takes (rows for the lanes of a wave, w total below 2^32), and where it pays.
+// (No more rows than lanes: a first form that read more than 64 rows in groups faulted the GPU once, with 100 rows of 700 keys.  The cause was not shown, that
+// form is not in the code, and such steps take blocks a row; whoever lifts the limit has that to explain first.)
 extern "C" int ri_attention_decode_as_list(int T, int Hkv, int hd, int page, int max_kv_len) {
     const long long spans = (long long)T * ((max_kv_len + LIST_SPAN - 1) / LIST_SPAN + 1);
     return T >= 3 && T <= LIST_ROWS && (page & (page - 1)) == 0 && spans < (1ll << 32) / LIST_WAVES && list_pays((long long)T * Hkv, hd, max_kv_len);

@@ -317,7 +317,8 @@ int columns_of_whole_rounds(int M, int N, int out_f32) {
     return rest * 2 <= round || (rounds == 2 && rest * 16 >= round * 11) ? rounds * round : 0;
 }
 
-// The calls of a product, part(first row, rows, first column, columns): a tuned kernel has been chosen by time, for all rows.  Where the library has nothing for
+// The calls of a product, part(first row, rows, first column, columns).  With tuning on there is one: its kernel has been chosen by time, among the library's
+// for the whole product (two calls are not among them, and may be faster).  Where the library has nothing for
 // a part, the whole product is asked for, and writes again what the other part wrote: that is the one whose refusal the caller hears of.
 template <typename Part>
 int in_rounds(int M, int N, int out_f32, Part part) {

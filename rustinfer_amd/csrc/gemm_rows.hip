@@ -370,8 +370,10 @@ int launch_rows_rope_groups(const bf16_t* A, int lda, const bf16_t* W, bf16_t* C
 
 // Slices of K, and wave groups a block, for a product of M rows, N columns and K inner values whose partial sums a norm adds up: blocks enough to
 // fill the chip twice, at most 8 slices (16 of 2048 x 8192 take less here and cost the norm more), then groups where that fills the units better with as many
-// slices or fewer.  Up to 16 rows: eight slices and four groups where their blocks are whole rounds of the 512 that the chip holds at once, two groups where
-// those of 64 columns are just that, else one group, and all blocks run at once; parts 1 where the few-row kernel is as fast.  us, few-row / this at 9 to 16 rows: 2048 x 2048 4.6
+// slices or fewer.  Up to 16 rows and for 16 to 80 blocks of 64 columns: eight slices, in four groups up to 32 blocks (and of 64 with rows of 8,192 values or more), in two for
+// 56 to 64 with shorter rows, else in one, whose blocks all run at once; parts 1 elsewhere, where the few-row kernel is as fast.  16 rows, us, few-row / eight slices in 1, 2, 4 groups:
+// 1088 x 8192 8.0 / 7.8 6.4 6.6, 1536 x 8960 9.6 / 10.4 8.0 8.2, 1984 x 4096 6.5 / 5.6 5.4 5.3, 2048 x 8192 9.3 / 9.1 8.5 7.9; 2560 x 9728 12.9 / 11.3 12.2 11.5, 3328 x 4096 9.8 /
+// 7.2 7.3 8.0; 3584 x 3584 9.2 / 7.0 6.9 8.0, 3584 x 7168 16.1 / 10.9 11.4 12.2, 3840 x 5120 12.2 / 8.6 8.8 9.9, 4096 x 4096 8.6 / 9.6 8.4 9.1.  us, few-row / this at 9 to 16 rows: 2048 x 2048 4.6
 // / 4.1, 2048 x 8192 8.8 / 7.7, 3072 x 8192 12.5 / 11.0, 4096 x 4096 8.7 / 8.5, 4096 x 14336 22.2 / 20.9, 5120 x 5120 14.0 / 12.1, 5120 x 13824 29.4 / 27.5.  With more: a block of two groups has a unit to itself (two share it up to 32 rows), three of one group share one
 // (four up to 32 rows), and one of four groups, of half the columns, has one to itself.  Measured, us (slices/groups), at 20, 32, 48, 64 rows: 2048 x 2048
 // 4/4 4.5 4.7 5.2 5.6, 8/1 4.9 5.2 5.7 6.0; 1024 x 3072 8/4 4.1 4.3 4.8 5.3, 8/1 4.7 5.0 5.5 5.9; 2048 x 8192 8/2 8.5 8.7 9.2 9.9, 4/4 9.9 10.4 11.2 11.7, 8/1 9.0 9.1
@@ -453,11 +455,8 @@ extern "C" int ri_gemm_rows_bf16(const void* A, int lda, const void* W, void* C,
 
 // The q/k/v projection of 9..64 tokens with rotation and cache write in the epilogue, as
 // ri_gemm_qkv_rope (gemm.hip) does it for fewer rows: W is the same row-permuted weight in tile
-// order, C [M, ldc] receives rotated q in its first H * hd columns.  Measured at 64 rows against
-// the few-row kernel (product alone, us): 6144 x 4096 25.9 -> 21.5, 5120 x 3072 21.1 -> 16.5,
-// 3072 x 2048 16.4 -> 10.9 (but no gain left there once the epilogue is in); from 32 rows down the
-// few-row kernel is as fast or faster at these sizes and slower at larger ones (24 rows: 12288 x
-// 4096 27.3 -> 23.5, 15360 x 5120 35.9 -> 28.8, 10240 x 8192 49.0 -> 42.4): the caller chooses.
+// order, C [M, ldc] receives rotated q in its first H * hd columns.  The caller chooses between this and the few-row
+// kernel (ops.py, QKV_ROPE_LDS_*, with the figures of both).
 //
 // Blocks of 32 columns (four pairs of waves) where all of them run at once, one a compute unit; else blocks of 64
 // columns (two groups of four waves), half as many: 288 blocks of 32 columns (9216 x 4096) took 27.1 us with 32 rows, 144 of 64 23.0 with 33.

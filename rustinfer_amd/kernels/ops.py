@@ -449,13 +449,15 @@ RESIDUAL_FORM_LARGE = 32 << 20  # elements of a weight from which the residual f
 
 def linear_residual_pays(M: int, w: torch.Tensor) -> bool:
     """Whether ``linear_residual`` is the faster way for ``M`` rows against ``w [N, K]``, compared
-    with partial sums over slices of K and the norm's own kernel (which costs 4.6 us).  A block of
-    the residual form owns 16 whole columns: it cannot divide K between blocks, so every block asks
+    with partial sums over slices of K and the norm's own kernel (which costs 3 to 6 us).  A block of
+    the residual form owns 16 whole columns (8 in ri_gemm_skinny_residual's other forms): it cannot divide K between blocks, so every block asks
     for all of its rows' activations (beyond eight rows that shows), and 320 blocks on 256 compute
-    units take as long as 512.  Measured, us, residual form / partial sums, at 1, 8, 16 rows:
-    4096 x 14336: 22.6 24.9 31.7 / 21.3 22.0 21.9; 4096 x 4096: 9.0 9.6 10.9 / 8.2 9.2 9.5;
-    5120 x 13824: 31.7 38.1 49.2 / 26.3 26.6 27.6; 5120 x 5120: 13.3 16.4 20.7 / 13.4 13.1 13.3;
-    8192 x 8192: 25.1 28.5 34.9 / 25.1 24.8 25.3; 3072 x 8192: 12.9 15.7 17.8 / 12.3 13.9 12.7."""
+    units take as long as 512.  Measured, us, residual form / partial sums and the norm, at 1, 8, 16 rows:
+    4096 x 14336: 19.2 23.2 28.6 / 23.1 24.1 24.4; 4096 x 4096: 7.5 9.0 10.5 / 12.2 13.3 13.1;
+    5120 x 5120: 12.8 15.4 20.9 / 17.6 17.3 17.3; 8192 x 8192: 22.8 26.5 32.5 / 28.8 28.6 31.0; 3072 x 8192: 10.8 13.3 16.9 / 15.4 17.0 14.7;
+    2048 x 8192 7.8 8.8 14.7 / 10.9 11.7 11.3; 2048 x 2048 4.0 4.6 6.2 / 6.9 7.6 7.7; 5120 x 13824: 26.6 33.2 48.5 / 29.7 30.5 31.0; 5120 x 8192: 15.6 20.3 30.0 /
+    21.3 21.6 23.0.  The line counts blocks of 16 columns, as the form was when it was drawn: up to eight rows of the last two sizes it leaves out pairs of steps that
+    would mostly pay, and 16 rows of 3072 x 8192, 2048 x 8192 and 5120 x 5120 it lets in."""
     N, K = w.shape
     if N * K < RESIDUAL_FORM_LARGE:
         return True
@@ -694,7 +696,7 @@ QKV_ROPE_LDS_FEW_ROWS = 9       # tokens up to 16 from which it takes weights of
                                 # this at 9, 12, 16: 6144 x 4096 14.0 15.2 15.9 / 13.9 14.0 14.3, 5120 x 3072 11.0 11.8 12.4 / 10.7 10.9 11.3, 12288 x 4096 25.8 26.8 26.8 /
                                 # 25.4 25.6 25.2, 10240 x 8192 39.5 42.1 45.4 / 39.5 34.2 35.3; not 3072 x 2048 6.4 6.6 7.0 / 7.1 7.3 7.5
 ROWS_LDS_MIN_ROWS = 17          # from here to 64 rows, products whose partial sums a norm adds up take the LDS kernel
-ROWS_LDS_WIDE_COLUMNS = 16384   # whole products (no slices of K) take it from this many columns on: the output head, 250 -> 205 us at 64 rows
+ROWS_LDS_WIDE_COLUMNS = 16384   # whole products (no slices of K) of this many columns have forms of their own (_rows_whole), and `linear_activated` takes them from 17 rows on
 
 
 def _swiglu_groups(I: int, M: int = 17) -> int:
