@@ -675,6 +675,33 @@ def test_linear_f32_from_digits_whatever_the_rows_hold(ops, form, M, N, K):
         assert (out.double() - ref).norm() <= 1.0005 * (plain.double() - ref).norm() + 2.0 ** -40 * ref.norm()
 
 
+@pytest.mark.parametrize("M,I,K", [(40, 1024, 2048), (130, 8192, 1024), (64, 2720, 1056), (33, 14336, 512)])
+def test_swiglu_mlp_f32_from_digits(ops, M, I, K):
+    """Both products of a 32-bit MLP through digits, in whole products and slices, the activation rounded between them: the second no further from 64 bits than 64-bit sums
+    of the same activation; a row that is not finite, one whose activation passes the 32-bit range, and one of widely spread values."""
+    from rustinfer_amd.engine.context import Workspace
+    D = 1024
+    x, wgu, wd = rnd(M, K, seed=1), rnd(2 * I, K, seed=2) * 0.05, rnd(D, I, seed=3) * 0.02
+    tgu, td, ws = ops.tile_weight(wgu), ops.tile_weight(wd), Workspace(torch.device(DEV))
+    scratch, act = torch.empty(M, 2 * I, device=DEV), torch.empty(M, I, device=DEV)
+    ops._linear_digits(x, wgu, scratch, tgu, ws, 1)
+    assert torch.all((scratch.double() - x.double() @ wgu.double().t()).abs() <= _digits_bound(x, wgu, x.double() @ wgu.double().t()))
+    scratch[1, 5] = float("nan")
+    scratch[2, 7], scratch[2, I + 7] = 1e20, 1e20
+    g = torch.Generator().manual_seed(3)
+    scratch[3, I:] = (torch.randn(I, generator=g) * 2.0 ** torch.randint(-60, 61, (I,), generator=g)).to(DEV)
+    ops.swiglu(scratch, act)
+    ref, want = act.double() @ wd.double().t(), torch.empty(M, D, device=DEV)
+    ops.linear(act, wd, want)
+    rows = [i for i in range(M) if i not in (1, 2)]
+    for parts in (1, 3):
+        got = torch.full((M, D), float("nan"), device=DEV)
+        ops._linear_digits(act, wd, got, td, ws, parts)
+        assert torch.isnan(got[1]).all() and torch.isinf(got[2]).all() and torch.equal(got[2], want[2])
+        assert torch.all((got[rows].double() - ref[rows]).abs() <= _digits_bound(act[rows], wd, ref[rows]))
+        assert torch.all((got[rows].double() - ref[rows]).norm(dim=1) <= (want[rows].double() - ref[rows]).norm(dim=1) * 1.05)
+
+
 @pytest.mark.parametrize("M", [3, 20])
 def test_linear_f32_of_rows_further_apart_than_32_bit_distances_reach(ops, M):
     far, K = (1 << 24) + 4, 12                          # 48 rows of such a distance: over 3 GiB
