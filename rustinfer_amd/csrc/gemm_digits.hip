@@ -10,7 +10,7 @@
 // by the inequality of Cauchy and Schwarz, and a result smaller than 2^27 times that is computed again from the 32-bit values in 64-bit sums.  So every
 // result is within half a unit of its last place and 2^-27 of itself, or a 64-bit sum.  What is lost in fact is a twelfth to a fortieth of the bound.  How many are computed again: of normal rows
 // against normal weights 0.03 % (K = 2048) and 0.07 % (8192), of a gated activation 0.1 and 0.2 %, with a value of 2^16 standard deviations in each row 0.4 and 4 %.  Their places are
-// noted a row at a time, N / 32 of them at most; a wave does such a result in 64-bit FMAs.  A row that has more goes to the kernel of 64-bit
+// noted a row at a time, N / 16 of them at most; a wave does such a result in 64-bit FMAs.  A row that has more goes to the kernel of 64-bit
 // sums whole, with the others like it, and so do rows that hold an infinity or a NaN, and rows most of whose values are cut off (these two without being
 // multiplied first where all 64 rows of a block are such).  A weight with such a row gets no digits.
 //
@@ -21,7 +21,8 @@
 // 600 rows of 16384 x 2048 724 / 362, 3072 x 2048 128 / 82, 2048 x 2048 95 / 71, 2048 x 8192 (a gated activation) 350 / 222; 194 rows 250 / 141
 // (16384 x 2048), 135 / 91 (2048 x 8192); 89 rows 113 / 81, 85 / 59.  (Five digits for both and 15 products, without the bound: 264 us for the
 // first, and results that were off by as much as their size where large values of the one row met small ones of the other.)  600 rows of which 1, 60, 600
-// have no digits: 16384 x 2048 462, 458, 760, 2048 x 8192 290, 288, 372, 2048 x 2048 90, 91, 113; all with a value of 2^12 standard deviations: 402, 390, 80.
+// have no digits: 16384 x 2048 462, 455, 765, 2048 x 8192 285, 284, 369, 2048 x 2048 90, 91, 112; all with a value of 2^12 standard deviations: 380, 330, 78 (2048 x 8192
+// with N / 32 places a row, so that 61 rows were done whole: 385).
 #include "common.h"
 #include <float.h>
 #include <limits.h>
@@ -68,7 +69,7 @@ struct Again {
     int* counts;             // [M]
     int* columns;            // [M][cap]
     int cap;
-    __host__ __device__ Again(int* buffer, int M, int N) : rows(buffer), counts(buffer + 1 + M), columns(buffer + 1 + 2 * (size_t)M), cap(N / 32) {}
+    __host__ __device__ Again(int* buffer, int M, int N) : rows(buffer), counts(buffer + 1 + M), columns(buffer + 1 + 2 * (size_t)M), cap(N / 16) {}
     // places for `many` results of row m, from the returned one on
     __device__ __forceinline__ int note(int m, int many) const {
         const int old = atomicAdd(counts + m, many);
@@ -374,7 +375,7 @@ extern "C" long long ri_digits_bytes(int rows, int K, int digits) { return (long
 extern "C" int ri_digits_max_k() { return MAX_K; }
 
 // Digits of X[rows, K] and what is known of each row (eight 32-bit words, rows up to whole tiles of 32; a row without digits has an infinity in the first).
-// For the rows of a product of N columns, `again`: the buffer of (1 + 2 rows + rows (N / 32)) integers that ri_gemm_digits takes.
+// For the rows of a product of N columns, `again`: the buffer of (1 + 2 rows + rows (N / 16)) integers that ri_gemm_digits takes.
 extern "C" int ri_digits_split(const float* X, int ld, int rows, int K, int digits, void* planes, void* known, int* again, int N, hipStream_t stream) {
     RI_REQUIRE(rows >= 1 && K >= 32 && K % 32 == 0 && K <= MAX_K, "ri_digits_split: needs K %% 32 == 0 and at most %d (rows=%d K=%d)", MAX_K, rows, K);
     RI_REQUIRE(digits == DA || digits == DW, "ri_digits_split: %d digits, not %d or %d", digits, DA, DW);

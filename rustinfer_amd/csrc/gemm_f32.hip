@@ -34,28 +34,18 @@ typedef double f64x4_t __attribute__((ext_vector_type(4)));
 // MT x NT tiles of 16 x 16 results a block, WAVES waves that share K, chunks of 16 U values of K (U = 1: two of them, one
 // after the other, are a wave's turn of 32).
 // STREAM: W is read once (a single row of tiles), past the caches.
-// LISTED: of the rows of A and C only those whose numbers stand in list[1] and on, list[0] of them, which the launch does not know: as many blocks as the chip
-// holds take their tiles in turn (an empty list 4.6 us, where a block for each tile of 600 rows of 16384 columns took 5.6).
-template <int MT, int NT, int WAVES, int U, bool STREAM, bool LISTED = false>
-__global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
+// The tile with number `id`.  LISTED: of the rows of A and C only the M whose numbers stand in list[1] and on.
+template <int MT, int NT, int WAVES, int U, bool STREAM, bool LISTED>
+__device__ __forceinline__ void f32_tile_of(
         const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
-        float* __restrict__ C, int ldc, int M, int N, int K, int mtiles, int ntiles, const int* __restrict__ list = nullptr) {
+        float* __restrict__ C, int ldc, int M, int N, int K, int mtiles, int ntiles, const int* __restrict__ list, int id) {
     constexpr int KC = 16 * U, TURN = WAVES * 32;
     static_assert(U == 1 || U == 2, "a wave's turn of K is 32 values");
     __shared__ double sums[WAVES][16][NT * 16];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, r = lane & 15, g = lane >> 4;
-    if (LISTED) {
-        M = list[0];
-        mtiles = (M + MT * 16 - 1) / (MT * 16);
-    }
-    for (int id = (int)blockIdx.x;; id += (int)gridDim.x) {
-    if (LISTED && id >= (ntiles + 7) / 8 * 8 * mtiles) return;
     const int xcd = id & 7, turn = id >> 3;
     const int nt = (turn / mtiles) * 8 + xcd, mt = turn % mtiles;
-    if (nt >= ntiles) {
-        if (LISTED) continue;
-        return;
-    }
+    if (nt >= ntiles) return;
     const int m0 = mt * MT * 16, n0 = nt * NT * 16;
     // the block's first rows, the same in all lanes, and each lane's rows as 32-bit distances in bytes from there (listed rows, which may lie
     // anywhere, as 64-bit ones from the first of all)
@@ -169,8 +159,23 @@ __global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
             if (m < M && n < N) C[(size_t)(LISTED ? list[1 + m] : m) * ldc + n] = (float)v;
         }
     }
-    if (!LISTED) return;
-    __syncthreads();
+}
+
+// A tile a block.  LISTED: the rows' number, list[0], is not known to the launch: as many blocks as the chip
+// holds take the tiles in turn (an empty list 4.6 us, where a block for each tile of 600 rows of 16384 columns took 5.6).
+template <int MT, int NT, int WAVES, int U, bool STREAM, bool LISTED = false>
+__global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
+        const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
+        float* __restrict__ C, int ldc, int M, int N, int K, int mtiles, int ntiles, const int* __restrict__ list = nullptr) {
+    if constexpr (LISTED) {
+        M = list[0];
+        mtiles = (M + MT * 16 - 1) / (MT * 16);
+        for (int id = (int)blockIdx.x; id < (ntiles + 7) / 8 * 8 * mtiles; id += (int)gridDim.x) {
+            f32_tile_of<MT, NT, WAVES, U, STREAM, true>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles, list, id);
+            __syncthreads();                     // the sums in LDS have been read
+        }
+    } else {
+        f32_tile_of<MT, NT, WAVES, U, STREAM, false>(A, lda, W, ldw, C, ldc, M, N, K, mtiles, ntiles, nullptr, (int)blockIdx.x);
     }
 }
 

@@ -819,7 +819,7 @@ def _linear_digits(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled:
     rows = (M + 31) // 32 * 32
     planes = workspace.get("digits.planes", rows, 6 * K, torch.uint8)
     known = workspace.get("digits.known", rows, 8, torch.float32)
-    again = workspace.get("digits.again", M + 1, N // 32 + 2, torch.int32)       # what is computed again: csrc/gemm_digits.hip
+    again = workspace.get("digits.again", M + 1, N // 16 + 2, torch.int32)       # what is computed again: csrc/gemm_digits.hip
     sums = workspace.get("digits.sums", parts * M, N, torch.float64) if parts > 1 else None
     _check(lib.ri_digits_split(_ptr(x), x.stride(0), M, K, 6, _ptr(planes), _ptr(known), _ptr(again), N, _stream()))
     _check(lib.ri_gemm_digits(_ptr(planes), _ptr(known), _ptr(x), x.stride(0), _ptr(w_tiled.planes), _ptr(w_tiled.known),

@@ -627,7 +627,7 @@ def test_linear_f32_rows_without_digits_are_those_of_64_bit_sums(ops, M, N, K, b
     ops.linear(x, w, want)
     for parts in (1, 3):
         ops._linear_digits(x, w, out[:, :N], wt, ws, parts)
-        again = ws.get("digits.again", M + 1, N // 32 + 2, torch.int32).flatten()
+        again = ws.get("digits.again", M + 1, N // 16 + 2, torch.int32).flatten()
         assert again[0] == bad and sorted(again[1:1 + bad].tolist()) == sorted(rows.tolist())
         assert torch.equal(out[rows.to(DEV), :N], want[rows.to(DEV)]) and torch.isnan(out[:, N:]).all()
 
