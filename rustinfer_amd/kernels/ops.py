@@ -10,6 +10,7 @@ if it cannot be built or loaded these functions raise.
 from __future__ import annotations
 
 import ctypes
+import weakref
 from typing import Optional
 
 import torch
@@ -487,6 +488,77 @@ def linear_residual(act: torch.Tensor, w: torch.Tensor, w_tiled: Optional[torch.
     _check(lib.ri_gemm_skinny_residual(_ptr(act), act.stride(0), _ptr(w_tiled), M, N, K, _ptr(x), _ptr(norm_weight),
                                        _dt(norm_weight), _ptr(a), _ptr(ssq), _stream()))
     return a, ssq
+
+
+DECODE_STACK_CLOSE_US = 200.0   # how long the first blocks of a one-launch step wait for the rest before they go on without them
+DECODE_STACK_LIMIT_US = 5e6     # and how long they wait for each other's results before they give up
+DECODE_STACK_GRID = 0           # blocks launched: 0 one a compute unit
+
+
+def decode_stack_takes(M: int, d: int, ff: int, H: int, Hkv: int, hd: int, page: int, V: int) -> bool:
+    """Whether a step of ``M`` single tokens of a Llama stack of these sizes may go in one launch."""
+    return not FORCE_LIBRARY_GEMM and bool(_lib().ri_decode_stack_takes(M, d, ff, H, Hkv, hd, page, V))
+
+
+def decode_stack_scratch(L: int, d: int, ff: int, H: int, Hkv: int, hd: int, rows: int = 8) -> int:
+    """Bytes of scratch that steps of up to ``rows`` tokens take."""
+    lib = _lib()
+    lib.ri_decode_stack_scratch.restype = ctypes.c_size_t
+    return max(lib.ri_decode_stack_scratch(L, M, d, ff, H, Hkv, hd) for M in range(1, rows + 1))
+
+
+def decode_stack_control(workspace) -> Optional[int]:
+    """The control block of the one-launch steps of ``workspace``: taken when it is first asked for, given back when the workspace
+    goes.  None if there is none left, or if the stream is under capture and none has been taken."""
+    block = getattr(workspace, "_stack_control", None)
+    if block is None and not torch.cuda.is_current_stream_capturing():
+        lib, p = _lib(), ctypes.c_void_p()
+        _check(lib.ri_decode_stack_take_control(ctypes.byref(p)))
+        block = p.value
+        if block is not None:
+            workspace._stack_control = block
+            weakref.finalize(workspace, lib.ri_decode_stack_give_control, ctypes.c_void_p(block))
+    return block
+
+
+def decode_stack(model: torch.Tensor, L: int, ctx, table: torch.Tensor, ff: int, H: int, Hkv: int, hd: int, cos: torch.Tensor, sin: torch.Tensor,
+                 k_pool: torch.Tensor, v_pool: torch.Tensor, block_table: torch.Tensor, page: int, scale: float, norm_dtype: torch.dtype,
+                 scratch: torch.Tensor, logits: torch.Tensor) -> None:
+    """One step of ``ctx.num_tokens`` single tokens through ``L`` layers, in one launch: embedding, layers, final norm, head; keys and values
+    go to the pools ``[L, pages, ...]``.  ``model``: the table of its weights (csrc/decode_stack.hip)."""
+    M, (V, d) = ctx.num_tokens, table.shape
+    lib = _lib()
+    tokens = getattr(ctx, "device_tokens", None)
+    _dev(model, table, cos, sin, k_pool, v_pool, block_table, scratch, logits)
+    if model.numel() != lib.ri_decode_stack_table(L) or model.dtype != torch.int64 or not model.is_contiguous():
+        raise KernelError("decode_stack: the model's table does not fit")
+    _i32(ctx.token_ids, "token_ids", M)
+    _i32(ctx.positions, "positions", M)
+    _i32(ctx.row_of_token, "row_of_token", M)
+    _i32(ctx.kv_lens, "kv_lens", ctx.num_rows)
+    _i32(block_table, "block_table")
+    if tokens is not None:
+        _i32(tokens, "device_tokens")
+    if block_table.dim() != 2 or block_table.shape[0] < ctx.num_rows:
+        raise KernelError("decode_stack: block_table must be [rows, max_blocks]")
+    if k_pool.shape[0] != L or v_pool.shape[0] != L or not k_pool.is_contiguous() or not v_pool.is_contiguous():
+        raise KernelError("decode_stack: the pools must be contiguous with one entry a layer")
+    _check_cache(k_pool[0], v_pool[0], Hkv, hd, page, torch.bfloat16, "decode_stack")
+    if table.dtype != torch.bfloat16 or not table.is_contiguous():
+        raise KernelError("decode_stack: the embedding must be contiguous bfloat16 [vocabulary, width]")
+    if cos.dtype != torch.float32 or cos.shape != sin.shape or cos.shape[1] * 2 != hd or not cos.is_contiguous() or not sin.is_contiguous():
+        raise KernelError("decode_stack: cos/sin must be contiguous float32 [positions, head_dim/2]")
+    if logits.dtype != torch.float32 or tuple(logits.shape) != (M, V) or not logits.is_contiguous():
+        raise KernelError(f"decode_stack: logits must be contiguous float32 [{M}, {V}]")
+    control = decode_stack_control(ctx.workspace)
+    if control is None:
+        raise KernelError("decode_stack: no control block")
+    _check(lib.ri_decode_stack(
+        _ptr(model), L, M, d, ff, H, Hkv, hd, V, _DT[norm_dtype], _ptr(ctx.token_ids), _ptr(tokens), _ptr(table), _ptr(ctx.positions),
+        _ptr(ctx.row_of_token), _ptr(ctx.kv_lens), _ptr(block_table), block_table.shape[1], _ptr(cos), _ptr(sin), _ptr(k_pool), _ptr(v_pool),
+        ctypes.c_size_t(k_pool.stride(0)), ctypes.c_size_t(v_pool.stride(0)), page, ctypes.c_float(scale), _ptr(logits), V,
+        _ptr(scratch), ctypes.c_size_t(scratch.numel()), ctypes.c_void_p(control), DECODE_STACK_GRID,
+        ctypes.c_double(DECODE_STACK_CLOSE_US), ctypes.c_double(DECODE_STACK_LIMIT_US), _stream()))
 
 
 DECODE_PAIR_BLOCKS = 0          # blocks of several waves a (kv head, token) pair in single-token attention: 0 the kernel's own choice, 1 one or the split form

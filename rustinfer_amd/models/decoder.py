@@ -18,6 +18,7 @@ import torch
 from ..parts.base import PagedKVNeed, ParamSpec, Part, PositionEncoding, Runtime, join_name, narrow_tensors
 from ..parts.block import Hidden
 from ..parts.embed import Embedding, LMHead
+from .stack import decode_stack
 
 
 @dataclass(frozen=True)
@@ -60,6 +61,7 @@ class DecoderModel(Part):
             self.names.update(names)
         self.hidden_size = embed.dim
         self.vocab_size = lm_head.vocab_size
+        self.stack = None            # how steps of few single tokens run in one launch, where they can (set by load)
 
     # -- weights ---------------------------------------------------------
     def _children(self):
@@ -83,6 +85,7 @@ class DecoderModel(Part):
         for prefix, part in self._children():
             sub = narrow_tensors(tensors, prefix)
             part.load(sub, rt)
+        self.stack = decode_stack(self, rt)
 
     @property
     def graph_safe(self) -> bool:
@@ -114,6 +117,8 @@ class DecoderModel(Part):
     # -- one step ------------------------------------------------------------
     def forward(self, ctx, caches) -> torch.Tensor:
         """Run the tokens of ``ctx`` and return 32-bit logits [len(ctx.want_rows), vocab]."""
+        if self.stack is not None and self.stack.takes(ctx, caches):
+            return self.stack.forward(ctx, caches)       # few single tokens: all of it in one launch
         rt, ws = self.rt, ctx.workspace
         T = ctx.num_tokens
         x = ws.get("model.x", T, self.hidden_size, torch.float32)

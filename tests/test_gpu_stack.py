@@ -1,0 +1,125 @@
+"""Steps of few single tokens as one launch (csrc/decode_stack.hip), against the plain implementation: every form of the
+kernel, one row to eight with parts of long rows, first tokens, captured steps with padding rows, tokens that the host has not
+seen, blocks that arrive too late; and against the same step part by part."""
+import gc
+
+import numpy as np
+import pytest
+import torch
+
+import plain_llama
+from helpers import random_requests
+
+pytestmark = pytest.mark.gpu
+
+LAST = 3                                    # tokens of every row that are decoded one by one
+
+
+def _cfg(d, ff, H, Hkv, hd, V=512, L=2, tied=True):
+    return dict(architectures=["LlamaForCausalLM"], model_type="llama", hidden_size=d, intermediate_size=ff, num_hidden_layers=L,
+                num_attention_heads=H, num_key_value_heads=Hkv, head_dim=hd, vocab_size=V, max_position_embeddings=2048, rms_norm_eps=1e-5,
+                rope_theta=500000.0, tie_word_embeddings=tied, hidden_act="silu", eos_token_id=V - 1)
+
+
+# name -> sizes: each form of the kernel (head size; up to 4096 or 8192 wide; up to 8192 or 14336 between), at the least
+# sizes and at ones that leave the waves remainders
+CONFIGS = {
+    "64": _cfg(512, 512, 8, 2, 64, L=3), "64 uneven": _cfg(2560, 4608, 40, 8, 64, tied=False), "64 wide": _cfg(512, 1024, 72, 9, 64),
+    "64 one head": _cfg(512, 1536, 8, 1, 64, V=528), "128": _cfg(1024, 1536, 16, 4, 128, tied=False), "128 long": _cfg(512, 8704, 8, 2, 128),
+    "128 wide": _cfg(1024, 1024, 36, 9, 128), "128 longest": _cfg(512, 14336, 8, 2, 128),
+}
+LONG = [5 + LAST, 40, 100, 513, LAST, 32, 1200, 64]
+CASES = [("64", [5 + LAST], "eager", 0), ("64", LONG, "eager", 0), ("64", LONG[4:7], "graph", 0), ("64", LONG, "graph", 0),
+         ("64 uneven", LONG[2:7], "graph", 0), ("64 uneven", LONG[:6], "eager", 8), ("64 wide", LONG[3:6], "eager", 0),
+         ("64 one head", [1700, 3, 640], "graph", 0), ("128", LONG[1:5], "graph", 0), ("128", [900], "eager", 64),
+         ("128 long", [33, 600], "eager", 0), ("128 wide", LONG[:7], "eager", 0),
+         ("128 longest", LONG, "graph", 0)]
+
+
+@pytest.fixture(scope="module")
+def engines(tmp_path_factory):
+    made = {}
+
+    def get(name):
+        if name not in made:
+            from rustinfer_amd.config import LlamaConfig
+            from rustinfer_amd.engine import build_engine
+            from rustinfer_amd.weights import write_random_model
+            d = str(tmp_path_factory.mktemp("stack"))
+            write_random_model(LlamaConfig.from_dict(CONFIGS[name]), 7 + len(made), d)
+            eng = build_engine(d, dtype="bfloat16", page_size=16, num_pages=256, max_requests=8, max_model_len=2048, max_batch_tokens=2048)
+            made[name] = (eng, plain_llama.read_model(d))
+        return made[name]
+    return get
+
+
+def _decode(eng, reqs, mode):
+    """The rows' last tokens one by one, after the rest: logits [LAST, rows, V].  The rows are released."""
+    from rustinfer_amd.engine import StepEntry
+    eng.enable_graphs(mode == "graph", capture_sizes=(1, 2, 4, 8))
+    for r, t in reqs.items():
+        if len(t) > LAST:
+            eng.step([StepEntry(r, t[:-LAST], [])])
+    out = []
+    for s in range(LAST):
+        entries = []
+        for i, (r, t) in enumerate(reqs.items()):
+            token = t[len(t) - LAST + s]
+            if s == 1:                      # one that only the device has
+                eng.device_tokens[i] = token
+                token = -(i + 1)
+            entries.append(StepEntry(r, [token], [0]))
+        out.append(eng.step(entries).double().cpu().numpy())
+    for r in reqs:
+        eng.release(r)
+    eng.cache.check()
+    return np.stack(out)
+
+
+@pytest.mark.parametrize("name,lengths,mode,grid", CASES, ids=[f"{c[0]}-{len(c[1])}-{c[2]}-{c[3]}" for c in CASES])
+def test_steps_in_one_launch(engines, monkeypatch, name, lengths, mode, grid):
+    from rustinfer_amd.kernels import ops
+    eng, (cfg, w) = engines(name)
+    stack = eng.model.stack
+    assert stack is not None
+    launches = []
+    real = ops.decode_stack
+    monkeypatch.setattr(ops, "decode_stack", lambda *a, **k: (launches.append(1), real(*a, **k))[1])
+    monkeypatch.setattr(ops, "DECODE_STACK_GRID", grid)     # fewer than are waited for: the step goes on without the rest
+    reqs = random_requests(cfg["vocab_size"], lengths, seed=3)
+    got = _decode(eng, reqs, mode)
+    assert len(launches) == (LAST if mode == "eager" else 2)             # (a graph: the pass before its capture, and the capture)
+    try:
+        eng.model.stack = None
+        parts = _decode(eng, reqs, mode)
+        assert len(launches) == (LAST if mode == "eager" else 2)
+    finally:
+        eng.model.stack = stack
+        eng.enable_graphs(False)
+    want = np.stack([plain_llama.forward(cfg, w, t)[-LAST:] for t in reqs.values()], 1)
+    # rounding noise, the same for all rows and the same as part by part: the root of the mean square of a row's error is at most
+    # 2 % of the logits' deviation (a wrong key, page or weight tile gives 10 % and more), and in the mean that of the parts' rows but for a tenth
+    s = want.std()
+    rms, rms_parts = (np.sqrt(np.mean((v - want) ** 2, axis=2)) for v in (got, parts))
+    print(f"{name} {mode} {lengths}: {rms.max() / s:.2%}, part by part {rms_parts.max() / s:.2%}")
+    assert np.isfinite(got).all() and rms.max() <= 0.02 * s, rms / s
+    assert rms.mean() <= 1.1 * rms_parts.mean() + 1e-4 * s, (rms.mean() / s, rms_parts.mean() / s)
+
+
+def test_control_blocks_are_given_back():
+    """A block belongs to one workspace; one that is gone leaves its block to the next, and when all are taken there is none."""
+    from rustinfer_amd.engine.context import Workspace
+    from rustinfer_amd.kernels import ops
+    held, blocks = [], []
+    while True:
+        held.append(Workspace(torch.device("cuda")))
+        b = ops.decode_stack_control(held[-1])
+        if b is None:
+            break
+        assert b not in blocks and b == ops.decode_stack_control(held[-1])
+        blocks.append(b)
+    assert 0 < len(blocks) <= 64
+    freed = blocks[3 % len(blocks)]
+    del held[3 % len(blocks)]
+    gc.collect()
+    assert ops.decode_stack_control(held[-1]) == freed

@@ -114,3 +114,16 @@ def test_a_library_product_in_parts_is_asked_for_whole_where_a_part_is_refused(l
         assert calls(parts[1]) == (0, parts + [whole])
         assert calls(parts[0]) == (0, [parts[0], whole])
     assert calls(whole) == ((0, parts) if len(parts) == 2 else (2, [whole]))
+
+
+@pytest.mark.parametrize("change,takes", [
+    ({}, 1), (dict(M=1), 1), (dict(M=0), 0), (dict(M=9), 0), (dict(hd=32), 0), (dict(hd=96), 0), (dict(hd=64), 1), (dict(page=32), 0), (dict(d=2048 + 256), 0),
+    (dict(d=0), 0), (dict(d=8192), 1), (dict(d=8704), 0), (dict(H=34), 0), (dict(H=24), 1), (dict(H=64), 0), (dict(H=64, Hkv=16), 1), (dict(H=68, Hkv=17), 0),
+    (dict(H=32, hd=64, Hkv=2), 0), (dict(H=32, hd=64, Hkv=4), 1), (dict(ff=14336), 1), (dict(ff=14848), 0), (dict(ff=1184), 0), (dict(ff=0), 0),
+    (dict(V=1000), 0), (dict(V=0), 0), (dict(Hkv=0), 0), (dict(M=8, H=64, Hkv=64, hd=64), 0)])
+def test_steps_that_go_in_one_launch(lib, change, takes):
+    """What the kernel holds: eight rows, whole steps of K for its eight waves, 512 outputs of a group of heads, pages of 16."""
+    sizes = dict(M=8, d=2048, ff=8192, H=32, Hkv=8, hd=128, page=16, V=128256)
+    sizes.update(change)
+    assert lib.ri_decode_stack_takes(*sizes.values()) == takes
+    assert lib.ri_decode_stack_give_control(ctypes.c_void_p(4096)) != 0           # (never taken)
