@@ -23,7 +23,9 @@ from ..parts.rope import RotaryEmbedding
 class DecodeStack:
     def __init__(self, model, rt):
         """For a model that ``describes`` allows."""
-        self.model, self.rt = model, rt
+        # (no reference to the model, which holds this: an engine that is let go is freed at once)
+        self.rt, self.layers, self.hidden_size, self.vocab_size = rt, len(model.schedule), model.hidden_size, model.vocab_size
+        self.embedding = model.embed.weight
         blocks = [model.layers[c.layer] for c in model.schedule]
         first = blocks[0]
         self.H, self.Hkv, self.hd = first.mixer.num_heads, first.mixer.num_kv_heads, first.mixer.head_dim
@@ -79,18 +81,18 @@ class DecodeStack:
         if ctx.max_q_len != 1 or ctx.num_want != T or not getattr(ctx, "want_all_in_order", False) or ctx.num_rows < T:
             return False
         groups = getattr(caches, "groups", None)
-        if not groups or len(groups) != 1 or len(groups[0].cache_ids) != len(self.model.schedule):
+        if not groups or len(groups) != 1 or len(groups[0].cache_ids) != self.layers:
             return False
         ops = self.rt.ops
-        return ops.decode_stack_takes(T, self.model.hidden_size, self.ff, self.H, self.Hkv, self.hd, groups[0].page_size, self.model.vocab_size) \
+        return ops.decode_stack_takes(T, self.hidden_size, self.ff, self.H, self.Hkv, self.hd, groups[0].page_size, self.vocab_size) \
             and ops.decode_stack_control(ctx.workspace) is not None
 
     def forward(self, ctx, caches) -> torch.Tensor:
-        m, g = self.model, caches.groups[0]
-        logits = ctx.workspace.get("model.logits", ctx.num_tokens, m.vocab_size, torch.float32)
+        g = caches.groups[0]
+        logits = ctx.workspace.get("model.logits", ctx.num_tokens, self.vocab_size, torch.float32)
         scratch = ctx.workspace.get("model.stack", self.scratch_bytes // 256, 256, torch.uint8)
         cos, sin, _ = self.rope.rotary()
-        self.rt.ops.decode_stack(self.table, len(m.schedule), ctx, m.embed.weight, self.ff, self.H, self.Hkv, self.hd, cos, sin, g.k_pool, g.v_pool,
+        self.rt.ops.decode_stack(self.table, self.layers, ctx, self.embedding, self.ff, self.H, self.Hkv, self.hd, cos, sin, g.k_pool, g.v_pool,
                                  ctx.block_tables[g.index], g.page_size, self.scale, self.norm_dtype, scratch, logits)
         return logits
 

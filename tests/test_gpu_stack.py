@@ -2,6 +2,7 @@
 kernel, one row to eight with parts of long rows, first tokens, captured steps with padding rows, tokens that the host has not
 seen, blocks that arrive too late; and against the same step part by part."""
 import gc
+import weakref
 
 import numpy as np
 import pytest
@@ -123,3 +124,22 @@ def test_control_blocks_are_given_back():
     del held[3 % len(blocks)]
     gc.collect()
     assert ops.decode_stack_control(held[-1]) == freed
+
+
+def test_an_engine_is_freed_with_its_last_reference(tmp_path):
+    """Weights and cache go when the engine does, and not when Python next looks for cycles."""
+    from rustinfer_amd.config import LlamaConfig
+    from rustinfer_amd.engine import build_engine
+    from rustinfer_amd.weights import write_random_model
+    write_random_model(LlamaConfig.from_dict(CONFIGS["64"]), 5, str(tmp_path))
+    gc.collect()
+    gc.disable()
+    try:
+        eng = build_engine(str(tmp_path), dtype="bfloat16", page_size=16, num_pages=64, max_requests=8, max_model_len=512, max_batch_tokens=512)
+        _decode(eng, random_requests(512, [9, 40], seed=4), "eager")
+        assert eng.model.stack is not None
+        seen = [weakref.ref(eng.model), weakref.ref(eng.model.embed.weight)]
+        del eng
+        assert [r() for r in seen] == [None, None]
+    finally:
+        gc.enable()
