@@ -179,47 +179,122 @@ __global__ __launch_bounds__(WAVES * 64, 4) void gemm_f32_kernel(
     }
 }
 
-// Up to eight rows: a tile of the instruction holds eight rows and eight columns of W twice, once for each of two turns of K.
-// Lanes r < 8 of A and W hold the values of K of wave w, lanes r >= 8 those of wave w + 4, so the tile's upper left
-// quarter is the one wave's sum and the lower right the other's (the other two are not read): four waves do what the eight of
-// the kernel above do, in the same order, and a block takes 8 NT columns, so that a product of 2,048 columns gives every
+// Up to eight rows: a tile of the instruction holds eight rows and eight columns of W twice, once for each of two shares of K.
+// The eight waves of the kernel above are halves of four here: lanes r < 8 of A and W hold the values of K of its wave 2 w,
+// lanes r >= 8 those of 2 w + 1, so the tile's upper left quarter is the one's sum and the lower right the other's (the other two are not
+// read), made in the same order, and a block takes 8 NT columns, so that a product of 2,048 columns gives every
 // compute unit a block and no lane loads what another has.  D turns of each wave are under way at a time.  What bounds it is the
-// one pass over W.  Measured, us, 6 rows, tiles of 16 rows (half of them no row of the product) with loads that the compiled loop waited for / this
-// kernel: 2048 x 2048 10.3 / 6.7, 3072 x 2048 10.8 / 10.2, 16384 x 2048 41 / 31 (134 MB: 4.3 TB/s),
-// 2048 x 8192 33 / 17.6, 128256 x 2048 264 / 193 (5.4 TB/s).
+// one pass over W.  A load takes 128 bytes of each of eight rows, a whole line: the lanes' second half asks for what the first half multiplies
+// behind its own 64 bytes, and the two change places on the way to the instruction (with 64 bytes of 16 places a load every line was
+// asked for twice).  Measured, us, 1 and 8 rows, 64 bytes / this:
+// 2048 x 2048 7.3 7.6 / 6.9 7.1, 16384 x 2048 28.9 30.5 / 28.1 27.6, 2048 x 8192 16.3 18.9 / 16.9 18.1, 12288 x 1536 17.9 19.6 / 16.5 18.0, 8 rows
+// of 4096 x 14336 55.8 / 45.5 (235 MB: 5.2 TB/s), 13824 x 2560 43.4 / 35.7, 27648 x 5120 140 / 114, 128256 x 2048 203 / 186 (5.7 TB/s).
 // SWIGLU: W is [2N, K] (gate rows, then up rows), a block's two tiles are the gate's and the up rows of the same eight columns, and
-// C = silu(gate) * up of the rounded sums, in place of the activation's kernel (six requests generating 12 tokens at the 1B sizes 32.81 -> 32.64 ms:
-// two streams of eight rows take most of what the launch of 4.3 us gives back).
-template <int NT, int D, bool SWIGLU = false>
+// C = silu(gate) * up of the rounded sums, in place of the activation's kernel (8 rows of 2 x 8192 x 2048 33.2 / 30.3, 2 x 14336 x 4096 93 / 84).
+//
+// A norm between two such products has no kernel of its own, as in gemm.hip.  RESID (the product before it): C is the residual stream, C += sums, and what is left for the
+// product behind it are rows C * weight of the norm, 32-bit, and the sums of C^2 over the block's columns.  With `scale.ssq` a product finishes such a norm:
+// row m of its sums is multiplied by 1 / sqrt(mean of the row's squares + eps), in 64 bits, before it is rounded.  A result then passes two roundings of 32 bits
+// where the norm's kernel makes three.
+// ROPE: the product is q/k/v: a block's two tiles are eight features of a head's first half and the eight that they turn with; q goes to C, k and v to the pages.
+// Each saves a launch of 4.6 to 5.6 us.
+enum FewKind { FEW_PLAIN, FEW_SWIGLU, FEW_RESID, FEW_ROPE };
+struct FewScale { const float* ssq; int parts; float eps; };                            // ssq [M, parts]
+struct FewResid { const float* w; float* a; float* ssq; };                              // w [N]; a [M, N]; ssq [M, blocks]
+struct FewRope {
+    const float* cos_t; const float* sin_t;        // [positions][hd / 2]
+    const int* positions; const int* row_of_token; // of a row of A
+    const int* table; int max_blocks;              // block table [rows][max_blocks]
+    float* kc; float* vc;                          // k [pages][Hkv][page][hd], v [pages][Hkv][hd][page]
+    int H, Hkv, hd, page;
+};
+template <int NT, int D, FewKind KIND = FEW_PLAIN>
 __global__ __launch_bounds__(256) void gemm_f32_few_kernel(
         const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
-        float* __restrict__ C, int ldc, int M, int N, int K) {
+        float* __restrict__ C, int ldc, int M, int N, int K, const FewScale scale, const FewResid resid, const FewRope rope) {
     constexpr int TURN = 256;
+    constexpr bool TWO = KIND == FEW_SWIGLU || KIND == FEW_ROPE;       // two streams of eight rows of W
     __shared__ double sums[8][8][NT * 8];
+    __shared__ double factors[8];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     const int r = lane & 7, second = (lane >> 3) & 1, g = lane >> 4;
-    static_assert(!SWIGLU || NT == 2, "a tile of gate rows and one of up rows");
-    constexpr int COLS = SWIGLU ? 8 : NT * 8;
-    const int n0 = (int)blockIdx.x * COLS;
-    const char* abase = reinterpret_cast<const char*>(A + wave * 32);
-    const char* wbase = reinterpret_cast<const char*>(W + (size_t)n0 * ldw + wave * 32);
-    const char* ubase = SWIGLU ? reinterpret_cast<const char*>(W + ((size_t)N + n0) * ldw + wave * 32) : wbase;     // of the last tile
-    const int kl = second * 128 + 4 * g;
-    const uint32_t arow = ((uint32_t)min(r, M - 1) * (uint32_t)lda + kl) * 4;
+    static_assert(!TWO || NT == 2, "a tile of each");
+    static_assert(KIND != FEW_RESID || NT <= 2, "a row's columns of a block lie in 8 or 16 lanes");
+    constexpr int COLS = TWO ? 8 : NT * 8;
+    // the block's first row of W, and rows from there to the other stream's
+    const int per_head = KIND == FEW_ROPE ? rope.hd >> 4 : 1;
+    const int head = KIND == FEW_ROPE ? (int)blockIdx.x / per_head : 0, feature = KIND == FEW_ROPE ? ((int)blockIdx.x - head * per_head) * 8 : 0;
+    const int n0 = KIND == FEW_ROPE ? head * rope.hd + feature : (int)blockIdx.x * COLS;
+    const size_t apart = KIND == FEW_ROPE ? (size_t)(rope.hd >> 1) : (size_t)N;
+    const char* abase = reinterpret_cast<const char*>(A + wave * 64);
+    const char* wbase = reinterpret_cast<const char*>(W + (size_t)n0 * ldw + wave * 64);
+    const char* ubase = TWO ? reinterpret_cast<const char*>(W + (apart + n0) * ldw + wave * 64) : wbase;     // of the last tile
+    // of a wave's 64 values of a turn: the 16-byte pieces of W that a lane asks for lie at wl and wl + 32, the ones of A that it multiplies at al and al + 16
+    const int wl = second * 16 + 4 * g, al = second * 32 + 4 * g;
+    const uint32_t arow = ((uint32_t)min(r, M - 1) * (uint32_t)lda + al) * 4;
     uint32_t wrow[NT];
 #pragma unroll
-    for (int j = 0; j < NT; ++j) wrow[j] = ((uint32_t)min((SWIGLU ? 0 : j * 8) + r, N - 1 - n0) * (uint32_t)ldw + kl) * 4;
+    for (int j = 0; j < NT; ++j) wrow[j] = ((uint32_t)min((TWO ? 0 : j * 8) + r, N - 1 - n0) * (uint32_t)ldw + wl) * 4;
+    // What the end needs beside the sums is asked for behind the first turns of W.  This thread's result is row `row`, column `col` of the block's.
+    const int row = (int)threadIdx.x / COLS, col = (int)threadIdx.x % COLS;
+    const bool mine = row < M && n0 + col < N;       // (an own bound of `row`: M <= 8)
+    const bool scaled = KIND != FEW_RESID && scale.ssq != nullptr;
+    float4 squares[2] = {};                          // of rows `wave` and `wave + 4`
+    float x_own = 0.f, w_own = 0.f, cs = 1.f, sn = 0.f;
+    int pos = 0, entry = -1, blk = -1;
+    auto early = [&]() {
+        if (scaled) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+                if (wave + 4 * i < M && lane * 4 < scale.parts) squares[i] = *reinterpret_cast<const float4*>(scale.ssq + (size_t)(wave + 4 * i) * scale.parts + lane * 4);
+        }
+        if constexpr (KIND == FEW_RESID) {
+            if (mine) {
+                x_own = C[(size_t)row * ldc + n0 + col];
+                w_own = resid.w[n0 + col];
+            }
+        }
+        if constexpr (KIND == FEW_ROPE) {
+            if (wave == 0) {                         // (64 results: the first wave's)
+                // scalar loads, which do not stand behind the weights
+#pragma unroll
+                for (int m = 0; m < 8; ++m) {
+                    if (m >= M) break;
+                    const int b = rope.row_of_token[m], p = rope.positions[m];
+                    const int at = b >= 0 ? rope.table[(size_t)b * rope.max_blocks + p / rope.page] : -1;
+                    if (row == m) { entry = b; pos = p; blk = at; }
+                }
+                if (entry >= 0) {
+                    cs = rope.cos_t[(size_t)pos * (rope.hd >> 1) + feature + col];
+                    sn = rope.sin_t[(size_t)pos * (rope.hd >> 1) + feature + col];
+                }
+            }
+        }
+    };
     f64x4_t acc[NT] = {};
     auto ask = [&](int turn, float4 (&a)[2], float4 (&w)[2][NT]) {
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            const size_t at = ((size_t)turn * TURN + 16 * u) * 4;
+            const size_t at = (size_t)turn * TURN * 4;
 #pragma unroll
-            for (int j = 0; j < NT; ++j) w[u][j] = ld_stream16<float4>((j == NT - 1 ? ubase : wbase) + at + wrow[j]);
-            a[u] = *reinterpret_cast<const float4*>(abase + at + arow);
+            for (int j = 0; j < NT; ++j) w[u][j] = ld_stream16<float4>((j == NT - 1 ? ubase : wbase) + at + 128 * u + wrow[j]);
+            a[u] = *reinterpret_cast<const float4*>(abase + at + 64 * u + arow);
         }
     };
-    auto add = [&](const float4 (&a)[2], const float4 (&w)[2][NT]) {
+    // the lanes' first half has the pieces of its own two steps in w[0] of both halves, the second in w[1] of both
+    auto swapped = [&](float& p, float& q) {
+        const int sent = __float_as_int(second ? p : q), got = __builtin_amdgcn_mov_dpp(sent, 0x128, 0xf, 0xf, true);       // lane ^ 8
+        if (second) p = __int_as_float(got);
+        else q = __int_as_float(got);
+    };
+    auto add = [&](const float4 (&a)[2], float4 (&w)[2][NT]) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            swapped(w[0][j].x, w[1][j].x);
+            swapped(w[0][j].y, w[1][j].y);
+            swapped(w[0][j].z, w[1][j].z);
+            swapped(w[0][j].w, w[1][j].w);
+        }
 #pragma unroll
         for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -232,14 +307,15 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(
                 }
             }
     };
-    // turns that are whole for both halves of the lanes
-    const int left = K - wave * 32 - 160;
+    // turns of which the wave's 64 values are all there
+    const int left = K - wave * 64 - 64;
     const int whole = left >= 0 ? left / TURN + 1 : 0;
     float4 a[D][2], w[D][2][NT];
     if (whole >= D) {
         int turn = 0;
 #pragma unroll
         for (int d = 0; d < D; ++d) ask(d, a[d], w[d]);
+        early();
         for (; turn + 2 * D <= whole; turn += D) {
 #pragma unroll
             for (int d = 0; d < D; ++d) {
@@ -261,39 +337,88 @@ __global__ __launch_bounds__(256) void gemm_f32_few_kernel(
             __builtin_amdgcn_sched_barrier(0);
         }
     } else {
+        early();
         for (int turn = 0; turn < whole; ++turn) {
             ask(turn, a[0], w[0]);
             add(a[0], w[0]);
         }
     }
-    if (wave * 32 + whole * TURN < K) {          // a turn that ends within the lanes' chunks, or before the second half's
+    if (const int k0 = wave * 64 + whole * TURN; k0 < K) {           // a turn that ends within the wave's values
+        const size_t at = (size_t)whole * TURN * 4;
 #pragma unroll
         for (int u = 0; u < 2; ++u) {
-            const bool in = wave * 32 + whole * TURN + 16 * u + kl < K;
-            const size_t at = ((size_t)whole * TURN + 16 * u) * 4;
+            const bool in_w = k0 + 32 * u + wl < K, in_a = k0 + 16 * u + al < K;
 #pragma unroll
             for (int j = 0; j < NT; ++j)
-                w[0][u][j] = in ? *reinterpret_cast<const float4*>((j == NT - 1 ? ubase : wbase) + at + wrow[j]) : make_float4(0.f, 0.f, 0.f, 0.f);
-            a[0][u] = in ? *reinterpret_cast<const float4*>(abase + at + arow) : make_float4(0.f, 0.f, 0.f, 0.f);
+                w[0][u][j] = in_w ? *reinterpret_cast<const float4*>((j == NT - 1 ? ubase : wbase) + at + 128 * u + wrow[j]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            a[0][u] = in_a ? *reinterpret_cast<const float4*>(abase + at + 64 * u + arow) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         add(a[0], w[0]);
     }
 #pragma unroll
     for (int j = 0; j < NT; ++j)
 #pragma unroll
-        for (int e = 0; e < 2; ++e) sums[wave + 4 * second][4 * e + g][j * 8 + r] = second ? acc[j][2 + e] : acc[j][e];
-    __syncthreads();
-    auto sum = [&](int row, int col) {
-        double v = sums[0][row][col];
+        for (int e = 0; e < 2; ++e) sums[2 * wave + second][4 * e + g][j * 8 + r] = second ? acc[j][2 + e] : acc[j][e];
+    if (scaled) {
 #pragma unroll
-        for (int i = 1; i < 8; ++i) v += sums[i][row][col];
-        return (float)v;
+        for (int i = 0; i < 2; ++i) {
+            const int m = wave + 4 * i;
+            if (m >= M) break;
+            double s = ((double)squares[i].x + (double)squares[i].y) + ((double)squares[i].z + (double)squares[i].w);
+            for (int p = 256 + lane * 4; p < scale.parts; p += 256) {
+                const float4 v = *reinterpret_cast<const float4*>(scale.ssq + (size_t)m * scale.parts + p);
+                s += ((double)v.x + (double)v.y) + ((double)v.z + (double)v.w);
+            }
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o, 64);
+            if (lane == 0) factors[m] = 1.0 / sqrt(s / K + (double)scale.eps);
+        }
+    }
+    __syncthreads();
+    auto sum = [&](int m, int c) {
+        double v = sums[0][m][c];
+#pragma unroll
+        for (int i = 1; i < 8; ++i) v += sums[i][m][c];
+        return (float)(scaled ? v * factors[m] : v);
     };
-    for (int e = threadIdx.x; e < 8 * COLS; e += 256) {
-        const int row = e / COLS, col = e % COLS;
+    if (threadIdx.x >= 8 * COLS) return;             // COLS <= 32
+    if constexpr (KIND == FEW_RESID) {
+        float v = 0.f;
+        if (mine) {
+            v = x_own + sum(row, col);
+            C[(size_t)row * ldc + n0 + col] = v;
+            resid.a[(size_t)row * N + n0 + col] = v * w_own;
+        }
+        float sq = v * v;
+#pragma unroll
+        for (int o = COLS / 2; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 64);
+        if (row < M && col == 0) resid.ssq[(size_t)row * gridDim.x + blockIdx.x] = sq;
+    } else if constexpr (KIND == FEW_ROPE) {
+        if (row >= M || entry < 0) return;           // a padding token
+        const float p = sum(row, col), q = sum(row, 8 + col);
+        const float first = p * cs - q * sn, behind = p * sn + q * cs;
+        const int half = rope.hd >> 1, i = feature + col, slot = pos % rope.page;
+        if (head < rope.H) {
+            float* to = C + (size_t)row * ldc + n0 + col;
+            to[0] = first;
+            to[half] = behind;
+        } else if (blk >= 0) {
+            const int group = (head - rope.H) % rope.Hkv;
+            const size_t at = ((size_t)blk * rope.Hkv + group) * rope.page * rope.hd;
+            if (head < rope.H + rope.Hkv) {
+                float* to = rope.kc + at + (size_t)slot * rope.hd + i;
+                to[0] = first;
+                to[half] = behind;
+            } else {
+                float* to = rope.vc + at + (size_t)i * rope.page + slot;
+                to[0] = p;
+                to[(size_t)half * rope.page] = q;
+            }
+        }
+    } else if (mine) {
         float v = sum(row, col);
-        if (SWIGLU) v = v / (1.f + expf(-v)) * sum(row, 8 + col);
-        if (row < M && n0 + col < N) C[(size_t)row * ldc + n0 + col] = v;
+        if (KIND == FEW_SWIGLU) v = v / (1.f + expf(-v)) * sum(row, 8 + col);
+        C[(size_t)row * ldc + n0 + col] = v;
     }
 }
 
@@ -362,9 +487,9 @@ extern "C" void ri_gemm_f32_tile(int M, int N, int* rows, int* columns) {
     *columns = 16 * t.nt;
 }
 
-// The form of gemm_f32_few_kernel: 0: 8 columns a block and 4 turns under way, 1: 16 and 2, 2: 16 and 1, 3: 24 and 1.  Above 4,096 columns
+// The form of gemm_f32_few_kernel: 0: 8 columns a block and 4 turns under way, 1 and 2: 16 and 2, 3: 24 and 2.  Above 4,096 columns
 // the one whose rounds of 256 blocks take the least (*cost: in rounds of 8 columns a block); with fewer columns a block the rows of A
-// are read more often.  Measured, us, forms 0 / 2 / 3 at 1 and 8 rows: 6144 x 4096 20.7 26.4 / 26.7 29.7 / 21.9 22.9, 16384 x 2048
+// are read more often.  Measured with 64 bytes a load, us, forms 0 / 2 / 3 at 1 and 8 rows: 6144 x 4096 20.7 26.4 / 26.7 29.7 / 21.9 22.9, 16384 x 2048
 // 27.7 35.4 / 27.9 30.7 / 30.6 33.4, 12288 x 4096 37 48 / 40 43 / 37 41, 28672 x 4096 81 108 / 84 93 / 85 92, 128256 x 1024 95 134 / 97
 // 113 / 92 107; 0 / 1: 2048 x 8192 16 19 / 24 28, 4096 x 4096 14.8 18.6 / 16.1 17.1, 4096 x 14336 49 64 / 49 56.  (Two forms by
 // columns alone, before: 6144 x 4096 29, 16384 x 2048 29 32, 4096 x 14336 49 64.)
@@ -413,16 +538,77 @@ extern "C" int ri_gemm_f32_swiglu_pays(int M, int I, int K, int ldw) {
     return !(K > 2048 && gemm_f32_rows_pay(M, 2 * I, K, ldw) && (K > 3072 || !full));
 }
 
+static bool few_scale_ok(const float* ssq, int parts, float eps) {
+    return !ssq || (parts >= 4 && parts % 4 == 0 && eps >= 0.f && (uintptr_t)ssq % 16 == 0);
+}
+
+static void launch_few(int form, const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int N, int K, const FewScale& scale,
+                       hipStream_t stream) {
+    if (form == 0) gemm_f32_few_kernel<1, 4><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, scale, FewResid{}, FewRope{});
+    else if (form == 3) gemm_f32_few_kernel<3, 2><<<(N + 23) / 24, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, scale, FewResid{}, FewRope{});
+    else gemm_f32_few_kernel<2, 2><<<(N + 15) / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, scale, FewResid{}, FewRope{});
+}
+
+#define FEW_REQUIRE(who) \
+    RI_REQUIRE(M >= 1 && M <= 8 && N > 0 && K > 0 && K % 4 == 0, who ": needs 1 to 8 rows and K %% 4 == 0 (M=%d N=%d K=%d)", M, N, K); \
+    RI_REQUIRE(lda >= K && ldw >= K && lda % 4 == 0 && ldw % 4 == 0 && lda <= (1 << 24) && ldw <= (1 << 24), \
+               who ": leading dimensions must be >= K, multiples of 4 and at most 2^24"); \
+    RI_REQUIRE(A && W && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && N <= (1 << 26), who ": null or unaligned pointer, or N=%d", N)
+
 // C[M, N] = silu(A . gate^T) * (A . up^T) of up to eight rows, W = [gate; up] of 2N rows: what the tiles of ri_gemm_f32 and the activation's
-// kernel give, bit for bit.
+// kernel give, bit for bit.  ssq [M, parts] (or null): see ri_gemm_f32_scaled.
 extern "C" int ri_gemm_f32_swiglu(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
-                                  int M, int N, int K, hipStream_t stream) {
-    RI_REQUIRE(M >= 1 && M <= 8 && N > 0 && K > 0 && K % 4 == 0, "ri_gemm_f32_swiglu: needs 1 to 8 rows and K %% 4 == 0 (M=%d N=%d K=%d)", M, N, K);
-    RI_REQUIRE(lda >= K && ldw >= K && ldc >= N && lda % 4 == 0 && ldw % 4 == 0 && lda <= (1 << 24) && ldw <= (1 << 24),
-               "ri_gemm_f32_swiglu: leading dimensions must be >= K, multiples of 4 and at most 2^24");
-    RI_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0 && N <= (1 << 26), "ri_gemm_f32_swiglu: null or unaligned pointer, or N=%d", N);
-    gemm_f32_few_kernel<2, 1, true><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K);
+                                  int M, int N, int K, const float* ssq, int parts, float eps, hipStream_t stream) {
+    FEW_REQUIRE("ri_gemm_f32_swiglu");
+    RI_REQUIRE(C && ldc >= N && few_scale_ok(ssq, parts, eps), "ri_gemm_f32_swiglu: bad result or partial sums of squares");
+    gemm_f32_few_kernel<2, 2, FEW_SWIGLU><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, FewScale{ssq, parts, eps}, FewResid{}, FewRope{});
     RI_LAUNCHED("ri_gemm_f32_swiglu");
+    return 0;
+}
+
+// C[M, N] = (A . W^T) of up to eight rows, row m times 1 / sqrt(sum(ssq[m]) / K + eps): ssq [M, parts], a multiple of 4 of them, as ri_gemm_f32_residual leaves them.
+extern "C" int ri_gemm_f32_scaled(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
+                                  int M, int N, int K, const float* ssq, int parts, float eps, hipStream_t stream) {
+    FEW_REQUIRE("ri_gemm_f32_scaled");
+    RI_REQUIRE(C && ldc >= N && ssq && few_scale_ok(ssq, parts, eps), "ri_gemm_f32_scaled: bad result or partial sums of squares");
+    float cost = 0.f;
+    launch_few(few_form(M, N, K, &cost), A, lda, W, ldw, C, ldc, M, N, K, FewScale{ssq, parts, eps}, stream);
+    RI_LAUNCHED("ri_gemm_f32_scaled");
+    return 0;
+}
+
+// Partial sums of squares that ri_gemm_f32_residual leaves of a row of N values: one for 8 or 16 columns, as ri_gemm_f32's form has them.
+extern "C" int ri_gemm_f32_residual_parts(int M, int N, int K) {
+    float cost = 0.f;
+    return N / (few_form(M, N, K, &cost) == 0 ? 8 : 16);
+}
+
+// x[M, N] += A . W^T of up to eight rows, and for the norm behind it (weights norm_w [N]) a[M, N] = x * norm_w and partial sums of x^2, ssq [M, parts].  N % 64 == 0.
+extern "C" int ri_gemm_f32_residual(const float* A, int lda, const float* W, int ldw, int M, int N, int K, float* x, const float* norm_w, float* a, float* ssq,
+                                    hipStream_t stream) {
+    FEW_REQUIRE("ri_gemm_f32_residual");
+    RI_REQUIRE(N % 64 == 0 && x && norm_w && a && ssq, "ri_gemm_f32_residual: null pointer, or N=%d", N);
+    const FewResid resid{norm_w, a, ssq};
+    if (ri_gemm_f32_residual_parts(M, N, K) == N / 8) gemm_f32_few_kernel<1, 4, FEW_RESID><<<N / 8, 256, 0, stream>>>(A, lda, W, ldw, x, N, M, N, K, FewScale{}, resid, FewRope{});
+    else gemm_f32_few_kernel<2, 2, FEW_RESID><<<N / 16, 256, 0, stream>>>(A, lda, W, ldw, x, N, M, N, K, FewScale{}, resid, FewRope{});
+    RI_LAUNCHED("ri_gemm_f32_residual");
+    return 0;
+}
+
+// q/k/v [M, (H + 2 Hkv) hd] of up to eight tokens, q and k turned by the token's position over the whole head: q to the first H hd columns of C, k and v to the
+// token's page.  Tokens of no request (row_of_token < 0) leave nothing.  ssq: see ri_gemm_f32_scaled, or null.
+extern "C" int ri_gemm_f32_qkv_rope(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M, int K, int H, int Hkv, int hd,
+                                    const float* cos_t, const float* sin_t, const int* positions, const int* row_of_token, float* kc, float* vc,
+                                    const int* table, int max_blocks, int page, const float* ssq, int parts, float eps, hipStream_t stream) {
+    RI_REQUIRE(H >= 1 && Hkv >= 1 && hd >= 16 && hd % 16 == 0 && H <= (1 << 12) && Hkv <= (1 << 12) && hd <= (1 << 12) && page >= 1 && max_blocks >= 1,
+               "ri_gemm_f32_qkv_rope: bad sizes H=%d Hkv=%d hd=%d page=%d", H, Hkv, hd, page);
+    const int N = (H + 2 * Hkv) * hd;
+    FEW_REQUIRE("ri_gemm_f32_qkv_rope");
+    RI_REQUIRE(C && ldc >= H * hd && cos_t && sin_t && positions && row_of_token && kc && vc && table && few_scale_ok(ssq, parts, eps),
+               "ri_gemm_f32_qkv_rope: null pointer, or bad result or partial sums of squares");
+    const FewRope rope{cos_t, sin_t, positions, row_of_token, table, max_blocks, kc, vc, H, Hkv, hd, page};
+    gemm_f32_few_kernel<2, 2, FEW_ROPE><<<N / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K, FewScale{ssq, parts, eps}, FewResid{}, rope);
+    RI_LAUNCHED("ri_gemm_f32_qkv_rope");
     return 0;
 }
 
@@ -437,13 +623,8 @@ extern "C" int ri_gemm_f32(const float* A, int lda, const float* W, int ldw, flo
     if (M <= 4 && (lda > (1 << 24) || ldw > (1 << 24))) return ri_gemm_rows_f32(A, lda, W, ldw, C, ldc, M, N, K, stream);
     if (lda > (1 << 24) || ldw > (1 << 24)) return ri_gemm_tiled(A, lda, W, ldw, C, ldc, M, N, K, RI_F32, RI_F32, stream);
     if (const int form = ri_gemm_f32_form(M, N, K, ldw); form < 4) {
-        switch (form) {
-            case -1: return ri_gemm_rows_f32(A, lda, W, ldw, C, ldc, M, N, K, stream);
-            case 0: gemm_f32_few_kernel<1, 4><<<(N + 7) / 8, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K); break;
-            case 1: gemm_f32_few_kernel<2, 2><<<(N + 15) / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K); break;
-            case 2: gemm_f32_few_kernel<2, 1><<<(N + 15) / 16, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K); break;
-            default: gemm_f32_few_kernel<3, 1><<<(N + 23) / 24, 256, 0, stream>>>(A, lda, W, ldw, C, ldc, M, N, K); break;
-        }
+        if (form < 0) return ri_gemm_rows_f32(A, lda, W, ldw, C, ldc, M, N, K, stream);
+        launch_few(form, A, lda, W, ldw, C, ldc, M, N, K, FewScale{}, stream);
         RI_LAUNCHED("ri_gemm_f32");
         return 0;
     }

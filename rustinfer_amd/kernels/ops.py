@@ -359,6 +359,33 @@ def qkv_rope_fused(x: torch.Tensor, w_fused: torch.Tensor, qkv: torch.Tensor, H:
     return True
 
 
+def qkv_rope_f32(x: torch.Tensor, w: torch.Tensor, qkv: torch.Tensor, H: int, Hkv: int, hd: int, rotary, positions: torch.Tensor,
+                 row_of_token: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor, block_table: torch.Tensor, page: int, scale=None) -> bool:
+    """``qkv_rope_fused`` for up to eight 32-bit rows and the weight as it is: 64-bit sums, q and k rotated over whole heads."""
+    M, K = x.shape
+    if FORCE_LIBRARY_GEMM or rotary is None or not 0 < M <= 8 or hd % 16 or K % 128 or not _f32_rows_ok(x, w) or qkv.dtype != torch.float32:
+        return False
+    cos, sin, rot = rotary
+    if rot != hd:
+        return False
+    _dev(x, w, qkv, cos, sin, positions, row_of_token, k_cache, v_cache, block_table)
+    if tuple(w.shape) != ((H + 2 * Hkv) * hd, K) or qkv.shape[0] != M or qkv.shape[1] < H * hd:
+        raise KernelError("qkv_rope_f32: shapes do not fit")
+    _rows2d(qkv, "qkv")
+    _check_cache(k_cache, v_cache, Hkv, hd, page, x.dtype, "qkv_rope_f32")
+    _i32(positions, "positions", M)
+    _i32(row_of_token, "row_of_token", M)
+    _i32(block_table, "block_table")
+    if block_table.dim() != 2 or cos.dtype != torch.float32 or sin.dtype != torch.float32 or cos.shape != sin.shape or cos.shape[1] * 2 != hd \
+            or not cos.is_contiguous() or not sin.is_contiguous():
+        raise KernelError("qkv_rope_f32: block_table must be [rows, max_blocks], cos/sin contiguous float32 [positions, head_dim/2]")
+    sq, sp, se = _scale_args(scale, M, "qkv_rope_f32")
+    _check(_lib().ri_gemm_f32_qkv_rope(
+        _ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(qkv), qkv.stride(0), M, K, H, Hkv, hd, _ptr(cos), _ptr(sin), _ptr(positions),
+        _ptr(row_of_token), _ptr(k_cache), _ptr(v_cache), _ptr(block_table), block_table.shape[1], page, sq, sp, se, _stream()))
+    return True
+
+
 def _mid_plan(M: int, N: int, K: int, swiglu: bool, rotated: bool = False):
     """(slices of K, whether blocks own 8 weight tiles) of ``ri_gemm_mid`` for this product; 0 slices: not its kind."""
     parts, wide = ctypes.c_int(0), ctypes.c_int(0)
@@ -437,9 +464,18 @@ def qkv_rope_split(x: torch.Tensor, w_fused: torch.Tensor, qkv: torch.Tensor, H:
 DEFERRED_NORM_MAX_ROWS = 16
 
 
+def _f32_rows_ok(*tensors: torch.Tensor) -> bool:
+    """Whether the rows of 32-bit operands lie as the kernels of few rows read them."""
+    return all(t.dtype == torch.float32 and t.stride(-1) == 1 and t.stride(0) % 4 == 0 and t.stride(0) <= 1 << 24 and t.data_ptr() % 16 == 0 for t in tensors)
+
+
 def linear_residual_ok(M: int, w: torch.Tensor, w_tiled: Optional[torch.Tensor], norm_weight: torch.Tensor) -> bool:
     """Whether ``linear_residual`` takes ``M`` rows against ``w [N, K]`` before a norm with this weight."""
     N, K = w.shape
+    if w.dtype == torch.float32:
+        # csrc/gemm_f32.hip; whole chunks of K for this product and for the one behind the norm
+        return (0 < M <= min(8, DEFERRED_NORM_MAX_ROWS) and N % 128 == 0 and K % 128 == 0 and _f32_rows_ok(w) and norm_weight.dtype == torch.float32
+                and norm_weight.numel() == N and norm_weight.is_contiguous())
     return (not FORCE_LIBRARY_GEMM and w.dtype == torch.bfloat16 and w_tiled is not None and 0 < M <= DEFERRED_NORM_MAX_ROWS
             and N % 16 == 0 and K % 32 == 0 and norm_weight.dtype in _DT and norm_weight.numel() == N
             and norm_weight.is_contiguous())
@@ -449,8 +485,8 @@ RESIDUAL_FORM_LARGE = 32 << 20  # elements of a weight from which the residual f
 
 
 def linear_residual_pays(M: int, w: torch.Tensor) -> bool:
-    """Whether ``linear_residual`` is the faster way for ``M`` rows against ``w [N, K]``, compared
-    with partial sums over slices of K and the norm's own kernel (which costs 3 to 6 us).  A block of
+    """Whether ``linear_residual`` is the faster way for ``M`` bfloat16 rows against ``w [N, K]`` (32-bit rows: always, the product is the
+    same as without it), compared with partial sums over slices of K and the norm's own kernel (which costs 3 to 6 us).  A block of
     the residual form owns 16 whole columns (8 in ri_gemm_skinny_residual's other forms): it cannot divide K between blocks, so every block asks
     for all of its rows' activations (beyond eight rows that shows), and 320 blocks on 256 compute
     units take as long as 512.  Measured, us, residual form / partial sums and the norm, at 1, 8, 16 rows:
@@ -471,17 +507,24 @@ def linear_residual_pays(M: int, w: torch.Tensor) -> bool:
 def linear_residual(act: torch.Tensor, w: torch.Tensor, w_tiled: Optional[torch.Tensor], x: torch.Tensor,
                     norm_weight: torch.Tensor, workspace, name: str):
     """``x += act @ w^T`` in place (32-bit residual stream), and for the norm that follows:
-    ``a = x * norm_weight`` in bfloat16 and partial sums of ``x^2``, ``ssq [M, P]``.  Returns
+    ``a = x * norm_weight`` in the dtype of ``w`` and partial sums of ``x^2``, ``ssq [M, P]``.  Returns
     ``(a, ssq)``.  For the shapes ``linear_residual_ok`` accepts."""
     M, K = act.shape
     N = w.shape[0]
-    if not linear_residual_ok(M, w, w_tiled, norm_weight) or not _skinny_ok(act, w, M, K) or w.shape[1] != K:
+    exact = w.dtype == torch.float32
+    if not linear_residual_ok(M, w, w_tiled, norm_weight) or not (_f32_rows_ok(act) if exact else _skinny_ok(act, w, M, K)) or w.shape[1] != K:
         raise KernelError(f"linear_residual: {tuple(act.shape)} x {tuple(w.shape)}^T is not a shape this form takes")
-    _dev(act, w_tiled, x, norm_weight)
-    _tiled_ok(w, w_tiled)
+    _dev(act, w if exact else w_tiled, x, norm_weight)
+    if not exact:
+        _tiled_ok(w, w_tiled)
     if x.dtype != torch.float32 or tuple(x.shape) != (M, N) or not x.is_contiguous():
         raise KernelError(f"linear_residual: x must be contiguous float32 [{M}, {N}]")
     lib = _lib()
+    if exact:
+        a = workspace.get(name + ".a", M, N, torch.float32)
+        ssq = workspace.get(name + ".ssq", M, lib.ri_gemm_f32_residual_parts(M, N, K), torch.float32)
+        _check(lib.ri_gemm_f32_residual(_ptr(act), act.stride(0), _ptr(w), w.stride(0), M, N, K, _ptr(x), _ptr(norm_weight), _ptr(a), _ptr(ssq), _stream()))
+        return a, ssq
     parts = lib.ri_gemm_skinny_residual_parts(M, N)      # a slot of partial sums for every 16 (or 8) columns
     a = workspace.get(name + ".a", M, N, torch.bfloat16)
     ssq = workspace.get(name + ".ssq", M, parts, torch.float32)
@@ -905,8 +948,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled=None,
     ``w_tiled`` (from ``tile_weight``) is read instead of ``w`` where the kernel has a use for it (the digits of a float32
     weight: with a ``workspace`` to hold those of ``x``).
     ``scale = (ssq [M, P], eps)``: the rows of ``x`` are ``(r * w_norm)`` of a norm this product
-    finishes: row m of the result is multiplied by ``rsqrt(sum(ssq[m]) / K + eps)`` (few bfloat16
-    rows only)."""
+    finishes: row m of the result is multiplied by ``rsqrt(sum(ssq[m]) / K + eps)`` (few rows
+    only)."""
     _dev(x, w, out)
     _rows2d(x, "x")
     _rows2d(w, "w")
@@ -934,8 +977,12 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled=None,
                                            _ptr(out), out.stride(0), M, N, K, _dt(out), 0, 1,
                                            ctypes.c_longlong(0), int(tiled), sq, sp, se, _stream()))
             return
+    if scale is not None and 0 < M <= 8 and out.dtype == torch.float32 and _f32_rows_ok(x, w) and K % 4 == 0:
+        sq, sp, se = _scale_args(scale, M, "linear")
+        _check(lib.ri_gemm_f32_scaled(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), M, N, K, sq, sp, se, _stream()))
+        return
     if scale is not None:
-        raise KernelError("linear: row factors of a deferred norm go with the few-row bfloat16 kernel only")
+        raise KernelError("linear: row factors of a deferred norm go with the kernels of few rows only")
     if x.dtype == torch.bfloat16:
         if ((LIBRARY_GEMM_MIN_ROWS and M >= LIBRARY_GEMM_MIN_ROWS) or FORCE_LIBRARY_GEMM or to_library) \
                 and out.dtype in (torch.bfloat16, torch.float32):
@@ -1082,14 +1129,19 @@ def linear_swiglu(x: torch.Tensor, w_gate_up: torch.Tensor, out: torch.Tensor,
             _check(_lib().ri_gemm_mid(_ptr(x), x.stride(0), _ptr(w_tiled), _ptr(out), out.stride(0), M, I, K, 1, 1, wide,
                                       ctypes.c_longlong(0), _stream()))
             return
+    if scale is not None and M <= 8 and K % 4 == 0 and _f32_rows_ok(x, w_gate_up):
+        sq, sp, se = _scale_args(scale, M, "linear_swiglu")
+        _check(_lib().ri_gemm_f32_swiglu(_ptr(x), x.stride(0), _ptr(w_gate_up), w_gate_up.stride(0), _ptr(out), out.stride(0), M, I, K, sq, sp, se, _stream()))
+        return
     if scale is not None:
-        raise KernelError("linear_swiglu: row factors of a deferred norm go with the few-row bfloat16 kernel only")
+        raise KernelError("linear_swiglu: row factors of a deferred norm go with the kernels of few rows only")
     if scratch is None or tuple(scratch.shape) != (M, 2 * I):
         raise KernelError("linear_swiglu: needs scratch [M, 2I] for this size")
     if x.dtype == torch.float32 and M <= 8 and K % 4 == 0 and all(t.stride(0) % 4 == 0 and t.stride(0) <= 1 << 24 and t.data_ptr() % 16 == 0 for t in (x, w_gate_up)) \
             and (_lib().ri_gemm_f32_swiglu_pays(M, I, K, w_gate_up.stride(0)) or not (out.is_contiguous() and scratch.is_contiguous())):
         # the exact path's few rows: the activation in the product's epilogue, on the rounded sums (the activation's kernel takes whole buffers only)
-        _check(_lib().ri_gemm_f32_swiglu(_ptr(x), x.stride(0), _ptr(w_gate_up), w_gate_up.stride(0), _ptr(out), out.stride(0), M, I, K, _stream()))
+        _check(_lib().ri_gemm_f32_swiglu(_ptr(x), x.stride(0), _ptr(w_gate_up), w_gate_up.stride(0), _ptr(out), out.stride(0), M, I, K,
+                                         ctypes.c_void_p(0), 0, ctypes.c_float(0.0), _stream()))
         return
     linear(x, w_gate_up, scratch, w_tiled if isinstance(w_tiled, DigitWeight) else None, workspace=workspace)
     swiglu(scratch, out)

@@ -111,6 +111,10 @@ class PagedAttention(Mixer):
             fused = ops.qkv_rope_fused(*args, **kw) or (
                 scale is None and split is not None
                 and ops.qkv_split_pays(rows.shape[0], self.qkv_fused.shape[0], self.qkv_fused.shape[1]) and split(*args, ws))
+        few = getattr(ops, "qkv_rope_f32", None)
+        if not fused and few is not None and rows.dtype == torch.float32 and self.own_kv and self.qk_transform is None and cache.write:
+            fused = few(rows, self.qkv.weight, qkv, self.num_heads, self.num_kv_heads, self.head_dim, rotary,
+                        ctx.positions, ctx.row_of_token, cache.k, cache.v, table, cache.page_size, **kw)
         if not fused:
             self.qkv.forward(rows, qkv, scale, workspace=ws)
             if self.qk_transform is not None:
@@ -139,7 +143,7 @@ class PagedAttention(Mixer):
         if ok is None or not ok(x.shape[0], self.o.weight, self.o.weight_tiled, next_norm.weight):
             return None
         pays = getattr(ops, "linear_residual_pays", None)
-        if pays is not None and not pays(x.shape[0], self.o.weight):
+        if pays is not None and self.rt.dtype != torch.float32 and not pays(x.shape[0], self.o.weight):
             return None
         qkv, table = self._project(ctx, normed, cache)
         attn = self._attend(ctx, qkv, cache, table)

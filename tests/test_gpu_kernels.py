@@ -2108,3 +2108,73 @@ def test_unary_in_wide_and_single_elements(ops, name, T, n, pad, shift):
         assert torch.equal(out[:, 3:], (z.clamp(min=0) ** 2).to(torch.bfloat16)[:, 3:])
     ops.unary(fn, x, x)
     assert torch.equal(x.contiguous().view(torch.int16), single.contiguous().view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 128, 128), (8, 384, 256), (3, 2176, 128), (6, 3072, 2048), (5, 4224, 640), (7, 2048, 384), (2, 8192, 128)])
+def test_a_norm_between_32bit_products_of_few_rows(ops, M, N, K):
+    """The product before the norm and each kind of product behind it, against 64 bits: 8 and 16 columns a block, fewer and more partial
+    sums of squares than lanes ask for at once, rows of the stream that are not finite with their own results only."""
+    from rustinfer_amd.engine.context import Workspace
+    ws = Workspace(torch.device(DEV))
+    act, w, x0, wn = rnd(M, K, seed=M), rnd(N, K, seed=N) * 0.1, rnd(M, N, seed=3), 1 + 0.2 * rnd(N, seed=4)
+    assert ops.linear_residual_ok(M, w, None, wn) and not ops.linear_residual_ok(9, w, None, wn)
+    x = x0.clone()
+    a, ssq = ops.linear_residual(act, w, None, x, wn, ws, "t")
+    want = x0.double() + act.double() @ w.double().t()
+    # the sum rounded to 32 bits, the addition, and one product with the norm's weight
+    scale = x0.double().abs() + (act.double() @ w.double().t()).abs()
+    assert torch.all((x.double() - want).abs() <= 2.0 ** -23 * scale)
+    assert torch.all((a.double() - want * wn.double()).abs() <= 2.0 ** -22 * scale * wn.double().abs())
+    squares = want.square().sum(1)
+    assert torch.all((ssq.double().sum(1) - squares).abs() <= 2.0 ** -18 * squares)
+    eps = 1e-5
+    n = want * torch.rsqrt(squares[:, None] / N + eps) * wn.double()
+    I = 72
+    wo = rnd(2 * I, N, seed=5) * (4.0 / N) ** 0.5
+    ref = n @ wo.double().t()
+    # each row's operand is off by 2^-22 of the largest terms at most, in any direction
+    slack = 2.0 ** -20 * ((scale * torch.rsqrt(squares[:, None] / N + eps) * wn.double().abs()) @ wo.double().abs().t()) + 2.0 ** -18 * ref.abs()
+    out = torch.full((M, 2 * I + 3), float("nan"), device=DEV)
+    ops.linear(a, wo, out[:, :2 * I], scale=(ssq, eps))
+    assert torch.all((out[:, :2 * I].double() - ref).abs() <= slack) and out[:, 2 * I:].isnan().all()
+    gated = torch.full((M, I + 1), float("nan"), device=DEV)
+    ops.linear_swiglu(a, wo, gated[:, :I], None, scale=(ssq, eps))
+    both = torch.nn.functional.silu(ref[:, :I]) * ref[:, I:]
+    # silu moves by at most 1.1 times what its argument does, and is at most the argument
+    assert torch.all((gated[:, :I].double() - both).abs() <= 1.1 * slack[:, :I] * ref[:, I:].abs() + slack[:, I:] * (ref[:, :I].abs() + slack[:, :I]) + 2.0 ** -20 * both.abs() + 1e-7)
+    if M > 1:
+        bad = x0.clone()
+        bad[M - 1, N - 1] = float("nan")
+        b, bq = ops.linear_residual(act, w, None, bad, wn, ws, "u")
+        other = torch.empty(M, 2 * I, device=DEV)
+        ops.linear(b, wo, other, scale=(bq, eps))
+        assert torch.equal(other[:M - 1], out[:M - 1, :2 * I]) and other[M - 1].isnan().all()
+
+
+@pytest.mark.parametrize("M,H,Hkv,hd,K", [(1, 1, 1, 16, 128), (8, 4, 2, 64, 256), (5, 6, 3, 48, 640), (7, 8, 2, 128, 2048)])
+def test_qkv_f32_of_few_rows_with_rotation_and_pages(ops, M, H, Hkv, hd, K):
+    """q in place, k and v in the pages, against the product and the kernel that rotates; a token of no request and one without a page leave nothing."""
+    page, rows, blocks = 16, 3, 8
+    x, w = rnd(M, K, seed=1), rnd((H + 2 * Hkv) * hd, K, seed=2) * 0.1
+    ang = torch.arange(128, device=DEV)[:, None] * (10000.0 ** (-torch.arange(hd // 2, device=DEV) / (hd / 2)))
+    rotary = (ang.cos().float().contiguous(), ang.sin().float().contiguous(), hd)
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=DEV)  # noqa: E731
+    positions = i32([(19 * i + 5) % 100 for i in range(M)])
+    row_of_token = i32([(i % rows) if i != 3 else -1 for i in range(M)])
+    table = torch.randperm(24, device=DEV).to(torch.int32)[:rows * blocks].view(rows, blocks).contiguous()
+    if M > 4:
+        table[4 % rows, int(positions[4]) // page] = -1
+    got, want = [[torch.full((M, (H + 2 * Hkv) * hd), 7.0, device=DEV), torch.full((24, Hkv, page, hd), 9.0, device=DEV), torch.full((24, Hkv, hd, page), 9.0, device=DEV)] for _ in range(2)]
+    ssq = (x.double().square().view(M, 4, -1).sum(2)).float().contiguous()
+    factor = torch.rsqrt(x.double().square().mean(1, keepdim=True) + 1e-5)
+    for scale in (None, (ssq, 1e-5)):
+        assert ops.qkv_rope_f32(x, w, got[0], H, Hkv, hd, rotary, positions, row_of_token, got[1], got[2], table, page, scale=scale)
+        full = x.double() @ w.double().t()
+        want[0].copy_(full if scale is None else full * factor)
+        ops.rope_kv_write(want[0], H, Hkv, hd, rotary, positions, row_of_token, want[1], want[2], table, page)
+        live = row_of_token >= 0
+        # both round the same sums (the factor's own error aside) and turn them: three 32-bit operations on either side
+        size = (x.double().abs() @ w.double().abs().t()).max() * (1 if scale is None else factor.max())
+        for a, b in ((got[0][live, :H * hd], want[0][live, :H * hd]), (got[1], want[1]), (got[2], want[2])):
+            assert (a - b).abs().max() <= 2.0 ** -20 * size
+    assert not ops.qkv_rope_f32(rnd(9, K, seed=1), w, rnd(9, (H + 2 * Hkv) * hd, seed=1), H, Hkv, hd, rotary, positions, row_of_token, got[1], got[2], table, page)
