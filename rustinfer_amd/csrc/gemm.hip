@@ -862,9 +862,12 @@ extern "C" int ri_gemm_skinny_bf16(const void* A, int lda, const void* W, int ld
 }
 
 // C[M, N] = A . W^T in bfloat16 (W in tile order) with one or two stretches of columns activated (see ActivationEpilogue):
-// columns [from, to), multiples of 16 (or `to` = N), leave as op(sum) in dst [M][ld].
+// columns [from, to), multiples of 16 (or `to` = N), leave as op(sum) in dst [M][ld].  ssq: row factors of a norm folded into this product (see RowScale), or null.
 extern "C" int ri_gemm_skinny_activated(const void* A, int lda, const void* W, void* C, int ldc, int M, int N, int K, int count,
-                                        const int* from, const int* to, const int* op, void* const* dst, const int* ld, hipStream_t stream) {
+                                        const int* from, const int* to, const int* op, void* const* dst, const int* ld,
+                                        const float* ssq, int ssq_parts, float eps, hipStream_t stream) {
+    RowScale sc;
+    if (int rc = row_scale(ssq, ssq_parts, eps, K, &sc, "ri_gemm_skinny_activated")) return rc;
     RI_REQUIRE(M >= 1 && M <= 64 && N > 0 && N % 16 == 0 && K > 0 && K % 32 == 0, "ri_gemm_skinny_activated: bad sizes M=%d N=%d K=%d", M, N, K);
     RI_REQUIRE(lda >= K && lda % 8 == 0 && ldc >= N, "ri_gemm_skinny_activated: leading dimensions must be >= K (a multiple of 8) and >= N");
     RI_REQUIRE(A && W && C && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0, "ri_gemm_skinny_activated: null or unaligned pointer");
@@ -876,7 +879,7 @@ extern "C" int ri_gemm_skinny_activated(const void* A, int lda, const void* W, v
         RI_REQUIRE((op[x] == 0 || op[x] == 1) && dst[x] && ld[x] >= to[x] - from[x], "ri_gemm_skinny_activated: bad stretch %d", x);
         ae.from[x] = from[x]; ae.to[x] = to[x]; ae.op[x] = op[x]; ae.dst[x] = (bf16_t*)dst[x]; ae.ld[x] = ld[x];
     }
-    return dispatch_skinny<bf16_t, false>((const bf16_t*)A, lda, (const bf16_t*)W, K, (bf16_t*)C, ldc, M, N, K, 1, 0, 1, RowScale{nullptr, 0, 0.f, 0.f}, stream, ae);
+    return dispatch_skinny<bf16_t, false>((const bf16_t*)A, lda, (const bf16_t*)W, K, (bf16_t*)C, ldc, M, N, K, 1, 0, 1, sc, stream, ae);
 }
 
 // The product before a norm, for M <= 16 rows (see ResidualEpilogue):

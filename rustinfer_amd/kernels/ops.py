@@ -1018,13 +1018,14 @@ def linear(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled=None,
                              M, N, K, _dt(x), _dt(out), _stream()))
 
 
-def linear_activated(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled, acts, workspace=None) -> None:
+def linear_activated(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tiled, acts, workspace=None, scale=None) -> None:
     """``linear``, and for each ``(c0, n, name, dst)`` of ``acts``: ``dst [M, n] = f(out[:, c0:c0 + n])`` for ``f`` in
     ``UNARY``; ``dst`` may be those columns of ``out`` (columns whose ``dst`` is another buffer need not be
-    left in ``out``).  Few bfloat16 rows: in the product's own epilogue, on sums that have not been rounded."""
+    left in ``out``).  Few bfloat16 rows: in the product's own epilogue, on sums that have not been rounded.
+    ``scale``: see ``linear``."""
     M, K = x.shape
     N = w.shape[0]
-    lds = N >= ROWS_LDS_WIDE_COLUMNS and out.stride(0) % 4 == 0 and _rows_ok(x, w, w_tiled, M, N, K)      # wide enough that the activations' own kernels cost less
+    lds = scale is None and N >= ROWS_LDS_WIDE_COLUMNS and out.stride(0) % 4 == 0 and _rows_ok(x, w, w_tiled, M, N, K)      # wide enough that the activations' own kernels cost less
     if 0 < len(acts) <= 2 and not lds and _skinny_ok(x, w, M, K) and _tiled_ok(w, w_tiled) and N % 16 == 0 and K % 32 == 0 \
             and out.dtype == torch.bfloat16 and all(c0 % 16 == 0 and n % 16 == 0 and dst.dtype == torch.bfloat16 for c0, n, _, dst in acts):
         _dev(x, w, out, *(dst for _, _, _, dst in acts))
@@ -1040,9 +1041,9 @@ def linear_activated(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, w_tile
         _check(_lib().ri_gemm_skinny_activated(
             _ptr(x), x.stride(0), _ptr(w_tiled), _ptr(out), out.stride(0), M, N, K, len(acts), ints([a[0] for a in acts]),
             ints([a[0] + a[1] for a in acts]), ints([UNARY[a[2]] for a in acts]), (ctypes.c_void_p * len(acts))(*[a[3].data_ptr() for a in acts]),
-            ints([a[3].stride(0) for a in acts]), _stream()))
+            ints([a[3].stride(0) for a in acts]), *_scale_args(scale, M, "linear_activated"), _stream()))
         return
-    linear(x, w, out, w_tiled, workspace=workspace)
+    linear(x, w, out, w_tiled, scale=scale, workspace=workspace)
     for c0, n, name, dst in acts:
         unary(name, out[:, c0:c0 + n], dst)
 

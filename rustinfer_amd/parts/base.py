@@ -477,7 +477,9 @@ class ProjectionSet:
 
     def project(self, ctx, normed, members=None):
         """(projected rows [T, n_in], the buffer [T, n_act] the parts' ``core`` fill), the parts' ``in_activations`` applied
-        (``members``: of the first so many parts alone, where the others' ``core`` does not run)."""
+        (``members``: of the first so many parts alone, where the others' ``core`` does not run).  ``normed``: rows, or a ``DeferredNorm``."""
+        normed, scale = split_normed(normed)
+        kw = {} if scale is None else {"scale": scale}
         T = normed.shape[0]
         proj = ctx.workspace.get("projset.in", T, self.n_in, self.rt.dtype)
         act = ctx.workspace.get("projset.act", T, self.n_act, self.rt.dtype)
@@ -487,9 +489,9 @@ class ProjectionSet:
                 c0, rows = self.in_slices[i][name]
                 acts.append((c0, rows, f, self.act_view(i, act) if into_act else proj[:, c0:c0 + rows]))
         if acts:
-            self.rt.ops.linear_activated(normed, self.w_in.weight, proj, self.w_in.weight_tiled, acts, workspace=ctx.workspace)
+            self.rt.ops.linear_activated(normed, self.w_in.weight, proj, self.w_in.weight_tiled, acts, workspace=ctx.workspace, **kw)
         else:
-            self.w_in.forward(normed, proj, workspace=ctx.workspace)
+            self.w_in.forward(normed, proj, workspace=ctx.workspace, **kw)
         for a, b in self._gaps:                          # scratch may hold anything, and 0 * NaN is NaN
             act[:, a:b].zero_()
         return proj, act
@@ -509,3 +511,15 @@ class ProjectionSet:
         32-bit partial sums that the next norm adds up."""
         return self.rt.ops.linear_delta(act, self.w_out.weight, ctx.workspace, "projset.out",
                                         self.w_out.weight_tiled, out_dtype=torch.float32)
+
+    def output_into(self, ctx, act, x, next_norm):
+        """Few rows: the parts' summed outputs added to ``x`` by their product, and the input behind ``next_norm`` as a
+        ``DeferredNorm``.  None, and nothing done, where that form does not apply."""
+        ops, w = self.rt.ops, self.w_out
+        ok = getattr(ops, "linear_residual_ok", None)
+        # (up to eight rows: with more, the plain products' other forms are the faster ones, and read normed rows)
+        if ok is None or self.rt.dtype != torch.bfloat16 or x.shape[0] > 8 or not ok(x.shape[0], w.weight, w.weight_tiled, next_norm.weight) \
+                or self.w_in.weight_tiled is None or not ops.linear_residual_pays(x.shape[0], w.weight):
+            return None
+        a, ssq = ops.linear_residual(act, w.weight, w.weight_tiled, x, next_norm.weight, ctx.workspace, "deferred")
+        return DeferredNorm(a, ssq, next_norm.eps)

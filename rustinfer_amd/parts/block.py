@@ -216,9 +216,11 @@ class ParallelBlock(Part):
 
     Both sub-layers are ``ProjectedPart``: their input projections are one product of ``n``, their
     output projections one product over the concatenated activations, whose result is the block's
-    one delta (left pending for the next norm, as in ``PreNormBlock``)."""
+    one delta (left pending for the next norm, as in ``PreNormBlock``; of few rows added to the stream by that
+    product, which prepares the input of what follows)."""
 
-    takes_follow = False
+    takes_follow = True          # forward() accepts ``follow``
+    takes_deferred_norm = True   # the block's input may be a ``DeferredNorm``
 
     def __init__(self, hidden_size: int, norm: Norm, mixer=None, ffn=None, names: Optional[Dict[str, str]] = None):
         if mixer is None and ffn is None:
@@ -252,9 +254,9 @@ class ParallelBlock(Part):
         return False
 
     def entry(self):
-        return (self.norm, None)
+        return (self.norm, self)
 
-    def _run(self, ctx, hidden: Hidden, cache, mixer_only: bool):
+    def _run(self, ctx, hidden: Hidden, cache, mixer_only: bool, follow=None):
         normed = ctx.workspace.get("block.normed", hidden.x.shape[0], self.hidden_size, self.rt.dtype)
         inp = hidden.input_behind(ctx, self.norm, normed)
         proj, act = self.set.project(ctx, inp, members=int(self.mixer is not None) if mixer_only else None)
@@ -266,10 +268,15 @@ class ParallelBlock(Part):
             return None
         if self.ffn is not None:
             self.ffn.core(ctx, self.set.views(i, proj), self.set.act_view(i, act), None)
-        return self.set.output(ctx, act)
+        if follow is not None and getattr(follow[0], "plain_rms", False) and getattr(follow[1], "takes_deferred_norm", False):
+            prepared = self.set.output_into(ctx, act, hidden.x, follow[0])
+            if prepared is not None:
+                return None, (follow[0], prepared)
+        return self.set.output(ctx, act), None
 
     def forward(self, ctx, hidden: Hidden, cache, out_rows=None, follow=None) -> None:
-        hidden.pending, hidden.deferred = self._run(ctx, hidden, cache, False), None
+        """``follow``: as in ``PreNormBlock``."""
+        hidden.pending, hidden.deferred = self._run(ctx, hidden, cache, False, follow)
 
     def update_cache_only(self, ctx, hidden: Hidden, cache) -> None:
         """The last block of a step whose logits nobody wants: the mixer alone runs, for what it

@@ -2178,3 +2178,23 @@ def test_qkv_f32_of_few_rows_with_rotation_and_pages(ops, M, H, Hkv, hd, K):
         for a, b in ((got[0][live, :H * hd], want[0][live, :H * hd]), (got[1], want[1]), (got[2], want[2])):
             assert (a - b).abs().max() <= 2.0 ** -20 * size
     assert not ops.qkv_rope_f32(rnd(9, K, seed=1), w, rnd(9, (H + 2 * Hkv) * hd, seed=1), H, Hkv, hd, rotary, positions, row_of_token, got[1], got[2], table, page)
+
+
+@pytest.mark.parametrize("M,N,K,acts", [(1, 64, 32, [(0, 64, "relu2")]), (8, 2064, 2048, [(16, 2048, "relu2"), (0, 16, "tanh")]), (5, 12304, 512, [(0, 8192, "relu2")]), (3, 80, 32, [(8, 24, "tanh")])])
+def test_activated_columns_behind_a_deferred_norm(ops, M, N, K, acts):
+    """The norm's factor comes before the activation, in the epilogue and behind the product (columns that begin inside a tile)."""
+    x = rnd(M, K, seed=M).to(torch.bfloat16)
+    w = (rnd(N, K, seed=N) * 0.2).to(torch.bfloat16)
+    ssq = (x.double().square().view(M, 4, -1).sum(2) * 3).float().contiguous()
+    out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+    bufs = [torch.empty(M, n, dtype=torch.bfloat16, device=DEV) for _, n, _ in acts]
+    ops.linear_activated(x, w, out, ops.tile_weight(w), [(c0, n, f, b) for (c0, n, f), b in zip(acts, bufs)], scale=(ssq, 1e-5))
+    ref = (x.double() @ w.double().t()) * torch.rsqrt(ssq.double().sum(1, keepdim=True) / K + 1e-5)
+    plain = torch.ones(N, dtype=torch.bool)
+    for (c0, n, f), b in zip(acts, bufs):
+        z = ref[:, c0:c0 + n]
+        want = torch.relu(z).square() if f == "relu2" else torch.tanh(z)
+        # bfloat16 rounds to 2^-8: the result, and behind the product the sum too, which the square doubles; 2^-6 covers the three
+        assert torch.all((b.double() - want).abs() <= 2.0 ** -6 * want.abs() + 2.0 ** -8 * z.abs().clamp(max=1.0) * (f == "tanh") + 1e-4)
+        plain[c0:c0 + n] = False
+    assert torch.all((out[:, plain].double() - ref[:, plain]).abs() <= 2.0 ** -7 * ref[:, plain].abs() + 1e-4)
