@@ -502,12 +502,13 @@ static int few_form(int M, int N, int K, float* cost) {
     return one == *cost ? 0 : two < three ? 2 : 3;
 }
 
-// Whether up to four rows go to the kernel of FMAs, gemm_rows_f32: it reads a kilobyte of a row of W at a time, the tiles 64 bytes
-// of each of 16 places, which costs more the longer the rows are.  But where rows begin a power of two apart its long reads meet on the same
-// channels of memory, and there it pays only against rounds of blocks that are far from full.  Measured, us, 1 and 4 rows, gemm_rows_f32 / the best form of
-// the tiles: 5120 x 3072 16.6 18.6 / 17.4 19.3, 5120 x 5120 23.7 27.1 / 28.5 30.5, 27648 x 5120 97 107 / 120 130, 12288 x 6912 60 68 / 68 71,
-// 128256 x 1536 129 141 / 146 155, 2560 x 11008 35 40 / 37 40, 7000 x 4096 25.1 26.6 / 25.9 27.4; not taken: 12288 x 1536 18.4 21.8 / 17.7
-// 18.9, 28672 x 4096 95 98 / 81 87, 16384 x 2048 34 37 / 28 29, 4096 x 3072 14.9 16.3 / 12.8 14.4, 2048 x 8192 21 24 / 16 17.
+// Whether up to four rows go to the kernel of FMAs, gemm_rows_f32: it reads a kilobyte of a row of W at a time, the tiles 128 bytes
+// of each of eight rows, which costs more the longer the rows are.  But where rows begin a power of two apart its long reads meet on the same
+// channels of memory, and there it pays only against rounds of blocks that are far from full.  Measured, us, 1 and 4 rows, gemm_rows_f32 / the form of
+// the tiles: 5120 x 3072 16.3 18.3 / 17.1 17.8, 5120 x 5120 23.2 26.6 / 25.6 26.4, 27648 x 5120 98 107 / 96 110, 128256 x 3072 242 259 / 251 270,
+// 7000 x 4096 24.6 25.9 / 25.2 26.9, 128256 x 2048 176 183 / 175 179.  The line lies where it did when the tiles read 64 bytes of 16 places (27648 x 5120 120 130, 128256 x 1536 146 155): it
+// takes in some that the tiles would now do faster, 12288 x 6912 61 68 / 59 60, 128256 x 1536 130 145 / 127 135, 2560 x 11008 34 39 / 32 37, 4096 x 14336 47 53 / 40 45.
+// Not taken, as measured then: 12288 x 1536 18.4 21.8 / 17.7 18.9, 28672 x 4096 95 98 / 81 87, 16384 x 2048 34 37 / 28 29, 4096 x 3072 14.9 16.3 / 12.8 14.4, 2048 x 8192 21 24 / 16 17.
 static bool gemm_f32_rows_pay(int M, int N, int K, int ldw) {
     if (M > 4) return false;
     if ((ldw & (ldw - 1)) == 0) {
@@ -530,8 +531,9 @@ extern "C" int ri_gemm_f32_form(int M, int N, int K, int ldw) {
 
 // Whether up to eight rows' gate and up product takes ri_gemm_f32_swiglu rather than ri_gemm_f32 and the activation's kernel: not where gemm_rows_f32
 // has that product to itself, but for rows of up to 3,072 values whose rounds of blocks are full.  Measured, us, 1 and 4 rows, two kernels / this:
-// 8192 x 3072 46.7 50.3 / 43.8 45.9, 9728 x 2560 40.4 44.2 / 42.4 45.4, 6912 x 2560 29.6 34.6 / 36.1 38.4, 13824 x 5120 98 109 / 128 137, 18944 x 3584
-// 92 98 / 107 115, 14336 x 4096 83 90 / 82 85, 8192 x 2048 29.7 30.9 / 29.0 29.8.
+// 8192 x 3072 48 51 / 39 40, 9728 x 2560 41 44 / 37 38, 6912 x 2560 29.7 34.8 / 30.8 31.6, 13824 x 5120 100 109 / 97 102, 18944 x 3584 93 98 / 91 95,
+// 14336 x 4096 80 87 / 76 78, 8192 x 2048 29.4 29.4 / 30.5 30.7.  The line lies where it did with 64 bytes a load (6912 x 2560 36 38, 13824 x 5120 128 137): it leaves out
+// what would now pay by 1 to 14 %.  (Behind a deferred norm the product is always this one.)
 extern "C" int ri_gemm_f32_swiglu_pays(int M, int I, int K, int ldw) {
     if (M > 8) return 0;
     const bool full = (float)((I + 2047) / 2048) * 2048.f <= 1.03f * (float)I;
