@@ -19,7 +19,8 @@
 // done (where a row's keys are divided, the block that leaves the last part merges them).  What a phase leaves for the next goes through memory:
 // stores of agent scope (written through the XCD's L2), acknowledged, then one of eight counters; readers poll the counters and read with plain
 // loads, which is sound because every buffer is written once a launch and nobody reads a line of it before it is complete (an L2 of another XCD
-// cannot hold an older copy: a launch begins with its L2 clean).  No fence is needed, which would cost tens of microseconds.  The counters lie in
+// cannot hold an older copy: a launch begins with its L2 clean).  What is read before a phase has ended, the parts of a divided row, lies in lines that
+// no other pair of row and key/value head has anything in.  No fence is needed, which would cost tens of microseconds.  The counters lie in
 // uncached memory and are polled by scalar loads, which do not stand behind the weights (of cached memory, by vector loads: 650 us).
 //
 // Which blocks take part is settled at the start: all of the grid, if all are on the chip (the usual case), else those that had arrived
@@ -74,7 +75,14 @@ struct Kind { int items, units, stride; unsigned tile, second; int whole; };
 // offsets within a layer's stretch of scratch, multiples of 256 bytes
 struct Offsets { size_t a, ssq, q, at, a2, ssq2, h, po, pml, all; };
 __host__ __device__ inline size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
-__host__ __device__ inline Offsets stack_offsets(int M, int d, int ff, int H, int hd, int slots) {
+// The parts of a row's keys for the G queries of a key/value head, a pair: a query's outputs of a part (hd floats) in `po`, its maximum and sum in `pml`.
+// A pair is merged when its own parts are there, while others still write theirs: its stretch of either is whole lines of its own (128 bytes; 256 here), or
+// the merge would bring a line into its L2 in which another pair's entries are not yet what a merge on the same XCD then reads.
+constexpr size_t LINE = 128;
+__host__ __device__ inline size_t pair_outputs(int G, int slots, int hd) { return (size_t)G * slots * hd * 4; }          // bytes; hd is 64 or 128
+__host__ __device__ inline size_t pair_sums(int G, int slots) { return up256((size_t)G * slots * 8); }
+static_assert(64 * 4 % LINE == 0 && 256 % LINE == 0, "a pair's stretches are whole lines");
+__host__ __device__ inline Offsets stack_offsets(int M, int d, int ff, int H, int Hkv, int hd, int slots) {
     Offsets o;
     size_t at = 0;
     auto take = [&](size_t n) { const size_t r = at; at += up256(n); return r; };
@@ -82,7 +90,7 @@ __host__ __device__ inline Offsets stack_offsets(int M, int d, int ff, int H, in
     o.q = take((size_t)M * H * hd * 2); o.at = take((size_t)M * H * hd * 2);
     o.a2 = take((size_t)M * d * 2); o.ssq2 = take((size_t)M * (d / 8) * 4);
     o.h = take((size_t)M * ff * 2);
-    o.po = take((size_t)M * H * slots * hd * 4); o.pml = take((size_t)M * H * slots * 8);
+    o.po = take(M * Hkv * pair_outputs(H / Hkv, slots, hd)); o.pml = take(M * Hkv * pair_sums(H / Hkv, slots));
     o.all = at;
     return o;
 }
@@ -496,11 +504,11 @@ __device__ __forceinline__ float sum_of_eight(float v) {
 
 // The parts of a row's keys for the G queries of a key/value head, by one wave: eight values a lane.
 template <int HD>
-__device__ __forceinline__ void merge(const float* po, const float* pml, size_t first, int slots, int parts, int G, bf16_t* out, int lane) {
+__device__ __forceinline__ void merge(const char* po, const char* pml, int pair, int slots, int parts, int G, bf16_t* out, int lane) {
     const int e = lane * 8, qi = e / HD;
     if (e >= G * HD) return;
-    const float* ml = pml + (first + (size_t)qi * slots) * 2;
-    const float* o = po + (first + (size_t)qi * slots) * HD + e % HD;
+    const float* ml = reinterpret_cast<const float*>(pml + pair * pair_sums(G, slots)) + (size_t)qi * slots * 2;
+    const float* o = reinterpret_cast<const float*>(po + pair * pair_outputs(G, slots, HD)) + (size_t)qi * slots * HD + e % HD;
     float top = -INFINITY, sum = 0.f, v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll 8
     for (int p = 0; p < parts; ++p) top = fmaxf(top, ml[p * 2]);
@@ -614,8 +622,8 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                 const Args P = again(A);
                 char* base = P->scratch + (size_t)l * P->layer_bytes;
                 bf16_t* attn = reinterpret_cast<bf16_t*>(base + P->off.at);
-                float* po = reinterpret_cast<float*>(base + P->off.po);
-                float* pml = reinterpret_cast<float*>(base + P->off.pml);
+                char* po = base + P->off.po;
+                char* pml = base + P->off.pml;
                 if (kind == ATTEND) {
                     // attention of this block's first job: what does not depend on this step is asked for now
                     const int lane = hidden_lane((int)threadIdx.x) & 63;
@@ -673,10 +681,10 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                                 st_agent(reinterpret_cast<unsigned*>(attn + (size_t)m * q_dim + (size_t)g * G * HD + e),
                                          (unsigned)f32_to_bf16(v0) | ((unsigned)f32_to_bf16(v1) << 16));
                             } else {
-                                const size_t slot = ((size_t)m * H + g * G + qi) * P->slots + part;
-                                st_agent(reinterpret_cast<unsigned long long*>(po + slot * HD + dd),
+                                const int slots = P->slots, pair = m * Hkv + g, slot = qi * slots + part;
+                                st_agent(reinterpret_cast<unsigned long long*>(po + pair * pair_outputs(G, slots, HD) + ((size_t)slot * HD + dd) * 4),
                                          (unsigned long long)__float_as_uint(v0) | ((unsigned long long)__float_as_uint(v1) << 32));
-                                if (dd == 0) st_agent(reinterpret_cast<unsigned long long*>(pml + slot * 2),
+                                if (dd == 0) st_agent(reinterpret_cast<unsigned long long*>(pml + pair * pair_sums(G, slots) + (size_t)slot * 8),
                                                       (unsigned long long)__float_as_uint(top) | ((unsigned long long)__float_as_uint(sum) << 32));
                             }
                         }
@@ -768,8 +776,7 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                         if (lane == 0) before = add_agent(ctl + C_PAIRS * 32 + pair * PAIR_WORDS, 1u);
                         if (__builtin_amdgcn_readfirstlane((int)before) != (l + 1) * parts - 1) continue;
                         asm volatile("" ::: "memory");
-                        merge<HD>(reinterpret_cast<const float*>(base + P->off.po), reinterpret_cast<const float*>(base + P->off.pml),
-                                  (size_t)(row * H + (pair - row * Hkv) * G) * P->slots, P->slots, parts, G,
+                        merge<HD>(base + P->off.po, base + P->off.pml, pair, P->slots, parts, G,
                                   reinterpret_cast<bf16_t*>(base + P->off.at) + (size_t)row * q_dim + (size_t)(pair - row * Hkv) * G * HD, lane);
                     }
                 }
@@ -962,13 +969,22 @@ extern "C" int ri_decode_stack_takes(int M, int d, int ff, int H, int Hkv, int h
         && H / Hkv <= 16 && H / Hkv * hd <= ATT_VALUES && d >= 512 && d % 512 == 0 && d <= 8192 && H * hd % 512 == 0 && H * hd <= 8192
         && ff >= 512 && ff % 512 == 0 && ff <= 14336 && V % 16 == 0 && V > 0;
 }
+// Where the parts of the keys of row m and key/value head g lie in a layer's stretch, with room for `slots` of them: from[0], to[0] their outputs, from[1], to[1]
+// their maxima and sums, in bytes; *line: what two pairs may not share.
+extern "C" void ri_decode_stack_pair(int M, int d, int ff, int H, int Hkv, int hd, int slots, int m, int g, size_t* from, size_t* to, size_t* line) {
+    const Offsets o = stack_offsets(M, d, ff, H, Hkv, hd, slots);
+    const int pair = m * Hkv + g, G = H / Hkv;
+    from[0] = o.po + pair * pair_outputs(G, slots, hd); to[0] = from[0] + (size_t)G * slots * hd * 4;
+    from[1] = o.pml + pair * pair_sums(G, slots); to[1] = from[1] + (size_t)G * slots * 8;
+    *line = LINE;
+}
 // Entries of the model's table.
 extern "C" int ri_decode_stack_table(int L) { return 4 * L + 1 + 2 * (2 * L + 1); }
 // Bytes of scratch for the stretches of L layers and the one behind them, and the residual stream.
 extern "C" size_t ri_decode_stack_scratch(int L, int M, int d, int ff, int H, int Hkv, int hd) {
     const int blocks = stack_blocks();
     if (blocks < 8 || M < 1 || Hkv < 1) return 0;
-    return (size_t)(L + 1) * stack_offsets(M, d, ff, H, hd, stack_slots(M, Hkv, blocks)).all + up256((size_t)d * MAX_ROWS * 4);
+    return (size_t)(L + 1) * stack_offsets(M, d, ff, H, Hkv, hd, stack_slots(M, Hkv, blocks)).all + up256((size_t)d * MAX_ROWS * 4);
 }
 
 // model: the table of L layers on the device (ri_decode_stack_table entries, see above), the weights in tile order (q/k/v with rows in
@@ -998,7 +1014,7 @@ extern "C" int ri_decode_stack(const void* model, int L, int M, int d, int ff, i
     A.cos_t = cos_t; A.sin_t = sin_t; A.kc = (bf16_t*)kc; A.vc = (bf16_t*)vc; A.k_layer = k_layer; A.v_layer = v_layer; A.scale = scale;
     A.logits = logits; A.ld_logits = ld_logits;
     A.slots = stack_slots(M, Hkv, all);
-    A.off = stack_offsets(M, d, ff, H, hd, A.slots);
+    A.off = stack_offsets(M, d, ff, H, Hkv, hd, A.slots);
     A.layer_bytes = A.off.all;
     A.scratch = (char*)scratch;
     A.x = (float*)(A.scratch + (size_t)(L + 1) * A.layer_bytes);

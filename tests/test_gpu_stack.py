@@ -28,7 +28,9 @@ CONFIGS = {
     "64": _cfg(512, 512, 8, 2, 64, L=3), "64 uneven": _cfg(2560, 4608, 40, 8, 64, tied=False), "64 wide": _cfg(512, 1024, 72, 9, 64),
     "64 one head": _cfg(512, 1536, 8, 1, 64, V=528), "128": _cfg(1024, 1536, 16, 4, 128, tied=False), "128 long": _cfg(512, 8704, 8, 2, 128),
     "128 wide": _cfg(1024, 1024, 36, 9, 128), "128 longest": _cfg(512, 14336, 8, 2, 128),
+    "128 three": _cfg(512, 1024, 24, 8, 128),
 }
+PAGES = {"128 three": 704}
 LONG = [5 + LAST, 40, 100, 513, LAST, 32, 1200, 64]
 CASES = [("64", [5 + LAST], "eager", 0), ("64", LONG, "eager", 0), ("64", LONG[4:7], "graph", 0), ("64", LONG, "graph", 0),
          ("64 uneven", LONG[2:7], "graph", 0), ("64 uneven", LONG[:6], "eager", 8), ("64 wide", LONG[3:6], "eager", 0),
@@ -48,7 +50,8 @@ def engines(tmp_path_factory):
             from rustinfer_amd.weights import write_random_model
             d = str(tmp_path_factory.mktemp("stack"))
             write_random_model(LlamaConfig.from_dict(CONFIGS[name]), 7 + len(made), d)
-            eng = build_engine(d, dtype="bfloat16", page_size=16, num_pages=256, max_requests=8, max_model_len=2048, max_batch_tokens=2048)
+            eng = build_engine(d, dtype="bfloat16", page_size=16, num_pages=PAGES.get(name, 256), max_requests=8, max_model_len=2048,
+                               max_batch_tokens=2048)
             made[name] = (eng, plain_llama.read_model(d))
         return made[name]
     return get
@@ -105,6 +108,36 @@ def test_steps_in_one_launch(engines, monkeypatch, name, lengths, mode, grid):
     print(f"{name} {mode} {lengths}: {rms.max() / s:.2%}, part by part {rms_parts.max() / s:.2%}")
     assert np.isfinite(got).all() and rms.max() <= 0.02 * s, rms / s
     assert rms.mean() <= 1.1 * rms_parts.mean() + 1e-4 * s, (rms.mean() / s, rms_parts.mean() / s)
+
+
+DIVIDED = [1203, 611, 1999, 640, 1024, 870, 1611, 770]
+
+
+@pytest.fixture(scope="module")
+def divided(engines):
+    _, (cfg, w) = engines("128 three")
+    reqs = random_requests(cfg["vocab_size"], DIVIDED, seed=11)
+    return reqs, np.stack([plain_llama.forward(cfg, w, t)[-LAST:] for t in reqs.values()], 1)
+
+
+@pytest.mark.parametrize("rows", range(3, 9))
+def test_divided_rows_are_the_same_every_time(engines, divided, monkeypatch, rows):
+    """Three query heads a key/value head, keys divided between blocks: what a merge reads is this step's, whatever the scratch held before it (other
+    rows' parts, of another number of rows), so a step gives the same bits again; and the error is that of undivided rows."""
+    from rustinfer_amd.kernels import ops
+    eng, (cfg, _) = engines("128 three")
+    reqs, want = dict(list(divided[0].items())[:rows]), divided[1][:, :rows]
+    first = _decode(eng, reqs, "eager")
+    for other in (rows - 1, rows):
+        _decode(eng, random_requests(cfg["vocab_size"], [1300 - 37 * i for i in range(other)], seed=20 + other), "eager")
+        assert np.array_equal(_decode(eng, reqs, "eager"), first)
+    monkeypatch.setattr(ops, "DECODE_STACK_GRID", 32)       # fewer than two blocks a pair: no row is divided
+    whole = _decode(eng, reqs, "eager")
+    s = want.std()
+    rms, rms_whole = (np.sqrt(np.mean((v - want) ** 2, axis=2)) for v in (first, whole))
+    print(f"{rows} divided rows: {rms.max() / s:.2%}, undivided {rms_whole.max() / s:.2%}")
+    assert np.isfinite(first).all() and rms.max() <= 0.02 * s, rms / s
+    assert rms.mean() <= 1.1 * rms_whole.mean() + 1e-4 * s, (rms.mean() / s, rms_whole.mean() / s)
 
 
 def test_control_blocks_are_given_back():

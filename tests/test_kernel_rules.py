@@ -127,3 +127,19 @@ def test_steps_that_go_in_one_launch(lib, change, takes):
     sizes.update(change)
     assert lib.ri_decode_stack_takes(*sizes.values()) == takes
     assert lib.ri_decode_stack_give_control(ctypes.c_void_p(4096)) != 0           # (never taken)
+
+
+@pytest.mark.parametrize("H,Hkv,hd", [(24, 8, 128), (32, 8, 64), (32, 8, 128), (40, 8, 64), (72, 9, 64), (8, 1, 64), (8, 8, 128), (36, 9, 128)])
+def test_divided_rows_share_no_line_in_the_one_launch_step(lib, H, Hkv, hd):
+    """A pair of row and key/value head is merged while others still write their parts, and its line may then stay in an L2: the parts of no two pairs have a
+    line in common, nor do outputs and sums."""
+    from_, to, line = (ctypes.c_size_t * 2)(), (ctypes.c_size_t * 2)(), ctypes.c_size_t(0)
+    for M in range(1, 9):
+        for slots in {max(1, min(64, 256 // (M * Hkv))), 1, 3, 7, 64}:
+            owner = {}
+            for pair in range(M * Hkv):
+                lib.ri_decode_stack_pair(M, 512, 512, H, Hkv, hd, slots, pair // Hkv, pair % Hkv, from_, to, ctypes.byref(line))
+                assert line.value >= 128 and to[0] - from_[0] == H // Hkv * slots * hd * 4 and to[1] - from_[1] == H // Hkv * slots * 8
+                for kind in range(2):
+                    for n in range(from_[kind] // line.value, (to[kind] - 1) // line.value + 1):
+                        assert owner.setdefault(n, (pair, kind)) == (pair, kind), (M, slots, pair, kind)
