@@ -26,7 +26,8 @@
 // Which blocks take part is settled at the start: all of the grid, if all are on the chip (the usual case), else those that had arrived
 // when the first of them had waited `close_ticks`; later ones leave at once.  Items are dealt round to those that take part, so every
 // block that is waited for is running, whatever else runs on the device, and the products do not depend on their number.  Every wait is bounded
-// all the same (`limit_ticks`, MOST_SPINS): then the launch ends and its logits are NaN.
+// all the same (the one at the start by `join_ticks`, as one block cannot go on alone; `limit_ticks`, MOST_SPINS): then the launch ends, its logits are NaN, and a word
+// in host memory says so.
 //
 // Products: weights in tile order ([N/16][K/32][64 lanes][8], gemm.hip); K is divided between the eight readers.  Activations (eight rows) are held
 // in registers for a phase, two steps of K an operand: columns 0 to 7 of the matrix instruction are the rows at the even step, 8 to 15 at the odd
@@ -108,7 +109,8 @@ struct StackArgs {
     float* x;                                           // [d / 8][8][8] the residual stream, by items
     int slots;                                          // parts of a row's keys there is room for
     unsigned* control; int expect;                      // blocks that may take part: a multiple of 8
-    unsigned long long close_ticks, limit_ticks;
+    unsigned* gave_up;                                  // host memory: set by a launch that did not run to its end
+    unsigned long long close_ticks, join_ticks, limit_ticks;
     Offsets off;
     Kind kinds[5];
 };
@@ -478,6 +480,7 @@ struct Attention {
 
 // The control wave's wait for everything up to `target` arrivals.
 __device__ __forceinline__ bool all_done(Args A, unsigned target, int lane, unsigned long long begun) {
+    if (A->limit_ticks == 0) return false;               // (no waiting at all)
     for (unsigned spin = 1;; ++spin) {
         unsigned c0, c1, c2, c3, c4, c5, c6, c7;
         asm volatile("s_load_dword %0, %8, 0x0 glc\n\ts_load_dword %1, %8, 0x80 glc\n\ts_load_dword %2, %8, 0x100 glc\n\ts_load_dword %3, %8, 0x180 glc\n\t"
@@ -542,7 +545,8 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
     volatile int* misc = reinterpret_cast<volatile int*>(lds + L_MISC);
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int shard = blockIdx.x & 7;
-    const unsigned long long begun = wall_clock64();
+    unsigned long long begun = wall_clock64();
+    bool given_up = false;                                // of the control wave
     unsigned* ctl = again(A)->control;
     if (wave == CONTROL) {
         misc[lane] = 0;
@@ -571,8 +575,10 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                     rank = __builtin_amdgcn_readfirstlane(rank);
                     break;
                 }
-                // (two blocks are the least that can go on: until then others hold the chip, and their work ends)
-                if (!tried && __builtin_amdgcn_readfirstlane(wall_clock64() - begun > again(A)->close_ticks ? 1 : 0)) {
+                // (two blocks are the least that can go on: until then others hold the chip)
+                const unsigned long long waited = wall_clock64() - begun;
+                if (__builtin_amdgcn_readfirstlane(waited > again(A)->join_ticks ? 1 : 0)) { given_up = true; break; }
+                if (!tried && __builtin_amdgcn_readfirstlane(waited > again(A)->close_ticks ? 1 : 0)) {
                     unsigned here = 0;
                     if (lane < 8) here = ld_agent(ctl + (C_ARRIVED + lane) * 32) & ~CLOSED;
                     here = (unsigned)__builtin_popcountll(__ballot(here > 0)) + (__ballot(here > 1) ? 1u : 0u);
@@ -598,6 +604,7 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
         }
         if (rank >= n) n = 0;                             // (an odd one out: items of half a tile keep their half from one to the next)
         if (lane == 0) { misc[W_RANK] = rank; misc[W_N] = n; }
+        begun = wall_clock64();
     }
     __syncthreads();
     const int rank = __builtin_amdgcn_readfirstlane(misc[W_RANK]), n = __builtin_amdgcn_readfirstlane(misc[W_N]);
@@ -716,7 +723,6 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
             const int blk = b >= 0 ? again(A)->blocks[(size_t)b * again(A)->max_blocks + pos / page] : -1, slot = pos % page;
             unsigned target = 0;
             int sums = 0, kind = EMBED, l = 0, begun_phases = 0;
-            bool given_up = false;
             float w0 = 0.f, w1 = 0.f, c0 = 1.f, s0 = 0.f, c1 = 1.f, s1 = 0.f;
             float* xs = reinterpret_cast<float*>(lds + L_X);
             int id = live ? again(A)->ids[m] : -1;
@@ -862,11 +868,12 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                 kind = kind == EMBED ? QKV : kind == QKV ? ATTEND : kind == ATTEND ? O : kind == O ? GATE_UP
                      : kind == GATE_UP ? DOWN : l == P->L ? HEAD : QKV;
             }
-            if (given_up) {
-                for (int r = 0; r < M; ++r)
-                    for (int i = lane; i < again(A)->V; i += 64) again(A)->logits[(size_t)r * again(A)->ld_logits + i] = NAN;
-            }
         }
+    }
+    if (given_up) {
+        if (lane == 0) __hip_atomic_store(again(A)->gave_up, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        for (int r = 0; r < again(A)->M; ++r)
+            for (int i = lane; i < again(A)->V; i += 64) again(A)->logits[(size_t)r * again(A)->ld_logits + i] = NAN;
     }
     // The last block to leave makes the control words zero again (all have read what they wanted of them).
     if (wave == CONTROL) {
@@ -916,16 +923,19 @@ int stack_slots(int M, int Hkv, int blocks) {
 // it), so a device has one stretch of MOST_BLOCKS, made when the first is taken.  A block belongs to whoever took it until it is given back.
 constexpr int MOST_BLOCKS = 64, BLOCK_BYTES = 16 * 1024;
 static_assert(CONTROL_WORDS * 4 <= BLOCK_BYTES, "a control block");
-struct ControlBlocks { char* base = nullptr; bool out[MOST_BLOCKS] = {}; };
+// With each goes a word of pinned host memory, likewise never freed, that a launch sets which gives up.
+struct ControlBlocks { char* base = nullptr; unsigned* words = nullptr; bool out[MOST_BLOCKS] = {}; };
+constexpr int WORD_STEP = 32;                            // a line each
 std::mutex control_mutex;
 ControlBlocks control_blocks[64];
 
 }  // namespace
 
-// A control block of zeros on the current device, or null in *block if all are taken.  Waits for the device: not under capture.
-extern "C" int ri_decode_stack_take_control(void** block) {
-    RI_REQUIRE(block, "ri_decode_stack_take_control: null pointer");
+// A control block of zeros on the current device and its word (0) on the host, or null in *block if all are taken.  Waits for the device: not under capture.
+extern "C" int ri_decode_stack_take_control(void** block, unsigned** gave_up) {
+    RI_REQUIRE(block && gave_up, "ri_decode_stack_take_control: null pointer");
     *block = nullptr;
+    *gave_up = nullptr;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
     RI_REQUIRE(e == hipSuccess && dev >= 0 && dev < 64, "ri_decode_stack_take_control: no current device: %s", hipGetErrorString(e));
@@ -937,6 +947,12 @@ extern "C" int ri_decode_stack_take_control(void** block) {
         RI_REQUIRE(e == hipSuccess, "ri_decode_stack_take_control: %d bytes of uncached memory refused: %s", MOST_BLOCKS * BLOCK_BYTES, hipGetErrorString(e));
         c.base = (char*)p;
     }
+    if (!c.words) {
+        void* p = nullptr;
+        e = hipHostMalloc(&p, (size_t)MOST_BLOCKS * WORD_STEP * 4, hipHostMallocPortable);
+        RI_REQUIRE(e == hipSuccess, "ri_decode_stack_take_control: %d bytes of pinned memory refused: %s", MOST_BLOCKS * WORD_STEP * 4, hipGetErrorString(e));
+        c.words = (unsigned*)p;
+    }
     for (int i = 0; i < MOST_BLOCKS; ++i) {
         if (c.out[i]) continue;
         // (a launch of the one who gave it back may still be under way)
@@ -945,6 +961,8 @@ extern "C" int ri_decode_stack_take_control(void** block) {
         if (e == hipSuccess) e = hipDeviceSynchronize();
         RI_REQUIRE(e == hipSuccess, "ri_decode_stack_take_control: %s", hipGetErrorString(e));
         c.out[i] = true;
+        c.words[i * WORD_STEP] = 0;
+        *gave_up = c.words + i * WORD_STEP;
         *block = c.base + (size_t)i * BLOCK_BYTES;
         return 0;
     }
@@ -990,16 +1008,18 @@ extern "C" size_t ri_decode_stack_scratch(int L, int M, int d, int ff, int H, in
 // model: the table of L layers on the device (ri_decode_stack_table entries, see above), the weights in tile order (q/k/v with rows in
 // ri_qkv_rope_row_order).  kc, vc: the first layer's caches, k_layer and v_layer values on to the next one's.
 // logits [M, ld_logits] 32-bit.  scratch: ri_decode_stack_scratch bytes, 256-byte aligned; control: a block of ri_decode_stack_take_control that no
-// launch that may overlap with this one has.  grid: blocks to launch (0: one a compute unit).
+// launch that may overlap with this one has, gave_up: its word (1 once a launch has not run to its end).  grid: blocks to launch (0: one a compute unit).
+// close_us: how long the first blocks wait for the rest; join_us: and at most, where they cannot go on without; limit_us: how long for each other's results.
 extern "C" int ri_decode_stack(const void* model, int L, int M, int d, int ff, int H, int Hkv, int hd, int V, int norm_dtype,
                                const int* ids, const int* device_tokens, const void* table, const int* positions, const int* row_of_token,
                                const int* kv_lens, const int* blocks, int max_blocks, const float* cos_t, const float* sin_t, void* kc, void* vc,
                                size_t k_layer, size_t v_layer, int page, float scale, float* logits, int ld_logits, void* scratch, size_t scratch_bytes,
-                               unsigned* control, int grid, double close_us, double limit_us, hipStream_t stream) {
+                               unsigned* control, unsigned* gave_up, int grid, double close_us, double join_us, double limit_us, hipStream_t stream) {
     RI_REQUIRE(ri_decode_stack_takes(M, d, ff, H, Hkv, hd, page, V) && L >= 1, "ri_decode_stack: M=%d d=%d ff=%d H=%d Hkv=%d hd=%d page=%d V=%d L=%d is not taken",
                M, d, ff, H, Hkv, hd, page, V, L);
     RI_REQUIRE(model && ids && table && positions && row_of_token && kv_lens && blocks && cos_t && sin_t && kc && vc && logits
-               && scratch && control, "ri_decode_stack: null pointer");
+               && scratch && control && gave_up, "ri_decode_stack: null pointer");
+    RI_REQUIRE(close_us >= 0 && join_us >= 0 && limit_us >= 0 && close_us <= 1e9 && join_us <= 1e9 && limit_us <= 1e9, "ri_decode_stack: bad times");
     RI_REQUIRE(ld_logits >= V && max_blocks >= 1 && (norm_dtype == RI_F32 || norm_dtype == RI_BF16), "ri_decode_stack: bad sizes or norm dtype");
     RI_REQUIRE(((uintptr_t)kc | (uintptr_t)vc) % 16 == 0 && k_layer % 8 == 0 && v_layer % 8 == 0 && (uintptr_t)scratch % 256 == 0
                && (uintptr_t)control % 128 == 0, "ri_decode_stack: unaligned pointer");
@@ -1019,7 +1039,8 @@ extern "C" int ri_decode_stack(const void* model, int L, int M, int d, int ff, i
     A.scratch = (char*)scratch;
     A.x = (float*)(A.scratch + (size_t)(L + 1) * A.layer_bytes);
     A.control = control; A.expect = all;
-    A.close_ticks = (unsigned long long)(close_us * 100.0); A.limit_ticks = (unsigned long long)(limit_us * 100.0);
+    A.gave_up = gave_up;
+    A.close_ticks = (unsigned long long)(close_us * 100.0); A.join_ticks = (unsigned long long)(join_us * 100.0); A.limit_ticks = (unsigned long long)(limit_us * 100.0);
     if (grid == 0) grid = all;
     for (int kind = 0; kind < 5; ++kind) {
         const bool whole = kind == QKV || kind == HEAD, pair = kind == O || kind == DOWN;

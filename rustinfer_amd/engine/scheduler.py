@@ -142,6 +142,18 @@ class Scheduler:
                     self.waiting.remove(req)
                 self._finish(req, "cancelled")
 
+    def fail_running(self) -> None:
+        """End every request that has started, as ``"error"``: what the cache holds of them is lost, and tokens that have not reached the host
+        do not come any more."""
+        for req in list(self.running):
+            self._finish(req, "error")
+        for req in self.finished + list(self.waiting):           # (ended by their length, or preempted, in the meantime)
+            if req.output and req.output[-1] == PENDING:
+                while req.output and req.output[-1] == PENDING:
+                    req.output.pop()
+                if req.state == FINISHED:
+                    req.finish_reason = "error"
+
     # -- one step's decisions ----------------------------------------------------
     def _preempt(self, req: Request) -> None:
         self.cache.release(req.request_id)

@@ -30,6 +30,11 @@ class StepError(ValueError):
     """A batch the step function cannot run (crates/infer-worker/src/application/runtime/plan.rs:24-124)."""
 
 
+class StepLost(StepError):
+    """A step that had begun on the device did not run to its end.  What the cache holds of the requests that are live then is not whole: they are
+    to be released and run again, and are refused until they are."""
+
+
 @dataclass
 class StepEntry:
     request_id: Hashable
@@ -116,6 +121,7 @@ class Engine:
         self.vocab_size = model.vocab_size
         self.steps_run = 0
         # tokens sampled on the device that the next step may read without the host seeing them first
+        self._lost: set = set()                      # requests whose cache is not whole (StepLost)
         self.device_tokens = torch.zeros(max(self.max_requests, 1), dtype=torch.int32, device=rt.device)
         pin = rt.device.type == "cuda"
         self._tok_host = [torch.zeros(max(self.max_requests, 1), dtype=torch.int32, pin_memory=pin) for _ in range(4)]
@@ -378,8 +384,18 @@ class Engine:
 
     # -- tokens that stay on the device ---------------------------------------------
     def synchronize(self) -> None:
-        """Wait for everything queued on the engine's device."""
+        """Wait for everything queued on the engine's device.  Raises ``StepLost`` if a step of it did not run to its end."""
         torch.cuda.synchronize(self.rt.device)
+        self.check_steps()
+
+    def check_steps(self) -> None:
+        """Raise ``StepLost`` if a step that the host has waited for (or any before the next) did not run to its end.  Such a step's logits
+        are NaN; whoever reads tokens drawn from them asks here first."""
+        gave_up = getattr(self.rt.ops, "decode_stack_gave_up", None)
+        if gave_up is not None and gave_up(self.workspace):
+            self._lost = set(self.cache.live_requests())
+            raise StepLost("a step waited too long for the rest of its blocks on the device and did not run to its end: "
+                           "its logits are NaN, and the requests that are live have to be released and run again")
 
     def read_device_tokens(self, n: int):
         """Start copying ``device_tokens[:n]`` to the host; returns ``(pinned tensor, event)``.
@@ -397,6 +413,7 @@ class Engine:
     # -- requests --------------------------------------------------------------
     def release(self, request_id) -> None:
         """Give back everything a request holds (finished, cancelled or preempted)."""
+        self._lost.discard(request_id)
         if self.cache.has_request(request_id):
             self.cache.release(request_id)
 
@@ -432,6 +449,8 @@ class Engine:
             for w in e.want:
                 if not (0 <= int(w) < n):
                     raise StepError(f"request {e.request_id!r}: wanted place {w} outside its {n} tokens")
+            if e.request_id in self._lost:
+                raise StepLost(f"request {e.request_id!r}: a step of it did not run to its end; it has to be released and run again")
             have = self.cache.kv_len(e.request_id) if self.cache.has_request(e.request_id) else 0
             if have + n > self.max_model_len:
                 raise StepError(f"request {e.request_id!r}: {have + n} tokens exceed max_model_len {self.max_model_len}")
@@ -444,10 +463,15 @@ class Engine:
         step overwrites.  Raises ``OutOfPages`` (nothing changed) if the cache cannot hold it.
         If the forward pass raises, every request is as long as it was before the step, its
         fixed-size state is what it was (eager steps copy the slots they touch first; a replayed
-        graph either runs whole or not at all), requests
+        graph either runs whole or not at all, but for steps in one launch, which keep no such state), requests
         the step started are gone, and the pages taken are free again (the reference gives a failed
         step's fresh slots back, crates/infer-worker/src/application/worker_scheduler.rs:1090-1133;
-        its leases must be consumed or returned, crates/infer-worker/src/domain/global_kv_alloc.rs:393-461)."""
+        its leases must be consumed or returned, crates/infer-worker/src/domain/global_kv_alloc.rs:393-461).
+        The pass runs on after the call: what goes wrong on the device then (``StepLost``) is raised by the next step,
+        ``synchronize`` or ``check_steps``."""
+        self.check_steps()
+        if self._lost:
+            self._lost.intersection_update(self.cache.live_requests())     # (the scheduler releases through the cache)
         self.validate(entries)
         cache = self.cache
         if not cache.can_append([(e.request_id, len(e.tokens)) for e in entries]):

@@ -534,7 +534,8 @@ def linear_residual(act: torch.Tensor, w: torch.Tensor, w_tiled: Optional[torch.
 
 
 DECODE_STACK_CLOSE_US = 200.0   # how long the first blocks of a one-launch step wait for the rest before they go on without them
-DECODE_STACK_LIMIT_US = 5e6     # and how long they wait for each other's results before they give up
+DECODE_STACK_JOIN_US = 2e7      # and how long one block waits for a second, without which it cannot go on, before it gives up
+DECODE_STACK_LIMIT_US = 5e6     # and how long blocks wait for each other's results before they do
 DECODE_STACK_GRID = 0           # blocks launched: 0 one a compute unit
 
 
@@ -555,13 +556,25 @@ def decode_stack_control(workspace) -> Optional[int]:
     goes.  None if there is none left, or if the stream is under capture and none has been taken."""
     block = getattr(workspace, "_stack_control", None)
     if block is None and not torch.cuda.is_current_stream_capturing():
-        lib, p = _lib(), ctypes.c_void_p()
-        _check(lib.ri_decode_stack_take_control(ctypes.byref(p)))
+        lib, p, word = _lib(), ctypes.c_void_p(), ctypes.c_void_p()
+        _check(lib.ri_decode_stack_take_control(ctypes.byref(p), ctypes.byref(word)))
         block = p.value
         if block is not None:
             workspace._stack_control = block
+            workspace._stack_gave_up = ctypes.c_uint.from_address(word.value)     # (host memory that is never freed)
             weakref.finalize(workspace, lib.ri_decode_stack_give_control, ctypes.c_void_p(block))
     return block
+
+
+def decode_stack_gave_up(workspace) -> bool:
+    """Whether a one-launch step of ``workspace`` did not run to its end: its logits are NaN, and not all of its keys and values are in
+    the cache.  Says so once, and of steps that the host has waited for."""
+    word = getattr(workspace, "_stack_gave_up", None)
+    if word is None or not word.value:
+        return False
+    torch.cuda.synchronize(workspace.device)              # (other blocks of that launch may still be about to say the same)
+    word.value = 0
+    return True
 
 
 def decode_stack(model: torch.Tensor, L: int, ctx, table: torch.Tensor, ff: int, H: int, Hkv: int, hd: int, cos: torch.Tensor, sin: torch.Tensor,
@@ -600,8 +613,8 @@ def decode_stack(model: torch.Tensor, L: int, ctx, table: torch.Tensor, ff: int,
         _ptr(model), L, M, d, ff, H, Hkv, hd, V, _DT[norm_dtype], _ptr(ctx.token_ids), _ptr(tokens), _ptr(table), _ptr(ctx.positions),
         _ptr(ctx.row_of_token), _ptr(ctx.kv_lens), _ptr(block_table), block_table.shape[1], _ptr(cos), _ptr(sin), _ptr(k_pool), _ptr(v_pool),
         ctypes.c_size_t(k_pool.stride(0)), ctypes.c_size_t(v_pool.stride(0)), page, ctypes.c_float(scale), _ptr(logits), V,
-        _ptr(scratch), ctypes.c_size_t(scratch.numel()), ctypes.c_void_p(control), DECODE_STACK_GRID,
-        ctypes.c_double(DECODE_STACK_CLOSE_US), ctypes.c_double(DECODE_STACK_LIMIT_US), _stream()))
+        _ptr(scratch), ctypes.c_size_t(scratch.numel()), ctypes.c_void_p(control), ctypes.byref(ctx.workspace._stack_gave_up), DECODE_STACK_GRID,
+        ctypes.c_double(DECODE_STACK_CLOSE_US), ctypes.c_double(DECODE_STACK_JOIN_US), ctypes.c_double(DECODE_STACK_LIMIT_US), _stream()))
 
 
 DECODE_PAIR_BLOCKS = 0          # blocks of several waves a (kv head, token) pair in single-token attention: 0 the kernel's own choice, 1 one or the split form

@@ -17,7 +17,7 @@ from .config.registry import load_model_config
 from .engine.factory import build_engine
 from .engine.markers import profile_range
 from .engine.scheduler import PENDING, Request, Scheduler
-from .engine.step import StepEntry, device_token
+from .engine.step import StepEntry, StepLost, device_token
 from .sampling.params import SamplingParams
 from .sampling.sampler import Sampler, fresh_seed
 
@@ -156,7 +156,16 @@ class LLM:
         """One scheduler step.  The step is queued on the GPU and its sampled tokens stay there:
         the next step reads them from the device, so it can be prepared and queued while this one
         runs.  Returns [(request, token)] for the tokens that reached the host during this call,
-        which are those of the step before."""
+        which are those of the step before.  If a step did not run to its end on the device (``StepLost``), the requests that had
+        started end as ``"error"``; those that wait are still there."""
+        try:
+            return self._step()
+        except StepLost:
+            self._inflight = None
+            self.scheduler.fail_running()
+            raise
+
+    def _step(self):
         t_start = time.perf_counter() if self._trace_ms is not None else 0.0
         with profile_range("schedule"):
             sched = self.scheduler.schedule()
@@ -228,6 +237,7 @@ class LLM:
             return []
         if event is not None:
             event.synchronize()
+            self.engine.check_steps()
         tokens = host.tolist()
         out = []
         for r, index, slot in marks:
@@ -237,9 +247,12 @@ class LLM:
 
     def drain(self):
         """Wait for the step that is still queued, if any."""
-        produced = self._resolve(self._inflight)
-        self._inflight = None
-        return produced
+        inflight, self._inflight = self._inflight, None
+        try:
+            return self._resolve(inflight)
+        except StepLost:
+            self.scheduler.fail_running()
+            raise
 
     def generate(self, prompts: Sequence[Sequence[int]],
                  sampling_params: Union[None, SamplingParams, Sequence[SamplingParams]] = None

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from rustinfer_amd.cache import OutOfPages
-from rustinfer_amd.engine import Engine, StepEntry, StepError, device_token
+from rustinfer_amd.engine import Engine, StepEntry, StepError, StepLost, device_token
 from rustinfer_amd.parts import PagedKVNeed, Runtime, StateNeed
 
 
@@ -196,3 +196,34 @@ def test_profile_forward_and_resize():
     eng.step([StepEntry("a", [1] * 9, [8])])
     with pytest.raises(CacheError, match="resized"):
         eng.resize_pool(12)
+
+
+def test_a_step_that_did_not_run_to_its_end_is_told_once_and_its_requests_are_refused():
+    """What the device says after the call: the next step, and whoever waits, raises; live requests are refused until they are released, by the engine or
+    through the cache."""
+    class Ops:
+        lost = 0
+
+        def decode_stack_gave_up(self, workspace):
+            said, self.lost = bool(self.lost), 0
+            return said
+
+    eng = engine()
+    eng.rt.ops = Ops()
+    eng.step([StepEntry("a", [1, 2], [1]), StepEntry("b", [3], [0])])
+    eng.check_steps()
+    eng.rt.ops.lost = 1
+    with pytest.raises(StepLost, match="did not run to its end"):
+        eng.step([StepEntry("a", [3], [0]), StepEntry("c", [3], [0])])
+    assert eng.cache.kv_len("a") == 2 and not eng.cache.has_request("c")
+    eng.check_steps()
+    for r in "ab":
+        with pytest.raises(StepLost, match="'%s'.*released and run again" % r):
+            eng.step([StepEntry("c", [3], [0]), StepEntry(r, [3], [0])])
+    assert not eng.cache.has_request("c")
+    eng.step([StepEntry("c", [3], [0])])
+    eng.release("a")
+    eng.cache.release("b")
+    eng.step([StepEntry("a", [1, 2], [1]), StepEntry("b", [3], [0])])
+    eng.step([StepEntry("a", [4], [0]), StepEntry("b", [3], [0])])
+    eng.cache.check()

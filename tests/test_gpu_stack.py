@@ -140,6 +140,70 @@ def test_divided_rows_are_the_same_every_time(engines, divided, monkeypatch, row
     assert rms.mean() <= 1.1 * rms_whole.mean() + 1e-4 * s, (rms.mean() / s, rms_whole.mean() / s)
 
 
+@pytest.mark.parametrize("mode", ["eager", "graph"])
+@pytest.mark.parametrize("times", [dict(LIMIT_US=0.0), dict(GRID=8, CLOSE_US=1e9, JOIN_US=2e3)], ids=["phase", "start"])
+def test_a_step_that_gives_up_is_an_error(engines, monkeypatch, mode, times):
+    """Blocks that wait too long, for each other's results or for a second block, end the step: NaN, and whatever comes next says so, once; the requests
+    have to be released.  The control words are zero again: the same steps then give the same bits as before."""
+    from rustinfer_amd.engine import StepEntry, StepLost
+    from rustinfer_amd.kernels import ops
+    eng, (cfg, _) = engines("64")
+    reqs = random_requests(cfg["vocab_size"], [40, 9, 600], seed=8)
+    before = _decode(eng, reqs, mode)
+    eng.enable_graphs(False)                                   # (drops the graphs)
+    eng.enable_graphs(mode == "graph", capture_sizes=(1, 2, 4, 8))
+    for r, t in reqs.items():
+        eng.step([StepEntry(r, t, [])])
+    with monkeypatch.context() as m:
+        for name, value in times.items():
+            m.setattr(ops, "DECODE_STACK_" + name, value)
+        if mode == "graph":                                    # (the pass before the capture gives up too)
+            with pytest.raises(StepLost, match="did not run to its end"):
+                eng.capture_graphs([3], 700)
+                eng.synchronize()
+            for r, t in reqs.items():
+                with pytest.raises(StepLost, match="released and run again"):
+                    eng.step([StepEntry(r, t[:1], [])])
+                eng.release(r)
+                eng.step([StepEntry(r, t, [])])
+        lost = eng.step([StepEntry(r, [5], [0]) for r in reqs])
+    with pytest.raises(StepLost, match="did not run to its end"):
+        eng.synchronize()
+    assert lost.shape == (3, cfg["vocab_size"]) and bool(torch.isnan(lost).all())
+    eng.synchronize()                                          # (said once)
+    for r in reqs:
+        with pytest.raises(StepLost, match="released and run again"):
+            eng.step([StepEntry(r, [5], [0])])
+        eng.release(r)
+    eng.enable_graphs(False)
+    eng.cache.check()
+    assert np.array_equal(_decode(eng, reqs, mode), before)
+    eng.enable_graphs(False)
+
+
+def test_generate_ends_with_an_error_where_a_step_gives_up(tmp_path, monkeypatch):
+    """No token is taken from logits that are none; requests that had started end as errors, and the next ones run."""
+    from rustinfer_amd import LLM, SamplingParams
+    from rustinfer_amd.config import LlamaConfig
+    from rustinfer_amd.engine import StepLost
+    from rustinfer_amd.kernels import ops
+    from rustinfer_amd.weights import write_random_model
+    monkeypatch.setenv("RUSTINFER_DISABLE_GRAPH", "1")
+    write_random_model(LlamaConfig.from_dict(CONFIGS["64"]), 5, str(tmp_path))
+    llm = LLM(model=str(tmp_path), dtype="bfloat16", paged_block_size=16, num_blocks=64, max_batch_seqs=8, max_model_len=512, max_batch_tokens=512)
+    prompts = [[3, 4, 5, 6], [7, 8, 9, 10, 11, 12]]
+    params = [SamplingParams(temperature=0.0, max_tokens=n, ignore_eos=True) for n in (2, 6)]      # (the first has ended when the step is missed)
+    good = [r.token_ids for r in llm.generate(prompts, params)]
+    with monkeypatch.context() as m:
+        m.setattr(ops, "DECODE_STACK_LIMIT_US", 0.0)
+        with pytest.raises(StepLost):
+            llm.generate(prompts, params)
+    bad = llm.scheduler.finished[-2:]
+    assert {r.finish_reason for r in bad} == {"error"} and all(0 <= t < 512 for r in bad for t in r.output)
+    assert not llm.scheduler.has_work() and not llm.engine.cache.live_requests()
+    assert [r.token_ids for r in llm.generate(prompts, params)] == good
+
+
 def test_control_blocks_are_given_back():
     """A block belongs to one workspace; one that is gone leaves its block to the next, and when all are taken there is none."""
     from rustinfer_amd.engine.context import Workspace

@@ -383,3 +383,28 @@ def test_stop_sequences_with_late_tokens():
 def test_stop_sequences_are_token_ids():
     with pytest.raises(ValueError):
         SamplingParams(stop_sequences=("ab",)).validate()
+
+
+def test_requests_that_have_started_end_as_errors_and_unknown_tokens_go():
+    """A step is lost: running requests end, tokens that never reached the host are off their outputs, also of one that had ended by its length; those that
+    wait still run."""
+    from rustinfer_amd.engine.scheduler import PENDING
+    s, c = make(max_batch_seqs=3)
+    for r, n in (("a", 1), ("b", 2), ("c", 9), ("d", 9)):
+        s.add(req(r, 5, max_tokens=n))
+    for _ in range(2):
+        st = s.schedule()
+        for e in st.entries:
+            c.has_request(e.request.request_id) or c.add_request(e.request.request_id)
+            c.append(e.request.request_id, e.count)
+        s.commit(st)
+        for r in s.running:
+            r.pending_slot = 0
+    a, b, cc, d = (next(r for r in s.finished + s.running + list(s.waiting) if r.request_id == i) for i in "abcd")
+    assert a.state == b.state == "finished" and a.output == [PENDING] and b.output == [PENDING] * 2 and cc.output == [PENDING] * 2
+    assert s.resolve(a, 0, 7) and s.resolve(b, 0, 8) and s.resolve(cc, 0, 9)       # the first step's have arrived
+    s.fail_running()
+    assert a.output == [7] and a.finish_reason == "length"
+    assert b.output == [8] and b.finish_reason == "error" and cc.output == [9] and cc.finish_reason == "error"
+    assert not s.running and d.finish_reason == ("error" if d in s.finished else None)
+    c.check()
