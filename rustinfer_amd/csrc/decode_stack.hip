@@ -5,9 +5,9 @@
 // of the one before to a full stream of its own, 20 us a layer of which the weights take 18.  Here a block a compute unit stays for the whole step
 // and reads ahead: weights do not depend on what is computed, so through the end of one product and while the blocks wait for each other's results
 // the next product's weights keep coming into LDS until the rings are full (128 KB a unit, 32 MB in all).
-// A step then takes, at 100 cached tokens and (2000) ones, parts against this launch, us:
-//     1B 1 row  715 -> 594 (733 -> 665)      3B 1 row  873 -> 796 (901 -> 885)      8B 1 row 1226 -> 1138 (1248 -> 1220)
-//     1B 8 rows 795 -> 683 (873 -> 783)      3B 8 rows 961 -> 907 (1099 -> 1051)    8B 8 rows 1322 -> 1253 (1423 -> 1373)
+// A step then takes, at 100 cached tokens and (2000) and [16000] ones, parts against this launch, us:
+//     1B 1 row  721 -> 581 (731 -> 642) [838 -> 730]       3B 1 row  901 -> 795 (899 -> 851) [1095 -> 974]      8B 1 row 1267 -> 1147 (1245 -> 1192) [1410 -> 1297]
+//     1B 8 rows 804 -> 669 (878 -> 793) [1502 -> 1345]     3B 8 rows 967 -> 893 (1110 -> 1050) [1999 -> 2013]   8B 8 rows 1323 -> 1234 (1446 -> 1381) [2214 -> 2203]
 // What is left above the weights are the five waits of a layer, 2.1 us each from the last block's result to the first block's go on.
 //
 // Waves of a block: eight multiply (readers), two fill their rings, one is the control wave: it waits for the other blocks, finishes the readers'
@@ -56,7 +56,8 @@ constexpr int L_RING = 0, L_RED = WAVES * RING * 1024, L_ATT = L_RED + 2 * WAVES
               L_MISC = L_ML + WAVES * 16 * 2 * 4, L_X = L_MISC + 256, L_BYTES = L_X + X_ITEMS * 256;
 static_assert(L_BYTES <= 160 * 1024, "a compute unit's LDS");
 // words of L_MISC
-enum { W_RANK = 0, W_N = 1, W_STOP = 2, W_GO = 3, W_LENGTH = 4, W_ROW = 12, W_LANDED = 20, W_READ = 24, W_SUMS = 32, W_FINISHED = 34, W_MEET = 35 };
+enum { W_RANK = 0, W_N = 1, W_STOP = 2, W_GO = 3, W_LENGTH = 4, W_ROW = 12, W_LANDED = 20, W_READ = 24, W_SUMS = 32, W_FINISHED = 34, W_MEET = 35,
+       W_FIRST = 40 };        // W_FIRST + m: parts of the rows before row m
 
 // control words, a line of 128 bytes each, and behind them counters of the parts of a row's keys; all zero between launches
 enum { C_ARRIVED = 0, C_FULL = 8, C_CLOSING = 9, C_STATE = 10, C_MEMBERS = 11, C_DONE = 12, C_LEFT = 20, C_ALL_LEFT = 28, C_PAIRS = 29 };
@@ -76,14 +77,17 @@ struct Kind { int items, units, stride; unsigned tile, second; int whole; };
 // offsets within a layer's stretch of scratch, multiples of 256 bytes
 struct Offsets { size_t a, ssq, q, at, a2, ssq2, h, po, pml, all; };
 __host__ __device__ inline size_t up256(size_t n) { return (n + 255) & ~(size_t)255; }
-// The parts of a row's keys for the G queries of a key/value head, a pair: a query's outputs of a part (hd floats) in `po`, its maximum and sum in `pml`.
-// A pair is merged when its own parts are there, while others still write theirs: its stretch of either is whole lines of its own (128 bytes; 256 here), or
-// the merge would bring a line into its L2 in which another pair's entries are not yet what a merge on the same XCD then reads.
+// A part of a row's keys, for the G queries of a key/value head, leaves its unnormalised outputs (G x hd floats) in a slot of `po` and their maxima and sums in one of
+// `pml`.  A row is merged when its own parts are there, while others still write theirs: a slot of either is whole lines of its own (128 bytes), or a merge
+// would bring a line into its L2 in which another row's entries are not yet what a merge on the same XCD then reads.
 constexpr size_t LINE = 128;
-__host__ __device__ inline size_t pair_outputs(int G, int slots, int hd) { return (size_t)G * slots * hd * 4; }          // bytes; hd is 64 or 128
-__host__ __device__ inline size_t pair_sums(int G, int slots) { return up256((size_t)G * slots * 8); }
-static_assert(64 * 4 % LINE == 0 && 256 % LINE == 0, "a pair's stretches are whole lines");
-__host__ __device__ inline Offsets stack_offsets(int M, int d, int ff, int H, int Hkv, int hd, int slots) {
+__host__ __device__ inline size_t slot_outputs(int G, int hd) { return (size_t)G * hd * 4; }                             // bytes; hd is 64 or 128
+constexpr size_t SLOT_SUMS = LINE;                                                                                       // G pairs of floats, G <= 16
+static_assert(64 * 4 % LINE == 0 && 16 * 8 <= SLOT_SUMS, "a slot is whole lines");
+// A row's keys are divided between blocks in parts of at most `share` (a multiple of PART_KEYS: a part's waves take spans of SPAN keys in turn).
+constexpr int SPAN = 32, PART_KEYS = WAVES * SPAN, WHOLE_KEYS = 2 * PART_KEYS;
+__host__ __device__ inline int parts_of(int len, int share) { return len <= share ? 1 : (len + share - 1) / share; }
+__host__ __device__ inline Offsets stack_offsets(int M, int d, int ff, int H, int Hkv, int hd, int blocks) {
     Offsets o;
     size_t at = 0;
     auto take = [&](size_t n) { const size_t r = at; at += up256(n); return r; };
@@ -91,7 +95,7 @@ __host__ __device__ inline Offsets stack_offsets(int M, int d, int ff, int H, in
     o.q = take((size_t)M * H * hd * 2); o.at = take((size_t)M * H * hd * 2);
     o.a2 = take((size_t)M * d * 2); o.ssq2 = take((size_t)M * (d / 8) * 4);
     o.h = take((size_t)M * ff * 2);
-    o.po = take(M * Hkv * pair_outputs(H / Hkv, slots, hd)); o.pml = take(M * Hkv * pair_sums(H / Hkv, slots));
+    o.po = take(blocks * slot_outputs(H / Hkv, hd)); o.pml = take(blocks * SLOT_SUMS);                       // (where rows are divided, a block has one part)
     o.all = at;
     return o;
 }
@@ -107,7 +111,6 @@ struct StackArgs {
     float* logits; int ld_logits;
     char* scratch; size_t layer_bytes;                  // buffers that the phases leave for each other, a stretch a layer
     float* x;                                           // [d / 8][8][8] the residual stream, by items
-    int slots;                                          // parts of a row's keys there is room for
     unsigned* control; int expect;                      // blocks that may take part: a multiple of 8
     unsigned* gave_up;                                  // host memory: set by a launch that did not run to its end
     unsigned long long close_ticks, join_ticks, limit_ticks;
@@ -353,12 +356,17 @@ struct Reader {
     }
 };
 
-// A row's keys are divided between `parts` blocks (the same for all rows at most); the blocks' waves take its spans of 32 keys in turn.
-constexpr int SPAN = 32, PART_KEYS = WAVES * SPAN, WHOLE_KEYS = 2 * PART_KEYS;
-__device__ __forceinline__ int most_parts(int longest, int slots, int n, int pairs) {
-    return longest <= WHOLE_KEYS ? 1 : max(1, min(min(slots, n / pairs), (longest + PART_KEYS - 1) / PART_KEYS));
+// How the rows' keys are divided: between all blocks by the rows' lengths, so that the longest share, which the others wait for, is as short as it can be (with as many parts
+// for every row, 8 rows of which one had 16,000 keys and the others 100 took 1,644 us at the 3B sizes, now 1,113, part by part 1,145; 4,000 and 100 1,103 / 1,002 / 1,069).  Not where the longest row has
+// WHOLE_KEYS keys or fewer: a merge costs more than it gives.  `total` of a share: the parts of all rows.
+template <typename F> __device__ __forceinline__ int share_of(F total, int longest, int budget, int rows, int lane) {
+    if (longest <= WHOLE_KEYS || budget <= rows) return 0x7fffffff;
+    for (int unit = PART_KEYS; unit < 1 << 24; unit *= 2) {                // (the 64 lanes try a multiple each)
+        const unsigned long long fits = __ballot(total(unit * (lane + 1)) <= budget);
+        if (fits) return unit * (__builtin_ctzll(fits) + 1);
+    }
+    return 0x7fffffff;
 }
-__device__ __forceinline__ int row_parts(int len, int most) { return min(most, max(1, (len + PART_KEYS - 1) / PART_KEYS)); }
 
 // A span's keys and values as the matrix instructions read them: tile e of the keys holds, in row r, key 8 (r / 4) + 4 e + r % 4.
 template <int HD> struct SpanOf { sbf16x8_t k[2][HD / 32], v[HD / 16]; };
@@ -505,24 +513,57 @@ __device__ __forceinline__ float sum_of_eight(float v) {
     return v;
 }
 
-// The parts of a row's keys for the G queries of a key/value head, by one wave: eight values a lane.
+// The parts of a row's keys for the G queries of a key/value head, by one wave: eight values a lane.  What is asked for stands behind the weights under way, so it
+// is asked for at once: maxima, sums and outputs of eight parts, those of head size 64 by two halves of the wave where 32 lanes hold a part (and by four
+// parts a turn, as that kernel gets slower with the registers of eight: 580 -> 615 us a step of one row).  us a step of one row of 8,000 keys, a trip for the maxima
+// and one for every four parts / this: 1B 707 / 689, 3B 993 / 908, 8B 1311 / 1242.
 template <int HD>
-__device__ __forceinline__ void merge(const char* po, const char* pml, int pair, int slots, int parts, int G, bf16_t* out, int lane) {
-    const int e = lane * 8, qi = e / HD;
+__device__ __forceinline__ void merge(const char* po, const char* pml, size_t first, int step, int parts, int G, bf16_t* out, int lane) {
+    constexpr int TURN = HD == 64 ? 4 : 8;
+    const bool halves = HD == 64 && G * HD <= 256;
+    const int e = (halves ? lane & 31 : lane) * 8, qi = e / HD, by = halves ? 2 : 1;
     if (e >= G * HD) return;
-    const float* ml = reinterpret_cast<const float*>(pml + pair * pair_sums(G, slots)) + (size_t)qi * slots * 2;
-    const float* o = reinterpret_cast<const float*>(po + pair * pair_outputs(G, slots, HD)) + (size_t)qi * slots * HD + e % HD;
+    const char* ml = pml + first * SLOT_SUMS + qi * 8;
+    const char* o = po + first * slot_outputs(G, HD) + (size_t)e * 4;
+    const size_t ml_step = step * SLOT_SUMS, o_step = step * slot_outputs(G, HD);
     float top = -INFINITY, sum = 0.f, v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int p = 0; p < parts; ++p) top = fmaxf(top, ml[p * 2]);
-#pragma unroll 4
-    for (int p = 0; p < parts; ++p) {
-        const float2 two = *reinterpret_cast<const float2*>(ml + p * 2);
-        const float4 a = *reinterpret_cast<const float4*>(o + (size_t)p * HD), b = *reinterpret_cast<const float4*>(o + (size_t)p * HD + 4);
-        const float w = two.x == -INFINITY ? 0.f : __expf(two.x - top);
-        sum += w * two.y;
-        v[0] += w * a.x; v[1] += w * a.y; v[2] += w * a.z; v[3] += w * a.w;
-        v[4] += w * b.x; v[5] += w * b.y; v[6] += w * b.z; v[7] += w * b.w;
+#pragma unroll 1
+    for (int p0 = halves ? lane >> 5 : 0; p0 < parts; p0 += TURN * by) {
+        float2 two[TURN];
+        float4 a[TURN], b[TURN];
+#pragma unroll
+        for (int u = 0; u < TURN; ++u) {
+            const size_t p = min(p0 + u * by, parts - 1);                  // (beyond the last: again, and without weight)
+            two[u] = *reinterpret_cast<const float2*>(ml + p * ml_step);
+            a[u] = *reinterpret_cast<const float4*>(o + p * o_step);
+            b[u] = *reinterpret_cast<const float4*>(o + p * o_step + 16);
+        }
+        __builtin_amdgcn_sched_barrier(0);                                 // (all of them under way before the first is waited for)
+        float most = top;
+#pragma unroll
+        for (int u = 0; u < TURN; ++u) most = fmaxf(most, two[u].x);
+        const float base = most == -INFINITY ? 0.f : most, alpha = __expf(top - base);
+        top = most;
+        sum *= alpha;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] *= alpha;
+#pragma unroll
+        for (int u = 0; u < TURN; ++u) {
+            const bool there = p0 + u * by < parts;
+            const float w = !there || two[u].x == -INFINITY ? 0.f : __expf(two[u].x - base);
+            sum += w * two[u].y;
+            if (!there) a[u] = b[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            v[0] += w * a[u].x; v[1] += w * a[u].y; v[2] += w * a[u].z; v[3] += w * a[u].w;
+            v[4] += w * b[u].x; v[5] += w * b[u].y; v[6] += w * b[u].z; v[7] += w * b[u].w;
+        }
+    }
+    if (halves) {
+        const float other = __shfl_xor(top, 32, 64), most = fmaxf(top, other), base = most == -INFINITY ? 0.f : most;
+        const float mine = __expf(top - base), theirs = __expf(other - base);
+        sum = sum * mine + __shfl_xor(sum, 32, 64) * theirs;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) v[i] = v[i] * mine + __shfl_xor(v[i], 32, 64) * theirs;
+        if (lane >= 32) return;
     }
 #pragma unroll
     for (int i = 0; i < 8; i += 2)
@@ -604,6 +645,19 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
         }
         if (rank >= n) n = 0;                             // (an odd one out: items of half a tile keep their half from one to the next)
         if (lane == 0) { misc[W_RANK] = rank; misc[W_N] = n; }
+        if (n > 0) {
+            const int M = again(A)->M, len = lane < MAX_ROWS ? misc[W_LENGTH + lane] : 0;
+            int longest = 0;
+            for (int m = 0; m < M; ++m) longest = max(longest, __builtin_amdgcn_readlane(len, m));
+            const int share = share_of([&](int s) {
+                int sum = 0;
+                for (int m = 0; m < M; ++m) sum += parts_of(__builtin_amdgcn_readlane(len, m), s);
+                return sum;
+            }, longest, n / again(A)->Hkv, M, lane);
+            int first = 0;
+            for (int m = 0; m < M; ++m) first += m < lane ? parts_of(__builtin_amdgcn_readlane(len, m), share) : 0;
+            if (lane <= MAX_ROWS) misc[W_FIRST + lane] = first;
+        }
         begun = wall_clock64();
     }
     __syncthreads();
@@ -611,11 +665,16 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
     const unsigned words = lds_address(lds + L_MISC);
     if (n > 0) {
         const int H = again(A)->H, Hkv = again(A)->Hkv, G = H / Hkv, q_dim = H * HD, M = again(A)->M;
-        const int pairs = M * Hkv;
-        int longest = 0;
-        for (int i = 0; i < M; ++i) longest = max(longest, misc[W_LENGTH + i]);
-        const int most = __builtin_amdgcn_readfirstlane(most_parts(longest, again(A)->slots, n, pairs));
-        const int jobs = pairs * most;
+        const int jobs = __builtin_amdgcn_readfirstlane(misc[W_FIRST + M]) * Hkv;                  // parts of rows, by key/value heads
+        // the row of a job, of which this is part `part` of `parts`
+        auto row_of = [&](int job, int& part, int& parts) {
+            const int at = job / Hkv;
+            int m = 0, from = 0, to = __builtin_amdgcn_readfirstlane(misc[W_FIRST + 1]);
+            while (at >= to) { ++m; from = to; to = __builtin_amdgcn_readfirstlane(misc[W_FIRST + 1 + m]); }
+            part = at - from;
+            parts = to - from;
+            return m;
+        };
         if (wave >= FIRST_LOADER) {
             Loader loader(A, rank, n, (wave - FIRST_LOADER) * SERVED, lane, lds + L_RING, words);
             loader.run();
@@ -642,8 +701,8 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                     int job = rank, m = 0, g = 0, part = 0, parts = 1;
                     bool asked = false;
                     auto take_job = [&]() {
-                        const int pair = job % pairs;
-                        part = job / pairs; m = pair / Hkv; g = pair - m * Hkv;
+                        m = row_of(job, part, parts);
+                        g = job % Hkv;
                         const int b = __builtin_amdgcn_readfirstlane(misc[W_ROW + m]);
                         at.len = __builtin_amdgcn_readfirstlane(misc[W_LENGTH + m]);
                         at.lane = lane;
@@ -651,12 +710,11 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                         at.kc = P->kc + (size_t)l * P->k_layer + (size_t)g * (16 * HD);
                         at.vc = P->vc + (size_t)l * P->v_layer + (size_t)g * (16 * HD);
                         at.pages = (const __attribute__((address_space(4))) int*)(uintptr_t)(P->blocks + (size_t)max(b, 0) * P->max_blocks);
-                        parts = row_parts(at.len, most);
                     };
                     if (job < jobs) {
                         take_job();
                         const int sp = part * WAVES + wave;
-                        asked = part < parts && (sp + 1) * SPAN < at.len;      // (not the span that this step's own key is in)
+                        asked = (sp + 1) * SPAN < at.len;      // (not the span that this step's own key is in)
                         if (asked) { at.keys(sp); at.values(sp); }
                     }
                     wait_word(words, W_GO, ++begun_phases);
@@ -664,11 +722,11 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                     const bf16_t* q = reinterpret_cast<const bf16_t*>(base + P->off.q);
                     for (; job < jobs; job += n, asked = false) {
                         if (job != rank) take_job();
-                        const bool some = at.len > 0 && part < parts;
+                        const bool some = at.len > 0;
                         if (some) at.run(q + (size_t)m * q_dim + (size_t)g * G * HD, G, P->scale, part * WAVES + wave, parts * WAVES, asked, att_o + wave * ATT_VALUES, att_ml + wave * 32);
                         s.meet();
                         const int e = (wave * 64 + lane) * 2;
-                        if (e < G * HD && part < parts) {
+                        if (e < G * HD) {
                             const int qi = e / HD, dd = e - qi * HD;
                             float v0 = 0.f, v1 = 0.f, top = -INFINITY, sum = 0.f;
                             if (some) {
@@ -688,10 +746,9 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                                 st_agent(reinterpret_cast<unsigned*>(attn + (size_t)m * q_dim + (size_t)g * G * HD + e),
                                          (unsigned)f32_to_bf16(v0) | ((unsigned)f32_to_bf16(v1) << 16));
                             } else {
-                                const int slots = P->slots, pair = m * Hkv + g, slot = qi * slots + part;
-                                st_agent(reinterpret_cast<unsigned long long*>(po + pair * pair_outputs(G, slots, HD) + ((size_t)slot * HD + dd) * 4),
+                                st_agent(reinterpret_cast<unsigned long long*>(po + job * slot_outputs(G, HD) + (size_t)e * 4),
                                          (unsigned long long)__float_as_uint(v0) | ((unsigned long long)__float_as_uint(v1) << 32));
-                                if (dd == 0) st_agent(reinterpret_cast<unsigned long long*>(pml + pair * pair_sums(G, slots) + (size_t)slot * 8),
+                                if (dd == 0) st_agent(reinterpret_cast<unsigned long long*>(pml + job * SLOT_SUMS + qi * 8),
                                                       (unsigned long long)__float_as_uint(top) | ((unsigned long long)__float_as_uint(sum) << 32));
                             }
                         }
@@ -775,15 +832,16 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                         wait_word(words, W_SUMS + (sums & 1), (sums / 2 + 1) * WAVES);
                         ++sums;
                         set_word(words + W_FINISHED * 4, sums);
-                        const int pair = job % pairs, row = pair / Hkv, parts = row_parts(__builtin_amdgcn_readfirstlane(misc[W_LENGTH + row]), most);
-                        if (parts == 1 || job / pairs >= parts) continue;
+                        int part, parts;
+                        const int row = row_of(job, part, parts), g = job % Hkv;
+                        if (parts == 1) continue;
                         // whoever leaves the last part of a row's keys merges them all
                         unsigned before = 0;
-                        if (lane == 0) before = add_agent(ctl + C_PAIRS * 32 + pair * PAIR_WORDS, 1u);
+                        if (lane == 0) before = add_agent(ctl + C_PAIRS * 32 + (row * Hkv + g) * PAIR_WORDS, 1u);
                         if (__builtin_amdgcn_readfirstlane((int)before) != (l + 1) * parts - 1) continue;
                         asm volatile("" ::: "memory");
-                        merge<HD>(base + P->off.po, base + P->off.pml, pair, P->slots, parts, G,
-                                  reinterpret_cast<bf16_t*>(base + P->off.at) + (size_t)row * q_dim + (size_t)(pair - row * Hkv) * G * HD, lane);
+                        merge<HD>(base + P->off.po, base + P->off.pml, job - part * Hkv, Hkv, parts, G,
+                                  reinterpret_cast<bf16_t*>(base + P->off.at) + (size_t)row * q_dim + (size_t)g * G * HD, lane);
                     }
                 }
                 float rs = 1.f;
@@ -914,11 +972,6 @@ int stack_blocks() {
     if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) return 0;
     return cu / 8 * 8;
 }
-int stack_slots(int M, int Hkv, int blocks) {
-    const int s = blocks / (M * Hkv);
-    return s < 1 ? 1 : s > 64 ? 64 : s;
-}
-
 // Control blocks, a launch's at a time: of uncached memory, which is never freed (memory of that kind has to stay once a kernel has read
 // it), so a device has one stretch of MOST_BLOCKS, made when the first is taken.  A block belongs to whoever took it until it is given back.
 constexpr int MOST_BLOCKS = 64, BLOCK_BYTES = 16 * 1024;
@@ -981,19 +1034,19 @@ extern "C" int ri_decode_stack_give_control(void* block) {
 }
 
 // Whether a step of M single tokens of such a stack goes in one launch: what the kernel holds in registers and LDS, whole steps of K for every
-// reader.  Where it fits it is the faster form at every size measured (1 to 8 rows, 1B to 8B, 100 to 2000 cached tokens: above).
+// reader.  (Whether it pays depends on the cached tokens too: ops.decode_stack_pays.)
 extern "C" int ri_decode_stack_takes(int M, int d, int ff, int H, int Hkv, int hd, int page, int V) {
     return M >= 1 && M <= MAX_ROWS && (hd == 64 || hd == 128) && page == 16 && Hkv >= 1 && M * Hkv <= MOST_PAIRS && H >= 1 && H % Hkv == 0
         && H / Hkv <= 16 && H / Hkv * hd <= ATT_VALUES && d >= 512 && d % 512 == 0 && d <= 8192 && H * hd % 512 == 0 && H * hd <= 8192
         && ff >= 512 && ff % 512 == 0 && ff <= 14336 && V % 16 == 0 && V > 0;
 }
-// Where the parts of the keys of row m and key/value head g lie in a layer's stretch, with room for `slots` of them: from[0], to[0] their outputs, from[1], to[1]
-// their maxima and sums, in bytes; *line: what two pairs may not share.
-extern "C" void ri_decode_stack_pair(int M, int d, int ff, int H, int Hkv, int hd, int slots, int m, int g, size_t* from, size_t* to, size_t* line) {
-    const Offsets o = stack_offsets(M, d, ff, H, Hkv, hd, slots);
-    const int pair = m * Hkv + g, G = H / Hkv;
-    from[0] = o.po + pair * pair_outputs(G, slots, hd); to[0] = from[0] + (size_t)G * slots * hd * 4;
-    from[1] = o.pml + pair * pair_sums(G, slots); to[1] = from[1] + (size_t)G * slots * 8;
+// Where slot `slot` of the parts of rows lies in a layer's stretch, with `blocks` of them: from[0], to[0] its outputs, from[1], to[1] its maxima and sums, in
+// bytes; *line: what two slots may not share.
+extern "C" void ri_decode_stack_slot(int M, int d, int ff, int H, int Hkv, int hd, int blocks, int slot, size_t* from, size_t* to, size_t* line) {
+    const Offsets o = stack_offsets(M, d, ff, H, Hkv, hd, blocks);
+    const int G = H / Hkv;
+    from[0] = o.po + slot * slot_outputs(G, hd); to[0] = from[0] + (size_t)G * hd * 4;
+    from[1] = o.pml + slot * SLOT_SUMS; to[1] = from[1] + (size_t)G * 8;
     *line = LINE;
 }
 // Entries of the model's table.
@@ -1002,7 +1055,7 @@ extern "C" int ri_decode_stack_table(int L) { return 4 * L + 1 + 2 * (2 * L + 1)
 extern "C" size_t ri_decode_stack_scratch(int L, int M, int d, int ff, int H, int Hkv, int hd) {
     const int blocks = stack_blocks();
     if (blocks < 8 || M < 1 || Hkv < 1) return 0;
-    return (size_t)(L + 1) * stack_offsets(M, d, ff, H, Hkv, hd, stack_slots(M, Hkv, blocks)).all + up256((size_t)d * MAX_ROWS * 4);
+    return (size_t)(L + 1) * stack_offsets(M, d, ff, H, Hkv, hd, blocks).all + up256((size_t)d * MAX_ROWS * 4);
 }
 
 // model: the table of L layers on the device (ri_decode_stack_table entries, see above), the weights in tile order (q/k/v with rows in
@@ -1033,8 +1086,7 @@ extern "C" int ri_decode_stack(const void* model, int L, int M, int d, int ff, i
     A.positions = positions; A.row_of_token = row_of_token; A.kv_lens = kv_lens; A.blocks = blocks; A.max_blocks = max_blocks;
     A.cos_t = cos_t; A.sin_t = sin_t; A.kc = (bf16_t*)kc; A.vc = (bf16_t*)vc; A.k_layer = k_layer; A.v_layer = v_layer; A.scale = scale;
     A.logits = logits; A.ld_logits = ld_logits;
-    A.slots = stack_slots(M, Hkv, all);
-    A.off = stack_offsets(M, d, ff, H, Hkv, hd, A.slots);
+    A.off = stack_offsets(M, d, ff, H, Hkv, hd, all);
     A.layer_bytes = A.off.all;
     A.scratch = (char*)scratch;
     A.x = (float*)(A.scratch + (size_t)(L + 1) * A.layer_bytes);

@@ -544,6 +544,19 @@ def decode_stack_takes(M: int, d: int, ff: int, H: int, Hkv: int, hd: int, page:
     return not FORCE_LIBRARY_GEMM and bool(_lib().ri_decode_stack_takes(M, d, ff, H, Hkv, hd, page, V))
 
 
+DECODE_STACK_MOST_KEYS = 80 << 10   # tokens x cached tokens beyond which steps of three tokens or more at head size 128 go part by part
+
+
+def decode_stack_pays(M: int, hd: int, max_kv_len: int) -> bool:
+    """Whether a step of ``M`` tokens over at most ``max_kv_len`` keys a row is faster in one launch.  At head size 128 the parts read the keys of three rows or more
+    as one list that all waves of the chip divide evenly, the launch reads a row's by one block a part, beside the weights; where keys are most of a step's bytes
+    that costs more than the launches saved.  Measured, us, parts / one launch, 3B and 8B sizes: 8 rows of 8,000 1501 1782 / 1451 1725, of 12,000 1754 2061 /
+    1733 2025, of 16,000 1999 2214 / 2013 2203, of 32,000 2989 3047 / 3116 3104; 6 of 16,000 1710 1953 / 1747 1961; 4 of 16,000 1449 1715 / 1415 1681, of 32,000
+    1929 2128 / 1999 2161; one of 130,000 beside 7 of 100 2065 2238 / 2178 2323.  One and two rows, and head size 64, at every length: 2 of 64,000 2054 2236 / 1977 2148,
+    one of 130,000 2093 2257 / 1980 2157; 1B, 8 of 64,000 3547 / 3200."""
+    return hd != 128 or M < 3 or M * max_kv_len <= DECODE_STACK_MOST_KEYS
+
+
 def decode_stack_scratch(L: int, d: int, ff: int, H: int, Hkv: int, hd: int, rows: int = 8) -> int:
     """Bytes of scratch that steps of up to ``rows`` tokens take."""
     lib = _lib()

@@ -75,8 +75,8 @@ class DecodeStack:
                                          first.mixer.head_dim, 16, model.vocab_size)
 
     def takes(self, ctx, caches) -> bool:
-        """Whether the step is of single tokens, all wanted, over one group of caches that holds a layer's after the other, and
-        there is a control block for it."""
+        """Whether the step is of single tokens, all wanted, over one group of caches that holds a layer's after the other, not so many keys that the
+        parts are faster, and there is a control block for it."""
         T = ctx.num_tokens
         if ctx.max_q_len != 1 or ctx.num_want != T or not getattr(ctx, "want_all_in_order", False) or ctx.num_rows < T:
             return False
@@ -84,6 +84,8 @@ class DecodeStack:
         if not groups or len(groups) != 1 or len(groups[0].cache_ids) != self.layers:
             return False
         ops = self.rt.ops
+        if not ops.decode_stack_pays(T, self.hd, ctx.max_kv_len):
+            return False
         return ops.decode_stack_takes(T, self.hidden_size, self.ff, self.H, self.Hkv, self.hd, groups[0].page_size, self.vocab_size) \
             and ops.decode_stack_control(ctx.workspace) is not None
 

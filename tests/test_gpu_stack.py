@@ -36,7 +36,8 @@ CASES = [("64", [5 + LAST], "eager", 0), ("64", LONG, "eager", 0), ("64", LONG[4
          ("64 uneven", LONG[2:7], "graph", 0), ("64 uneven", LONG[:6], "eager", 8), ("64 wide", LONG[3:6], "eager", 0),
          ("64 one head", [1700, 3, 640], "graph", 0), ("128", LONG[1:5], "graph", 0), ("128", [900], "eager", 64),
          ("128 long", [33, 600], "eager", 0), ("128 wide", LONG[:7], "eager", 0),
-         ("128 longest", LONG, "graph", 0)]
+         ("128 longest", LONG, "graph", 0), ("128 three", [LAST, 40, 1999, 513, 9, 700, 64, 100], "graph", 0),
+         ("128 three", [9, 1030, 30, 1999], "eager", 64)]
 
 
 @pytest.fixture(scope="module")
@@ -202,6 +203,31 @@ def test_generate_ends_with_an_error_where_a_step_gives_up(tmp_path, monkeypatch
     assert {r.finish_reason for r in bad} == {"error"} and all(0 <= t < 512 for r in bad for t in r.output)
     assert not llm.scheduler.has_work() and not llm.engine.cache.live_requests()
     assert [r.token_ids for r in llm.generate(prompts, params)] == good
+
+
+def test_steps_of_many_keys_go_part_by_part(engines, monkeypatch):
+    """The rule goes by the longest row and the number of rows, of a captured step by what its key says of them."""
+    from rustinfer_amd.engine import StepEntry
+    from rustinfer_amd.kernels import ops
+    eng, (cfg, _) = engines("128")
+    launches = []
+    real = ops.decode_stack
+    monkeypatch.setattr(ops, "decode_stack", lambda *a, **k: (launches.append(1), real(*a, **k))[1])
+    monkeypatch.setattr(ops, "DECODE_STACK_MOST_KEYS", 4 * 100)
+    for r in range(4):
+        eng.step([StepEntry(r, [5] * (99 - r), [])])
+    eng.step([StepEntry(r, [5], [0]) for r in range(4)])              # 4 x 100
+    assert len(launches) == 1
+    eng.step([StepEntry(r, [5], [0]) for r in range(4)])              # 4 x 101
+    assert len(launches) == 1
+    eng.step([StepEntry(r, [5], [0]) for r in range(2)])
+    assert len(launches) == 2
+    eng.enable_graphs(True, capture_sizes=(1, 2, 4, 8))
+    eng.step([StepEntry(r, [5], [0]) for r in range(4)])              # 4 x 1024
+    assert len(launches) == 2
+    eng.enable_graphs(False)
+    for r in range(4):
+        eng.release(r)
 
 
 def test_control_blocks_are_given_back():

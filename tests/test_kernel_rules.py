@@ -131,15 +131,22 @@ def test_steps_that_go_in_one_launch(lib, change, takes):
 
 @pytest.mark.parametrize("H,Hkv,hd", [(24, 8, 128), (32, 8, 64), (32, 8, 128), (40, 8, 64), (72, 9, 64), (8, 1, 64), (8, 8, 128), (36, 9, 128)])
 def test_divided_rows_share_no_line_in_the_one_launch_step(lib, H, Hkv, hd):
-    """A pair of row and key/value head is merged while others still write their parts, and its line may then stay in an L2: the parts of no two pairs have a
-    line in common, nor do outputs and sums."""
+    """A row is merged while others still write their parts, and its lines may then stay in an L2: no two slots of parts have a line in common, nor
+    do outputs and sums, and all lie within the stretch."""
     from_, to, line = (ctypes.c_size_t * 2)(), (ctypes.c_size_t * 2)(), ctypes.c_size_t(0)
     for M in range(1, 9):
-        for slots in {max(1, min(64, 256 // (M * Hkv))), 1, 3, 7, 64}:
+        for blocks in (8, 256):
             owner = {}
-            for pair in range(M * Hkv):
-                lib.ri_decode_stack_pair(M, 512, 512, H, Hkv, hd, slots, pair // Hkv, pair % Hkv, from_, to, ctypes.byref(line))
-                assert line.value >= 128 and to[0] - from_[0] == H // Hkv * slots * hd * 4 and to[1] - from_[1] == H // Hkv * slots * 8
+            for slot in range(blocks):
+                lib.ri_decode_stack_slot(M, 512, 512, H, Hkv, hd, blocks, slot, from_, to, ctypes.byref(line))
+                assert line.value >= 128 and to[0] - from_[0] == H // Hkv * hd * 4 and to[1] - from_[1] == H // Hkv * 8
                 for kind in range(2):
                     for n in range(from_[kind] // line.value, (to[kind] - 1) // line.value + 1):
-                        assert owner.setdefault(n, (pair, kind)) == (pair, kind), (M, slots, pair, kind)
+                        assert owner.setdefault(n, (slot, kind)) == (slot, kind), (M, blocks, slot, kind)
+
+
+@pytest.mark.parametrize("rows,hd,keys,pays", [(1, 128, 1 << 20, True), (2, 128, 131072, True), (8, 128, 8192, True), (8, 128, 10240, True), (8, 128, 11264, False),
+                                               (4, 128, 20480, True), (4, 128, 32768, False), (3, 128, 131072, False), (8, 64, 131072, True)])
+def test_long_rows_leave_the_one_launch_step(rows, hd, keys, pays):
+    from rustinfer_amd.kernels import ops
+    assert ops.decode_stack_pays(rows, hd, keys) is pays
