@@ -37,6 +37,7 @@
 // us: fewer items are dealt less evenly.)  The norms are the products' own, as in gemm.hip (RESID, SCALE).
 #include "common.h"
 #include <math.h>
+#include <stdio.h>
 #include <mutex>
 
 typedef __bf16 sbf16x8_t __attribute__((ext_vector_type(8)));
@@ -977,34 +978,42 @@ int stack_blocks() {
 constexpr int MOST_BLOCKS = 64, BLOCK_BYTES = 16 * 1024;
 static_assert(CONTROL_WORDS * 4 <= BLOCK_BYTES, "a control block");
 // With each goes a word of pinned host memory, likewise never freed, that a launch sets which gives up.
-struct ControlBlocks { char* base = nullptr; unsigned* words = nullptr; bool out[MOST_BLOCKS] = {}; };
+struct ControlBlocks { char* base = nullptr; unsigned* words = nullptr; bool refused = false, out[MOST_BLOCKS] = {}; };
 constexpr int WORD_STEP = 32;                            // a line each
 std::mutex control_mutex;
 ControlBlocks control_blocks[64];
 
 }  // namespace
 
-// A control block of zeros on the current device and its word (0) on the host, or null in *block if all are taken.  Waits for the device: not under capture.
+// A control block of zeros on the current device and its word (0) on the host, or null in *block if none is to be had: all are taken, or the memory for them is
+// refused (which is said once, and not asked for again).  Waits for the device: not under capture.
 extern "C" int ri_decode_stack_take_control(void** block, unsigned** gave_up) {
     RI_REQUIRE(block && gave_up, "ri_decode_stack_take_control: null pointer");
     *block = nullptr;
     *gave_up = nullptr;
     int dev = 0;
     hipError_t e = hipGetDevice(&dev);
-    RI_REQUIRE(e == hipSuccess && dev >= 0 && dev < 64, "ri_decode_stack_take_control: no current device: %s", hipGetErrorString(e));
+    if (e != hipSuccess || dev < 0 || dev >= 64) {
+        (void)hipGetLastError();
+        return 0;
+    }
     std::lock_guard<std::mutex> lock(control_mutex);
     ControlBlocks& c = control_blocks[dev];
+    if (c.refused) return 0;
     if (!c.base) {
-        void* p = nullptr;
-        e = hipExtMallocWithFlags(&p, (size_t)MOST_BLOCKS * BLOCK_BYTES, hipDeviceMallocUncached);
-        RI_REQUIRE(e == hipSuccess, "ri_decode_stack_take_control: %d bytes of uncached memory refused: %s", MOST_BLOCKS * BLOCK_BYTES, hipGetErrorString(e));
-        c.base = (char*)p;
-    }
-    if (!c.words) {
-        void* p = nullptr;
-        e = hipHostMalloc(&p, (size_t)MOST_BLOCKS * WORD_STEP * 4, hipHostMallocPortable);
-        RI_REQUIRE(e == hipSuccess, "ri_decode_stack_take_control: %d bytes of pinned memory refused: %s", MOST_BLOCKS * WORD_STEP * 4, hipGetErrorString(e));
-        c.words = (unsigned*)p;
+        void *base = nullptr, *words = nullptr;
+        e = hipHostMalloc(&words, (size_t)MOST_BLOCKS * WORD_STEP * 4, hipHostMallocPortable);
+        if (e == hipSuccess) e = hipExtMallocWithFlags(&base, (size_t)MOST_BLOCKS * BLOCK_BYTES, hipDeviceMallocUncached);
+        if (e != hipSuccess) {
+            if (words) (void)hipHostFree(words);
+            (void)hipGetLastError();
+            c.refused = true;
+            fprintf(stderr, "[rustinfer_amd] decoding steps run part by part, not in one launch: %d bytes for their control blocks refused (%s)\n",
+                    MOST_BLOCKS * BLOCK_BYTES, hipGetErrorString(e));
+            return 0;
+        }
+        c.base = (char*)base;
+        c.words = (unsigned*)words;
     }
     for (int i = 0; i < MOST_BLOCKS; ++i) {
         if (c.out[i]) continue;

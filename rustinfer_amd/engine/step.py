@@ -111,6 +111,9 @@ class Engine:
         self.cache = CacheManager(model.cache_needs(), page_size, num_pages, max_requests,
                                   max_model_len, device=rt.device, dtype=rt.dtype)
         self.workspace = Workspace(rt.device)
+        if getattr(model, "stack", None) is not None:
+            # now, and not in the first step that asks: it takes memory and waits for the device, which another thread's capture would not survive
+            rt.ops.decode_stack_control(self.workspace)
         # the largest step: max_batch_tokens tokens (or max_requests single tokens padded to a
         # captured batch size) of max_requests rows, every table at full length
         t_max = max(self.max_batch_tokens, self.max_requests)

@@ -565,8 +565,8 @@ def decode_stack_scratch(L: int, d: int, ff: int, H: int, Hkv: int, hd: int, row
 
 
 def decode_stack_control(workspace) -> Optional[int]:
-    """The control block of the one-launch steps of ``workspace``: taken when it is first asked for, given back when the workspace
-    goes.  None if there is none left, or if the stream is under capture and none has been taken."""
+    """The control block of the one-launch steps of ``workspace``: taken when it is first asked for (which waits for the device), given back when the
+    workspace goes.  None if there is none to be had, or if the stream is under capture and none has been taken."""
     block = getattr(workspace, "_stack_control", None)
     if block is None and not torch.cuda.is_current_stream_capturing():
         lib, p, word = _lib(), ctypes.c_void_p(), ctypes.c_void_p()

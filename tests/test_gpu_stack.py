@@ -230,6 +230,60 @@ def test_steps_of_many_keys_go_part_by_part(engines, monkeypatch):
         eng.release(r)
 
 
+def test_an_engine_without_a_control_block_steps_part_by_part(engines, monkeypatch):
+    """None left for this engine's workspace: the same steps, no launch of the whole stack, the parts' own results."""
+    from rustinfer_amd.kernels import ops
+    eng, (cfg, _) = engines("64")
+    assert eng.workspace._stack_control is not None                  # (taken when the engine was built)
+    reqs = random_requests(cfg["vocab_size"], [40, 9, 600], seed=8)
+    stack = eng.model.stack
+    try:
+        eng.model.stack = None
+        parts = _decode(eng, reqs, "eager")
+    finally:
+        eng.model.stack = stack
+    monkeypatch.setattr(ops, "decode_stack_control", lambda workspace: None)
+    monkeypatch.setattr(ops, "decode_stack", None)
+    assert np.array_equal(_decode(eng, reqs, "eager"), parts)
+
+
+@pytest.mark.parametrize("mode", ["eager", "graph"])
+def test_two_engines_step_on_two_streams(engines, mode):
+    """Launches that overlap, each with a control block of its own: what one holds of the chip the other waits for or goes on without, and the results
+    are those of steps by themselves (rows that are not divided: no bit depends on how many blocks took part)."""
+    from rustinfer_amd.engine import StepEntry
+    both = [(engines("64")[0], [40, 9, 300]), (engines("128")[0], [100, 480, 17, 3])]
+    steps = 12
+    rng = np.random.default_rng(5)
+    tokens = rng.integers(0, 512, (2, 8, 512))
+
+    def run(streams):
+        out = [[], []]
+        for k, (eng, lens) in enumerate(both):
+            eng.enable_graphs(mode == "graph", capture_sizes=(1, 2, 4, 8))
+            for r, n in enumerate(lens):
+                eng.step([StepEntry(r, tokens[k, r, :n].tolist(), [])])
+            if mode == "graph":
+                eng.capture_graphs([len(lens)], 512)
+        torch.cuda.synchronize()
+        for s in range(steps):
+            for k, (eng, lens) in enumerate(both):
+                with torch.cuda.stream(streams[k]):
+                    out[k].append(eng.step([StepEntry(r, [int(tokens[k, r, (n + s) % 512])], [0]) for r, n in enumerate(lens)]).clone())
+        torch.cuda.synchronize()
+        for eng, lens in both:
+            eng.check_steps()
+            for r in range(len(lens)):
+                eng.release(r)
+            eng.enable_graphs(False)
+        return [torch.stack(o).cpu().numpy() for o in out]
+
+    alone = run([torch.cuda.current_stream()] * 2)
+    beside = run([torch.cuda.Stream(), torch.cuda.Stream()])
+    for a, b in zip(alone, beside):
+        assert np.isfinite(a).all() and np.array_equal(a, b)
+
+
 def test_control_blocks_are_given_back():
     """A block belongs to one workspace; one that is gone leaves its block to the next, and when all are taken there is none."""
     from rustinfer_amd.engine.context import Workspace

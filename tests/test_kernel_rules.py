@@ -150,3 +150,21 @@ def test_divided_rows_share_no_line_in_the_one_launch_step(lib, H, Hkv, hd):
 def test_long_rows_leave_the_one_launch_step(rows, hd, keys, pays):
     from rustinfer_amd.kernels import ops
     assert ops.decode_stack_pays(rows, hd, keys) is pays
+
+
+def test_no_control_block_is_no_error(lib):
+    """Where the memory of the one-launch step's control blocks is not to be had, here as there is no device, there is no block: steps go part by part."""
+    import torch
+    if torch.cuda.is_available():
+        pytest.skip("there is a device")
+    block, word = ctypes.c_void_p(1), ctypes.c_void_p(1)
+    assert lib.ri_decode_stack_take_control(ctypes.byref(block), ctypes.byref(word)) == 0
+    assert block.value is None and word.value is None
+    from rustinfer_amd.engine.context import Workspace
+    from rustinfer_amd.kernels import ops
+    real, ops.torch.cuda.is_current_stream_capturing = ops.torch.cuda.is_current_stream_capturing, lambda: False
+    try:
+        ws = Workspace(torch.device("cpu"))
+        assert ops.decode_stack_control(ws) is None and not ops.decode_stack_gave_up(ws)
+    finally:
+        ops.torch.cuda.is_current_stream_capturing = real
