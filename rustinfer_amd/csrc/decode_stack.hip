@@ -24,7 +24,10 @@
 // uncached memory and are polled by scalar loads, which do not stand behind the weights (of cached memory, by vector loads: 650 us).
 //
 // Which blocks take part is settled at the start: all of the grid, if all are on the chip (the usual case), else those that had arrived
-// when the first of them had waited `close_ticks`; later ones leave at once.  Items are dealt round to those that take part, so every
+// when the first of them had waited `close_ticks` times what the step takes longer without the rest (of 256 blocks 64: four times); later ones leave at once.
+// (Four rows at the 1B sizes beside a kernel of another stream that holds so many units for 1 ms, us, after `close_ticks` whoever is there / this: 128 units 1115 / 1324,
+// 200 1865 / 1714, 250 12670 / 1617; 254 for 8 ms 36900 / 8700.)  A step has the whole chip or waits for it: part by part those take 825 us, and of two engines that
+// step on two streams, four rows at 1B and eight at 3B, both steps take 1,385 us where launches one after the other take 1,570.  Items are dealt round to those that take part, so every
 // block that is waited for is running, whatever else runs on the device, and the products do not depend on their number.  Every wait is bounded
 // all the same (the one at the start by `join_ticks`, as one block cannot go on alone; `limit_ticks`, MOST_SPINS): then the launch ends, its logits are NaN, and a word
 // in host memory says so.
@@ -623,8 +626,9 @@ __global__ __launch_bounds__(THREADS) void decode_stack_kernel(const StackArgs) 
                 if (!tried && __builtin_amdgcn_readfirstlane(waited > again(A)->close_ticks ? 1 : 0)) {
                     unsigned here = 0;
                     if (lane < 8) here = ld_agent(ctl + (C_ARRIVED + lane) * 32) & ~CLOSED;
-                    here = (unsigned)__builtin_popcountll(__ballot(here > 0)) + (__ballot(here > 1) ? 1u : 0u);
-                    if (here < 2) continue;
+                    unsigned sum = 0;
+                    for (int i = 0; i < 8; ++i) sum += (unsigned)__builtin_amdgcn_readlane((int)here, i);
+                    if (sum < 2 || __builtin_amdgcn_readfirstlane(waited * sum < again(A)->close_ticks * (unsigned)again(A)->expect ? 1 : 0)) continue;
                     tried = true;
                     unsigned first = 0;
                     if (lane == 0) first = add_agent(ctl + C_CLOSING * 32, 1u);

@@ -533,7 +533,7 @@ def linear_residual(act: torch.Tensor, w: torch.Tensor, w_tiled: Optional[torch.
     return a, ssq
 
 
-DECODE_STACK_CLOSE_US = 200.0   # how long the first blocks of a one-launch step wait for the rest before they go on without them
+DECODE_STACK_CLOSE_US = 200.0   # how long the first blocks of a one-launch step wait for the rest before they go on without them, times (all blocks / blocks there)
 DECODE_STACK_JOIN_US = 2e7      # and how long one block waits for a second, without which it cannot go on, before it gives up
 DECODE_STACK_LIMIT_US = 5e6     # and how long blocks wait for each other's results before they do
 DECODE_STACK_GRID = 0           # blocks launched: 0 one a compute unit
