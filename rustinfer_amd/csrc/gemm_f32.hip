@@ -487,29 +487,34 @@ extern "C" void ri_gemm_f32_tile(int M, int N, int* rows, int* columns) {
     *columns = 16 * t.nt;
 }
 
-// The form of gemm_f32_few_kernel: 0: 8 columns a block and 4 turns under way, 1 and 2: 16 and 2, 3: 24 and 2.  Above 4,096 columns
+// The form of gemm_f32_few_kernel: 0: 8 columns a block and 4 turns under way, 1 (up to 4,096 columns) and 2 (above): 16 and 2, 3: 24 and 2.  Above 4,096 columns
 // the one whose rounds of 256 blocks take the least (*cost: in rounds of 8 columns a block); with fewer columns a block the rows of A
-// are read more often.  Measured with 64 bytes a load, us, forms 0 / 2 / 3 at 1 and 8 rows: 6144 x 4096 20.7 26.4 / 26.7 29.7 / 21.9 22.9, 16384 x 2048
-// 27.7 35.4 / 27.9 30.7 / 30.6 33.4, 12288 x 4096 37 48 / 40 43 / 37 41, 28672 x 4096 81 108 / 84 93 / 85 92, 128256 x 1024 95 134 / 97
-// 113 / 92 107; 0 / 1: 2048 x 8192 16 19 / 24 28, 4096 x 4096 14.8 18.6 / 16.1 17.1, 4096 x 14336 49 64 / 49 56.  (Two forms by
-// columns alone, before: 6144 x 4096 29, 16384 x 2048 29 32, 4096 x 14336 49 64.)
+// are read more often.  Measured, us, 8 / 16 / 24 columns at 1 and 8 rows: 6144 x 4096 19.8 24.5 / 26.8 28.1 / 21.0 21.5, 16384 x 2048
+// 27.0 32.2 / 27.8 28.4 / 30.2 30.6, 12288 x 4096 35 46 / 43 45 / 38 39, 28672 x 4096 78 102 / 89 95 / 84 88, 128256 x 1024 89 122 / 100 111 / 88 94.
+// Up to there 8 and 16 at 8 rows: 4096 x 4096 17.4 / 18.6, 4096 x 8192 32.5 / 33.2 (these two take the slower), 4096 x 14336 54 / 49, 4096 x 16384 63 / 55,
+// 3072 x 8192 31.6 / 28.2, 2560 x 8192 31.4 / 27.4, 3072 x 3584 at 0.89 of the time with 16; 2048 x 8192 18.6 / 27.3: one round of half the blocks.
 static int few_form(int M, int N, int K, float* cost) {
     auto rounds = [&](int columns) { return (float)(((N + columns - 1) / columns + 255) / 256); };
     const float one = rounds(8) * (0.96f + 0.0225f * (float)M + (K < 1024 ? 0.1f : 0.f));
     const float two = rounds(16) * 2.f, three = rounds(24) * 2.8f;
     *cost = fminf(one, fminf(two, three));
-    if (N <= 4096) return M > 4 && N > 2048 && K >= 1536 && !(K >= 8192 && (K & (K - 1)) == 0) ? 1 : 0;
+    if (N <= 4096) return M > 4 && N > 2048 && K >= 1536 && !(N < 2560 && K >= 8192 && (K & (K - 1)) == 0) ? 1 : 0;
     return one == *cost ? 0 : two < three ? 2 : 3;
 }
 
 // Whether up to four rows go to the kernel of FMAs, gemm_rows_f32: it reads a kilobyte of a row of W at a time, the tiles 128 bytes
-// of each of eight rows, which costs more the longer the rows are.  But where rows begin a power of two apart its long reads meet on the same
-// channels of memory, and there it pays only against rounds of blocks that are far from full.  Measured, us, 1 and 4 rows, gemm_rows_f32 / the form of
-// the tiles: 5120 x 3072 16.3 18.3 / 17.1 17.8, 5120 x 5120 23.2 26.6 / 25.6 26.4, 27648 x 5120 98 107 / 96 110, 128256 x 3072 242 259 / 251 270,
-// 7000 x 4096 24.6 25.9 / 25.2 26.9, 128256 x 2048 176 183 / 175 179.  The line lies where it did when the tiles read 64 bytes of 16 places (27648 x 5120 120 130, 128256 x 1536 146 155): it
-// takes in some that the tiles would now do faster, 12288 x 6912 61 68 / 59 60, 128256 x 1536 130 145 / 127 135, 2560 x 11008 34 39 / 32 37, 4096 x 14336 47 53 / 40 45.
-// Not taken, as measured then: 12288 x 1536 18.4 21.8 / 17.7 18.9, 28672 x 4096 95 98 / 81 87, 16384 x 2048 34 37 / 28 29, 4096 x 3072 14.9 16.3 / 12.8 14.4, 2048 x 8192 21 24 / 16 17.
-static bool gemm_f32_rows_pay(int M, int N, int K, int ldw) {
+// of each of eight rows.  Measured, time of gemm_rows_f32 / of the tiles' form, at 1, 2, 3 and 4 rows, for 23 numbers of columns and 11 lengths of rows:
+// whole tiles (N % 8 == 0) and chunks (K % 128 == 0), rows no power of two apart:
+//     up to 4,096 columns 1.06 to 1.29 everywhere; 8,192 < N <= 20,480 1.00 to 1.50 (10240 x 5120 1.20 1.21 1.20 1.21)
+//     5,120 to 8,192 columns, K > 3072: 0.88 to 1.05 at one row (7168 x 6912 0.88, 5120 x 9216 0.90, 8192 x 5120 1.05), 0.94 to 1.08 at two (from 4,608 values on
+//     0.94 to 1.05), 0.95 to 1.10 at three, 1.01 to 1.13 at four; shorter rows 0.97 to 1.35
+//     24,576 columns and more: K <= 2304 0.95 to 1.46; longer ones 0.87 to 1.15 (65536 x 4608 0.92 0.87 0.94 0.94, 36864 x 6912 0.95 0.97 0.97 0.98,
+//     28672 x 3072 1.15 0.99 1.07 1.05, 50304 x 5120 0.99 0.97 0.90 0.91)
+// Where rows begin a power of two apart its long reads meet on the same channels of memory, and there it pays only against rounds of blocks that are far from
+// full: us, 1 and 4 rows, gemm_rows_f32 / tiles, taken: 5120 x 4096 at 4 rows 21.4 / 20.3, 9216 x 8192 72 / 64, 128256 x 2048 173 179 / 164 173; not
+// 28672 x 4096 96 102 / 78 85, 16384 x 2048 34 37 / 27 27, 12288 x 4096 39 43 / 38 38, 2048 x 8192 21 24 / 17 17.
+// Sizes with remainders keep the line that was drawn for rows of 64 bytes a load (5001 x 2304, 2049 x 5124, 4111 x 772 are on its side).
+static bool gemm_f32_long_rows(int M, int N, int K, int ldw) {
     if (M > 4) return false;
     if ((ldw & (ldw - 1)) == 0) {
         float cost = 0.f;
@@ -518,6 +523,10 @@ static bool gemm_f32_rows_pay(int M, int N, int K, int ldw) {
     }
     if (N > 4096) return K > 2048 || (K > 1024 && N > 32768) || (K >= 768 && K % 128 != 0);
     return N > 2048 && K >= (N > 3072 ? 7168 : 5120);
+}
+static bool gemm_f32_rows_pay(int M, int N, int K, int ldw) {
+    if (M > 4 || (ldw & (ldw - 1)) == 0 || N % 8 != 0 || K % 128 != 0) return gemm_f32_long_rows(M, N, K, ldw);
+    return N > 20480 ? K > 2304 : N > 4096 && N <= 8192 && ((M == 1 && K > 3072) || (M == 2 && K > 4096));
 }
 
 // The kernel that ri_gemm_f32 takes: -1 gemm_rows_f32, 0 to 3 the form of gemm_f32_few_kernel, 4 the tiles of 16 rows and more.
@@ -529,15 +538,16 @@ extern "C" int ri_gemm_f32_form(int M, int N, int K, int ldw) {
     return few_form(M, N, K, &cost);
 }
 
-// Whether up to eight rows' gate and up product takes ri_gemm_f32_swiglu rather than ri_gemm_f32 and the activation's kernel: not where gemm_rows_f32
-// has that product to itself, but for rows of up to 3,072 values whose rounds of blocks are full.  Measured, us, 1 and 4 rows, two kernels / this:
-// 8192 x 3072 48 51 / 39 40, 9728 x 2560 41 44 / 37 38, 6912 x 2560 29.7 34.8 / 30.8 31.6, 13824 x 5120 100 109 / 97 102, 18944 x 3584 93 98 / 91 95,
-// 14336 x 4096 80 87 / 76 78, 8192 x 2048 29.4 29.4 / 30.5 30.7.  The line lies where it did with 64 bytes a load (6912 x 2560 36 38, 13824 x 5120 128 137): it leaves out
-// what would now pay by 1 to 14 %.  (Behind a deferred norm the product is always this one.)
+// Whether up to eight rows' gate and up product takes ri_gemm_f32_swiglu rather than ri_gemm_f32 and the activation's kernel.  Its blocks hold eight columns of each,
+// so its rounds of 256 blocks are of 2,048 columns; where rows are long the line is at rounds 8/9 full.  Measured, us, 1 and 4 rows, two kernels / this:
+// 9216 x 2304 38.7 42.3 / 33.9 35.0, 9728 x 2560 40 44 / 37 38, 13824 x 2560 55 60 / 49 50, 8192 x 3072 46 51 / 37 38, 14336 x 3584 73 78 / 66 69, 18944 x 3584 93 97 / 91 94,
+// 13824 x 5120 100 108 / 97 102, 17408 x 5120 119 127 / 118 125; not taken 6912 x 2560 29.9 35.0 / 31.7 32.4, 2560 x 3588 21.3 23.2 / 24.3 25.7, 6912 x 5120 53 60 / 57 59, 7168 x 3584
+// 38.7 43.8 / 39.7 41.5; rows of more than 5,120 values keep the two, 24576 x 6144 183 188 / 182 195 (6144 x 6144 57 63 / 51 53).  Rows a power of two apart: 14336 x 4096 78 87 / 75 77,
+// 8192 x 2048 29.6 29.6 / 30.3 30.7.  (Behind a deferred norm the product is always this one.)
 extern "C" int ri_gemm_f32_swiglu_pays(int M, int I, int K, int ldw) {
     if (M > 8) return 0;
-    const bool full = (float)((I + 2047) / 2048) * 2048.f <= 1.03f * (float)I;
-    return !(K > 2048 && gemm_f32_rows_pay(M, 2 * I, K, ldw) && (K > 3072 || !full));
+    const bool full = (I + 2047) / 2048 * 2048 * 8 <= I * 9;
+    return !(K > 2048 && gemm_f32_long_rows(M, 2 * I, K, ldw) && (K > 5120 || !full));
 }
 
 static bool few_scale_ok(const float* ssq, int parts, float eps) {

@@ -168,3 +168,22 @@ def test_no_control_block_is_no_error(lib):
         assert ops.decode_stack_control(ws) is None and not ops.decode_stack_gave_up(ws)
     finally:
         ops.torch.cuda.is_current_stream_capturing = real
+
+
+@pytest.mark.parametrize("N,K,forms", [
+    # columns, values, the kernel at 1, 2, 3, 4 and 8 rows (-1: the one of FMAs): whole tiles and chunks, rows no power of two apart
+    (4096, 14336, (0, 0, 0, 0, 1)), (2560, 11008, (0, 0, 0, 0, 1)), (5120, 5120, (-1, -1, 3, 3, 3)), (7168, 3584, (-1, 2, 2, 2, 2)), (8192, 3072, (0, 2, 2, 2, 2)),
+    (10240, 2560, (0, 0, 0, 0, 3)), (12288, 6912, (3, 3, 3, 3, 3)), (16384, 2304, (0, 2, 2, 2, 2)), (20480, 9216, (0, 2, 2, 2, 2)), (24576, 2304, (3, 3, 3, 3, 3)),
+    (24576, 2560, (-1, -1, -1, -1, 3)), (128256, 1536, (3, 3, 3, 3, 3)), (128256, 3072, (-1, -1, -1, -1, 3)),
+    # remainders, and rows a power of two apart: as they were
+    (5001, 2304, (-1, -1, -1, -1, 3)), (10240, 2564, (-1, -1, -1, -1, 4)), (16384, 2048, (0, 2, 2, 2, 2)), (128256, 2048, (-1, -1, -1, -1, 3)),
+    # five rows and more: sixteen columns a block from 2,560 on, also where rows are 8,192 values or more apart
+    (2056, 8192, (0, 0, 0, 0, 0)), (2560, 8192, (0, 0, 0, 0, 1)), (3072, 8192, (0, 0, 0, 0, 1)), (2048, 8192, (0, 0, 0, 0, 0))])
+def test_kernel_of_32_bit_products_of_few_rows(lib, N, K, forms):
+    assert tuple(lib.ri_gemm_f32_form(M, N, K, K) for M in (1, 2, 3, 4, 8)) == forms
+
+
+@pytest.mark.parametrize("I,K,pays", [(9728, 2560, 1), (13824, 5120, 1), (18944, 3584, 1), (9216, 3072, 1), (6912, 2560, 0), (7168, 3584, 0), (2560, 3588, 0), (24576, 6144, 0),
+                                      (14336, 4096, 1), (8192, 2048, 1)])
+def test_swiglu_in_the_32_bit_product_of_few_rows(lib, I, K, pays):
+    assert [lib.ri_gemm_f32_swiglu_pays(M, I, K, K) for M in (1, 4, 8, 9)] == [pays, pays, 1, 0]
