@@ -26,7 +26,8 @@ SKINNY_MAX_ROWS = 64
 LIBRARY_GEMM_MIN_ROWS = 65
 UNTILED_LIBRARY_MIN_ROWS = 17   # a weight without a second, tile-ordered copy: from this many rows on the GEMM library reads it faster
 UNTILED_LIBRARY_LARGE = 20 << 20 # ... and with fewer rows where it has this many elements, see _untiled_to_library
-FORCE_LIBRARY_GEMM = False      # every bfloat16 product through the GEMM library, no few-row kernels and none of their fused forms
+FORCE_LIBRARY_GEMM = False      # every bfloat16 product through the GEMM library, no few-row kernels and none of their fused forms; of 32-bit products
+                                # neither the norm between two of them nor rotation and cache write fused
                                 # (the reference's RUSTINFER_FORCE_GEMM, crates/infer-backend-cuda/src/kernels/matmul/mod.rs:188-204)
 LIBRARY_GEMM_WORKSPACE_BYTES = 64 << 20
 
@@ -474,7 +475,7 @@ def linear_residual_ok(M: int, w: torch.Tensor, w_tiled: Optional[torch.Tensor],
     N, K = w.shape
     if w.dtype == torch.float32:
         # csrc/gemm_f32.hip; whole chunks of K for this product and for the one behind the norm
-        return (0 < M <= min(8, DEFERRED_NORM_MAX_ROWS) and N % 128 == 0 and K % 128 == 0 and _f32_rows_ok(w) and norm_weight.dtype == torch.float32
+        return (not FORCE_LIBRARY_GEMM and 0 < M <= min(8, DEFERRED_NORM_MAX_ROWS) and N % 128 == 0 and K % 128 == 0 and _f32_rows_ok(w) and norm_weight.dtype == torch.float32
                 and norm_weight.numel() == N and norm_weight.is_contiguous())
     return (not FORCE_LIBRARY_GEMM and w.dtype == torch.bfloat16 and w_tiled is not None and 0 < M <= DEFERRED_NORM_MAX_ROWS
             and N % 16 == 0 and K % 32 == 0 and norm_weight.dtype in _DT and norm_weight.numel() == N

@@ -170,6 +170,16 @@ def test_no_control_block_is_no_error(lib):
         ops.torch.cuda.is_current_stream_capturing = real
 
 
+def test_the_library_switch_leaves_no_norm_between_products_out(monkeypatch):
+    """FORCE_LIBRARY_GEMM: no fused form, of 32-bit products as of bfloat16 ones (the rotation's obeys it too)."""
+    import torch
+    from rustinfer_amd.kernels import ops
+    w, norm = torch.zeros(256, 128), torch.ones(256)
+    assert ops.linear_residual_ok(4, w, None, norm) and ops.linear_residual_ok(4, w.bfloat16(), w, norm)
+    monkeypatch.setattr(ops, "FORCE_LIBRARY_GEMM", True)
+    assert not ops.linear_residual_ok(4, w, None, norm) and not ops.linear_residual_ok(4, w.bfloat16(), w, norm)
+
+
 @pytest.mark.parametrize("N,K,forms", [
     # columns, values, the kernel at 1, 2, 3, 4 and 8 rows (-1: the one of FMAs): whole tiles and chunks, rows no power of two apart
     (4096, 14336, (0, 0, 0, 0, 1)), (2560, 11008, (0, 0, 0, 0, 1)), (5120, 5120, (-1, -1, 3, 3, 3)), (7168, 3584, (-1, 2, 2, 2, 2)), (8192, 3072, (0, 2, 2, 2, 2)),
