@@ -493,10 +493,11 @@ extern "C" void ri_gemm_f32_tile(int M, int N, int* rows, int* columns) {
 // 27.0 32.2 / 27.8 28.4 / 30.2 30.6, 12288 x 4096 35 46 / 43 45 / 38 39, 28672 x 4096 78 102 / 89 95 / 84 88, 128256 x 1024 89 122 / 100 111 / 88 94.
 // Up to there 8 and 16 at 8 rows: 4096 x 4096 17.4 / 18.6, 4096 x 8192 32.5 / 33.2 (these two take the slower), 4096 x 14336 54 / 49, 4096 x 16384 63 / 55,
 // 3072 x 8192 31.6 / 28.2, 2560 x 8192 31.4 / 27.4, 3072 x 3584 at 0.89 of the time with 16; 2048 x 8192 18.6 / 27.3: one round of half the blocks.
+static float few_rounds(int N, int columns) { return (float)(((N + columns - 1) / columns + 255) / 256); }
+static float few_cost8(int M, int N, int K) { return few_rounds(N, 8) * (0.96f + 0.0225f * (float)M + (K < 1024 ? 0.1f : 0.f)); }
 static int few_form(int M, int N, int K, float* cost) {
-    auto rounds = [&](int columns) { return (float)(((N + columns - 1) / columns + 255) / 256); };
-    const float one = rounds(8) * (0.96f + 0.0225f * (float)M + (K < 1024 ? 0.1f : 0.f));
-    const float two = rounds(16) * 2.f, three = rounds(24) * 2.8f;
+    const float one = few_cost8(M, N, K);
+    const float two = few_rounds(N, 16) * 2.f, three = few_rounds(N, 24) * 2.8f;
     *cost = fminf(one, fminf(two, three));
     if (N <= 4096) return M > 4 && N > 2048 && K >= 1536 && !(N < 2560 && K >= 8192 && (K & (K - 1)) == 0) ? 1 : 0;
     return one == *cost ? 0 : two < three ? 2 : 3;
@@ -589,10 +590,13 @@ extern "C" int ri_gemm_f32_scaled(const float* A, int lda, const float* W, int l
     return 0;
 }
 
-// Partial sums of squares that ri_gemm_f32_residual leaves of a row of N values: one for 8 or 16 columns, as ri_gemm_f32's form has them.
+// Partial sums of squares that ri_gemm_f32_residual leaves of a row of N values: one for 8 or 16 columns a block, whichever of the two takes the
+// fewer rounds (24 columns are not among them: their sums lie in no 8 or 16 lanes).  us with the gate/up product behind it, 16 columns for every size that takes 24 elsewhere / this, 1 and
+// 4 rows: 5120 x 13824 and 2 x 3840 104 105 / 88 97, 5120 x 5120 and 2 x 13824 129 133 / 121 129, 6144 x 6144 and 2 x 6144 88 91 / 81 87.
 extern "C" int ri_gemm_f32_residual_parts(int M, int N, int K) {
     float cost = 0.f;
-    return N / (few_form(M, N, K, &cost) == 0 ? 8 : 16);
+    const bool eight = N <= 4096 ? few_form(M, N, K, &cost) == 0 : few_cost8(M, N, K) <= few_rounds(N, 16) * 2.f;
+    return N / (eight ? 8 : 16);
 }
 
 // x[M, N] += A . W^T of up to eight rows, and for the norm behind it (weights norm_w [N]) a[M, N] = x * norm_w and partial sums of x^2, ssq [M, parts].  N % 64 == 0.

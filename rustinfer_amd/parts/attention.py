@@ -143,7 +143,7 @@ class PagedAttention(Mixer):
         if ok is None or not ok(x.shape[0], self.o.weight, self.o.weight_tiled, next_norm.weight):
             return None
         pays = getattr(ops, "linear_residual_pays", None)
-        if pays is not None and self.rt.dtype != torch.float32 and not pays(x.shape[0], self.o.weight):
+        if pays is not None and not pays(x.shape[0], self.o.weight):
             return None
         qkv, table = self._project(ctx, normed, cache)
         attn = self._attend(ctx, qkv, cache, table)

@@ -69,7 +69,7 @@ class SwiGLUMLP(FeedForward):
         if ok is None or not ok(x.shape[0], self.down.weight, self.down.weight_tiled, next_norm.weight):
             return None
         pays = getattr(ops, "linear_residual_pays", None)
-        if pays is not None and self.rt.dtype != torch.float32 and not pays(x.shape[0], self.down.weight):
+        if pays is not None and not pays(x.shape[0], self.down.weight):
             return None
         act = self._activation(ctx, normed)
         a, ssq = ops.linear_residual(act, self.down.weight, self.down.weight_tiled, x, next_norm.weight,

@@ -180,6 +180,28 @@ def test_the_library_switch_leaves_no_norm_between_products_out(monkeypatch):
     assert not ops.linear_residual_ok(4, w, None, norm) and not ops.linear_residual_ok(4, w.bfloat16(), w, norm)
 
 
+@pytest.mark.parametrize("N,K,pays", [
+    (2048, 2048, (1, 1, 1, 1)), (4096, 14336, (1, 1, 1, 1)), (5120, 5120, (1, 1, 1, 0)), (6144, 6144, (1, 1, 1, 0)), (5120, 13824, (0, 0, 0, 0)), (6144, 16384, (0, 0, 0, 0)),
+    (6656, 6656, (0, 0, 1, 1)), (7168, 18944, (0, 0, 1, 1)), (8192, 8192, (1, 1, 1, 1)), (9216, 9216, (1, 1, 1, 0))])
+def test_norms_between_32_bit_products(N, K, pays):
+    """At 1, 2, 4 and 8 rows: not where the product by itself is a faster kernel by more than the norm's own takes."""
+    import torch
+    from rustinfer_amd.kernels import ops
+    w = torch.empty(N, K, device="meta")
+    assert tuple(int(ops.linear_residual_pays(M, w)) for M in (1, 2, 4, 8)) == pays
+
+
+@pytest.mark.parametrize("N,K", [(5120, 13824), (5120, 5120), (6144, 6144), (4608, 4608), (4096, 4096), (8192, 8192), (2048, 8192), (4224, 128)])
+def test_residual_form_of_32_bit_rows_takes_the_fewer_rounds(lib, N, K):
+    """Of 8 and 16 columns a block, in rounds of 256 blocks (16 columns take twice as long): never the one with the more, where they differ by a quarter."""
+    for M in range(1, 9):
+        parts = lib.ri_gemm_f32_residual_parts(M, N, K)
+        assert parts in (N // 8, N // 16) and parts % 4 == 0
+        eight, sixteen = -(-N // 8 // 256), 2 * -(-N // 16 // 256)
+        if N > 4096 and 4 * eight <= 3 * sixteen:
+            assert parts == N // 8
+
+
 @pytest.mark.parametrize("N,K,forms", [
     # columns, values, the kernel at 1, 2, 3, 4 and 8 rows (-1: the one of FMAs): whole tiles and chunks, rows no power of two apart
     (4096, 14336, (0, 0, 0, 0, 1)), (2560, 11008, (0, 0, 0, 0, 1)), (5120, 5120, (-1, -1, 3, 3, 3)), (7168, 3584, (-1, 2, 2, 2, 2)), (8192, 3072, (0, 2, 2, 2, 2)),
