@@ -269,7 +269,7 @@ class ParallelBlock(Part):
         if self.ffn is not None:
             self.ffn.core(ctx, self.set.views(i, proj), self.set.act_view(i, act), None)
         if follow is not None and getattr(follow[0], "plain_rms", False) and getattr(follow[1], "takes_deferred_norm", False):
-            prepared = self.set.output_into(ctx, act, hidden.x, follow[0])
+            prepared = self.set.output_into(ctx, act, hidden.x, *follow)
             if prepared is not None:
                 return None, (follow[0], prepared)
         return self.set.output(ctx, act), None

@@ -198,6 +198,23 @@ def test_profile_forward_and_resize():
         eng.resize_pool(12)
 
 
+@pytest.mark.parametrize("own", [None, "copy"])
+@pytest.mark.parametrize("kind", ["block", "head"])
+def test_a_block_prepares_the_next_ones_input_where_that_one_reads_tiles(own, kind):
+    """The budget of second copies may end between two layers: whose product applies the norm's factor is asked, not the block that prepares it."""
+    from types import SimpleNamespace as S
+    from rustinfer_amd.parts.base import DeferredNorm, ProjectionSet
+    ops = S(linear_residual_ok=lambda *a: True, linear_residual_pays=lambda *a: True, linear_residual=lambda *a: ("rows", "sums"))
+    block = ProjectionSet.__new__(ProjectionSet)
+    block.rt, block.w_in, block.w_out = S(dtype=torch.bfloat16, ops=ops), S(weight_tiled=own), S(weight=None, weight_tiled="copy")
+    x, norm = torch.zeros(3, 8), S(weight=None, eps=1e-5)
+    for copy in (None, "copy"):
+        consumer = S(set=S(w_in=S(weight_tiled=copy))) if kind == "block" else S(weight_tiled=copy)
+        got = block.output_into(S(workspace=None), None, x, norm, consumer)
+        assert (got is None) if copy is None else isinstance(got, DeferredNorm)
+    assert block.output_into(S(workspace=None), None, torch.zeros(9, 8), norm, consumer) is None
+
+
 def test_a_step_that_did_not_run_to_its_end_is_told_once_and_its_requests_are_refused():
     """What the device says after the call: the next step, and whoever waits, raises; live requests are refused until they are released, by the engine or
     through the cache."""
