@@ -37,6 +37,7 @@ class DecodeStack:
         table = struct.pack(f"<{len(addresses)}Q{len(norms)}d", *addresses, *(n.eps for n in norms))
         self.table = torch.frombuffer(bytearray(table), dtype=torch.int64).to(rt.device)
         self._held = weights + [n.weight for n in norms]       # (the table holds addresses: the tensors stay as long as it does)
+        self._taken = rt.weights_taken                         # (and are the parts' own as long as none of them takes another)
         self.norm_dtype = model.final_norm.weight.dtype
         self.scratch_bytes = rt.ops.decode_stack_scratch(len(blocks), model.hidden_size, self.ff, self.H, self.Hkv, self.hd)
 
@@ -75,9 +76,11 @@ class DecodeStack:
                                          first.mixer.head_dim, 16, model.vocab_size)
 
     def takes(self, ctx, caches) -> bool:
-        """Whether the step is of single tokens, all wanted, over one group of caches that holds a layer's after the other, not so many keys that the
+        """Whether the weights are those that were loaded, and the step is of single tokens, all wanted, over one group of caches that holds a layer's after the other, not so many keys that the
         parts are faster, and there is a control block for it."""
         T = ctx.num_tokens
+        if self.rt.weights_taken != self._taken:
+            return False
         if ctx.max_q_len != 1 or ctx.num_want != T or not getattr(ctx, "want_all_in_order", False) or ctx.num_rows < T:
             return False
         groups = getattr(caches, "groups", None)

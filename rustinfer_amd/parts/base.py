@@ -236,6 +236,7 @@ class Runtime:
     # others as the checkpoint has them.
     tile_budget: Optional[int] = None
     tiled_bytes: int = 0          # what the second copies have taken so far
+    weights_taken: int = 0        # how often a part has taken a weight: who keeps weights of several parts sees that one was replaced
 
     def take_tile_budget(self, nbytes: int) -> bool:
         """Whether a second copy of ``nbytes`` may be made; if so it is taken off the budget."""
@@ -319,6 +320,7 @@ class PositionEncoding(Part):
 def stored_to(t: torch.Tensor, rt: Runtime, keep_fp32: bool = False) -> torch.Tensor:
     """Bring a checkpoint tensor to the device.  Floating tensors go to the run
     dtype, except that with ``keep_fp32`` a tensor stored in 32-bit stays 32-bit."""
+    rt.weights_taken += 1
     if t.dtype in (torch.int32, torch.int64, torch.uint8, torch.int8):
         return t.to(device=rt.device, dtype=torch.int32).contiguous()
     if keep_fp32 and t.dtype == torch.float32:

@@ -16,10 +16,13 @@ class Linear:
         self.weight_tiled = None
 
     def set_weight(self, w: torch.Tensor, rt: Runtime, tile: bool = True) -> None:
-        """``tile=False``: the caller keeps a copy of its own for the few-row kernels."""
+        """``tile=False``: the caller keeps a copy of its own for the few-row kernels.  After ``DecoderModel.load`` steps that do not run part by part
+        (models/stack.py), and graphs, hold the addresses of the weights as they were then: the former are not taken any more until the model
+        is loaded again, the latter have to be captured again."""
         if tuple(w.shape) != (self.out_features, self.in_features):
             raise ValueError(f"linear weight {tuple(w.shape)} != {(self.out_features, self.in_features)}")
         self.rt = rt
+        rt.weights_taken += 1
         self.weight = w.to(device=rt.device, dtype=rt.dtype).contiguous()
         # a second copy in the order the few-row kernel streams it (memory is plentiful, bandwidth is not)
         self.weight_tiled = rt.tile(self.weight) if tile else None

@@ -44,6 +44,7 @@ class RMSNorm(Norm):
 
     def load(self, tensors, rt: Runtime) -> None:
         self.rt = rt
+        rt.weights_taken += 1
         if self.one_plus:
             self.weight = (tensors[self.weight_name].to(device=rt.device, dtype=torch.float32) + 1.0).contiguous()
         elif self.weight_32bit:

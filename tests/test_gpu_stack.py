@@ -284,6 +284,27 @@ def test_two_engines_step_on_two_streams(engines, mode):
         assert np.isfinite(a).all() and np.array_equal(a, b)
 
 
+def test_a_replaced_weight_is_read(tmp_path):
+    """A part that takes another weight after the model was loaded: no step reads the old one, of few rows or of many; once the model is loaded again, steps
+    go in one launch again."""
+    from rustinfer_amd.config import LlamaConfig
+    from rustinfer_amd.engine import build_engine
+    from rustinfer_amd.weights import write_random_model
+    write_random_model(LlamaConfig.from_dict(CONFIGS["64"]), 5, str(tmp_path))
+    eng = build_engine(str(tmp_path), dtype="bfloat16", page_size=16, num_pages=64, max_requests=8, max_model_len=512, max_batch_tokens=512)
+    reqs = random_requests(512, [9, 40], seed=4)
+    before = _decode(eng, reqs, "eager")
+    down = eng.model.layers[1].ffn.down
+    down.set_weight(-down.weight, eng.rt)
+    after = _decode(eng, reqs, "eager")
+    eng.model.stack = None
+    assert np.array_equal(_decode(eng, reqs, "eager"), after) and np.abs(after - before).max() > 0.1 * before.std()
+    from rustinfer_amd.models.stack import decode_stack
+    eng.model.stack = decode_stack(eng.model, eng.rt)
+    again = _decode(eng, reqs, "eager")
+    assert not np.array_equal(again, after) and np.abs(again - after).max() < 0.1 * after.std()      # (the launch, with the new weight)
+
+
 def test_control_blocks_are_given_back():
     """A block belongs to one workspace; one that is gone leaves its block to the next, and when all are taken there is none."""
     from rustinfer_amd.engine.context import Workspace
