@@ -485,21 +485,31 @@ def linear_residual_ok(M: int, w: torch.Tensor, w_tiled: Optional[torch.Tensor],
 RESIDUAL_FORM_LARGE = 32 << 20  # elements of a weight from which the residual form's weaknesses cost more than a norm kernel
 
 
-RESIDUAL_FORM_F32_LARGE = 40 << 20  # ... of a 32-bit weight, where its product by itself is another kernel
-
-
 def linear_residual_pays(M: int, w: torch.Tensor) -> bool:
-    """Whether ``linear_residual`` is the faster way for ``M`` rows against ``w [N, K]``, compared
-    with partial sums over slices of K (32-bit rows: the whole product) and the norm's own kernel (which costs 3 to 6 us).  A block of
-    the bfloat16 residual form owns 16 whole columns (8 in ri_gemm_skinny_residual's other forms): it cannot divide K between blocks, so every block asks
+    """Whether ``linear_residual`` is the faster way for ``M`` bfloat16 rows against ``w [N, K]``, compared
+    with partial sums over slices of K and the norm's own kernel (which costs 3 to 6 us).  A block of
+    the residual form owns 16 whole columns (8 in ri_gemm_skinny_residual's other forms): it cannot divide K between blocks, so every block asks
     for all of its rows' activations (beyond eight rows that shows), and 320 blocks on 256 compute
     units take as long as 512.  Measured, us, residual form / partial sums and the norm, at 1, 8, 16 rows:
     4096 x 14336: 19.2 23.2 28.6 / 23.1 24.1 24.4; 4096 x 4096: 7.5 9.0 10.5 / 12.2 13.3 13.1;
     5120 x 5120: 12.8 15.4 20.9 / 17.6 17.3 17.3; 8192 x 8192: 22.8 26.5 32.5 / 28.8 28.6 31.0; 3072 x 8192: 10.8 13.3 16.9 / 15.4 17.0 14.7;
     2048 x 8192 7.8 8.8 14.7 / 10.9 11.7 11.3; 2048 x 2048 4.0 4.6 6.2 / 6.9 7.6 7.7; 5120 x 13824: 26.6 33.2 48.5 / 29.7 30.5 31.0; 5120 x 8192: 15.6 20.3 30.0 /
     21.3 21.6 23.0.  The line counts blocks of 16 columns, as the form was when it was drawn: up to eight rows of the last two sizes it leaves out pairs of steps that
-    would mostly pay, and 16 rows of 3072 x 8192, 2048 x 8192 and 5120 x 5120 it lets in.
+    would mostly pay, and 16 rows of 3072 x 8192, 2048 x 8192 and 5120 x 5120 it lets in."""
+    N, K = w.shape
+    if N * K < RESIDUAL_FORM_LARGE:
+        return True
+    tiles = N // 16
+    blocks = tiles * 2 if tiles <= 128 else tiles
+    at_once = 256 * -(-blocks // 256)
+    return M <= 8 and blocks * 4 >= at_once * 3
 
+
+RESIDUAL_FORM_F32_LARGE = 40 << 20  # elements of a 32-bit weight up to which the norm's kernel costs four rows more than another kernel for the product gives
+
+
+def linear_residual_f32_pays(M: int, w: torch.Tensor) -> bool:
+    """``linear_residual_pays`` for ``M`` 32-bit rows, compared with the whole product and the norm's own kernel.
     The 32-bit residual form is a tile of 8 or 16 columns: where the product by itself takes tiles of 24 columns or the kernel of FMAs and is long, that is worth
     more than the norm's kernel.  Measured with the gate/up product behind it (2 I of its columns after the colon), us, product and norm / residual form, at 1, 2, 4, 8 rows:
     2048 x 2048: 8192 39.5 39.1 40.0 42.2 / 36.5 36.7 37.7 40.0; 4096 x 14336: 3072 67 69 74 80 / 64 66 71 77; 5120 x 5120: 13824 124 125 131 141 / 121 123 129 146;
@@ -507,14 +517,7 @@ def linear_residual_pays(M: int, w: torch.Tensor) -> bool:
     6656 x 6656: 6656 102 105 114 124 / 108 108 111 121; 7168 x 18944: 2048 117 123 131 141 / 126 126 128 138; 8192 x 22016: 1024 153 154 161 171 / 149 154 158 169;
     9216 x 9216: 4096 121 124 133 142 / 116 117 125 145."""
     N, K = w.shape
-    if w.dtype == torch.float32:
-        return N <= 4096 or (M <= 4 and N * K <= RESIDUAL_FORM_F32_LARGE) or _lib().ri_gemm_f32_form(M, N, K, w.stride(0)) in (0, 2)
-    if N * K < RESIDUAL_FORM_LARGE:
-        return True
-    tiles = N // 16
-    blocks = tiles * 2 if tiles <= 128 else tiles
-    at_once = 256 * -(-blocks // 256)
-    return M <= 8 and blocks * 4 >= at_once * 3
+    return N <= 4096 or (M <= 4 and N * K <= RESIDUAL_FORM_F32_LARGE) or _lib().ri_gemm_f32_form(M, N, K, w.stride(0)) in (0, 2)
 
 
 def linear_residual(act: torch.Tensor, w: torch.Tensor, w_tiled: Optional[torch.Tensor], x: torch.Tensor,

@@ -188,7 +188,7 @@ def test_norms_between_32_bit_products(N, K, pays):
     import torch
     from rustinfer_amd.kernels import ops
     w = torch.empty(N, K, device="meta")
-    assert tuple(int(ops.linear_residual_pays(M, w)) for M in (1, 2, 4, 8)) == pays
+    assert tuple(int(ops.linear_residual_f32_pays(M, w)) for M in (1, 2, 4, 8)) == pays
 
 
 @pytest.mark.parametrize("N,K", [(5120, 13824), (5120, 5120), (6144, 6144), (4608, 4608), (4096, 4096), (8192, 8192), (2048, 8192), (4224, 128)])
