@@ -307,11 +307,14 @@ def qkv_rope_weight(w_qkv: torch.Tensor, hd: int) -> Optional[torch.Tensor]:
     return tile_weight(w_qkv[order].contiguous())
 
 
+_NO_SCALE = (ctypes.c_void_p(0), 0, ctypes.c_float(0.0))
+
+
 def _scale_args(scale, M: int, who: str):
     """``scale`` = (ssq [M, P] float32, eps) of a norm whose factor this product applies itself
     (see ``linear_residual``), or None."""
     if scale is None:
-        return ctypes.c_void_p(0), 0, ctypes.c_float(0.0)
+        return _NO_SCALE
     ssq, eps = scale
     _dev(ssq)
     if ssq.dtype != torch.float32 or ssq.dim() != 2 or ssq.shape[0] != M or not ssq.is_contiguous():

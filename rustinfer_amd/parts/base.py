@@ -514,14 +514,16 @@ class ProjectionSet:
         return self.rt.ops.linear_delta(act, self.w_out.weight, ctx.workspace, "projset.out",
                                         self.w_out.weight_tiled, out_dtype=torch.float32)
 
+    INTO_MOST_ROWS = 8       # with more, the plain products' other forms are the faster ones, and read normed rows
+
     def output_into(self, ctx, act, x, next_norm, consumer):
         """Few rows: the parts' summed outputs added to ``x`` by their product, and the input of ``consumer`` (a block of such parts, or the head) behind
         ``next_norm`` as a ``DeferredNorm``.  None, and nothing done, where that form does not apply."""
         ops, w = self.rt.ops, self.w_out
         ok = getattr(ops, "linear_residual_ok", None)
         reader = getattr(getattr(consumer, "set", None), "w_in", consumer)       # whose product applies the norm's factor
-        # (up to eight rows: with more, the plain products' other forms are the faster ones, and read normed rows; so they are for a weight without a copy in tile order)
-        if ok is None or self.rt.dtype != torch.bfloat16 or x.shape[0] > 8 or not ok(x.shape[0], w.weight, w.weight_tiled, next_norm.weight) \
+        # (the plain products' other forms are the faster ones for a weight without a copy in tile order, too)
+        if ok is None or self.rt.dtype != torch.bfloat16 or x.shape[0] > self.INTO_MOST_ROWS or not ok(x.shape[0], w.weight, w.weight_tiled, next_norm.weight) \
                 or getattr(reader, "weight_tiled", None) is None or not ops.linear_residual_pays(x.shape[0], w.weight):
             return None
         a, ssq = ops.linear_residual(act, w.weight, w.weight_tiled, x, next_norm.weight, ctx.workspace, "deferred")

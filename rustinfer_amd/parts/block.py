@@ -257,7 +257,8 @@ class ParallelBlock(Part):
         return (self.norm, self)
 
     def _run(self, ctx, hidden: Hidden, cache, mixer_only: bool, follow=None):
-        normed = ctx.workspace.get("block.normed", hidden.x.shape[0], self.hidden_size, self.rt.dtype)
+        T = hidden.x.shape[0]
+        normed = ctx.workspace.get("block.normed", T, self.hidden_size, self.rt.dtype)
         inp = hidden.input_behind(ctx, self.norm, normed)
         proj, act = self.set.project(ctx, inp, members=int(self.mixer is not None) if mixer_only else None)
         i = 0
@@ -268,7 +269,7 @@ class ParallelBlock(Part):
             return None
         if self.ffn is not None:
             self.ffn.core(ctx, self.set.views(i, proj), self.set.act_view(i, act), None)
-        if follow is not None and getattr(follow[0], "plain_rms", False) and getattr(follow[1], "takes_deferred_norm", False):
+        if T <= self.set.INTO_MOST_ROWS and follow is not None and getattr(follow[0], "plain_rms", False) and getattr(follow[1], "takes_deferred_norm", False):
             prepared = self.set.output_into(ctx, act, hidden.x, *follow)
             if prepared is not None:
                 return None, (follow[0], prepared)
