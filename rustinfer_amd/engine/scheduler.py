@@ -144,9 +144,14 @@ class Scheduler:
 
     def fail_running(self) -> None:
         """End every request that has started, as ``"error"``: what the cache holds of them is lost, and tokens that have not reached the host
-        do not come any more."""
-        for req in list(self.running):
-            self._finish(req, "error")
+        do not come any more.  Those of which no step has run yet wait again."""
+        for req in reversed(list(self.running)):
+            if self.cache.has_request(req.request_id) or req.num_computed or req.output:
+                self._finish(req, "error")
+            else:
+                self.running.remove(req)
+                req.state = WAITING
+                self.waiting.appendleft(req)
         for req in self.finished + list(self.waiting):           # (ended by their length, or preempted, in the meantime)
             if req.output and req.output[-1] == PENDING:
                 while req.output and req.output[-1] == PENDING:

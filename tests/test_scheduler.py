@@ -403,8 +403,12 @@ def test_requests_that_have_started_end_as_errors_and_unknown_tokens_go():
     a, b, cc, d = (next(r for r in s.finished + s.running + list(s.waiting) if r.request_id == i) for i in "abcd")
     assert a.state == b.state == "finished" and a.output == [PENDING] and b.output == [PENDING] * 2 and cc.output == [PENDING] * 2
     assert s.resolve(a, 0, 7) and s.resolve(b, 0, 8) and s.resolve(cc, 0, 9)       # the first step's have arrived
+    e, f = s.add(req("e", 5)), s.add(req("f", 5))
+    s.schedule()                                            # e and f are let in, and the step that was missed comes to light before theirs runs
+    assert [r.request_id for r in s.running] == ["c", "d", "e"]
     s.fail_running()
     assert a.output == [7] and a.finish_reason == "length"
     assert b.output == [8] and b.finish_reason == "error" and cc.output == [9] and cc.finish_reason == "error"
-    assert not s.running and d.finish_reason == ("error" if d in s.finished else None)
+    assert d.finish_reason == "error" and not s.running and list(s.waiting) == [e, f]
+    assert portions(s.schedule()) == [("e", 0, 5, True), ("f", 0, 5, True)]
     c.check()
