@@ -88,7 +88,7 @@ constexpr size_t LINE = 128;
 __host__ __device__ inline size_t slot_outputs(int G, int hd) { return (size_t)G * hd * 4; }                             // bytes; hd is 64 or 128
 constexpr size_t SLOT_SUMS = LINE;                                                                                       // G pairs of floats, G <= 16
 static_assert(64 * 4 % LINE == 0 && 16 * 8 <= SLOT_SUMS, "a slot is whole lines");
-// A row's keys are divided between blocks in parts of at most `share` (a multiple of PART_KEYS: a part's waves take spans of SPAN keys in turn).
+// A row's keys are divided between blocks in parts of `share` keys or fewer, PART_KEYS at least: the waves of all of a row's parts take spans of SPAN keys in turn.
 constexpr int SPAN = 32, PART_KEYS = WAVES * SPAN, WHOLE_KEYS = 2 * PART_KEYS;
 __host__ __device__ inline int parts_of(int len, int share) { return len <= share ? 1 : (len + share - 1) / share; }
 __host__ __device__ inline Offsets stack_offsets(int M, int d, int ff, int H, int Hkv, int hd, int blocks) {
@@ -361,13 +361,14 @@ struct Reader {
 };
 
 // How the rows' keys are divided: between all blocks by the rows' lengths, so that the longest share, which the others wait for, is as short as it can be (with as many parts
-// for every row, 8 rows of which one had 16,000 keys and the others 100 took 1,644 us at the 3B sizes, now 1,113, part by part 1,145; 4,000 and 100 1,103 / 1,002 / 1,069).  Not where the longest row has
+// for every row, 8 rows of which one had 16,000 keys and the others 100 took 1,644 us at the 3B sizes, now 1,113, part by part 1,145; 4,000 and 100 1,103 / 1,002 / 1,069).  The share
+// goes by spans: by PART_KEYS eight rows of 2,100 keys had three parts each where four fit, 1,402 us a step at the 8B sizes, now 1,387.  Not where the longest row has
 // WHOLE_KEYS keys or fewer: a merge costs more than it gives.  `total` of a share: the parts of all rows.
 template <typename F> __device__ __forceinline__ int share_of(F total, int longest, int budget, int rows, int lane) {
     if (longest <= WHOLE_KEYS || budget <= rows) return 0x7fffffff;
-    for (int unit = PART_KEYS; unit < 1 << 24; unit *= 2) {                // (the 64 lanes try a multiple each)
-        const unsigned long long fits = __ballot(total(unit * (lane + 1)) <= budget);
-        if (fits) return unit * (__builtin_ctzll(fits) + 1);
+    for (int from = PART_KEYS, unit = SPAN; unit < 1 << 24; from += 64 * unit, unit *= 2) {        // (the 64 lanes try one each)
+        const unsigned long long fits = __ballot(total(from + unit * lane) <= budget);
+        if (fits) return from + unit * __builtin_ctzll(fits);
     }
     return 0x7fffffff;
 }
