@@ -111,10 +111,10 @@ class PagedAttention(Mixer):
             fused = ops.qkv_rope_fused(*args, **kw) or (
                 scale is None and split is not None
                 and ops.qkv_split_pays(rows.shape[0], self.qkv_fused.shape[0], self.qkv_fused.shape[1]) and split(*args, ws))
-        few = getattr(ops, "qkv_rope_f32", None)
-        if not fused and few is not None and rows.dtype == torch.float32 and self.own_kv and self.qk_transform is None and cache.write:
-            fused = few(rows, self.qkv.weight, qkv, self.num_heads, self.num_kv_heads, self.head_dim, rotary,
-                        ctx.positions, ctx.row_of_token, cache.k, cache.v, table, cache.page_size, **kw)
+        if not fused and self.rt.dtype == torch.float32 and self.own_kv and self.qk_transform is None and cache.write:
+            few = getattr(ops, "qkv_rope_f32", None)
+            fused = few is not None and few(rows, self.qkv.weight, qkv, self.num_heads, self.num_kv_heads, self.head_dim, rotary,
+                                            ctx.positions, ctx.row_of_token, cache.k, cache.v, table, cache.page_size, **kw)
         if not fused:
             self.qkv.forward(rows, qkv, scale, workspace=ws)
             if self.qk_transform is not None:
